@@ -30,9 +30,12 @@ __device__ __forceinline__ uint16_t f2bf(float f) {
   return __builtin_bit_cast(uint16_t, b);
 }
 
-// Pack two floats into one dword of two bf16 (lo in bits 0..15).
+// Pack two floats into one dword of two bf16 (lo in bits 0..15): one v_cvt_pk_bf16_f32 (converted one by one and joined
+// with shifts it takes four instructions).
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t pack2bf(float lo, float hi) {
-  return (uint32_t)f2bf(lo) | ((uint32_t)f2bf(hi) << 16);
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t{lo, hi}), bf16x2_t));
 }
 
 // 8 bf16 <-> 8 floats through one 16-byte vector.
@@ -54,7 +57,6 @@ __device__ __forceinline__ u32x4_t pack8(const float* f) {
 // operands never widened in VGPRs): the decode GEMVs' inner product
 // (The pairs are taken with __builtin_shufflevector from the bf16x8 view: bit-casting the extracted
 // dword a[i] to bf16x2 made hipcc (ROCm 7.2) feed element 0's registers to all four instructions.)
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ float dot8_bf16(const u32x4_t& a, const u32x4_t& b, float acc) {
   const bf16x8_t av = __builtin_bit_cast(bf16x8_t, a), bv = __builtin_bit_cast(bf16x8_t, b);
   acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_shufflevector(av, av, 0, 1), __builtin_shufflevector(bv, bv, 0, 1), acc, false);
