@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include "common.h"
+#include "few_rows.h"
 
 #include <execinfo.h>
 #include <csignal>
@@ -662,8 +663,12 @@ void topk_sample(at::Tensor x, int64_t k, double temperature, c10::optional<at::
            "topk_sample");
 }
 
+// Rows from which a decode projection of bf16 weights runs on the matrix cores (csrc/few_rows.hip) instead of a dot product a
+// wave (csrc/decode_fused.hip, gemv.hip)
+constexpr int kFewRows = 3;
+
 // y[M, N] = x[M, K] @ W^T (W bf16 or int8 [Nw, K], Nw = N or 2N with glu), optional per-row fp32
-// scale / per-tensor scale, optional bias [Nw]; M <= 8.
+// scale / per-tensor scale, optional bias [Nw]; M <= 8, without a bias M <= 32.
 void gemv(at::Tensor x, at::Tensor w, c10::optional<at::Tensor> scale, double tscale, c10::optional<at::Tensor> bias,
           at::Tensor y, bool glu) {
   check_cuda(x, "x");
@@ -674,7 +679,7 @@ void gemv(at::Tensor x, at::Tensor w, c10::optional<at::Tensor> scale, double ts
   const bool i8 = w.scalar_type() == at::kChar;
   TORCH_CHECK(i8 || w.scalar_type() == at::kBFloat16, "gemv: weight must be bf16 or int8");
   const int M = x.size(0), K = x.size(1), N = y.size(1);
-  TORCH_CHECK(M >= 1 && M <= 8 && y.size(0) == M, "gemv: 1 <= M <= 8");
+  TORCH_CHECK(M >= 1 && M <= (bias.has_value() ? 8 : nxd::FEW_MAX_ROWS) && y.size(0) == M, "gemv: 1 <= M <= 8 (32 without a bias)");
   TORCH_CHECK(w.size(1) == K && w.size(0) == (glu ? 2 * N : N), "gemv: weight shape mismatch");
   const int epl = i8 ? 16 : 8;
   TORCH_CHECK(K % epl == 0 && x.stride(0) % 8 == 0 && w.stride(0) % epl == 0, "gemv: K / leading dims must be multiples of ",
@@ -693,6 +698,25 @@ void gemv(at::Tensor x, at::Tensor w, c10::optional<at::Tensor> scale, double ts
     TORCH_CHECK(bias->is_contiguous() && bias->numel() == w.size(0), "gemv: bias must be [Nw]");
     bp = bias->data_ptr();
   }
+  // The matrix-core kernel from kFewRows rows on, and for all int8 rows with a scale a row (one row of 16384 x 2048
+  // int8: 13.6 us against 16.7 of the vector kernel)
+  if (!bp && (i8 ? sp != nullptr && tscale == 1.0 : M >= kFewRows && !sp && tscale == 1.0)) {
+    nxd::FewRowsParams f{};
+    f.x = static_cast<const uint16_t*>(x.data_ptr());
+    f.ldx = x.stride(0);
+    f.w = w.data_ptr();
+    f.ldw = w.stride(0);
+    f.wscale = sp;
+    f.ws_stride = 1;
+    f.y = static_cast<uint16_t*>(y.data_ptr());
+    f.ldy = y.stride(0);
+    f.M = M;
+    f.N = N;
+    f.K = K;
+    const int rc = nxd::few_rows_launch(glu ? nxd::FEW_GLU : nxd::FEW_STORE, f, cur_stream());
+    if (rc >= 0) return check_rc(rc, "gemv");
+  }
+  TORCH_CHECK(M <= 8, "gemv: more than 8 rows of a size the matrix-core kernel does not take");
   check_rc(nxd::gemv_launch(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), i8, sp, (float)tscale, bp,
                             y.data_ptr(), y.stride(0), M, N, K, glu, cur_stream()),
            "gemv");
@@ -911,14 +935,20 @@ void moe_combine_bwd(at::Tensor dout, at::Tensor ys, at::Tensor inv, at::Tensor 
 
 // Fused decode GEMV (csrc/decode_fused.hip).  epi: 0 plain, 1 residual add into y (in place),
 // 2 SwiGLU on a fused [2N, K] gate/up weight, 3 QKV with RoPE + KV-cache write.  norm_w: RMSNorm
-// of x fused as a prologue.  x [M, K], w [Nw, K], y [M, N] bf16, M <= 8.
+// of x fused as a prologue.  x [M, K], w [Nw, K], y [M, N] bf16, M <= 8; M <= 32 where csrc/few_rows.hip takes the
+// call (dgemv_rows).  int8 w: wscale [Nw] or [1] fp32.  tickets: zeroed int32 counters (left zeroed) with which a long
+// reduction may be split over workgroups.
 void dgemv(int64_t epi, at::Tensor x, c10::optional<at::Tensor> norm_w, double eps, at::Tensor w, at::Tensor y,
            int64_t nq, int64_t nkv, int64_t D, c10::optional<at::Tensor> cos_t, c10::optional<at::Tensor> sin_t,
            c10::optional<at::Tensor> pos, int64_t T, c10::optional<at::Tensor> kc, c10::optional<at::Tensor> vc,
            c10::optional<at::Tensor> cache_idx, c10::optional<at::Tensor> xadd, c10::optional<at::Tensor> yadd,
-           c10::optional<at::Tensor> xidx, c10::optional<at::Tensor> xcopy) {
+           c10::optional<at::Tensor> xidx, c10::optional<at::Tensor> xcopy, c10::optional<at::Tensor> wscale,
+           c10::optional<at::Tensor> tickets) {
   check_bf16(x, "x");
-  check_bf16(w, "w");
+  const bool i8 = w.scalar_type() == at::kChar;
+  if (!i8) check_bf16(w, "w");
+  TORCH_CHECK(w.is_cuda(), "dgemv: w must be a GPU tensor");
+  TORCH_CHECK(i8 == wscale.has_value(), "dgemv: a scale for int8 weights, and only for them");
   // epi 0 with an fp32 y: the unrounded partial sum (row-parallel projection at TP > 1)
   float* yf = nullptr;
   if (epi == 0 && y.scalar_type() == at::kFloat) {
@@ -946,8 +976,9 @@ void dgemv(int64_t epi, at::Tensor x, c10::optional<at::Tensor> norm_w, double e
       xc = xcopy->data_ptr();
     }
   }
-  TORCH_CHECK(M >= 1 && M <= 8 && y.size(0) == M, "dgemv: 1..8 rows");
-  TORCH_CHECK(K % 8 == 0 && x.stride(0) % 8 == 0 && w.stride(0) % 8 == 0 && w.size(1) == K, "dgemv: K / strides");
+  TORCH_CHECK(M >= 1 && M <= nxd::FEW_MAX_ROWS && y.size(0) == M, "dgemv: 1..32 rows");
+  const int unit = i8 ? 16 : 8;
+  TORCH_CHECK(K % unit == 0 && x.stride(0) % 8 == 0 && w.stride(0) % unit == 0 && w.size(1) == K, "dgemv: K / strides");
   check_aligned16(x, "x");
   check_aligned16(w, "w");
   TORCH_CHECK(w.size(0) == (epi == 2 ? 2 * N : N), "dgemv: weight rows vs output columns");
@@ -956,7 +987,6 @@ void dgemv(int64_t epi, at::Tensor x, c10::optional<at::Tensor> norm_w, double e
     check_bf16(*norm_w, "norm_w");
     TORCH_CHECK(norm_w->is_contiguous() && norm_w->numel() == K, "dgemv: norm weight [K]");
     check_aligned16(*norm_w, "norm_w");
-    TORCH_CHECK(M * K * 2 <= 65536, "dgemv: fused norm needs M * K <= 32768");
     nw = norm_w->data_ptr();
   }
   const float *cp = nullptr, *sp = nullptr;
@@ -1017,6 +1047,59 @@ void dgemv(int64_t epi, at::Tensor x, c10::optional<at::Tensor> norm_w, double e
                 "dgemv: yadd fp32 contiguous [>=M, N]");
     ya = yadd->data_ptr<float>();
   }
+  if ((i8 || M >= kFewRows) && !xa && !ya) {
+    nxd::FewRowsParams f{};
+    f.x = static_cast<const uint16_t*>(x.data_ptr());
+    f.ldx = x.stride(0);
+    f.xidx = xi;
+    f.xrows = x.size(0);
+    f.xcopy = static_cast<uint16_t*>(xc);
+    f.norm_w = static_cast<const uint16_t*>(nw);
+    f.eps = (float)eps;
+    f.w = w.data_ptr();
+    f.ldw = w.stride(0);
+    if (i8) {
+      TORCH_CHECK(wscale->scalar_type() == at::kFloat && wscale->is_cuda() && wscale->is_contiguous() &&
+                      (wscale->numel() == 1 || wscale->numel() == w.size(0)),
+                  "dgemv: wscale fp32 [Nw] or [1]");
+      f.wscale = wscale->data_ptr<float>();
+      f.ws_stride = wscale->numel() == 1 ? 0 : 1;
+    }
+    f.y = yf ? nullptr : static_cast<uint16_t*>(y.data_ptr());
+    f.ldy = y.stride(0);
+    f.yf = yf;
+    f.alpha = 1.f;
+    f.M = (int)M;
+    f.N = (int)N;
+    f.K = (int)K;
+    f.nq = (int)nq;
+    f.nkv = (int)nkv;
+    f.D = (int)D;
+    f.cos_t = cp;
+    f.sin_t = sp;
+    f.pos = pp;
+    f.T = (int)T;
+    f.kc = static_cast<uint16_t*>(kp);
+    f.vc = static_cast<uint16_t*>(vp);
+    f.c_sb = c_sb;
+    f.c_sh = c_sh;
+    f.c_sl = c_sl;
+    f.cache_idx = ci;
+    f.Lmax = Lmax;
+    f.max_pos = max_pos;
+    at::Tensor ws;
+    int need = 0;
+    const int64_t floats = epi == 1 && tickets.has_value() ? nxd::few_rows_workspace((int)M, (int)N, (int)K, &need) : 0;
+    if (floats && tickets->numel() >= need) {
+      TORCH_CHECK(tickets->scalar_type() == at::kInt && tickets->is_cuda() && tickets->is_contiguous(), "dgemv: int32 tickets");
+      ws = at::empty({floats}, x.options().dtype(at::kFloat));
+      f.ws = ws.data_ptr<float>();
+      f.tickets = tickets->data_ptr<int>();
+    }
+    const int rc = nxd::few_rows_launch(yf ? nxd::FEW_F32 : (int)epi, f, cur_stream());
+    if (rc >= 0) return check_rc(rc, "dgemv");
+  }
+  TORCH_CHECK(M <= 8 && !i8 && (!nw || M * K * 2 <= 65536), "dgemv: up to 8 rows of bf16 weights (M * K <= 32768 with a norm) at these sizes");
   check_rc(nxd::dgemv_launch((int)epi, x.data_ptr(), x.stride(0), nw, (float)eps, w.data_ptr(), w.stride(0), y.data_ptr(),
                              y.stride(0), (int)M, (int)N, (int)K, (int)nq, (int)nkv, (int)D, cp, sp, pp, (int)T, kp, vp,
                              c_sb, c_sh, c_sl, ci, Lmax, max_pos, xa, ya, cur_stream(), xi, x.size(0), xc, yf),
@@ -1118,7 +1201,8 @@ PYBIND11_MODULE(_C, m) {
   m.def("dgemv", &dgemv, py::arg("epi"), py::arg("x"), py::arg("norm_w"), py::arg("eps"), py::arg("w"), py::arg("y"),
         py::arg("nq"), py::arg("nkv"), py::arg("D"), py::arg("cos_t"), py::arg("sin_t"), py::arg("pos"), py::arg("T"),
         py::arg("kc"), py::arg("vc"), py::arg("cache_idx"), py::arg("xadd") = py::none(), py::arg("yadd") = py::none(),
-        py::arg("xidx") = py::none(), py::arg("xcopy") = py::none());
+        py::arg("xidx") = py::none(), py::arg("xcopy") = py::none(), py::arg("wscale") = py::none(),
+        py::arg("tickets") = py::none());
   // decode A/B knobs: 0 = GLU row pairs per wave, 1 = GEMV k-slices (0 auto), 2 = MFMA decode attention on/off,
   // 3 = GEMV early epilogue / prologue reads on/off, 5 = bs = 1 GEMV forced occupancy (0 natural | 7 | 8 waves / SIMD)
   m.def("decode_set_knob", [](int which, int value) {

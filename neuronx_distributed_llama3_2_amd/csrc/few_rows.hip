@@ -1,0 +1,652 @@
+// y[M, N] = epilogue(x[M, K] w[N, K]^T) for 1 to 32 activation rows, bf16 or int8 weights: the projections of a decode
+// step, each one launch with the element-wise work around it (RMSNorm of the input, residual add, SwiGLU, rotary
+// positions and cache write, squared ReLU, capped fp32 logits).
+//
+// What bounds it is reading the weights once.  So weights go from memory straight to LDS (global_load_lds: no registers
+// held while they are on the way), 256 contiguous bytes (int8: 128) of a row at a time -- whole lines --, with several
+// stages of every wave under way; the row pieces are stored rotated (XOR of the piece's number with the row's), so that
+// the MFMA operands (16 rows x 16 bytes) are read back without bank conflicts.  A workgroup has tiles of R weight rows;
+// its waves take 128 elements of the reduction in turn, and their sums meet in LDS, where a wave of its own finishes
+// them (epilogue reads and stores never wait for weights, nor weights for them).  The activations are the other operand of
+// v_mfma_f32_16x16x32_bf16.  What a CU gets from the caches is about what it gets from memory, so activations count
+// like weights: they are read in operand order once a workgroup and kept in registers over its tiles where they fit.
+// RMSNorm costs no pass over the rows: the products are those of bf16(x g), the sums of squares come from the same
+// operands, and 1 / rms is a factor of the finished sums.  int8 weights are widened exactly (to bf16) on their way from LDS.
+#include "few_rows.h"
+
+namespace nxd {
+namespace few {
+
+constexpr int KC = 128;   // reduction elements of a stage
+
+__device__ __forceinline__ void dma16(const void* base, uint32_t at, uint32_t lds) {   // 64 lanes x 16 B: base + at -> LDS lds + 16 lane
+  uint32_t keep;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep)
+               : "v"(at), "s"(base), "s"(lds)
+               : "memory");
+}
+
+// int8 x 8 -> bf16 x 8 (exact)
+__device__ __forceinline__ u32x4_t widen8(uint32_t lo, uint32_t hi) {
+  float f[8];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    f[i] = (float)(int8_t)(lo >> (8 * i));
+    f[4 + i] = (float)(int8_t)(hi >> (8 * i));
+  }
+  return pack8(f);
+}
+
+// weight row r of a tile
+template <int EPI, int R>
+__device__ __forceinline__ int row_of(const FewRowsParams& p, int tile, int r) {
+  constexpr int HR = R / 2;
+  if (EPI == FEW_GLU) return min(tile * HR + (r & (HR - 1)), p.N - 1) + (r < HR ? 0 : p.N);
+  if (EPI == FEW_ROPE_KV) {
+    const int half = p.D / 2, qk = (p.nq + p.nkv) * (half / HR);
+    if (tile < qk) return tile / (half / HR) * p.D + tile % (half / HR) * HR + (r & (HR - 1)) + (r < HR ? 0 : half);
+    return min((p.nq + p.nkv) * p.D + (tile - qk) * R + r, p.N - 1);
+  }
+  return min(tile * R + r, p.N - 1);
+}
+
+// Geometry of a workgroup: NW waves that stream weights and FW that finish tiles; R weight rows a tile; M in MT tiles of
+// 16 rows; D stages of a wave under way; CW chunks of the reduction a wave, their activations held in registers for
+// all tiles (0: any number, activations streamed beside the weights)
+template <int R, int MT, bool I8, int NW, int CW, int D>
+struct Shape {
+  static constexpr int ROWB = I8 ? KC : 2 * KC;          // bytes of a row in a stage
+  static constexpr int STAGE = R * ROWB;                 // bytes of a stage of a wave
+  static constexpr int DMAS = STAGE / 1024;              // loads of a stage
+  static constexpr int RING = NW * D * STAGE;
+  static constexpr int PART = NW * MT * 64 * 16;         // the waves' sums of a tile
+  static constexpr int SQ = NW * MT * 16 * 4;            // the waves' sums of squares
+  static constexpr int FW = NW + MT > 12 ? 1 : MT;       // waves that finish tiles (12 waves leave each 168 registers)
+};
+
+// all loads but those of the newest n stages have come (OPS loads a stage, n < D)
+template <int OPS, int D, int N = D - 1>
+__device__ __forceinline__ void wait_stages(int n) {
+  static_assert(OPS * (D - 1) < 64, "the counter has 6 bits");
+  if constexpr (N > 0) {
+    if (n >= N) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(OPS * N) : "memory");
+    else wait_stages<OPS, D, N - 1>(n);
+  } else {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
+}
+
+__device__ __forceinline__ void meet() {   // LDS writes are there; loads from memory stay under way
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// The input rows: row m is x[m], or the table's row xidx[m] (as zeros for an id outside it)
+template <bool XI>
+__device__ __forceinline__ uint32_t input_row(const FewRowsParams& p, int m, bool& ok) {   // element offset
+  ok = true;
+  if constexpr (XI) {
+    const int64_t id = p.xidx[m];
+    ok = id >= 0 && id < p.xrows;
+    return (uint32_t)((id < 0 ? 0 : id >= p.xrows ? p.xrows - 1 : id) * p.ldx);
+  } else {
+    return (uint32_t)(m * p.ldx);
+  }
+}
+
+// The wave that finishes row tile t of every weight tile: sums of the streaming waves -> epilogue.  Lane (c, q) has
+// activation row m = 16 t + c and weight rows 4 q .. 4 q + 3 of the tile (R == 8: q < 2, the rest are copies).
+template <int EPI, bool NORM, int R, bool I8>
+struct Finish {
+  static constexpr int HR = R / 2;
+  const FewRowsParams& p;
+  const int lane, q, m, half;
+  const bool live, wide, wide_c;   // a row that is there; its 4 values go out in one store (also to the cache)
+  int row, tile, n;
+  bool rot;
+  float rstd;
+  uint16_t y_pre[4];
+  float cs[4], sn[4], scale[4];
+  int64_t at, slot;
+
+  __device__ __forceinline__ Finish(const FewRowsParams& p_, int lane_, int t)
+      : p(p_), lane(lane_), q(lane_ >> 4), m(min(16 * t + (lane_ & 15), p_.M - 1)), half(p_.D / 2), live(16 * t + (lane_ & 15) < p_.M),
+        wide(p_.ldy % 4 == 0 && (EPI == FEW_F32 ? (uintptr_t)p_.yf % 16 : (uintptr_t)p_.y % 8) == 0),
+        wide_c(EPI == FEW_ROPE_KV && (p_.c_sb | p_.c_sh | p_.c_sl) % 4 == 0 && ((uintptr_t)p_.kc | (uintptr_t)p_.vc) % 8 == 0) {
+    if (EPI == FEW_ROPE_KV) {
+      at = p.pos[m];
+      slot = p.cache_idx ? p.cache_idx[m / p.T] : m / p.T;
+    }
+  }
+
+  template <int NW>
+  __device__ __forceinline__ void squares(const float* sq, int stride) {   // 1 / rms of the row
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) s += sq[i * stride];
+    rstd = rsqrtf(s / (float)p.K + p.eps);
+  }
+
+  __device__ __forceinline__ void fetch(int tile_) {   // what the epilogue reads, before the sums are there
+    tile = tile_;
+    const int r = (4 * q) & (R - 1);
+    row = row_of<EPI, R>(p, tile, r);
+    rot = EPI == FEW_ROPE_KV && tile < (p.nq + p.nkv) * (half / HR);
+    n = EPI == FEW_GLU ? tile * HR + (r & (HR - 1)) : EPI == FEW_ROPE_KV ? row : tile * R + r;
+    if (I8) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) scale[i] = p.wscale[row_of<EPI, R>(p, tile, r + i) * p.ws_stride];
+    }
+    if (EPI == FEW_RESID) {
+      const uint16_t* y = p.y + (int64_t)m * p.ldy;
+      if (wide && n + 4 <= p.N) {
+        const u32x2_t v = *reinterpret_cast<const u32x2_t*>(y + n);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) y_pre[i] = (uint16_t)(v[i >> 1] >> (16 * (i & 1)));
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) y_pre[i] = y[min(n + i, p.N - 1)];
+      }
+    }
+    if (rot) {
+      const int64_t a = (at < 0 ? 0 : at >= p.max_pos ? p.max_pos - 1 : at) * half + (row % p.D) % half;
+      const f32x4_t cv = *reinterpret_cast<const f32x4_t*>(p.cos_t + a), sv = *reinterpret_cast<const f32x4_t*>(p.sin_t + a);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) cs[i] = cv[i], sn[i] = sv[i];
+    }
+  }
+
+  __device__ __forceinline__ void put(uint16_t* to, const uint16_t (&o)[4], int left, bool whole) const {   // `left` of the 4 values are there
+    if (whole && left >= 4) {
+      *reinterpret_cast<u32x2_t*>(to) = u32x2_t{(uint32_t)o[0] | (uint32_t)o[1] << 16, (uint32_t)o[2] | (uint32_t)o[3] << 16};
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (i < left) to[i] = o[i];
+    }
+  }
+
+  // A part of the reduction: its sums go through to memory (every part has a place of its own) ...
+  __device__ __forceinline__ float* parts(int at) const { return p.ws + (int64_t)at * p.splits * 256 + lane; }
+  __device__ __forceinline__ void leave(const f32x4_t& v, int at) const {
+    float* ws = parts(at) + blockIdx.x % p.splits * 256;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) __hip_atomic_store(ws + 64 * i, v[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  // ... and are added up in the parts' order, whichever comes last
+  __device__ __forceinline__ f32x4_t collect(int at) const {
+    const float* ws = parts(at);
+    f32x4_t v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int j = 0; j < p.splits; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] += __hip_atomic_load(ws + j * 256 + 64 * i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return v;
+  }
+
+  __device__ __forceinline__ void finish(f32x4_t v) {
+    if (NORM) v *= rstd;
+    if (I8) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] *= scale[i];
+    }
+    f32x4_t other;   // the pairs' other halves: HR rows away
+    if (EPI == FEW_GLU || EPI == FEW_ROPE_KV) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) other[i] = __shfl_xor(v[i], 16 * (HR / 4), 64);
+    }
+    if (!live || 4 * q >= (EPI == FEW_GLU ? HR : R)) return;
+    uint16_t o[4];
+    if (EPI == FEW_F32) {
+      float* y = p.yf + (int64_t)m * p.ldy + n;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float z = v[i] * p.alpha;
+        v[i] = p.cap > 0.f ? p.cap * tanhf(z / p.cap) : z;
+      }
+      if (wide && n + 4 <= p.N) {
+        *reinterpret_cast<f32x4_t*>(y) = v;
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (n + i < p.N) y[i] = v[i];
+      }
+      return;
+    }
+    const bool first = 4 * q < HR;   // of the pairs' halves
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (EPI == FEW_GLU) {
+        o[i] = f2bf(v[i] / (1.f + __expf(-v[i])) * other[i]);
+      } else if (EPI == FEW_RESID) {
+        o[i] = f2bf(bf2f(y_pre[i]) + bf2f(f2bf(v[i])));
+      } else if (EPI == FEW_RELU2) {
+        o[i] = f2bf(fmaxf(v[i], 0.f) * fmaxf(v[i], 0.f));
+      } else if (EPI == FEW_ROPE_KV && rot) {
+        const float one = bf2f(f2bf(v[i])), two = bf2f(f2bf(other[i]));   // bf16 projection outputs
+        o[i] = f2bf(first ? one * cs[i] - two * sn[i] : one * cs[i] + two * sn[i]);
+      } else {
+        o[i] = f2bf(v[i]);
+      }
+    }
+    if (EPI == FEW_ROPE_KV) {
+      const int qk_rows = (p.nq + p.nkv) * p.D;
+      const int left = rot ? 4 : p.N - (qk_rows + (tile - (p.nq + p.nkv) * (half / HR)) * R + 4 * q);
+      if (left <= 0) return;
+      put(p.y + (int64_t)m * p.ldy + row, o, left, wide);
+      const int vr = row - (rot ? p.nq * p.D : qk_rows);   // of the keys, or of the values
+      if (vr < 0 || at < 0 || at >= p.Lmax) return;
+      put((rot ? p.kc : p.vc) + slot * p.c_sb + (int64_t)(vr / p.D) * p.c_sh + at * p.c_sl + vr % p.D, o, left, wide_c);
+    } else {
+      if (n < p.N) put(p.y + (int64_t)m * p.ldy + n, o, p.N - n, wide);
+    }
+  }
+};
+
+template <int EPI, bool NORM, bool XI, int R, int MT, bool I8, int NW, int CW, int D, bool SPLIT>
+__global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) kernel(FewRowsParams p, int tiles) {
+  using S = Shape<R, MT, I8, NW, CW, D>;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  f32x4_t* part = reinterpret_cast<f32x4_t*>(smem + S::RING);       // [NW][MT][64]
+  float* sq = reinterpret_cast<float*>(smem + S::RING + S::PART);   // [NW][16 MT]
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 15, q = lane >> 4;
+  static_assert(!SPLIT || (CW > 0 && !NORM), "split reductions hold their activations and need no norm");
+  const int step = SPLIT ? gridDim.x / p.splits : gridDim.x, tile0 = SPLIT ? blockIdx.x / p.splits : blockIdx.x;
+
+  // NORM: the weight of the norm waits in `part` for the activations to come
+  uint16_t* gs = reinterpret_cast<uint16_t*>(part);
+  constexpr bool GS = NORM && CW > 0;
+  static_assert(!GS || NW * CW * KC * 2 <= S::PART, "the norm's weight in LDS");
+
+  // Twice a tile all waves meet: when `part` is free, and when it is full
+  if (w >= NW) {
+    if (GS) {
+      for (int k = (tid - NW * 64) * 8; k < p.K; k += S::FW * 512)
+        *reinterpret_cast<u32x4_t*>(gs + k) = *reinterpret_cast<const u32x4_t*>(p.norm_w + k);
+      meet();
+    }
+    constexpr int T = MT / S::FW;
+    Finish<EPI, NORM, R, I8> f0(p, lane, (w - NW) * T);
+    Finish<EPI, NORM, R, I8> f1(p, lane, (w - NW) * T + T - 1);
+    for (int tile = tile0; tile < tiles; tile += step) {
+      if (!SPLIT) {
+        f0.fetch(tile);
+        if (T > 1) f1.fetch(tile);
+      }
+      meet();
+      meet();
+      if (NORM && tile == tile0) {
+        const float* mine = sq + (w - NW) * T * 16 + c;
+        f0.template squares<NW>(mine, 16 * MT);
+        if (T > 1) f1.template squares<NW>(mine + 16, 16 * MT);
+      }
+      const f32x4_t* mine = part + (w - NW) * T * 64 + lane;
+      f32x4_t v = mine[0];
+#pragma unroll
+      for (int i = 1; i < NW; ++i) v += mine[i * MT * 64];
+      f32x4_t u;
+      if (T > 1) {
+        u = mine[64];
+#pragma unroll
+        for (int i = 1; i < NW; ++i) u += mine[(i * MT + 1) * 64];
+      }
+      if constexpr (SPLIT) {
+        f0.leave(v, tile * MT + (w - NW) * T);
+        if (T > 1) f1.leave(u, tile * MT + (w - NW) * T + 1);
+      } else {
+        f0.finish(v);
+        if (T > 1) f1.finish(u);
+      }
+    }
+    if constexpr (SPLIT) {   // lane j: a ticket of the j-th tile; the last part to take one finishes the tile
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        const int mine = (tile0 + lane * step) * MT + (w - NW) * T + t;
+        const bool there = tile0 + lane * step < tiles;
+        int n = -1;
+        if (there) n = __hip_atomic_fetch_add(p.tickets + mine, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const bool last = n == p.splits - 1;
+        if (last) __hip_atomic_store(p.tickets + mine, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");   // (no instruction: keeps the loads below the tickets)
+        for (uint64_t todo = __ballot(last); todo; todo &= todo - 1) {
+          const int tile = tile0 + __builtin_ctzll(todo) * step;
+          if (t == 0) {
+            f0.fetch(tile);
+            f0.finish(f0.collect(tile * MT + (w - NW) * T));
+          } else {
+            f1.fetch(tile);
+            f1.finish(f1.collect(tile * MT + (w - NW) * T + 1));
+          }
+        }
+      }
+    }
+    return;
+  }
+
+  const int nck = (p.K + KC - 1) / KC;
+  int c0 = 0, c1 = nck;   // chunks of this workgroup
+  if (SPLIT) {
+    const int part = blockIdx.x % p.splits, n = (nck + p.splits - 1) / p.splits;
+    c0 = min(part * n, nck), c1 = min(c0 + n, nck);
+  }
+  const int wc = c0 + w, cw = (c1 - wc + NW - 1) / NW;   // of this wave: wc, wc + NW, ...
+  char* ring = smem + w * D * S::STAGE;
+  const uint32_t ring_at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)ring;
+
+  // ---- this lane's input rows (rows past M repeat the last one: their sums are not stored)
+  uint32_t xrow[MT];   // (element offsets: the rows lie within 4 GB)
+  bool xok[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) xrow[t] = input_row<XI>(p, min(16 * t + c, p.M - 1), xok[t]);
+  // element of operand f of a chunk that this lane starts at
+  auto kof = [&](int f) { return I8 ? 64 * (f >> 1) + 16 * q + 8 * (f & 1) : 32 * f + 8 * q; };
+  auto load_x = [&](u32x4_t (&xv)[MT][4], int chunk) {
+#pragma unroll
+    for (int t = 0; t < MT; ++t)   // (both halves of a line one after the other)
+#pragma unroll
+      for (int f = 0; f < 4; ++f) xv[t][f] = *reinterpret_cast<const u32x4_t*>(p.x + (xrow[t] + (uint32_t)min(chunk * KC + kof(f), p.K - 8)));
+  };
+  auto load_g = [&](u32x4_t (&g)[4], int chunk) {
+#pragma unroll
+    for (int f = 0; f < 4; ++f) g[f] = *reinterpret_cast<const u32x4_t*>(p.norm_w + min(chunk * KC + kof(f), p.K - 8));
+  };
+  float ss[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) ss[t] = 0.f;
+  // raw rows -> operands: zeros past the end; NORM: times the weight, with the squares summed the first time (1 / rms is
+  // a factor of the sums)
+  auto ready_x = [&](u32x4_t (&xv)[MT][4], const u32x4_t (&g)[4], int chunk, bool first) {
+    const bool tail = (chunk + 1) * KC > p.K;
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int f = 0; f < 4; ++f) {
+        const int k = chunk * KC + kof(f);
+        u32x4_t v = xv[t][f];
+        if (XI && !xok[t]) v = u32x4_t{0u, 0u, 0u, 0u};
+        if (tail && k >= p.K) v = u32x4_t{0u, 0u, 0u, 0u};
+        if (XI && first && p.xcopy && blockIdx.x == 0 && 16 * t + c < p.M && k < p.K)
+          *reinterpret_cast<u32x4_t*>(p.xcopy + (int64_t)(16 * t + c) * p.K + k) = v;
+        if (NORM) {
+          if (first) ss[t] = dot8_bf16(v, v, ss[t]);
+          float a[8], b[8];
+          unpack8(v, a);
+          unpack8(g[f], b);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) a[j] *= b[j];
+          v = pack8(a);
+        }
+        xv[t][f] = v;
+      }
+  };
+
+  // ---- weights: the next stage to issue
+  uint32_t wrow[S::DMAS];   // (byte offsets: the weights take less than 4 GB)
+  int it = tile0, ic = 0, is = 0, ahead = 0;   // its tile, chunk and place in the ring; stages under way
+  // Every workgroup begins elsewhere in the reduction: rows lie a power of two apart, and the same piece of all of
+  // them for all workgroups at a time is one channel's work
+  const int rot = CW == 0 && cw > 0 ? blockIdx.x % cw : 0;
+  auto order = [&](int i) {
+    if (CW > 0) return i;
+    const int j = i + rot;
+    return j < cw ? j : j - cw;
+  };
+  auto issue = [&]() {
+    if (it >= tiles || cw <= 0) return;
+    if (ic == 0) {
+#pragma unroll
+      for (int j = 0; j < S::DMAS; ++j) {
+        const int r = I8 ? 8 * j + (lane >> 3) : 4 * j + (lane >> 4);
+        wrow[j] = (uint32_t)row_of<EPI, R>(p, it, r) * (uint32_t)p.ldw * (I8 ? 1 : 2);
+      }
+    }
+    const int chunk = wc + order(ic) * NW;
+#pragma unroll
+    for (int j = 0; j < S::DMAS; ++j) {
+      int seg;   // the piece of the row that goes to this lane's place
+      if (I8) {
+        const int r = 8 * j + (lane >> 3);
+        seg = (lane & 7) ^ ((r >> 1) & 7);
+      } else {
+        const int r = 4 * j + (lane >> 4);
+        seg = (lane & 15) ^ (r & 15);
+      }
+      const uint32_t at = min(chunk * S::ROWB + 16 * seg, p.K * (I8 ? 1 : 2) - 16);
+      dma16(p.w, wrow[j] + at, __builtin_amdgcn_readfirstlane(ring_at + is * S::STAGE + j * 1024));
+    }
+    ++ahead;
+    if (++ic == cw) ic = 0, it += step;
+    if (++is == D) is = 0;
+  };
+
+  f32x4_t acc[MT];
+  int cs = 0;   // place in the ring of the stage to use
+  auto take = [&](u32x4_t (&wf)[I8 ? 2 : 4]) {   // its pieces, as this lane's operands
+    const char* st = ring + cs * S::STAGE;
+    const int r = c & (R - 1);
+#pragma unroll
+    for (int s = 0; s < (I8 ? 2 : 4); ++s)
+      wf[s] = *reinterpret_cast<const u32x4_t*>(st + r * S::ROWB + (((4 * s + q) ^ (I8 ? (r >> 1) & 7 : r & 15)) << 4));
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (the place may be filled again)
+    --ahead;
+    if (++cs == D) cs = 0;
+  };
+  auto multiply = [&](const u32x4_t (&wf)[I8 ? 2 : 4], const u32x4_t (&xv)[MT][4]) {
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+      u32x4_t b;
+      if constexpr (I8) b = widen8(wf[f >> 1][2 * (f & 1)], wf[f >> 1][2 * (f & 1) + 1]);
+      else b = wf[f];
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, b), __builtin_bit_cast(bf16x8_t, xv[t][f]), acc[t], 0, 0, 0);
+    }
+  };
+  auto clear = [&]() {
+#pragma unroll
+    for (int t = 0; t < MT; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  };
+  auto squares = [&]() {
+    if (!NORM) return;
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      float v = ss[t];
+      v += __shfl_xor(v, 16, 64);
+      v += __shfl_xor(v, 32, 64);
+      if (q == 0) sq[w * 16 * MT + 16 * t + c] = v;
+    }
+  };
+  auto publish = [&]() {
+    meet();
+#pragma unroll
+    for (int t = 0; t < MT; ++t) part[(w * MT + t) * 64 + lane] = acc[t];
+    meet();
+  };
+
+  if constexpr (CW > 0) {
+    u32x4_t x[CW][MT][4];
+#pragma unroll
+    for (int i = 0; i < CW; ++i) load_x(x[i], min(wc + i * NW, nck - 1));   // (chunks past the last one are not used)
+#pragma unroll
+    for (int i = 0; i < D; ++i) issue();
+    if (GS) meet();
+#pragma unroll
+    for (int i = 0; i < CW; ++i) {
+      u32x4_t g[4];
+      if (GS) {
+#pragma unroll
+        for (int f = 0; f < 4; ++f) g[f] = *reinterpret_cast<const u32x4_t*>(gs + min((wc + i * NW) * KC + kof(f), p.K - 8));
+      }
+      ready_x(x[i], g, wc + i * NW, i < cw);
+    }
+    squares();
+    for (int tile = tile0; tile < tiles; tile += step) {
+      clear();
+#pragma unroll
+      for (int i = 0; i < CW; ++i) {
+        if (i >= cw) break;
+        u32x4_t wf[I8 ? 2 : 4];
+        wait_stages<S::DMAS, D>(ahead - 1);
+        take(wf);
+        issue();
+        multiply(wf, x[i]);
+      }
+      publish();
+    }
+  } else {
+    constexpr int XL = 4 * MT + (NORM ? 4 : 0);   // loads of a stage beside the weights'
+    u32x4_t x[D][MT][4], g[NORM ? D : 1][4];
+    auto fetch = [&](u32x4_t (&xv)[MT][4], u32x4_t (&gv)[4]) {
+      if (it < tiles && cw > 0) {
+        load_x(xv, wc + order(ic) * NW);
+        if (NORM) load_g(gv, wc + order(ic) * NW);
+      }
+      issue();
+    };
+#pragma unroll
+    for (int i = 0; i < D; ++i) fetch(x[i], g[NORM ? i : 0]);
+    int tile = tile0, i = 0;
+    bool first = true;
+    clear();
+    if (cw <= 0) squares();
+    for (; cw <= 0 && tile < tiles; tile += step) publish();
+    while (tile < tiles) {
+#pragma unroll
+      for (int u = 0; u < D; ++u) {
+        if (tile >= tiles) break;
+        u32x4_t wf[I8 ? 2 : 4];
+        wait_stages<XL, D>(ahead - 1);   // (of XL + DMAS loads a stage: the stage has come, and the next one's x nearly)
+        take(wf);
+        ready_x(x[u], g[NORM ? u : 0], wc + order(i) * NW, first);
+        multiply(wf, x[u]);
+        fetch(x[u], g[NORM ? u : 0]);
+        if (++i == cw) {
+          if (first) squares();
+          first = false;
+          publish();
+          clear();
+          i = 0, tile += step;
+        }
+      }
+    }
+  }
+}
+
+template <int EPI, int R>
+static int64_t tiles_of(const FewRowsParams& p) {
+  if (EPI == FEW_GLU) return ceil_div64(p.N, R / 2);
+  if (EPI == FEW_ROPE_KV) return (int64_t)(p.nq + p.nkv) * (p.D / 2 / (R / 2)) + ceil_div64((int64_t)p.nkv * p.D, R);
+  return ceil_div64(p.N, R);
+}
+
+
+template <int EPI, bool NORM, bool XI, int R, int MT, bool I8, int NW, int CW, int D, bool SPLIT = false>
+static int launch(FewRowsParams p, hipStream_t s, int splits = 1) {
+  using S = Shape<R, MT, I8, NW, CW, D>;
+  const int nck = ceil_div(p.K, KC);
+  if (CW > 0 && ceil_div(nck, splits) > NW * CW) return -2;
+  constexpr size_t lds = S::RING + S::PART + S::SQ;
+  static_assert(lds <= 160 * 1024, "LDS of a workgroup");
+  const int64_t tiles = tiles_of<EPI, R>(p);
+  auto* f = &kernel<EPI, NORM, XI, R, MT, I8, NW, CW, D, SPLIT>;
+  static const int per = [&] {   // workgroups of a CU
+    int n = 0;
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(f), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, f, (NW + S::FW) * 64, lds) != hipSuccess) return 0;
+    return n;
+  }();
+  if (per < 1) return 1;
+  const int64_t room = 256 * (int64_t)per / splits;   // workgroups side by side along the rows
+  const int64_t rounds = ceil_div64(tiles, room < 1 ? 1 : room), groups = ceil_div64(tiles, rounds);
+  if (SPLIT && rounds > 64) return -2;   // (a lane for every tile's ticket)
+  p.splits = splits;
+  hipLaunchKernelGGL(f, dim3((unsigned)(groups * splits)), dim3((NW + S::FW) * 64), lds, s, p, (int)tiles);
+  return hipGetLastError() == hipSuccess ? 0 : 1;
+}
+
+// Which geometry (times in us at 4 / 16 / 32 rows, bf16, weights from memory):
+//   K <= 2048: activations stay in 8 waves' registers and a workgroup goes over the tiles of 16 rows: 16384 x 2048 with
+//     norm and SwiGLU 14.1 / 15.0 / 16.9 (activations streamed 15.8 / 19.0 / 71; int8 11.6 / 12.4 / 14.8),
+//     128256 x 2048 86 / 92 / 98 (int8 46 / 50 / 54).
+//     Up to 256 tiles there is a tile or less for a CU and streaming begins sooner: 3072 x 2048 6.1 / 6.8 against
+//     6.6 / 7.9 (up to 16 rows: two tiles' operands of a streamed norm do not fit the registers, 19.9 against 10.5).
+//   K <= 4224: 11 waves of 3 chunks: 28672 x 4096 40 / 43 / 55 (streamed 46 / 55 / 225; int8 25 / 27 / 40); without a norm and
+//     up to 256 tiles streamed: 4096 x 4096 9.0 / 10.9 / 13.1 against 9.0 / 10.8 / 14.8.
+//   longer: streamed, tiles of 16 rows for more than 2048 weight rows (4096 x 14336 23 / 28 / 38, of 8 rows 25 / 39 / 58),
+//     else of 8, so that every CU has one (2048 x 8192 9.5 / 13.0 / 18.8, of 16 rows 11.5 / 15.4 / 20.8).  A workgroup of 8
+//     weight rows reads all of the activations for them, 4 times the weights' bytes at 32 rows and past what the caches
+//     deliver to a CU; from 9 rows on the reduction is split instead, each workgroup keeping the activations of
+//     2048 elements for its tiles: 10.7 / 12.1 / 14.5 (2048 x 12288: 12.9 / 19.1 / 27 -> 14.9 / 16.8 / 20).
+constexpr int kSplitFrom = 9;   // rows
+
+template <int EPI, bool NORM, bool XI, int MT, bool I8>
+static int pick(const FewRowsParams& p, hipStream_t s) {
+  constexpr int DA = I8 ? (MT == 1 ? 6 : 4) : MT == 1 ? 4 : 3;   // (int8 stages have half the bytes)
+  const int nck = ceil_div(p.K, KC);
+  const int64_t tiles = tiles_of<EPI, 16>(p);
+  if constexpr (NORM) {
+    if (nck > 33) return -1;
+    if (MT == 1 && tiles <= 256 && nck <= 16) return launch<EPI, true, XI, 16, 1, I8, 8, 0, 2>(p, s);
+    if (nck <= 16) return launch<EPI, true, XI, 16, MT, I8, 8, 2, DA>(p, s);
+    return launch<EPI, true, XI, 16, MT, I8, 11, 3, 3>(p, s);
+  } else {
+    constexpr int D = MT == 1 ? 4 : 2;
+    if (tiles > 256) {
+      if (nck <= 16) return launch<EPI, false, false, 16, MT, I8, 8, 2, DA>(p, s);
+      if (nck <= 33) return launch<EPI, false, false, 16, MT, I8, 11, 3, 3>(p, s);
+    }
+    if (tiles > 128) return launch<EPI, false, false, 16, MT, I8, 8, 0, D>(p, s);
+    if constexpr (EPI == FEW_STORE || EPI == FEW_RESID) {
+      if (p.ws && p.M >= kSplitFrom && nck > 33) return launch<EPI, false, false, 16, MT, I8, 8, 2, I8 ? 4 : 2, true>(p, s, ceil_div(nck, 16));
+    }
+    return launch<EPI, false, false, 8, MT, I8, 8, 0, D>(p, s);
+  }
+}
+
+template <int EPI, bool NORM, bool XI>
+static int rows(const FewRowsParams& p, hipStream_t s) {
+  if constexpr (EPI != FEW_RELU2) {   // (the squared ReLU's model has no int8 weights)
+    if (p.wscale) return p.M <= 16 ? pick<EPI, NORM, XI, 1, true>(p, s) : pick<EPI, NORM, XI, 2, true>(p, s);
+  }
+  if (p.wscale) return -1;
+  return p.M <= 16 ? pick<EPI, NORM, XI, 1, false>(p, s) : pick<EPI, NORM, XI, 2, false>(p, s);
+}
+
+template <int EPI>
+static int norms(const FewRowsParams& p, hipStream_t s) {
+  return p.norm_w ? rows<EPI, true, false>(p, s) : rows<EPI, false, false>(p, s);
+}
+
+}  // namespace few
+
+int64_t few_rows_workspace(int M, int N, int K, int* tickets) {
+  const int nck = ceil_div(K, few::KC), MT = M <= 16 ? 1 : 2;
+  if (M < few::kSplitFrom || M > FEW_MAX_ROWS || nck <= 33 || N > 2048) return *tickets = 0;
+  *tickets = ceil_div(N, 16) * MT;
+  return (int64_t)*tickets * ceil_div(nck, 16) * 256;
+}
+
+int few_rows_launch(int epi, const FewRowsParams& p, hipStream_t s) {
+  const int unit = p.wscale ? 16 : 8;   // elements of 16 bytes of weights
+  if (p.M < 1 || p.M > FEW_MAX_ROWS || p.N < 1 || p.K < unit || p.K % unit || p.ldw % unit || p.ldx % 8) return -1;
+  // 32-bit offsets, and their sums with a row's length
+  const int64_t wrows = epi == FEW_GLU ? 2 * (int64_t)p.N : p.N;
+  if ((wrows + 16) * p.ldw * (p.wscale ? 1 : 2) >= (1LL << 32) || ((p.xidx ? p.xrows : p.M) + 1) * p.ldx >= (1LL << 31)) return -1;
+  if (p.xidx && (epi != FEW_ROPE_KV || !p.norm_w || p.xrows < 1)) return -4;
+  if (epi == FEW_ROPE_KV && (p.D % 32 || !p.norm_w || ((uintptr_t)p.cos_t | (uintptr_t)p.sin_t) % 16)) return -1;
+  switch (epi) {
+    case FEW_STORE: return few::norms<FEW_STORE>(p, s);
+    case FEW_RESID: return p.norm_w ? -1 : few::rows<FEW_RESID, false, false>(p, s);
+    case FEW_GLU: return few::norms<FEW_GLU>(p, s);
+    case FEW_ROPE_KV: return p.xidx ? few::rows<FEW_ROPE_KV, true, true>(p, s) : few::rows<FEW_ROPE_KV, true, false>(p, s);
+    case FEW_F32: return few::norms<FEW_F32>(p, s);
+    case FEW_RELU2: return p.norm_w ? -1 : few::rows<FEW_RELU2, false, false>(p, s);
+  }
+  return -1;
+}
+
+}  // namespace nxd

@@ -3,6 +3,7 @@
 #include "bindings_util.h"
 #include "channel_delta.h"
 #include "experts.h"
+#include "few_rows.h"
 #include "group_norm.h"
 
 namespace nxd {
@@ -15,7 +16,6 @@ int moe_route_launch(const RouterParams&, hipStream_t);
 int clamped_glu_launch(bool, const GluParams&, bool, hipStream_t);
 int gather_rows_launch(const void*, const int*, void*, int64_t, int64_t, int64_t, hipStream_t);
 int experts_few_launch(const RouterParams&, const ExpertFewParams&, hipStream_t);
-int linear_few_launch(const LinearFewParams&, hipStream_t);
 int expert_rows_launch(bool, const ExpertRowsParams&, hipStream_t);
 int grouped_gemm_launch(int, const void*, const void*, void*, const int*, int, int, int, int, int, hipStream_t);
 int grouped_rowgemm_launch(int, const void*, const void*, void*, const int*, int, int, int, int, hipStream_t);
@@ -312,25 +312,42 @@ void experts_few(Tensor h, Tensor router, std::vector<int64_t> rule, double scal
   check_rc(nxd::experts_few_launch(r, p, cur_stream()), "experts_few");
 }
 
-// y [M, N] = x [M, K] w^T, up to 16 rows
-void linear_few(Tensor x, Tensor w, Tensor y) {
-  for (const Tensor* t : {&x, &w, &y})
+// y [M, N] = epilogue(x [M, K] w^T), up to 32 rows (csrc/few_rows.hip).  epi: 0 bf16, 4 fp32 alpha y (cap > 0: cap tanh(alpha y / cap)),
+// 5 squared ReLU.  tickets: zeroed int32 counters (left zeroed) with which a long reduction may be split over workgroups
+void linear_few(Tensor x, Tensor w, Tensor y, int64_t epi, double alpha, double cap, Opt tickets) {
+  for (const Tensor* t : {&x, &w})
     TORCH_CHECK(t->is_cuda() && t->scalar_type() == at::kBFloat16 && t->dim() == 2 && t->stride(1) == 1, "linear_few: bf16 matrices");
-  nxd::LinearFewParams p{};
+  TORCH_CHECK(epi == nxd::FEW_STORE || epi == nxd::FEW_F32 || epi == nxd::FEW_RELU2, "linear_few: epilogue");
+  TORCH_CHECK(y.is_cuda() && y.scalar_type() == (epi == nxd::FEW_F32 ? at::kFloat : at::kBFloat16) && y.dim() == 2 && y.stride(1) == 1, "linear_few: y");
+  nxd::FewRowsParams p{};
   p.M = (int)x.size(0);
   p.K = (int)x.size(1);
   p.N = (int)w.size(0);
-  TORCH_CHECK(p.M >= 1 && p.M <= 16 && p.K >= 8 && p.K % 8 == 0 && p.N >= 1 && x.stride(0) < (1 << 24), "linear_few: 1..16 rows, K a multiple of 8");
+  TORCH_CHECK(p.M >= 1 && p.M <= nxd::FEW_MAX_ROWS && p.K >= 8 && p.K % 8 == 0 && p.N >= 1 && x.stride(0) < (1 << 24), "linear_few: 1..32 rows, K a multiple of 8");
   TORCH_CHECK(w.is_contiguous() && w.size(1) == p.K && y.size(0) == p.M && y.size(1) == p.N && x.stride(0) % 8 == 0, "linear_few: shapes");
+  TORCH_CHECK(w.numel() < (1LL << 31) - 16 * w.size(1), "linear_few: weights of 4 GB");
   check_align(x, "x");
   check_align(w, "w");
   check_align(y, "y");
   p.x = static_cast<const uint16_t*>(x.data_ptr());
   p.ldx = x.stride(0);
-  p.w = static_cast<const uint16_t*>(w.data_ptr());
-  p.y = static_cast<uint16_t*>(y.data_ptr());
+  p.w = w.data_ptr();
+  p.ldw = p.K;
+  if (epi == nxd::FEW_F32) p.yf = y.data_ptr<float>();
+  else p.y = static_cast<uint16_t*>(y.data_ptr());
   p.ldy = y.stride(0);
-  check_rc(nxd::linear_few_launch(p, cur_stream()), "linear_few");
+  p.alpha = (float)alpha;
+  p.cap = (float)cap;
+  Tensor ws;
+  int need = 0;
+  const int64_t floats = epi == nxd::FEW_STORE && tickets.has_value() ? nxd::few_rows_workspace(p.M, p.N, p.K, &need) : 0;
+  if (floats && tickets->numel() >= need) {
+    TORCH_CHECK(tickets->scalar_type() == at::kInt && tickets->is_cuda() && tickets->is_contiguous(), "linear_few: int32 tickets");
+    ws = at::empty({floats}, x.options().dtype(at::kFloat));
+    p.ws = ws.data_ptr<float>();
+    p.tickets = tickets->data_ptr<int>();
+  }
+  check_rc(nxd::few_rows_launch((int)epi, p, cur_stream()), "linear_few");
 }
 
 }  // namespace
@@ -344,5 +361,6 @@ void register_parallel(pybind11::module& m) {
   m.def("grouped_linear", &grouped_linear);
   m.def("expert_rows", &expert_rows);
   m.def("experts_few", &experts_few);
-  m.def("linear_few", &linear_few);
+  m.def("linear_few", &linear_few, py::arg("x"), py::arg("w"), py::arg("y"), py::arg("epi") = 0, py::arg("alpha") = 1.0,
+        py::arg("cap") = 0.0, py::arg("tickets") = py::none());
 }

@@ -10,10 +10,11 @@
   kernel (inference.hip) reading the KV cache up to a per-sequence DEVICE length, so a decode
   step has static shapes and no host sync — it is captured into hipGraphs (inference/graphs.py).
 
-Decode fast path (TP = 1, bf16 weights, <= 8 new tokens): each projection is one fused GEMV
-(csrc/decode_fused.hip) that also does the surrounding element-wise work -- RMSNorm prologues,
-RoPE + KV-cache write after QKV, residual adds after o_proj / down -- so a layer is 5 launches
-(QKV, attention, o_proj, gate_up, down) instead of 10 (`NXD_DECODE_FUSED=0` disables it).
+Decode fast path (bf16 or int8 weights, <= 32 new tokens; at TP > 1 bf16 and <= 8): each projection is one launch
+(csrc/decode_fused.hip for 1 and 2 rows of bf16 weights, csrc/few_rows.hip otherwise) that also does the
+surrounding element-wise work -- RMSNorm prologues, RoPE + KV-cache write after QKV, residual adds after
+o_proj / down -- so a layer is 5 launches (QKV, attention, o_proj, gate_up, down) instead of 10
+(`NXD_DECODE_FUSED=0` disables it).
 
 KV cache: ONE allocation [layers, 2, max_batch, kv_heads_local, max_len, head_dim] (bf16);
 `seq_ids` selects cache rows (continuous batching).
@@ -54,6 +55,9 @@ _ATTN_OPROJ_MAXB = int(os.environ.get("NXD_DECODE_ATTN_OPROJ_MAXB", "2"))
 # embedding row of each token id and workgroup 0 writes it to the residual stream): one launch less
 # per decode step.  NXD_DECODE_EMB_FUSED=0 keeps the separate embedding kernel (A/B).
 _EMB_FUSED = os.environ.get("NXD_DECODE_EMB_FUSED", "1") == "1"
+# Limits of the matrix-core projections (csrc/few_rows.hip): rows, width of a norm's rows, bytes of a weight matrix; counters for
+# any of its split reductions
+_FEW_ROWS, _FEW_NORM_WIDTH, _FEW_WEIGHT_BYTES, _FEW_TICKETS = 32, 4224, 2 ** 31, 256
 
 
 class DecoderInferenceMixin:
@@ -173,8 +177,8 @@ class DecoderInferenceMixin:
 
     # ------------------------------------------------------------------ fused decode path
     def _fused_ffn_weights(self, layer):
-        """(post-attention norm weight, fused gate/up [2I, H], down [H, I]) when the feed-forward
-        block is a dense bias-free SwiGLU MLP the fused decode kernels can run, else None."""
+        """(post-attention norm weight, modules of the fused gate/up [2I, H] and of down [H, I]) when the
+        feed-forward block is a dense SwiGLU MLP, else None."""
         return None
 
     def _decode_fusable(self, input_ids: torch.Tensor) -> bool:
@@ -182,8 +186,12 @@ class DecoderInferenceMixin:
         if ok is None:
             ok = self._check_decode_fusable()
             self._decode_fused_ok = ok
-        M = input_ids.numel()
-        return ok and input_ids.is_cuda and M <= 8 and M * self.config.hidden_size <= 32768
+        M, H = input_ids.numel(), self.config.hidden_size
+        if not ok or not input_ids.is_cuda or self.tp > 1 and M > 8:
+            return False
+        if self._decode_few_ok and M <= _FEW_ROWS:
+            return True
+        return not self._decode_int8 and M <= 8 and M * H <= 32768
 
     def _check_decode_fusable(self) -> bool:
         if os.environ.get("NXD_DECODE_FUSED", "1") == "0":
@@ -194,16 +202,37 @@ class DecoderInferenceMixin:
             return False
         if self.head_dim % 2 or self.head_dim > 256:
             return False
+        H = self.config.hidden_size
+        mods = [self.lm_head]
         for layer in self.model.layers:
-            attn = layer.self_attn
-            w, b = attn.qkv_proj._fused_weight_bias() if hasattr(attn.qkv_proj, "_fused_weight_bias") \
-                else (attn.qkv_proj.weight, getattr(attn.qkv_proj, "bias", None))
-            if b is not None or w.dtype != torch.bfloat16 or getattr(attn.o_proj, "bias", None) is not None:
+            if self._fused_ffn_weights(layer) is None:
                 return False
-            if attn.o_proj.weight.dtype != torch.bfloat16 or self._fused_ffn_weights(layer) is None:
-                return False
-        lm = self.lm_head.weight
-        return lm.dtype == torch.bfloat16 and getattr(self.lm_head, "bias", None) is None
+            mods += [layer.self_attn.qkv_proj, layer.self_attn.o_proj, *self._fused_ffn_weights(layer)[1:]]
+        if any(self._weight_bias(m)[1] is not None for m in mods):
+            return False
+        weights = [self._weight_bias(m)[0] for m in mods]
+        self._decode_int8 = any(w.dtype == torch.int8 for w in weights)
+        if any(w.dtype not in (torch.bfloat16, torch.int8) for w in weights) or self.model.embed_tokens.weight.dtype != torch.bfloat16:
+            return False
+        # (with int8 weights the fused step is that of the matrix-core projections alone)
+        self._decode_few_ok = (H <= _FEW_NORM_WIDTH and self.head_dim % 32 == 0
+                               and all(w.shape[1] % (16 if w.dtype == torch.int8 else 8) == 0 and w.is_contiguous()
+                                       and w.numel() * w.element_size() < _FEW_WEIGHT_BYTES
+                                       for w in [*weights, self.model.embed_tokens.weight]))
+        return not self._decode_int8 or self._decode_few_ok and self.tp == 1
+
+    @staticmethod
+    def _weight_bias(mod):
+        """(weight, bias) of a projection module, or of a plain weight tensor."""
+        if isinstance(mod, torch.Tensor):
+            return mod, None
+        return mod._fused_weight_bias() if hasattr(mod, "_fused_weight_bias") else (mod.weight, getattr(mod, "bias", None))
+
+    @classmethod
+    def _weight_scale(cls, mod):
+        """(weight, its scale if it is int8) of a projection module."""
+        w = cls._weight_bias(mod)[0]
+        return w, mod._row_scale() if w.dtype == torch.int8 else None
 
     def _decode_oacc(self, M: int, res: torch.Tensor) -> torch.Tensor:
         """fp32 [8, H] o_proj accumulator of the fused attention + o_proj decode launch: zero between
@@ -234,28 +263,32 @@ class DecoderInferenceMixin:
         else:
             res = ops.vocab_parallel_embedding(input_ids, ew, emb.start_index).reshape(M, -1).contiguous()
         qkv = torch.empty((M, W), dtype=res.dtype, device=res.device)
+        # counters with which a long reduction (down) is split over workgroups; one launch clears them for all layers
+        tickets = torch.zeros(_FEW_TICKETS, dtype=torch.int32, device=res.device) if 8 < M <= _FEW_ROWS else None
         for i, layer in enumerate(self.model.layers):
             attn = layer.self_attn
-            w_qkv = attn.qkv_proj._fused_weight_bias()[0] if hasattr(attn.qkv_proj, "_fused_weight_bias") \
-                else attn.qkv_proj.weight
+            w_qkv, s_qkv = self._weight_scale(attn.qkv_proj)
+            w_o, s_o = self._weight_scale(attn.o_proj)
             kc, vc = self.kv_cache[i, 0], self.kv_cache[i, 1]
             # RMSNorm -> QKV -> RoPE -> k/v into the cache, one launch (layer 0: + the embedding gather)
             if i == 0 and emb_fused:
                 C.dgemv(3, ew, layer.input_layernorm.weight, self.eps, w_qkv, qkv, nq, nkv, D, cos_t, sin_t, pos, T,
-                        kc, vc, sid32, xidx=ids, xcopy=res)
+                        kc, vc, sid32, xidx=ids, xcopy=res, wscale=s_qkv)
             else:
                 C.dgemv(3, res, layer.input_layernorm.weight, self.eps, w_qkv, qkv, nq, nkv, D, cos_t, sin_t, pos, T,
-                        kc, vc, sid32)
+                        kc, vc, sid32, wscale=s_qkv)
             q = qkv.view(B, T, nq + 2 * nkv, D)[:, :, :nq]
-            ln2, w_gu, w_d = self._fused_ffn_weights(layer)
+            ln2, gate_up, down = self._fused_ffn_weights(layer)
+            (w_gu, s_gu), (w_d, s_d) = self._weight_scale(gate_up), self._weight_scale(down)
             if _PREFETCH_MB > 0:
                 # spare workgroups of the attention launch pull o_proj and the head of gate_up into
                 # the Infinity Cache while the (latency-bound) attention leaves HBM idle
-                C.decode_attn_prefetch(attn.o_proj.weight, -1, w_gu, int(_PREFETCH_MB * 2**20), _PREFETCH_WGS)
-            fuse_o = (_ATTN_OPROJ and _PREFETCH_MB <= 0 and B <= _ATTN_OPROJ_MAXB
+                C.decode_attn_prefetch(w_o, -1, w_gu, int(_PREFETCH_MB * 2**20), _PREFETCH_WGS)
+            # (from 3 rows on the projections without the pending sum are the faster ones)
+            fuse_o = (_ATTN_OPROJ and _PREFETCH_MB <= 0 and B <= _ATTN_OPROJ_MAXB and M <= 2 and not self._decode_int8
                       and not getattr(self, "_decode_deterministic", False))
             oacc = self._decode_oacc(M, res) if fuse_o else None
-            if oacc is not None and C.decode_attn_oproj(q, kc, vc, sid32, cache_len.to(torch.int32), attn.o_proj.weight,
+            if oacc is not None and C.decode_attn_oproj(q, kc, vc, sid32, cache_len.to(torch.int32), w_o,
                                                         oacc, 1.0 / math.sqrt(D)):
                 # oacc += o_proj(attention) (one launch); the GLU prologue sees res + oacc, the down
                 # epilogue folds it into res with the unfused rounding and zeroes it
@@ -264,18 +297,20 @@ class DecoderInferenceMixin:
                 C.dgemv(1, a, None, 0.0, w_d, res, 0, 0, 0, None, None, None, 1, None, None, None, None, oacc)
                 continue
             o = ops.decode_attention(q, kc, vc, cache_len, sid32)
-            C.dgemv(1, o.reshape(M, nq * D), None, 0.0, attn.o_proj.weight, res, 0, 0, 0, None, None, None, 1,
-                    None, None, None)                                   # res += o_proj(o)
+            C.dgemv(1, o.reshape(M, nq * D), None, 0.0, w_o, res, 0, 0, 0, None, None, None, 1,
+                    None, None, None, wscale=s_o, tickets=tickets)              # res += o_proj(o)
             a = torch.empty((M, w_d.shape[1]), dtype=res.dtype, device=res.device)
-            C.dgemv(2, res, ln2, self.eps, w_gu, a, 0, 0, 0, None, None, None, 1, None, None, None)  # norm+SwiGLU
-            C.dgemv(1, a, None, 0.0, w_d, res, 0, 0, 0, None, None, None, 1, None, None, None)   # res += down(a)
+            C.dgemv(2, res, ln2, self.eps, w_gu, a, 0, 0, 0, None, None, None, 1, None, None, None, wscale=s_gu)  # norm+SwiGLU
+            C.dgemv(1, a, None, 0.0, w_d, res, 0, 0, 0, None, None, None, 1, None, None, None, wscale=s_d,
+                    tickets=tickets)                                            # res += down(a)
         h = res.view(B, T, -1)
         if last_index is not None:
             h = h[torch.arange(B, device=h.device), last_index]
         h2 = h.reshape(-1, h.shape[-1]).contiguous()
-        logits = torch.empty((h2.shape[0], self.lm_head.weight.shape[0]), dtype=res.dtype, device=res.device)
-        C.dgemv(0, h2, self.model.norm.weight, self.eps, self.lm_head.weight, logits, 0, 0, 0, None, None, None, 1,
-                None, None, None)                                       # final norm + lm_head
+        w_lm, s_lm = self._weight_scale(self.lm_head)
+        logits = torch.empty((h2.shape[0], w_lm.shape[0]), dtype=res.dtype, device=res.device)
+        C.dgemv(0, h2, self.model.norm.weight, self.eps, w_lm, logits, 0, 0, 0, None, None, None, 1,
+                None, None, None, wscale=s_lm)                          # final norm + lm_head
         logits = logits.view(h.shape[:-1] + (logits.shape[-1],))
         if return_hidden:
             return logits, ops.rms_norm(h, self.model.norm.weight, self.eps)[0]
@@ -364,7 +399,8 @@ class DecoderInferenceMixin:
             C.dgemv(3, res, layer.input_layernorm.weight, self.eps, w_qkv, qkv, nq, nkv, D, cos_t, sin_t, pos, T,
                     kc, vc, sid32)
             q = qkv.view(B, T, nq + 2 * nkv, D)[:, :, :nq]
-            ln2, w_gu, w_d = self._fused_ffn_weights(layer)
+            ln2, gate_up, down = self._fused_ffn_weights(layer)
+            w_gu, w_d = self._weight_bias(gate_up)[0], self._weight_bias(down)[0]
             if not (fuse_o and C.decode_attn_oproj(q, kc, vc, sid32, clen32, attn.o_proj.weight, oacc, 1.0 / math.sqrt(D))):
                 o = ops.decode_attention(q, kc, vc, cache_len, sid32)
                 C.dgemv(0, o.reshape(M, nq * D), None, 0.0, attn.o_proj.weight, oacc[:M], 0, 0, 0, None, None, None, 1,
@@ -460,7 +496,7 @@ class DecoderInferenceMixin:
             b = None
         scale = mod._row_scale() if w.dtype == torch.int8 else None
         M = x.numel() // x.shape[-1]
-        if w.dtype == torch.int8 or (M <= 8 and x.is_cuda):
+        if w.dtype == torch.int8 or (x.is_cuda and (M <= 8 or M <= _FEW_ROWS and x.dtype == w.dtype == torch.bfloat16 and b is None)):
             return skinny_linear(x, w, scale, b, glu=glu)
         from ..trace.weight_layout import packed_linear
 

@@ -18,7 +18,7 @@ import torch.nn as nn
 from .. import ops
 from ..models.bezurax import BezuraxConfig
 from ..modules.hybrid import ChannelDelta, ParallelMixer, PooledAttention, RoutedExperts, StepContext
-from ..modules.hybrid.context import few_rows, small
+from ..modules.hybrid.context import SOME_ROWS, few_rows, small, step_tickets
 from ..ops.experts import RouterRule
 from ..ops.gemm import linear_f32
 from ..parallel_layers.parallel_state import get_tensor_model_parallel_size
@@ -120,6 +120,8 @@ class BezuraxInferenceModel(DecoderInferenceMixin, nn.Module):
                           lengths.to(torch.int32) if lengths is not None else None,
                           seq_ids.to(torch.int32) if seq_ids is not None else None, prefill,
                           self._decode_fused_ok is not False and input_ids.is_cuda)
+        if ctx.fused:
+            ctx.tickets = step_tickets(B * T, input_ids.device)
         emb = self.model.embed_tokens.weight
         if logit_rows is None and last_index is not None:
             logit_rows = torch.arange(B, device=input_ids.device) * T + last_index
@@ -137,6 +139,8 @@ class BezuraxInferenceModel(DecoderInferenceMixin, nn.Module):
         w, scale = self.lm_head.weight, self.config.logit_scale
         if ctx.fused and few_rows(h, w):
             logits = ops.decode_linear(w, h, epilogue="f32", alpha=scale)
+        elif ctx.fused and few_rows(h, w, SOME_ROWS) and w.numel() < 2 ** 30:
+            logits = ops.linear_few(h, w, "f32", alpha=scale)
         else:
             logits = linear_f32(h, w, scale)
         if logit_rows is None:

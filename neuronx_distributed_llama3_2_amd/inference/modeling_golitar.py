@@ -20,7 +20,7 @@ from .. import ops
 from ..models.golitar import GolitarConfig
 from ..modules.hybrid import (DifferentialAttentionMixer, GatedDeltaMixer, HyperConnection, SquaredReluMLP,
                               StepContext)
-from ..modules.hybrid.context import small
+from ..modules.hybrid.context import SOME_ROWS, few_rows, small, step_tickets
 from ..ops.gemm import linear_f32
 from ..ops.hyper import FUSED_NORM_ELEMENTS, FUSED_ROWS
 from ..parallel_layers.parallel_state import get_tensor_model_parallel_size
@@ -151,6 +151,8 @@ class GolitarInferenceModel(DecoderInferenceMixin, nn.Module):
                           lengths.to(torch.int32) if lengths is not None else None,
                           seq_ids.to(torch.int32) if seq_ids is not None else None, prefill,
                           self._fused(input_ids))
+        if ctx.fused:
+            ctx.tickets = step_tickets(B * T, input_ids.device)
         emb = self.model.embed_tokens.weight
         M, dt = B * T, emb.dtype
         if logit_rows is None and last_index is not None:
@@ -165,7 +167,7 @@ class GolitarInferenceModel(DecoderInferenceMixin, nn.Module):
             last = dict(y=y, y_bias=mod.o_bias, mix=hc.mix, write=hc.write)
         h = ops.hyper_step(streams, read=self._ones(emb.device), norm_w=self.model.norm.weight, eps=self.eps, dtype=dt,
                            rows=logit_rows, store=False, **last)
-        logits = self._logits(h)
+        logits = self._logits(h, ctx.fused)
         if logit_rows is None:
             logits, h = logits.view(B, T, -1), h.view(B, T, -1)
         return (logits, h) if return_hidden else logits
@@ -198,7 +200,9 @@ class GolitarInferenceModel(DecoderInferenceMixin, nn.Module):
             self._ones_buf = torch.ones(self.config.streams, dtype=torch.float32, device=device)
         return self._ones_buf
 
-    def _logits(self, h: torch.Tensor) -> torch.Tensor:
+    def _logits(self, h: torch.Tensor, fused: bool = False) -> torch.Tensor:
+        if fused and few_rows(h, self.lm_head.weight, SOME_ROWS) and self.lm_head.weight.numel() < 2 ** 30:
+            return ops.linear_few(h, self.lm_head.weight, "f32", cap=self.config.logit_softcap)
         logits = linear_f32(h, self.lm_head.weight)
         return ops.softcap_(logits, self.config.logit_softcap) if self.config.logit_softcap > 0 else logits
 

@@ -21,6 +21,7 @@ class StepContext:
     slots: Optional[torch.Tensor]
     prompt: bool
     fused: bool = True
+    tickets: Optional[torch.Tensor] = None   # of ops.linear_few, for steps of few rows
 
 
 # rows of a fused projection are padded to this, so that every row of its output is 16-byte aligned
@@ -32,23 +33,36 @@ def padded_rows(n: int) -> int:
 
 
 # rows up to which a projection is a dot product a wave (csrc/hybrid/gemv_hyper.hip), and up to which it is
-# 16 weight rows a workgroup (csrc/hybrid/expert_decode.hip)
-FEW_ROWS, SOME_ROWS = 2, 16
+# a matrix-core product that streams the weights (csrc/few_rows.hip)
+FEW_ROWS, SOME_ROWS = 2, 32
 
 
 def few_rows(x: torch.Tensor, w: torch.Tensor, limit: int = FEW_ROWS) -> bool:
     return x.is_cuda and x.shape[0] <= limit and x.dtype == w.dtype == torch.bfloat16 and w.shape[1] % 8 == 0 and x.is_contiguous()
 
 
-def linear(x: torch.Tensor, mod: torch.nn.Module, fused: bool = False) -> torch.Tensor:
+def linear(x: torch.Tensor, mod: torch.nn.Module, fused: bool = False, epilogue: str = "store",
+           tickets: Optional[torch.Tensor] = None) -> torch.Tensor:
     """x [M, K] @ mod.weight^T: through the module's packed copy when the layout pass chose it; fused: a few
-    rows by the kernels that stream the weights."""
+    rows by the kernels that stream the weights.  epilogue "relu2": its squared ReLU."""
     from ... import ops
     from ...trace.weight_layout import packed_linear
 
-    if fused and few_rows(x, mod.weight, SOME_ROWS):
-        return ops.decode_linear(mod.weight, x) if x.shape[0] <= FEW_ROWS else ops.linear_few(x, mod.weight)
-    return packed_linear(mod, x, mod.weight)
+    if fused and few_rows(x, mod.weight, SOME_ROWS) and mod.weight.numel() < 2 ** 30:
+        if x.shape[0] <= FEW_ROWS:
+            return ops.decode_linear(mod.weight, x, epilogue=epilogue)
+        return ops.linear_few(x, mod.weight, epilogue, tickets=tickets)
+    y = packed_linear(mod, x, mod.weight)
+    return ops.relu_squared(y) if epilogue == "relu2" else y
+
+
+def step_tickets(rows: int, device) -> Optional[torch.Tensor]:
+    """Zeroed counters for the projections of a step of so many rows."""
+    from ...ops.experts import LINEAR_TICKETS
+
+    if torch.device(device).type != "cuda" or not FEW_ROWS < rows <= SOME_ROWS:
+        return None
+    return torch.zeros(LINEAR_TICKETS, dtype=torch.int32, device=device)
 
 
 def small(*shape, device=None) -> torch.nn.Parameter:

@@ -112,4 +112,4 @@ class DifferentialAttentionMixer(nn.Module):
                                     cache["k"], cache["v"], ctx.prompt, ctx.fused)
 
     def forward(self, h: torch.Tensor, cache: Dict[str, torch.Tensor], ctx: StepContext) -> torch.Tensor:
-        return linear(self.core(linear(h, self.qkv_proj), cache, ctx), self.o_proj)
+        return linear(self.core(linear(h, self.qkv_proj, ctx.fused), cache, ctx), self.o_proj, ctx.fused, tickets=ctx.tickets)

@@ -59,4 +59,4 @@ class GatedDeltaMixer(nn.Module):
                               self.eps, ctx.positions, ctx.lengths, ctx.slots, cache["state"], cache["ring"], ctx.fused)
 
     def forward(self, h: torch.Tensor, cache: Dict[str, torch.Tensor], ctx: StepContext) -> torch.Tensor:
-        return linear(self.core(linear(h, self.in_proj), cache, ctx), self.o_proj)
+        return linear(self.core(linear(h, self.in_proj, ctx.fused), cache, ctx), self.o_proj, ctx.fused, tickets=ctx.tickets)

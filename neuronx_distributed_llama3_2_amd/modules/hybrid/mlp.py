@@ -5,7 +5,6 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 
-from ... import ops
 from .context import linear
 
 
@@ -30,4 +29,6 @@ class SquaredReluMLP(nn.Module):
         return a
 
     def forward(self, h: torch.Tensor, cache=None, ctx=None) -> torch.Tensor:
-        return linear(ops.relu_squared(linear(h, self.up_proj)), self.down_proj)
+        fused = ctx is not None and ctx.fused
+        tickets = ctx.tickets if ctx is not None else None
+        return linear(linear(h, self.up_proj, fused, "relu2"), self.down_proj, fused, tickets=tickets)

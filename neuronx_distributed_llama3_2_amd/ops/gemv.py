@@ -1,5 +1,5 @@
-"""Decode-path linear ops (csrc/gemv.hip): skinny GEMM for M <= 8 tokens with bf16 or int8 weights,
-optional per-row / per-tensor scale, bias and fused SwiGLU epilogue; int8 -> bf16 dequantisation
+"""Decode-path linear ops (csrc/few_rows.hip, gemv.hip): skinny GEMM for M <= 32 tokens (8 with a bias) with bf16 or int8
+weights, optional per-row / per-tensor scale, bias and fused SwiGLU epilogue; int8 -> bf16 dequantisation
 for the prefill path.  CPU / large-M calls fall back to dequantise + GEMM."""
 
 from __future__ import annotations
@@ -42,7 +42,8 @@ def skinny_linear(x: torch.Tensor, w: torch.Tensor, scale: Optional[torch.Tensor
     M = x.numel() // K
     Nw = w.shape[0]
     N = Nw // 2 if glu else Nw
-    if use_native(x, w) and M <= 8 and x.dtype == torch.bfloat16 and w.stride(-1) == 1:
+    few = bias is None and w.numel() * w.element_size() < 2 ** 31   # csrc/few_rows.hip takes up to 32 rows of these
+    if use_native(x, w) and M <= (32 if few else 8) and x.dtype == torch.bfloat16 and w.stride(-1) == 1:
         x2 = x.reshape(M, K)
         if x2.stride(0) % 8 or x2.data_ptr() % 16:
             x2 = x2.contiguous()

@@ -1,0 +1,146 @@
+"""Products of 1 to 32 rows (csrc/few_rows.hip) against 64-bit references: edges of the tiles of rows, weight rows and
+reduction chunks, every geometry of the dispatch, both weight types and all epilogues.
+
+Tolerance: outputs and x times the norm's weight are rounded to bf16 (relative error of at most 2^-9 each, 2^-9 / sqrt(3)
+on average), sums are fp32: 2-norm within 3 x 2^-9 of the reference; the rotary epilogue rounds twice."""
+
+import pytest
+import torch
+
+from neuronx_distributed_llama3_2_amd import ops
+
+pytestmark = pytest.mark.gpu
+TOL = 3 * 2 ** -9
+EPS = 1e-5
+
+
+def _weights(N, K, int8, gen):
+    if int8:
+        return (torch.randint(-128, 128, (N, K), generator=gen, device="cuda", dtype=torch.int8),
+                torch.rand(N, generator=gen, device="cuda") * 3e-4 + 1e-5)
+    return (torch.randn(N, K, generator=gen, device="cuda") * 0.02).bfloat16(), None
+
+
+def _exact(x, norm, w, scale):
+    x = x.double()
+    if norm is not None:
+        x = x * torch.rsqrt(x.square().mean(-1, keepdim=True) + EPS) * norm.double()
+    return x @ (w.double() if scale is None else w.double() * scale.double()[:, None]).t()
+
+
+def _close(got, want, tol=TOL):
+    assert float((got.double() - want).norm() / want.norm()) < tol
+
+
+SHAPES = [(1, 64, 128), (3, 40, 8), (3, 100, 136), (16, 1000, 2048), (17, 3072, 2048), (32, 4112, 2048), (5, 2048, 2048),
+          (32, 6144, 4096), (13, 4096, 4096), (29, 40, 4224), (16, 4096, 1920)]
+LONG = [(4, 2048, 8192), (9, 2048, 8192), (32, 100, 5000), (13, 4096, 14336), (17, 4096, 4352), (16, 33, 4240)]
+
+
+@pytest.mark.parametrize("int8", [False, True])
+@pytest.mark.parametrize("M,N,K", SHAPES + LONG)
+def test_store_and_residual(M, N, K, int8):
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+    if int8 and K % 16:
+        K += 8
+    w, s = _weights(N, K, int8, gen)
+    M = M if int8 else max(M, 3)
+    x = torch.randn(M, K, generator=gen, device="cuda").bfloat16()
+    y0 = torch.randn(M, N, generator=gen, device="cuda").bfloat16()
+    want = _exact(x, None, w, s)
+    C = ops.ext()
+    tickets = torch.zeros(256, dtype=torch.int32, device="cuda")
+    outs = []
+    for _ in range(2):   # (the counters are left as they were, and the order of the sums does not change)
+        y = y0.clone()
+        C.dgemv(1, x, None, 0.0, w, y, 0, 0, 0, None, None, None, 1, None, None, None, wscale=s, tickets=tickets)
+        outs.append(y)
+    _close(outs[0], y0.double() + want)
+    assert torch.equal(outs[0], outs[1]) and not tickets.any()
+    y = torch.empty_like(y0)
+    C.dgemv(0, x, None, 0.0, w, y, 0, 0, 0, None, None, None, 1, None, None, None, wscale=s)
+    _close(y, want)
+    if not int8:
+        yf = torch.empty(M, N, device="cuda")
+        C.dgemv(0, x, None, 0.0, w, yf, 0, 0, 0, None, None, None, 1, None, None, None)
+        _close(yf, want, 1e-5)
+
+
+@pytest.mark.parametrize("int8", [False, True])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_norm_and_swiglu(M, N, K, int8):
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K + 1)
+    if int8 and K % 16:
+        K += 8
+    M = M if int8 else max(M, 3)
+    w, s = _weights(2 * N, K, int8, gen)
+    x = (torch.randn(M, K, generator=gen, device="cuda") * 3).bfloat16()
+    g = (1 + 0.1 * torch.randn(K, generator=gen, device="cuda")).bfloat16()
+    z = _exact(x, g, w, s)
+    C = ops.ext()
+    y = torch.empty(M, 2 * N, dtype=torch.bfloat16, device="cuda")
+    C.dgemv(0, x, g, EPS, w, y, 0, 0, 0, None, None, None, 1, None, None, None, wscale=s)
+    _close(y, z)
+    y = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    C.dgemv(2, x, g, EPS, w, y, 0, 0, 0, None, None, None, 1, None, None, None, wscale=s)
+    _close(y, torch.nn.functional.silu(z[:, :N]) * z[:, N:])
+
+
+@pytest.mark.parametrize("M,T,nq,nkv,D,H,int8,table", [(3, 1, 4, 2, 64, 512, False, True), (8, 2, 8, 2, 64, 2048, False, False),
+                                                       (32, 1, 32, 8, 64, 2048, False, True), (18, 3, 8, 8, 128, 4096, False, True),
+                                                       (6, 1, 6, 2, 32, 144, True, False), (20, 4, 48, 8, 128, 4096, True, True)])
+def test_qkv_rope_cache(M, T, nq, nkv, D, H, int8, table):
+    gen = torch.Generator(device="cuda").manual_seed(M * D)
+    N, Lmax, B = (nq + 2 * nkv) * D, 64, M // T
+    w, s = _weights(N, H, int8, gen)
+    g = (1 + 0.1 * torch.randn(H, generator=gen, device="cuda")).bfloat16()
+    rows = torch.randn(50, H, generator=gen, device="cuda").bfloat16()
+    ids = torch.randint(0, 50, (M,), generator=gen, device="cuda")
+    pos = torch.arange(M, device="cuda") * 5 % (Lmax + 9)   # (some past the cache's end: not written)
+    if table:
+        ids[0] = -1                                         # (not a row of the table: zeros)
+    x = rows[ids.clamp(min=0)] * (ids >= 0)[:, None]
+    ang = torch.rand(Lmax + 9, D // 2, generator=gen, device="cuda") * 6
+    cos, sin = ang.cos(), ang.sin()
+    idx = torch.randperm(B, generator=gen, device="cuda").to(torch.int32)
+    kc, vc = (torch.zeros(B, nkv, Lmax, D, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    y, copy = torch.empty(M, N, dtype=torch.bfloat16, device="cuda"), torch.full((M, H), 7.0, device="cuda").bfloat16()
+    kw = dict(xidx=ids, xcopy=copy) if table else {}
+    ops.ext().dgemv(3, rows if table else x.contiguous(), g, EPS, w, y, nq, nkv, D, cos, sin, pos, T, kc, vc, idx, wscale=s, **kw)
+    if table:
+        assert torch.equal(copy, x)
+    z = _exact(x, g, w, s).view(M, nq + 2 * nkv, D)
+    c, si = cos[pos].double()[:, None], sin[pos].double()[:, None]
+    a, b = z[:, :nq + nkv].chunk(2, -1)
+    want = torch.cat([torch.cat([a * c - b * si, b * c + a * si], -1), z[:, nq + nkv:]], 1)
+    _close(y.view(M, -1, D), want, 2 * TOL)
+    for m in range(M):
+        if pos[m] < Lmax:
+            slot = int(idx[m // T])
+            assert torch.equal(kc[slot, :, pos[m]], y.view(M, -1, D)[m, nq:nq + nkv])
+            assert torch.equal(vc[slot, :, pos[m]], y.view(M, -1, D)[m, nq + nkv:])
+
+
+@pytest.mark.parametrize("M,N,K", [(3, 48, 64), (16, 12288, 2048), (32, 2064, 1024), (17, 2048, 12288)])
+def test_linear_few_epilogues(M, N, K):
+    gen = torch.Generator(device="cuda").manual_seed(M + N)
+    w, _ = _weights(N, K, False, gen)
+    x = torch.randn(M, K, generator=gen, device="cuda").bfloat16()
+    z = _exact(x, None, w, None)
+    tickets = torch.zeros(ops.experts.LINEAR_TICKETS, dtype=torch.int32, device="cuda")
+    _close(ops.linear_few(x, w, tickets=tickets), z)
+    assert not tickets.any()
+    _close(ops.linear_few(x, w, "relu2"), z.clamp(min=0).square())
+    _close(ops.linear_few(x, w, "f32", alpha=0.5), 0.5 * z, 1e-5)
+    _close(ops.linear_few(x, w, "f32", alpha=0.5, cap=0.3), 0.3 * torch.tanh(0.5 * z / 0.3), 1e-5)
+
+
+def test_rows_of_a_view_and_unaligned_outputs():
+    """Inputs between other columns; outputs whose rows start at odd places."""
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    w, _ = _weights(51, 256, False, gen)
+    x = torch.randn(7, 512, generator=gen, device="cuda").bfloat16()[:, 128:384]
+    y = torch.zeros(7, 53, dtype=torch.bfloat16, device="cuda")
+    ops.ext().dgemv(0, x, None, 0.0, w, y[:, 1:52], 0, 0, 0, None, None, None, 1, None, None, None)
+    _close(y[:, 1:52], _exact(x, None, w, None))
+    assert not y[:, 0].any() and not y[:, 52].any()
