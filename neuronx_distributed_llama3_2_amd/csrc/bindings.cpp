@@ -48,7 +48,7 @@ int scale_flat_launch(float*, int64_t, const float*, hipStream_t);
 int embedding_fwd_launch(const int64_t*, const void*, void*, int64_t, int, int64_t, int64_t, hipStream_t);
 int embedding_bwd_launch(const int64_t*, const void*, float*, int64_t, int, int64_t, int64_t, hipStream_t);
 int decode_attn_launch(const void*, const int64_t*, const void*, const void*, const int64_t*, const int*, const int*,
-                       float*, float*, float*, int*, void*, const int64_t*, int, int, int, int, int, int, float, hipStream_t);
+                       float*, float*, float*, int*, void*, const int64_t*, int, int, int, int, int, int, float, hipStream_t, int*);
 int kv_cache_write_launch(const void*, const void*, const int64_t*, void*, void*, const int64_t*, const int*, const int*,
                           int, int, int, int, int, hipStream_t);
 int argmax_launch(const void*, int, int64_t, int, int, int64_t*, hipStream_t);
@@ -537,7 +537,7 @@ bool decode_attn_oproj(at::Tensor q, at::Tensor kc, at::Tensor vc, c10::optional
 }
 
 void decode_attn(at::Tensor q, at::Tensor kc, at::Tensor vc, c10::optional<at::Tensor> cache_idx, at::Tensor seq_len,
-                 at::Tensor out, double scale, int64_t nsplit) {
+                 at::Tensor out, double scale, int64_t nsplit, c10::optional<at::Tensor> tickets) {
   int64_t qs[3], os[3];
   bshd_strides(q, "q", qs);
   bshd_strides(out, "out", os);
@@ -569,9 +569,15 @@ void decode_attn(at::Tensor q, at::Tensor kc, at::Tensor vc, c10::optional<at::T
   (void)Lmax;
   TORCH_CHECK(os[2] % 8 == 0 || Hq == 1, "out head stride must keep 16-byte alignment");
   int* counters = decode_counters(q.device().index(), (int64_t)B * Hkv);
+  int* tk = nullptr;
+  if (tickets.has_value()) {
+    TORCH_CHECK(tickets->is_cuda() && tickets->scalar_type() == at::kInt && tickets->is_contiguous() && tickets->numel() >= (int64_t)B * Hkv,
+                "decode_attn: int32 tickets [>= B * Hkv]");
+    tk = tickets->data_ptr<int>();
+  }
   check_rc(nxd::decode_attn_launch(q.data_ptr(), qs, kc.data_ptr(), vc.data_ptr(), cs, ci, seq_len.data_ptr<int>(),
                                    po.data_ptr<float>(), pm.data_ptr<float>(), pl.data_ptr<float>(), counters, out.data_ptr(),
-                                   os, B, T, Hq, Hkv, D, (int)nsplit, (float)scale, cur_stream()),
+                                   os, B, T, Hq, Hkv, D, (int)nsplit, (float)scale, cur_stream(), tk),
            "decode_attn");
   nxd::decode_attn_set_prefetch(nullptr, 0, nullptr, 0, 0);   // armed ranges never outlive one call
 }
@@ -1237,7 +1243,8 @@ PYBIND11_MODULE(_C, m) {
   m.def("scale_flat", &scale_flat);
   m.def("embedding_fwd", &embedding_fwd);
   m.def("embedding_bwd", &embedding_bwd);
-  m.def("decode_attn", &decode_attn);
+  m.def("decode_attn", &decode_attn, py::arg("q"), py::arg("k_cache"), py::arg("v_cache"), py::arg("cache_idx"), py::arg("seq_len"),
+        py::arg("out"), py::arg("scale"), py::arg("nsplit"), py::arg("tickets") = py::none());
   m.def("decode_attn_oproj", &decode_attn_oproj);
   m.def("decode_attn_sync_error", [](bool reset) { return nxd::decode_attn_sync_error(reset); }, py::arg("reset") = false);
   m.def("decode_attn_set_sync", [](int64_t v) { nxd::decode_attn_set_sync((int)v); });

@@ -1,7 +1,7 @@
 // Decode attention on MFMA for small query groups (M = (Hq/Hkv) * T <= 16 rows per kv head):
-// one workgroup (8 waves at D 64, 4 at D 128) owns a (batch, kv head, key split); the keys per split
-// (128-1,024, keys_per_split) are sized so the grid reaches ~128 workgroups; every wave runs an
-// online-softmax flash-decoding loop over 64-key chunks entirely in registers:
+// one workgroup of 4 waves (FUSE: 8 at D 64) owns a (batch, kv head, key split); the keys per split
+// (128-1,024, keys_per_split) are sized so the grid reaches ~512 workgroups; every wave runs an
+// online-softmax flash-decoding loop over 32-key chunks (FUSE: 64) entirely in registers:
 //
 //   S^T[key][m] = K.Q^T   v_mfma_f32_16x16x32_bf16, K rows straight from the cache (16-B loads),
 //                         Q^T fragments held for the whole loop (rows >= M are zero);
@@ -11,8 +11,8 @@
 //                         through a per-wave LDS tile and read transposed (ds_read_b64_tr_b16);
 //
 // then the waves merge their (max, sum, O) through LDS once.  With one split the workgroup writes
-// the final bf16 output; otherwise it writes the (m, l, o) partials that inference.hip's merge kernel
-// -- or, fused with o_proj, merge_oproj_kernel below -- combines.  Compared with the 128-key-chunk
+// the final bf16 output; otherwise it writes the (m, l, o) partials that the last split of the head to
+// finish (with tickets), inference.hip's merge kernel or, fused with o_proj, merge_oproj_kernel below combines.  Compared with the 128-key-chunk
 // kernel there (four workgroup barriers per chunk and a merge launch at every length) this is one
 // barrier per call.
 //
@@ -33,8 +33,8 @@
 namespace nxd {
 namespace dattn {
 
-constexpr int KB = 64;            // keys per chunk (one wave)
-constexpr int KPS = 1024;         // most keys per workgroup split (one pass of 8 waves x 2 chunks)
+constexpr int KB = 64;            // keys per chunk of a wave with FUSE; splits are multiples of it
+constexpr int KPS = 1024;         // most keys per workgroup split
 
 struct Params {
   const uint16_t* q;
@@ -74,6 +74,9 @@ struct Params {
   unsigned* sync_cnt;
   int* sync_err;
   float* mo;          // SYNC: [B * Hkv, M, D] merged attention rows (the merger's hand-off)
+  // key splits without FUSE: zeroed counters [B * Hkv] (left zeroed) with which the last split of a head to finish
+  // merges them; null: a launch of its own does
+  int* tickets;
 };
 static_assert(std::is_trivially_copyable<Params>::value && sizeof(Params) <= 4096, "kernel-argument struct");
 
@@ -156,18 +159,37 @@ __device__ __forceinline__ void oproj_tail(const Params& p, const float* of, con
 // 17.9 with every workgroup merging all partials itself -- vs 5.7 + 5.6 us; 0.759 vs 0.686
 // ms/token; profiles/r6_decode/sync_ab.txt): the in-launch wait on the slowest split of a head costs
 // more than a kernel boundary, so it is off by default (NXD_DECODE_ATTN_SYNC=1).
+//
+// Without FUSE the keys and values of a step are read once and the time is their way from memory plus what comes before
+// and after it.  Measured per layer, before -> now (before: 8 waves at D 64, chunks of 64 keys, splits next to each other in
+// the grid, a merge launch of 4.2 us):
+//   4 sequences of 350-700 keys, 8 heads of 64       10.2 ->  7.6 us
+//   6 of 512-1,024, 8 of 64                          12.0 ->  8.8
+//   13 of 750-1,500, 8 of 128                        25.6 -> 19.5
+//   32 of 1,024-2,048, 8 of 64 (100 MB)              32.2 -> 24.2 (4.2 TB/s; the loads alone 23.5)
+// - chunks of 32 keys leave the registers for two to three workgroups a CU, so that one computes while the other's keys
+//   are on their way (64 keys at D 128: one workgroup, 22.5 us instead of 18.5 at the same splits);
+// - the first splits of all heads come first in the grid and the last, short or empty ones last: neighbours go to
+//   different XCDs, and with an even number of splits next to each other half of the XCDs had the long ones;
+// - values are read non-temporally (24.2 instead of 27.2 us at the largest), keys are not: a wave's read of 16 half lines
+//   needs the cache for the other halves;
+// - the sums of the waves lie over their V tiles, and the last split merges with 8 splits' sums in flight (one trip to
+//   memory where weights first, sums then were two: 1 us).
 template <int D, int NWV, bool FUSE, bool WO_LATE = true, bool SYNC = false>
 __global__ void __launch_bounds__(64 * NWV) attn_kernel(Params p) {
   static_assert(!SYNC || FUSE, "SYNC is a FUSE form");
   constexpr int NS = D / 32;      // k-steps of the score MFMA
   constexpr int NDT = D / 16;     // 16-wide d tiles of the output
-  constexpr int VL = D / 8;       // 16-B V loads per lane for 64 keys x D
+  constexpr int KC = FUSE ? KB : 32;   // keys of a wave's chunk
+  constexpr int KT = KC / 16;
+  constexpr int VL = KC * D / 512;   // 16-B V loads per lane
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const int mi = lane & 15, g = lane >> 4;
-  uint16_t* vt = reinterpret_cast<uint16_t*>(smem) + wid * KB * D;              // this wave's V tile [64][D]
-  float* red_o = reinterpret_cast<float*>(smem + NWV * KB * D * 2);             // [NWV][16][D]
-  float* red_m = red_o + NWV * 16 * D;                                          // [NWV][16]
+  uint16_t* vt = reinterpret_cast<uint16_t*>(smem) + wid * KC * D;              // this wave's V tile [KC][D]
+  constexpr int RED = FUSE ? 16 * D : KC * D / 2;                               // floats from a wave's sums to the next one's
+  float* red_o = reinterpret_cast<float*>(smem + (FUSE ? NWV * KC * D * 2 : 0));   // [NWV][16][D], or over the V tiles
+  float* red_m = reinterpret_cast<float*>(smem + NWV * KC * D * 2) + (FUSE ? NWV * 16 * D : 0);   // [NWV][16]
   float* red_l = red_m + NWV * 16;
 
   if (!FUSE && (int)blockIdx.x >= p.attn_wgs) {
@@ -175,8 +197,9 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(Params p) {
     return;
   }
   if (p.trace != nullptr && tid == 0) p.trace[2 * blockIdx.x] = __builtin_amdgcn_s_memrealtime();
-  const int split = FUSE ? (SYNC ? (int)blockIdx.x % p.R : 0) : (int)blockIdx.x % p.nsplit;
-  const int bh = FUSE ? (int)blockIdx.x / p.R : (int)blockIdx.x / p.nsplit;
+  const int heads = p.B * p.Hkv;
+  const int split = FUSE ? (SYNC ? (int)blockIdx.x % p.R : 0) : (int)blockIdx.x / heads;
+  const int bh = FUSE ? (int)blockIdx.x / p.R : (int)blockIdx.x % heads;
   const int b = bh / p.Hkv, hkv = bh % p.Hkv;
   const int G = p.Hq / p.Hkv, M = G * p.T;
   // FUSE: this workgroup's Wo block (rows rc * NR .., columns of head group hkv) into registers,
@@ -191,6 +214,9 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(Params p) {
   if constexpr (FUSE && !WO_LATE) load_wo();   // round-3 order (A/B: NXD_DECODE_WO_LATE=0)
   const int cb = p.cache_idx ? p.cache_idx[b] : b;
   const int slen = p.seq_len[b];
+  // splits that have keys; with tickets the others leave (a sequence without keys has one, which writes zeros)
+  const int live = !FUSE && p.tickets ? max(1, min(p.nsplit, (slen + p.kps - 1) / p.kps)) : 0;
+  if (!FUSE && p.tickets && split >= live) return;
   const uint16_t* kbase = p.kc + (int64_t)cb * p.c_sb + (int64_t)hkv * p.c_sh;
   const uint16_t* vbase = p.vc + (int64_t)cb * p.c_sb + (int64_t)hkv * p.c_sh;
 
@@ -215,32 +241,33 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(Params p) {
   // FUSE: the whole cache in one pass per workgroup (no key splits, no merge launch)
   const int kend = (FUSE && !SYNC) ? slen : min(slen, (split + 1) * p.kps);
   // K fragments and the V chunk of the NEXT chunk are loaded while this one runs its softmax and P.V
-  u32x4_t kf[4][NS], vv[VL];
+  u32x4_t kf[KT][NS], vv[VL];
   auto load_chunk = [&](int k0) {
 #pragma unroll
     for (int i = 0; i < VL; ++i) {
       const int idx = lane + 64 * i, key = idx / (D / 8), c = idx % (D / 8);
-      vv[i] = *reinterpret_cast<const u32x4_t*>(vbase + (int64_t)min(k0 + key, slen - 1) * p.c_sl + 8 * c);
+      const u32x4_t* a = reinterpret_cast<const u32x4_t*>(vbase + (int64_t)min(k0 + key, slen - 1) * p.c_sl + 8 * c);
+      vv[i] = FUSE ? *a : __builtin_nontemporal_load(a);
     }
 #pragma unroll
-    for (int kt = 0; kt < 4; ++kt) {
+    for (int kt = 0; kt < KT; ++kt) {
       const uint16_t* kr = kbase + (int64_t)min(k0 + kt * 16 + mi, slen - 1) * p.c_sl + 8 * g;
 #pragma unroll
       for (int s = 0; s < NS; ++s) kf[kt][s] = *reinterpret_cast<const u32x4_t*>(kr + 32 * s);
     }
   };
-  int k0 = split * p.kps + wid * KB;
+  int k0 = split * p.kps + wid * KC;
   if (k0 < kend) load_chunk(k0);
   // FUSE: the Wo block is issued AFTER the q and first K / V loads.  vmcnt retires in issue order:
   // issued first (round 3), the cold-HBM Wo loads had to land before the first score MFMA could
   // read its L2-resident K fragments, so their latency was added to the attention instead of
   // hidden behind it (attention + o_proj 7.16 -> 6.92 us, 0.619 -> 0.614 ms/token alternating, profiles/r4_decode_wo_late_ab.txt).
   if constexpr (FUSE && WO_LATE) load_wo();
-  for (; k0 < kend; k0 += NWV * KB) {
+  for (; k0 < kend; k0 += NWV * KC) {
     // ---- scores S^T[key][m] for 4 key tiles of 16
-    f32x4_t sc[4];
+    f32x4_t sc[KT];
 #pragma unroll
-    for (int kt = 0; kt < 4; ++kt) {
+    for (int kt = 0; kt < KT; ++kt) {
       sc[kt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int s = 0; s < NS; ++s)
@@ -253,11 +280,11 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(Params p) {
       const int idx = lane + 64 * i, key = idx / (D / 8), c = idx % (D / 8);
       *reinterpret_cast<u32x4_t*>(vt + key * D + 8 * c) = vv[i];
     }
-    if (k0 + NWV * KB < kend) load_chunk(k0 + NWV * KB);
+    if (k0 + NWV * KC < kend) load_chunk(k0 + NWV * KC);
     // ---- online softmax of query row mi over this chunk: lane holds keys k0 + 16 kt + 4 g + v
     float cm = -INFINITY;
 #pragma unroll
-    for (int kt = 0; kt < 4; ++kt)
+    for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const int key = k0 + kt * 16 + 4 * g + v;
@@ -271,9 +298,9 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(Params p) {
     const float mu = nm == -INFINITY ? 0.f : nm;
     const float alpha = run_m == -INFINITY ? 0.f : exp2f(run_m - mu);
     float ls = 0.f;
-    uint32_t p2[4][2];
+    uint32_t p2[KT][2];
 #pragma unroll
-    for (int kt = 0; kt < 4; ++kt) {
+    for (int kt = 0; kt < KT; ++kt) {
       float e[4];
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
@@ -298,7 +325,7 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(Params p) {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
+    for (int ks = 0; ks < KC / 32; ++ks) {
       const int src0 = (2 * (g & 1)) * 16 + mi, src1 = src0 + 16;
       const bool hi = (g >> 1) != 0;
       uint32_t w[4];
@@ -332,7 +359,7 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(Params p) {
 #pragma unroll
   for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
-    for (int v = 0; v < 4; ++v) red_o[(wid * 16 + 4 * g + v) * D + 16 * dt + (lane & 15)] = o[dt][v];
+    for (int v = 0; v < 4; ++v) red_o[wid * RED + (4 * g + v) * D + 16 * dt + (lane & 15)] = o[dt][v];
   __syncthreads();
   const int64_t pbase = ((int64_t)bh * p.nsplit + split) * M;
   for (int it = tid; it < M * D; it += 64 * NWV) {
@@ -346,7 +373,7 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(Params p) {
       const float mw = red_m[w * 16 + m];
       const float wt = (mw == -INFINITY) ? 0.f : exp2f(mw - gm);
       L += wt * red_l[w * 16 + m];
-      acc += wt * red_o[(w * 16 + m) * D + d];
+      acc += wt * red_o[w * RED + m * D + d];
     }
     if (FUSE && !SYNC) {   // bf16-rounded as the unfused path's attention output, then o_proj below
       reinterpret_cast<float*>(smem)[m * D + d] = bf2f(f2bf(L > 0.f ? acc / L : 0.f));
@@ -359,10 +386,16 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(Params p) {
           __hip_atomic_store(p.pl + pbase + m, L, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
       }
-    } else if (p.nsplit == 1) {
+    } else if (p.nsplit == 1 || live == 1) {
       const int tt = m / G, gg = m % G;
       p.out[(int64_t)b * p.o_sb + (int64_t)tt * p.o_st + (int64_t)(hkv * G + gg) * p.o_sh + d] =
           f2bf(L > 0.f ? acc / L : 0.f);
+    } else if (live > 1) {   // (through to memory: another workgroup reads them in this launch)
+      __hip_atomic_store(p.po + (pbase + m) * D + d, acc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (d == 0) {
+        __hip_atomic_store(p.pm + pbase + m, gm == -INFINITY ? -INFINITY : gm * 0.69314718056f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(p.pl + pbase + m, L, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
     } else {
       p.po[(pbase + m) * D + d] = acc;
       if (d == 0) {
@@ -370,6 +403,51 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(Params p) {
         p.pl[pbase + m] = L;
       }
     }
+  }
+  // ---- the last split of the head to come merges all of them (no split waits for another), in their order, so
+  // the bits are the same whichever comes last
+  if (!FUSE && live > 1) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    int* flg = reinterpret_cast<int*>(red_m);
+    if (tid == 0) {
+      flg[0] = __hip_atomic_fetch_add(p.tickets + bh, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == live - 1;
+      if (flg[0]) __hip_atomic_store(p.tickets + bh, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (!flg[0]) return;
+    // statistics and sums of 8 splits in flight together
+    const int64_t pb = (int64_t)bh * p.nsplit * M;
+    auto get = [](const float* a) { return __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+    for (int it = tid; it < M * D; it += 64 * NWV) {
+      const int m = it / D, d = it % D, tt = m / G, gg = m % G;
+      float gm = -INFINITY, L = 0.f, acc = 0.f;
+      for (int s0 = 0; s0 < live; s0 += 8) {
+        float ms[8], ls[8], os[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const int64_t at = pb + (int64_t)min(s0 + i, live - 1) * M + m;
+          ms[i] = get(p.pm + at);
+          ls[i] = get(p.pl + at);
+          os[i] = s0 + i < live ? get(p.po + at * D + d) : 0.f;
+        }
+        float nm = gm;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) nm = fmaxf(nm, ms[i]);
+        const float mu = nm == -INFINITY ? 0.f : nm, a = __expf(gm - mu);
+        L *= a;
+        acc *= a;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float w = __expf(ms[i] - mu);
+          L += s0 + i < live ? w * ls[i] : 0.f;
+          acc += w * os[i];
+        }
+        gm = nm;
+      }
+      p.out[(int64_t)b * p.o_sb + (int64_t)tt * p.o_st + (int64_t)(hkv * G + gg) * p.o_sh + d] = f2bf(L > 0.f ? acc / L : 0.f);
+    }
+    return;
   }
   if constexpr (SYNC) {
     int* flg = reinterpret_cast<int*>(red_m);   // [0] lost, [1] merger: red_m is free once the waves are
@@ -469,16 +547,16 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(Params p) {
   if (p.trace != nullptr && tid == 0) p.trace[2 * blockIdx.x + 1] = __builtin_amdgcn_s_memrealtime();
 }
 
-// Keys per split: enough splits that the (batch, kv head, split) grid reaches ~NXD_DECODE_ATTN_WGS
-// workgroups (default 128) -- the KV cache streams from HBM at the per-CU rate, so 24 workgroups on a
-// 2,304-key cache took 9.8 us -- between 128 keys (the caller's partial buffers hold Lmax / 128
-// splits) and 1,024 (one pass of the 8 waves x 2 chunks).  0.786 -> 0.726 ms/token at the notebook
-// config (profiles/r6_decode/attn_split_ab.txt).
+// Keys per split: enough splits that the (batch, kv head, split) grid reaches ~NXD_DECODE_ATTN_WGS workgroups (default
+// 512: two a CU, so that one's loads cover the other's arithmetic), between 128 keys (one pass of 4 waves; the caller's
+// partial buffers hold Lmax / 128 splits) and 1,024.  Targets of 128 / 256 / 512 / 1,024: 11.4 / 9.9 / 8.8 / 9.8 us for 6
+// sequences of up to 1,024 keys of 8 heads of 64; 20.3 / 18.6 / 19.5 / 21.4 for 13 of up to 1,500 of 8 of 128; the same
+// within 3 % for 1 and 4 sequences; 24.2 / 25.3 at 512 / 1,024 for 32 of up to 2,048.
 static int keys_per_split(int Lmax, int B, int Hkv) {
   static const int target = [] {
     const char* e = getenv("NXD_DECODE_ATTN_WGS");
-    const int v = e ? atoi(e) : 128;
-    return v > 0 ? v : 128;
+    const int v = e ? atoi(e) : 512;
+    return v > 0 ? v : 512;
   }();
   int kps = (int)(((int64_t)Lmax * B * Hkv + target - 1) / target);
   kps = (kps + KB - 1) / KB * KB;
@@ -619,7 +697,7 @@ void decode_attn_set_prefetch(const void* a, int64_t a_bytes, const void* b, int
 int decode_attn2_launch(const void* q, const int64_t* qs, const void* kc, const void* vc, const int64_t* cs,
                         const int* cache_idx, const int* seq_len, float* po, float* pm, float* pl, void* out,
                         const int64_t* os, int B, int T, int Hq, int Hkv, int D, int Lmax, float scale, int* nsplit_out,
-                        hipStream_t stream) {
+                        hipStream_t stream, int* tickets = nullptr) {
   if (Hkv <= 0 || Hq % Hkv) return -1;
   const int M = (Hq / Hkv) * T;
   if (M > 16 || (D != 64 && D != 128)) return -1;
@@ -636,9 +714,10 @@ int decode_attn2_launch(const void* q, const int64_t* qs, const void* kc, const 
   p.nsplit = (Lmax + kps - 1) / kps;
   p.scale_log2 = scale * 1.4426950408889634f;
   *nsplit_out = p.nsplit;
-  // D = 64: 8 waves (<= 2 chunks each per 1024-key split); D = 128: 4 waves (LDS: V tiles + merge)
-  const int nwv = D == 64 ? 8 : 4;
-  const size_t lds = (size_t)nwv * dattn::KB * D * 2 + (size_t)nwv * 16 * D * 4 + (size_t)2 * nwv * 16 * 4;
+  constexpr int nwv = 4;
+  const size_t lds = (size_t)nwv * dattn::KB * 64 * 2 + (size_t)2 * nwv * 16 * 4;   // (a chunk of V is 8 KB for both D)
+  p.tickets = tickets;
+  if (p.tickets) *nsplit_out = 1;   // (nothing left to merge)
   p.attn_wgs = B * Hkv * p.nsplit;
   p.trace = dattn::g_trace;
   int pf_wgs = 0;
@@ -653,8 +732,8 @@ int decode_attn2_launch(const void* q, const int64_t* qs, const void* kc, const 
   dattn::g_pf_bytes[0] = dattn::g_pf_bytes[1] = 0;
   const dim3 grid(p.attn_wgs + pf_wgs), block(64 * nwv);
   if (D == 64) {
-    (void)hipFuncSetAttribute((const void*)dattn::attn_kernel<64, 8, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    hipLaunchKernelGGL((dattn::attn_kernel<64, 8, false>), grid, block, lds, stream, p);
+    (void)hipFuncSetAttribute((const void*)dattn::attn_kernel<64, 4, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipLaunchKernelGGL((dattn::attn_kernel<64, 4, false>), grid, block, lds, stream, p);
   } else {
     (void)hipFuncSetAttribute((const void*)dattn::attn_kernel<128, 4, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     hipLaunchKernelGGL((dattn::attn_kernel<128, 4, false>), grid, block, lds, stream, p);

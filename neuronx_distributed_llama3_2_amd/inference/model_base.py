@@ -263,8 +263,11 @@ class DecoderInferenceMixin:
         else:
             res = ops.vocab_parallel_embedding(input_ids, ew, emb.start_index).reshape(M, -1).contiguous()
         qkv = torch.empty((M, W), dtype=res.dtype, device=res.device)
-        # counters with which a long reduction (down) is split over workgroups; one launch clears them for all layers
-        tickets = torch.zeros(_FEW_TICKETS, dtype=torch.int32, device=res.device) if 8 < M <= _FEW_ROWS else None
+        # counters with which the workgroups of a split reduction (down) or of a sequence's key splits find the last of
+        # them; one launch clears them for all layers
+        tickets = None
+        if 2 < M <= _FEW_ROWS:
+            tickets = torch.zeros(max(_FEW_TICKETS, B * nkv), dtype=torch.int32, device=res.device)
         for i, layer in enumerate(self.model.layers):
             attn = layer.self_attn
             w_qkv, s_qkv = self._weight_scale(attn.qkv_proj)
@@ -296,7 +299,7 @@ class DecoderInferenceMixin:
                 C.dgemv(2, res, ln2, self.eps, w_gu, a, 0, 0, 0, None, None, None, 1, None, None, None, oacc, None)
                 C.dgemv(1, a, None, 0.0, w_d, res, 0, 0, 0, None, None, None, 1, None, None, None, None, oacc)
                 continue
-            o = ops.decode_attention(q, kc, vc, cache_len, sid32)
+            o = ops.decode_attention(q, kc, vc, cache_len, sid32, tickets=tickets)
             C.dgemv(1, o.reshape(M, nq * D), None, 0.0, w_o, res, 0, 0, 0, None, None, None, 1,
                     None, None, None, wscale=s_o, tickets=tickets)              # res += o_proj(o)
             a = torch.empty((M, w_d.shape[1]), dtype=res.dtype, device=res.device)

@@ -20,9 +20,10 @@ CHUNK = 128
 
 def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, seq_len: torch.Tensor,
                      cache_idx: Optional[torch.Tensor] = None, softmax_scale: Optional[float] = None,
-                     out: Optional[torch.Tensor] = None) -> torch.Tensor:
+                     out: Optional[torch.Tensor] = None, tickets: Optional[torch.Tensor] = None) -> torch.Tensor:
     """q: [B, T, Hq, D] new-token queries; keys [0, seq_len[b]) are valid for the LAST token, and
-    token t sees keys < seq_len[b] - (T - 1 - t).  Returns [B, T, Hq, D]."""
+    token t sees keys < seq_len[b] - (T - 1 - t).  Returns [B, T, Hq, D].  tickets: at least B * Hkv zeroed
+    int32 (left zeroed; calls in one stream may share them): key splits are merged in the same launch."""
     B, T, Hq, D = q.shape
     scale = softmax_scale if softmax_scale is not None else 1.0 / math.sqrt(D)
     if out is None:
@@ -30,7 +31,7 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     if use_native(q, k_cache):
         nsplit = max(1, (k_cache.shape[2] + CHUNK - 1) // CHUNK)
         ext().decode_attn(q, k_cache, v_cache, cache_idx.to(torch.int32) if cache_idx is not None else None,
-                          seq_len.to(torch.int32), out, float(scale), nsplit)
+                          seq_len.to(torch.int32), out, float(scale), nsplit, tickets)
         return out
     Hkv = k_cache.shape[1]
     g = Hq // Hkv
