@@ -28,10 +28,12 @@
 //     c ^ 2 * ((t & 3) | ((t >> 3) & 1) << 2): the two 16-lane groups of a transposed read (4 token
 //     rows x 16 features each, rows t, t + 8) land on 16 distinct bank quads — conflict-free.  The
 //     swizzle is applied to each lane's SOURCE address (the DMA writes lane-linearly, rule 21);
-//   * epilogue: the fp32 tile goes through LDS (padded rows) so that every global atomic add covers
-//     256 contiguous bytes (MI355X_MICROARCH "Global float atomics": full rate), issued without
-//     return and left in flight when the workgroup exits; with one token split per tile each
-//     element receives exactly one add (deterministic), with S splits S adds in any order.
+//   * epilogue: the fp32 tile goes through LDS (padded rows) so that every global access covers
+//     256 contiguous bytes.  With one token split per tile the workgroup alone adds to its tile: it
+//     loads, adds and stores, 32 rows ahead.  With S splits the adds are S atomics in any order,
+//     issued without return and left in flight when the workgroup exits.  One split by atomics had
+//     run at 2.4 TB/s: 8 experts' 4096 x 14336 and 4096 x 28672 gradients over 8,192 rows 2.63 ms a
+//     launch, 1.73 without an epilogue, 1.97 with loads and stores (non-temporal or not: the same).
 //   * grouped (MoE expert weight gradients, dW[e] += x_e^T dy_e over expert-sorted rows): the grid
 //     covers (split, expert, tile); each workgroup reads its expert's row range from the device
 //     offsets (no host sync) and its ragged token tail DMAs a zero chunk instead of a foreign row.
@@ -62,6 +64,7 @@ struct Params {
   int band;             // row tiles per raster band
   int ablate;           // A/B diagnostics only (wgrad_gemm_set_ablate): 1 = skip the epilogue adds,
                         // 2 = skip the MFMAs, 4 = skip the LDS-DMA refills of stages >= 3
+  int own;              // one split, aligned rows: a workgroup alone adds to its tile (load, add, store), else atomics
   // grouped mode: expert e owns rows offs[e] .. offs[e+1] of dy / x; c += e * c_es
   const int* offs;
   int E;
@@ -291,12 +294,44 @@ __global__ void __launch_bounds__(NT, 1) wgrad_kernel(Params p) {
 
   // ---- epilogue: per wave, 4 rounds of 32 rows x 64 columns through a private padded LDS slab
   // ([32][68] fp32: the two row groups of a 32-lane store half are 4 rows apart -> 16 banks apart),
-  // then one row (64 floats, 256 contiguous bytes) per atomic wave-instruction.
+  // then 4 rows (of 256 contiguous bytes) per load and store, or one per atomic wave-instruction.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();   // every wave is done with the ring
   constexpr int LD = 68;
   float* slab = reinterpret_cast<float*>(smem) + wid * (32 * LD);
   const int ccol = lane & 15, crow = 4 * (lane >> 4);
+  if (p.own) {
+    const int col = n0 + wn * 64 + 4 * ccol, row = m0 + wm * 128 + (lane >> 4);
+    float* cp = cbase + (int64_t)row * p.ldc + col;
+    const int left = col < p.N ? p.M - row : 0;   // rows of this lane that there are
+    f32x4_t cur[8];
+    auto load = [&](int rnd) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        if (32 * rnd + 4 * k < left) cur[k] = *reinterpret_cast<const f32x4_t*>(cp + (int64_t)(32 * rnd + 4 * k) * p.ldc);
+    };
+    load(0);
+    __syncthreads();   // every wave is done with the ring
+#pragma unroll
+    for (int rnd = 0; rnd < 4; ++rnd) {
+#pragma unroll
+      for (int ii = 0; ii < 2; ++ii)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) slab[(16 * ii + crow + r) * LD + 16 * j + ccol] = acc[2 * rnd + ii][j][r];
+      __builtin_amdgcn_wave_barrier();
+      f32x4_t sum[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) sum[k] = cur[k] + *reinterpret_cast<const f32x4_t*>(slab + (4 * k + (lane >> 4)) * LD + 4 * ccol);
+      if (rnd < 3) load(rnd + 1);
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        if (32 * rnd + 4 * k < left && !(p.ablate & 1)) *reinterpret_cast<f32x4_t*>(cp + (int64_t)(32 * rnd + 4 * k) * p.ldc) = sum[k];
+      __builtin_amdgcn_wave_barrier();
+    }
+    return;
+  }
+  __syncthreads();   // every wave is done with the ring
 #pragma unroll
   for (int rnd = 0; rnd < 4; ++rnd) {
 #pragma unroll
@@ -387,6 +422,7 @@ int wgrad_gemm_launch(const void* dy, int64_t ld_dy, const void* x, int64_t ld_x
   splits = splits < 1 ? 1 : (splits > steps ? steps : splits);
   p.t_per_split = ceil_div(steps, splits) * wg::BK;
   p.splits = ceil_div(T, p.t_per_split);
+  p.own = p.splits == 1 && ldc % 4 == 0 && ldc >= N && (reinterpret_cast<uintptr_t>(c) & 15) == 0;
   p.band = wg::band_rows();
   p.ablate = wg::g_ablate;
   const int64_t nwg = (int64_t)p.mt * p.nt * p.splits;
@@ -416,6 +452,7 @@ int wgrad_gemm_grouped_launch(const void* dy, int64_t ld_dy, const void* x, int6
   // splits for the mean group (all E groups' tiles share the grid)
   const int mean = std::max(wg::BK, (rows / E) / wg::BK * wg::BK);
   p.splits = wgrad_gemm_choose_splits(mean, (int)std::min<int64_t>((int64_t)M * E, INT32_MAX), N);
+  p.own = p.splits == 1 && ldc % 4 == 0 && ldc >= N && c_es % 4 == 0 && (E == 1 || c_es >= (int64_t)(M - 1) * ldc + N) && (reinterpret_cast<uintptr_t>(c) & 15) == 0;
   p.band = wg::band_rows();
   p.ablate = wg::g_ablate;
   const int64_t nwg = (int64_t)p.mt * p.nt * E * p.splits;

@@ -136,7 +136,11 @@ class GroupedLinearFunc(torch.autograd.Function):
         if ctx.needs_input_grad[1]:
             mg = getattr(w, "main_grad", None)
             if mg is not None and mg.dtype == torch.float32 and mg.is_contiguous():
+                from ..parallel_layers import stream_split
+
+                stream_split.accumulate_begin(w)   # (a load and a store of main_grad, as in the dense layers)
                 wgrad(mg, True)
+                stream_split.accumulate_end(w)
                 cb = getattr(w, "_nxd_grad_ready", None)
                 if cb is not None:
                     cb(w)

@@ -1,0 +1,46 @@
+"""The weight-gradient kernel's epilogue: load, add and store where a workgroup alone owns its tile, atomics otherwise.
+Against float64, on partial tiles, strided and misaligned gradients, empty and one-row experts; what lies beside the
+gradient stays."""
+import pytest
+import torch
+
+from neuronx_distributed_llama3_2_amd.ops._ext import ext
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(mg, before, dy, x):
+    # sums of T products of bf16 in fp32: T roundings of 2^-24 of the sum of magnitudes, at the most
+    ref = before.double() + dy.double().t() @ x.double()
+    scale = dy.double().abs().t() @ x.double().abs() + before.double().abs()
+    assert ((mg.double() - ref).abs() <= (dy.shape[0] + 1) * 2.0 ** -24 * scale + 1e-30).all()
+
+
+@pytest.mark.parametrize("pad,shift", [(0, 0), (4, 0), (8, 4), (1, 0), (0, 1)])   # the last two: atomics
+@pytest.mark.parametrize("T,M,N,splits", [(32, 8, 8, 1), (64, 256, 256, 1), (96, 264, 248, 1), (160, 520, 72, 1), (512, 264, 264, 4)])
+def test_dense(T, M, N, splits, pad, shift):
+    g = torch.Generator(device="cuda").manual_seed(T + M)
+    dy, x = (torch.randn(T, n, generator=g, device="cuda").bfloat16() for n in (M, N))
+    flat = torch.randn(M * (N + pad) + shift + 64, generator=g, device="cuda")
+    start = flat.clone()
+    view = lambda f: f[shift:shift + M * (N + pad)].view(M, N + pad)[:, :N]
+    ext().wgrad_gemm(view(flat), dy, x, splits)
+    _check(view(flat), view(start), dy, x)
+    view(flat).copy_(view(start))
+    assert torch.equal(flat, start)
+
+
+@pytest.mark.parametrize("sizes", [[0, 1, 31, 64, 200], [512, 0, 513, 0, 0], [0, 0, 0, 0, 7]])
+@pytest.mark.parametrize("K,N", [(264, 72), (256, 512)])
+def test_grouped(sizes, K, N):
+    g = torch.Generator(device="cuda").manual_seed(sum(sizes))
+    rows, E = sum(sizes), len(sizes)
+    x, dy = (torch.randn(rows, n, generator=g, device="cuda").bfloat16() for n in (K, N))
+    offs = torch.tensor([0] + sizes, device="cuda").cumsum(0).to(torch.int32)
+    mg = torch.randn(E, K, N, generator=g, device="cuda")
+    before = mg.clone()
+    ext().grouped_gemm(2, x, dy, offs, mg, True)
+    for e in range(E):
+        a, b = int(offs[e]), int(offs[e + 1])
+        _check(mg[e], before[e], x[a:b], dy[a:b]) if b > a else None
+        assert b > a or torch.equal(mg[e], before[e])
