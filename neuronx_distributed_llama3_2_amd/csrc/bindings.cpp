@@ -769,8 +769,8 @@ void dequant_int8(at::Tensor w, c10::optional<at::Tensor> scale, double tscale, 
 }
 
 // main_grad [M, N] fp32 += dy [T, M]^T x [T, N] (csrc/wgrad_gemm.hip): token-major bf16 operands with
-// unit inner strides, row strides multiples of 8 elements, T % 32 == 0; splits <= 0 -> auto.
-void wgrad_gemm(at::Tensor mg, at::Tensor dy, at::Tensor x, int64_t splits) {
+// unit inner strides, row strides multiples of 8 elements, T % 32 == 0 unless tail; splits <= 0 -> auto.
+void wgrad_gemm(at::Tensor mg, at::Tensor dy, at::Tensor x, int64_t splits, bool tail) {
   check_bf16(dy, "dy");
   check_bf16(x, "x");
   check_cuda(mg, "main_grad");
@@ -780,7 +780,7 @@ void wgrad_gemm(at::Tensor mg, at::Tensor dy, at::Tensor x, int64_t splits) {
   TORCH_CHECK(x.size(0) == T && mg.size(0) == M && mg.size(1) == N, "wgrad_gemm: shape mismatch");
   TORCH_CHECK(dy.stride(1) == 1 && x.stride(1) == 1 && mg.stride(1) == 1, "wgrad_gemm: unit inner strides");
   TORCH_CHECK(dy.stride(0) % 8 == 0 && x.stride(0) % 8 == 0, "wgrad_gemm: row strides must be multiples of 8");
-  TORCH_CHECK(T % 32 == 0 && M % 8 == 0 && N % 8 == 0, "wgrad_gemm: T % 32, M % 8, N % 8 must be 0");
+  TORCH_CHECK((tail || T % 32 == 0) && M % 8 == 0 && N % 8 == 0, "wgrad_gemm: T % 32, M % 8, N % 8 must be 0");
   TORCH_CHECK(T <= INT32_MAX && M <= INT32_MAX && N <= INT32_MAX, "wgrad_gemm: dims too large");
   check_aligned16(dy, "dy");
   check_aligned16(x, "x");
@@ -1161,7 +1161,7 @@ PYBIND11_MODULE(_C, m) {
   m.def("dequant_int8", &dequant_int8);
   m.def("expert_gemv", &expert_gemv);
   m.def("grouped_gemm", &grouped_gemm);
-  m.def("wgrad_gemm", &wgrad_gemm);
+  m.def("wgrad_gemm", &wgrad_gemm, py::arg("main_grad"), py::arg("dy"), py::arg("x"), py::arg("splits"), py::arg("tail") = false);
   m.def("dense_gemm", &dense_gemm, py::arg("layout"), py::arg("epi"), py::arg("a"), py::arg("b"), py::arg("c"),
         py::arg("splits") = 0);
   m.def("dense_gemm_set_pipe", [](int64_t v) { nxd::dense_gemm_set_pipe((int)v); });

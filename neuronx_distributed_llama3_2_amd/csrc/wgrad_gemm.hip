@@ -110,7 +110,8 @@ __device__ __forceinline__ void wait_vm(int newer) {   // this thread's pieces o
 // profiles/r3_wgrad_kernel_prio_rejected.jsonl)
 // PP: the ping-pong main loop of csrc/grouped_rowgemm.hip (two 16-MFMA phases per stage, wave group
 // 1 one barrier behind group 0; ring-safety argument there).
-template <bool GROUPED, bool PP>
+// TAIL: the last stage may have fewer than 32 tokens, the others are zeros (always with GROUPED).
+template <bool GROUPED, bool PP, bool TAIL>
 __global__ void __launch_bounds__(NT, 1) wgrad_kernel(Params p) {
   __shared__ __attribute__((aligned(16))) char smem[LDS_BYTES];
   const int tiles = p.mt * p.nt;
@@ -140,9 +141,9 @@ __global__ void __launch_bounds__(NT, 1) wgrad_kernel(Params p) {
   } else {
     t_begin = split * p.t_per_split;
     t_end = min(p.T, t_begin + p.t_per_split);
-    nk = (t_end - t_begin) / BK;
+    nk = TAIL ? ceil_div(t_end - t_begin, BK) : (t_end - t_begin) / BK;
   }
-  const int rows = t_end - t_begin;   // grouped: token rows >= rows of the last stage read zeros
+  const int rows = t_end - t_begin;   // TAIL: token rows >= rows of the last stage read zeros
 
   const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int wm = wid >> 2, wn = wid & 3;   // 2 x 4 waves: rows 128 wm.., cols 64 wn..
@@ -176,7 +177,7 @@ __global__ void __launch_bounds__(NT, 1) wgrad_kernel(Params p) {
     for (int i = 0; i < PIECES; ++i) {
       const uint16_t* sa = src_a[i] + oa;
       const uint16_t* sb = src_b[i] + ob;
-      if constexpr (GROUPED) {
+      if constexpr (TAIL) {
         if (s * BK + tt_of[i] >= rows) sa = sb = reinterpret_cast<const uint16_t*>(g_zero16);   // past the group's end
       }
       dma16(sa, __builtin_amdgcn_readfirstlane(img + i * 1024));
@@ -199,7 +200,7 @@ __global__ void __launch_bounds__(NT, 1) wgrad_kernel(Params p) {
       const uint32_t img = lds0 + (s % STAGES) * STAGE_BYTES + wid * PIECES * 1024;
       const uint16_t* sa = src_a[hh] + (int64_t)s * BK * p.ld_dy;
       const uint16_t* sb = src_b[hh] + (int64_t)s * BK * p.ld_x;
-      if constexpr (GROUPED) {
+      if constexpr (TAIL) {
         if (s * BK + tt_of[hh] >= rows) sa = sb = reinterpret_cast<const uint16_t*>(g_zero16);
       }
       dma16(sa, __builtin_amdgcn_readfirstlane(img + hh * 1024));
@@ -372,12 +373,12 @@ static bool use_pp() {
   return g_pp != 0;
 }
 
-template <bool G>
+template <bool G, bool TAIL>
 void launch(const Params& p, int64_t nwg, hipStream_t stream) {
   if (use_pp())
-    hipLaunchKernelGGL((wgrad_kernel<G, true>), dim3((unsigned)nwg), dim3(NT), 0, stream, p);
+    hipLaunchKernelGGL((wgrad_kernel<G, true, TAIL>), dim3((unsigned)nwg), dim3(NT), 0, stream, p);
   else
-    hipLaunchKernelGGL((wgrad_kernel<G, false>), dim3((unsigned)nwg), dim3(NT), 0, stream, p);
+    hipLaunchKernelGGL((wgrad_kernel<G, false, TAIL>), dim3((unsigned)nwg), dim3(NT), 0, stream, p);
 }
 
 }  // namespace wg
@@ -390,7 +391,7 @@ void wgrad_gemm_set_pp(int v) { wg::g_pp = v != 0; }
 // of minimal cost (fewer splits = fewer fp32 atomic adds per element).
 int wgrad_gemm_choose_splits(int T, int M, int N) {
   const int tiles = ceil_div(M, wg::BM) * ceil_div(N, wg::BN);
-  const int steps = T / wg::BK;
+  const int steps = ceil_div(T, wg::BK);
   int best = 1;
   int64_t best_cost = INT64_MAX;
   for (int s = 1; s <= 32 && s <= steps; ++s) {
@@ -404,11 +405,11 @@ int wgrad_gemm_choose_splits(int T, int M, int N) {
   return best;
 }
 
-// c [M, N] fp32 += dy[T, M]^T x[T, N]; T % 32 == 0, M % 8 == 0, N % 8 == 0, 16-B aligned rows.
+// c [M, N] fp32 += dy[T, M]^T x[T, N]; M % 8 == 0, N % 8 == 0, 16-B aligned rows.
 int wgrad_gemm_launch(const void* dy, int64_t ld_dy, const void* x, int64_t ld_x, float* c, int64_t ldc, int T, int M,
                       int N, int splits, hipStream_t stream) {
   if (T <= 0 || M <= 0 || N <= 0) return 0;
-  if (T % wg::BK || M % 8 || N % 8 || ld_dy % 8 || ld_x % 8) return -1;
+  if (M % 8 || N % 8 || ld_dy % 8 || ld_x % 8) return -1;
   wg::Params p{};
   p.dy = static_cast<const uint16_t*>(dy);
   p.x = static_cast<const uint16_t*>(x);
@@ -418,7 +419,7 @@ int wgrad_gemm_launch(const void* dy, int64_t ld_dy, const void* x, int64_t ld_x
   p.mt = ceil_div(M, wg::BM);
   p.nt = ceil_div(N, wg::BN);
   if (splits <= 0) splits = wgrad_gemm_choose_splits(T, M, N);
-  const int steps = T / wg::BK;
+  const int steps = ceil_div(T, wg::BK);
   splits = splits < 1 ? 1 : (splits > steps ? steps : splits);
   p.t_per_split = ceil_div(steps, splits) * wg::BK;
   p.splits = ceil_div(T, p.t_per_split);
@@ -427,7 +428,10 @@ int wgrad_gemm_launch(const void* dy, int64_t ld_dy, const void* x, int64_t ld_x
   p.ablate = wg::g_ablate;
   const int64_t nwg = (int64_t)p.mt * p.nt * p.splits;
   if (nwg > INT32_MAX) return -2;
-  wg::launch<false>(p, nwg, stream);
+  if (T % wg::BK)
+    wg::launch<false, true>(p, nwg, stream);
+  else
+    wg::launch<false, false>(p, nwg, stream);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
@@ -457,7 +461,7 @@ int wgrad_gemm_grouped_launch(const void* dy, int64_t ld_dy, const void* x, int6
   p.ablate = wg::g_ablate;
   const int64_t nwg = (int64_t)p.mt * p.nt * E * p.splits;
   if (nwg > INT32_MAX) return -2;
-  wg::launch<true>(p, nwg, stream);
+  wg::launch<true, true>(p, nwg, stream);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 

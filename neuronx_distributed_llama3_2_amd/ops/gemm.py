@@ -110,9 +110,18 @@ def _use_wgrad_t(go2: torch.Tensor, x2: torch.Tensor = None, K: int = None) -> b
 # vocabulary-sized output (lm_head) when no producer wrote a feature-major copy: TP=8 1201 vs 1074
 # TF/s for the hipBLASLt path and its two transposes (the 1 GiB logits gradient), TP=1 a tie.
 # NXD_WGRAD_KERNEL = auto | 1 (whenever the shapes allow) | 0.
+#
+# Token counts that are no multiple of 64 have neither producer copies nor the dense kernel below, and go to this kernel
+# where its 256 x 256 tiles fill the chip (below 128 tiles its splits lose: 3,072 x 2,048 over 3,000 tokens 85 us, library
+# 68) or there are few tokens (over 104: 15 and 41).  Over 1,000 / 3,000 / 8,200 tokens, library with its two transposes ->
+# this kernel, us: 16,384 x 2,048 125 -> 99, 249 -> 212, 597 -> 509; 2,048 x 8,192 72 -> 52, 127 -> 113, 294 -> 249;
+# 128,256 x 2,048 1,078 -> 777, 2,262 -> 1,680, 5,862 -> 4,256; 22,016 x 4,096 363 -> 297, 720 -> 611, 1,570 -> 1,532.  The
+# transposes' share falls as M N / (M + N) grows; measured up to 3,631.  Odd token counts take no transposes: 8-18 % up to
+# 1,001 tokens, 0-7 % at 3,001, slower from 4,001 on.
 _WG_KERNEL = os.environ.get("NXD_WGRAD_KERNEL", "auto")
 _WG_SKINNY = 1100.0
 _WG_WIDE = 16000
+_WG_RAGGED = 4000.0
 
 
 def _use_wgrad_kernel(mg: torch.Tensor, go2: torch.Tensor, x2: torch.Tensor, has_copy: bool = False) -> bool:
@@ -120,11 +129,14 @@ def _use_wgrad_kernel(mg: torch.Tensor, go2: torch.Tensor, x2: torch.Tensor, has
         return False
     T, M = go2.shape
     N = x2.shape[1]
-    if T % 32 or M % 8 or N % 8 or go2.stride(1) != 1 or x2.stride(1) != 1 or mg.stride(1) != 1:
+    if T == 0 or M % 8 or N % 8 or go2.stride(1) != 1 or x2.stride(1) != 1 or mg.stride(1) != 1:
         return False
     if go2.stride(0) % 8 or x2.stride(0) % 8 or go2.data_ptr() % 16 or x2.data_ptr() % 16:
         return False
-    return _WG_KERNEL == "1" or M * N / (M + N) < _WG_SKINNY or (not has_copy and max(M, N) >= _WG_WIDE)
+    if T % 64 and not has_copy and (T % 8 == 0 or T <= 3072) and M * N / (M + N) < _WG_RAGGED \
+            and (T <= 320 or -(-M // 256) * -(-N // 256) >= 128):
+        return True
+    return T % 32 == 0 and (_WG_KERNEL == "1" or M * N / (M + N) < _WG_SKINNY or (not has_copy and max(M, N) >= _WG_WIDE))
 
 
 # The hand-written dense GEMM (csrc/dense_gemm.hip) in its TN form reads the token-major dy / x
@@ -188,7 +200,7 @@ def wgrad_accumulate_(mg: torch.Tensor, go2: torch.Tensor, x2, go_t: torch.Tenso
         _dense_wgrad(mg, go2, x2)
         return
     if _use_wgrad_kernel(mg, go2, x2, has_copy=has_copy):
-        ext().wgrad_gemm(mg, go2, x2, 0)
+        ext().wgrad_gemm(mg, go2, x2, 0, True)
         return
     if x_t is not None and not (x_t.dim() == 2 and x_t.is_contiguous() and x_t.shape[1] == go2.shape[0]):
         x_t = None

@@ -1,6 +1,6 @@
-"""The weight-gradient kernel's epilogue: load, add and store where a workgroup alone owns its tile, atomics otherwise.
-Against float64, on partial tiles, strided and misaligned gradients, empty and one-row experts; what lies beside the
-gradient stays."""
+"""The weight-gradient kernel's epilogue (load, add and store where a workgroup alone owns its tile, atomics otherwise) and
+its last, partial token stage.  Against float64, on partial tiles, strided and misaligned gradients, empty and one-row
+experts, any token count; what lies beside the gradient stays."""
 import pytest
 import torch
 
@@ -44,3 +44,34 @@ def test_grouped(sizes, K, N):
         a, b = int(offs[e]), int(offs[e + 1])
         _check(mg[e], before[e], x[a:b], dy[a:b]) if b > a else None
         assert b > a or torch.equal(mg[e], before[e])
+
+
+@pytest.mark.parametrize("T,splits", [(1, 1), (7, 0), (31, 1), (33, 1), (65, 1), (100, 3), (129, 1), (1000, 0), (1001, 4)])
+@pytest.mark.parametrize("M,N", [(8, 264), (264, 512)])
+def test_any_token_count(T, splits, M, N):
+    g = torch.Generator(device="cuda").manual_seed(T + M)
+    dy, x = (torch.full((T + 64, n + 8), float("nan"), device="cuda", dtype=torch.bfloat16) for n in (M, N))
+    for t, n in ((dy, M), (x, N)):
+        t[:T, :n] = torch.randn(T, n, generator=g, device="cuda")
+    dy, x = dy[:T, :M], x[:T, :N]                # NaNs all around
+    mg = torch.randn(M, N, generator=g, device="cuda")
+    before = mg.clone()
+    ext().wgrad_gemm(mg, dy, x, splits, True)
+    _check(mg, before, dy, x)
+
+
+@pytest.mark.parametrize("T,M,N,own", [
+    (72, 512, 512, True), (301, 512, 512, True), (328, 512, 512, False),       # few tiles: few tokens only
+    (328, 4096, 2048, True), (1001, 4096, 2048, True), (3080, 4096, 2048, True), (3081, 4096, 2048, False),
+    (1000, 8192, 8192, False), (1000, 4096, 2052, False),
+])
+def test_route_of_ragged_token_counts(T, M, N, own):
+    from neuronx_distributed_llama3_2_amd.ops import gemm as G
+
+    g = torch.Generator(device="cuda").manual_seed(T)
+    dy, x = (torch.randn(T, n, generator=g, device="cuda").bfloat16() for n in (M, N))
+    mg = torch.randn(M, N, generator=g, device="cuda")
+    before = mg.clone()
+    assert G._use_wgrad_kernel(mg, dy, x) == (own and G._WG_KERNEL != "0")
+    G.wgrad_accumulate_(mg, dy, x)
+    _check(mg, before, dy, x)
