@@ -179,10 +179,16 @@ struct Finish {
   __device__ __forceinline__ f32x4_t collect(int at) const {
     const float* ws = parts(at);
     f32x4_t v = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-    for (int j = 0; j < p.splits; ++j)
+    for (int j0 = 0; j0 < p.splits; j0 += 8) {   // 8 parts in flight together
+      f32x4_t u[8];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] += __hip_atomic_load(ws + j * 256 + 64 * i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) u[j][i] = __hip_atomic_load(ws + min(j0 + j, p.splits - 1) * 256 + 64 * i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (j0 + j < p.splits) v += u[j];
+    }
     return v;
   }
 
@@ -261,6 +267,25 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
   constexpr bool GS = NORM && CW > 0;
   static_assert(!GS || NW * CW * KC * 2 <= S::PART, "the norm's weight in LDS");
 
+  // SPLIT: all waves of a workgroup share the tiles of which its part was the last to come
+  auto finish_last = [&]() {
+    meet();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");   // (keeps the loads below the tickets)
+    int turn = 0;
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      Finish<EPI, NORM, R, I8> f(p, lane, t);
+      uint64_t todo = reinterpret_cast<const uint64_t*>(sq)[t];
+      for (todo = (uint64_t)__builtin_amdgcn_readfirstlane((int)(todo >> 32)) << 32 | (uint32_t)__builtin_amdgcn_readfirstlane((int)todo);
+           todo; todo &= todo - 1, ++turn) {
+        if (turn % (NW + S::FW) != w) continue;
+        const int tile = tile0 + __builtin_ctzll(todo) * step;
+        f.fetch(tile);
+        f.finish(f.collect(tile * MT + t));
+      }
+    }
+  };
+
   // Twice a tile all waves meet: when `part` is free, and when it is full
   if (w >= NW) {
     if (GS) {
@@ -305,24 +330,15 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
       for (int t = 0; t < T; ++t) {
-        const int mine = (tile0 + lane * step) * MT + (w - NW) * T + t;
-        const bool there = tile0 + lane * step < tiles;
+        const int mt = (w - NW) * T + t, mine = (tile0 + lane * step) * MT + mt;
         int n = -1;
-        if (there) n = __hip_atomic_fetch_add(p.tickets + mine, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (tile0 + lane * step < tiles) n = __hip_atomic_fetch_add(p.tickets + mine, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         const bool last = n == p.splits - 1;
         if (last) __hip_atomic_store(p.tickets + mine, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");   // (no instruction: keeps the loads below the tickets)
-        for (uint64_t todo = __ballot(last); todo; todo &= todo - 1) {
-          const int tile = tile0 + __builtin_ctzll(todo) * step;
-          if (t == 0) {
-            f0.fetch(tile);
-            f0.finish(f0.collect(tile * MT + (w - NW) * T));
-          } else {
-            f1.fetch(tile);
-            f1.finish(f1.collect(tile * MT + (w - NW) * T + 1));
-          }
-        }
+        const uint64_t todo = __ballot(last);
+        if (lane == 0) reinterpret_cast<uint64_t*>(sq)[mt] = todo;
       }
+      finish_last();
     }
     return;
   }
@@ -497,6 +513,7 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
       }
       publish();
     }
+    if constexpr (SPLIT) finish_last();
   } else {
     constexpr int XL = 4 * MT + (NORM ? 4 : 0);   // loads of a stage beside the weights'
     u32x4_t x[D][MT][4], g[NORM ? D : 1][4];
@@ -577,11 +594,24 @@ static int launch(FewRowsParams p, hipStream_t s, int splits = 1) {
 //   K <= 4224: 11 waves of 3 chunks: 28672 x 4096 40 / 43 / 55 (streamed 46 / 55 / 225; int8 25 / 27 / 40); without a norm and
 //     up to 256 tiles streamed: 4096 x 4096 9.0 / 10.9 / 13.1 against 9.0 / 10.8 / 14.8.
 //   longer: streamed, tiles of 16 rows for more than 2048 weight rows (4096 x 14336 23 / 28 / 38, of 8 rows 25 / 39 / 58),
-//     else of 8, so that every CU has one (2048 x 8192 9.5 / 13.0 / 18.8, of 16 rows 11.5 / 15.4 / 20.8).  A workgroup of 8
-//     weight rows reads all of the activations for them, 4 times the weights' bytes at 32 rows and past what the caches
-//     deliver to a CU; from 9 rows on the reduction is split instead, each workgroup keeping the activations of
-//     2048 elements for its tiles: 10.7 / 12.1 / 14.5 (2048 x 12288: 12.9 / 19.1 / 27 -> 14.9 / 16.8 / 20).
-constexpr int kSplitFrom = 9;   // rows
+//     else of 8, so that every CU has one (2048 x 8192 9.5 / 13.0 / 18.8, of 16 rows 11.5 / 15.4 / 20.8).  Streamed, a
+//     workgroup reads all of the activations for its one tile: at 16 rows as much as the tile's weights, or twice that.
+//     So with more rows the reduction is split (`parts`): a workgroup keeps the activations of its part for several tiles.
+//     2048 x 8192 at 9 / 13 / 32 rows 10.7 / 12.2 / 18.9 streamed, 10.9 / 11.2 / 12.8 in parts of 1024 elements (two
+//     workgroups a CU; of 1792, one a CU: 11.7 / 12.0 / 14.6); 2048 x 12288 at 9 / 16 / 32 16.0 / 18.9 / 27.3 -> 13.4 / 14.0 /
+//     16.5 in parts of 1792 (of 1024 15.0 / 15.5 / 18.8: more parts to add up, more tiles a workgroup); 4096 x 14336 at 9 / 13 /
+//     32 24.1 / 26.5 / 38.7 -> 24.4 / 24.5 / 29.2; 4096 x 11008 19.2 / 21.0 / 30.1 -> 21.0 / 21.3 / 25.6; 8192 x 8192 27.6 / 28.9 /
+//     41.9 -> 28.8 / 29.0 / 33.5; 8192 x 28672 at 13 / 32 92 / 142 -> 88 / 102.
+//     The parts' sums meet in memory; the last to come adds them up, its waves sharing its tiles (by one wave: 2.5 us more).
+constexpr int kLongPart = 72;   // chunks of the reduction from which parts are long
+
+static int parts(int M, int N, int K) {   // of the reduction; 0: not split
+  const int nck = ceil_div(K, KC), tiles = ceil_div(N, 16), per = nck > kLongPart ? 14 : 8;
+  if (nck <= 33 || M > FEW_MAX_ROWS) return 0;
+  if (tiles <= 128 ? M < (nck > kLongPart ? 9 : 12) : M <= 16 && (M < 12 || nck <= 96)) return 0;
+  const int n = ceil_div(nck, per);
+  return n > 32 || ceil_div(tiles, 256 / n) > 64 ? 0 : n;   // (a lane for every tile's ticket)
+}
 
 template <int EPI, bool NORM, bool XI, int MT, bool I8>
 static int pick(const FewRowsParams& p, hipStream_t s) {
@@ -599,10 +629,13 @@ static int pick(const FewRowsParams& p, hipStream_t s) {
       if (nck <= 16) return launch<EPI, false, false, 16, MT, I8, 8, 2, DA>(p, s);
       if (nck <= 33) return launch<EPI, false, false, 16, MT, I8, 11, 3, 3>(p, s);
     }
-    if (tiles > 128) return launch<EPI, false, false, 16, MT, I8, 8, 0, D>(p, s);
     if constexpr (EPI == FEW_STORE || EPI == FEW_RESID) {
-      if (p.ws && p.M >= kSplitFrom && nck > 33) return launch<EPI, false, false, 16, MT, I8, 8, 2, I8 ? 4 : 2, true>(p, s, ceil_div(nck, 16));
+      constexpr int X = I8 ? 2 : 1;
+      const int n = p.ws ? parts(p.M, p.N, p.K) : 0;
+      if (n && nck > kLongPart) return launch<EPI, false, false, 16, MT, I8, 7, 2, 4 * X, true>(p, s, n);
+      if (n) return launch<EPI, false, false, 16, MT, I8, 8, 1, 2 * X, true>(p, s, n);
     }
+    if (tiles > 128) return launch<EPI, false, false, 16, MT, I8, 8, 0, D>(p, s);
     return launch<EPI, false, false, 8, MT, I8, 8, 0, D>(p, s);
   }
 }
@@ -624,10 +657,9 @@ static int norms(const FewRowsParams& p, hipStream_t s) {
 }  // namespace few
 
 int64_t few_rows_workspace(int M, int N, int K, int* tickets) {
-  const int nck = ceil_div(K, few::KC), MT = M <= 16 ? 1 : 2;
-  if (M < few::kSplitFrom || M > FEW_MAX_ROWS || nck <= 33 || N > 2048) return *tickets = 0;
-  *tickets = ceil_div(N, 16) * MT;
-  return (int64_t)*tickets * ceil_div(nck, 16) * 256;
+  const int n = few::parts(M, N, K);
+  *tickets = n ? ceil_div(N, 16) * (M <= 16 ? 1 : 2) : 0;
+  return (int64_t)*tickets * n * 256;
 }
 
 int few_rows_launch(int epi, const FewRowsParams& p, hipStream_t s) {

@@ -57,7 +57,7 @@ _ATTN_OPROJ_MAXB = int(os.environ.get("NXD_DECODE_ATTN_OPROJ_MAXB", "2"))
 _EMB_FUSED = os.environ.get("NXD_DECODE_EMB_FUSED", "1") == "1"
 # Limits of the matrix-core projections (csrc/few_rows.hip): rows, width of a norm's rows, bytes of a weight matrix; counters for
 # any of its split reductions
-_FEW_ROWS, _FEW_NORM_WIDTH, _FEW_WEIGHT_BYTES, _FEW_TICKETS = 32, 4224, 2 ** 31, 256
+_FEW_ROWS, _FEW_NORM_WIDTH, _FEW_WEIGHT_BYTES, _FEW_TICKETS = 32, 4224, 2 ** 31, 1024
 
 
 class DecoderInferenceMixin:

@@ -107,7 +107,7 @@ FEW_TOKENS, FEW_ROWS = 64, 16
 
 
 # rows up to which linear_few takes a product, and counters that serve any of its calls
-LINEAR_ROWS, LINEAR_TICKETS = 32, 256
+LINEAR_ROWS, LINEAR_TICKETS = 32, 1024
 _LINEAR_EPI = {"store": 0, "f32": 4, "relu2": 5}
 
 

@@ -144,3 +144,34 @@ def test_rows_of_a_view_and_unaligned_outputs():
     ops.ext().dgemv(0, x, None, 0.0, w, y[:, 1:52], 0, 0, 0, None, None, None, 1, None, None, None)
     _close(y[:, 1:52], _exact(x, None, w, None))
     assert not y[:, 0].any() and not y[:, 52].any()
+
+
+@pytest.mark.parametrize("int8", [False, True])
+@pytest.mark.parametrize("M,N,K", [
+    (12, 40, 4368), (13, 2048, 9216), (9, 24, 9232), (9, 2048, 12288),            # up to 128 tiles, both lengths of parts
+    (12, 4096, 12432), (17, 2064, 4368), (32, 4096, 11008), (19, 8200, 14336),    # more of them, two tiles of rows
+])
+def test_split_reductions(M, N, K, int8):
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+    w, s = _weights(N, K, int8, gen)
+    x = torch.randn(M, K, generator=gen, device="cuda").bfloat16()
+    y0 = torch.randn(M, N, generator=gen, device="cuda").bfloat16()
+    want = _exact(x, None, w, s)
+    tickets = torch.zeros(1024 + 2, dtype=torch.int32, device="cuda")
+    run = lambda y, e, t: ops.ext().dgemv(e, x, None, 0.0, w, y, 0, 0, 0, None, None, None, 1, None, None, None, wscale=s, tickets=t)
+    outs = []
+    for t in (tickets[:1024], tickets[:1024], tickets[:1]):   # (too few counters: not split)
+        y = y0.clone()
+        run(y, 1, t)
+        outs.append(y)
+        _close(y, y0.double() + want)
+    assert torch.equal(outs[0], outs[1]) and not tickets.any()
+    graph = torch.cuda.CUDAGraph()
+    y = y0.clone()
+    with torch.cuda.graph(graph):
+        run(y, 1, tickets[:1024])
+    for _ in range(3):
+        y.copy_(y0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, outs[0]) and not tickets.any()
