@@ -51,8 +51,8 @@ __device__ __forceinline__ int row_of(const FewRowsParams& p, int tile, int r) {
   return min(tile * R + r, p.N - 1);
 }
 
-// Geometry of a workgroup: NW waves that stream weights and FW that finish tiles; R weight rows a tile; M in MT tiles of
-// 16 rows; D stages of a wave under way; CW chunks of the reduction a wave, their activations held in registers for
+// Geometry of a workgroup: NW waves that stream weights and FW that finish tiles; R weight rows a tile; MT tiles of 16
+// activation rows (the grid's second dimension has the rest of M); D stages of a wave under way; CW chunks of the reduction a wave, their activations held in registers for
 // all tiles (0: any number, activations streamed beside the weights)
 template <int R, int MT, bool I8, int NW, int CW, int D>
 struct Shape {
@@ -111,8 +111,8 @@ struct Finish {
   float cs[4], sn[4], scale[4];
   int64_t at, slot;
 
-  __device__ __forceinline__ Finish(const FewRowsParams& p_, int lane_, int t)
-      : p(p_), lane(lane_), q(lane_ >> 4), m(min(16 * t + (lane_ & 15), p_.M - 1)), half(p_.D / 2), live(16 * t + (lane_ & 15) < p_.M),
+  __device__ __forceinline__ Finish(const FewRowsParams& p_, int lane_, int m0)
+      : p(p_), lane(lane_), q(lane_ >> 4), m(min(m0 + (lane_ & 15), p_.M - 1)), half(p_.D / 2), live(m0 + (lane_ & 15) < p_.M),
         wide(p_.ldy % 4 == 0 && (EPI == FEW_F32 ? (uintptr_t)p_.yf % 16 : (uintptr_t)p_.y % 8) == 0),
         wide_c(EPI == FEW_ROPE_KV && (p_.c_sb | p_.c_sh | p_.c_sl) % 4 == 0 && ((uintptr_t)p_.kc | (uintptr_t)p_.vc) % 8 == 0) {
     if (EPI == FEW_ROPE_KV) {
@@ -258,7 +258,7 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
   f32x4_t* part = reinterpret_cast<f32x4_t*>(smem + S::RING);       // [NW][MT][64]
   float* sq = reinterpret_cast<float*>(smem + S::RING + S::PART);   // [NW][16 MT]
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int c = lane & 15, q = lane >> 4;
+  const int c = lane & 15, q = lane >> 4, m0 = SPLIT ? 0 : blockIdx.y * 16 * MT;   // its first row
   static_assert(!SPLIT || (CW > 0 && !NORM), "split reductions hold their activations and need no norm");
   const int step = SPLIT ? gridDim.x / p.splits : gridDim.x, tile0 = SPLIT ? blockIdx.x / p.splits : blockIdx.x;
 
@@ -274,7 +274,7 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
     int turn = 0;
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
-      Finish<EPI, NORM, R, I8> f(p, lane, t);
+      Finish<EPI, NORM, R, I8> f(p, lane, 16 * t);
       uint64_t todo = reinterpret_cast<const uint64_t*>(sq)[t];
       for (todo = (uint64_t)__builtin_amdgcn_readfirstlane((int)(todo >> 32)) << 32 | (uint32_t)__builtin_amdgcn_readfirstlane((int)todo);
            todo; todo &= todo - 1, ++turn) {
@@ -294,8 +294,8 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
       meet();
     }
     constexpr int T = MT / S::FW;
-    Finish<EPI, NORM, R, I8> f0(p, lane, (w - NW) * T);
-    Finish<EPI, NORM, R, I8> f1(p, lane, (w - NW) * T + T - 1);
+    Finish<EPI, NORM, R, I8> f0(p, lane, m0 + 16 * (w - NW) * T);
+    Finish<EPI, NORM, R, I8> f1(p, lane, m0 + 16 * ((w - NW) * T + T - 1));
     for (int tile = tile0; tile < tiles; tile += step) {
       if (!SPLIT) {
         f0.fetch(tile);
@@ -357,7 +357,7 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
   uint32_t xrow[MT];   // (element offsets: the rows lie within 4 GB)
   bool xok[MT];
 #pragma unroll
-  for (int t = 0; t < MT; ++t) xrow[t] = input_row<XI>(p, min(16 * t + c, p.M - 1), xok[t]);
+  for (int t = 0; t < MT; ++t) xrow[t] = input_row<XI>(p, min(m0 + 16 * t + c, p.M - 1), xok[t]);
   // element of operand f of a chunk that this lane starts at
   auto kof = [&](int f) { return I8 ? 64 * (f >> 1) + 16 * q + 8 * (f & 1) : 32 * f + 8 * q; };
   auto load_x = [&](u32x4_t (&xv)[MT][4], int chunk) {
@@ -385,8 +385,8 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
         u32x4_t v = xv[t][f];
         if (XI && !xok[t]) v = u32x4_t{0u, 0u, 0u, 0u};
         if (tail && k >= p.K) v = u32x4_t{0u, 0u, 0u, 0u};
-        if (XI && first && p.xcopy && blockIdx.x == 0 && 16 * t + c < p.M && k < p.K)
-          *reinterpret_cast<u32x4_t*>(p.xcopy + (int64_t)(16 * t + c) * p.K + k) = v;
+        if (XI && first && p.xcopy && blockIdx.x == 0 && m0 + 16 * t + c < p.M && k < p.K)
+          *reinterpret_cast<u32x4_t*>(p.xcopy + (int64_t)(m0 + 16 * t + c) * p.K + k) = v;
         if (NORM) {
           if (first) ss[t] = dot8_bf16(v, v, ss[t]);
           float a[8], b[8];
@@ -581,7 +581,7 @@ static int launch(FewRowsParams p, hipStream_t s, int splits = 1) {
   const int64_t rounds = ceil_div64(tiles, room < 1 ? 1 : room), groups = ceil_div64(tiles, rounds);
   if (SPLIT && rounds > 64) return -2;   // (a lane for every tile's ticket)
   p.splits = splits;
-  hipLaunchKernelGGL(f, dim3((unsigned)(groups * splits)), dim3((NW + S::FW) * 64), lds, s, p, (int)tiles);
+  hipLaunchKernelGGL(f, dim3((unsigned)(groups * splits), (unsigned)(SPLIT ? 1 : ceil_div(p.M, 16 * MT))), dim3((NW + S::FW) * 64), lds, s, p, (int)tiles);
   return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
@@ -602,6 +602,9 @@ static int launch(FewRowsParams p, hipStream_t s, int splits = 1) {
 //     16.5 in parts of 1792 (of 1024 15.0 / 15.5 / 18.8: more parts to add up, more tiles a workgroup); 4096 x 14336 at 9 / 13 /
 //     32 24.1 / 26.5 / 38.7 -> 24.4 / 24.5 / 29.2; 4096 x 11008 19.2 / 21.0 / 30.1 -> 21.0 / 21.3 / 25.6; 8192 x 8192 27.6 / 28.9 /
 //     41.9 -> 28.8 / 29.0 / 33.5; 8192 x 28672 at 13 / 32 92 / 142 -> 88 / 102.
+//     Unsplit, up to 128 tiles and above 16 rows, a workgroup takes 16 of the rows only, so that every CU has one: 2048 x
+//     2048 at 17 / 32 rows 5.8 / 7.1 -> 5.9 / 6.1 (int8 6.9 -> 5.3 at 32); with more tiles two would share a CU and its loads
+//     (4096 x 4096 at 32 13.2 -> 18.7).
 //     The parts' sums meet in memory; the last to come adds them up, its waves sharing its tiles (by one wave: 2.5 us more).
 constexpr int kLongPart = 72;   // chunks of the reduction from which parts are long
 
@@ -636,7 +639,8 @@ static int pick(const FewRowsParams& p, hipStream_t s) {
       if (n) return launch<EPI, false, false, 16, MT, I8, 8, 1, 2 * X, true>(p, s, n);
     }
     if (tiles > 128) return launch<EPI, false, false, 16, MT, I8, 8, 0, D>(p, s);
-    return launch<EPI, false, false, 8, MT, I8, 8, 0, D>(p, s);
+    if (MT == 2) return launch<EPI, false, false, 16, 1, I8, 8, 0, 4>(p, s);
+    return launch<EPI, false, false, 8, 1, I8, 8, 0, 4>(p, s);
   }
 }
 

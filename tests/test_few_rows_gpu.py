@@ -175,3 +175,15 @@ def test_split_reductions(M, N, K, int8):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, outs[0]) and not tickets.any()
+
+
+@pytest.mark.parametrize("M", [17, 20, 31, 32])
+@pytest.mark.parametrize("N,K", [(8, 64), (1000, 4224), (2048, 2048), (2049, 136)])   # (the last: both halves by one workgroup)
+def test_rows_in_two_halves(M, N, K):
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+    w, _ = _weights(N, K, False, gen)
+    x = torch.randn(M, K, generator=gen, device="cuda").bfloat16()
+    z = _exact(x, None, w, None)
+    _close(ops.linear_few(x, w), z)
+    _close(ops.linear_few(x, w, "relu2"), z.clamp(min=0).square())
+    _close(ops.linear_few(x, w, "f32", alpha=0.5, cap=0.3), 0.3 * torch.tanh(0.5 * z / 0.3), 1e-5)
