@@ -1,4 +1,5 @@
-// Fused decode-step GEMVs (token generation, M <= 8 rows): each projection of a Llama layer is ONE
+// Fused decode-step GEMVs (token generation; 1 and 2 rows, and up to 8 where few_rows.hip does not take
+// the step): each projection of a Llama layer is ONE
 // launch that also does the element-wise work around it, so a decode layer is 5 kernels instead of
 // 10 (reference: examples/inference/modules/attention/attention_base.py:141-170 and
 // model_base.py:388-422 run RMSNorm, QKV, RoPE, the KV-cache scatter, o_proj, the residual adds,

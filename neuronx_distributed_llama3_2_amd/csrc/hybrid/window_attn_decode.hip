@@ -13,33 +13,50 @@
 namespace nxd {
 namespace hybrid {
 
-// bias, RMS norm, rotary turn of one head by one wave; out [D], rounded to the activation type
+// bias, RMS norm, rotary turn of one head by one wave, pairs lane and 64 + lane of its elements; first everything that is
+// read (so that a wave has several heads on their way), then the rest: out [D], rounded to the activation type
+struct HeadIn {
+  float u[2], w[2], nu[2], nw[2], cs[2], sn[2];
+};
 template <typename T>
-__device__ __forceinline__ void prepare_head(const WindowAttnParams& p, const T* x, const float* bias, const float* nw,
-                                             int64_t pt, float* out, float row_r = 0.f) {
+__device__ __forceinline__ HeadIn load_head(const WindowAttnParams& p, const T* x, const float* bias, const float* nw, int64_t pt) {
   const int lane = threadIdx.x & 63, D = p.D, half = p.rot / 2;
-  float u[2], w[2], ss = 0.f;
+  HeadIn in;
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {   // pair lane + 64 i
-    const int d = 2 * (lane + 64 * i);
-    u[i] = d < D ? ld(x + d) + (bias ? bias[d] : 0.f) : 0.f;
-    w[i] = d + 1 < D ? ld(x + d + 1) + (bias ? bias[d + 1] : 0.f) : 0.f;
-    ss += u[i] * u[i] + w[i] * w[i];
+  for (int i = 0; i < 2; ++i) {
+    const int pr = lane + 64 * i, d = 2 * pr, d0 = min(d, D - 1), d1 = min(d + 1, D - 1);
+    in.u[i] = ld(x + d0), in.w[i] = ld(x + d1);
+    if (bias) in.u[i] += bias[d0], in.w[i] += bias[d1];
+    if (nw) in.nu[i] = nw[d0], in.nw[i] = nw[d1];
+    if (half > 0) {
+      const int64_t at = pt * half + min(pr, half - 1);
+      in.cs[i] = p.cos_t[at], in.sn[i] = p.sin_t[at];
+    }
   }
-  const float r = row_r > 0.f ? row_r : (nw ? 1.f / sqrtf(sum64(ss) / (float)D + p.eps) : 1.f);
+  return in;
+}
+template <typename T>
+__device__ __forceinline__ void prepare_head(const WindowAttnParams& p, const HeadIn& in, bool norm, float* out, float row_r = 0.f) {
+  const int lane = threadIdx.x & 63, D = p.D, half = p.rot / 2;
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int d = 2 * (lane + 64 * i);
+    ss += (d < D ? in.u[i] * in.u[i] : 0.f) + (d + 1 < D ? in.w[i] * in.w[i] : 0.f);
+  }
+  const float r = row_r > 0.f ? row_r : (norm ? 1.f / sqrtf(sum64(ss) / (float)D + p.eps) : 1.f);
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int pr = lane + 64 * i, d = 2 * pr;
     if (d >= D) continue;
-    float a = u[i] * r, c = w[i] * r;
-    if (nw) {
-      a *= nw[d];
-      if (d + 1 < D) c *= nw[d + 1];
+    float a = in.u[i] * r, c = d + 1 < D ? in.w[i] * r : 0.f;
+    if (norm) {
+      a *= in.nu[i];
+      if (d + 1 < D) c *= in.nw[i];
     }
     if (pr < half) {
-      const float cs = p.cos_t[pt * half + pr], sn = p.sin_t[pt * half + pr];
-      const float a2 = a * cs - c * sn;
-      c = c * cs + a * sn;
+      const float a2 = a * in.cs[i] - c * in.sn[i];
+      c = c * in.cs[i] + a * in.sn[i];
       a = a2;
     }
     T t;
@@ -50,6 +67,11 @@ __device__ __forceinline__ void prepare_head(const WindowAttnParams& p, const T*
       out[d + 1] = ld(&t);
     }
   }
+}
+template <typename T>
+__device__ __forceinline__ void prepare_head(const WindowAttnParams& p, const T* x, const float* bias, const float* nw,
+                                             int64_t pt, float* out, float row_r = 0.f) {
+  prepare_head<T>(p, load_head(p, x, bias, nw, pt), nw != nullptr, out, row_r);
 }
 
 // 1 / sqrt(mean of squares + eps) of n elements, by every wave for itself
@@ -391,14 +413,25 @@ __global__ void __launch_bounds__(256) attn_decode_kernel(WindowAttnParams p) {
       rq = row_rms(row, p.H * D, p.eps);
       if (owner) rk = row_rms(row + qk0, p.G * D, p.eps);
     }
-    for (int job = w; job < (owner ? NJ + MAPS + 1 : NJ); job += 4) {
-      if (job < NJ) {
-        const int64_t o = ((int64_t)h0 * MAPS + job) * D;
-        prepare_head<T>(p, row + o, p.bias ? p.bias + o : nullptr, POOL && p.norm_all ? p.qn_w + o : p.qn_w, pt, q[job], rq);
-      } else if (job < NJ + MAPS) {
-        const int64_t o = qk0 + ((int64_t)g * MAPS + job - NJ) * D;
-        prepare_head<T>(p, row + o, p.bias ? p.bias + o : nullptr, POOL && p.norm_all ? p.kn_w + (int64_t)g * D : p.kn_w, pt,
-                        kn[job - NJ], rk);
+    // heads w, w + 4, ... of the queries, then the new key's maps and the new value; all are on their way before the first
+    // is used (16 sequences: 28.6 -> 27.2 us with 4 heads a workgroup)
+    constexpr int JOBS = (NJ + MAPS + 4) / 4;
+    HeadIn in[JOBS];
+    auto norm_of = [&](int job) { return job < NJ ? p.qn_w : p.kn_w; };
+#pragma unroll
+    for (int i = 0; i < JOBS; ++i) {
+      const int job = w + 4 * i;
+      if (job >= (owner ? NJ + MAPS : NJ)) continue;
+      const int64_t o = job < NJ ? ((int64_t)h0 * MAPS + job) * D : qk0 + ((int64_t)g * MAPS + job - NJ) * D;
+      const int64_t on = POOL && p.norm_all ? (job < NJ ? o : (int64_t)g * D) : 0;
+      in[i] = load_head<T>(p, row + o, p.bias ? p.bias + o : nullptr, norm_of(job) ? norm_of(job) + on : nullptr, pt);
+    }
+#pragma unroll
+    for (int i = 0; i < JOBS; ++i) {
+      const int job = w + 4 * i;
+      if (job >= (owner ? NJ + MAPS + 1 : NJ)) continue;
+      if (job < NJ + MAPS) {
+        prepare_head<T>(p, in[i], norm_of(job) != nullptr, job < NJ ? q[job] : kn[job - NJ], job < NJ ? rq : rk);
       } else {
         const int64_t o = p.v_off + (int64_t)g * V;
         for (int d = lane; d < V; d += 64) {
@@ -602,10 +635,11 @@ static int run_decode(const WindowAttnParams& p, hipStream_t s) {
 void attn_decode_plan(WindowAttnParams& p, int64_t seen) {
   const int rep = p.H / p.G;
   if (p.D % 8 == 0 && p.V % 8 == 0 && p.D <= 128) {
-    // heads share a workgroup's keys once there are enough workgroups without that (16 heads, 1,024 visible
-    // keys, us with 1 / 4 heads a workgroup: 1 sequence 13 / 20, 16 sequences 31 / 25, 32 sequences 49 / 33)
+    // heads share a workgroup's keys once there are enough workgroups without that (16 heads of 64 + 128, two maps,
+    // 1,024 visible keys, us with 1 / 2 / 4 heads a workgroup: 8 sequences 20.1 / 19.2 / -, 16 sequences 30.9 / 25.0 / 27.2,
+    // 32 sequences 48.1 / 37.1 / 34.2; 300 visible keys: 16 sequences 20.2 / 18.8 / 22.5)
     const int64_t all = (int64_t)p.B * p.H;
-    p.share = all >= 256 && rep % 4 == 0 ? 4 : (all >= 128 && rep % 2 == 0 ? 2 : 1);
+    p.share = all >= 512 && rep % 4 == 0 ? 4 : (all >= 128 && rep % 2 == 0 ? 2 : 1);
     // about 512 workgroups, but not more than 8 a group before each has 4 tiles: the merge has its price
     const int64_t tiles = (seen + 63) / 64, groups = (int64_t)p.B * p.H / p.share;
     const int64_t most = tiles / 4 > 8 ? tiles / 4 : (tiles < 8 ? tiles : 8);
