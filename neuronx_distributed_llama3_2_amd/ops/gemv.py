@@ -42,10 +42,13 @@ def skinny_linear(x: torch.Tensor, w: torch.Tensor, scale: Optional[torch.Tensor
     M = x.numel() // K
     Nw = w.shape[0]
     N = Nw // 2 if glu else Nw
-    few = bias is None and w.numel() * w.element_size() < 2 ** 31   # csrc/few_rows.hip takes up to 32 rows of these
+    # what csrc/few_rows.hip takes, up to 32 rows: int8 with a scale or bf16 without, no bias, weights under 2 GB at 32-bit
+    # offsets (rows of a strided weight lie further apart than numel says)
+    few = (bias is None and w.dtype == (torch.bfloat16 if scale is None else torch.int8) and N > 0
+           and w.numel() * w.element_size() < 2 ** 31 and (Nw + 16) * w.stride(0) * w.element_size() < 2 ** 32)
     if use_native(x, w) and M <= (32 if few else 8) and x.dtype == torch.bfloat16 and w.stride(-1) == 1:
         x2 = x.reshape(M, K)
-        if x2.stride(0) % 8 or x2.data_ptr() % 16:
+        if x2.stride(1) != 1 or x2.stride(0) % 8 or x2.stride(0) >= 2 ** 24 or x2.data_ptr() % 16:
             x2 = x2.contiguous()
         epl = 16 if w.dtype == torch.int8 else 8
         if K % epl == 0 and w.data_ptr() % 16 == 0 and w.stride(0) % epl == 0:

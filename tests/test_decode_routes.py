@@ -1,0 +1,37 @@
+"""Which kernel a decode product goes to, where the choice can be seen without a GPU."""
+import types
+
+import pytest
+import torch
+
+from neuronx_distributed_llama3_2_amd.ops import gemv
+
+
+class _Taken(Exception):
+    pass
+
+
+def _refuse(*_):
+    raise _Taken
+
+
+@pytest.mark.parametrize("rows,stride,dtype,few", [
+    (64, 4096, torch.bfloat16, True),
+    (18, 2 ** 26, torch.bfloat16, False),      # rows 128 MB apart: past 32-bit offsets, whatever numel says
+    (12, 2 ** 27, torch.int8, True),
+    (17, 2 ** 27, torch.int8, False),
+    (0, 4096, torch.bfloat16, False),
+])
+def test_rows_far_apart_leave_the_few_rows_kernel(monkeypatch, rows, stride, dtype, few):
+    monkeypatch.setattr(gemv, "use_native", lambda *_: True)
+    monkeypatch.setattr(gemv, "ext", lambda: types.SimpleNamespace(gemv=_refuse))
+    monkeypatch.setattr(gemv, "dequantize_weight", lambda w, s, d: w)
+    monkeypatch.setattr(gemv, "_linear", lambda x, w, b: "library")
+    w = torch.empty(0, dtype=dtype, device="meta").as_strided((rows, 256), (stride, 1))
+    x = torch.empty(9, 256, dtype=torch.bfloat16, device="meta")
+    scale = torch.ones(1, device="meta") if dtype == torch.int8 else None
+    if few:
+        with pytest.raises(_Taken):
+            gemv.skinny_linear(x, w, scale)
+    else:
+        assert gemv.skinny_linear(x, w, scale) == "library"

@@ -1,0 +1,59 @@
+"""Decode products of 9 to 32 rows through the public op: every form of weight and input that it takes, whichever kernel
+or library product serves it, against 64-bit references."""
+import pytest
+import torch
+
+from neuronx_distributed_llama3_2_amd.ops.gemv import skinny_linear
+
+pytestmark = pytest.mark.gpu
+
+
+def _near(got, want, terms, roundings=2):
+    """Single values: `roundings` to bf16 of the result (2^-9 each), and of the weights that a route may round (2^-9 each, at
+    random: six standard deviations of their sum; terms = sum of magnitudes / sqrt(K))."""
+    bound = roundings * 2.0 ** -9 * want.abs() + 6 * 2.0 ** -9 * terms + 1e-6
+    err = (got.double() - want).abs()
+    assert torch.isfinite(got.float()).all() and (err <= bound).all(), float((err - bound).max())
+    assert float((got.double() - want).norm() / want.norm()) < 6 * 2.0 ** -9
+
+
+def _weight(kind, Nw, K, gen):
+    if kind.startswith("int8"):
+        w = torch.randint(-128, 128, (Nw, K), generator=gen, device="cuda", dtype=torch.int8)
+        scale = {"int8": None, "int8-one": torch.full((1,), 3e-4, device="cuda"),
+                 "int8-row": torch.rand(Nw, 1, generator=gen, device="cuda") * 3e-4 + 1e-5}[kind]
+        return w, scale, w.double() * (1.0 if scale is None else scale.double())
+    w = (torch.randn(Nw, 2 * K, generator=gen, device="cuda") * 0.02).bfloat16()
+    w = w[:, K // 2 // 8 * 8:][:, :K] if kind == "bf16-strided" else w[:, :K].contiguous()
+    return w, torch.ones(1, device="cuda") if kind == "bf16-scale" else None, w.double()
+
+
+@pytest.mark.parametrize("glu", [False, True])
+@pytest.mark.parametrize("kind", ["int8", "int8-one", "int8-row", "bf16", "bf16-scale", "bf16-strided"])
+@pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 32])
+@pytest.mark.parametrize("N,K", [(40, 256), (520, 4368)])
+def test_skinny_linear_takes_every_form(M, N, K, kind, glu):
+    gen = torch.Generator(device="cuda").manual_seed(M + N)
+    w, scale, wd = _weight(kind, 2 * N if glu else N, K, gen)
+    x = torch.randn(M, K, generator=gen, device="cuda").bfloat16()
+    if kind == "int8":
+        x *= 2.0 ** -10
+    z, terms = x.double() @ wd.t(), x.double().abs() @ wd.abs().t() * K ** -0.5
+    got = skinny_linear(x, w, scale, glu=glu)
+    if not glu:
+        return _near(got, z, terms)
+    a, b = z.chunk(2, -1)
+    ta, tb = terms.chunk(2, -1)
+    # (a and b may be rounded as well; |silu'| < 1.1, |silu(a)| < |a|)
+    _near(got, torch.nn.functional.silu(a) * b, 1.1 * (ta + a.abs()) * b.abs() + a.abs() * (tb + b.abs()) + ta * tb)
+
+
+def test_inputs_in_any_layout():
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    w, _, wd = _weight("bf16", 136, 512, gen)
+    wide = torch.randn(24, 1040, generator=gen, device="cuda").bfloat16()
+    for x in (torch.randn(512, 24, generator=gen, device="cuda").bfloat16().t(), wide[:, 3:515], wide[:, :512], wide[::2, 8:520],
+              wide[:, :512].reshape(4, 6, 512)):
+        z = x.double() @ wd.t()
+        _near(skinny_linear(x, w), z, x.double().abs() @ wd.abs().t() * 512 ** -0.5)
+
