@@ -187,9 +187,10 @@ class DecoderInferenceMixin:
             ok = self._check_decode_fusable()
             self._decode_fused_ok = ok
         M, H = input_ids.numel(), self.config.hidden_size
-        if not ok or not input_ids.is_cuda or self.tp > 1 and M > 8:
+        if not ok or not input_ids.is_cuda:
             return False
-        if self._decode_few_ok and M <= _FEW_ROWS:
+        # (the tensor-parallel step's norm + gate / up product with a pending sum is csrc/decode_fused.hip's at any rows)
+        if self.tp == 1 and self._decode_few_ok and M <= _FEW_ROWS:
             return True
         return not self._decode_int8 and M <= 8 and M * H <= 32768
 

@@ -35,3 +35,17 @@ def test_rows_far_apart_leave_the_few_rows_kernel(monkeypatch, rows, stride, dty
             gemv.skinny_linear(x, w, scale)
     else:
         assert gemv.skinny_linear(x, w, scale) == "library"
+
+
+@pytest.mark.parametrize("tp,rows,width,fused", [
+    (2, 8, 4096, True), (2, 8, 4160, False), (2, 7, 4224, True), (2, 9, 2048, False), (2, 32, 2048, False), (2, 3, 8192, True),
+    (1, 8, 4160, True), (1, 32, 4224, True), (1, 33, 2048, False),
+])
+def test_steps_that_are_fused(tp, rows, width, fused):
+    """A tensor-parallel step has the limits of csrc/decode_fused.hip (8 rows, 32,768 elements of a norm's rows)."""
+    from neuronx_distributed_llama3_2_amd.inference.model_base import DecoderInferenceMixin as Model
+
+    model = types.SimpleNamespace(tp=tp, config=types.SimpleNamespace(hidden_size=width), _decode_fused_ok=True,
+                                  _decode_few_ok=width <= 4224, _decode_int8=False)
+    ids = types.SimpleNamespace(numel=lambda: rows, is_cuda=True)
+    assert Model._decode_fusable(model, ids) is fused
