@@ -231,9 +231,10 @@ class DecoderInferenceMixin:
 
     @classmethod
     def _weight_scale(cls, mod):
-        """(weight, its scale if it is int8) of a projection module."""
+        """(weight, its fp32 scale if it is int8; a cast of the module may have changed the type it is kept in) of a
+        projection module."""
         w = cls._weight_bias(mod)[0]
-        return w, mod._row_scale() if w.dtype == torch.int8 else None
+        return w, mod._row_scale().float() if w.dtype == torch.int8 else None
 
     def _decode_oacc(self, M: int, res: torch.Tensor) -> torch.Tensor:
         """fp32 [8, H] o_proj accumulator of the fused attention + o_proj decode launch: zero between

@@ -49,3 +49,18 @@ def test_steps_that_are_fused(tp, rows, width, fused):
                                   _decode_few_ok=width <= 4224, _decode_int8=False)
     ids = types.SimpleNamespace(numel=lambda: rows, is_cuda=True)
     assert Model._decode_fusable(model, ids) is fused
+
+
+def test_scales_of_int8_weights_are_fp32():
+    """Also after a cast of the whole model, which takes the scales along."""
+    from neuronx_distributed_llama3_2_amd.inference.model_base import DecoderInferenceMixin as Model
+    from neuronx_distributed_llama3_2_amd.quantization.quantization_layers import QuantizedRowParallel
+
+    for kind in ("per_channel_symmetric", "per_tensor_symmetric"):
+        mod = QuantizedRowParallel(32, 48, bias=False, quantization_type=kind, quantization_per_channel_axis=0 if "channel" in kind else None)
+        mod.quantize_from(torch.randn(48, 32))
+        want = mod.scale.reshape(-1)
+        for cast in (torch.bfloat16, torch.float32):
+            w, scale = Model._weight_scale(mod.to(cast))
+            assert w.dtype == torch.int8 and scale.dtype == torch.float32 and scale.is_contiguous()
+            assert torch.allclose(scale, want, rtol=2.0 ** -8)
