@@ -14,6 +14,8 @@
 // operands, and 1 / rms is a factor of the finished sums.  int8 weights are widened exactly (to bf16) on their way from LDS.
 #include "few_rows.h"
 
+#include <atomic>
+
 namespace nxd {
 namespace few {
 
@@ -570,13 +572,16 @@ static int launch(FewRowsParams p, hipStream_t s, int splits = 1) {
   static_assert(lds <= 160 * 1024, "LDS of a workgroup");
   const int64_t tiles = tiles_of<EPI, R>(p);
   auto* f = &kernel<EPI, NORM, XI, R, MT, I8, NW, CW, D, SPLIT>;
-  static const int per = [&] {   // workgroups of a CU
-    int n = 0;
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(f), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, f, (NW + S::FW) * 64, lds) != hipSuccess) return 0;
-    return n;
-  }();
-  if (per < 1) return 1;
+  // workgroups of a CU; the limit on LDS and what follows from it are set once on each device
+  static std::atomic<int> known[16];
+  int dev = 0, per = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return 1;
+  if (dev < 16) per = known[dev].load(std::memory_order_relaxed);
+  if (per < 1) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(f), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return 1;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, f, (NW + S::FW) * 64, lds) != hipSuccess || per < 1) return 1;
+    if (dev < 16) known[dev].store(per, std::memory_order_relaxed);
+  }
   const int64_t room = 256 * (int64_t)per / splits;   // workgroups side by side along the rows
   const int64_t rounds = ceil_div64(tiles, room < 1 ? 1 : room), groups = ceil_div64(tiles, rounds);
   if (SPLIT && rounds > 64) return -2;   // (a lane for every tile's ticket)
