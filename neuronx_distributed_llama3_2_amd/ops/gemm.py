@@ -210,6 +210,8 @@ def wgrad_accumulate_(mg: torch.Tensor, go2: torch.Tensor, x2, go_t: torch.Tenso
         x_t = None
     if x2 is None or (_native(go2, x2) and mg.is_contiguous()):
         if x2 is None or _use_wgrad_t(go2, x2):
+    if go2.shape[0] == 0:
+        return
             # T-contiguous operands: both transposed by the HIP kernel (~5 TB/s) into scratch, then
             # the TN GEMM (1.30-1.44 vs 1.06-1.16 PF/s on the NT layout, profiles/r2_gemm_layouts)
             T, N = go2.shape[0], go2.shape[1]

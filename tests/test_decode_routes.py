@@ -64,3 +64,18 @@ def test_scales_of_int8_weights_are_fp32():
             w, scale = Model._weight_scale(mod.to(cast))
             assert w.dtype == torch.int8 and scale.dtype == torch.float32 and scale.is_contiguous()
             assert torch.allclose(scale, want, rtol=2.0 ** -8)
+
+
+@pytest.mark.parametrize("M,N", [(8, 8), (16384, 2048), (4096, 14336), (64, 4096)])
+def test_a_weight_gradient_over_no_tokens_launches_nothing(monkeypatch, M, N):
+    from neuronx_distributed_llama3_2_amd.ops import gemm
+
+    def refuse(*_):
+        raise AssertionError("launched")
+
+    monkeypatch.setattr(gemm, "_native", lambda *_: True)
+    monkeypatch.setattr(gemm, "ext", refuse)
+    monkeypatch.setattr(gemm, "gemm_ext", refuse)
+    dy, x = (torch.empty(0, n, dtype=torch.bfloat16) for n in (M, N))
+    mg = torch.empty(M, N, device="meta")
+    gemm.wgrad_accumulate_(mg, dy, x)
