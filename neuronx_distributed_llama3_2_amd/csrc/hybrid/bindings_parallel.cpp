@@ -6,6 +6,8 @@
 #include "few_rows.h"
 #include "group_norm.h"
 
+#include <algorithm>
+
 namespace nxd {
 int residual_norms_launch(bool, const GroupNormParams&, bool, hipStream_t);
 int channel_delta_chunk(int);
@@ -325,7 +327,6 @@ void linear_few(Tensor x, Tensor w, Tensor y, int64_t epi, double alpha, double 
   p.N = (int)w.size(0);
   TORCH_CHECK(p.M >= 1 && p.M <= nxd::FEW_MAX_ROWS && p.K >= 8 && p.K % 8 == 0 && p.N >= 1 && x.stride(0) < (1 << 24), "linear_few: 1..32 rows, K a multiple of 8");
   TORCH_CHECK(w.is_contiguous() && w.size(1) == p.K && y.size(0) == p.M && y.size(1) == p.N && x.stride(0) % 8 == 0, "linear_few: shapes");
-  TORCH_CHECK(w.numel() < (1LL << 31) - 16 * w.size(1), "linear_few: weights of 4 GB");
   check_align(x, "x");
   check_align(w, "w");
   check_align(y, "y");
@@ -338,16 +339,25 @@ void linear_few(Tensor x, Tensor w, Tensor y, int64_t epi, double alpha, double 
   p.ldy = y.stride(0);
   p.alpha = (float)alpha;
   p.cap = (float)cap;
-  Tensor ws;
-  int need = 0;
-  const int64_t floats = epi == nxd::FEW_STORE && tickets.has_value() ? nxd::few_rows_workspace(p.M, p.N, p.K, &need) : 0;
-  if (floats && tickets->numel() >= need) {
-    TORCH_CHECK(tickets->scalar_type() == at::kInt && tickets->is_cuda() && tickets->is_contiguous(), "linear_few: int32 tickets");
-    ws = at::empty({floats}, x.options().dtype(at::kFloat));
-    p.ws = ws.data_ptr<float>();
-    p.tickets = tickets->data_ptr<int>();
+  // the kernel's offsets are 32 bits: larger weights go by parts of their rows (a multiple of 16 of up to 2 GB)
+  const int64_t rows = p.N, most = std::max<int64_t>(16, (1LL << 30) / p.K / 16 * 16);
+  for (int64_t n0 = 0; n0 < rows; n0 += most) {
+    nxd::FewRowsParams q = p;
+    q.N = (int)std::min(most, rows - n0);
+    q.w = static_cast<const uint16_t*>(p.w) + n0 * p.K;
+    if (p.yf) q.yf += n0;
+    else q.y += n0;
+    Tensor ws;
+    int need = 0;
+    const int64_t floats = epi == nxd::FEW_STORE && tickets.has_value() ? nxd::few_rows_workspace(q.M, q.N, q.K, &need) : 0;
+    if (floats && tickets->numel() >= need) {
+      TORCH_CHECK(tickets->scalar_type() == at::kInt && tickets->is_cuda() && tickets->is_contiguous(), "linear_few: int32 tickets");
+      ws = at::empty({floats}, x.options().dtype(at::kFloat));
+      q.ws = ws.data_ptr<float>();
+      q.tickets = tickets->data_ptr<int>();
+    }
+    check_rc(nxd::few_rows_launch((int)epi, q, cur_stream()), "linear_few");
   }
-  check_rc(nxd::few_rows_launch((int)epi, p, cur_stream()), "linear_few");
 }
 
 }  // namespace

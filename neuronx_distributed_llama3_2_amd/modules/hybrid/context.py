@@ -48,7 +48,7 @@ def linear(x: torch.Tensor, mod: torch.nn.Module, fused: bool = False, epilogue:
     from ... import ops
     from ...trace.weight_layout import packed_linear
 
-    if fused and few_rows(x, mod.weight, SOME_ROWS) and mod.weight.numel() < 2 ** 30:
+    if fused and few_rows(x, mod.weight, SOME_ROWS):
         if x.shape[0] <= FEW_ROWS:
             return ops.decode_linear(mod.weight, x, epilogue=epilogue)
         return ops.linear_few(x, mod.weight, epilogue, tickets=tickets)

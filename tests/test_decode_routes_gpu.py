@@ -57,3 +57,27 @@ def test_inputs_in_any_layout():
         z = x.double() @ wd.t()
         _near(skinny_linear(x, w), z, x.double().abs() @ wd.abs().t() * 512 ** -0.5)
 
+
+
+def test_weights_of_4_gb():
+    """linear_few over more weights than 32-bit offsets reach, and the layer's route to it and to the one-row kernel."""
+    from neuronx_distributed_llama3_2_amd import ops
+    from neuronx_distributed_llama3_2_amd.modules.hybrid import context
+
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    w = torch.empty(131240, 16384, dtype=torch.bfloat16, device="cuda")
+    for part in w.split(8192):
+        part.copy_(torch.randn(part.shape, generator=gen, device="cuda") * 0.02)
+    x = torch.randn(9, 16384, generator=gen, device="cuda").bfloat16()
+    rows = torch.cat([torch.arange(a, a + 40) for a in (0, 65520, 131072 - 20, 131200)]).cuda()
+    z, terms = x.double() @ w[rows].double().t(), x.double().abs() @ w[rows].double().abs().t() / 128
+    tickets = torch.zeros(ops.experts.LINEAR_TICKETS, dtype=torch.int32, device="cuda")
+    _near(ops.linear_few(x, w, tickets=tickets)[:, rows], z, terms)
+    assert not tickets.any()
+    _near(ops.linear_few(x, w, "relu2")[:, rows], z.clamp(min=0).square(), 2 * z.abs() * terms + terms.square())
+    f32 = ops.linear_few(x, w, "f32", alpha=0.5)[:, rows]
+    assert float((f32.double() - 0.5 * z).norm() / z.norm()) < 1e-5
+    layer = torch.nn.Module()
+    layer.weight = w
+    for m in (1, 3):
+        _near(context.linear(x[:m].contiguous(), layer, True)[:, rows], z[:m], terms[:m])
