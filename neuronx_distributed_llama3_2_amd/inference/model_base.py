@@ -31,7 +31,7 @@ import torch.distributed as dist
 
 from .. import ops
 from ..ops.gemm import linear as _linear
-from ..ops.gemv import skinny_linear
+from ..ops.gemv import few_rows_pay, skinny_linear
 from ..parallel_layers import parallel_state as ps
 from ..parallel_layers.parallel_state import get_tensor_model_parallel_size
 
@@ -501,7 +501,8 @@ class DecoderInferenceMixin:
             b = None
         scale = mod._row_scale() if w.dtype == torch.int8 else None
         M = x.numel() // x.shape[-1]
-        if w.dtype == torch.int8 or (x.is_cuda and (M <= 8 or M <= _FEW_ROWS and x.dtype == w.dtype == torch.bfloat16 and b is None)):
+        if w.dtype == torch.int8 or (x.is_cuda and (M <= 8 or M <= _FEW_ROWS and x.dtype == w.dtype == torch.bfloat16
+                                                       and b is None and few_rows_pay(M, *w.shape, glu))):
             return skinny_linear(x, w, scale, b, glu=glu)
         from ..trace.weight_layout import packed_linear
 

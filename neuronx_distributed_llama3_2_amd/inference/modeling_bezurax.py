@@ -21,6 +21,7 @@ from ..modules.hybrid import ChannelDelta, ParallelMixer, PooledAttention, Route
 from ..modules.hybrid.context import SOME_ROWS, few_rows, small, step_tickets
 from ..ops.experts import RouterRule
 from ..ops.gemm import linear_f32
+from ..ops.gemv import few_rows_pay
 from ..parallel_layers.parallel_state import get_tensor_model_parallel_size
 from .layer_cache import LayerCache
 from .model_base import DecoderInferenceMixin
@@ -139,7 +140,7 @@ class BezuraxInferenceModel(DecoderInferenceMixin, nn.Module):
         w, scale = self.lm_head.weight, self.config.logit_scale
         if ctx.fused and few_rows(h, w):
             logits = ops.decode_linear(w, h, epilogue="f32", alpha=scale)
-        elif ctx.fused and few_rows(h, w, SOME_ROWS) and w.numel() < 2 ** 30:
+        elif ctx.fused and few_rows(h, w, SOME_ROWS) and few_rows_pay(h.shape[0], *w.shape, True):
             logits = ops.linear_few(h, w, "f32", alpha=scale)
         else:
             logits = linear_f32(h, w, scale)

@@ -22,6 +22,7 @@ from ..modules.hybrid import (DifferentialAttentionMixer, GatedDeltaMixer, Hyper
                               StepContext)
 from ..modules.hybrid.context import SOME_ROWS, few_rows, small, step_tickets
 from ..ops.gemm import linear_f32
+from ..ops.gemv import few_rows_pay
 from ..ops.hyper import FUSED_NORM_ELEMENTS, FUSED_ROWS
 from ..parallel_layers.parallel_state import get_tensor_model_parallel_size
 from .layer_cache import LayerCache
@@ -201,9 +202,10 @@ class GolitarInferenceModel(DecoderInferenceMixin, nn.Module):
         return self._ones_buf
 
     def _logits(self, h: torch.Tensor, fused: bool = False) -> torch.Tensor:
-        if fused and few_rows(h, self.lm_head.weight, SOME_ROWS) and self.lm_head.weight.numel() < 2 ** 30:
-            return ops.linear_few(h, self.lm_head.weight, "f32", cap=self.config.logit_softcap)
-        logits = linear_f32(h, self.lm_head.weight)
+        w = self.lm_head.weight
+        if fused and few_rows(h, w, SOME_ROWS) and few_rows_pay(h.shape[0], *w.shape, True):
+            return ops.linear_few(h, w, "f32", cap=self.config.logit_softcap)
+        logits = linear_f32(h, w)
         return ops.softcap_(logits, self.config.logit_softcap) if self.config.logit_softcap > 0 else logits
 
     def forward_tree(self, *a, **k):

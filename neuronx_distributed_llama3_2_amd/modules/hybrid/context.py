@@ -7,6 +7,8 @@ from typing import Optional
 
 import torch
 
+from ...ops.gemv import few_rows_pay
+
 
 @dataclass
 class StepContext:
@@ -41,6 +43,15 @@ def few_rows(x: torch.Tensor, w: torch.Tensor, limit: int = FEW_ROWS) -> bool:
     return x.is_cuda and x.shape[0] <= limit and x.dtype == w.dtype == torch.bfloat16 and w.shape[1] % 8 == 0 and x.is_contiguous()
 
 
+def streams(rows: int, weight_rows: int, K: int, fused: bool) -> bool:
+    """Whether ops.linear_few is the faster product of up to SOME_ROWS rows.  Up to 16 rows it was taken for the kernel that
+    it replaced; with more, long reductions are split (up to 8,192 weight rows: 0.45-1.18 of the library's time, mostly below 1;
+    12,288 x 8,192 unsplit at 32 rows 57 us, library 47)."""
+    if rows <= 16:
+        return True
+    return weight_rows <= 8192 if K > 4224 else few_rows_pay(rows, weight_rows, K, fused)
+
+
 def linear(x: torch.Tensor, mod: torch.nn.Module, fused: bool = False, epilogue: str = "store",
            tickets: Optional[torch.Tensor] = None) -> torch.Tensor:
     """x [M, K] @ mod.weight^T: through the module's packed copy when the layout pass chose it; fused: a few
@@ -48,7 +59,7 @@ def linear(x: torch.Tensor, mod: torch.nn.Module, fused: bool = False, epilogue:
     from ... import ops
     from ...trace.weight_layout import packed_linear
 
-    if fused and few_rows(x, mod.weight, SOME_ROWS):
+    if fused and few_rows(x, mod.weight, SOME_ROWS) and streams(x.shape[0], *mod.weight.shape, epilogue != "store"):
         if x.shape[0] <= FEW_ROWS:
             return ops.decode_linear(mod.weight, x, epilogue=epilogue)
         return ops.linear_few(x, mod.weight, epilogue, tickets=tickets)

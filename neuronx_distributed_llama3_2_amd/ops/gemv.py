@@ -33,6 +33,22 @@ def dequantize_weight(w: torch.Tensor, scale: Optional[torch.Tensor], dtype=torc
     return (w.float() * s).to(dtype)
 
 
+def few_rows_pay(rows: int, weight_rows: int, K: int, fused: bool = False) -> bool:
+    """Whether a bf16 product of up to 32 rows is faster in csrc/few_rows.hip than in the library's product.  fused: with
+    an element-wise epilogue (SwiGLU, squared ReLU), which the library follows with a launch.
+
+    Up to 8 rows always (the library's time is that of 16).  Up to K = 4,224 the kernel keeps the activations in registers:
+    9 to 16 rows take 0.42-1.01 of the library's time over 256 to 128,256 weight rows; 17 to 32 rows 0.43-1.04 up to K = 2,048,
+    beyond it 0.69-1.01 up to 4,096 weight rows and 24 rows (1.09 at 32) and 0.79-1.01 from 16,384 weight rows on, but 1.01-1.13
+    between (4,096 x 6,144 at 32: 16.9 us, library 15.6).  Longer reductions read them once per workgroup: 8,192 x
+    10,240 at 9 / 16 / 32 rows 33.9 / 40.1 / 56.4 us, library 34.8 / 35.6 / 37.4."""
+    if rows <= 8:
+        return True
+    if K > 4224:
+        return False
+    return rows <= 16 or K <= 2048 or fused or weight_rows >= 16384 or weight_rows <= 4096 and rows <= 24
+
+
 def skinny_linear(x: torch.Tensor, w: torch.Tensor, scale: Optional[torch.Tensor] = None,
                   bias: Optional[torch.Tensor] = None, glu: bool = False) -> torch.Tensor:
     """x [..., K] @ W^T (+ bias) (W bf16 or int8 [Nw, K]); glu=True: W = [gate; up] rows and the
@@ -44,8 +60,9 @@ def skinny_linear(x: torch.Tensor, w: torch.Tensor, scale: Optional[torch.Tensor
     N = Nw // 2 if glu else Nw
     # what csrc/few_rows.hip takes, up to 32 rows: int8 with a scale or bf16 without, no bias, weights under 2 GB at 32-bit
     # offsets (rows of a strided weight lie further apart than numel says)
+    # (int8: the other way is to widen the weights in memory first, 2 to 5 times slower)
     few = (bias is None and w.dtype == (torch.bfloat16 if scale is None else torch.int8) and N > 0
-           and w.numel() * w.element_size() < 2 ** 31 and (Nw + 16) * w.stride(0) * w.element_size() < 2 ** 32)
+           and (w.dtype == torch.int8 or few_rows_pay(M, Nw, K, glu)) and w.numel() * w.element_size() < 2 ** 31 and (Nw + 16) * w.stride(0) * w.element_size() < 2 ** 32)
     if use_native(x, w) and M <= (32 if few else 8) and x.dtype == torch.bfloat16 and w.stride(-1) == 1:
         x2 = x.reshape(M, K)
         if x2.stride(1) != 1 or x2.stride(0) % 8 or x2.stride(0) >= 2 ** 24 or x2.data_ptr() % 16:

@@ -79,3 +79,43 @@ def test_a_weight_gradient_over_no_tokens_launches_nothing(monkeypatch, M, N):
     dy, x = (torch.empty(0, n, dtype=torch.bfloat16) for n in (M, N))
     mg = torch.empty(M, N, device="meta")
     gemm.wgrad_accumulate_(mg, dy, x)
+
+
+@pytest.mark.parametrize("rows,N,K,fused,few", [
+    (8, 64, 28672, False, True), (9, 64, 4224, False, True), (16, 128256, 4224, False, True), (9, 64, 4232, False, False),
+    (32, 128256, 2048, False, True), (17, 6144, 2056, False, False), (32, 16384, 4096, False, True), (24, 4096, 4096, False, True),
+    (25, 4096, 4096, False, False), (32, 8192, 4096, True, True), (32, 8192, 8192, True, False),
+])
+def test_products_that_stream_their_weights(monkeypatch, rows, N, K, fused, few):
+    """9 to 32 rows go to csrc/few_rows.hip only where that is the faster product, in the op and in the unfused step."""
+    from neuronx_distributed_llama3_2_amd.inference import model_base
+
+    assert gemv.few_rows_pay(rows, N, K, fused) is few
+    monkeypatch.setattr(gemv, "use_native", lambda *_: True)
+    monkeypatch.setattr(gemv, "ext", lambda: types.SimpleNamespace(gemv=_refuse))
+    monkeypatch.setattr(gemv, "_linear", lambda x, w, b: torch.empty(x.shape[0], w.shape[0], device="meta"))
+    mod = types.SimpleNamespace(weight=torch.empty(N, K, dtype=torch.bfloat16, device="meta"), bias=None)
+    x = torch.empty(rows, K, dtype=torch.bfloat16, device="meta")
+    if few:
+        with pytest.raises(_Taken):
+            gemv.skinny_linear(x, mod.weight, glu=fused)
+    else:
+        monkeypatch.setattr("neuronx_distributed_llama3_2_amd.ops.activations.swiglu", lambda y: y)
+        assert gemv.skinny_linear(x, mod.weight, glu=fused).shape == (rows, N)
+    taken = []
+    monkeypatch.setattr(model_base, "skinny_linear", lambda *a, **k: taken.append(1))
+    monkeypatch.setattr("neuronx_distributed_llama3_2_amd.trace.weight_layout.packed_linear", lambda *a: x)
+    monkeypatch.setattr(model_base.ops, "swiglu", lambda y: y)
+    on_gpu = type("X", (), {"is_cuda": True, "dtype": torch.bfloat16, "shape": (rows, K), "numel": lambda self: rows * K})()
+    model_base.DecoderInferenceMixin._proj(mod, on_gpu, glu=fused)
+    assert bool(taken) is few
+
+
+@pytest.mark.parametrize("rows,N,K,fused,few", [
+    (16, 12288, 8192, False, True), (17, 8192, 8192, False, True), (32, 8200, 8192, False, False), (32, 8192, 3072, False, False),
+    (32, 8192, 3072, True, True), (17, 2048, 2048, False, True),
+])
+def test_hybrid_projections_that_stream_their_weights(rows, N, K, fused, few):
+    from neuronx_distributed_llama3_2_amd.modules.hybrid.context import streams
+
+    assert streams(rows, N, K, fused) is few
