@@ -704,9 +704,12 @@ void gemv(at::Tensor x, at::Tensor w, c10::optional<at::Tensor> scale, double ts
     TORCH_CHECK(bias->is_contiguous() && bias->numel() == w.size(0), "gemv: bias must be [Nw]");
     bp = bias->data_ptr();
   }
-  // The matrix-core kernel from kFewRows rows on, and for all int8 rows with a scale a row (one row of 16384 x 2048
-  // int8: 13.6 us against 16.7 of the vector kernel)
-  if (!bp && (i8 ? sp != nullptr && tscale == 1.0 : M >= kFewRows && !sp && tscale == 1.0)) {
+  // The matrix-core kernel from kFewRows rows on, and for fewer of int8 with a scale a row where the weights are large: us of
+  // one row here / by the vector kernel 256 x 4096 5.1 / 3.7, 2048 x 2048 4.4 / 4.2, 8192 x 2048 6.9 / 6.0, 16384 x 2048 9.9 / 9.5,
+  // 28672 x 2048 13.4 / 14.6, 4096 x 8192 10.6 / 13.4, 4096 x 14336 14.7 / 21.9, 128256 x 4096 83 / 96; of two rows equal at 4 M weights.
+  const int64_t weights = w.numel();
+  const bool few = M >= kFewRows || i8 && weights >= (M == 2 ? 1 << 22 : K > 2048 ? 1 << 25 : 3 << 24);
+  if (!bp && few && tscale == 1.0 && i8 == (sp != nullptr)) {
     nxd::FewRowsParams f{};
     f.x = static_cast<const uint16_t*>(x.data_ptr());
     f.ldx = x.stride(0);

@@ -81,3 +81,12 @@ def test_weights_of_4_gb():
     layer.weight = w
     for m in (1, 3):
         _near(context.linear(x[:m].contiguous(), layer, True)[:, rows], z[:m], terms[:m])
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 4096, 8192), (1, 4096, 8176), (1, 24576, 2048), (1, 24560, 2048), (2, 2048, 2048), (2, 2032, 2048)])
+def test_few_rows_of_int8(M, N, K):
+    """Both sides of the line between the vector and the matrix-core kernel."""
+    gen = torch.Generator(device="cuda").manual_seed(N)
+    w, scale, wd = _weight("int8-row", N, K, gen)
+    x = torch.randn(M, K, generator=gen, device="cuda").bfloat16()
+    _near(skinny_linear(x, w, scale), x.double() @ wd.t(), x.double().abs() @ wd.abs().t() * K ** -0.5)
