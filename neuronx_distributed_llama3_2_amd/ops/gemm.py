@@ -112,31 +112,46 @@ def _use_wgrad_t(go2: torch.Tensor, x2: torch.Tensor = None, K: int = None) -> b
 # NXD_WGRAD_KERNEL = auto | 1 (whenever the shapes allow) | 0.
 #
 # Token counts that are no multiple of 64 have neither producer copies nor the dense kernel below, and go to this kernel
-# where its 256 x 256 tiles fill the chip (below 128 tiles its splits lose: 3,072 x 2,048 over 3,000 tokens 85 us, library
-# 68) or there are few tokens (over 104: 15 and 41).  Over 1,000 / 3,000 / 8,200 tokens, library with its two transposes ->
-# this kernel, us: 16,384 x 2,048 125 -> 99, 249 -> 212, 597 -> 509; 2,048 x 8,192 72 -> 52, 127 -> 113, 294 -> 249;
-# 128,256 x 2,048 1,078 -> 777, 2,262 -> 1,680, 5,862 -> 4,256; 22,016 x 4,096 363 -> 297, 720 -> 611, 1,570 -> 1,532.  The
-# transposes' share falls as M N / (M + N) grows; measured up to 3,631.  Odd token counts take no transposes: 8-18 % up to
-# 1,001 tokens, 0-7 % at 3,001, slower from 4,001 on.
+# (unsplit from 128 tiles of 256 x 256 on: a second split's atomics cost more than the chip's idle part, 6,144 x 4,096 over 1,000
+# tokens 88 us, in two splits 201, library 99) by how full its rounds of 256 tiles are.  Time of the library with its two
+# transposes = 1: few tokens always (72: 0.39-0.89, 200: 0.50-0.92; 500, from 128 tiles on: 0.76-0.98); rounds three quarters full up
+# to 1,000 (0.75-0.92; at 1,500 0.89-1.07), and from 7/8 at any even count (0.73-0.97 from 224 to 1,576 tiles up to 16,392
+# tokens).  Less full: 128 tiles 1.13 over 1,000, 1.70 over 8,200; 280 tiles 1.22 over 3,000; 96 tiles 1.08 over 500.  Odd
+# counts take no transposes: 0.83-0.95 at 1,001, 0.91-0.98 at 3,071, slower from 4,001 on.  M N / (M + N) measured up to 3,737.
 _WG_KERNEL = os.environ.get("NXD_WGRAD_KERNEL", "auto")
 _WG_SKINNY = 1100.0
 _WG_WIDE = 16000
 _WG_RAGGED = 4000.0
 
 
-def _use_wgrad_kernel(mg: torch.Tensor, go2: torch.Tensor, x2: torch.Tensor, has_copy: bool = False) -> bool:
+def _ragged_tokens(tiles: int, odd: bool) -> int:
+    """Token counts (no multiple of 64) up to which a product of so many tiles goes to the wgrad kernel."""
+    full = tiles / (256 * -(-tiles // 256))
+    if tiles < 128:
+        return 320
+    return 512 if full < 0.75 else 1000 if full < 0.875 else 3072 if odd else 1 << 31
+
+
+def _wgrad_kernel_splits(mg: torch.Tensor, go2: torch.Tensor, x2: torch.Tensor, has_copy: bool = False):
+    """Token splits with which the wgrad kernel takes this product (0: its own choice), None: it does not."""
     if _WG_KERNEL == "0" or x2 is None or not _native(go2, x2) or mg.dtype != torch.float32:
-        return False
+        return None
     T, M = go2.shape
     N = x2.shape[1]
-    if T == 0 or M % 8 or N % 8 or go2.stride(1) != 1 or x2.stride(1) != 1 or mg.stride(1) != 1:
-        return False
+    if M % 8 or N % 8 or go2.stride(1) != 1 or x2.stride(1) != 1 or mg.stride(1) != 1:
+        return None
     if go2.stride(0) % 8 or x2.stride(0) % 8 or go2.data_ptr() % 16 or x2.data_ptr() % 16:
-        return False
-    if T % 64 and not has_copy and (T % 8 == 0 or T <= 3072) and M * N / (M + N) < _WG_RAGGED \
-            and (T <= 320 or -(-M // 256) * -(-N // 256) >= 128):
-        return True
-    return T % 32 == 0 and (_WG_KERNEL == "1" or M * N / (M + N) < _WG_SKINNY or (not has_copy and max(M, N) >= _WG_WIDE))
+        return None
+    if T % 32 == 0 and (_WG_KERNEL == "1" or M * N / (M + N) < _WG_SKINNY or (not has_copy and max(M, N) >= _WG_WIDE)):
+        return 0
+    tiles = -(-M // 256) * -(-N // 256)
+    if T % 64 and not has_copy and M * N / (M + N) < _WG_RAGGED and T <= _ragged_tokens(tiles, T % 8 != 0):
+        return 1 if tiles >= 128 else 0
+    return None
+
+
+def _use_wgrad_kernel(mg: torch.Tensor, go2: torch.Tensor, x2: torch.Tensor, has_copy: bool = False) -> bool:
+    return _wgrad_kernel_splits(mg, go2, x2, has_copy) is not None
 
 
 # The hand-written dense GEMM (csrc/dense_gemm.hip) in its TN form reads the token-major dy / x
@@ -195,12 +210,15 @@ def wgrad_accumulate_(mg: torch.Tensor, go2: torch.Tensor, x2, go_t: torch.Tenso
     into a reused scratch, then an fp32 add (the per-micro-batch weight gradient is rounded to
     bf16 before the fp32 accumulation — the precision of the reference's XLA matmul + fp32
     grad accumulation; hipBLASLt's bf16-output solutions run faster than its fp32-output ones)."""
+    if go2.shape[0] == 0:
+        return
     has_copy = go_t is not None or x_t is not None
     if _use_dense_wgrad(mg, go2, x2, has_copy):
         _dense_wgrad(mg, go2, x2)
         return
-    if _use_wgrad_kernel(mg, go2, x2, has_copy=has_copy):
-        ext().wgrad_gemm(mg, go2, x2, 0, True)
+    splits = _wgrad_kernel_splits(mg, go2, x2, has_copy)
+    if splits is not None:
+        ext().wgrad_gemm(mg, go2, x2, splits, True)
         return
     if x_t is not None and not (x_t.dim() == 2 and x_t.is_contiguous() and x_t.shape[1] == go2.shape[0]):
         x_t = None
@@ -210,8 +228,6 @@ def wgrad_accumulate_(mg: torch.Tensor, go2: torch.Tensor, x2, go_t: torch.Tenso
         x_t = None
     if x2 is None or (_native(go2, x2) and mg.is_contiguous()):
         if x2 is None or _use_wgrad_t(go2, x2):
-    if go2.shape[0] == 0:
-        return
             # T-contiguous operands: both transposed by the HIP kernel (~5 TB/s) into scratch, then
             # the TN GEMM (1.30-1.44 vs 1.06-1.16 PF/s on the NT layout, profiles/r2_gemm_layouts)
             T, N = go2.shape[0], go2.shape[1]

@@ -62,7 +62,9 @@ def test_any_token_count(T, splits, M, N):
 
 @pytest.mark.parametrize("T,M,N,own", [
     (72, 512, 512, True), (301, 512, 512, True), (328, 512, 512, False),       # few tiles: few tokens only
-    (328, 4096, 2048, True), (1001, 4096, 2048, True), (3080, 4096, 2048, True), (3081, 4096, 2048, False),
+    (328, 4096, 2048, True), (504, 4096, 2048, True), (520, 4096, 2048, False),            # half of the chip idle
+    (1000, 6144, 4096, True), (1001, 6144, 4096, False), (1032, 6144, 4096, False),        # a quarter of the rounds
+    (1001, 4096, 4096, True), (3080, 4096, 4096, True), (3071, 4096, 4096, True), (3081, 4096, 4096, False),
     (1000, 8192, 8192, False), (1000, 4096, 2052, False),
 ])
 def test_route_of_ragged_token_counts(T, M, N, own):
@@ -73,5 +75,7 @@ def test_route_of_ragged_token_counts(T, M, N, own):
     mg = torch.randn(M, N, generator=g, device="cuda")
     before = mg.clone()
     assert G._use_wgrad_kernel(mg, dy, x) == (own and G._WG_KERNEL != "0")
+    if own and G._WG_KERNEL != "0":   # unsplit where the tiles can fill the chip
+        assert G._wgrad_kernel_splits(mg, dy, x) == (1 if -(-M // 256) * -(-N // 256) >= 128 else 0)
     G.wgrad_accumulate_(mg, dy, x)
     _check(mg, before, dy, x)
