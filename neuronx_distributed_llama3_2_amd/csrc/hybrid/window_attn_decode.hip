@@ -635,11 +635,15 @@ static int run_decode(const WindowAttnParams& p, hipStream_t s) {
 void attn_decode_plan(WindowAttnParams& p, int64_t seen) {
   const int rep = p.H / p.G;
   if (p.D % 8 == 0 && p.V % 8 == 0 && p.D <= 128) {
-    // heads share a workgroup's keys once there are enough workgroups without that (16 heads of 64 + 128, two maps,
-    // 1,024 visible keys, us with 1 / 2 / 4 heads a workgroup: 8 sequences 20.1 / 19.2 / -, 16 sequences 30.9 / 25.0 / 27.2,
-    // 32 sequences 48.1 / 37.1 / 34.2; 300 visible keys: 16 sequences 20.2 / 18.8 / 22.5)
-    const int64_t all = (int64_t)p.B * p.H;
-    p.share = all >= 512 && rep % 4 == 0 ? 4 : (all >= 128 && rep % 2 == 0 ? 2 : 1);
+    // Heads share a workgroup's keys once there are enough workgroups without that.  Four of them read the keys half as often
+    // as two, which counts once there are many keys; two have fewer registers and more workgroups.  us with 1 / 2 / 4 heads,
+    // 16 heads of 64 + 128 with two maps: 8 sequences of 1,024 visible keys 19.9 / 18.5 / 22.1; 16 of 300 17.5 / 16.4 / 19.2, of 1,024
+    // 30.0 / 24.6 / 25.4, of 4,096 91 / 61 / 51; 24 of 1,024 46 / 35 / 33; 32 of 1,024 48 / 36 / 34.  One map of 128: 16 of 300 15.5 / 13.8 / 15.2, of
+    // 1,024 27.1 / 20.9 / 19.9, 24 of 300 17.6 / 16.4 / 15.9, of 4,096 155 / 95 / 57; pooled blocks (576 keys) 22.0 / 19.7 / 17.9.  Two maps of
+    // 128 + 256: 16 of 1,024 48 / 35 / 52, of 4,096 166 / 93 / 120.
+    const int64_t all = (int64_t)p.B * p.H, keys = all * seen;
+    const bool two = all < 256 || all < 512 && (keys <= (p.maps == 2 ? 1 << 18 : 3 << 15) || p.maps == 2 && p.V > 128);
+    p.share = !two && rep % 4 == 0 ? 4 : (all >= 128 && rep % 2 == 0 ? 2 : 1);
     // about 512 workgroups, but not more than 8 a group before each has 4 tiles: the merge has its price
     const int64_t tiles = (seen + 63) / 64, groups = (int64_t)p.B * p.H / p.share;
     const int64_t most = tiles / 4 > 8 ? tiles / 4 : (tiles < 8 ? tiles : 8);

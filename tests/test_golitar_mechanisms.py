@@ -376,6 +376,26 @@ def test_decode_shares_keys_between_heads(B, H, G):
     assert int(a.tickets.abs().sum()) == 0
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,R,V,window", [
+    (40, 2, 40, 130), (34, 2, 40, 960), (34, 2, 40, 990), (40, 2, 136, 990), (40, 1, 40, 300), (40, 1, 40, 320), (72, 1, 40, 130),
+])
+def test_decode_key_sharing_rule(B, R, V, window):
+    """Both sides of each line at which two or four of a group's heads share a workgroup, against the one-wave-a-query
+    kernel on the same cache."""
+    H, G, T = 8, 2, window + 2
+    a = Attn(("cuda", torch.float32, 5e-5), B, T, H, G, R, 24, V, 8, window, 20.0, cap=T, seed=12)
+    a.step(0, T - 1, True)
+    pos = torch.randint(0, T, (B, 1), generator=torch.Generator().manual_seed(3)).cuda()
+    buf = a.buf[:, T - 1].contiguous()
+    prep = (a.bias.cuda(), a.qn.cuda(), a.kn.cuda(), 1e-5, a.cos.cuda(), a.sin.cuda(), pos)
+    got = ops.attn_decode(buf, a.sz, a.rule, *prep, a.slots, a.kc.clone(), a.vc.clone(), a.tickets)
+    row = buf.clone()
+    ops.attn_prep_(row, B, 1, a.sz, *prep, None, a.slots, a.kc, a.vc)
+    want = ops.window_attention(row, B, 1, a.sz, a.rule, pos, None, a.slots, a.kc, a.vc, False, False)
+    assert rel_err(got, want.cpu()) < 5e-5 and not a.tickets.any()
+
+
 # ------------------------------------------------------------------ fused decode projections
 @pytest.mark.gpu
 @pytest.mark.parametrize("M", [1, 2, 3, 4])
