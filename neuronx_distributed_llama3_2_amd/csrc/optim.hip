@@ -96,11 +96,10 @@ __device__ __forceinline__ uint16_t f2bf_sr(float f, uint32_t seed, int64_t idx)
 // captured optimizer step (hipGraph) replays with the current step's values.
 //
 // Seven streams of memory, 30 bytes a parameter (32-bit gradients, bf16 weights written), nothing else counts.  A workgroup
-// takes 4 x 4 KB of each stream, all its loads in flight before the first is used, stores non-temporally, and ends: 491 M
-// parameters in two launches of 1.69 ms -> 1.44 (4.35 -> 5.1 TB/s; a large copy reaches 4.9).  Of that, 4 vectors a thread
-// instead of one gave 1.50 with 2,048 workgroups that went on from block to block, 8 vectors 1.49, as many workgroups as
-// blocks the rest.
-template <bool GBF16, bool HAS_OUT>
+// takes U x 4 KB of each stream, all its loads in flight before the first is used, stores non-temporally, and ends.  491 M
+// parameters with U = 4: two launches of 1.69 ms -> 1.44 (4.35 -> 5.1 TB/s; a large copy reaches 4.9); 2,048 workgroups that go
+// on from block to block take 1.50.  Which U: see adamw_flat_launch.
+template <bool GBF16, bool HAS_OUT, int U>
 __global__ void __launch_bounds__(256) adamw_kernel(float* __restrict__ p, const void* __restrict__ g, float* __restrict__ m,
                                                     float* __restrict__ v, uint16_t* __restrict__ p16, int64_t n, AdamHyper h,
                                                     const float* __restrict__ gscale_ptr, float gscale_host,
@@ -121,7 +120,6 @@ __global__ void __launch_bounds__(256) adamw_kernel(float* __restrict__ p, const
     const float denom = sqrtf(vv) * rbc2 + h.eps;
     pv = pv * decay - step * mv / denom;
   };
-  constexpr int U = 4;
   const int64_t n4 = n / 4;
   for (int64_t i0 = (int64_t)blockIdx.x * 256 * U; i0 < n4; i0 += (int64_t)gridDim.x * 256 * U) {
     float gf[U][4];
@@ -206,12 +204,18 @@ int adamw_flat_launch(float* p, const void* g, int g_is_bf16, float* m, float* v
   using namespace optim;
   if (n == 0) return 0;
   AdamHyper h{lr, beta1, beta2, eps, wd, bc1, bc2, sr_seed};
-  // a workgroup per 4,096 parameters; past 2^32 of them they go on
-  const int grid = (int)std::min<int64_t>(1 << 20, std::max<int64_t>(1, (n + 4095) / 4096));
-#define AK(B, O) hipLaunchKernelGGL((adamw_kernel<B, O>), dim3(grid), dim3(256), 0, stream, p, g, m, v, (uint16_t*)p16, n, h, gscale_ptr, gscale_host, hyper)
+  // Vectors a thread, by what fills the chip: us with 1 / 2 / 4 (32-bit gradients) 64 K parameters 2.9 / 3.2 / 4.1, 1 M 5.7 /
+  // 5.5 / 5.9, 2 M 9.0 / 7.9 / 7.8, 4 M 19.9 / 19.8 / 20.9, 16 M 73.4 / 72.9 / 75.0, 64 M 382 / 369 / 373; 256 M 1,457 / 1,502 /
+  // 1,493, the boxes' spread.  2,048 workgroups that go on with 1 each: 2.8, 5.7, 9.0, 19.8, 77.0, 423, 1,768.
+  const int u = n < (1 << 21) ? 1 : n < (1 << 26) ? 2 : 4;
+  // a workgroup per block; past 2^32 parameters they go on
+  const int grid = (int)std::min<int64_t>(1 << 20, std::max<int64_t>(1, (n + 1024 * u - 1) / (1024 * u)));
+#define AU(B, O, U) hipLaunchKernelGGL((adamw_kernel<B, O, U>), dim3(grid), dim3(256), 0, stream, p, g, m, v, (uint16_t*)p16, n, h, gscale_ptr, gscale_host, hyper)
+#define AK(B, O) do { if (u == 1) AU(B, O, 1); else if (u == 2) AU(B, O, 2); else AU(B, O, 4); } while (0)
   if (g_is_bf16) { if (p16) AK(true, true); else AK(true, false); }
   else { if (p16) AK(false, true); else AK(false, false); }
 #undef AK
+#undef AU
   return (int)hipGetLastError();
 }
 
