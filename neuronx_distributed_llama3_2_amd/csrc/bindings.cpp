@@ -49,6 +49,7 @@ int embedding_fwd_launch(const int64_t*, const void*, void*, int64_t, int, int64
 int embedding_bwd_launch(const int64_t*, const void*, float*, int64_t, int, int64_t, int64_t, hipStream_t);
 int decode_attn_launch(const void*, const int64_t*, const void*, const void*, const int64_t*, const int*, const int*,
                        float*, float*, float*, int*, void*, const int64_t*, int, int, int, int, int, int, float, hipStream_t, int*);
+void decode_attn_plan(int, int, int, int, int, int, bool, int*);
 int kv_cache_write_launch(const void*, const void*, const int64_t*, void*, void*, const int64_t*, const int*, const int*,
                           int, int, int, int, int, hipStream_t);
 int argmax_launch(const void*, int, int64_t, int, int, int64_t*, hipStream_t);
@@ -1248,6 +1249,13 @@ PYBIND11_MODULE(_C, m) {
   m.def("embedding_bwd", &embedding_bwd);
   m.def("decode_attn", &decode_attn, py::arg("q"), py::arg("k_cache"), py::arg("v_cache"), py::arg("cache_idx"), py::arg("seq_len"),
         py::arg("out"), py::arg("scale"), py::arg("nsplit"), py::arg("tickets") = py::none());
+  // (splits, keys of a split of a sequence of len keys, whether the last split merges) of decode_attn
+  m.def("decode_attn_plan", [](int Lmax, int B, int Hkv, int M, int D, int len, bool tickets) {
+    TORCH_CHECK(Lmax > 0 && B > 0 && Hkv > 0 && M > 0 && M <= 16 && (D == 64 || D == 128) && len <= Lmax, "decode_attn_plan: sizes");
+    int out[3];
+    nxd::decode_attn_plan(Lmax, B, Hkv, M, D, len, tickets, out);
+    return std::make_tuple(out[0], out[1], out[2] != 0);
+  });
   m.def("decode_attn_oproj", &decode_attn_oproj);
   m.def("decode_attn_sync_error", [](bool reset) { return nxd::decode_attn_sync_error(reset); }, py::arg("reset") = false);
   m.def("decode_attn_set_sync", [](int64_t v) { nxd::decode_attn_set_sync((int)v); });

@@ -1,6 +1,6 @@
 // Decode attention on MFMA for small query groups (M = (Hq/Hkv) * T <= 16 rows per kv head):
 // one workgroup of 4 waves (FUSE: 8 at D 64) owns a (batch, kv head, key split); the keys per split
-// (128-1,024, keys_per_split) are sized so the grid reaches ~512 workgroups; every wave runs an
+// (128-1,024, splits_of) are sized so the grid reaches ~512 workgroups; every wave runs an
 // online-softmax flash-decoding loop over 32-key chunks (FUSE: 64) entirely in registers:
 //
 //   S^T[key][m] = K.Q^T   v_mfma_f32_16x16x32_bf16, K rows straight from the cache (16-B loads),
@@ -27,6 +27,7 @@
 // the residual stream with the rounding of the unfused o_proj epilogue and zeroes it.
 #include "common.h"
 
+#include <algorithm>
 #include <cstdlib>
 #include <type_traits>
 
@@ -34,7 +35,19 @@ namespace nxd {
 namespace dattn {
 
 constexpr int KB = 64;            // keys per chunk of a wave with FUSE; splits are multiples of it
-constexpr int KPS = 1024;         // most keys per workgroup split
+constexpr int KPS = 1024;         // most keys per workgroup split (room for more than 64 K keys: more)
+constexpr int WAVES = 4;          // waves of a workgroup without FUSE
+
+// Keys of a split (splits_of): those of a full cache, halved once for a sequence of at most a quarter of its room, again for an
+// eighth, and so on (a few scalar instructions: with divisions, or 64-bit products in their place, every launch took 0.2 us more)
+struct Splits {
+  int room, full, least, most;
+  __host__ __device__ int keys(int slen) const {   // slen <= room
+    const int n = slen > 1 ? slen : 1, a = __builtin_clz(n) - __builtin_clz(room), s = a - 1 - ((uint32_t)n << a > (uint32_t)room);
+    const int k = ((s > 0 ? full >> s : full) + KB - 1) & -KB;
+    return k < least ? least : (k > most ? most : k);
+  }
+};
 
 struct Params {
   const uint16_t* q;
@@ -50,7 +63,8 @@ struct Params {
   float* pm;   // natural-log row max
   float* pl;
   int B, T, Hq, Hkv, nsplit;
-  int kps;            // keys per split (multiple of KB; FUSE: unused)
+  Splits sp;          // keys per split (FUSE: none)
+  int kps;            // SYNC: keys per split (multiple of KB)
   float scale_log2;   // softmax scale * log2(e)
   // weight prefetch riding on the (tiny) attention grid: workgroups >= attn_wgs stream the two
   // byte ranges through the memory hierarchy so the next projections (o_proj, gate_up) find them
@@ -213,9 +227,10 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(Params p) {
   auto load_wo = [&]() { load_wo_regs(p, row0, hkv * G * D + 32 * seg, rpp, wreg); };
   if constexpr (FUSE && !WO_LATE) load_wo();   // round-3 order (A/B: NXD_DECODE_WO_LATE=0)
   const int cb = p.cache_idx ? p.cache_idx[b] : b;
-  const int slen = p.seq_len[b];
+  const int slen = FUSE ? p.seq_len[b] : min(p.seq_len[b], p.sp.room);
+  const int kps = FUSE ? p.kps : p.sp.keys(slen);
   // splits that have keys; with tickets the others leave (a sequence without keys has one, which writes zeros)
-  const int live = !FUSE && p.tickets ? max(1, min(p.nsplit, (slen + p.kps - 1) / p.kps)) : 0;
+  const int live = !FUSE && p.tickets ? max(1, min(p.nsplit, ceil_div(slen, kps))) : 0;
   if (!FUSE && p.tickets && split >= live) return;
   const uint16_t* kbase = p.kc + (int64_t)cb * p.c_sb + (int64_t)hkv * p.c_sh;
   const uint16_t* vbase = p.vc + (int64_t)cb * p.c_sb + (int64_t)hkv * p.c_sh;
@@ -239,7 +254,7 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(Params p) {
   for (int i = 0; i < NDT; ++i) o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
   // FUSE: the whole cache in one pass per workgroup (no key splits, no merge launch)
-  const int kend = (FUSE && !SYNC) ? slen : min(slen, (split + 1) * p.kps);
+  const int kend = (FUSE && !SYNC) ? slen : min(slen, (split + 1) * kps);
   // K fragments and the V chunk of the NEXT chunk are loaded while this one runs its softmax and P.V
   u32x4_t kf[KT][NS], vv[VL];
   auto load_chunk = [&](int k0) {
@@ -256,7 +271,7 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(Params p) {
       for (int s = 0; s < NS; ++s) kf[kt][s] = *reinterpret_cast<const u32x4_t*>(kr + 32 * s);
     }
   };
-  int k0 = split * p.kps + wid * KC;
+  int k0 = split * kps + wid * KC;
   if (k0 < kend) load_chunk(k0);
   // FUSE: the Wo block is issued AFTER the q and first K / V loads.  vmcnt retires in issue order:
   // issued first (round 3), the cold-HBM Wo loads had to land before the first score MFMA could
@@ -264,7 +279,7 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(Params p) {
   // hidden behind it (attention + o_proj 7.16 -> 6.92 us, 0.619 -> 0.614 ms/token alternating, profiles/r4_decode_wo_late_ab.txt).
   if constexpr (FUSE && WO_LATE) load_wo();
   for (; k0 < kend; k0 += NWV * KC) {
-    // ---- scores S^T[key][m] for 4 key tiles of 16
+    // ---- scores S^T[key][m] for key tiles of 16
     f32x4_t sc[KT];
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt) {
@@ -547,21 +562,35 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(Params p) {
   if (p.trace != nullptr && tid == 0) p.trace[2 * blockIdx.x + 1] = __builtin_amdgcn_s_memrealtime();
 }
 
-// Keys per split: enough splits that the (batch, kv head, split) grid reaches ~NXD_DECODE_ATTN_WGS workgroups (default
-// 512: two a CU, so that one's loads cover the other's arithmetic), between 128 keys (one pass of 4 waves; the caller's
-// partial buffers hold Lmax / 128 splits) and 1,024.  Targets of 128 / 256 / 512 / 1,024: 11.4 / 9.9 / 8.8 / 9.8 us for 6
-// sequences of up to 1,024 keys of 8 heads of 64; 20.3 / 18.6 / 19.5 / 21.4 for 13 of up to 1,500 of 8 of 128; the same
-// within 3 % for 1 and 4 sequences; 24.2 / 25.3 at 512 / 1,024 for 32 of up to 2,048.
-static int keys_per_split(int Lmax, int B, int Hkv) {
+// Keys of a split of a full cache: as many splits as bring the (batch, kv head, split) grid to ~NXD_DECODE_ATTN_WGS workgroups
+// (default 512: two a CU, so that one's loads cover the other's arithmetic), of 128 keys (one pass of 4 waves; the caller's
+// partial buffers hold Lmax / 128 splits) to 1,024.  Targets of 128 / 256 / 512 / 1,024: 11.4 / 9.9 / 8.8 / 9.8 us for 6 sequences of up
+// to 1,024 keys of 8 heads of 64; 20.3 / 18.6 / 19.5 / 21.4 for 13 of up to 1,500 of 8 of 128; the same within 3 % for 1 and 4
+// sequences; 24.2 / 25.3 at 512 / 1,024 for 32 of up to 2,048.
+// Few heads of a long cache have fewer splits than that, since they have to be added up: 16, or where a head has no more than
+// 256 sums 24 (merged by the last split) or 32.  8,000 keys of 8 heads in 64 / so many, us: 64 wide 18.3 / 12.2 with tickets, 12.6 /
+// 11.9 without; 128 wide 27.5 / 16.0 and 17.8 / 15.8; four new tokens 40.6 / 15.9 and 68 / 20.9; with o_proj 128 wide 36.6 / 29.8,
+// two new tokens 56.6 / 38.8.
+// Short sequences in a large cache: 4 of 350-700 keys take 8.0 us with room for 1,024, 8,192 and 131,072 (9.9 by the share of a
+// full cache), 13 of 750-1,500 19.9 / 20.6 with room for 1,792 / 8,192 (22.6), 8 of 2 heads of 750-1,500 9.1 in 16,384 (13.6).  Where the
+// last split merges and 64 heads fill a quarter of the chip, 512 keys stay together: 16 of 250-500 8.4 us, in splits of 128 8.9.
+static Splits splits_of(int Lmax, int B, int Hkv, int MD, bool tickets) {
   static const int target = [] {
     const char* e = getenv("NXD_DECODE_ATTN_WGS");
     const int v = e ? atoi(e) : 512;
     return v > 0 ? v : 512;
   }();
-  int kps = (int)(((int64_t)Lmax * B * Hkv + target - 1) / target);
-  kps = (kps + KB - 1) / KB * KB;
-  return kps < 128 ? 128 : (kps > KPS ? KPS : kps);
+  const int64_t fill = ceil_div64((int64_t)Lmax * B * Hkv, target);
+  const int n = (int)std::max<int64_t>(std::min<int64_t>(fill, Lmax), ceil_div(Lmax, MD > 256 ? 16 : tickets ? 24 : 32));
+  const int full = std::max(128, (n + KB - 1) / KB * KB);
+  return {Lmax, full, std::min(full, tickets && (int64_t)B * Hkv >= 64 ? 512 : 128), std::max(KPS, ceil_div(Lmax, KB * 64) * KB)};
 }
+static int most_splits(const Splits& sp) { return ceil_div(sp.room, std::min(sp.full, sp.most)); }
+
+// Whether the last split merges: its trips to memory (8 splits at a time) come one after another, 0.7-1.2 us each, and a launch of
+// its own takes about 4 us.  In the launch / apart, us: 2 trips 8.5 / 10.0, 3 trips 7.8 / 9.0, 4 trips 9.9 / 11.4 and 12.2 / 13.3, 6 trips
+// 12.2 / 11.5, 8 trips 13.0 / 12.6 and 16.8 / 14.3, 12 trips 14.9 / 13.8, 64 trips (four tokens, 128 wide, 64 splits) 68 / 31.
+static bool merge_in_launch(int MD, const Splits& sp) { return ceil_div(MD, 64 * WAVES) * ceil_div(ceil_div(sp.room, sp.full), 8) <= 4; }
 
 // Split attention's partials -> merged attention row block (bf16-rounded, as the merge kernel's
 // output the o_proj GEMV would read) -> this workgroup's o_proj partial, fp32 atomics into oacc: the
@@ -693,6 +722,15 @@ void decode_attn_set_prefetch(const void* a, int64_t a_bytes, const void* b, int
   dattn::g_pf_wgs = wgs;
 }
 
+// The plan of an attention without o_proj over a cache of Lmax keys: {splits, keys of a split of a sequence of len keys, whether
+// the last split merges}
+void decode_attn_plan(int Lmax, int B, int Hkv, int M, int D, int len, bool tickets, int* out) {
+  const dattn::Splits sp = dattn::splits_of(Lmax, B, Hkv, M * D, tickets);
+  out[0] = dattn::most_splits(sp);
+  out[1] = sp.keys(len);
+  out[2] = tickets && dattn::merge_in_launch(M * D, sp);
+}
+
 // Returns -1 when the shape is not covered (caller falls back to the 128-key-chunk kernel).
 int decode_attn2_launch(const void* q, const int64_t* qs, const void* kc, const void* vc, const int64_t* cs,
                         const int* cache_idx, const int* seq_len, float* po, float* pm, float* pl, void* out,
@@ -709,14 +747,13 @@ int decode_attn2_launch(const void* q, const int64_t* qs, const void* kc, const 
   p.out = (uint16_t*)out; p.o_sb = os[0]; p.o_st = os[1]; p.o_sh = os[2];
   p.po = po; p.pm = pm; p.pl = pl;
   p.B = B; p.T = T; p.Hq = Hq; p.Hkv = Hkv;
-  const int kps = dattn::keys_per_split(Lmax, B, Hkv);
-  p.kps = kps;
-  p.nsplit = (Lmax + kps - 1) / kps;
+  p.sp = dattn::splits_of(Lmax, B, Hkv, M * D, tickets != nullptr);
+  p.nsplit = dattn::most_splits(p.sp);
   p.scale_log2 = scale * 1.4426950408889634f;
   *nsplit_out = p.nsplit;
-  constexpr int nwv = 4;
+  constexpr int nwv = dattn::WAVES;
   const size_t lds = (size_t)nwv * dattn::KB * 64 * 2 + (size_t)2 * nwv * 16 * 4;   // (a chunk of V is 8 KB for both D)
-  p.tickets = tickets;
+  p.tickets = dattn::merge_in_launch(M * D, p.sp) ? tickets : nullptr;
   if (p.tickets) *nsplit_out = 1;   // (nothing left to merge)
   p.attn_wgs = B * Hkv * p.nsplit;
   p.trace = dattn::g_trace;
@@ -783,7 +820,7 @@ int decode_attn_oproj_launch(const void* q, const int64_t* qs, const void* kc, c
   const int maxl = decode_attn_oproj_maxl();
   // past maxl: split attention into the partials, then merge + o_proj (needs the partial buffers:
   // [B * Hkv * ceil(Lmax / 128) * M] rows of D, plus the two stats)
-  const bool split = Lmax > maxl && po != nullptr && dattn::keys_per_split(Lmax, B, Hkv) < Lmax;
+  const bool split = Lmax > maxl && po != nullptr && dattn::most_splits(dattn::splits_of(Lmax, B, Hkv, M * D, false)) > 1;
   if (M > 16 || (D != 64 && D != 128) || (Lmax > maxl && !split) || (G * D) % 32 || ldwo % 8) return -1;
   const int nwv = D == 64 ? 8 : 4;
   const int nt = 64 * nwv, tpr = (G * D) / 32;
@@ -847,7 +884,7 @@ int decode_attn_oproj_launch(const void* q, const int64_t* qs, const void* kc, c
     }
   }
   if (split) {
-    const int kps = dattn::keys_per_split(Lmax, B, Hkv), ns = (Lmax + kps - 1) / kps;
+    const int ns = dattn::most_splits(dattn::splits_of(Lmax, B, Hkv, M * D, false));
     const size_t mlds = (size_t)16 * D * 4 + (size_t)ns * 16 * 4 + (size_t)2 * 16 * D * 4;
     if (mlds > 64 * 1024) return -1;
     int ns2 = 0;
