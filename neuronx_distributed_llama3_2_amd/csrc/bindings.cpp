@@ -1057,7 +1057,13 @@ void dgemv(int64_t epi, at::Tensor x, c10::optional<at::Tensor> norm_w, double e
                 "dgemv: yadd fp32 contiguous [>=M, N]");
     ya = yadd->data_ptr<float>();
   }
-  if ((i8 || M >= kFewRows) && !xa && !ya) {
+  // The matrix-core kernel from 3 rows on, but for 3 of them over few, long weight rows, where its tiles leave the chip idle: us
+  // there / dot products a wave, residual and fp32 epilogues 256 x 4096 5.5, 5.3 / 4.9, 3.9, 512 x 8192 7.5, 7.4 / 6.6, 5.7, 1280 x 14336 14.2,
+  // 14.1 / 13.2, 12.2, 1280 x 28672 25.0 / 22.4, but 768 x 4096 5.6, 5.4 / 6.0, 4.9, 1536 x 28672 25.6, 25.2 / 25.7, 24.7; with a norm 512 x 3072
+  // 7.9 / 7.1, 512 x 4096 8.6 / 7.6, 768 x 4096 8.7 / 8.4, 1024 x 4096 8.7 / 9.7
+  const int64_t wr = w.size(0);
+  const bool waves = M == kFewRows && (nw ? K >= 3072 && wr <= 512 : K >= 4096 && wr <= std::min<int64_t>(1280, 256 + K / 14));
+  if ((i8 || M >= kFewRows && !waves) && !xa && !ya) {
     nxd::FewRowsParams f{};
     f.x = static_cast<const uint16_t*>(x.data_ptr());
     f.ldx = x.stride(0);

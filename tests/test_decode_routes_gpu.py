@@ -90,3 +90,36 @@ def test_few_rows_of_int8(M, N, K):
     w, scale, wd = _weight("int8-row", N, K, gen)
     x = torch.randn(M, K, generator=gen, device="cuda").bfloat16()
     _near(skinny_linear(x, w, scale), x.double() @ wd.t(), x.double().abs() @ wd.abs().t() * K ** -0.5)
+
+
+@pytest.mark.parametrize("N,K", [(512, 4096), (520, 4096), (548, 4096), (552, 4096), (512, 3072), (512, 3064), (1280, 14336), (1288, 14336), (64, 8192)])
+def test_three_rows_of_long_weights(N, K):
+    """Both sides of the line between dot products a wave and the matrix-core kernel, all epilogues but the rotary one."""
+    from neuronx_distributed_llama3_2_amd import ops
+
+    gen = torch.Generator(device="cuda").manual_seed(N + K)
+    w, _, wd = _weight("bf16", N, K, gen)
+    x = torch.randn(3, K, generator=gen, device="cuda").bfloat16()
+    z, terms = x.double() @ wd.t(), x.double().abs() @ wd.abs().t() * K ** -0.5
+    rest = (0, 0, 0, None, None, None, 1, None, None, None)
+    y0 = torch.randn(3, N, generator=gen, device="cuda").bfloat16()
+    y = y0.clone()
+    tickets = torch.zeros(1024, dtype=torch.int32, device="cuda")
+    ops.ext().dgemv(1, x, None, 0.0, w, y, *rest, tickets=tickets)
+    _near(y, z + y0.double(), terms + z.abs())
+    assert not tickets.any()
+    yf = torch.empty(3, N, device="cuda")
+    ops.ext().dgemv(0, x, None, 0.0, w, yf, *rest)
+    assert ((yf.double() - z).abs() <= K ** 0.5 * 2.0 ** -22 * terms + 1e-7).all()   # (fp32 sums of K products)
+    if K > 4224:
+        return
+    g = (1 + 0.1 * torch.randn(K, generator=gen, device="cuda")).bfloat16()
+    xn = x.double() * torch.rsqrt(x.double().square().mean(-1, keepdim=True) + 1e-5) * g.double()
+    z, terms = xn @ wd.t(), xn.abs() @ wd.abs().t() * K ** -0.5
+    ops.ext().dgemv(0, x, g, 1e-5, w, y, *rest)
+    _near(y, z, terms)
+    yg = torch.empty(3, N // 2, dtype=torch.bfloat16, device="cuda")
+    ops.ext().dgemv(2, x, g, 1e-5, w, yg, *rest)
+    a, b = z.chunk(2, -1)
+    ta, tb = terms.chunk(2, -1)
+    _near(yg, torch.nn.functional.silu(a) * b, 1.1 * (ta + a.abs()) * b.abs() + a.abs() * (tb + b.abs()) + ta * tb)
