@@ -36,7 +36,8 @@ namespace dattn {
 
 constexpr int KB = 64;            // keys per chunk of a wave with FUSE; splits are multiples of it
 constexpr int KPS = 1024;         // most keys per workgroup split (room for more than 64 K keys: more)
-constexpr int WAVES = 4;          // waves of a workgroup without FUSE
+constexpr int WAVES = 4;          // without FUSE: waves of a workgroup,
+constexpr int CHUNK = 32;         // keys per chunk of a wave
 
 // Keys of a split (splits_of): those of a full cache, halved once for a sequence of at most a quarter of its room, again for an
 // eighth, and so on (a few scalar instructions: with divisions, or 64-bit products in their place, every launch took 0.2 us more)
@@ -194,7 +195,7 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(Params p) {
   static_assert(!SYNC || FUSE, "SYNC is a FUSE form");
   constexpr int NS = D / 32;      // k-steps of the score MFMA
   constexpr int NDT = D / 16;     // 16-wide d tiles of the output
-  constexpr int KC = FUSE ? KB : 32;   // keys of a wave's chunk
+  constexpr int KC = FUSE ? KB : CHUNK;   // keys of a wave's chunk
   constexpr int KT = KC / 16;
   constexpr int VL = KC * D / 512;   // 16-B V loads per lane
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -210,7 +211,10 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(Params p) {
     prefetch_body(p, blockIdx.x - p.attn_wgs, gridDim.x - p.attn_wgs);
     return;
   }
-  if (p.trace != nullptr && tid == 0) p.trace[2 * blockIdx.x] = __builtin_amdgcn_s_memrealtime();
+  auto stamp = [&](int end) {
+    if (p.trace != nullptr && tid == 0) p.trace[2 * blockIdx.x + end] = __builtin_amdgcn_s_memrealtime();
+  };
+  stamp(0);
   const int heads = p.B * p.Hkv;
   const int split = FUSE ? (SYNC ? (int)blockIdx.x % p.R : 0) : (int)blockIdx.x / heads;
   const int bh = FUSE ? (int)blockIdx.x / p.R : (int)blockIdx.x % heads;
@@ -231,7 +235,7 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(Params p) {
   const int kps = FUSE ? p.kps : p.sp.keys(slen);
   // splits that have keys; with tickets the others leave (a sequence without keys has one, which writes zeros)
   const int live = !FUSE && p.tickets ? max(1, min(p.nsplit, ceil_div(slen, kps))) : 0;
-  if (!FUSE && p.tickets && split >= live) return;
+  if (!FUSE && p.tickets && split >= live) return stamp(1);
   const uint16_t* kbase = p.kc + (int64_t)cb * p.c_sb + (int64_t)hkv * p.c_sh;
   const uint16_t* vbase = p.vc + (int64_t)cb * p.c_sb + (int64_t)hkv * p.c_sh;
 
@@ -430,7 +434,7 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(Params p) {
       if (flg[0]) __hip_atomic_store(p.tickets + bh, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     __syncthreads();
-    if (!flg[0]) return;
+    if (!flg[0]) return stamp(1);
     // statistics and sums of 8 splits in flight together
     const int64_t pb = (int64_t)bh * p.nsplit * M;
     auto get = [](const float* a) { return __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
@@ -462,7 +466,7 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(Params p) {
       }
       p.out[(int64_t)b * p.o_sb + (int64_t)tt * p.o_st + (int64_t)(hkv * G + gg) * p.o_sh + d] = f2bf(L > 0.f ? acc / L : 0.f);
     }
-    return;
+    return stamp(1);
   }
   if constexpr (SYNC) {
     int* flg = reinterpret_cast<int*>(red_m);   // [0] lost, [1] merger: red_m is free once the waves are
@@ -559,7 +563,7 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(Params p) {
     __syncthreads();
     oproj_tail<D>(p, reinterpret_cast<const float*>(smem), wreg, b, row0, rpp, tpr, seg, G);
   }
-  if (p.trace != nullptr && tid == 0) p.trace[2 * blockIdx.x + 1] = __builtin_amdgcn_s_memrealtime();
+  stamp(1);
 }
 
 // Keys of a split of a full cache: as many splits as bring the (batch, kv head, split) grid to ~NXD_DECODE_ATTN_WGS workgroups
@@ -752,7 +756,7 @@ int decode_attn2_launch(const void* q, const int64_t* qs, const void* kc, const 
   p.scale_log2 = scale * 1.4426950408889634f;
   *nsplit_out = p.nsplit;
   constexpr int nwv = dattn::WAVES;
-  const size_t lds = (size_t)nwv * dattn::KB * 64 * 2 + (size_t)2 * nwv * 16 * 4;   // (a chunk of V is 8 KB for both D)
+  const size_t lds = (size_t)nwv * dattn::CHUNK * D * 2 + (size_t)2 * nwv * 16 * 4;
   p.tickets = dattn::merge_in_launch(M * D, p.sp) ? tickets : nullptr;
   if (p.tickets) *nsplit_out = 1;   // (nothing left to merge)
   p.attn_wgs = B * Hkv * p.nsplit;
