@@ -946,7 +946,7 @@ void moe_combine_bwd(at::Tensor dout, at::Tensor ys, at::Tensor inv, at::Tensor 
 // Fused decode GEMV (csrc/decode_fused.hip).  epi: 0 plain, 1 residual add into y (in place),
 // 2 SwiGLU on a fused [2N, K] gate/up weight, 3 QKV with RoPE + KV-cache write.  norm_w: RMSNorm
 // of x fused as a prologue.  x [M, K], w [Nw, K], y [M, N] bf16, M <= 8; M <= 32 where csrc/few_rows.hip takes the
-// call (dgemv_rows).  int8 w: wscale [Nw] or [1] fp32.  tickets: zeroed int32 counters (left zeroed) with which a long
+// call.  int8 w: wscale [Nw] or [1] fp32.  tickets: zeroed int32 counters (left zeroed) with which a long
 // reduction may be split over workgroups.
 void dgemv(int64_t epi, at::Tensor x, c10::optional<at::Tensor> norm_w, double eps, at::Tensor w, at::Tensor y,
            int64_t nq, int64_t nkv, int64_t D, c10::optional<at::Tensor> cos_t, c10::optional<at::Tensor> sin_t,
@@ -1221,6 +1221,11 @@ PYBIND11_MODULE(_C, m) {
         py::arg("tickets") = py::none());
   // decode A/B knobs: 0 = GLU row pairs per wave, 1 = GEMV k-slices (0 auto), 2 = MFMA decode attention on/off,
   // 3 = GEMV early epilogue / prologue reads on/off, 5 = bs = 1 GEMV forced occupancy (0 natural | 7 | 8 waves / SIMD)
+  m.def("few_rows_tickets", [](int M, int N, int K) {   // counters with which dgemv and linear_few split a reduction (0: never)
+    int need = 0;
+    nxd::few_rows_workspace(M, N, K, &need);
+    return need;
+  });
   m.def("decode_set_knob", [](int which, int value) {
     if (which == 2) nxd::decode_attn_set_v2(value);
     else if (which == 3) nxd::dgemv_set_knob(2, value);

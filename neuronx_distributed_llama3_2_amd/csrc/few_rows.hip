@@ -602,8 +602,8 @@ static int launch(FewRowsParams p, hipStream_t s, int splits = 1) {
 //     else of 8, so that every CU has one (2048 x 8192 9.5 / 13.0 / 18.8, of 16 rows 11.5 / 15.4 / 20.8).  Streamed, a
 //     workgroup reads all of the activations for its one tile: at 16 rows as much as the tile's weights, or twice that.
 //     So with more rows the reduction is split (`parts`): a workgroup keeps the activations of its part for several tiles.
-//     2048 x 8192 at 9 / 13 / 32 rows 10.7 / 12.2 / 18.9 streamed, 10.9 / 11.2 / 12.8 in parts of 1024 elements (two
-//     workgroups a CU; of 1792, one a CU: 11.7 / 12.0 / 14.6); 2048 x 12288 at 9 / 16 / 32 16.0 / 18.9 / 27.3 -> 13.4 / 14.0 /
+//     2048 x 8192 at 9 / 13 / 32 rows 10.7 / 12.2 / 18.9 streamed, 10.9 / 11.2 / 12.8 in parts of 1024 elements (up to 16
+//     rows two workgroups a CU; of 1792, one a CU: 11.7 / 12.0 / 14.6); 2048 x 12288 at 9 / 16 / 32 16.0 / 18.9 / 27.3 -> 13.4 / 14.0 /
 //     16.5 in parts of 1792 (of 1024 15.0 / 15.5 / 18.8: more parts to add up, more tiles a workgroup); 4096 x 14336 at 9 / 13 /
 //     32 24.1 / 26.5 / 38.7 -> 24.4 / 24.5 / 29.2; 4096 x 11008 19.2 / 21.0 / 30.1 -> 21.0 / 21.3 / 25.6; 8192 x 8192 27.6 / 28.9 /
 //     41.9 -> 28.8 / 29.0 / 33.5; 8192 x 28672 at 13 / 32 92 / 142 -> 88 / 102.

@@ -56,7 +56,7 @@ _ATTN_OPROJ_MAXB = int(os.environ.get("NXD_DECODE_ATTN_OPROJ_MAXB", "2"))
 # per decode step.  NXD_DECODE_EMB_FUSED=0 keeps the separate embedding kernel (A/B).
 _EMB_FUSED = os.environ.get("NXD_DECODE_EMB_FUSED", "1") == "1"
 # Limits of the matrix-core projections (csrc/few_rows.hip): rows, width of a norm's rows, bytes of a weight matrix; counters for
-# any of its split reductions
+# its split reductions of up to 8,192 weight rows (16,384 up to 16 activation rows; longer ones are not split)
 _FEW_ROWS, _FEW_NORM_WIDTH, _FEW_WEIGHT_BYTES, _FEW_TICKETS = 32, 4224, 2 ** 31, 1024
 
 

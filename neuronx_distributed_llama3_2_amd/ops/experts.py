@@ -106,7 +106,8 @@ def expert_linear_rows(x: torch.Tensor, w: torch.Tensor, offs: torch.Tensor, tok
 FEW_TOKENS, FEW_ROWS = 64, 16
 
 
-# rows up to which linear_few takes a product, and counters that serve any of its calls
+# rows up to which linear_few takes a product, and counters for a split reduction of up to 8,192 weight rows (16,384 up
+# to 16 activation rows; with more it is not split)
 LINEAR_ROWS, LINEAR_TICKETS = 32, 1024
 _LINEAR_EPI = {"store": 0, "f32": 4, "relu2": 5}
 
