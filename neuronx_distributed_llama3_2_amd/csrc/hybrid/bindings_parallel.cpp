@@ -18,6 +18,7 @@ int moe_route_launch(const RouterParams&, hipStream_t);
 int clamped_glu_launch(bool, const GluParams&, bool, hipStream_t);
 int gather_rows_launch(const void*, const int*, void*, int64_t, int64_t, int64_t, hipStream_t);
 int experts_few_launch(const RouterParams&, const ExpertFewParams&, hipStream_t);
+int linear_few_launch(const LinearFewParams&, hipStream_t);
 int expert_rows_launch(bool, const ExpertRowsParams&, hipStream_t);
 int grouped_gemm_launch(int, const void*, const void*, void*, const int*, int, int, int, int, int, hipStream_t);
 int grouped_rowgemm_launch(int, const void*, const void*, void*, const int*, int, int, int, int, hipStream_t);
@@ -355,6 +356,15 @@ void linear_few(Tensor x, Tensor w, Tensor y, int64_t epi, double alpha, double 
       ws = at::empty({floats}, x.options().dtype(at::kFloat));
       q.ws = ws.data_ptr<float>();
       q.tickets = tickets->data_ptr<int>();
+    }
+    // The kernel of the experts for 9 to 16 rows whose reduction neither stays in registers nor is split: it reads the rows 16 at a
+    // time beside the weights, where few_rows.hip has all of them in operand order.  us there / here at 9, 12, 16 rows: 4096 x 4352 8.8 /
+    // 9.2, 8.9 / 9.7, 9.8 / 10.3; 5120 x 4352 - / 1.14 of it at 9; 10240 x 5120 22.6 / 23.5, 23.7 / 25.4, 25.2 / 28.1; 2064 x 8192 12.6 / 12.9, 12.7 / 14.2, 13.5 / 15.4; 8192 x 8192 -,
+    // 28.3 / 28.5, 28.3 / 29.4; 16384 x 12288 -, 69.8 / 72.5, 73.8 / 80.4; fewer rows here: 8192 x 8192 at 3 / 6 0.89 / 0.97 of it
+    if (!q.ws && epi == nxd::FEW_STORE && q.M >= 9 && q.M <= 16 && q.K > 4224 && q.N > 2048) {
+      const nxd::LinearFewParams o{q.M, q.N, q.K, q.x, q.ldx, static_cast<const uint16_t*>(q.w), q.y, q.ldy};
+      check_rc(nxd::linear_few_launch(o, cur_stream()), "linear_few");
+      continue;
     }
     check_rc(nxd::few_rows_launch((int)epi, q, cur_stream()), "linear_few");
   }

@@ -1,5 +1,7 @@
-// A whole routed feed-forward of a few tokens (bf16, up to 64) in three launches, without sorting its pairs.
+// A whole routed feed-forward of a few tokens (bf16, up to 64) in three launches, without sorting its pairs; some products of
+// up to 16.
 //
+//   linear_few  : x w^T, up to 16 tokens
 //   moe_gate    : router logits (32-bit) and the chosen experts of one token; the shared expert's gate
 //   expert_few  : gate and up rows -> clamped gated activation times the pair's weight; then the down rows.
 //                 The shared expert is one more expert, which every token uses
@@ -136,6 +138,29 @@ union FewLds {
   }
 };
 
+// y = x w^T (linear_few in bindings_parallel.cpp says when)
+__global__ void __launch_bounds__(FEW_WAVES * 64) linear_few_kernel(LinearFewParams p) {
+  __shared__ __attribute__((aligned(16))) FewLds<1> sums;
+  const int lane = threadIdx.x & 63, lr = lane & 15, lq = lane >> 4, w = threadIdx.x >> 6, row0 = blockIdx.x * 16;
+  FewRows xr;
+#pragma unroll
+  for (int s = 0; s < 4; ++s) xr.at[s] = 4 * s + lq < p.M ? (4 * s + lq) * (int)p.ldx : -1;
+  f32x4_t acc[1];
+  few_product<1>(p.w + (int64_t)row0 * p.K, 0, p.N - row0, p.x, xr, p.K, sums.patch[w], acc);
+  sums.put(acc);
+  const int n = row0 + 4 * lq;
+  if (w > 0 || lr >= p.M) return;
+  const f32x4_t v = sums.get(0);
+  uint16_t* y = p.y + (int64_t)lr * p.ldy + n;
+  if (n + 4 <= p.N && p.ldy % 4 == 0) {
+    st4(y, v);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (n + i < p.N) st(y + i, v[i]);
+  }
+}
+
 // UP: a[pair] = activation of h; else y[slot] = down rows times a[pair]
 template <bool UP>
 __global__ void __launch_bounds__(FEW_WAVES * 64) expert_few_kernel(ExpertFewParams p) {
@@ -215,6 +240,12 @@ int experts_few_launch(const RouterParams& r, const ExpertFewParams& p, hipStrea
   hipLaunchKernelGGL(hybrid::moe_gate_kernel, dim3((unsigned)p.M), dim3(hybrid::GATE_WAVES * 64), 0, s, r, p);
   hybrid::launch_few<true>(p, s);
   hybrid::launch_few<false>(p, s);
+  return hipGetLastError() == hipSuccess ? 0 : 1;
+}
+
+int linear_few_launch(const LinearFewParams& p, hipStream_t s) {
+  if (p.M < 1 || p.M > 16 || p.K % 8) return -1;
+  hipLaunchKernelGGL(hybrid::linear_few_kernel, dim3((unsigned)ceil_div(p.N, 16)), dim3(hybrid::FEW_WAVES * 64), 0, s, p);
   return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 

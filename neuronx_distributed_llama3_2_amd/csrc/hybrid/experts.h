@@ -46,6 +46,15 @@ struct ExpertRowsParams {
 };
 
 // a few tokens (expert_decode.hip)
+struct LinearFewParams {
+  int M, N, K;
+  const uint16_t* x;       // [M, ldx]
+  int64_t ldx;
+  const uint16_t* w;       // [N, K]
+  uint16_t* y;             // [M, ldy]
+  int64_t ldy;
+};
+
 struct ExpertFewParams {
   int M, E, top, shared;   // shared: 1 with a shared expert (else 0)
   int W, F, FS;            // width, feed-forward sizes

@@ -123,3 +123,18 @@ def test_three_rows_of_long_weights(N, K):
     a, b = z.chunk(2, -1)
     ta, tb = terms.chunk(2, -1)
     _near(yg, torch.nn.functional.silu(a) * b, 1.1 * (ta + a.abs()) * b.abs() + a.abs() * (tb + b.abs()) + ta * tb)
+
+
+@pytest.mark.parametrize("M,N,K", [(8, 2064, 4240), (9, 2064, 4240), (16, 2064, 4224), (16, 2063, 4232), (13, 2049, 5120), (16, 2048, 4240), (17, 2064, 4240), (11, 4100, 12296)])
+@pytest.mark.parametrize("split", [False, True])
+def test_unsplit_products_of_nine_to_sixteen_rows(M, N, K, split):
+    """Both sides of each line between linear_few's two kernels; inputs between other columns."""
+    from neuronx_distributed_llama3_2_amd import ops
+
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+    w, _, wd = _weight("bf16", N, K, gen)
+    tickets = torch.zeros(ops.experts.LINEAR_TICKETS, dtype=torch.int32, device="cuda") if split else None
+    for x in (torch.randn(M, K, generator=gen, device="cuda").bfloat16(), torch.randn(M, K + 24, generator=gen, device="cuda").bfloat16()[:, 8:K + 8]):
+        z, terms = x.double() @ wd.t(), x.double().abs() @ wd.abs().t() * K ** -0.5
+        _near(ops.linear_few(x, w, tickets=tickets), z, terms, roundings=1)
+        assert tickets is None or not tickets.any()
