@@ -35,7 +35,7 @@ def padded_rows(n: int) -> int:
 
 
 # rows up to which a projection is a dot product a wave (csrc/hybrid/gemv_hyper.hip), and up to which it is
-# a matrix-core product that streams the weights (csrc/few_rows.hip)
+# a matrix-core product that streams the weights (csrc/few_rows.hip, some in csrc/hybrid/expert_decode.hip)
 FEW_ROWS, SOME_ROWS = 2, 32
 
 
@@ -44,8 +44,8 @@ def few_rows(x: torch.Tensor, w: torch.Tensor, limit: int = FEW_ROWS) -> bool:
 
 
 def streams(rows: int, weight_rows: int, K: int, fused: bool) -> bool:
-    """Whether ops.linear_few is the faster product of up to SOME_ROWS rows.  Up to 16 rows it was taken for the kernel that
-    it replaced; with more, long reductions are split (up to 8,192 weight rows: 0.45-1.18 of the library's time, mostly below 1;
+    """Whether ops.linear_few is the faster product of up to SOME_ROWS rows.  Up to 16 rows it has the faster of two kernels;
+    with more, long reductions are split (up to 8,192 weight rows: 0.45-1.18 of the library's time, mostly below 1;
     12,288 x 8,192 unsplit at 32 rows 57 us, library 47)."""
     if rows <= 16:
         return True

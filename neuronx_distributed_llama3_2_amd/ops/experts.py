@@ -115,9 +115,9 @@ _LINEAR_EPI = {"store": 0, "f32": 4, "relu2": 5}
 def linear_few(x: torch.Tensor, w: torch.Tensor, epilogue: str = "store", alpha: float = 1.0, cap: float = 0.0,
                tickets: Optional[torch.Tensor] = None) -> torch.Tensor:
     """epilogue(x [M, K] w^T) for up to LINEAR_ROWS rows (GPU, bf16, K a multiple of 8): the weights are streamed once
-    (csrc/few_rows.hip).  "store": bf16, "relu2": bf16 squared ReLU, "f32": fp32 alpha y, with cap > 0 cap tanh(alpha y /
-    cap).  tickets: LINEAR_TICKETS zeroed int32 (left zeroed; calls in one stream may share them): a long reduction is
-    split over workgroups where that is faster."""
+    (csrc/few_rows.hip; csrc/hybrid/expert_decode.hip for 9 to 16 long rows).  "store": bf16, "relu2": bf16 squared ReLU,
+    "f32": fp32 alpha y, with cap > 0 cap tanh(alpha y / cap).  tickets: LINEAR_TICKETS zeroed int32 (left zeroed; calls in
+    one stream may share them): a long reduction is split over workgroups where that is faster."""
     y = torch.empty((x.shape[0], w.shape[0]), dtype=torch.float32 if epilogue == "f32" else x.dtype, device=x.device)
     hybrid_ext().linear_few(x, w, y, _LINEAR_EPI[epilogue], float(alpha), float(cap), tickets)
     return y
