@@ -74,7 +74,8 @@ int wgrad_gemm_launch(const void*, int64_t, const void*, int64_t, float*, int64_
 int wgrad_gemm_choose_splits(int, int, int);
 int decode_attn_oproj_launch(const void*, const int64_t*, const void*, const void*, const int64_t*, const int*, const int*,
                              const void*, int64_t, int, float*, float*, float*, float*, float*, int, int, int, int, int, int, float, hipStream_t);
-int grouped_rowgemm_launch(int, const void*, const void*, void*, const int*, int, int, int, int, hipStream_t);
+int grouped_rowgemm_launch(int, const void*, const void*, void*, const int*, int, int, int, int, hipStream_t, float*, int*);
+int64_t grouped_rowgemm_workspace(int, int*);
 int wgrad_gemm_grouped_launch(const void*, int64_t, const void*, int64_t, float*, int64_t, int64_t, const int*, int, int,
                               int, int, hipStream_t);
 void wgrad_gemm_set_ablate(int);
@@ -85,7 +86,6 @@ void decode_attn_set_oproj_maxl(int);
 int decode_attn_oproj_maxl();
 int decode_attn_sync_error(bool);
 void decode_attn_set_sync(int);
-void grouped_rowgemm_set_pp(int);
 void wgrad_gemm_set_pp(int);
 int cu_stream_launch(const void*, void*, int64_t, int, int64_t, hipStream_t);
 int moe_combine_fwd_launch(const void*, const int64_t*, const float*, void*, int64_t, int, int, hipStream_t);
@@ -886,8 +886,16 @@ void grouped_gemm(int64_t mode, at::Tensor a, at::Tensor b, at::Tensor offs, at:
   }();
   if ((mode == 0 || mode == 1) && row_kernel) {
     // 256 x 256 tiles (csrc/grouped_rowgemm.hip); -1 = shape it does not take (reduction % 32)
+    int tickets = 0;
+    const int64_t floats = M > 0 ? nxd::grouped_rowgemm_workspace((int)(mode == 0 ? K : N), &tickets) : 0;
+    at::Tensor ws, counters;
+    if (floats) {
+      ws = at::empty({floats}, a.options().dtype(at::kFloat));
+      counters = at::zeros({tickets}, a.options().dtype(at::kInt));
+    }
     const int rc = nxd::grouped_rowgemm_launch((int)mode, a.data_ptr(), b.data_ptr(), c.data_ptr(),
-                                               offs.data_ptr<int32_t>(), (int)E, (int)M, (int)K, (int)N, cur_stream());
+                                               offs.data_ptr<int32_t>(), (int)E, (int)M, (int)K, (int)N, cur_stream(),
+                                               floats ? ws.data_ptr<float>() : nullptr, floats ? counters.data_ptr<int>() : nullptr);
     if (rc != -1) {
       check_rc(rc, "grouped_gemm (256-tile)");
       return;
@@ -1208,8 +1216,7 @@ PYBIND11_MODULE(_C, m) {
              "cu_stream");
   });
   m.def("wgrad_gemm_set_ablate", [](int64_t v) { nxd::wgrad_gemm_set_ablate((int)v); });
-  // ping-pong (staggered wave-group) main loops of the two hand-written GEMMs, for in-process A/B
-  m.def("grouped_rowgemm_set_pp", [](int64_t v) { nxd::grouped_rowgemm_set_pp((int)v); });
+  // ping-pong (staggered wave-group) main loop of the weight gradients, for in-process A/B
   m.def("wgrad_gemm_set_pp", [](int64_t v) { nxd::wgrad_gemm_set_pp((int)v); });
   m.def("wgrad_gemm_splits", [](int64_t T, int64_t M, int64_t N) { return nxd::wgrad_gemm_choose_splits((int)T, (int)M, (int)N); });
   m.def("moe_combine_fwd", &moe_combine_fwd);

@@ -1,0 +1,202 @@
+// The main loop of the 256 x 256-tile products (grouped_rowgemm.hip): C = A B over a reduction in steps of 64, bf16 operands, fp32 sums.
+//
+// What bounds it is power (2.1 GHz and less under matrix cores that are half busy) and what feeds them: LDS reads, and loads of a CU.
+//   * 4 waves, one a SIMD, of 128 x 128 results each: 64 v_mfma_f32_16x16x32_bf16 for 16 fragments read from LDS, two thirds of what
+//     8 waves of 128 x 64 read -- those read 192 KB a step where LDS gives 128 bytes a clock, as long as the MFMAs take.  The
+//     256 sums of a lane are in AGPRs; the MFMAs are written in asm, because hipcc moves such sums between registers
+//     (216 moves and 124 waits a step of 128 MFMAs: 0.22 PFLOP/s).
+//   * A step's operands are 64 KB of LDS, two steps are there.  The MFMAs of one half of a step (32 of the reduction) are interleaved
+//     with the reads of the next half, four to a read; after the first half a barrier says that the step has been read and the
+//     next one is there, and the loads of the step after that go out between the MFMAs of the second half.
+//   * Loads go straight to LDS, 128 bytes of a row and more: whole lines (with 64 bytes of a row a CU gets 50 GB/s, with 128 it gets 90).
+//   8192 x 8192 x 8192 of random numbers 1.24 PFLOP/s, 8192 x 4096 x 28672 1.38 (of zeros 1.60, 1.53); the ping-pong of two wave groups
+//   that was here before 0.9.
+//
+// Images of a step in LDS, 16-byte chunks XORed so that 16 lanes of a read cover all banks once:
+//   ROW  the reduction is contiguous: [256 rows][64], 128-byte rows
+//   TR   the rows / columns are contiguous: [64][256], 512-byte rows, read with ds_read_b64_tr_b16
+#pragma once
+#include "common.h"
+
+namespace nxd {
+namespace tile {
+
+constexpr int BM = 256, BN = 256, BK = 64, THREADS = 256;
+constexpr int IMG_BYTES = 256 * BK * 2, STEP_BYTES = 2 * IMG_BYTES, LDS_BYTES = 2 * STEP_BYTES;
+
+typedef __attribute__((address_space(3))) short4_t lds_short4_t;
+
+__device__ __forceinline__ void load_lds(uint32_t at, const char* base, uint32_t lds) {   // 64 lanes x 16 B: base + at -> LDS lds + 16 lane
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(at), "s"(base), "s"(lds) : "memory", "m0");
+}
+template <typename T>
+__device__ __forceinline__ T* uniform(T* p) {   // one address for the wave
+  const uint64_t a = reinterpret_cast<uint64_t>(p);
+  return reinterpret_cast<T*>((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(a >> 32)) << 32 | (uint32_t)__builtin_amdgcn_readfirstlane((int)a));
+}
+
+// ROW images: chunk c of a row at c ^ row_swz.  Rows that are read together: 16 in a row, or 4 of every 8 (the columns of a B
+// fragment, below); either way the last bit and row_swz differ in all 16.
+__device__ __forceinline__ int row_swz(int row) { return (row >> 1 & 1) | (row >> 3 & 1) << 1 | ((row >> 2 ^ row >> 4) & 1) << 2; }
+// TR images: chunk c of reduction row t at c ^ tr_swz
+__device__ __forceinline__ int tr_swz(int t) { return 2 * ((t & 3) | (t >> 3 & 1) << 2); }
+
+// Wave (wm, wn) has row fragments i at 32 i + 16 wm (all waves have as much of a tile with few rows) and the columns from 128 wn on.
+// acc[i][j][e] is row 32 i + 16 wm + (lane & 15), column col(j, e): of B in ROW images 8 columns of a lane are contiguous over a pair
+// of fragments, in TR images 4.
+template <bool BT>
+__device__ __forceinline__ int col(int wn, int j, int lane) {
+  const int g = lane >> 4;
+  return 128 * wn + (BT ? 16 * j + 4 * g : 32 * (j >> 1) + 8 * g + 4 * (j & 1));
+}
+
+template <bool AT, bool BT>
+struct Loop {
+  char* smem;
+  int lane, wid, wm, wn;
+  uint32_t lds;
+  uint32_t off[16];        // of this lane's pieces of A (0 .. 7) and B from a step's base
+  const char *pa, *pb;     // the bases of the next step to load
+  int64_t da, db;          // ... and from one step to the next
+  uint32_t back;           // (reductions that end with half a step) pieces of the last step whose second half is past the end, a bit each
+
+  // A: rows 0 .. rows - 1 from `a` on (ROW: a row is lda elements; TR: a reduction row), clamped to the last; B likewise
+  __device__ __forceinline__ Loop(char* smem_, const uint16_t* a, int64_t lda, int rows, const uint16_t* b, int64_t ldb, int cols) : smem(smem_) {
+    lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wid >> 1, wn = wid & 1;
+    lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+    pa = uniform(reinterpret_cast<const char*>(a)), pb = uniform(reinterpret_cast<const char*>(b));
+    da = AT ? (int64_t)BK * lda * 2 : BK * 2, db = BT ? (int64_t)BK * ldb * 2 : BK * 2;
+    back = 0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const bool tr = i < 8 ? AT : BT;
+      const int piece = 8 * wid + (i & 7), n = i < 8 ? rows : cols;
+      const int64_t ld = i < 8 ? lda : ldb;
+      if (tr) {
+        const int t = 2 * piece + (lane >> 5), c = (lane & 31) ^ tr_swz(t);
+        off[i] = (uint32_t)(t * ld + min(8 * c, n - 8)) * 2;
+        if (t >= BK / 2) back |= 1u << i;
+      } else {
+        const int row = 8 * piece + (lane >> 3), c = (lane & 7) ^ row_swz(row);
+        off[i] = (uint32_t)(min(row, n - 1) * ld + 8 * c) * 2;
+        if (c >= 4) back |= 1u << i;
+      }
+    }
+  }
+
+  // the half step's fragment addresses (of the first buffer): ROW: [chunk bit 2], TR: [fragment]
+  int ra[AT ? 8 : 2], rb[BT ? 8 : 2];
+  __device__ __forceinline__ void addresses() {
+    const int r = lane & 15, g = lane >> 4;
+    if constexpr (AT) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) ra[i] = tr_at(32 * i + 16 * wm);
+    } else {
+      const int row = 16 * wm + r;
+      ra[0] = row * 128 + 16 * (g ^ row_swz(row));
+      ra[1] = ra[0] ^ 64;
+    }
+    if constexpr (BT) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) rb[j] = IMG_BYTES + tr_at(128 * wn + 16 * j);
+    } else {
+      const int c = 128 * wn + 8 * (r >> 2) + (r & 3);
+      rb[0] = IMG_BYTES + c * 128 + 16 * (g ^ row_swz(c));
+      rb[1] = rb[0] ^ 64;
+    }
+  }
+  __device__ __forceinline__ int tr_at(int c0) const {   // lane 16 g + 4 q + p: 4 columns from c0 + 4 p on, of reduction rows 8 g + q (and + 4)
+    const int t = 8 * (lane >> 4) + (lane >> 2 & 3), c = c0 + 4 * (lane & 3);
+    return t * 512 + 16 * (c >> 3 ^ tr_swz(t)) + 8 * (c >> 2 & 1);
+  }
+  __device__ __forceinline__ bf16x8_t read_tr(int at) const {
+    const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(smem + at));
+    const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(smem + at + 4 * 512));
+    const short __attribute__((ext_vector_type(8))) v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    return __builtin_bit_cast(bf16x8_t, v);
+  }
+  __device__ __forceinline__ bf16x8_t read_row(int at) const { return __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(smem + at)); }
+  __device__ __forceinline__ bf16x8_t frag_a(int i, int h, int buf) const {
+    if constexpr (AT) return read_tr(ra[i] + buf + h * (IMG_BYTES / 2));
+    else return read_row(ra[h] + buf + i * 4096);
+  }
+  __device__ __forceinline__ bf16x8_t frag_b(int j, int h, int buf) const {
+    if constexpr (BT) return read_tr(rb[j] + buf + h * (IMG_BYTES / 2));
+    else return read_row(rb[h ^ (j & 1)] + buf + (j & 1) * 512 + (j >> 1) * 4096);
+  }
+
+  template <bool HALF>
+  __device__ __forceinline__ void load(int i, int buf, bool last) {   // piece i of the next step; HALF, last: its second half is past the end
+    const uint32_t to = lds + buf + (i < 8 ? 0 : IMG_BYTES) + (8 * wid + (i & 7)) * 1024;
+    uint32_t from = off[i];
+    if constexpr (HALF) {   // (the first half again: not used)
+      const bool tr = i < 8 ? AT : BT;
+      if (last) from -= (back >> i & 1) * (tr ? (uint32_t)((i < 8 ? da : db) / 2) : 64u);
+    }
+    load_lds(from, i < 8 ? pa : pb, to);
+  }
+
+  // acc += the first steps' products.  IM: row fragments that have rows.  HALF, end: the last step has half the reduction.
+  template <int IM, bool HALF>
+  __device__ __forceinline__ void run(f32x4_t (&acc)[8][8], int steps, bool end = false) {
+    static_assert(IM == 8 || IM == 4, "rows");
+    bf16x8_t a0[IM], b0[8], a1[IM], b1[8];
+    auto advance = [&](int s) {   // towards step s
+      if (s < steps) pa += da, pb += db;
+    };
+#pragma unroll
+    for (int i = 0; i < 16; ++i) load<HALF>(i, 0, end && steps == 1);
+    advance(1);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) load<HALF>(i, STEP_BYTES, end && steps <= 2);   // (past the end: the last step again, not used)
+    advance(2);
+    addresses();
+    asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int j = 0; j < 8; ++j) b0[j] = frag_b(j, 0, 0);
+#pragma unroll
+    for (int i = 0; i < IM; ++i) a0[i] = frag_a(i, 0, 0);
+    // chunk u of a half: a read of the next half's, a load, IM / 2 MFMAs
+    auto mfmas = [&](int u, const bf16x8_t (&a)[IM], const bf16x8_t (&b)[8]) {
+#pragma unroll
+      for (int v = 0; v < IM / 2; ++v) {
+        const int m = u * (IM / 2) + v, i = m >> 3, j = m & 7;
+        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(b[j]), "v"(a[i]));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    int buf = 0;
+#pragma unroll 1
+    for (int t = 0, whole = steps - (HALF && end); t < whole; ++t) {
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        if (u < 8) b1[u] = frag_b(u, 1, buf);
+        else if (u - 8 < IM) a1[u - 8] = frag_a(u - 8, 1, buf);
+        mfmas(u, a0, b0);
+      }
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      const int next = buf ^ STEP_BYTES;
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        if (u < 8) b0[u] = frag_b(u, 0, next);
+        else if (u - 8 < IM) a0[u - 8] = frag_a(u - 8, 0, next);
+        load<HALF>(u, buf, end && t + 3 >= steps);
+        mfmas(u, a1, b1);
+      }
+      buf = next;
+      advance(t + 3);
+    }
+    if (HALF && end) {
+#pragma unroll
+      for (int u = 0; u < 16; ++u) mfmas(u, a0, b0);
+    }
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");   // (loads that nothing reads; the last sums)
+  }
+};
+
+}  // namespace tile
+}  // namespace nxd

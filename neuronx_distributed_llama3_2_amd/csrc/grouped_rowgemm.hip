@@ -9,34 +9,22 @@
 // drop); here only the chosen rows are computed.  The weight gradients of the same layer run on the
 // token-major wgrad kernel (csrc/wgrad_gemm.hip, grouped mode).
 //
-// Structure (shared with csrc/wgrad_gemm.hip, cdna_hip_programming.md §5):
-//   * 8 waves (512 threads), 256 x 256 output tile, one workgroup per CU; waves 2 (M) x 4 (N) of
-//     128 x 64 = 8 x 4 v_mfma_f32_16x16x32_bf16 tiles, 128 fp32 accumulators per lane;
-//   * reduction step BK = 32, 4-stage LDS ring (4 x 32 KiB) filled by LDS-DMA (1 KiB lane-linear
-//     pieces, swizzle applied to the source address), counted vmcnt; default main loop = the
-//     ping-pong one (PP below: wave groups staggered by one barrier, +3-9 % over one barrier per
-//     stage, bitwise-identical output, profiles/r3_pp_mainloop_ab.jsonl);
-//   * operands consumed along their contiguous axis (A; DGRAD's B) sit in a [256][32] row image
-//     (64-B rows, 16-B chunk c stored at c ^ g[(row >> 2) & 3], g = {0, 2, 3, 1}: every 16-lane
-//     group of a ds_read_b128 fragment read covers all 64 banks once); FWD's B (reduction along its
-//     rows) sits in a [32][256] image read with ds_read_b64_tr_b16 (as the wgrad kernel);
-//   * row tiles: worst-case count ceil(rows / 256) + E, each workgroup finds (expert, tile) by a
-//     scan of the offsets; the L2 band raster of the wgrad kernel over (row tile, column tile);
-//   * epilogue: per wave, 32-row slabs through padded LDS, bf16 pairs stored 128 B per row per
-//     wave-instruction, rows outside the expert's range masked.
-#include "common.h"
+// Structure: the loop of gemm_tile.h (4 waves, 256 x 256 tile, one workgroup per CU).  A and DGRAD's B are contiguous along the
+// reduction (ROW images), FWD's B along the columns (TR).  Each workgroup finds its (expert, row tile) by a scan of the offsets;
+// the tiles are numbered in an L2 band raster over (row tile, column tile).
+// 8,192 rows of 8 experts, 4096 -> 28672 and 14336 -> 4096, us: FWD 2,170 -> 1,934 and 1,049 -> 943, DGRAD 2,263 -> 1,770 and
+// 1,057 -> 832 (two ping-pong groups of 4 waves, grid of the worst case's tiles).
+#include "gemm_tile.h"
 
 #include <cstdlib>
 
 namespace nxd {
 namespace grg {
 
-constexpr int BM = 256, BN = 256, BK = 32, STAGES = 4, NT = 512;
-constexpr int IMG_BYTES = 256 * BK * 2;            // 16 KiB: one operand stage
-constexpr int STAGE_BYTES = 2 * IMG_BYTES;
-constexpr int LDS_BYTES = STAGES * STAGE_BYTES;    // 128 KiB
-constexpr int PIECES = IMG_BYTES / 1024 / (NT / 64);   // 2 per wave per operand
-constexpr int DMA_PER_STAGE = 2 * PIECES;
+using tile::BK;
+using tile::BM;
+using tile::BN;
+constexpr int NT = tile::THREADS;
 enum Mode { FWD = 0, DGRAD = 1 };
 
 struct Params {
@@ -50,73 +38,46 @@ struct Params {
   int64_t lda, ldb, ldc, b_es;
   int rt, nt;           // worst-case row tiles, column tiles
   int band;
+  // Sums of the tiles left over from whole rounds of an XCD's CUs, their reductions in parts (nullable: never), and zeroed counters
+  // (left zeroed); sizes: grouped_rowgemm_workspace
+  float* ws;
+  int* tickets;
 };
 
-__device__ __forceinline__ int rswz(int row) {   // {0, 2, 3, 1}[(row >> 2) & 3]
-  const int j = (row >> 2) & 3;
-  return (0x78 >> (2 * j)) & 3;                 // 0b01'11'10'00, two bits per j: 0, 2, 3, 1
-}
-__device__ __forceinline__ int row_off(int row, int ch) { return row * 64 + 16 * (ch ^ rswz(row)); }
-__device__ __forceinline__ int tswz(int t) { return 2 * ((t & 3) | (((t >> 3) & 1) << 2)); }
-__device__ __forceinline__ int tr_off(int t, int ch) { return t * 512 + 16 * (ch ^ tswz(t)); }
+constexpr int XCDS = 8, XCD_CUS = 32;
+// Parts of a tile at most; reduction steps of a part at least: writing a part's sums and reading them all back takes 25-40 us, 32
+// steps take 55
+constexpr int MAX_PARTS = 8, MIN_STEPS = 32;
+constexpr int TILE_FLOATS = BM * BN;
 
-typedef __attribute__((address_space(3))) char lds_char_t;
-typedef __attribute__((address_space(3))) short4_t lds_short4_t;
-__device__ __forceinline__ uint32_t lds_addr(const char* q) { return (uint32_t)(uintptr_t)(const lds_char_t*)q; }
 
-__device__ __forceinline__ void dma16(const void* src, uint32_t lds_dst) {
-  uint32_t sv;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
-               : "=&s"(sv) : "v"(src), "s"(lds_dst) : "memory");
-}
-
-// 16x16x32 fragment of rows [r0, r0 + 16) from a row image: lane l -> row r0 + (l & 15), k 8 (l >> 4) .. + 7
-__device__ __forceinline__ bf16x8_t frag_row(const char* img, int r0) {
-  const int l = threadIdx.x & 63;
-  return __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(img + row_off(r0 + (l & 15), l >> 4)));
-}
-// the same fragment of columns [c0, c0 + 16) from a [32 k][256] image (two transposed reads)
-__device__ __forceinline__ bf16x8_t frag_tr(const char* img, int c0) {
-  const int l = threadIdx.x & 63, g = l >> 4, i = l & 15, q = i >> 2, p = i & 3;
-  const int col = c0 + 4 * p;
-  const int t = 8 * g + q;
-  const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(img + tr_off(t, col >> 3) + 8 * (p & 1)));
-  const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(img + tr_off(t + 4, col >> 3) + 8 * (p & 1)));
-  const short __attribute__((ext_vector_type(8))) a8 = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-  return __builtin_bit_cast(bf16x8_t, a8);
-}
-
-// this thread's pieces of the oldest outstanding stage landed (`newer` younger stages left in flight)
-__device__ __forceinline__ void wait_vm(int newer) {
-  if (newer >= 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(DMA_PER_STAGE) : "memory");
-  else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-}
-
-// Measured and not kept (profiles/r3_grouped_rowgemm_variants.jsonl): a 5-stage ring (160 KiB) and
-// s_setprio around the MFMA clusters or for the younger wave half -- all within +-2 %.
-//
-// PP (ping-pong): each 32-deep stage is two phases of 16 MFMAs per wave, every phase
-// [LDS-DMA half-stage][fragment reads] barrier [16 MFMAs at raised priority] barrier, and wave group
-// 1 (waves 4-7; every SIMD holds one wave of each group) runs one barrier behind group 0, so on each
-// SIMD one wave's MFMA burst covers the other wave's reads and DMA issue (cdna_hip_programming.md,
-// "The 256^2 8-phase template").  Ring safety, global barrier instances #n (group 0 passes #(4t+2h)
-// and #(4t+2h+1) in phase (t, h); group 1 one later):
-//   * stage S is read from #(4S-1) on (group 0, phase (S, 0)); both groups retire their pieces of S
-//     before arriving there (group 0 after its MFMAs of (S-1, 1), group 1 before its reads of (S-1, 1));
-//   * the last reads of stage S complete before #(4S+4) (group 1's MFMAs of (S, 1)); its slot is
-//     refilled with S+4 after that: group 1 in (S+1, 0/1), group 0 in (S+1, 1) and (S+2, 0);
-//   * pieces issued after stage S's last: S+1 (4) and S+2's first half (2) -> vmcnt(6), less at the tail.
-// Measured and not kept: the LDS-DMA issued inside the MFMA bursts instead of the load phases
-// (vmcnt(8) / (6) by group) -- 1-5 % slower than this on every MoE / dense shape
-// (profiles/r3_pp_dma_in_mfma_rejected.jsonl).
-template <int MODE, bool PP>
+// HALF: the reduction ends with half a step
+template <int MODE, bool HALF>
 __global__ void __launch_bounds__(NT, 1) rowgemm_kernel(Params p) {
-  __shared__ __attribute__((aligned(16))) char smem[LDS_BYTES];
-  const int id = xcd_remap(blockIdx.x, gridDim.x);
+  __shared__ __attribute__((aligned(16))) char smem[tile::LDS_BYTES];
+  // The tiles that there are (expert by expert), in equal shares for the XCDs (a grid of the worst case's left one with hardly any:
+  // 36 of 40 row tiles x 16).  What is left of a share after whole rounds of 32 CUs is split along the reduction so that the
+  // last round's CUs all have some: 72 tiles a share, 8192 rows of 8 experts x 4096 columns, take 2.25 rounds instead of 3.
+  int real = 0;
+  for (int i = 0; i < p.E; ++i) real += (max(p.offs[i + 1] - p.offs[i], 0) + BM - 1) / BM;
+  const int total = real * p.nt, xcd = blockIdx.x % XCDS, idx = blockIdx.x / XCDS;
+  const int share = total / XCDS + (xcd < total % XCDS), base = xcd * (total / XCDS) + min(xcd, total % XCDS);
+  const int whole = share / XCD_CUS * XCD_CUS, tail = share - whole;
+  const int steps = (p.red + BK - 1) / BK;
+  int parts = 1, part = 0, id = base + idx;
+  if (p.ws && tail > 0) parts = max(1, min(min(XCD_CUS / tail, MAX_PARTS), steps / MIN_STEPS));
+  if (idx >= whole) {
+    const int j = idx - whole;
+    if (j >= tail * parts) return;
+    part = j % parts;
+    id = base + whole + j / parts;
+  } else {
+    parts = 1;
+  }
   int rt, ct;
   {
     const int kb = p.band, bnd = id / (kb * p.nt), rem = id - bnd * kb * p.nt;
-    const int h = min(kb, p.rt - bnd * kb);
+    const int h = min(kb, real - bnd * kb);
     rt = bnd * kb + rem % h;
     ct = rem / h;
   }
@@ -136,182 +97,80 @@ __global__ void __launch_bounds__(NT, 1) rowgemm_kernel(Params p) {
       acc += nt_e;
     }
   }
-  if (e < 0) return;   // beyond the real tile count (workgroup-uniform)
+  if (e < 0) return;   // (not reached)
   const int n0 = ct * BN;
-  const int nk = p.red / BK;
-  const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int wm = wid >> 2, wn = wid & 3;
+  // this part's reduction steps
+  const int per = (steps + parts - 1) / parts, first = min(part * per, steps), nk = min(per, steps - first);
+  e = __builtin_amdgcn_readfirstlane(e), r0 = __builtin_amdgcn_readfirstlane(r0), r1 = __builtin_amdgcn_readfirstlane(r1);
   const uint16_t* bw = p.b + (int64_t)e * p.b_es;
-
-  f32x4_t acc[8][4];
+  tile::Loop<false, MODE == FWD> loop(smem, p.a + (int64_t)r0 * p.lda + first * BK, p.lda, r1 - r0,
+                                      MODE == FWD ? bw + (int64_t)first * BK * p.ldb + n0 : bw + (int64_t)n0 * p.ldb + first * BK, p.ldb,
+                                      min(BN, p.ncols - n0));
+  f32x4_t acc[8][8];
 #pragma unroll
   for (int i = 0; i < 8; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-  const uint32_t lds0 = lds_addr(smem);
-  // per-lane DMA sources of reduction step 0; step s adds s * BK elements (row images) or s * BK
-  // rows (the k-major image)
-  const uint16_t* src_a[PIECES];
-  const uint16_t* src_b[PIECES];
-#pragma unroll
-  for (int i = 0; i < PIECES; ++i) {
-    const int piece = wid * PIECES + i;
-    {  // row image: piece = rows 16 piece .. + 15, lane -> row 16 piece + l / 4, slot l % 4
-      const int row = 16 * piece + (lane >> 2), ch = (lane & 3) ^ rswz(row);
-      const int gr = min(r0 + row, r1 - 1);   // rows past the expert's range re-read a valid row (never stored)
-      src_a[i] = p.a + (int64_t)gr * p.lda + 8 * ch;
-      if (MODE == DGRAD) {
-        const int col = min(n0 + row, p.ncols - 1);   // output column k_out = a row of W[e]
-        src_b[i] = bw + (int64_t)col * p.ldb + 8 * ch;
-      }
-    }
-    if (MODE == FWD) {  // k-major image: piece = k rows 2 piece, 2 piece + 1; lane -> k 2 piece + l / 32, slot l % 32
-      const int t = 2 * piece + (lane >> 5), ch = (lane & 31) ^ tswz(t);
-      src_b[i] = bw + (int64_t)t * p.ldb + min(n0 + 8 * ch, p.ncols - 8);
-    }
-  }
-  auto issue = [&](int s) {
-    const uint32_t img = lds0 + (s % STAGES) * STAGE_BYTES + wid * PIECES * 1024;
-    const int oa = s * BK;
-    const int64_t ob = MODE == FWD ? (int64_t)s * BK * p.ldb : (int64_t)s * BK;
-#pragma unroll
-    for (int i = 0; i < PIECES; ++i) {
-      dma16(src_a[i] + oa, __builtin_amdgcn_readfirstlane(img + i * 1024));
-      dma16(src_b[i] + ob, __builtin_amdgcn_readfirstlane(img + IMG_BYTES + i * 1024));
-    }
-  };
-  auto bfrag = [&](const char* img, int c0) { return MODE == FWD ? frag_tr(img, c0) : frag_row(img, c0); };
-
-  if constexpr (PP) {
-    const int grp = wm;
-    auto issue_half = [&](int s, int hh) {
-      if (s >= nk) return;
-      const uint32_t img = lds0 + (s % STAGES) * STAGE_BYTES + wid * PIECES * 1024;
-      const int oa = s * BK;
-      const int64_t ob = MODE == FWD ? (int64_t)s * BK * p.ldb : (int64_t)s * BK;
-      dma16(src_a[hh] + oa, __builtin_amdgcn_readfirstlane(img + hh * 1024));
-      dma16(src_b[hh] + ob, __builtin_amdgcn_readfirstlane(img + IMG_BYTES + hh * 1024));
-    };
-    auto wait_stage = [&](int S) {   // this thread's pieces of stage S landed
-      if (S + 2 < nk) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
-      else if (S + 1 < nk) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    };
-    auto barrier = [] {
-      __builtin_amdgcn_sched_barrier(0);
-      __builtin_amdgcn_s_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-    };
-    issue_half(0, 0); issue_half(0, 1); issue_half(1, 0); issue_half(1, 1); issue_half(2, 0);
-    wait_stage(0);
-    if (grp == 1) issue_half(2, 1);
-    barrier();
-    if (grp == 1) barrier();   // the stagger
-    bf16x8_t af[4], bf[4];
-    for (int t = 0; t < nk; ++t) {
-      const char* img = smem + (t % STAGES) * STAGE_BYTES;
-      // ---- phase (t, 0): B fragments + A rows 0..63 of the wave
-      if (grp == 0) issue_half(t + 2, 1); else issue_half(t + 3, 0);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) bf[j] = bfrag(img + IMG_BYTES, wn * 64 + 16 * j);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) af[i] = frag_row(img, wm * 128 + 16 * i);
-      barrier();
-      __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bf[j], acc[i][j], 0, 0, 0);
-      __builtin_amdgcn_s_setprio(0);
-      barrier();
-      // ---- phase (t, 1): A rows 64..127
-      if (grp == 1) {
-        if (t + 1 < nk) wait_stage(t + 1);
-        issue_half(t + 3, 1);
-      } else {
-        issue_half(t + 3, 0);
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) af[i] = frag_row(img, wm * 128 + 16 * (4 + i));
-      barrier();
-      __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[4 + i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bf[j], acc[4 + i][j], 0, 0, 0);
-      __builtin_amdgcn_s_setprio(0);
-      if (grp == 0 && t + 1 < nk) wait_stage(t + 1);
-      barrier();
-    }
-    if (grp == 0) barrier();   // equal barrier counts before the epilogue's __syncthreads
-  } else {
-  for (int s = 0; s < STAGES - 1 && s < nk; ++s) issue(s);
-  bf16x8_t af[8], bf[4];
+    for (int j = 0; j < 8; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  // (an expert's last tile: with at most half the rows half the work)
+  const bool end = HALF && part == parts - 1;
   if (nk > 0) {
-    wait_vm(min(STAGES - 2, nk - 1));
-    __builtin_amdgcn_s_barrier();
-#pragma unroll
-    for (int j = 0; j < 4; ++j) bf[j] = bfrag(smem + IMG_BYTES, wn * 64 + 16 * j);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) af[i] = frag_row(smem, wm * 128 + 16 * i);
+    if (r1 - r0 > BM / 2) loop.template run<8, HALF>(acc, nk, end);
+    else loop.template run<4, HALF>(acc, nk, end);
   }
-  for (int t = 0; t < nk; ++t) {
-    const bool more = t + 1 < nk;
-    if (more) wait_vm(min(STAGES - 3, nk - 2 - t));
-    __builtin_amdgcn_s_barrier();
-    if (t + STAGES - 1 < nk) issue(t + STAGES - 1);
-    const char* n_img = smem + ((more ? t + 1 : t) % STAGES) * STAGE_BYTES;
-    bf16x8_t bn[4];
+  const int lane = loop.lane, wid = loop.wid, wm = loop.wm, wn = loop.wn;
+
+  // ---- parts of a tile: sums to memory; the last part to come adds them up, in their order
+  if (parts > 1) {
+    const int slot = xcd * XCD_CUS + idx - whole - part;   // of the tile's first part
+    float* sums = p.ws + (int64_t)slot * TILE_FLOATS;
+    auto at = [&](int s, int i, int j) { return reinterpret_cast<f32x4_t*>(sums + (int64_t)s * TILE_FLOATS) + ((wid * 8 + i) * 8 + j) * 64 + lane; };
 #pragma unroll
-    for (int j = 0; j < 4; ++j) bn[j] = bfrag(n_img + IMG_BYTES, wn * 64 + 16 * j);
+    for (int i = 0; i < 8; ++i)
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bf[j], acc[i][j], 0, 0, 0);
-      af[i] = frag_row(n_img, wm * 128 + 16 * i);
+      for (int j = 0; j < 8; ++j) *at(part, i, j) = acc[i][j];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    __syncthreads();
+    int* last = reinterpret_cast<int*>(smem);
+    if (threadIdx.x == 0) {
+      *last = __hip_atomic_fetch_add(p.tickets + slot, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == parts - 1;
+      if (*last) __hip_atomic_store(p.tickets + slot, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+    __syncthreads();
+    if (!*last) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    for (int s = 0; s < parts; ++s) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) bf[j] = bn[j];
-  }
+      for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const f32x4_t v = *at(s, i, j);
+          acc[i][j] = s == 0 ? v : acc[i][j] + v;
+        }
+    }
   }
 
-  // ---- epilogue: 4 rounds of 32 rows x 64 columns per wave through a padded LDS slab, then bf16
-  // pairs: lane l stores columns 2 (l & 31), +1 of row 2 rr + (l >> 5) (128 B per row per instruction)
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  // ---- results through LDS, a wave's 128 x 128 in 32 KB of its own (16-byte chunks XORed with the row): 256 contiguous bytes of a row
+  // a store
   __syncthreads();
-  constexpr int LD = 68;
-  float* slab = reinterpret_cast<float*>(smem) + wid * (32 * LD);
-  const int ccol = lane & 15, crow = 4 * (lane >> 4);
-  const int pc = 2 * (lane & 31), ph = lane >> 5;
-  const int col = n0 + wn * 64 + pc;
+  char* own = smem + wid * (tile::LDS_BYTES / 4);
 #pragma unroll
-  for (int rnd = 0; rnd < 4; ++rnd) {
+  for (int i = 0; i < 8; ++i)
 #pragma unroll
-    for (int ii = 0; ii < 2; ++ii)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) slab[(16 * ii + crow + r) * LD + 16 * j + ccol] = acc[2 * rnd + ii][j][r];
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll 4
-    for (int rr = 0; rr < 16; ++rr) {
-      const int lr = 2 * rr + ph;
-      const int row = r0 + wm * 128 + 32 * rnd + lr;
-      const float v0 = slab[lr * LD + pc], v1 = slab[lr * LD + pc + 1];
-      if (row < r1 && col < p.ncols) *reinterpret_cast<uint32_t*>(p.c + (int64_t)row * p.ldc + col) = pack2bf(v0, v1);
+    for (int j = 0; j < 8; j += MODE == FWD ? 1 : 2) {
+      const int r = 16 * i + (lane & 15), c = tile::col<MODE == FWD>(0, j, lane);
+      const u32x2_t lo = {pack2bf(acc[i][j][0], acc[i][j][1]), pack2bf(acc[i][j][2], acc[i][j][3])};
+      char* to = own + r * 256 + 16 * ((c >> 3) ^ (r & 15));
+      if (MODE == FWD) *reinterpret_cast<u32x2_t*>(to + 2 * (c & 7)) = lo;
+      else *reinterpret_cast<u32x4_t*>(to) = u32x4_t{lo[0], lo[1], pack2bf(acc[i][j + 1][0], acc[i][j + 1][1]), pack2bf(acc[i][j + 1][2], acc[i][j + 1][3])};
     }
-    __builtin_amdgcn_wave_barrier();
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  const int c0 = 128 * wn + 8 * (lane & 15);
+#pragma unroll
+  for (int k = 0; k < 32; ++k) {
+    const int r = 4 * k + (lane >> 4), row = r0 + 32 * (r >> 4) + 16 * wm + (r & 15);
+    const u32x4_t v = *reinterpret_cast<const u32x4_t*>(own + r * 256 + 16 * ((lane & 15) ^ (r & 15)));
+    if (row < r1 && n0 + c0 < p.ncols) *reinterpret_cast<u32x4_t*>(p.c + (int64_t)row * p.ldc + n0 + c0) = v;
   }
-}
-
-static int g_pp = -1;   // ping-pong variant (NXD_GRG_PP; settable for in-process A/B)
-static bool use_pp() {
-  if (g_pp < 0) {
-    const char* e = getenv("NXD_GRG_PP");
-    g_pp = e ? (atoi(e) != 0) : 1;
-  }
-  return g_pp != 0;
 }
 
 static int band_rows() {
@@ -325,14 +184,20 @@ static int band_rows() {
 
 }  // namespace grg
 
-void grouped_rowgemm_set_pp(int v) { grg::g_pp = v != 0; }
+// Floats of ws and the number of tickets for a reduction of `red` (0: its tiles are never split)
+int64_t grouped_rowgemm_workspace(int red, int* tickets) {
+  const bool pays = red / grg::BK >= 2 * grg::MIN_STEPS;
+  *tickets = pays ? grg::XCDS * grg::XCD_CUS : 0;
+  return (int64_t)*tickets * grg::TILE_FLOATS;
+}
 
 // mode 0 FWD:   a = x [rows, K],  W [E, K, N], c = y  [rows, N]
 // mode 1 DGRAD: a = dy [rows, N], W [E, K, N], c = dx [rows, K]
 // Requires the reduction length % 32 == 0 and K, N % 8 == 0 (checked; returns -1 otherwise, the
 // caller then takes the 128-tile kernel).  Rows past offs[E] are not written.
+// ws, tickets: of grouped_rowgemm_workspace()'s sizes (tickets zeroed), or null.
 int grouped_rowgemm_launch(int mode, const void* a, const void* w, void* c, const int* offs, int E, int rows, int K,
-                           int N, hipStream_t stream) {
+                           int N, hipStream_t stream, float* ws, int* tickets) {
   if (E <= 0 || K <= 0 || N <= 0 || rows < 0 || K % 8 || N % 8) return -1;
   grg::Params p{};
   p.a = static_cast<const uint16_t*>(a);
@@ -350,21 +215,19 @@ int grouped_rowgemm_launch(int mode, const void* a, const void* w, void* c, cons
   } else {
     return -1;
   }
-  if (p.red % grg::BK) return -1;
+  if (p.red % 32) return -1;
   if (rows == 0) return 0;
   p.rt = ceil_div(rows, grg::BM) + E;
   p.nt = ceil_div(p.ncols, grg::BN);
   p.band = grg::band_rows();
-  const int64_t nwg = (int64_t)p.rt * p.nt;
+  p.ws = tickets ? ws : nullptr;
+  p.tickets = tickets;
+  const int64_t nwg = (ceil_div64((int64_t)p.rt * p.nt, grg::XCDS) + (p.ws ? grg::XCD_CUS : 0)) * grg::XCDS;
   if (nwg > INT32_MAX) return -2;
-  const bool pp = grg::use_pp();
-  if (mode == grg::FWD) {
-    if (pp) hipLaunchKernelGGL((grg::rowgemm_kernel<grg::FWD, true>), dim3((unsigned)nwg), dim3(grg::NT), 0, stream, p);
-    else hipLaunchKernelGGL((grg::rowgemm_kernel<grg::FWD, false>), dim3((unsigned)nwg), dim3(grg::NT), 0, stream, p);
-  } else {
-    if (pp) hipLaunchKernelGGL((grg::rowgemm_kernel<grg::DGRAD, true>), dim3((unsigned)nwg), dim3(grg::NT), 0, stream, p);
-    else hipLaunchKernelGGL((grg::rowgemm_kernel<grg::DGRAD, false>), dim3((unsigned)nwg), dim3(grg::NT), 0, stream, p);
-  }
+  const bool half = p.red % grg::BK != 0;
+  auto* f = mode == grg::FWD ? (half ? &grg::rowgemm_kernel<grg::FWD, true> : &grg::rowgemm_kernel<grg::FWD, false>)
+                             : (half ? &grg::rowgemm_kernel<grg::DGRAD, true> : &grg::rowgemm_kernel<grg::DGRAD, false>);
+  hipLaunchKernelGGL(f, dim3((unsigned)nwg), dim3(grg::NT), 0, stream, p);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 

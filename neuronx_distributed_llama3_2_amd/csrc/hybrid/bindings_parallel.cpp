@@ -21,7 +21,8 @@ int experts_few_launch(const RouterParams&, const ExpertFewParams&, hipStream_t)
 int linear_few_launch(const LinearFewParams&, hipStream_t);
 int expert_rows_launch(bool, const ExpertRowsParams&, hipStream_t);
 int grouped_gemm_launch(int, const void*, const void*, void*, const int*, int, int, int, int, int, hipStream_t);
-int grouped_rowgemm_launch(int, const void*, const void*, void*, const int*, int, int, int, int, hipStream_t);
+int grouped_rowgemm_launch(int, const void*, const void*, void*, const int*, int, int, int, int, hipStream_t, float*, int*);
+int64_t grouped_rowgemm_workspace(int, int*);
 }  // namespace nxd
 
 namespace {
@@ -240,7 +241,15 @@ void grouped_linear(Tensor x, Tensor w, Tensor offs, Tensor y) {
   check_align(x, "x");
   check_align(w, "w");
   check_align(y, "y");
-  int rc = nxd::grouped_rowgemm_launch(1, x.data_ptr(), w.data_ptr(), y.data_ptr(), o, (int)E, (int)P, (int)N, (int)K, cur_stream());
+  int tickets = 0;
+  const int64_t floats = nxd::grouped_rowgemm_workspace((int)K, &tickets);
+  Tensor ws, counters;
+  if (floats) {
+    ws = at::empty({floats}, x.options().dtype(at::kFloat));
+    counters = at::zeros({tickets}, x.options().dtype(at::kInt));
+  }
+  int rc = nxd::grouped_rowgemm_launch(1, x.data_ptr(), w.data_ptr(), y.data_ptr(), o, (int)E, (int)P, (int)N, (int)K, cur_stream(),
+                                       floats ? ws.data_ptr<float>() : nullptr, floats ? counters.data_ptr<int>() : nullptr);
   if (rc == -1)
     rc = nxd::grouped_gemm_launch(1, x.data_ptr(), w.data_ptr(), y.data_ptr(), o, (int)E, (int)P, (int)N, (int)K, 0, cur_stream());
   check_rc(rc, "grouped_linear");

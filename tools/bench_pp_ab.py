@@ -1,8 +1,6 @@
 """A/B of the ping-pong main loop (staggered wave groups, two 16-MFMA phases per stage) against the
-one-barrier-per-stage loop of the two hand-written GEMMs: the grouped MoE row GEMM
-(csrc/grouped_rowgemm.hip, Mixtral-8x7B shapes) and the token-major weight-gradient kernel
-(csrc/wgrad_gemm.hip, dense Llama-3-8B TP=1 / TP=8 shards and grouped MoE).  Interleaved rounds in
-one process; each line also reports the max relative difference of each PP output to the old one.
+one-barrier-per-stage loop of the token-major weight-gradient kernel (csrc/wgrad_gemm.hip, dense
+Llama-3-8B TP=1 / TP=8 shards and grouped MoE).  Interleaved rounds in one process; each line also reports the max relative difference of each PP output to the old one.
 v0 = one barrier per stage, v1 = ping-pong with the LDS-DMA issued in the load phase."""
 import json
 import os
@@ -66,18 +64,13 @@ def main():
         I = 14336 // tp
         for name, (K, N) in {"gate_up": (H, 2 * I), "down": (I, H)}.items():
             x = torch.randn(M, K, device="cuda", dtype=torch.bfloat16)
-            w = torch.randn(E, K, N, device="cuda", dtype=torch.bfloat16) * 0.02
             dy = torch.randn(M, N, device="cuda", dtype=torch.bfloat16)
-            y = torch.empty(M, N, device="cuda", dtype=torch.bfloat16)
-            dx = torch.empty(M, K, device="cuda", dtype=torch.bfloat16)
             dw = torch.zeros(E, K, N, device="cuda", dtype=torch.float32)
             fl = 2.0 * M * K * N
             info = {"tp": tp, "proj": name, "M": M, "K": K, "N": N}
-            ab("moe_fwd", fl, lambda: C.grouped_gemm(0, x, w, offs, y, False), y, C.grouped_rowgemm_set_pp, **info)
-            ab("moe_dgrad", fl, lambda: C.grouped_gemm(1, dy, w, offs, dx, False), dx, C.grouped_rowgemm_set_pp, **info)
             ab("moe_wgrad", fl, lambda: C.grouped_gemm(2, x, dy, offs, dw, True), dw, C.wgrad_gemm_set_pp, zero=True,
                **info)
-            del x, w, dy, y, dx, dw
+            del x, dy, dw
             torch.cuda.empty_cache()
     for name, tp, Tt, Mo, Ni in [("qkv", 8, 32768, 768, 4096), ("o", 8, 32768, 4096, 512), ("qkv", 1, 8192, 6144, 4096),
                                  ("gate_up", 1, 8192, 28672, 4096)]:
