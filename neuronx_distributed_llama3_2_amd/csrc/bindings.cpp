@@ -78,7 +78,6 @@ int grouped_rowgemm_launch(int, const void*, const void*, void*, const int*, int
 int64_t grouped_rowgemm_workspace(int, int*);
 int wgrad_gemm_grouped_launch(const void*, int64_t, const void*, int64_t, float*, int64_t, int64_t, const int*, int, int,
                               int, int, hipStream_t);
-void wgrad_gemm_set_ablate(int);
 int dense_gemm_launch(int, int, const void*, int64_t, const void*, int64_t, void*, int64_t, int, int, int, int, hipStream_t);
 int dense_gemm_choose_splits(int, int, int);
 void dense_gemm_set_pipe(int);
@@ -86,7 +85,6 @@ void decode_attn_set_oproj_maxl(int);
 int decode_attn_oproj_maxl();
 int decode_attn_sync_error(bool);
 void decode_attn_set_sync(int);
-void wgrad_gemm_set_pp(int);
 int cu_stream_launch(const void*, void*, int64_t, int, int64_t, hipStream_t);
 int moe_combine_fwd_launch(const void*, const int64_t*, const float*, void*, int64_t, int, int, hipStream_t);
 int moe_combine_bwd_launch(const void*, const void*, const int64_t*, const float*, void*, float*, int64_t, int, int,
@@ -1215,9 +1213,6 @@ PYBIND11_MODULE(_C, m) {
     check_rc(nxd::cu_stream_launch(src.data_ptr(), dst.data_ptr(), bytes_per_block, (int)blocks, ticks, cur_stream()),
              "cu_stream");
   });
-  m.def("wgrad_gemm_set_ablate", [](int64_t v) { nxd::wgrad_gemm_set_ablate((int)v); });
-  // ping-pong (staggered wave-group) main loop of the weight gradients, for in-process A/B
-  m.def("wgrad_gemm_set_pp", [](int64_t v) { nxd::wgrad_gemm_set_pp((int)v); });
   m.def("wgrad_gemm_splits", [](int64_t T, int64_t M, int64_t N) { return nxd::wgrad_gemm_choose_splits((int)T, (int)M, (int)N); });
   m.def("moe_combine_fwd", &moe_combine_fwd);
   m.def("moe_combine_bwd", &moe_combine_bwd);

@@ -136,24 +136,49 @@ struct Loop {
     load_lds(from, i < 8 ? pa : pb, to);
   }
 
-  // acc += the first steps' products.  IM: row fragments that have rows.  HALF, end: the last step has half the reduction.
-  template <int IM, bool HALF>
-  __device__ __forceinline__ void run(f32x4_t (&acc)[8][8], int steps, bool end = false) {
+  // acc += the products of so many steps.  IM: row fragments that have rows.  HALF, end: the last step has half the reduction.
+  // FIRST (TR images): the first step has `rows` of the reduction only (1 .. 64); nothing past them is read.
+  template <int IM, bool HALF, bool FIRST = false>
+  __device__ __forceinline__ void run(f32x4_t (&acc)[8][8], int steps, bool end = false, int rows = BK) {
+    static_assert(!FIRST || AT && BT && !HALF, "images of whole reduction rows");
     static_assert(IM == 8 || IM == 4, "rows");
     bf16x8_t a0[IM], b0[8], a1[IM], b1[8];
     auto advance = [&](int s) {   // towards step s
       if (s < steps) pa += da, pb += db;
     };
+    if constexpr (FIRST) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) load<HALF>(i, 0, end && steps == 1);
-    advance(1);
+      for (int i = 0; i < 16; ++i) {   // (rows past the last: that one again)
+        const int past = max(0, 2 * (8 * wid + (i & 7)) + (lane >> 5) - (rows - 1));
+        const uint32_t from = off[i] - past * (uint32_t)((i < 8 ? da : db) / BK);
+        load_lds(from, i < 8 ? pa : pb, lds + (i < 8 ? 0 : IMG_BYTES) + (8 * wid + (i & 7)) * 1024);
+        if (steps == 1) off[i] = from;   // (for the loads that nothing reads)
+      }
+      if (steps > 1) pa += da / BK * rows, pb += db / BK * rows;
+    } else {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) load<HALF>(i, STEP_BYTES, end && steps <= 2);   // (past the end: the last step again, not used)
+      for (int i = 0; i < 16; ++i) load<HALF>(i, 0, end && steps == 1);
+      advance(1);
+    }
+    if (!FIRST || steps > 1) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) load<HALF>(i, STEP_BYTES, end && steps <= 2);   // (past the end: the last step again, not used)
+    }
     advance(2);
     addresses();
-    asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+    if (FIRST && steps == 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
+    if constexpr (FIRST) {   // what was loaded twice counts nothing
+      for (int i = threadIdx.x; i < 2 * (BK - rows) * 32; i += THREADS) {
+        const int t = rows + (i >> 6);
+        *reinterpret_cast<u32x4_t*>(smem + (i >> 5 & 1) * IMG_BYTES + t * 512 + (i & 31) * 16) = u32x4_t{0u, 0u, 0u, 0u};
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    }
 #pragma unroll
     for (int j = 0; j < 8; ++j) b0[j] = frag_b(j, 0, 0);
 #pragma unroll

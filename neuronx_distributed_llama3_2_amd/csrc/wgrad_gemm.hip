@@ -14,30 +14,18 @@
 // (src/neuronx_distributed/modules/qkv_linear.py:131-150), fp32 gradient accumulation as in the
 // reference's use_fp32_grad_acc ZeRO-1 mode.
 //
-// Structure (cdna_hip_programming.md §5, "Pipelining across barriers"):
-//   * workgroup = 8 waves (512 threads), 256 x 256 output tile, one workgroup per CU (128 KiB LDS);
-//     waves 2 (M) x 4 (N), 128 x 64 outputs each = 8 x 4 v_mfma_f32_16x16x32_bf16 tiles, 128 fp32
-//     accumulators per lane;
-//   * token step BK = 32, a 4-stage LDS ring (4 x 32 KiB): stage t + 3 is issued by LDS-DMA
-//     (global_load_lds_dwordx4, lane-linear 1 KiB pieces) while stage t is consumed, each wave
-//     waits with a COUNTED vmcnt for its own pieces of stage t only, and one raw s_barrier per
-//     stage publishes it (no vmcnt(0) in the loop: two stages stay in flight across every barrier);
-//     default: the ping-pong variant of that loop (two 16-MFMA phases per stage, wave groups one
-//     barrier apart; +3-16 %, profiles/r3_pp_mainloop_ab.jsonl);
-//   * LDS image of an operand stage: [32 tokens][256 features], 512-B rows, 16-B chunk c stored at
-//     c ^ 2 * ((t & 3) | ((t >> 3) & 1) << 2): the two 16-lane groups of a transposed read (4 token
-//     rows x 16 features each, rows t, t + 8) land on 16 distinct bank quads — conflict-free.  The
-//     swizzle is applied to each lane's SOURCE address (the DMA writes lane-linearly, rule 21);
-//   * epilogue: the fp32 tile goes through LDS (padded rows) so that every global access covers
-//     256 contiguous bytes.  With one token split per tile the workgroup alone adds to its tile: it
-//     loads, adds and stores, 32 rows ahead.  With S splits the adds are S atomics in any order,
-//     issued without return and left in flight when the workgroup exits.  One split by atomics had
-//     run at 2.4 TB/s: 8 experts' 4096 x 14336 and 4096 x 28672 gradients over 8,192 rows 2.63 ms a
-//     launch, 1.73 without an epilogue, 1.97 with loads and stores (non-temporal or not: the same).
-//   * grouped (MoE expert weight gradients, dW[e] += x_e^T dy_e over expert-sorted rows): the grid
-//     covers (split, expert, tile); each workgroup reads its expert's row range from the device
-//     offsets (no host sync) and its ragged token tail DMAs a zero chunk instead of a foreign row.
-#include "common.h"
+// Structure: the loop of gemm_tile.h (4 waves of 128 x 128 results, one workgroup per CU), both operands' images with contiguous
+// features, read with the hardware's transposing read; a token count that is no multiple of 64 makes the first step a partial one.
+//   * With one token split per tile the workgroup alone adds to its tile: it loads, adds and stores straight from the registers, 64
+//     contiguous bytes of 16 rows each, the line's other half right after, the loads of 6 of 8 rounds on their way together.  Through LDS, 512
+//     bytes of a row each, 1,000 tokens 128256 x 2048 took 900 us instead of 777, 3,000 1,623 instead of 1,532, 8 experts' 4096 x 28672 over 16,384
+//     4,693 instead of 4,385.  With S splits the adds are S atomics in any order, through LDS so that they cover 256 contiguous bytes, issued
+//     without return and left in flight when the workgroup exits.
+//   * Against 8 waves of 128 x 64 in ping-pong: 1,000 tokens 4096 x 4096 54 -> 48 us, 16384 x 2048 97 -> 86; 3,000 128256 x 2048 1,708 -> 1,526; 8,192
+//     6144 x 4096 406 -> 372; 8 experts' 14336 x 4096 over 32,768 3,903 -> 3,561.
+//   * grouped (MoE expert weight gradients, dW[e] += x_e^T dy_e over expert-sorted rows): the grid covers (split, expert, tile); each
+//     workgroup reads its expert's row range from the device offsets (no host sync).
+#include "gemm_tile.h"
 
 #include <algorithm>
 #include <cstdlib>
@@ -45,12 +33,10 @@
 namespace nxd {
 namespace wg {
 
-constexpr int BM = 256, BN = 256, BK = 32, STAGES = 4, NT = 512;
-constexpr int IMG_BYTES = BK * 256 * 2;           // 16 KiB: one operand stage
-constexpr int STAGE_BYTES = 2 * IMG_BYTES;        // A | B
-constexpr int LDS_BYTES = STAGES * STAGE_BYTES;   // 128 KiB
-constexpr int PIECES = IMG_BYTES / 1024 / (NT / 64);   // LDS-DMA pieces per wave per operand stage (2)
-constexpr int DMA_PER_STAGE = 2 * PIECES;               // per thread per stage (A and B): 4
+using tile::BK;
+using tile::BM;
+using tile::BN;
+constexpr int NT = tile::THREADS;
 
 struct Params {
   const uint16_t* dy;   // [T, M], row stride ld_dy
@@ -62,14 +48,127 @@ struct Params {
   int splits;           // token splits per tile
   int t_per_split;      // tokens per split (multiple of BK)
   int band;             // row tiles per raster band
-  int ablate;           // A/B diagnostics only (wgrad_gemm_set_ablate): 1 = skip the epilogue adds,
-                        // 2 = skip the MFMAs, 4 = skip the LDS-DMA refills of stages >= 3
   int own;              // one split, aligned rows: a workgroup alone adds to its tile (load, add, store), else atomics
   // grouped mode: expert e owns rows offs[e] .. offs[e+1] of dy / x; c += e * c_es
   const int* offs;
   int E;
   int64_t c_es;
 };
+
+// TAIL: a split may have a partial step (the first one)
+template <bool GROUPED, bool TAIL>
+__global__ void __launch_bounds__(NT, 1) wgrad_kernel(Params p) {
+  __shared__ __attribute__((aligned(16))) char smem[tile::LDS_BYTES];
+  const int tiles = p.mt * p.nt;
+  const int id = xcd_remap(blockIdx.x, gridDim.x);
+  const int groups = GROUPED ? p.E : 1;
+  const int split = id / (tiles * groups);   // splits outermost: a tile's partial sums land in different grid waves
+  const int ge = GROUPED ? (id / tiles) % groups : 0;
+  int rt, ct;
+  {
+    const int within = id % tiles;
+    const int kb = p.band, bnd = within / (kb * p.nt), rem = within - bnd * kb * p.nt;
+    const int h = min(kb, p.mt - bnd * kb);
+    rt = bnd * kb + rem % h;
+    ct = rem / h;
+  }
+  const int m0 = rt * BM, n0 = ct * BN;
+  int t_begin, t_end;
+  float* cbase = p.c;
+  if constexpr (GROUPED) {
+    const int g0 = p.offs[ge], g1 = p.offs[ge + 1];
+    const int per = ceil_div(ceil_div(max(g1 - g0, 0), BK), p.splits) * BK;
+    t_begin = g0 + split * per;
+    t_end = min(g1, t_begin + per);
+    if (t_begin >= t_end) return;      // empty group / split: nothing to add (workgroup-uniform)
+    cbase += ge * p.c_es;
+  } else {
+    t_begin = split * p.t_per_split;
+    t_end = min(p.T, t_begin + p.t_per_split);
+  }
+  t_begin = __builtin_amdgcn_readfirstlane(t_begin), t_end = __builtin_amdgcn_readfirstlane(t_end);
+  tile::Loop<true, true> loop(smem, p.dy + (int64_t)t_begin * p.ld_dy + m0, p.ld_dy, min(BM, p.M - m0),
+                              p.x + (int64_t)t_begin * p.ld_x + n0, p.ld_x, min(BN, p.N - n0));
+  f32x4_t acc[8][8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int tokens = t_end - t_begin;
+  loop.template run<8, false, TAIL>(acc, ceil_div(tokens, BK), false, (tokens - 1) % BK + 1);
+  const int lane = loop.lane, wid = loop.wid, wm = loop.wm, wn = loop.wn;
+
+  // 8 rounds of a wave's 16 rows x 128 columns through a padded LDS slab of its own
+  constexpr int LD = 132;
+  float* slab = reinterpret_cast<float*>(smem) + wid * (2 * 16 * LD);
+  if (p.own) {
+    const int row = m0 + 16 * wm + (lane & 15), col = n0 + tile::col<true>(wn, 0, lane);
+    float* cp = cbase + (int64_t)row * p.ldc + col;
+    constexpr int AHEAD = 6;
+    f32x4_t cur[AHEAD][8];
+    const bool whole = m0 + BM <= p.M && n0 + BN <= p.N;
+    auto all = [&](auto ok) {
+      auto load = [&](int i) {   // 16 rows
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          if (ok(i, j)) cur[i % AHEAD][j] = *reinterpret_cast<const f32x4_t*>(cp + (int64_t)(32 * i) * p.ldc + 16 * j);
+      };
+#pragma unroll
+      for (int i = 0; i < AHEAD; ++i) load(i);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          if (ok(i, j)) *reinterpret_cast<f32x4_t*>(cp + (int64_t)(32 * i) * p.ldc + 16 * j) = cur[i % AHEAD][j] + acc[i][j];
+        if (i + AHEAD < 8) load(i + AHEAD);
+      }
+    };
+    if (whole) all([](int, int) { return true; });
+    else all([&](int i, int j) { return row + 32 * i < p.M && col + 16 * j < p.N; });
+    return;
+  }
+  __syncthreads();   // every wave is done with the ring
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) *reinterpret_cast<f32x4_t*>(slab + (lane & 15) * LD + tile::col<true>(0, j, lane)) = acc[i][j];
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll 8
+    for (int rr = 0; rr < 32; ++rr) {
+      const int row = m0 + 32 * i + 16 * wm + (rr >> 1), c = 64 * (rr & 1) + lane, col = n0 + 128 * wn + c;
+      const float v = slab[(rr >> 1) * LD + c];
+      if (row < p.M && col < p.N) unsafeAtomicAdd(cbase + (int64_t)row * p.ldc + col, v);
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+// Few tokens, where most of the time goes into the gradient's reads and writes and into starting and ending a workgroup: 8 waves of
+// 128 x 64 results with a load, an add and a store of 32 rows at a time, steps of 32 tokens in a ring of four, half the registers to fill and
+// to empty.  us here / by the loop above:
+//   * 8 experts' 4096 x 28672 and 14336 x 4096 gradients: 256 tokens each 1,762, 821 / 1,909, 947; 1,024 2,756, 1,372 / 2,867, 1,483;
+//     1,536 3,639, 1,824 / 3,545, 1,803; 4,096 7,857, 3,903 / 7,070, 3,561;
+//   * one gradient of 4096 x 4096, 480 tokens 36 / 38, 500 40 / 36, 700 45 / 40; 768 x 4096 or 128256 x 2048, 500 24, 560 / 28, 608, 700 29, 659 /
+//     32, 668, 1,000 38, 794 / 38, 788.
+//
+// Ping-pong: each stage is two phases of 16 MFMAs per wave, every phase [LDS-DMA half-stage][fragment reads] barrier [16 MFMAs at raised
+// priority] barrier, and wave group 1 (waves 4-7; every SIMD holds one wave of each group) runs one barrier behind group 0.  Ring
+// safety, global barrier instances #n (group 0 passes #(4t+2h) and #(4t+2h+1) in phase (t, h); group 1 one later):
+//   * stage S is read from #(4S-1) on (group 0, phase (S, 0)); both groups retire their pieces of S before arriving there (group 0 after
+//     its MFMAs of (S-1, 1), group 1 before its reads of (S-1, 1));
+//   * the last reads of stage S complete before #(4S+4) (group 1's MFMAs of (S, 1)); its slot is refilled with S+4 after that: group 1
+//     in (S+1, 0/1), group 0 in (S+1, 1) and (S+2, 0);
+//   * pieces issued after stage S's last: S+1 (4) and S+2's first half (2) -> vmcnt(6), less at the tail.
+namespace few {
+
+constexpr int FEW = 1400;   // tokens of a group
+inline bool dense(int T, int tiles) { return T <= 450 || (T <= 700 && (tiles < 192 || tiles > 1024)); }
+constexpr int BK = 32, STAGES = 4, NT = 512;
+constexpr int IMG_BYTES = BK * 256 * 2;           // 16 KiB: one operand stage
+constexpr int STAGE_BYTES = 2 * IMG_BYTES;        // A | B
+constexpr int LDS_BYTES = STAGES * STAGE_BYTES;   // 128 KiB
+constexpr int PIECES = IMG_BYTES / 1024 / (NT / 64);   // LDS-DMA pieces per wave per operand stage (2)
+constexpr int DMA_PER_STAGE = 2 * PIECES;               // per thread per stage (A and B): 4
 
 __device__ __attribute__((aligned(16))) uint32_t g_zero16[4];   // zero-initialised device global: the DMA
                                                                   // source of token rows past a group's end
@@ -101,24 +200,11 @@ __device__ __forceinline__ bf16x8_t frag(const char* img, int c0) {
   return __builtin_bit_cast(bf16x8_t, a8);
 }
 
-__device__ __forceinline__ void wait_vm(int newer) {   // this thread's pieces of the oldest stage landed
-  if (newer >= 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(DMA_PER_STAGE) : "memory");
-  else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-}
-
-// s_setprio around the MFMA clusters or for the younger wave half measured within +-2 % (not kept,
-// profiles/r3_wgrad_kernel_prio_rejected.jsonl)
-// PP: the ping-pong main loop of csrc/grouped_rowgemm.hip (two 16-MFMA phases per stage, wave group
-// 1 one barrier behind group 0; ring-safety argument there).
-// TAIL: the last stage may have fewer than 32 tokens, the others are zeros (always with GROUPED).
-template <bool GROUPED, bool PP, bool TAIL>
-__global__ void __launch_bounds__(NT, 1) wgrad_kernel(Params p) {
+__global__ void __launch_bounds__(NT, 1) kernel(Params p) {
   __shared__ __attribute__((aligned(16))) char smem[LDS_BYTES];
   const int tiles = p.mt * p.nt;
   const int id = xcd_remap(blockIdx.x, gridDim.x);
-  const int groups = GROUPED ? p.E : 1;
-  const int split = id / (tiles * groups);   // splits outermost: a tile's partial sums land in different grid waves
-  const int ge = GROUPED ? (id / tiles) % groups : 0;
+  const int ge = id / tiles;
   int rt, ct;
   {
     const int within = id % tiles;
@@ -128,22 +214,11 @@ __global__ void __launch_bounds__(NT, 1) wgrad_kernel(Params p) {
     ct = rem / h;
   }
   const int m0 = rt * BM, n0 = ct * BN;
-  int t_begin, t_end, nk;
-  float* cbase = p.c;
-  if constexpr (GROUPED) {
-    const int g0 = p.offs[ge], g1 = p.offs[ge + 1];
-    const int per = ceil_div(ceil_div(max(g1 - g0, 0), BK), p.splits) * BK;
-    t_begin = g0 + split * per;
-    t_end = min(g1, t_begin + per);
-    if (t_begin >= t_end) return;      // empty group / split: nothing to add (workgroup-uniform)
-    nk = ceil_div(t_end - t_begin, BK);
-    cbase += ge * p.c_es;
-  } else {
-    t_begin = split * p.t_per_split;
-    t_end = min(p.T, t_begin + p.t_per_split);
-    nk = TAIL ? ceil_div(t_end - t_begin, BK) : (t_end - t_begin) / BK;
-  }
-  const int rows = t_end - t_begin;   // TAIL: token rows >= rows of the last stage read zeros
+  const int t_begin = p.offs ? p.offs[ge] : 0, t_end = p.offs ? p.offs[ge + 1] : p.T;
+  if (t_begin >= t_end) return;      // empty group: nothing to add (workgroup-uniform)
+  const int nk = ceil_div(t_end - t_begin, BK);
+  float* cbase = p.c + ge * p.c_es;
+  const int rows = t_end - t_begin;   // token rows >= rows of the last stage read zeros
 
   const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int wm = wid >> 2, wn = wid & 3;   // 2 x 4 waves: rows 128 wm.., cols 64 wn..
@@ -170,168 +245,84 @@ __global__ void __launch_bounds__(NT, 1) wgrad_kernel(Params p) {
       src_b[i] = p.x + (int64_t)(t_begin + tt) * p.ld_x + min(n0 + 8 * ch, p.N - 8);
     }
   }
-  auto issue = [&](int s) {
+  const int grp = wm;
+  auto issue_half = [&](int s, int hh) {
+    if (s >= nk) return;
     const uint32_t img = lds0 + (s % STAGES) * STAGE_BYTES + wid * PIECES * 1024;
-    const int64_t oa = (int64_t)s * BK * p.ld_dy, ob = (int64_t)s * BK * p.ld_x;
-#pragma unroll
-    for (int i = 0; i < PIECES; ++i) {
-      const uint16_t* sa = src_a[i] + oa;
-      const uint16_t* sb = src_b[i] + ob;
-      if constexpr (TAIL) {
-        if (s * BK + tt_of[i] >= rows) sa = sb = reinterpret_cast<const uint16_t*>(g_zero16);   // past the group's end
-      }
-      dma16(sa, __builtin_amdgcn_readfirstlane(img + i * 1024));
-      dma16(sb, __builtin_amdgcn_readfirstlane(img + IMG_BYTES + i * 1024));
-    }
+    const uint16_t* sa = src_a[hh] + (int64_t)s * BK * p.ld_dy;
+    const uint16_t* sb = src_b[hh] + (int64_t)s * BK * p.ld_x;
+    if (s * BK + tt_of[hh] >= rows) sa = sb = reinterpret_cast<const uint16_t*>(g_zero16);
+    dma16(sa, __builtin_amdgcn_readfirstlane(img + hh * 1024));
+    dma16(sb, __builtin_amdgcn_readfirstlane(img + IMG_BYTES + hh * 1024));
   };
-
-  // Software pipeline, one barrier per 32-token stage.  Fragments of stage t sit in registers
-  // (read during iteration t-1); iteration t publishes stage t+1 (counted vmcnt for this thread's
-  // pieces + barrier), refills the slot of stage t-1 (all reads of t-1 completed before the MFMAs
-  // of t-1, i.e. before this barrier) with stage t+3, and runs the 32 MFMAs of stage t with the
-  // transposed reads of stage t+1 interleaved (each A fragment is re-read right after its last
-  // MFMA; B fragments into a second set) -- the MFMA pipe never waits on an LDS read after a
-  // barrier.  LDS-DMA: stages t+1 .. t+3 in flight at most; a stage is waited for two iterations
-  // after its issue.
-  if constexpr (PP) {
-    const int grp = wm;
-    auto issue_half = [&](int s, int hh) {
-      if (s >= nk || (p.ablate & 4 && s >= STAGES - 1)) return;
-      const uint32_t img = lds0 + (s % STAGES) * STAGE_BYTES + wid * PIECES * 1024;
-      const uint16_t* sa = src_a[hh] + (int64_t)s * BK * p.ld_dy;
-      const uint16_t* sb = src_b[hh] + (int64_t)s * BK * p.ld_x;
-      if constexpr (TAIL) {
-        if (s * BK + tt_of[hh] >= rows) sa = sb = reinterpret_cast<const uint16_t*>(g_zero16);
-      }
-      dma16(sa, __builtin_amdgcn_readfirstlane(img + hh * 1024));
-      dma16(sb, __builtin_amdgcn_readfirstlane(img + IMG_BYTES + hh * 1024));
-    };
-    auto wait_stage = [&](int S) {
-      if (S + 2 < nk) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
-      else if (S + 1 < nk) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    };
-    auto barrier = [] {
-      __builtin_amdgcn_sched_barrier(0);
-      __builtin_amdgcn_s_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-    };
-    issue_half(0, 0); issue_half(0, 1); issue_half(1, 0); issue_half(1, 1); issue_half(2, 0);
-    wait_stage(0);
-    if (grp == 1) issue_half(2, 1);
-    barrier();
-    if (grp == 1) barrier();   // the stagger
-    bf16x8_t af[4], bf[4];
-    for (int t = 0; t < nk; ++t) {
-      const char* img = smem + (t % STAGES) * STAGE_BYTES;
-      if (grp == 0) issue_half(t + 2, 1); else issue_half(t + 3, 0);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) bf[j] = frag(img + IMG_BYTES, wn * 64 + 16 * j);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) af[i] = frag(img, wm * 128 + 16 * i);
-      barrier();
-      __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bf[j], acc[i][j], 0, 0, 0);
-      __builtin_amdgcn_s_setprio(0);
-      barrier();
-      if (grp == 1) {
-        if (t + 1 < nk) wait_stage(t + 1);
-        issue_half(t + 3, 1);
-      } else {
-        issue_half(t + 3, 0);
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) af[i] = frag(img, wm * 128 + 16 * (4 + i));
-      barrier();
-      __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[4 + i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bf[j], acc[4 + i][j], 0, 0, 0);
-      __builtin_amdgcn_s_setprio(0);
-      if (grp == 0 && t + 1 < nk) wait_stage(t + 1);
-      barrier();
-    }
-    if (grp == 0) barrier();
-  } else {
-  for (int s = 0; s < STAGES - 1 && s < nk; ++s) issue(s);
-  bf16x8_t af[8], bf[4];
-  if (nk > 0) {
-    wait_vm(min(STAGES - 2, nk - 1));
+  auto wait_stage = [&](int S) {
+    if (S + 2 < nk) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+    else if (S + 1 < nk) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  };
+  auto barrier = [] {
+    __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_barrier();
-    const char* a_img = smem;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) bf[j] = frag(a_img + IMG_BYTES, wn * 64 + 16 * j);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) af[i] = frag(a_img, wm * 128 + 16 * i);
-  }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  issue_half(0, 0); issue_half(0, 1); issue_half(1, 0); issue_half(1, 1); issue_half(2, 0);
+  wait_stage(0);
+  if (grp == 1) issue_half(2, 1);
+  barrier();
+  if (grp == 1) barrier();   // the stagger
+  bf16x8_t af[4], bf[4];
   for (int t = 0; t < nk; ++t) {
-    const bool more = t + 1 < nk;
-    if (more) wait_vm(min(STAGES - 3, nk - 2 - t));
-    __builtin_amdgcn_s_barrier();
-    if (t + STAGES - 1 < nk && !(p.ablate & 4)) issue(t + STAGES - 1);
-    // stage t+1 (or, on the last iteration, stage t again: harmless, never consumed)
-    const char* n_img = smem + ((more ? t + 1 : t) % STAGES) * STAGE_BYTES;
-    bf16x8_t bn[4];
+    const char* img = smem + (t % STAGES) * STAGE_BYTES;
+    if (grp == 0) issue_half(t + 2, 1); else issue_half(t + 3, 0);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) bn[j] = frag(n_img + IMG_BYTES, wn * 64 + 16 * j);
+    for (int j = 0; j < 4; ++j) bf[j] = frag(img + IMG_BYTES, wn * 64 + 16 * j);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      if (!(p.ablate & 2)) {
+    for (int i = 0; i < 4; ++i) af[i] = frag(img, wm * 128 + 16 * i);
+    barrier();
+    __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bf[j], acc[i][j], 0, 0, 0);
-      } else {
-        asm volatile("" ::"v"(af[i]), "v"(bf[0]), "v"(bf[1]), "v"(bf[2]), "v"(bf[3]));
-      }
-      af[i] = frag(n_img, wm * 128 + 16 * i);
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bf[j], acc[i][j], 0, 0, 0);
+    __builtin_amdgcn_s_setprio(0);
+    barrier();
+    if (grp == 1) {
+      if (t + 1 < nk) wait_stage(t + 1);
+      issue_half(t + 3, 1);
+    } else {
+      issue_half(t + 3, 0);
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) bf[j] = bn[j];
+    for (int i = 0; i < 4; ++i) af[i] = frag(img, wm * 128 + 16 * (4 + i));
+    barrier();
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[4 + i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bf[j], acc[4 + i][j], 0, 0, 0);
+    __builtin_amdgcn_s_setprio(0);
+    if (grp == 0 && t + 1 < nk) wait_stage(t + 1);
+    barrier();
   }
-  }
+  if (grp == 0) barrier();
 
   // ---- epilogue: per wave, 4 rounds of 32 rows x 64 columns through a private padded LDS slab
   // ([32][68] fp32: the two row groups of a 32-lane store half are 4 rows apart -> 16 banks apart),
-  // then 4 rows (of 256 contiguous bytes) per load and store, or one per atomic wave-instruction.
+  // then 4 rows (of 256 contiguous bytes) per load and store.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   constexpr int LD = 68;
   float* slab = reinterpret_cast<float*>(smem) + wid * (32 * LD);
   const int ccol = lane & 15, crow = 4 * (lane >> 4);
-  if (p.own) {
-    const int col = n0 + wn * 64 + 4 * ccol, row = m0 + wm * 128 + (lane >> 4);
-    float* cp = cbase + (int64_t)row * p.ldc + col;
-    const int left = col < p.N ? p.M - row : 0;   // rows of this lane that there are
-    f32x4_t cur[8];
-    auto load = [&](int rnd) {
+  const int col = n0 + wn * 64 + 4 * ccol, row = m0 + wm * 128 + (lane >> 4);
+  float* cp = cbase + (int64_t)row * p.ldc + col;
+  const int left = col < p.N ? p.M - row : 0;   // rows of this lane that there are
+  f32x4_t cur[8];
+  auto load = [&](int rnd) {
 #pragma unroll
-      for (int k = 0; k < 8; ++k)
-        if (32 * rnd + 4 * k < left) cur[k] = *reinterpret_cast<const f32x4_t*>(cp + (int64_t)(32 * rnd + 4 * k) * p.ldc);
-    };
-    load(0);
-    __syncthreads();   // every wave is done with the ring
-#pragma unroll
-    for (int rnd = 0; rnd < 4; ++rnd) {
-#pragma unroll
-      for (int ii = 0; ii < 2; ++ii)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) slab[(16 * ii + crow + r) * LD + 16 * j + ccol] = acc[2 * rnd + ii][j][r];
-      __builtin_amdgcn_wave_barrier();
-      f32x4_t sum[8];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) sum[k] = cur[k] + *reinterpret_cast<const f32x4_t*>(slab + (4 * k + (lane >> 4)) * LD + 4 * ccol);
-      if (rnd < 3) load(rnd + 1);
-#pragma unroll
-      for (int k = 0; k < 8; ++k)
-        if (32 * rnd + 4 * k < left && !(p.ablate & 1)) *reinterpret_cast<f32x4_t*>(cp + (int64_t)(32 * rnd + 4 * k) * p.ldc) = sum[k];
-      __builtin_amdgcn_wave_barrier();
-    }
-    return;
-  }
+    for (int k = 0; k < 8; ++k)
+      if (32 * rnd + 4 * k < left) cur[k] = *reinterpret_cast<const f32x4_t*>(cp + (int64_t)(32 * rnd + 4 * k) * p.ldc);
+  };
+  load(0);
   __syncthreads();   // every wave is done with the ring
 #pragma unroll
   for (int rnd = 0; rnd < 4; ++rnd) {
@@ -342,16 +333,18 @@ __global__ void __launch_bounds__(NT, 1) wgrad_kernel(Params p) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) slab[(16 * ii + crow + r) * LD + 16 * j + ccol] = acc[2 * rnd + ii][j][r];
     __builtin_amdgcn_wave_barrier();
-    const int col = n0 + wn * 64 + lane;
-#pragma unroll 8
-    for (int rr = 0; rr < 32; ++rr) {
-      const int row = m0 + wm * 128 + 32 * rnd + rr;
-      const float v = slab[rr * LD + lane];
-      if (row < p.M && col < p.N && !(p.ablate & 1)) unsafeAtomicAdd(cbase + (int64_t)row * p.ldc + col, v);
-    }
+    f32x4_t sum[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) sum[k] = cur[k] + *reinterpret_cast<const f32x4_t*>(slab + (4 * k + (lane >> 4)) * LD + 4 * ccol);
+    if (rnd < 3) load(rnd + 1);
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      if (32 * rnd + 4 * k < left) *reinterpret_cast<f32x4_t*>(cp + (int64_t)(32 * rnd + 4 * k) * p.ldc) = sum[k];
     __builtin_amdgcn_wave_barrier();
   }
 }
+
+}  // namespace few
 
 static int band_rows() {
   static const int b = [] {
@@ -362,41 +355,25 @@ static int band_rows() {
   return b;
 }
 
-static int g_ablate = 0;
-
-static int g_pp = -1;   // ping-pong main loop (NXD_WG_PP; settable for in-process A/B)
-static bool use_pp() {
-  if (g_pp < 0) {
-    const char* e = getenv("NXD_WG_PP");
-    g_pp = e ? (atoi(e) != 0) : 1;
-  }
-  return g_pp != 0;
-}
-
 template <bool G, bool TAIL>
 void launch(const Params& p, int64_t nwg, hipStream_t stream) {
-  if (use_pp())
-    hipLaunchKernelGGL((wgrad_kernel<G, true, TAIL>), dim3((unsigned)nwg), dim3(NT), 0, stream, p);
-  else
-    hipLaunchKernelGGL((wgrad_kernel<G, false, TAIL>), dim3((unsigned)nwg), dim3(NT), 0, stream, p);
+  hipLaunchKernelGGL((wgrad_kernel<G, TAIL>), dim3((unsigned)nwg), dim3(NT), 0, stream, p);
 }
 
 }  // namespace wg
 
-void wgrad_gemm_set_ablate(int v) { wg::g_ablate = v; }
-void wgrad_gemm_set_pp(int v) { wg::g_pp = v != 0; }
-
-// Token splits per output tile.  Cost model in token steps (BK = 32) of one workgroup: grid waves
-// of 256 workgroups x (steps per split + ~10 for the atomic epilogue); the smallest split count
-// of minimal cost (fewer splits = fewer fp32 atomic adds per element).
+// Token splits per output tile.  Cost model in token steps (1.3 us) of one workgroup, times 256: grid waves of 256 workgroups x the steps
+// per split, and the epilogues: 8 steps without a split; with splits the atomics' rate bounds all workgroups together, 40 steps for 256
+// tiles.  The smallest split count of minimal cost.  Unsplit / in the given splits, us: 1,000 tokens 6144 x 4096 83 / 2: 199, 2048 x 2048
+// 40 / 2: 40; 3,000 tokens 3072 x 2048 76 / 2: 73 / 3: 109, 2048 x 2048 76 / 2: 59 / 4: 71; 8,192 tokens 6144 x 4096 372 / 2: 411,
+// 512 x 4096 168 / 4: 67 / 8: 76; 32,768 tokens 6144 x 4096 1,485 / 2: 1,305, 768 x 4096 670 / 5: 195 / 6: 288.
 int wgrad_gemm_choose_splits(int T, int M, int N) {
-  const int tiles = ceil_div(M, wg::BM) * ceil_div(N, wg::BN);
+  const int64_t tiles = (int64_t)ceil_div(M, wg::BM) * ceil_div(N, wg::BN);
   const int steps = ceil_div(T, wg::BK);
   int best = 1;
   int64_t best_cost = INT64_MAX;
   for (int s = 1; s <= 32 && s <= steps; ++s) {
-    if (s > 1 && steps / s < 16) break;
-    const int64_t cost = (int64_t)ceil_div(tiles * s, 256) * (ceil_div(steps, s) + 10);
+    const int64_t cost = (tiles * s + 255) / 256 * 256 * ceil_div(steps, s) + (s == 1 ? 8 * 256 : 40 * tiles * s);
     if (cost < best_cost) {
       best_cost = cost;
       best = s;
@@ -425,10 +402,11 @@ int wgrad_gemm_launch(const void* dy, int64_t ld_dy, const void* x, int64_t ld_x
   p.splits = ceil_div(T, p.t_per_split);
   p.own = p.splits == 1 && ldc % 4 == 0 && ldc >= N && (reinterpret_cast<uintptr_t>(c) & 15) == 0;
   p.band = wg::band_rows();
-  p.ablate = wg::g_ablate;
   const int64_t nwg = (int64_t)p.mt * p.nt * p.splits;
   if (nwg > INT32_MAX) return -2;
-  if (T % wg::BK)
+  if (p.own && wg::few::dense(T, p.mt * p.nt))
+    hipLaunchKernelGGL(wg::few::kernel, dim3((unsigned)nwg), dim3(wg::few::NT), 0, stream, p);
+  else if (T % wg::BK)
     wg::launch<false, true>(p, nwg, stream);
   else
     wg::launch<false, false>(p, nwg, stream);
@@ -458,9 +436,12 @@ int wgrad_gemm_grouped_launch(const void* dy, int64_t ld_dy, const void* x, int6
   p.splits = wgrad_gemm_choose_splits(mean, (int)std::min<int64_t>((int64_t)M * E, INT32_MAX), N);
   p.own = p.splits == 1 && ldc % 4 == 0 && ldc >= N && c_es % 4 == 0 && (E == 1 || c_es >= (int64_t)(M - 1) * ldc + N) && (reinterpret_cast<uintptr_t>(c) & 15) == 0;
   p.band = wg::band_rows();
-  p.ablate = wg::g_ablate;
   const int64_t nwg = (int64_t)p.mt * p.nt * E * p.splits;
   if (nwg > INT32_MAX) return -2;
+  if (p.own && rows / E <= wg::few::FEW) {
+    hipLaunchKernelGGL(wg::few::kernel, dim3((unsigned)nwg), dim3(wg::few::NT), 0, stream, p);
+    return hipGetLastError() == hipSuccess ? 0 : -3;
+  }
   wg::launch<true, true>(p, nwg, stream);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
