@@ -26,7 +26,7 @@ from ..parallel_layers import parallel_state as ps
 from ..parallel_layers.sharding import shard_state_dict
 from ..utils.logger import get_logger
 from ..utils.sampling import Sampler
-from .bucketing import pad_to_bucket
+from .bucketing import pad_to_bucket, prefill_lengths
 from .config import InferenceConfig
 from .graphs import DecodeGraph, DecodeState, decode_step
 from .modeling_llama import LlamaInferenceModel
@@ -328,7 +328,7 @@ class LlamaForCausalLMInference:
         attention_mask = attention_mask.to(dev)
         lengths = attention_mask.sum(1)
         pad = self.model_config.pad_token_id if getattr(self.model_config, "pad_token_id", None) is not None else 0
-        ids, mask = pad_to_bucket(input_ids, attention_mask, self.config.buckets + [self.config.max_length], pad)
+        ids, mask = pad_to_bucket(input_ids, attention_mask, prefill_lengths(self.config, B), pad)
         Tb = ids.shape[1]
         seq_ids = torch.arange(B, device=dev) if seq_ids is None else seq_ids.to(dev)
         if want is not None:
