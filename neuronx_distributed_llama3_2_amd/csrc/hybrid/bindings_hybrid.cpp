@@ -24,7 +24,7 @@ int attn_prep_launch(bool, const WindowAttnParams&, hipStream_t);
 bool attn_prompt_supported(const WindowAttnParams&);
 int attn_prompt_launch(const WindowAttnParams&, hipStream_t);
 int attn_row_launch(bool, const WindowAttnParams&, hipStream_t);
-void attn_decode_plan(WindowAttnParams&, int64_t);
+void attn_decode_plan(WindowAttnParams&, int64_t, bool);
 int attn_decode_launch(bool, const WindowAttnParams&, hipStream_t);
 int gemv_hyper_launch(int, const GemvHyperParams&, hipStream_t);
 int pooled_prep_launch(bool, const WindowAttnParams&, hipStream_t);
@@ -285,7 +285,7 @@ void attn_decode(Tensor buf, std::vector<int64_t> sizes, Opt bias, Opt qn_w, Opt
   set_rule(p, scale, softcap, window, lam, out_scale, out_eps, buf, y);
   TORCH_CHECK(p.H <= 65535 && B <= 65535, "attn_decode: grid");
   const int64_t seen = p.window > 0 ? std::min<int64_t>(p.window, p.cap) : p.cap;
-  nxd::attn_decode_plan(p, seen);
+  nxd::attn_decode_plan(p, seen, buf.scalar_type() == at::kFloat);
   TORCH_CHECK(tickets.is_cuda() && tickets.scalar_type() == at::kInt && tickets.is_contiguous() && tickets.numel() >= B * p.H,
               "attn_decode: int32 tickets, B H of them");
   Tensor part;
@@ -408,7 +408,7 @@ void pooled_decode(Tensor buf, std::vector<int64_t> sizes, Tensor qn_w, Tensor k
   set_pooled_norms(p, qn_w, kn_w, eps);
   set_pooled_out(p, scale, buf, out, out_scale);
   p.max_pos = 1 << 30;
-  nxd::attn_decode_plan(p, std::min(p.window, p.cap) + p.pcap);
+  nxd::attn_decode_plan(p, std::min(p.window, p.cap) + p.pcap, buf.scalar_type() == at::kFloat);
   TORCH_CHECK(tickets.is_cuda() && tickets.scalar_type() == at::kInt && tickets.is_contiguous() && tickets.numel() >= B * p.H,
               "pooled_decode: int32 tickets, B H of them");
   Tensor part;

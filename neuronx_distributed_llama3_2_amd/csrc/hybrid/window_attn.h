@@ -42,6 +42,7 @@ struct WindowAttnParams {
   // split decode
   int share;              // query heads of a workgroup (of one key / value head)
   int splits, tiles;      // workgroups per (sequence, heads), 64-key tiles each
+  bool mfma;              // on the matrix instructions, all heads of a key / value head a workgroup
   float* part;            // [B H, splits, maps (V + 2)] partial sums (splits > 1)
   int* tickets;           // [B H] arrivals, zero between launches (splits > 1)
 };

@@ -309,6 +309,96 @@ __global__ void __launch_bounds__(256) attn_decode_any_kernel(WindowAttnParams p
   finish<T, MAPS>(p, b, h, sp, m, l, a, red, &arrival);
 }
 
+// The sums val(j, v) of a workgroup's R heads from h0 on (row j = head x map, column v), with their maxima and weights' sums: merged with
+// those of the other workgroups that have keys of these heads, if there are any, combined over the maps and stored, a wave a head
+// (columns lane, lane + 64, ...).
+template <typename T, int MAPS, typename F>
+__device__ __forceinline__ void finish_heads(const WindowAttnParams& p, int V, int b, int h0, int R, int sp, const float* msum,
+                                             const float* lsum, F val, int* arrival) {
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), NJ = R * MAPS;
+  const int hd = b * (p.H / R) + blockIdx.y, stride = NJ * (V + 2);
+  if (p.splits > 1) {
+    float* part_ = p.part + ((int64_t)hd * p.splits + sp) * stride;
+    for (int i = tid; i < NJ * V; i += 256) {
+      const int j = i / V, v = i % V;
+      __hip_atomic_store(part_ + j * (V + 2) + 2 + v, val(j, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (tid < NJ) {
+      __hip_atomic_store(part_ + tid * (V + 2), msum[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(part_ + tid * (V + 2) + 1, lsum[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // every wave's stores have left before the ticket
+    __syncthreads();
+    if (tid == 0) *arrival = __hip_atomic_fetch_add(p.tickets + hd, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (*arrival != p.splits - 1) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    if (tid == 0) __hip_atomic_store(p.tickets + hd, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  for (int r = w; r < R; r += 4) {
+    float l[MAPS], a[MAPS][4];
+    if (p.splits > 1) {
+      float m[MAPS];
+#pragma unroll
+      for (int k = 0; k < MAPS; ++k) {
+        m[k] = -INFINITY;
+        l[k] = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) a[k][i] = 0.f;
+      }
+      for (int s0 = 0; s0 < p.splits; s0 += 8) {   // eight splits' partial sums per round trip
+        float ms[MAPS][8], lp[MAPS][8], as[MAPS][8][4];
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+#pragma unroll
+          for (int k = 0; k < MAPS; ++k) {
+            const float* o = p.part + ((int64_t)hd * p.splits + min(s0 + s, p.splits - 1)) * stride + (r * MAPS + k) * (V + 2);
+            ms[k][s] = __hip_atomic_load(o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            lp[k][s] = __hip_atomic_load(o + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              as[k][s][i] = i == 0 || 64 * i < V ? __hip_atomic_load(o + 2 + min(lane + 64 * i, V - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.f;
+          }
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+#pragma unroll
+          for (int k = 0; k < MAPS; ++k) {
+            if (s0 + s >= p.splits || ms[k][s] == -INFINITY) continue;   // (no split, or one past the visible keys)
+            const float m2 = fmaxf(m[k], ms[k][s]), f = m[k] == -INFINITY ? 0.f : expf(m[k] - m2), f2 = expf(ms[k][s] - m2);
+            l[k] = l[k] * f + lp[k][s] * f2;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) a[k][i] = a[k][i] * f + as[k][s][i] * f2;
+            m[k] = m2;
+          }
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < MAPS; ++k) {
+        const int j = r * MAPS + k;
+        l[k] = lsum[j];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int v = min(lane + 64 * i, V - 1);
+          a[k][i] = val(j, v);
+        }
+      }
+    }
+    float o[4], ss = 0.f, sc_out = p.out_scale;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      o[i] = a[0][i] / l[0];
+      if constexpr (MAPS == 2) o[i] -= p.lam * (a[MAPS - 1][i] / l[MAPS - 1]);
+      if (lane + 64 * i < V) ss += o[i] * o[i];
+    }
+    if constexpr (MAPS == 2) sc_out = p.out_scale / sqrtf(sum64(ss) / (float)V + p.out_eps);
+    T* y = static_cast<T*>(p.y) + (int64_t)b * p.ldy + (int64_t)(h0 + r) * V;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (lane + 64 * i < V) st(y + lane + 64 * i, o[i] * sc_out);
+
+  }
+}
+
 // ---- head sizes that are multiples of 8, D <= 128: 64 keys a tile.  Keys and values of a tile are on
 // their way before they are needed (the first tile's before the query is even prepared).  Neighbouring
 // lanes read neighbouring pieces of a row: a key's score is a sum over LR lanes, a value row is spread
@@ -528,86 +618,226 @@ __global__ void __launch_bounds__(256) attn_decode_kernel(WindowAttnParams p) {
   }
   __syncthreads();
 
-  // ---- wave r finishes head h0 + r: columns lane, lane + 64, ...
-  float l[MAPS], a[MAPS][4];
-  const int hd = b * (p.H / R) + blockIdx.y, stride = NJ * (V + 2);
-  if (p.splits > 1) {
-    float* part_ = p.part + ((int64_t)hd * p.splits + sp) * stride;
-    for (int i = tid; i < NJ * V; i += 256) {
-      const int j = i / V, v = i % V;
-      __hip_atomic_store(part_ + j * (V + 2) + 2 + v, acc[0][j][v] + acc[1][j][v] + acc[2][j][v] + acc[3][j][v], __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
+  finish_heads<T, MAPS>(p, V, b, h0, R, sp, msum, lsum, [&](int j, int v) { return acc[0][j][v] + acc[1][j][v] + acc[2][j][v] + acc[3][j][v]; },
+                        &arrival);
+}
+
+// ---- bf16 keys and values, D a multiple of 32, V of 16, all query heads of a key / value head (R MAPS <= 16 rows) in a workgroup: the same on
+// the matrix instructions.  The kernel above does 12 products a key, row and column pair of lanes with what it reads; here every wave runs
+// over chunks of 32 keys by itself, with a softmax of its own:
+//   S^T[key][row] = K_c Q^T   summed over the maps c, of the queries' rows only those of map c in c's product (the others zero);
+//   O[row][v] += P V          a lane's weights are the A operand as they are: of the 32 keys it has 16 i + 4 g + e (i < 2, e < 4), so V's
+//                             rows are read back from LDS in that order.  The weights keep their 24 bits, as three bf16 numbers that add
+//                             up to them exactly (the products of bf16 numbers are exact in fp32).
+// The waves' sums meet in LDS once.
+template <int MAPS, int NS, int NDT>
+__global__ void __launch_bounds__(256, 2) attn_decode_mfma_kernel(WindowAttnParams p) {
+  constexpr int D = 32 * NS, V = 16 * NDT, VL = V / 16, CPR = V / 8;   // 16-byte loads of a chunk's values a lane, of a row
+  typedef short short8_t __attribute__((ext_vector_type(8)));
+  typedef __attribute__((address_space(3))) short4_t lds_s4_t;
+  __shared__ __attribute__((aligned(16))) float q[16][D], kn[MAPS][D], vn[V];
+  __shared__ __attribute__((aligned(16))) uint16_t vt[4][32 * V];   // a wave's values; then its sums [16][V] fp32
+  __shared__ float red_m[4][16], red_l[4][16], wgt[4][16], msum[16], lsum[16];
+  __shared__ int arrival;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), mi = lane & 15, g4 = lane >> 4;
+  const int sp = blockIdx.x, g = blockIdx.y, b = blockIdx.z, R = p.H / p.G, h0 = g * R, NJ = R * MAPS;
+  const int slot = slot_of(p.slots, b, p.nslots);
+  const int64_t ps = pos_of(p.pos, p.pos_stride, b);
+  const int64_t pt = ps < p.max_pos ? ps : p.max_pos - 1;
+  int64_t j0 = p.window > 0 && ps - p.window + 1 > 0 ? ps - p.window + 1 : 0;
+  if (ps - j0 >= p.cap) j0 = ps - p.cap + 1;            // the ring holds no more (a position beyond the cache)
+  const int n = (int)(ps - j0 + 1);                     // visible keys, the new one last
+  const int e0 = (int)((uint32_t)j0 % (uint32_t)p.cap); // (positions are below 2^31)
+  auto entry = [&](int i) { return e0 + i >= p.cap ? e0 + i - p.cap : e0 + i; };
+  const uint16_t* row = static_cast<const uint16_t*>(p.buf) + (int64_t)b * p.ldb;
+  uint16_t* kc = static_cast<uint16_t*>(p.kc) + ((int64_t)slot * p.G + g) * MAPS * p.cap * D;
+  uint16_t* vc = static_cast<uint16_t*>(p.vc) + ((int64_t)slot * p.G + g) * p.cap * V;
+  const int first = sp * p.tiles * 64, end = min(n, first + p.tiles * 64);
+  const bool owner = first < n && end == n;             // this workgroup has the new key
+
+  u32x4_t kf[MAPS][2][NS], vv[VL];
+  auto fetch = [&](int k0) {   // (keys past the end re-read the last)
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) {
+      const int64_t e = entry(min(k0 + 16 * kt + mi, n - 1));
+#pragma unroll
+      for (int c = 0; c < MAPS; ++c)
+#pragma unroll
+        for (int s = 0; s < NS; ++s) kf[c][kt][s] = *reinterpret_cast<const u32x4_t*>(kc + (c * p.cap + e) * D + 32 * s + 8 * g4);
     }
-    if (tid < NJ) {
-      __hip_atomic_store(part_ + tid * (V + 2), msum[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(part_ + tid * (V + 2) + 1, lsum[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+    for (int i = 0; i < VL; ++i) {
+      const int idx = lane + 64 * i, key = idx / CPR, c = idx % CPR;
+      vv[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(vc + (int64_t)entry(min(k0 + key, n - 1)) * V + 8 * c));
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // every wave's stores have left before the ticket
-    __syncthreads();
-    if (tid == 0) arrival = __hip_atomic_fetch_add(p.tickets + hd, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    if (arrival != p.splits - 1) return;
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    if (tid == 0) __hip_atomic_store(p.tickets + hd, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (w >= R) return;
-    float m[MAPS];
+  };
+  int k0 = first + 32 * w;
+  if (first < n) {
+    if (k0 < end) fetch(k0);
+    // the queries' rows, then the new key's maps and the new value, a wave each in turn: all are on their way before the first is used
+    const int64_t qk0 = (int64_t)p.H * MAPS * D;
+    const int heads = owner ? NJ + MAPS : NJ;
+    constexpr int JOBS = (16 + MAPS + 3) / 4;
+    HeadIn in[JOBS];
 #pragma unroll
-    for (int k = 0; k < MAPS; ++k) {
-      m[k] = -INFINITY;
-      l[k] = 0.f;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) a[k][i] = 0.f;
+    for (int i = 0; i < JOBS; ++i) {
+      const int job = w + 4 * i;
+      if (job >= heads) continue;
+      const int64_t o = job < NJ ? ((int64_t)h0 * MAPS + job) * D : qk0 + ((int64_t)g * MAPS + job - NJ) * D;
+      in[i] = load_head<uint16_t>(p, row + o, p.bias ? p.bias + o : nullptr, job < NJ ? p.qn_w : p.kn_w, pt);
     }
-    for (int s0 = 0; s0 < p.splits; s0 += 8) {   // eight splits' partial sums per round trip
-      float ms[MAPS][8], lp[MAPS][8], as[MAPS][8][4];
+    if (owner) {
+      const int64_t o = p.v_off + (int64_t)g * V;
+      for (int d = tid; d < V; d += 256) vn[d] = bf2f(f2bf(bf2f(row[o + d]) + (p.bias ? p.bias[o + d] : 0.f)));
+    }
 #pragma unroll
-      for (int s = 0; s < 8; ++s)
+    for (int i = 0; i < JOBS; ++i) {
+      const int job = w + 4 * i;
+      if (job >= heads) continue;
+      prepare_head<uint16_t>(p, in[i], (job < NJ ? p.qn_w : p.kn_w) != nullptr, job < NJ ? q[job] : kn[job - NJ]);
+    }
+  }
+  lds_barrier();
+  if (owner) {   // (the values are exact in the activation type)
+    const int e = entry(n - 1);
+    for (int i = tid; i < MAPS * D; i += 256) kc[((int64_t)(i / D) * p.cap + e) * D + i % D] = f2bf(kn[i / D][i % D]);
+    for (int i = tid; i < V; i += 256) vc[(int64_t)e * V + i] = f2bf(vn[i]);
+  }
+  auto pack8 = [](const float* a) { return u32x4_t{pack2bf(a[0], a[1]), pack2bf(a[2], a[3]), pack2bf(a[4], a[5]), pack2bf(a[6], a[7])}; };
+  const u32x4_t none = {0u, 0u, 0u, 0u};
+  bf16x8_t qf[MAPS][NS];   // row mi's piece, in the product of its own map
 #pragma unroll
-        for (int k = 0; k < MAPS; ++k) {
-          const float* o = p.part + ((int64_t)hd * p.splits + min(s0 + s, p.splits - 1)) * stride + (w * MAPS + k) * (V + 2);
-          ms[k][s] = __hip_atomic_load(o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          lp[k][s] = __hip_atomic_load(o + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  for (int c = 0; c < MAPS; ++c)
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            as[k][s][i] = i == 0 || 64 * i < V ? __hip_atomic_load(o + 2 + min(lane + 64 * i, V - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.f;
+    for (int s = 0; s < NS; ++s)
+      qf[c][s] = __builtin_bit_cast(bf16x8_t, first < n && mi < NJ && mi % MAPS == c ? pack8(q[mi] + 32 * s + 8 * g4) : none);
+
+  float run_m = -INFINITY, run_l = 0.f;   // of row mi
+  f32x4_t o[NDT];
+#pragma unroll
+  for (int i = 0; i < NDT; ++i) o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  char* tile = reinterpret_cast<char*>(vt[w]);
+  auto at = [&](int key, int c) { return tile + key * 2 * V + 16 * (c ^ (2 * (key & 3)) % CPR); };   // 4 rows that are read together: other banks
+  for (; k0 < end; k0 += 128) {
+    if (k0 + 32 >= n) {   // the new key's entry may hold an old key or the new one by now: taken from LDS
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+        if (k0 + 16 * kt + mi == n - 1) {
+#pragma unroll
+          for (int c = 0; c < MAPS; ++c)
+#pragma unroll
+            for (int s = 0; s < NS; ++s) kf[c][kt][s] = pack8(kn[c] + 32 * s + 8 * g4);
         }
 #pragma unroll
-      for (int s = 0; s < 8; ++s)
-#pragma unroll
-        for (int k = 0; k < MAPS; ++k) {
-          if (s0 + s >= p.splits || ms[k][s] == -INFINITY) continue;   // (no split, or one past the visible keys)
-          const float m2 = fmaxf(m[k], ms[k][s]), f = m[k] == -INFINITY ? 0.f : expf(m[k] - m2), f2 = expf(ms[k][s] - m2);
-          l[k] = l[k] * f + lp[k][s] * f2;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) a[k][i] = a[k][i] * f + as[k][s][i] * f2;
-          m[k] = m2;
-        }
-    }
-  } else {
-    if (w >= R) return;
-#pragma unroll
-    for (int k = 0; k < MAPS; ++k) {
-      const int j = w * MAPS + k;
-      l[k] = lsum[j];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int v = min(lane + 64 * i, V - 1);
-        a[k][i] = acc[0][j][v] + acc[1][j][v] + acc[2][j][v] + acc[3][j][v];
+      for (int i = 0; i < VL; ++i) {   // (past the end: any finite value, its weight is zero)
+        const int idx = lane + 64 * i;
+        if (k0 + idx / CPR >= n - 1) vv[i] = pack8(vn + 8 * (idx % CPR));
       }
     }
-  }
-  float o[4], ss = 0.f, sc_out = p.out_scale;
+    f32x4_t sc[2];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    o[i] = a[0][i] / l[0];
-    if constexpr (MAPS == 2) o[i] -= p.lam * (a[MAPS - 1][i] / l[MAPS - 1]);
-    if (lane + 64 * i < V) ss += o[i] * o[i];
-  }
-  if constexpr (MAPS == 2) sc_out = p.out_scale / sqrtf(sum64(ss) / (float)V + p.out_eps);
-  T* y = static_cast<T*>(p.y) + (int64_t)b * p.ldy + (int64_t)(h0 + w) * V;
+    for (int kt = 0; kt < 2; ++kt) {
+      sc[kt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-    if (lane + 64 * i < V) st(y + lane + 64 * i, o[i] * sc_out);
+      for (int c = 0; c < MAPS; ++c)
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+          sc[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kf[c][kt][s]), qf[c][s], sc[kt], 0, 0, 0);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the last chunk's transposed reads
+#pragma unroll
+    for (int i = 0; i < VL; ++i) {
+      const int idx = lane + 64 * i;
+      *reinterpret_cast<u32x4_t*>(at(idx / CPR, idx % CPR)) = vv[i];
+    }
+    if (k0 + 128 < end) fetch(k0 + 128);
+    float x[8], cm = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      float sv = sc[j >> 2][j & 3] * p.scale;
+      if (p.softcap > 0.f) sv = p.softcap * tanhf(sv / p.softcap);
+      x[j] = k0 + 16 * (j >> 2) + 4 * g4 + (j & 3) < end ? sv : -INFINITY;
+      cm = fmaxf(cm, x[j]);
+    }
+    cm = fmaxf(cm, __shfl_xor(cm, 16, 64));
+    cm = fmaxf(cm, __shfl_xor(cm, 32, 64));
+    const float nm = fmaxf(run_m, cm), mu = nm == -INFINITY ? 0.f : nm, alpha = run_m == -INFINITY ? 0.f : expf(run_m - mu);
+    float sum = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      x[j] = expf(x[j] - mu);
+      sum += x[j];
+    }
+    sum += __shfl_xor(sum, 16, 64);
+    sum += __shfl_xor(sum, 32, 64);
+    run_l = run_l * alpha + sum;
+    run_m = nm;
+    bf16x8_t pf[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      u32x4_t part;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        part[j] = pack2bf(x[2 * j], x[2 * j + 1]);
+        x[2 * j] -= __uint_as_float(part[j] << 16), x[2 * j + 1] -= __uint_as_float(part[j] & 0xffff0000u);
+      }
+      pf[k] = __builtin_bit_cast(bf16x8_t, part);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {   // rows 4 g4 + e of O by their alpha
+      const float a = __shfl(alpha, 4 * g4 + e, 64);
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt) o[dt][e] *= a;
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+    const int key = 4 * g4 + (mi >> 2), c4 = mi & 3;
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt) {
+      const int c = 2 * dt + (c4 >> 1);
+      const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4_t*)(at(key, c) + 8 * (c4 & 1)));
+      const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4_t*)(at(key + 16, c) + 8 * (c4 & 1)));
+      const short8_t v8 = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+#pragma unroll
+      for (int k = 0; k < 3; ++k) o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf[k], __builtin_bit_cast(bf16x8_t, v8), o[dt], 0, 0, 0);
+    }
+  }
+  // ---- the waves' sums together: O's rows are 4 g4 + e, columns 16 dt + mi
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_wave_barrier();
+  float* mine = reinterpret_cast<float*>(vt[w]);
+#pragma unroll
+  for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) mine[(4 * g4 + e) * V + 16 * dt + mi] = o[dt][e];
+  if (g4 == 0) red_m[w][mi] = run_m, red_l[w][mi] = run_l;
+  __syncthreads();
+  if (tid < 16) {
+    const float m = fmaxf(fmaxf(red_m[0][tid], red_m[1][tid]), fmaxf(red_m[2][tid], red_m[3][tid]));
+    float l = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float f = red_m[i][tid] == -INFINITY ? 0.f : expf(red_m[i][tid] - m);
+      wgt[i][tid] = f;
+      l += red_l[i][tid] * f;
+    }
+    msum[tid] = m, lsum[tid] = l;
+  }
+  __syncthreads();
+  finish_heads<uint16_t, MAPS>(p, V, b, h0, R, sp, msum, lsum, [&](int j, int v) {
+    float a = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) a += wgt[i][j] * reinterpret_cast<const float*>(vt[i])[j * V + v];
+    return a;
+  }, &arrival);
+}
+
+template <int MAPS>
+static void launch_mfma(const WindowAttnParams& p, hipStream_t s) {
+  const dim3 grid((unsigned)p.splits, (unsigned)p.G, (unsigned)p.B);
+  auto* f = p.D == 64 ? (p.V == 64 ? &attn_decode_mfma_kernel<MAPS, 2, 4> : &attn_decode_mfma_kernel<MAPS, 2, 8>)
+                      : (p.V == 64 ? &attn_decode_mfma_kernel<MAPS, 4, 4> : &attn_decode_mfma_kernel<MAPS, 4, 8>);
+  hipLaunchKernelGGL(f, grid, dim3(256), 0, s, p);
 }
 
 template <typename T, int MAPS, int R, bool POOL>
@@ -620,6 +850,12 @@ static void launch_decode(const WindowAttnParams& p, hipStream_t s) {
 
 template <typename T, int MAPS, bool POOL>
 static int run_decode(const WindowAttnParams& p, hipStream_t s) {
+  if constexpr (sizeof(T) == 2 && !POOL) {
+    if (p.mfma) {
+      launch_mfma<MAPS>(p, s);
+      return hipGetLastError() == hipSuccess ? 0 : 1;
+    }
+  }
   if (p.tiles == 0)
     hipLaunchKernelGGL((attn_decode_any_kernel<T, MAPS, POOL>), dim3((unsigned)p.splits, (unsigned)p.H, (unsigned)p.B), dim3(256), 0, s, p);
   else if (p.share == 4) launch_decode<T, MAPS, 4, POOL>(p, s);
@@ -632,8 +868,23 @@ static int run_decode(const WindowAttnParams& p, hipStream_t s) {
 
 // heads a workgroup takes, workgroups per such group and 64-key tiles each (0: the any-size kernel) for at
 // most `seen` visible keys
-void attn_decode_plan(WindowAttnParams& p, int64_t seen) {
+void attn_decode_plan(WindowAttnParams& p, int64_t seen, bool f32) {
   const int rep = p.H / p.G;
+  p.mfma = !f32 && p.pool == 0 && (p.D == 64 || p.D == 128) && (p.V == 64 || p.V == 128) && rep * p.maps <= 16;
+  if (p.mfma) {
+    // One workgroup a CU, as long as each of its waves has a chunk of 32 keys.  us by the kernel above -> here (256 workgroups / 512 / 1,024),
+    // 16 heads of 64 + 128 with two maps and 4 key / value heads: 1 sequence of 1,024 visible keys 13.1 -> 11.2 (in twice as many parts 12.8),
+    // 8 17.7 -> 13.5, 16 24.1 -> 16.1 / 17.4 / 17.3 (33 MB), 32 33.2 -> 20.7 / 21.3 / 30.4; 16 of 4,096 52 -> 31 / 32 / 40, of 300 20.6 -> 13.9; one map of
+    // 128 16 of 1,024 19.2 -> 14.4 / 15.1 / 14.9.  A key / value head a head: two maps of 64 + 64, 16 of 1,024 29.2 -> 21.5; one of 64,
+    // 32 of 300 13.3 -> 13.3.
+    p.share = rep;
+    const int64_t tiles = (seen + 63) / 64, groups = (int64_t)p.B * p.G, most = (tiles + 1) / 2;
+    int64_t splits = 256 / groups;
+    splits = splits < 1 ? 1 : (splits > most ? most : splits);
+    p.tiles = (int)((tiles + splits - 1) / splits);
+    p.splits = (int)((tiles + p.tiles - 1) / p.tiles);
+    return;
+  }
   if (p.D % 8 == 0 && p.V % 8 == 0 && p.D <= 128) {
     // Heads share a workgroup's keys once there are enough workgroups without that.  Four of them read the keys half as often
     // as two, which counts once there are many keys; two have fewer registers and more workgroups.  us with 1 / 2 / 4 heads,
