@@ -38,7 +38,7 @@ struct FewRowsParams {
   // counters as it says (left zeroed)
   float* ws;
   int* tickets;
-  int splits;                   // (the kernel's own)
+  int splits, half;             // (the kernel's own)
 };
 
 // Floats of FewRowsParams::ws and the number of its tickets for a product that is better split (0: it is not)

@@ -253,14 +253,15 @@ struct Finish {
   }
 };
 
-template <int EPI, bool NORM, bool XI, int R, int MT, bool I8, int NW, int CW, int D, bool SPLIT>
+template <int EPI, bool NORM, bool XI, int R, int MT, bool I8, int NW, int CW, int D, bool SPLIT, bool HALF>
 __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) kernel(FewRowsParams p, int tiles) {
   using S = Shape<R, MT, I8, NW, CW, D>;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   f32x4_t* part = reinterpret_cast<f32x4_t*>(smem + S::RING);       // [NW][MT][64]
   float* sq = reinterpret_cast<float*>(smem + S::RING + S::PART);   // [NW][16 MT]
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int c = lane & 15, q = lane >> 4, m0 = SPLIT ? 0 : blockIdx.y * 16 * MT;   // its first row
+  const int c = lane & 15, q = lane >> 4, m0 = SPLIT ? 0 : blockIdx.y * (HALF ? p.half : 16 * MT);   // its first row
+  if constexpr (HALF) p.M = min(p.M, m0 + p.half);
   static_assert(!SPLIT || (CW > 0 && !NORM), "split reductions hold their activations and need no norm");
   const int step = SPLIT ? gridDim.x / p.splits : gridDim.x, tile0 = SPLIT ? blockIdx.x / p.splits : blockIdx.x;
 
@@ -563,7 +564,8 @@ static int64_t tiles_of(const FewRowsParams& p) {
 }
 
 
-template <int EPI, bool NORM, bool XI, int R, int MT, bool I8, int NW, int CW, int D, bool SPLIT = false>
+// HALF: two workgroups for the halves of the activation rows, one a CU
+template <int EPI, bool NORM, bool XI, int R, int MT, bool I8, int NW, int CW, int D, bool SPLIT = false, bool HALF = false>
 static int launch(FewRowsParams p, hipStream_t s, int splits = 1) {
   using S = Shape<R, MT, I8, NW, CW, D>;
   const int nck = ceil_div(p.K, KC);
@@ -571,7 +573,7 @@ static int launch(FewRowsParams p, hipStream_t s, int splits = 1) {
   constexpr size_t lds = S::RING + S::PART + S::SQ;
   static_assert(lds <= 160 * 1024, "LDS of a workgroup");
   const int64_t tiles = tiles_of<EPI, R>(p);
-  auto* f = &kernel<EPI, NORM, XI, R, MT, I8, NW, CW, D, SPLIT>;
+  auto* f = &kernel<EPI, NORM, XI, R, MT, I8, NW, CW, D, SPLIT, HALF>;
   // workgroups of a CU; the limit on LDS and what follows from it are set once on each device
   static std::atomic<int> known[16];
   int dev = 0, per = 0;
@@ -582,11 +584,15 @@ static int launch(FewRowsParams p, hipStream_t s, int splits = 1) {
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, f, (NW + S::FW) * 64, lds) != hipSuccess || per < 1) return 1;
     if (dev < 16) known[dev].store(per, std::memory_order_relaxed);
   }
-  const int64_t room = 256 * (int64_t)per / splits;   // workgroups side by side along the rows
-  const int64_t rounds = ceil_div64(tiles, room < 1 ? 1 : room), groups = ceil_div64(tiles, rounds);
+  const int64_t room = (HALF ? 128 : 256 * (int64_t)per) / splits;   // workgroups side by side along the rows
+  const int64_t rounds = ceil_div64(tiles, room < 1 ? 1 : room);
+  int64_t groups = ceil_div64(tiles, rounds);
+  // the two that read the same weights on one XCD (11008 x 4096 with SwiGLU, 17 rows, 126 groups 57.6 us, 128 35.2)
+  if (HALF) groups = (groups + 7) / 8 * 8;
   if (SPLIT && rounds > 64) return -2;   // (a lane for every tile's ticket)
   p.splits = splits;
-  hipLaunchKernelGGL(f, dim3((unsigned)(groups * splits), (unsigned)(SPLIT ? 1 : ceil_div(p.M, 16 * MT))), dim3((NW + S::FW) * 64), lds, s, p, (int)tiles);
+  if (HALF) p.half = (p.M + 1) / 2;
+  hipLaunchKernelGGL(f, dim3((unsigned)(groups * splits), (unsigned)(SPLIT ? 1 : HALF ? 2 : ceil_div(p.M, 16 * MT))), dim3((NW + S::FW) * 64), lds, s, p, (int)tiles);
   return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
@@ -596,7 +602,7 @@ static int launch(FewRowsParams p, hipStream_t s, int splits = 1) {
 //     128256 x 2048 86 / 92 / 98 (int8 46 / 50 / 54).
 //     Up to 256 tiles there is a tile or less for a CU and streaming begins sooner: 3072 x 2048 6.1 / 6.8 against
 //     6.6 / 7.9 (up to 16 rows: two tiles' operands of a streamed norm do not fit the registers, 19.9 against 10.5).
-//   K <= 4224: 11 waves of 3 chunks: 28672 x 4096 40 / 43 / 55 (streamed 46 / 55 / 225; int8 25 / 27 / 40); without a norm and
+//   K <= 4224: 11 waves of 3 chunks: 28672 x 4096 40 / 43 / 55 (streamed 46 / 55 / 225; int8 25 / 27 / 40; below for 17 rows and more); without a norm and
 //     up to 256 tiles streamed: 4096 x 4096 9.0 / 10.9 / 13.1 against 9.0 / 10.8 / 14.8.
 //   longer: streamed, tiles of 16 rows for more than 2048 weight rows (4096 x 14336 23 / 28 / 38, of 8 rows 25 / 39 / 58),
 //     else of 8, so that every CU has one (2048 x 8192 9.5 / 13.0 / 18.8, of 16 rows 11.5 / 15.4 / 20.8).  Streamed, a
@@ -607,6 +613,12 @@ static int launch(FewRowsParams p, hipStream_t s, int splits = 1) {
 //     16.5 in parts of 1792 (of 1024 15.0 / 15.5 / 18.8: more parts to add up, more tiles a workgroup); 4096 x 14336 at 9 / 13 /
 //     32 24.1 / 26.5 / 38.7 -> 24.4 / 24.5 / 29.2; 4096 x 11008 19.2 / 21.0 / 30.1 -> 21.0 / 21.3 / 25.6; 8192 x 8192 27.6 / 28.9 /
 //     41.9 -> 28.8 / 29.0 / 33.5; 8192 x 28672 at 13 / 32 92 / 142 -> 88 / 102.
+//     With a norm and above 16 rows a workgroup takes half of the rows, up to 512 tiles (K > 2048: 2,048): what the CU has to
+//     read of the activations and to do for their norm counts more than the weights, which come from the XCD's cache the second time.  At 17 /
+//     32 rows: 512 x 2048 7.8 / 9.2 -> 6.3 / 6.8, 3072 x 2048 8.5 / 9.9 -> 7.6 / 7.9 (4 stages under way 8.3 / 8.5), 8192 x 2048 11.5 / 12.3 -> 11.4 / 11.1
+//     (12288 x 2048 13.5 / 15.2 -> 14.2 / 14.5); 1536 x 4096 15.9 / 18.5 -> 9.5 / 10.8, 6144 x 4096 20.5 / 23.0 -> 14.1 / 15.2, 28672 x 4096 with SwiGLU 50.5 / 53.4 ->
+//     44.8 / 47.8 (int8 35.1 / 38.3 -> 30.6 / 32.0), 32000 x 4096 54 / 57 -> 50 / 54 (128256 x 4096 178 / 184 -> 194 / 215: halves that drift
+//     apart read the weights twice).
 //     Unsplit, up to 128 tiles and above 16 rows, a workgroup takes 16 of the rows only, so that every CU has one: 2048 x
 //     2048 at 17 / 32 rows 5.8 / 7.1 -> 5.9 / 6.1 (int8 6.9 -> 5.3 at 32); with more tiles two would share a CU and its loads
 //     (4096 x 4096 at 32 13.2 -> 18.7).
@@ -629,6 +641,8 @@ static int pick(const FewRowsParams& p, hipStream_t s) {
   if constexpr (NORM) {
     if (nck > 33) return -1;
     if (MT == 1 && tiles <= 256 && nck <= 16) return launch<EPI, true, XI, 16, 1, I8, 8, 0, 2>(p, s);
+    if (MT == 2 && nck <= 16 && tiles <= 512) return launch<EPI, true, XI, 16, 1, I8, 8, 2, 2, false, true>(p, s);
+    if (MT == 2 && nck > 16 && tiles <= 2048) return launch<EPI, true, XI, 16, 1, I8, 11, 3, 3, false, true>(p, s);
     if (nck <= 16) return launch<EPI, true, XI, 16, MT, I8, 8, 2, DA>(p, s);
     return launch<EPI, true, XI, 16, MT, I8, 11, 3, 3>(p, s);
   } else {
