@@ -1,6 +1,6 @@
 // Decode attention on MFMA for small query groups (M = (Hq/Hkv) * T <= 16 rows per kv head):
-// one workgroup of 4 waves (FUSE: 8 at D 64) owns a (batch, kv head, key split); the keys per split
-// (128-1,024, splits_of) are sized so the grid reaches ~512 workgroups; every wave runs an
+// one workgroup of 4 or 8 waves (splits_of; FUSE: 8 at D 64) owns a (batch, kv head, key split); the keys per
+// split (128-2,560) are sized so the grid reaches 256 to 512 workgroups; every wave runs an
 // online-softmax flash-decoding loop over 32-key chunks (FUSE: 64) entirely in registers:
 //
 //   S^T[key][m] = K.Q^T   v_mfma_f32_16x16x32_bf16, K rows straight from the cache (16-B loads),
@@ -36,13 +36,13 @@ namespace dattn {
 
 constexpr int KB = 64;            // keys per chunk of a wave with FUSE; splits are multiples of it
 constexpr int KPS = 1024;         // most keys per workgroup split (room for more than 64 K keys: more)
-constexpr int WAVES = 4;          // without FUSE: waves of a workgroup,
+constexpr int WAVES = 4;          // without FUSE: waves of a workgroup where they are not 8,
 constexpr int CHUNK = 32;         // keys per chunk of a wave
 
 // Keys of a split (splits_of): those of a full cache, halved once for a sequence of at most a quarter of its room, again for an
 // eighth, and so on (a few scalar instructions: with divisions, or 64-bit products in their place, every launch took 0.2 us more)
 struct Splits {
-  int room, full, least, most;
+  int room, full, least, most, waves;   // (waves of a workgroup)
   __host__ __device__ int keys(int slen) const {   // slen <= room
     const int n = slen > 1 ? slen : 1, a = __builtin_clz(n) - __builtin_clz(room), s = a - 1 - ((uint32_t)n << a > (uint32_t)room);
     const int k = ((s > 0 ? full >> s : full) + KB - 1) & -KB;
@@ -182,6 +182,7 @@ __device__ __forceinline__ void oproj_tail(const Params& p, const float* of, con
 //   6 of 512-1,024, 8 of 64                          12.0 ->  8.8
 //   13 of 750-1,500, 8 of 128                        25.6 -> 19.5
 //   32 of 1,024-2,048, 8 of 64 (100 MB)              32.2 -> 24.2 (4.2 TB/s; the loads alone 23.5)
+// and with 8 waves again, now of chunks of 32, in parts that are a workgroup a CU (splits_of): 8.3, 17.6, 20.8 us for the last three.
 // - chunks of 32 keys leave the registers for two to three workgroups a CU, so that one computes while the other's keys
 //   are on their way (64 keys at D 128: one workgroup, 22.5 us instead of 18.5 at the same splits);
 // - the first splits of all heads come first in the grid and the last, short or empty ones last: neighbours go to
@@ -578,7 +579,24 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(Params p) {
 // Short sequences in a large cache: 4 of 350-700 keys take 8.0 us with room for 1,024, 8,192 and 131,072 (9.9 by the share of a
 // full cache), 13 of 750-1,500 19.9 / 20.6 with room for 1,792 / 8,192 (22.6), 8 of 2 heads of 750-1,500 9.1 in 16,384 (13.6).  Where the
 // last split merges and 64 heads fill a quarter of the chip, 512 keys stay together: 16 of 250-500 8.4 us, in splits of 128 8.9.
-static Splits splits_of(int Lmax, int B, int Hkv, int MD, bool tickets) {
+static Splits splits_of(int Lmax, int B, int Hkv, int M, int D, bool tickets) {
+  const int MD = M * D;
+  if (tickets && Lmax <= 4608) {
+    // 8 waves, one workgroup a CU: about 256 that have keys, at D 128 320 if all sequences were as long as the cache.  What such a call waits for
+    // is the longest workgroup, and a merge costs 1-2 us: parts that are an eighth of a round too many cost more than parts that are
+    // longer.  us by the rule below / here, sequences of 0.45 to 0.9 of the cache, 8 heads: D 64 4 of 2,304 keys 10.1 / 8.5, 6 of 1,280 9.3 / 8.2,
+    // 8 of 2,304 11.2 / 10.3, 16 of 4,352 22.2 / 22.0, 32 of 640, 1,280, 2,304 11.0, 15.4, 23.0 / 8.9, 13.4, 20.8; D 128 1 of 4,352 11.8 / 9.6, 4 of
+    // 1,756 13.0 / 10.5, 8 of 2,304 18.0 / 15.2, 13 of 1,756 20.1 / 17.6, 32 of 1,280 27.3 / 24.1; four new tokens, D 64, 16 of 1,280 14.9 / 12.5.
+    // Not where two parts a head leave a sixth of the CUs idle and three are too many (D 64, 12 of 2,304 keys 13.1 / 13.7), nor where the call is
+    // so short that 8 waves start later than 4 (1 of 640 6.7 / 7.3).  Whole heads of many keys only where the rule below gives a wave as many:
+    // one long sequence among short ones is what the call waits for then (no more than 2,560 keys for 8 waves; D 128, 24 heads x 8 of 2,304 keys, all 36.0 / 32.5, one 18.5 / 26.8).
+    const int64_t heads = (int64_t)B * Hkv, fit = std::max<int64_t>(1, (D == 64 ? 270 : heads < 40 ? 256 : 320) / heads);
+    const int n = D == 64 && Lmax <= 640 ? 1 : (int)std::min<int64_t>(fit, MD > 256 ? 16 : 24);
+    const int least = D == 64 || heads >= 64 ? 256 : 128, full = std::max(least, (ceil_div(Lmax, n) + KB - 1) / KB * KB);
+    const bool idle = D == 64 && n == 2 && heads < 112, brief = D == 64 && heads < 32 && Lmax <= 1280;
+    const bool uneven = n == 1 && heads < 224 && Lmax > (D == 64 ? 1280 : 640);
+    if (full <= 2560 && !idle && !brief && !uneven) return {Lmax, full, std::min(full, heads >= 64 ? 512 : least), full, 8};
+  }
   static const int target = [] {
     const char* e = getenv("NXD_DECODE_ATTN_WGS");
     const int v = e ? atoi(e) : 512;
@@ -587,7 +605,7 @@ static Splits splits_of(int Lmax, int B, int Hkv, int MD, bool tickets) {
   const int64_t fill = ceil_div64((int64_t)Lmax * B * Hkv, target);
   const int n = (int)std::max<int64_t>(std::min<int64_t>(fill, Lmax), ceil_div(Lmax, MD > 256 ? 16 : tickets ? 24 : 32));
   const int full = std::max(128, (n + KB - 1) / KB * KB);
-  return {Lmax, full, std::min(full, tickets && (int64_t)B * Hkv >= 64 ? 512 : 128), std::max(KPS, ceil_div(Lmax, KB * 64) * KB)};
+  return {Lmax, full, std::min(full, tickets && (int64_t)B * Hkv >= 64 ? 512 : 128), std::max(KPS, ceil_div(Lmax, KB * 64) * KB), WAVES};
 }
 static int most_splits(const Splits& sp) { return ceil_div(sp.room, std::min(sp.full, sp.most)); }
 
@@ -729,7 +747,7 @@ void decode_attn_set_prefetch(const void* a, int64_t a_bytes, const void* b, int
 // The plan of an attention without o_proj over a cache of Lmax keys: {splits, keys of a split of a sequence of len keys, whether
 // the last split merges}
 void decode_attn_plan(int Lmax, int B, int Hkv, int M, int D, int len, bool tickets, int* out) {
-  const dattn::Splits sp = dattn::splits_of(Lmax, B, Hkv, M * D, tickets);
+  const dattn::Splits sp = dattn::splits_of(Lmax, B, Hkv, M, D, tickets);
   out[0] = dattn::most_splits(sp);
   out[1] = sp.keys(len);
   out[2] = tickets && dattn::merge_in_launch(M * D, sp);
@@ -751,11 +769,11 @@ int decode_attn2_launch(const void* q, const int64_t* qs, const void* kc, const 
   p.out = (uint16_t*)out; p.o_sb = os[0]; p.o_st = os[1]; p.o_sh = os[2];
   p.po = po; p.pm = pm; p.pl = pl;
   p.B = B; p.T = T; p.Hq = Hq; p.Hkv = Hkv;
-  p.sp = dattn::splits_of(Lmax, B, Hkv, M * D, tickets != nullptr);
+  p.sp = dattn::splits_of(Lmax, B, Hkv, M, D, tickets != nullptr);
   p.nsplit = dattn::most_splits(p.sp);
   p.scale_log2 = scale * 1.4426950408889634f;
   *nsplit_out = p.nsplit;
-  constexpr int nwv = dattn::WAVES;
+  const int nwv = p.sp.waves;
   const size_t lds = (size_t)nwv * dattn::CHUNK * D * 2 + (size_t)2 * nwv * 16 * 4;
   p.tickets = dattn::merge_in_launch(M * D, p.sp) ? tickets : nullptr;
   if (p.tickets) *nsplit_out = 1;   // (nothing left to merge)
@@ -772,13 +790,10 @@ int decode_attn2_launch(const void* q, const int64_t* qs, const void* kc, const 
   dattn::g_pf[0] = dattn::g_pf[1] = nullptr;
   dattn::g_pf_bytes[0] = dattn::g_pf_bytes[1] = 0;
   const dim3 grid(p.attn_wgs + pf_wgs), block(64 * nwv);
-  if (D == 64) {
-    (void)hipFuncSetAttribute((const void*)dattn::attn_kernel<64, 4, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    hipLaunchKernelGGL((dattn::attn_kernel<64, 4, false>), grid, block, lds, stream, p);
-  } else {
-    (void)hipFuncSetAttribute((const void*)dattn::attn_kernel<128, 4, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    hipLaunchKernelGGL((dattn::attn_kernel<128, 4, false>), grid, block, lds, stream, p);
-  }
+  auto* f = nwv == 8 ? (D == 64 ? &dattn::attn_kernel<64, 8, false> : &dattn::attn_kernel<128, 8, false>)
+                     : (D == 64 ? &dattn::attn_kernel<64, dattn::WAVES, false> : &dattn::attn_kernel<128, dattn::WAVES, false>);
+  (void)hipFuncSetAttribute((const void*)f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  hipLaunchKernelGGL(f, grid, block, lds, stream, p);
   return (int)hipGetLastError();
 }
 
@@ -824,7 +839,7 @@ int decode_attn_oproj_launch(const void* q, const int64_t* qs, const void* kc, c
   const int maxl = decode_attn_oproj_maxl();
   // past maxl: split attention into the partials, then merge + o_proj (needs the partial buffers:
   // [B * Hkv * ceil(Lmax / 128) * M] rows of D, plus the two stats)
-  const bool split = Lmax > maxl && po != nullptr && dattn::most_splits(dattn::splits_of(Lmax, B, Hkv, M * D, false)) > 1;
+  const bool split = Lmax > maxl && po != nullptr && dattn::most_splits(dattn::splits_of(Lmax, B, Hkv, M, D, false)) > 1;
   if (M > 16 || (D != 64 && D != 128) || (Lmax > maxl && !split) || (G * D) % 32 || ldwo % 8) return -1;
   const int nwv = D == 64 ? 8 : 4;
   const int nt = 64 * nwv, tpr = (G * D) / 32;
@@ -888,7 +903,7 @@ int decode_attn_oproj_launch(const void* q, const int64_t* qs, const void* kc, c
     }
   }
   if (split) {
-    const int ns = dattn::most_splits(dattn::splits_of(Lmax, B, Hkv, M * D, false));
+    const int ns = dattn::most_splits(dattn::splits_of(Lmax, B, Hkv, M, D, false));
     const size_t mlds = (size_t)16 * D * 4 + (size_t)ns * 16 * 4 + (size_t)2 * 16 * D * 4;
     if (mlds > 64 * 1024) return -1;
     int ns2 = 0;
