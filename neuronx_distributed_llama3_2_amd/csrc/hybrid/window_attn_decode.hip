@@ -870,7 +870,9 @@ static int run_decode(const WindowAttnParams& p, hipStream_t s) {
 // most `seen` visible keys
 void attn_decode_plan(WindowAttnParams& p, int64_t seen, bool f32) {
   const int rep = p.H / p.G;
-  p.mfma = !f32 && p.pool == 0 && (p.D == 64 || p.D == 128) && (p.V == 64 || p.V == 128) && rep * p.maps <= 16;
+  // (few heads of few keys of one map have nothing to share: 1 sequence of 320 keys, 16 heads of 128 8.4 us by the kernel above, 8.7 here)
+  const bool brief = p.maps == 1 && (int64_t)p.B * p.G < 16 && seen <= 512;
+  p.mfma = !f32 && p.pool == 0 && (p.D == 64 || p.D == 128) && (p.V == 64 || p.V == 128) && rep * p.maps <= 16 && !brief;
   if (p.mfma) {
     // One workgroup a CU, as long as each of its waves has a chunk of 32 keys.  us by the kernel above -> here (256 workgroups / 512 / 1,024),
     // 16 heads of 64 + 128 with two maps and 4 key / value heads: 1 sequence of 1,024 visible keys 13.1 -> 11.2 (in twice as many parts 12.8),
