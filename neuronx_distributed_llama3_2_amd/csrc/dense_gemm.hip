@@ -3,8 +3,8 @@
 //
 //   NT  C[m, n] = sum_k A[m, k] B[n, k]    A [M][K], B [N][K]  (contraction contiguous in both):
 //       the forward y = x W^T and the input gradient dx = dy W (W's K-major copy);
-//   TN  C[m, n] = sum_k A[k, m] B[k, n]    A [K][M], B [K][N]  (contraction along the ROWS):
-//       the weight gradient dW = dy^T x straight from the token-major activations -- no transposes.
+//   TN  C[m, n] = sum_k A[k, m] B[k, n]    A [K][M], B [K][N]  (contraction along the ROWS), BF16 only: the
+//       weight gradient dW += dy^T x goes to wgrad_gemm.hip (8,192 tokens, 4096 x 4096: 240 us here, 211 there).
 //   Epilogues: BF16 store, F32_ACC (C fp32 += acc, one read-modify-write per element: exact and
 //   deterministic), F32_ATOMIC (split-K partial sums into C fp32 by no-return float atomics).
 //
@@ -632,6 +632,9 @@ int dense_gemm_choose_splits(int M, int N, int K) {
   return best;
 }
 
+int wgrad_gemm_launch(const void* dy, int64_t ld_dy, const void* x, int64_t ld_x, float* c, int64_t ldc, int T, int M, int N, int splits,
+                      hipStream_t stream);   // wgrad_gemm.hip
+
 // layout 0 NT: a [M][K] (lda), b [N][K] (ldb); layout 1 TN: a [K][M], b [K][N].
 // epi 0: c bf16 [M][N] = acc; 1: c fp32 += acc (splits forced to 1); 2: c fp32 += acc by atomics,
 // `splits` K splits (<= 0: chosen).  K % 64 == 0, N % 8 == 0, TN also M % 8 == 0, ld* % 8 == 0.
@@ -641,6 +644,8 @@ int dense_gemm_launch(int layout, int epi, const void* a, int64_t lda, const voi
   if (K % dg::BK || N % 8 || lda % 8 || ldb % 8 || ldc % 4) return -1;
   if (layout == dg::LTN && M % 8) return -1;
   if (epi == dg::BF16 && ldc % 8) return -1;
+  if (layout == dg::LTN && epi != dg::BF16)   // weight gradients have a kernel of their own
+    return wgrad_gemm_launch(a, lda, b, ldb, static_cast<float*>(c), ldc, K, M, N, epi == dg::F32_ACC ? 1 : splits, stream);
   dg::Params p{};
   p.a = static_cast<const uint16_t*>(a);
   p.b = static_cast<const uint16_t*>(b);
@@ -675,9 +680,7 @@ int dense_gemm_launch(int layout, int epi, const void* a, int64_t lda, const voi
     else if (epi == dg::F32_ACC) NXD_DG_LAUNCH(dg::LNT, dg::F32_ACC);
     else NXD_DG_LAUNCH(dg::LNT, dg::F32_ATOMIC);
   } else {
-    if (epi == dg::BF16) NXD_DG_LAUNCH(dg::LTN, dg::BF16);
-    else if (epi == dg::F32_ACC) NXD_DG_LAUNCH(dg::LTN, dg::F32_ACC);
-    else NXD_DG_LAUNCH(dg::LTN, dg::F32_ATOMIC);
+    NXD_DG_LAUNCH(dg::LTN, dg::BF16);
   }
 #undef NXD_DG_LAUNCH
   return hipGetLastError() == hipSuccess ? 0 : -3;

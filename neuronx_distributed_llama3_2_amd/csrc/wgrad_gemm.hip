@@ -364,15 +364,16 @@ void launch(const Params& p, int64_t nwg, hipStream_t stream) {
 
 // Token splits per output tile.  Cost model in token steps (1.3 us) of one workgroup, times 256: grid waves of 256 workgroups x the steps
 // per split, and the epilogues: 8 steps without a split; with splits the atomics' rate bounds all workgroups together, 40 steps for 256
-// tiles.  The smallest split count of minimal cost.  Unsplit / in the given splits, us: 1,000 tokens 6144 x 4096 83 / 2: 199, 2048 x 2048
-// 40 / 2: 40; 3,000 tokens 3072 x 2048 76 / 2: 73 / 3: 109, 2048 x 2048 76 / 2: 59 / 4: 71; 8,192 tokens 6144 x 4096 372 / 2: 411,
-// 512 x 4096 168 / 4: 67 / 8: 76; 32,768 tokens 6144 x 4096 1,485 / 2: 1,305, 768 x 4096 670 / 5: 195 / 6: 288.
+// tiles.  The smallest split count of minimal cost, of 8 steps at least.  Unsplit / in the given splits, us: 1,000 tokens 6144 x 4096 83 / 2:
+// 199, 2048 x 2048 40 / 2: 40; 3,000 tokens 3072 x 2048 76 / 2: 73 / 3: 109, 2048 x 2048 76 / 2: 59 / 4: 71; 8,192 tokens 6144 x 4096 372 / 2:
+// 411, 512 x 4096 168 / 4: 67 / 8: 76; 32,768 tokens 6144 x 4096 1,485 / 2: 1,305, 768 x 4096 670 / 5: 195 / 6: 288.
 int wgrad_gemm_choose_splits(int T, int M, int N) {
   const int64_t tiles = (int64_t)ceil_div(M, wg::BM) * ceil_div(N, wg::BN);
   const int steps = ceil_div(T, wg::BK);
   int best = 1;
   int64_t best_cost = INT64_MAX;
   for (int s = 1; s <= 32 && s <= steps; ++s) {
+    if (s > 1 && steps / s < 8) break;
     const int64_t cost = (tiles * s + 255) / 256 * 256 * ceil_div(steps, s) + (s == 1 ? 8 * 256 : 40 * tiles * s);
     if (cost < best_cost) {
       best_cost = cost;

@@ -122,6 +122,10 @@ _WG_KERNEL = os.environ.get("NXD_WGRAD_KERNEL", "auto")
 _WG_SKINNY = 1100.0
 _WG_WIDE = 16000
 _WG_RAGGED = 4000.0
+# Larger products without a producer's copy, where the last round of 256 tiles is at least seven eighths full: time of the library with
+# its two transposes = 1, 12,288 x 4,096 0.92-0.94, 22,016 x 4,096 0.89-0.93, 4,096 x 14,336 0.93-0.99, 8,192 x 8,192 0.94-1.01 from 4,096 to
+# 32,768 tokens (2,048 tokens 0.88-1.03; 6,144 x 4,096, one and a half rounds, 1.02-1.03 up to 8,192).
+_WG_FULL_TOKENS = 4096
 
 
 def _ragged_tokens(tiles: int, odd: bool) -> int:
@@ -145,6 +149,8 @@ def _wgrad_kernel_splits(mg: torch.Tensor, go2: torch.Tensor, x2: torch.Tensor, 
     if T % 32 == 0 and (_WG_KERNEL == "1" or M * N / (M + N) < _WG_SKINNY or (not has_copy and max(M, N) >= _WG_WIDE)):
         return 0
     tiles = -(-M // 256) * -(-N // 256)
+    if T % 32 == 0 and T >= _WG_FULL_TOKENS and not has_copy and 8 * tiles >= 7 * 256 * -(-tiles // 256):
+        return 0
     if T % 64 and not has_copy and M * N / (M + N) < _WG_RAGGED and T <= _ragged_tokens(tiles, T % 8 != 0):
         return 1 if tiles >= 128 else 0
     return None
@@ -154,15 +160,11 @@ def _use_wgrad_kernel(mg: torch.Tensor, go2: torch.Tensor, x2: torch.Tensor, has
     return _wgrad_kernel_splits(mg, go2, x2, has_copy) is not None
 
 
-# The hand-written dense GEMM (csrc/dense_gemm.hip) in its TN form reads the token-major dy / x
-# directly (no transposes) and adds into the fp32 main_grad: one read-modify-write per element when
-# a single K split fills the chip, split-K float atomics otherwise.  Measured against this module's
-# other routes at the Llama-3-8B shapes (profiles/r6_dense_gemm_pipes_vs_hipblaslt.jsonl, T = 8192 /
-# 65536): it wins every TP=8 shard -- qkv 1018 vs 880 TF/s, o_proj 1005 vs 904, gate_up 1180 vs 1164,
-# down 1073 vs 961 -- and the TP=1 o_proj (1236 vs 1092, whose hipBLASLt route transposes both
-# operands), and loses the wide TP=1 shapes to hipBLASLt's TN GEMM on producer-written copies
-# (qkv 955 vs 1070, gate_up 1130 vs 1195, down 1063 vs 1152).  Rule: no producer copy, and
-# M N / (M + N) < 2200.  NXD_DENSE_WGRAD = auto | 1 (whenever the shapes allow) | 0.
+# Whole steps of 64 tokens and no producer copy, M N / (M + N) < 2200: the wgrad kernel as well, with its own choice of splits.
+# Against the library with its two transposes / the TN form of csrc/dense_gemm.hip that was here before, time of the former = 1:
+# 4,096 x 4,096 0.71-0.89 / 0.85-0.92 over 64 to 32,768 tokens, 16,384 x 2,048 0.82-0.90 / 0.67-0.90, 2,048 x 8,192 0.75-0.85 /
+# 0.89-1.01, 768 x 4,096 0.83 / 0.94 over 32,768 (1.3-1.9 / 0.80-0.99 over 512 to 4,096).  NXD_DENSE_WGRAD = auto | 1 (whenever the
+# shapes allow) | 0.
 _DENSE_WG = os.environ.get("NXD_DENSE_WGRAD", "auto")
 _DENSE_WG_SKINNY = 2200.0
 
@@ -179,13 +181,6 @@ def _use_dense_wgrad(mg: torch.Tensor, go2: torch.Tensor, x2, has_copy: bool) ->
     if go2.data_ptr() % 16 or x2.data_ptr() % 16 or mg.data_ptr() % 16:
         return False
     return _DENSE_WG == "1" or (not has_copy and M * N / (M + N) < _DENSE_WG_SKINNY)
-
-
-def _dense_wgrad(mg: torch.Tensor, go2: torch.Tensor, x2: torch.Tensor) -> None:
-    C = ext()
-    T, M = go2.shape
-    splits = C.dense_gemm_splits(M, x2.shape[1], T)
-    C.dense_gemm(1, 1 if splits == 1 else 2, go2, x2, mg, splits)
 
 
 def _wgrad_scratch(n: int, dtype, device, tag: str = "") -> torch.Tensor:
@@ -214,7 +209,7 @@ def wgrad_accumulate_(mg: torch.Tensor, go2: torch.Tensor, x2, go_t: torch.Tenso
         return
     has_copy = go_t is not None or x_t is not None
     if _use_dense_wgrad(mg, go2, x2, has_copy):
-        _dense_wgrad(mg, go2, x2)
+        ext().wgrad_gemm(mg, go2, x2, 0, True)
         return
     splits = _wgrad_kernel_splits(mg, go2, x2, has_copy)
     if splits is not None:
