@@ -31,6 +31,8 @@ int rmsnorm_bwd_num_partials(int64_t);
 void rmsnorm_set_rows_path(int);
 int rmsnorm_bwd_launch(const void*, const void*, const void*, const float*, const void*, void*, float*, float*, int,
                        int64_t, int, hipStream_t);
+int rope_kv_write_launch(void*, int64_t, int, int, int, int, const float*, const float*, const int64_t*, void*, void*, int64_t, int64_t,
+                         int, const int*, const int*, hipStream_t);
 int rope_inplace_launch(void*, int64_t, int64_t, int, int, int, const float*, const float*, const int64_t*, int64_t,
                         int64_t, float, hipStream_t);
 int swiglu_fwd_launch(const void*, void*, int64_t, int, hipStream_t);
@@ -582,6 +584,39 @@ void decode_attn(at::Tensor q, at::Tensor kc, at::Tensor vc, c10::optional<at::T
 }
 
 // k, v: [B, T, Hkv, D] strided; caches [Bc, Hkv, Lmax, D]; pos: int32 [B] position of token 0
+// rope_inplace of the first nq + nkv heads of qkv [B, T, (nq + 2 nkv) D] and kv_cache_write of the last 2 nkv
+void rope_kv_write(at::Tensor qkv, int64_t nq, int64_t nkv, at::Tensor cos_t, at::Tensor sin_t, at::Tensor pos, at::Tensor kc, at::Tensor vc,
+                   c10::optional<at::Tensor> cache_idx, at::Tensor pos0) {
+  check_bf16(qkv, "qkv");
+  check_aligned16(qkv, "qkv");
+  check_bf16(kc, "k_cache");
+  check_bf16(vc, "v_cache");
+  TORCH_CHECK(kc.dim() == 4 && kc.is_contiguous() && vc.sizes() == kc.sizes() && vc.is_contiguous() && kc.size(1) == nkv, "bad caches");
+  check_aligned16(kc, "k_cache");
+  check_aligned16(vc, "v_cache");
+  const int64_t D = kc.size(3);
+  TORCH_CHECK(D == 64 || D == 128 || D == 256, "rope head_dim must be 64/128/256");
+  TORCH_CHECK(qkv.dim() == 3 && qkv.is_contiguous() && nq >= 0 && nkv >= 1 && qkv.size(2) == (nq + 2 * nkv) * D, "qkv [B, T, (nq + 2 nkv) D]");
+  const int64_t B = qkv.size(0), T = qkv.size(1);
+  TORCH_CHECK(cos_t.scalar_type() == at::kFloat && sin_t.scalar_type() == at::kFloat && cos_t.is_contiguous() && sin_t.is_contiguous() &&
+                  cos_t.size(-1) == D / 2 && sin_t.sizes() == cos_t.sizes(),
+              "cos/sin tables must be contiguous fp32 [max_pos, D/2]");
+  TORCH_CHECK(pos.scalar_type() == at::kLong && pos.is_contiguous() && pos.numel() == B * T, "pos must be int64 [B T]");
+  TORCH_CHECK(pos0.scalar_type() == at::kInt && pos0.is_contiguous() && pos0.numel() == B, "pos0 must be int32 [B]");
+  const int* ci = nullptr;
+  if (cache_idx.has_value()) {
+    TORCH_CHECK(cache_idx->scalar_type() == at::kInt && cache_idx->is_contiguous() && cache_idx->numel() == B, "cache_idx must be int32 [B]");
+    ci = cache_idx->data_ptr<int>();
+  } else {
+    TORCH_CHECK(kc.size(0) >= B, "cache batch too small");
+  }
+  if (B * T == 0) return;
+  check_rc(nxd::rope_kv_write_launch(qkv.data_ptr(), B * T, (int)T, (int)nq, (int)nkv, (int)D, cos_t.data_ptr<float>(), sin_t.data_ptr<float>(),
+                                     pos.data_ptr<int64_t>(), kc.data_ptr(), vc.data_ptr(), kc.stride(0), kc.stride(1), (int)kc.size(2), ci,
+                                     pos0.data_ptr<int>(), cur_stream()),
+           "rope_kv_write");
+}
+
 void kv_cache_write(at::Tensor k, at::Tensor v, at::Tensor kc, at::Tensor vc, c10::optional<at::Tensor> cache_idx,
                     at::Tensor pos) {
   int64_t ks[3], vs[3];
@@ -1275,6 +1310,7 @@ PYBIND11_MODULE(_C, m) {
   m.def("decode_attn_set_oproj_maxl", [](int64_t v) { nxd::decode_attn_set_oproj_maxl((int)v); });
   m.def("decode_attn_prefetch", &decode_attn_prefetch);
   m.def("kv_cache_write", &kv_cache_write);
+  m.def("rope_kv_write", &rope_kv_write);
   m.def("argmax_rows", &argmax_rows);
   m.def("greedy_advance", &greedy_advance);
   m.def("topk_sample", &topk_sample);

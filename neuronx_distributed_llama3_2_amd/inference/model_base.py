@@ -123,7 +123,6 @@ class DecoderInferenceMixin:
         if not prefill and logit_rows is None and self._decode_fusable(input_ids):
             return self._forward_decode_fused(input_ids, positions, seq_ids, cache_len, last_index, return_hidden)
         nq, nkv, D = self.nq, self.nkv, self.head_dim
-        W = (nq + 2 * nkv) * D
         cos_t, sin_t = self.model.rope_cache.tables(input_ids.device)
         pos_flat = positions.reshape(-1)
         pos0 = positions[:, 0].to(torch.int32)
@@ -136,12 +135,11 @@ class DecoderInferenceMixin:
             attn = layer.self_attn
             h, residual = self._norm(x, layer.input_layernorm.weight, residual)
             qkv = self._qkv_hook(self._proj(attn.qkv_proj, h))  # [B, T, W]
-            ops.rope_inplace_(qkv.view(B * T, W), 0, nq + nkv, D, cos_t, sin_t, pos_flat)
+            kc, vc = self.kv_cache[i, 0], self.kv_cache[i, 1]
+            ops.rope_kv_write_(qkv, nq, nkv, cos_t, sin_t, pos_flat, kc, vc, pos0, sid32)
             q = qkv.view(B, T, nq + 2 * nkv, D)[:, :, :nq]
             k = qkv.view(B, T, nq + 2 * nkv, D)[:, :, nq:nq + nkv]
             v = qkv.view(B, T, nq + 2 * nkv, D)[:, :, nq + nkv:]
-            kc, vc = self.kv_cache[i, 0], self.kv_cache[i, 1]
-            ops.kv_cache_write(k, v, kc, vc, pos0, sid32)
             if prefill:
                 o, _ = ops.flash_attn_fwd_lse(q, k, v, causal=True)
             else:

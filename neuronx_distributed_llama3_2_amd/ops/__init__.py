@@ -20,5 +20,5 @@ from .optim import (adamw_flat_, clip_coefficient, flat_absmax, flat_sumsq, scal
                     stochastic_round_bf16)
 from .pooled_attention import (PooledRule, PooledSizes, pooled_attention, pooled_decode,  # noqa: F401
                                pooled_prep_)
-from .rope import apply_rotary_reference, inv_freq_from_config, llama3_inv_freq, rope_inplace_, rope_tables  # noqa: F401
+from .rope import apply_rotary_reference, inv_freq_from_config, llama3_inv_freq, rope_inplace_, rope_kv_write_, rope_tables  # noqa: F401
 from .window_attention import AttnRule, AttnSizes, attn_decode, attn_prep_, window_attention  # noqa: F401

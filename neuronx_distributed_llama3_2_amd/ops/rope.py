@@ -88,6 +88,24 @@ def rope_inplace_(buf2d: torch.Tensor, col0: int, nheads: int, head_dim: int, co
     return buf2d
 
 
+def rope_kv_write_(qkv: torch.Tensor, nq: int, nkv: int, cos_t: torch.Tensor, sin_t: torch.Tensor, positions: torch.Tensor,
+                   k_cache: torch.Tensor, v_cache: torch.Tensor, pos0: torch.Tensor, cache_idx: Optional[torch.Tensor] = None) -> None:
+    """rope_inplace_ of the queries and keys of qkv [B, T, (nq + 2 nkv) D] at positions [B T] and kv_cache_write of its keys and
+    values at pos0[b] + t, in one launch where the layouts allow it."""
+    B, T, W = qkv.shape
+    D = W // (nq + 2 * nkv)
+    if (use_native(qkv, k_cache) and D in (64, 128, 256) and qkv.is_contiguous() and k_cache.is_contiguous() and v_cache.is_contiguous()
+            and qkv.dtype == k_cache.dtype == torch.bfloat16 and B * T * (nq + 2 * nkv) < 2 ** 30):
+        ext().rope_kv_write(qkv, nq, nkv, cos_t, sin_t, positions.to(torch.int64).contiguous(), k_cache, v_cache,
+                            cache_idx.to(torch.int32).contiguous() if cache_idx is not None else None, pos0.to(torch.int32).contiguous())
+        return
+    from .decode import kv_cache_write
+
+    rope_inplace_(qkv.view(B * T, W), 0, nq + nkv, D, cos_t, sin_t, positions)
+    heads = qkv.view(B, T, nq + 2 * nkv, D)
+    kv_cache_write(heads[:, :, nq:nq + nkv], heads[:, :, nq + nkv:], k_cache, v_cache, pos0, cache_idx)
+
+
 def apply_rotary_reference(x: torch.Tensor, cos_t: torch.Tensor, sin_t: torch.Tensor, positions: torch.Tensor) -> torch.Tensor:
     """Out-of-place fp32 reference for [..., S, H, D] tensors with positions [S] (HF rotate_half)."""
     D = x.shape[-1]
