@@ -36,12 +36,12 @@ def select_bucket(length: int, buckets: Sequence[int]) -> int:
 HALFWAY_TOKENS = 1024
 
 
-def prefill_lengths(config, batch: int) -> List[int]:
+def prefill_lengths(config, batch: int, halfway: bool = True) -> List[int]:
     """Lengths that prompts of a batch are padded to: the configuration's buckets and its maximum length, and where the buckets are
-    the generated ones (a caller's own list stands as it is) 1.5 times every bucket whose next one holds HALFWAY_TOKENS in the batch."""
+    the generated ones (a caller's own list stands as it is) and `halfway` lengths may be used 1.5 times every bucket whose next one holds HALFWAY_TOKENS in the batch."""
     lengths = list(config.buckets)
     top = getattr(config, "max_context_length", 0)
-    if getattr(config, "enable_bucketing", False) and top and lengths == generate_buckets(min(128, top), top):
+    if halfway and getattr(config, "enable_bucketing", False) and top and lengths == generate_buckets(min(128, top), top):
         lengths += [lo * 3 // 2 for lo, hi in zip(lengths, lengths[1:]) if lo >= 128 and batch * hi >= HALFWAY_TOKENS and lo * 3 // 2 < hi]
     return lengths + [config.max_length]
 

@@ -131,9 +131,11 @@ class _SubModel:
 class LlamaForCausalLMInference:
     """Model family hooks (overridden by the MoE applications in inference/moe.py):
     `_model_cls` the device module, `_hf_to_nxd` HF full state dict -> framework names,
-    `_config_from_dir` HF config.json -> model config."""
+    `_config_from_dir` HF config.json -> model config, `_halfway_lengths` whether prompts may be padded to
+    halfway between two buckets."""
 
     _model_cls = LlamaInferenceModel
+    _halfway_lengths = True
 
     @staticmethod
     def _hf_to_nxd(hf_sd, model_config):
@@ -328,7 +330,7 @@ class LlamaForCausalLMInference:
         attention_mask = attention_mask.to(dev)
         lengths = attention_mask.sum(1)
         pad = self.model_config.pad_token_id if getattr(self.model_config, "pad_token_id", None) is not None else 0
-        ids, mask = pad_to_bucket(input_ids, attention_mask, prefill_lengths(self.config, B), pad)
+        ids, mask = pad_to_bucket(input_ids, attention_mask, prefill_lengths(self.config, B, self._halfway_lengths), pad)
         Tb = ids.shape[1]
         seq_ids = torch.arange(B, device=dev) if seq_ids is None else seq_ids.to(dev)
         if want is not None:

@@ -20,6 +20,7 @@ def test_lengths(batch, top, given, want):
     assert sorted(prefill_lengths(cfg, batch)) == want + [4096] and cfg.buckets == kept
     plain = InferenceConfig(batch_size=batch, seq_len=4096, max_context_length=top)
     assert prefill_lengths(plain, batch) == [top, 4096]
+    assert prefill_lengths(cfg, batch, False) == kept + [4096]
     for T in range(1, 4097, 61):   # never longer than the bucket, and what none holds is refused as before
         ids = torch.zeros((1, T), dtype=torch.long)
         n = pad_to_bucket(ids, ids, prefill_lengths(cfg, batch), 0)[0].shape[1]
