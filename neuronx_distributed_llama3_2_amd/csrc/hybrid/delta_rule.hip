@@ -19,6 +19,8 @@
 #include "hybrid.h"
 #include "delta_rule.h"
 
+#include <algorithm>
+
 namespace nxd {
 namespace hybrid {
 
@@ -96,6 +98,8 @@ __device__ __forceinline__ void conv_silu_run(const DeltaParams& p, const T* pro
 
 constexpr int PREP_TOKENS = 8;   // tokens of one sequence a prep workgroup handles
 
+// A workgroup takes an eighth of the heads and value columns of its tokens (one with all of them went through 8 heads a wave one after
+// another: 4,096 tokens, 16 heads of 128, 70 us a launch, 49 now; 128 tokens 50 and 14).
 // N = 2: two neighbouring channels a lane (even head sizes), 1: one.  NJ steps of 64 N columns cover DP.
 template <typename T, int N, int NJ>
 __global__ void __launch_bounds__(256) delta_prep_kernel(DeltaParams p) {
@@ -113,7 +117,8 @@ __global__ void __launch_bounds__(256) delta_prep_kernel(DeltaParams p) {
   const T* ring = static_cast<const T*>(p.ring) + (int64_t)slot * p.taps * p.C;
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const int G = p.G, D = p.D, DP = p.DP, H = p.H, HV = p.H * p.V, NB = DP / 16;
-  for (int hd = wid; hd < 2 * G; hd += 4) {   // q heads, then k heads: a wave per unit vector
+  const int z = blockIdx.z, nz = gridDim.z;   // (its part of the heads and columns)
+  for (int hd = wid + 4 * z; hd < 2 * G; hd += 4 * nz) {   // q heads, then k heads: a wave per unit vector
     const bool isq = hd < G;
     const int g = isq ? hd : hd - G;
     float x[NJ][N][TT], ss[TT];
@@ -200,7 +205,7 @@ __global__ void __launch_bounds__(256) delta_prep_kernel(DeltaParams p) {
   }
   if (n <= 0) return;
   float* vo = p.vn + m0 * HV;
-  for (int c = N * tid; c < HV; c += 256 * N) {
+  for (int c = N * (tid + 256 * z); c < HV; c += 256 * N * nz) {
     float x[N][TT];
     conv_silu_run<T, TT, N>(p, proj, ring, m0, t0, n, p0, 2 * G * D + c, x);
 #pragma unroll
@@ -210,7 +215,7 @@ __global__ void __launch_bounds__(256) delta_prep_kernel(DeltaParams p) {
         else vo[(int64_t)i * HV + c] = x[0][i];
       }
   }
-  for (int i = tid; i < n * H; i += 256) {
+  for (int i = tid + 256 * z; i < n * H; i += 256 * nz) {
     const int h = i % H;
     const int64_t m = m0 + i / H;
     const T* gates = proj + m * p.ldp + p.C + HV;
@@ -459,7 +464,8 @@ __global__ void __launch_bounds__(NTH) delta_decode_kernel(DeltaParams p) {
 
 template <typename T>
 static int run_prep(const DeltaParams& p, hipStream_t s) {
-  const dim3 grid((unsigned)ceil_div(p.nch > 0 ? p.nch * 64 : p.T, PREP_TOKENS), (unsigned)p.B);
+  const unsigned runs = (unsigned)ceil_div(p.nch > 0 ? p.nch * 64 : p.T, PREP_TOKENS);
+  const dim3 grid(runs, (unsigned)p.B, (unsigned)std::min(8, ceil_div(2 * p.G, 4)));   // (a wave has one of 2 G heads at least)
   const bool pairs = p.D % 2 == 0 && p.V % 2 == 0 && p.ldp % 2 == 0;
   if (pairs && p.DP <= 128) hipLaunchKernelGGL((delta_prep_kernel<T, 2, 1>), grid, dim3(256), 0, s, p);
   else if (pairs) hipLaunchKernelGGL((delta_prep_kernel<T, 2, 2>), grid, dim3(256), 0, s, p);
