@@ -32,9 +32,10 @@ __device__ __forceinline__ f32x4_t mma4(const f32x4_t& a, const f32x4_t& b, f32x
   return c;
 }
 
-// NB = DP / 16 column blocks of the keys.  One workgroup (4 waves) per (head, chunk, sequence).
-template <int NB>
-__global__ void __launch_bounds__(256) delta_chunk_prepare_kernel(DeltaParams p) {
+// NB = DP / 16 column blocks of the keys.  One workgroup of NW waves per (head, chunk, sequence): what a short
+// prompt waits for is one chunk's chain of products (2 chunks of 16 heads 26 us with 4 waves, 15.7 with 16; 64 chunks 77, 74).
+template <int NB, int NW>
+__global__ void __launch_bounds__(64 * NW) delta_chunk_prepare_kernel(DeltaParams p) {
   constexpr int DP = NB * 16, KS = DP + 4, AS = CH + 4;   // LDS row strides (floats)
   extern __shared__ __attribute__((aligned(16))) float sm[];
   float* kt = sm;                       // [64][KS] keys
@@ -50,7 +51,7 @@ __global__ void __launch_bounds__(256) delta_chunk_prepare_kernel(DeltaParams p)
   const int64_t cell = ((int64_t)b * p.nch + ch) * H + h;
 
   const int64_t qkcell = (((int64_t)b * p.nch + ch) * G + g) * CH * DP;
-  for (int i = tid; i < CH * (DP / 4); i += 256) {   // block (d / 16, t / 16), lane i % 64: column d, four tokens
+  for (int i = tid; i < CH * (DP / 4); i += 64 * NW) {   // block (d / 16, t / 16), lane i % 64: column d, four tokens
     const int d = 16 * (i / 256) + (i & 15), t = 16 * ((i / 64) & 3) + 4 * ((i / 16) & 3);
     const f32x4_t v = ld4(p.kn + qkcell + 4 * i);
 #pragma unroll
@@ -73,9 +74,9 @@ __global__ void __launch_bounds__(256) delta_chunk_prepare_kernel(DeltaParams p)
   }
   __syncthreads();
 
-  // ---- the 10 lower blocks of K K^T and of Q K^T, five products a wave
+  // ---- the 10 lower blocks of K K^T and of Q K^T, a wave each in turn
   float* P = p.cp + cell * (CH * CH);
-  for (int job = w; job < 20; job += 4) {
+  for (int job = w; job < 20; job += NW) {
     const bool isq = job >= 10;
     int bi = 0, bj = isq ? job - 10 : job;
     while (bj > bi) bj -= ++bi;               // (0,0) (1,0) (1,1) (2,0) ...
@@ -103,7 +104,7 @@ __global__ void __launch_bounds__(256) delta_chunk_prepare_kernel(DeltaParams p)
   __syncthreads();
 
   // ---- diagonal block w: (I + A_ww)^-1, column lr by the 16 lanes of the first quarter
-  {
+  if (w < 4) {
     float x[16];
     const float* a = am + (16 * w) * AS + 16 * w;
 #pragma unroll
@@ -121,9 +122,9 @@ __global__ void __launch_bounds__(256) delta_chunk_prepare_kernel(DeltaParams p)
   }
   __syncthreads();
 
-  // ---- (I + A) [Y | W] = diag(beta) [V | e^G K], 16 columns at a time; a wave takes every fourth
+  // ---- (I + A) [Y | W] = diag(beta) [V | e^G K], 16 columns at a time, a wave each in turn
   const int nv = (V + 15) / 16;
-  for (int ct = w; ct < nv + NB; ct += 4) {
+  for (int ct = w; ct < nv + NB; ct += NW) {
     const bool isv = ct < nv;
     const int col = (isv ? ct : ct - nv) * 16 + lr;
     f32x4_t y[4];
@@ -291,14 +292,20 @@ __global__ void __launch_bounds__(512, 2) delta_chunk_scan_kernel(DeltaParams p)
   if (v0 == 0 && h == 0) ring_write<T>(p, b, slot, p0, len, tid, 512);
 }
 
-template <typename T, int NB>
-static int run_chunk(const DeltaParams& p, hipStream_t s) {
+template <int NB, int NW>
+static int run_prepare(const DeltaParams& p, hipStream_t s) {
   const size_t lds = (size_t)CH * (NB * 16 + 4 + CH + 4) * 4;
-  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&delta_chunk_prepare_kernel<NB>),
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&delta_chunk_prepare_kernel<NB, NW>),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (attr != hipSuccess) return 2;
-  hipLaunchKernelGGL((delta_chunk_prepare_kernel<NB>), dim3((unsigned)p.H, (unsigned)p.nch, (unsigned)p.B), dim3(256), lds, s, p);
-  if (hipGetLastError() != hipSuccess) return 1;
+  hipLaunchKernelGGL((delta_chunk_prepare_kernel<NB, NW>), dim3((unsigned)p.H, (unsigned)p.nch, (unsigned)p.B), dim3(64 * NW), lds, s, p);
+  return hipGetLastError() == hipSuccess ? 0 : 1;
+}
+
+template <typename T, int NB>
+static int run_chunk(const DeltaParams& p, hipStream_t s) {
+  const int rc = run_prepare<NB, NB <= 8 ? 16 : 8>(p, s);   // (16 waves have 128 registers each)
+  if (rc) return rc;
   const int64_t grid = (int64_t)ceil_div(p.V, 16) * p.B * p.H;
   hipLaunchKernelGGL((delta_chunk_scan_kernel<T, NB>), dim3((unsigned)grid), dim3(512), 0, s, p);
   return hipGetLastError() == hipSuccess ? 0 : 1;
