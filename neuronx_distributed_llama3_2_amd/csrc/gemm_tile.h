@@ -1,4 +1,4 @@
-// The main loop of the 256 x 256-tile products (grouped_rowgemm.hip): C = A B over a reduction in steps of 64, bf16 operands, fp32 sums.
+// The main loop of the 256 x 256-tile products (grouped_rowgemm.hip, wgrad_gemm.hip): C = A B over a reduction in steps of 64, bf16 operands, fp32 sums.
 //
 // What bounds it is power (2.1 GHz and less under matrix cores that are half busy) and what feeds them: LDS reads, and loads of a CU.
 //   * 4 waves, one a SIMD, of 128 x 128 results each: 64 v_mfma_f32_16x16x32_bf16 for 16 fragments read from LDS, two thirds of what

@@ -2,9 +2,9 @@
 
 Buckets are powers of two from the minimum up to (and including) the maximum length.  Prompts are
 right-padded to the smallest bucket that holds the longest prompt of the batch (`prefill_lengths`: or
-to halfway between two of them, for batches of 1,024 tokens and more) so the context encoder sees a handful of distinct shapes (stable allocator pools, reusable GEMM heuristics); the
-decode path needs no length buckets because attention reads the KV cache up to a per-sequence
-device-side length.
+to halfway between two of them, for batches of 1,024 tokens and more) so the context encoder sees a
+handful of distinct shapes (stable allocator pools, reusable GEMM heuristics); the decode path needs
+no length buckets because attention reads the KV cache up to a per-sequence device-side length.
 """
 
 from __future__ import annotations
@@ -38,7 +38,8 @@ HALFWAY_TOKENS = 1024
 
 def prefill_lengths(config, batch: int, halfway: bool = True) -> List[int]:
     """Lengths that prompts of a batch are padded to: the configuration's buckets and its maximum length, and where the buckets are
-    the generated ones (a caller's own list stands as it is) and `halfway` lengths may be used 1.5 times every bucket whose next one holds HALFWAY_TOKENS in the batch."""
+    the generated ones (a caller's own list stands as it is) and `halfway` lengths may be used 1.5 times every bucket whose next one
+    holds HALFWAY_TOKENS in the batch."""
     lengths = list(config.buckets)
     top = getattr(config, "max_context_length", 0)
     if halfway and getattr(config, "enable_bucketing", False) and top and lengths == generate_buckets(min(128, top), top):

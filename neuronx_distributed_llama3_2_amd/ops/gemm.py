@@ -111,7 +111,7 @@ def _use_wgrad_t(go2: torch.Tensor, x2: torch.Tensor = None, K: int = None) -> b
 # TF/s for the hipBLASLt path and its two transposes (the 1 GiB logits gradient), TP=1 a tie.
 # NXD_WGRAD_KERNEL = auto | 1 (whenever the shapes allow) | 0.
 #
-# Token counts that are no multiple of 64 have neither producer copies nor the dense kernel below, and go to this kernel
+# Token counts that are no multiple of 64 have no producer copies, and go to this kernel
 # (unsplit from 128 tiles of 256 x 256 on: a second split's atomics cost more than the chip's idle part, 6,144 x 4,096 over 1,000
 # tokens 88 us, in two splits 201, library 99) by how full its rounds of 256 tiles are.  Time of the library with its two
 # transposes = 1: few tokens always (72: 0.39-0.89, 200: 0.50-0.92; 500, from 128 tiles on: 0.76-0.98); rounds three quarters full up
