@@ -625,10 +625,11 @@ __global__ void __launch_bounds__(256) attn_decode_kernel(WindowAttnParams p) {
 // ---- bf16 keys and values, D a multiple of 32, V of 16, all query heads of a key / value head (R MAPS <= 16 rows) in a workgroup: the same on
 // the matrix instructions.  The kernel above does 12 products a key, row and column pair of lanes with what it reads; here every wave runs
 // over chunks of 32 keys by itself, with a softmax of its own:
-//   S^T[key][row] = K_c Q^T   summed over the maps c, of the queries' rows only those of map c in c's product (the others zero);
+//   S^T[key][row] = K_c Q^T   for each map c, of which a lane keeps its row's (an infinite key is its own map's affair);
 //   O[row][v] += P V          a lane's weights are the A operand as they are: of the 32 keys it has 16 i + 4 g + e (i < 2, e < 4), so V's
 //                             rows are read back from LDS in that order.  The weights keep their 24 bits, as three bf16 numbers that add
-//                             up to them exactly (the products of bf16 numbers are exact in fp32).
+//                             up to them exactly (the products of bf16 numbers are exact in fp32), none negative, nor zero where the weight
+//                             is not: an infinite value stays what it is in all three products.
 // The waves' sums meet in LDS once.
 template <int MAPS, int NS, int NDT>
 __global__ void __launch_bounds__(256, 2) attn_decode_mfma_kernel(WindowAttnParams p) {
@@ -705,12 +706,9 @@ __global__ void __launch_bounds__(256, 2) attn_decode_mfma_kernel(WindowAttnPara
   }
   auto pack8 = [](const float* a) { return u32x4_t{pack2bf(a[0], a[1]), pack2bf(a[2], a[3]), pack2bf(a[4], a[5]), pack2bf(a[6], a[7])}; };
   const u32x4_t none = {0u, 0u, 0u, 0u};
-  bf16x8_t qf[MAPS][NS];   // row mi's piece, in the product of its own map
+  bf16x8_t qf[NS];   // row mi's piece
 #pragma unroll
-  for (int c = 0; c < MAPS; ++c)
-#pragma unroll
-    for (int s = 0; s < NS; ++s)
-      qf[c][s] = __builtin_bit_cast(bf16x8_t, first < n && mi < NJ && mi % MAPS == c ? pack8(q[mi] + 32 * s + 8 * g4) : none);
+  for (int s = 0; s < NS; ++s) qf[s] = __builtin_bit_cast(bf16x8_t, first < n && mi < NJ ? pack8(q[mi] + 32 * s + 8 * g4) : none);
 
   float run_m = -INFINITY, run_l = 0.f;   // of row mi
   f32x4_t o[NDT];
@@ -729,20 +727,21 @@ __global__ void __launch_bounds__(256, 2) attn_decode_mfma_kernel(WindowAttnPara
             for (int s = 0; s < NS; ++s) kf[c][kt][s] = pack8(kn[c] + 32 * s + 8 * g4);
         }
 #pragma unroll
-      for (int i = 0; i < VL; ++i) {   // (past the end: any finite value, its weight is zero)
-        const int idx = lane + 64 * i;
-        if (k0 + idx / CPR >= n - 1) vv[i] = pack8(vn + 8 * (idx % CPR));
+      for (int i = 0; i < VL; ++i) {   // (past the end, where the weight is zero: zeros)
+        const int idx = lane + 64 * i, key = k0 + idx / CPR;
+        if (key >= n - 1) vv[i] = key == n - 1 ? pack8(vn + 8 * (idx % CPR)) : none;
       }
     }
     f32x4_t sc[2];
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt) {
-      sc[kt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int c = 0; c < MAPS; ++c)
+      for (int c = 0; c < MAPS; ++c) {
+        f32x4_t of = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int s = 0; s < NS; ++s)
-          sc[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kf[c][kt][s]), qf[c][s], sc[kt], 0, 0, 0);
+        for (int s = 0; s < NS; ++s) of = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kf[c][kt][s]), qf[s], of, 0, 0, 0);
+        if (c == 0 || mi % MAPS == c) sc[kt] = of;
+      }
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the last chunk's transposed reads
 #pragma unroll
@@ -772,14 +771,20 @@ __global__ void __launch_bounds__(256, 2) attn_decode_mfma_kernel(WindowAttnPara
     sum += __shfl_xor(sum, 32, 64);
     run_l = run_l * alpha + sum;
     run_m = nm;
-    bf16x8_t pf[3];
+    bf16x8_t pf[3];   // the largest bf16 number below the weight, the largest one below what is left, and the rest
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
       u32x4_t part;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        part[j] = pack2bf(x[2 * j], x[2 * j + 1]);
-        x[2 * j] -= __uint_as_float(part[j] << 16), x[2 * j + 1] -= __uint_as_float(part[j] & 0xffff0000u);
+        uint32_t hi[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const uint32_t bits = __float_as_uint(x[2 * j + i]);
+          hi[i] = (k < 2 ? __builtin_elementwise_sub_sat(bits, 1u) : bits) & 0xffff0000u;
+          x[2 * j + i] -= __uint_as_float(hi[i]);
+        }
+        part[j] = hi[0] >> 16 | hi[1];
       }
       pf[k] = __builtin_bit_cast(bf16x8_t, part);
     }
