@@ -583,7 +583,6 @@ void decode_attn(at::Tensor q, at::Tensor kc, at::Tensor vc, c10::optional<at::T
   nxd::decode_attn_set_prefetch(nullptr, 0, nullptr, 0, 0);   // armed ranges never outlive one call
 }
 
-// k, v: [B, T, Hkv, D] strided; caches [Bc, Hkv, Lmax, D]; pos: int32 [B] position of token 0
 // rope_inplace of the first nq + nkv heads of qkv [B, T, (nq + 2 nkv) D] and kv_cache_write of the last 2 nkv
 void rope_kv_write(at::Tensor qkv, int64_t nq, int64_t nkv, at::Tensor cos_t, at::Tensor sin_t, at::Tensor pos, at::Tensor kc, at::Tensor vc,
                    c10::optional<at::Tensor> cache_idx, at::Tensor pos0) {
@@ -617,6 +616,7 @@ void rope_kv_write(at::Tensor qkv, int64_t nq, int64_t nkv, at::Tensor cos_t, at
            "rope_kv_write");
 }
 
+// k, v: [B, T, Hkv, D] strided; caches [Bc, Hkv, Lmax, D]; pos: int32 [B] position of token 0
 void kv_cache_write(at::Tensor k, at::Tensor v, at::Tensor kc, at::Tensor vc, c10::optional<at::Tensor> cache_idx,
                     at::Tensor pos) {
   int64_t ks[3], vs[3];

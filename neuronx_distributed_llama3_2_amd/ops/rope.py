@@ -94,13 +94,20 @@ def rope_kv_write_(qkv: torch.Tensor, nq: int, nkv: int, cos_t: torch.Tensor, si
     values at pos0[b] + t, in one launch where the layouts allow it."""
     B, T, W = qkv.shape
     D = W // (nq + 2 * nkv)
-    if (use_native(qkv, k_cache) and D in (64, 128, 256) and qkv.is_contiguous() and k_cache.is_contiguous() and v_cache.is_contiguous()
-            and qkv.dtype == k_cache.dtype == torch.bfloat16 and B * T * (nq + 2 * nkv) < 2 ** 30):
+    native = use_native(qkv, k_cache)
+    if (native and D in (64, 128, 256) and qkv.is_contiguous() and k_cache.is_contiguous() and v_cache.is_contiguous()
+            and qkv.dtype == k_cache.dtype == torch.bfloat16 and k_cache.data_ptr() % 16 == v_cache.data_ptr() % 16 == 0
+            and B * T * (nq + 2 * nkv) < 2 ** 30):
         ext().rope_kv_write(qkv, nq, nkv, cos_t, sin_t, positions.to(torch.int64).contiguous(), k_cache, v_cache,
                             cache_idx.to(torch.int32).contiguous() if cache_idx is not None else None, pos0.to(torch.int32).contiguous())
         return
     from .decode import kv_cache_write
 
+    # what the cache write refuses is refused before qkv is rotated: a caller that makes good and calls again rotates once
+    if native and not (k_cache.dim() == 4 and k_cache.shape == v_cache.shape and k_cache.shape[1] == nkv and k_cache.shape[3] == D
+                       and k_cache.dtype == v_cache.dtype == torch.bfloat16 and k_cache.is_contiguous() and v_cache.is_contiguous()
+                       and pos0.numel() == B and (k_cache.shape[0] >= B if cache_idx is None else cache_idx.numel() == B)):
+        raise RuntimeError("rope_kv_write_: contiguous bf16 caches [slots, nkv, length, D], pos0 and cache_idx [B]")
     rope_inplace_(qkv.view(B * T, W), 0, nq + nkv, D, cos_t, sin_t, positions)
     heads = qkv.view(B, T, nq + 2 * nkv, D)
     kv_cache_write(heads[:, :, nq:nq + nkv], heads[:, :, nq + nkv:], k_cache, v_cache, pos0, cache_idx)

@@ -1,5 +1,5 @@
 """Rotation and cache write in one launch against the two launches: every head size, odd rows, entries before and past the cache's
-ends, other cache rows; layouts that it does not take go to the two."""
+ends, other cache rows, caches that are not aligned (the two).  Caches that neither takes are refused with the queries as they were."""
 import pytest
 import torch
 
@@ -35,3 +35,31 @@ def test_against_two_launches(B, T, nq, nkv, D, idx, view):
     ops.kv_cache_write(h[:, :, nq:nq + nkv], h[:, :, nq + nkv:], a[0], a[1], pos0, ci)
     ops.rope_kv_write_(qkv, nq, nkv, cos, sin, pos, b[0], b[1], pos0, ci)
     assert torch.equal(qkv, want) and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("what", ["view", "heads", "slots", "type"])
+def test_refused_before_the_rotation(what):
+    B, T, nq, nkv, D, L = 2, 5, 4, 2, 64, 16
+    qkv = torch.randn(B, T, (nq + 2 * nkv) * D, device="cuda").bfloat16()
+    cos, sin = (torch.randn(64, D // 2, device="cuda") for _ in range(2))
+    pos, pos0 = torch.arange(T, device="cuda").repeat(B), torch.zeros(B, dtype=torch.int32, device="cuda")
+    kc, vc = (torch.zeros(B, nkv, L, D, device="cuda").bfloat16() for _ in range(2))
+    bad = {"view": (kc[:, :, :8], vc[:, :, :8]), "heads": (kc[:, :1].contiguous(), vc[:, :1].contiguous()), "slots": (kc[:1], vc[:1]),
+           "type": (kc, vc.float())}[what]
+    kept = qkv.clone()
+    with pytest.raises(RuntimeError):
+        ops.rope_kv_write_(qkv, nq, nkv, cos, sin, pos, *bad, pos0)
+    assert torch.equal(qkv, kept)
+
+
+def test_caches_of_any_alignment():
+    B, T, nq, nkv, D, L = 2, 5, 4, 2, 64, 16
+    qkv = torch.randn(B, T, (nq + 2 * nkv) * D, device="cuda").bfloat16()
+    cos, sin = (torch.randn(64, D // 2, device="cuda") for _ in range(2))
+    pos, pos0 = torch.arange(T, device="cuda").repeat(B), torch.tensor([3, 0], dtype=torch.int32, device="cuda")
+    n = B * nkv * L * D
+    caches = [[torch.zeros(n + 2, device="cuda").bfloat16()[at:at + n].view(B, nkv, L, D) for _ in range(2)] for at in (0, 2)]
+    rows = [qkv.clone() for _ in caches]
+    for q, (kc, vc) in zip(rows, caches):
+        ops.rope_kv_write_(q, nq, nkv, cos, sin, pos, kc, vc, pos0)
+    assert torch.equal(rows[0], rows[1]) and all(torch.equal(a, b) for a, b in zip(*caches)) and caches[0][0].any()
