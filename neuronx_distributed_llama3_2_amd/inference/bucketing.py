@@ -42,7 +42,7 @@ def prefill_lengths(config, batch: int, halfway: bool = True) -> List[int]:
     holds HALFWAY_TOKENS in the batch."""
     lengths = list(config.buckets)
     top = getattr(config, "max_context_length", 0)
-    if halfway and getattr(config, "enable_bucketing", False) and top and lengths == generate_buckets(min(128, top), top):
+    if halfway and getattr(config, "buckets_generated", False) and top and lengths == generate_buckets(min(128, top), top):
         lengths += [lo * 3 // 2 for lo, hi in zip(lengths, lengths[1:]) if lo >= 128 and batch * hi >= HALFWAY_TOKENS and lo * 3 // 2 < hi]
     return lengths + [config.max_length]
 

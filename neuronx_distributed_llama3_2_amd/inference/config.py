@@ -37,9 +37,12 @@ class InferenceConfig:
         self.is_continuous_batching = kwargs.pop("is_continuous_batching", False)
         self.on_device_sampling = kwargs.pop("on_device_sampling", True)
         self.enable_bucketing = kwargs.pop("enable_bucketing", False)
-        self.buckets: List[int] = kwargs.pop("buckets", None) or (
+        given = kwargs.pop("buckets", None)
+        self.buckets: List[int] = given or (
             generate_buckets(min(128, self.max_context_length), self.max_context_length) if self.enable_bucketing
             else [self.max_context_length])
+        # a caller's list stands as it is, also where it equals the generated one (bucketing.prefill_lengths)
+        self.buckets_generated = kwargs.pop("buckets_generated", self.enable_bucketing and not given)
         self.token_generation_buckets: List[int] = kwargs.pop("token_generation_buckets", None) or [seq_len]
         self.bucket_n_active_tokens = False
         self.quantized = kwargs.pop("quantized", False)

@@ -29,6 +29,27 @@ def test_lengths(batch, top, given, want):
         pad_to_bucket(torch.zeros((1, 4097)), torch.zeros((1, 4097)), prefill_lengths(cfg, batch), 0)
 
 
+def test_a_list_of_the_callers_own_stands(tmp_path):
+    """Also where it is the one that would have been generated, and after saving; files from before the list's origin was kept in
+    them hold a list."""
+    import json
+
+    kw = dict(batch_size=3, seq_len=2048, max_context_length=1024, enable_bucketing=True)
+    made = InferenceConfig(**kw)
+    own = InferenceConfig(buckets=[128, 256, 512, 1024], **kw)
+    assert made.buckets == own.buckets
+    for cfg, more in ((made, [384, 768]), (own, [])):
+        cfg.save_pretrained(str(tmp_path))
+        for c in (cfg, InferenceConfig.from_pretrained(str(tmp_path))):
+            assert sorted(prefill_lengths(c, 3)) == sorted([128, 256, 512, 1024, 2048] + more)
+    made.save_pretrained(str(tmp_path))
+    path = tmp_path / "nxd_inference_config.json"
+    kept = json.loads(path.read_text())
+    del kept["buckets_generated"]
+    path.write_text(json.dumps(kept))
+    assert prefill_lengths(InferenceConfig.from_pretrained(str(tmp_path)), 3) == [128, 256, 512, 1024, 2048]
+
+
 def test_logits_do_not_depend_on_the_length():
     from test_inference import _hf_model, _tiny_cfg
     from neuronx_distributed_llama3_2_amd.inference import LlamaForCausalLMInference
