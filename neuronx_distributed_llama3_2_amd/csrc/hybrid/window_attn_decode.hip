@@ -597,7 +597,7 @@ __global__ void __launch_bounds__(256) attn_decode_kernel(WindowAttnParams p) {
       if (i * kpp < 16) {
         const int k = 16 * w + i * kpp + ks;
         f32x4_t x = widen(vr[i]);
-        if (has_new && k >= cnt - 1) x = k == cnt - 1 ? ld4(vn + col) : f32x4_t{0.f, 0.f, 0.f, 0.f};   // (past the end, where the weight is zero: zeros)
+        if (has_new && k >= cnt - 1) x = ld4(vn + col);   // (past the end: any finite value, its weight is zero)
 #pragma unroll
         for (int j = 0; j < NJ; ++j) a4[j] += x * pw[j][k];
       }
