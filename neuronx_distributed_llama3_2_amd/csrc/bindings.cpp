@@ -74,6 +74,7 @@ int dgemv_launch(int, const void*, int64_t, const void*, float, const void*, int
 int grouped_gemm_launch(int, const void*, const void*, void*, const int*, int, int, int, int, int, hipStream_t);
 int wgrad_gemm_launch(const void*, int64_t, const void*, int64_t, float*, int64_t, int, int, int, int, hipStream_t);
 int wgrad_gemm_choose_splits(int, int, int);
+void wgrad_gemm_plan(int, int, int, int, int*);
 int decode_attn_oproj_launch(const void*, const int64_t*, const void*, const void*, const int64_t*, const int*, const int*,
                              const void*, int64_t, int, float*, float*, float*, float*, float*, int, int, int, int, int, int, float, hipStream_t);
 int grouped_rowgemm_launch(int, const void*, const void*, void*, const int*, int, int, int, int, hipStream_t, float*, int*);
@@ -1248,6 +1249,13 @@ PYBIND11_MODULE(_C, m) {
     check_rc(nxd::cu_stream_launch(src.data_ptr(), dst.data_ptr(), bytes_per_block, (int)blocks, ticks, cur_stream()),
              "cu_stream");
   });
+  // {splits, whether the kernel for few tokens takes it} of wgrad_gemm into an aligned gradient
+  m.def("wgrad_gemm_plan", [](int64_t T, int64_t M, int64_t N, int64_t splits) {
+    TORCH_CHECK(T > 0 && M > 0 && N > 0 && T <= INT32_MAX && M <= INT32_MAX && N <= INT32_MAX, "wgrad_gemm_plan: sizes");
+    int out[2];
+    nxd::wgrad_gemm_plan((int)T, (int)M, (int)N, (int)splits, out);
+    return std::make_pair(out[0], (bool)out[1]);
+  }, py::arg("T"), py::arg("M"), py::arg("N"), py::arg("splits") = 0);
   m.def("wgrad_gemm_splits", [](int64_t T, int64_t M, int64_t N) { return nxd::wgrad_gemm_choose_splits((int)T, (int)M, (int)N); });
   m.def("moe_combine_fwd", &moe_combine_fwd);
   m.def("moe_combine_bwd", &moe_combine_bwd);

@@ -148,8 +148,11 @@ __global__ void __launch_bounds__(NT, 1) wgrad_kernel(Params p) {
 // to empty.  us here / by the loop above:
 //   * 8 experts' 4096 x 28672 and 14336 x 4096 gradients: 256 tokens each 1,762, 821 / 1,909, 947; 1,024 2,756, 1,372 / 2,867, 1,483;
 //     1,536 3,639, 1,824 / 3,545, 1,803; 4,096 7,857, 3,903 / 7,070, 3,561;
-//   * one gradient of 4096 x 4096, 480 tokens 36 / 38, 500 40 / 36, 700 45 / 40; 768 x 4096 or 128256 x 2048, 500 24, 560 / 28, 608, 700 29, 659 /
-//     32, 668, 1,000 38, 794 / 38, 788.
+//   * one gradient, whole steps of 32 tokens: 512 x 512 512 tokens 20 / 27, 1,024 32 / 37, 2,048 53 / 56, 3,072 75.3 / 74.9; 2048 x 2048 23 / 30, 34 /
+//     39, 56 / 58, 78 / 78; 3072 x 4096 1,056 46.3 / 48.9, 2,048 68 / 69; 4096 x 4096 512 39 / 42, 1,056 54 / 56, 1,536 69 / 67; 16384 x 2048 1,024
+//     102 / 109, 2,080 155 / 157, 3,072 205 / 199;
+//   * a partial last step (the loop's is its first): 4096 x 4096, 500 tokens 40 / 36, 700 45 / 40; 768 x 4096 or 128256 x 2048, 500 24, 560 / 28,
+//     608, 700 29, 659 / 32, 668, 1,000 38, 794 / 38, 788.
 //
 // Ping-pong: each stage is two phases of 16 MFMAs per wave, every phase [LDS-DMA half-stage][fragment reads] barrier [16 MFMAs at raised
 // priority] barrier, and wave group 1 (waves 4-7; every SIMD holds one wave of each group) runs one barrier behind group 0.  Ring
@@ -162,8 +165,11 @@ __global__ void __launch_bounds__(NT, 1) wgrad_kernel(Params p) {
 namespace few {
 
 constexpr int FEW = 1400;   // tokens of a group
-inline bool dense(int T, int tiles) { return T <= 450 || (T <= 700 && (tiles < 192 || tiles > 1024)); }
 constexpr int BK = 32, STAGES = 4, NT = 512;
+inline bool dense(int T, int tiles) {   // (one gradient, unsplit)
+  if (T % BK) return T <= 450 || (T <= 700 && (tiles < 192 || tiles > 1024));
+  return T <= 1056 || (T <= 2080 && (tiles < 160 || tiles > 256));
+}
 constexpr int IMG_BYTES = BK * 256 * 2;           // 16 KiB: one operand stage
 constexpr int STAGE_BYTES = 2 * IMG_BYTES;        // A | B
 constexpr int LDS_BYTES = STAGES * STAGE_BYTES;   // 128 KiB
@@ -200,21 +206,24 @@ __device__ __forceinline__ bf16x8_t frag(const char* img, int c0) {
   return __builtin_bit_cast(bf16x8_t, a8);
 }
 
+// TAIL: the last step may be a partial one (always with GROUPED).  The look at it costs every load a comparison and a selection:
+// without them 1024 x 1024 over 512 tokens 22.9 -> 21.2 us, 800 30.0 -> 27.3, 16384 x 2048 over 800 97 -> 93.
+template <bool GROUPED, bool TAIL>
 __global__ void __launch_bounds__(NT, 1) kernel(Params p) {
   __shared__ __attribute__((aligned(16))) char smem[LDS_BYTES];
   const int tiles = p.mt * p.nt;
   const int id = xcd_remap(blockIdx.x, gridDim.x);
-  const int ge = id / tiles;
+  const int ge = GROUPED ? id / tiles : 0;
   int rt, ct;
   {
-    const int within = id % tiles;
+    const int within = GROUPED ? id % tiles : id;
     const int kb = p.band, bnd = within / (kb * p.nt), rem = within - bnd * kb * p.nt;
     const int h = min(kb, p.mt - bnd * kb);
     rt = bnd * kb + rem % h;
     ct = rem / h;
   }
   const int m0 = rt * BM, n0 = ct * BN;
-  const int t_begin = p.offs ? p.offs[ge] : 0, t_end = p.offs ? p.offs[ge + 1] : p.T;
+  const int t_begin = GROUPED ? p.offs[ge] : 0, t_end = GROUPED ? p.offs[ge + 1] : p.T;
   if (t_begin >= t_end) return;      // empty group: nothing to add (workgroup-uniform)
   const int nk = ceil_div(t_end - t_begin, BK);
   float* cbase = p.c + ge * p.c_es;
@@ -251,7 +260,7 @@ __global__ void __launch_bounds__(NT, 1) kernel(Params p) {
     const uint32_t img = lds0 + (s % STAGES) * STAGE_BYTES + wid * PIECES * 1024;
     const uint16_t* sa = src_a[hh] + (int64_t)s * BK * p.ld_dy;
     const uint16_t* sb = src_b[hh] + (int64_t)s * BK * p.ld_x;
-    if (s * BK + tt_of[hh] >= rows) sa = sb = reinterpret_cast<const uint16_t*>(g_zero16);
+    if (TAIL && s * BK + tt_of[hh] >= rows) sa = sb = reinterpret_cast<const uint16_t*>(g_zero16);
     dma16(sa, __builtin_amdgcn_readfirstlane(img + hh * 1024));
     dma16(sb, __builtin_amdgcn_readfirstlane(img + IMG_BYTES + hh * 1024));
   };
@@ -362,25 +371,36 @@ void launch(const Params& p, int64_t nwg, hipStream_t stream) {
 
 }  // namespace wg
 
-// Token splits per output tile.  Cost model in token steps (1.3 us) of one workgroup, times 256: grid waves of 256 workgroups x the steps
-// per split, and the epilogues: 8 steps without a split; with splits the atomics' rate bounds all workgroups together, 40 steps for 256
-// tiles.  The smallest split count of minimal cost, of 8 steps at least.  Unsplit / in the given splits, us: 1,000 tokens 6144 x 4096 83 / 2:
-// 199, 2048 x 2048 40 / 2: 40; 3,000 tokens 3072 x 2048 76 / 2: 73 / 3: 109, 2048 x 2048 76 / 2: 59 / 4: 71; 8,192 tokens 6144 x 4096 372 / 2:
-// 411, 512 x 4096 168 / 4: 67 / 8: 76; 32,768 tokens 6144 x 4096 1,485 / 2: 1,305, 768 x 4096 670 / 5: 195 / 6: 288.
+// Token splits per output tile.  Cost model in token steps (1.2 us) of one workgroup, times 256: grid waves of 256 workgroups x the steps
+// per split, and the epilogues: 8 steps without a split; with splits 10 for one of them, and the atomics' rate bounds all workgroups together, 40
+// steps for 256 tiles.  The smallest split count of minimal cost, of 4 steps at least, from 1,024 tokens on (below, unsplit products of few tiles take
+// no longer than the shortest split ones and add in one order).  Unsplit / in the given splits, us: 1,000 tokens 6144 x 4096 83 / 2: 199,
+// 2048 x 2048 40 / 2: 40; 1,024 tokens 512 x 512 32 / 2: 25.7 / 4: 21.0, 1024 x 1024 32 / 2: 26.3 / 4: 22.0 / 8: 32, 768 x 4096 34 / 2: 34 / 3: 40;
+// 3,000 tokens 3072 x 2048 76 / 2: 73 / 3: 109, 2048 x 2048 76 / 2: 59 / 4: 71; 4,096 tokens 512 x 512 94 / 8: 26 / 16: 22; 8,192 tokens 6144 x 4096
+// 372 / 2: 411, 512 x 4096 168 / 4: 67 / 8: 76; 32,768 tokens 6144 x 4096 1,485 / 2: 1,305, 768 x 4096 670 / 5: 195 / 6: 288.
 int wgrad_gemm_choose_splits(int T, int M, int N) {
   const int64_t tiles = (int64_t)ceil_div(M, wg::BM) * ceil_div(N, wg::BN);
   const int steps = ceil_div(T, wg::BK);
   int best = 1;
   int64_t best_cost = INT64_MAX;
   for (int s = 1; s <= 32 && s <= steps; ++s) {
-    if (s > 1 && steps / s < 8) break;
-    const int64_t cost = (tiles * s + 255) / 256 * 256 * ceil_div(steps, s) + (s == 1 ? 8 * 256 : 40 * tiles * s);
+    if (s > 1 && (steps < 16 || steps / s < 4)) break;
+    const int64_t cost = (tiles * s + 255) / 256 * 256 * ceil_div(steps, s) + (s == 1 ? 8 * 256 : std::max<int64_t>(10 * 256, 40 * tiles * s));
     if (cost < best_cost) {
       best_cost = cost;
       best = s;
     }
   }
   return best;
+}
+
+// Of a product into an aligned gradient: {splits, whether the kernel for few tokens takes it}
+void wgrad_gemm_plan(int T, int M, int N, int splits, int* out) {
+  const int steps = ceil_div(T, wg::BK);
+  if (splits <= 0) splits = wgrad_gemm_choose_splits(T, M, N);
+  splits = std::min(splits, steps);
+  out[0] = ceil_div(steps, ceil_div(steps, splits));
+  out[1] = out[0] == 1 && wg::few::dense(T, (int)std::min<int64_t>((int64_t)ceil_div(M, wg::BM) * ceil_div(N, wg::BN), INT32_MAX));
 }
 
 // c [M, N] fp32 += dy[T, M]^T x[T, N]; M % 8 == 0, N % 8 == 0, 16-B aligned rows.
@@ -406,7 +426,7 @@ int wgrad_gemm_launch(const void* dy, int64_t ld_dy, const void* x, int64_t ld_x
   const int64_t nwg = (int64_t)p.mt * p.nt * p.splits;
   if (nwg > INT32_MAX) return -2;
   if (p.own && wg::few::dense(T, p.mt * p.nt))
-    hipLaunchKernelGGL(wg::few::kernel, dim3((unsigned)nwg), dim3(wg::few::NT), 0, stream, p);
+    hipLaunchKernelGGL((T % wg::few::BK ? &wg::few::kernel<false, true> : &wg::few::kernel<false, false>), dim3((unsigned)nwg), dim3(wg::few::NT), 0, stream, p);
   else if (T % wg::BK)
     wg::launch<false, true>(p, nwg, stream);
   else
@@ -440,7 +460,7 @@ int wgrad_gemm_grouped_launch(const void* dy, int64_t ld_dy, const void* x, int6
   const int64_t nwg = (int64_t)p.mt * p.nt * E * p.splits;
   if (nwg > INT32_MAX) return -2;
   if (p.own && rows / E <= wg::few::FEW) {
-    hipLaunchKernelGGL(wg::few::kernel, dim3((unsigned)nwg), dim3(wg::few::NT), 0, stream, p);
+    hipLaunchKernelGGL((wg::few::kernel<true, true>), dim3((unsigned)nwg), dim3(wg::few::NT), 0, stream, p);
     return hipGetLastError() == hipSuccess ? 0 : -3;
   }
   wg::launch<true, true>(p, nwg, stream);

@@ -161,10 +161,11 @@ def _use_wgrad_kernel(mg: torch.Tensor, go2: torch.Tensor, x2: torch.Tensor, has
 
 
 # Whole steps of 64 tokens and no producer copy, M N / (M + N) < 2200: the wgrad kernel as well, with its own choice of splits.
-# Against the library with its two transposes / the TN form of csrc/dense_gemm.hip that was here before, time of the former = 1:
-# 4,096 x 4,096 0.71-0.89 / 0.85-0.92 over 64 to 32,768 tokens, 16,384 x 2,048 0.82-0.90 / 0.67-0.90, 2,048 x 8,192 0.75-0.85 /
-# 0.89-1.01, 768 x 4,096 0.83 / 0.94 over 32,768 (1.3-1.9 / 0.80-0.99 over 512 to 4,096).  NXD_DENSE_WGRAD = auto | 1 (whenever the
-# shapes allow) | 0.
+# Its time over the library's (with two transposes from M N / (M + N) = 1,200 on), 64 to 32,768 tokens: 4,096 x 4,096 0.74-0.88,
+# 2,048 x 8,192 0.77-0.85, 16,384 x 2,048 0.82-0.95, 3,584 x 4,096 0.81-0.95, 3,072 x 4,096 0.81-1.0; from 16,384 tokens on also smaller
+# ones (2,048 x 2,048 0.8, 512 x 4,096 0.7-0.8).  The library is faster for few tiles over few tokens: 2,048 x 2,048 1.4-1.6 over 64 to 4,096
+# tokens, 768 x 4,096 1.3-1.9, 512 x 512 1.2-2.5.  Time over that of the TN form of csrc/dense_gemm.hip, which was here before: 0.67-1.01.
+# NXD_DENSE_WGRAD = auto | 1 (whenever the shapes allow) | 0.
 _DENSE_WG = os.environ.get("NXD_DENSE_WGRAD", "auto")
 _DENSE_WG_SKINNY = 2200.0
 

@@ -1,0 +1,33 @@
+"""Which loop of the weight-gradient kernel takes a product, and in how many splits; and both loops at the line between them, against
+float64.  The lines were measured: the kernel for few tokens is faster up to them, the tile loop from them on."""
+import pytest
+import torch
+
+from test_wgrad_tiles_gpu import _among_nans, _check
+
+from neuronx_distributed_llama3_2_amd.ops._ext import ext
+
+
+@pytest.mark.parametrize("T,M,N,splits,few", [
+    (64, 512, 512, 1, True), (512, 1024, 1024, 1, True), (800, 2048, 2048, 1, True), (960, 768, 4096, 1, True), (960, 256, 2048, 1, True),
+    (1056, 3072, 4096, 1, True), (1056, 4096, 4096, 1, True), (1088, 4096, 4096, 1, False), (1088, 3072, 4096, 1, False),    # 192, 256 tiles
+    (2080, 2048, 4096, 1, True), (2112, 2048, 4096, 1, False), (2080, 16384, 2048, 1, True), (2112, 16384, 2048, 1, False),  # 128, 512
+    (450, 4096, 4096, 1, True), (451, 4096, 4096, 1, False), (700, 2048, 2048, 1, True), (701, 2048, 2048, 1, False),        # partial steps
+    (1024, 512, 512, 4, False), (1024, 1024, 1024, 4, False), (1024, 768, 4096, 2, False), (2048, 256, 2048, 8, False),      # few tiles
+    (4096, 512, 512, 16, False), (2048, 2048, 2048, 2, False), (8192, 6144, 4096, 1, False), (32768, 768, 4096, 5, False),
+])
+def test_plan(T, M, N, splits, few):
+    assert ext().wgrad_gemm_plan(T, M, N) == (splits, few)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,M,N", [(1024, 264, 8), (1056, 264, 8), (1024, 3328, 3848), (1056, 3328, 3848), (1057, 3328, 3848), (1088, 3328, 3848),
+                                   (2080, 520, 512), (2112, 520, 512), (4096, 264, 520), (4095, 8, 8)])
+@pytest.mark.parametrize("splits", [0, 1])
+def test_at_the_lines(T, M, N, splits):
+    g = torch.Generator(device="cuda").manual_seed(T + M)
+    dy, x = _among_nans(T, M, g), _among_nans(T, N, g)
+    mg = torch.randn(M, N, generator=g, device="cuda")
+    before = mg.clone()
+    ext().wgrad_gemm(mg, dy, x, splits, True)
+    _check(mg, before, dy, x)
