@@ -590,12 +590,23 @@ static Splits splits_of(int Lmax, int B, int Hkv, int M, int D, bool tickets) {
     // Not where two parts a head leave a sixth of the CUs idle and three are too many (D 64, 12 of 2,304 keys 13.1 / 13.7), nor where the call is
     // so short that 8 waves start later than 4 (1 of 640 6.7 / 7.3).  Whole heads of many keys only where the rule below gives a wave as many:
     // one long sequence among short ones is what the call waits for then (no more than 2,560 keys for 8 waves; D 128, 24 heads x 8 of 2,304 keys, all 36.0 / 32.5, one 18.5 / 26.8).
-    const int64_t heads = (int64_t)B * Hkv, fit = std::max<int64_t>(1, (D == 64 ? 270 : heads < 40 ? 256 : 320) / heads);
-    const int n = D == 64 && Lmax <= 640 ? 1 : (int)std::min<int64_t>(fit, MD > 256 ? 16 : 24);
-    const int least = D == 64 || heads >= 64 ? 256 : 128, full = std::max(least, (ceil_div(Lmax, n) + KB - 1) / KB * KB);
+    // No more than about one workgroup a CU where all of them have keys, or a second round begins: with full parts of less than 320 keys (D 128, us in 320
+    // workgroups / in 288 at most / by the rule below: 5 of 1,024 keys 13.0 / 9.8 / 11.7, 8 of 1,280 14.4 / 12.0 / 14.1, 13 of 768 14.2 / 12.5 / 13.8, 20
+    // of 512 14.4 / 11.8 / 13.9; the last part half empty, 13 of 640 10.5 / 11.2 / 13.4), and where a launch of its own merges (more than 1,024 sums a head; four new tokens, 5 of 1,024 19.9 / 15.9 / 17.5, 8
+    // of 1,280 22.4 / 18.5 / 20.2, 13 of 1,536 26.9 / 23.4 / 24.3; but two parts of 160 heads from 1,280 keys on, 20 of 1,756 29.9 / 31.3 by the rule
+    // below).  There parts of 128 keys, half a chunk a wave, of more than 256 workgroups, or a last one that is mostly empty, are no better
+    // than 4 waves: 7 of 640 17.5 / 16.4 by the rule below, 6 of 768 17.3 / 16.3, three new tokens 8 of 384 13.9 / 13.4.
+    const int64_t heads = (int64_t)B * Hkv;
+    const bool apart = MD > 1024;   // (merge_in_launch)
+    const int least = D == 64 || heads >= 64 ? 256 : 128;
+    auto parts = [&](int64_t wgs) { return D == 64 && Lmax <= 640 ? 1 : (int)std::min(std::max<int64_t>(1, wgs / heads), MD > 256 ? int64_t{16} : int64_t{24}); };
+    auto keys = [&](int n) { return std::max(least, (ceil_div(Lmax, n) + KB - 1) / KB * KB); };
+    int n = parts(D == 64 ? 270 : heads < 40 ? 256 : apart && (heads <= 144 || Lmax < 1280) ? 288 : 320), full = keys(n);
+    if (n * heads > 288 && full < 320 && n * full < Lmax + full / 2) n = parts(288), full = keys(n);
     const bool idle = D == 64 && n == 2 && heads < 112, brief = D == 64 && heads < 32 && Lmax <= 1280;
     const bool uneven = n == 1 && heads < 224 && Lmax > (D == 64 ? 1280 : 640);
-    if (full <= 2560 && !idle && !brief && !uneven) return {Lmax, full, std::min(full, heads >= 64 ? 512 : least), full, 8};
+    const bool thin = apart && n > 1 && (full < 192 && n * heads > 256 || heads == 64 && Lmax <= 2 * full);
+    if (full <= 2560 && !idle && !brief && !uneven && !thin) return {Lmax, full, std::min(full, heads >= 64 ? 512 : least), full, 8};
   }
   static const int target = [] {
     const char* e = getenv("NXD_DECODE_ATTN_WGS");

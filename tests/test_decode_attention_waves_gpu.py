@@ -42,3 +42,31 @@ def test_attention(D, B, Hkv, G, T, L):
         assert torch.isfinite(out).all() and rms(err) <= 2.0 ** -8 * rms(ref)
         assert (err <= 2.0 ** -9 * ref.abs() + 2.0 ** -8 * 4.5 * 0.25 + 1e-6).all()   # (values up to 4.5 or so)
     assert not tickets.any()
+
+
+@pytest.mark.parametrize("room,B,M,splits,keys", [
+    (1024, 5, 4, 6, 192), (1024, 5, 8, 6, 192), (1536, 5, 4, 6, 256), (1280, 8, 4, 4, 320), (1024, 10, 4, 3, 384), (768, 13, 4, 2, 384), (512, 20, 4, 1, 512),
+    (640, 13, 4, 3, 256), (1756, 13, 4, 3, 640), (2304, 5, 4, 8, 320),                                  # the last part half empty; longer parts
+    (1024, 5, 16, 6, 192), (1280, 8, 16, 4, 320), (1280, 10, 12, 3, 448), (1536, 13, 16, 2, 768),       # merged by a launch of its own
+    (640, 7, 16, 5, 128), (768, 6, 16, 6, 128), (384, 8, 12, 3, 128), (512, 8, 16, 4, 128), (640, 8, 16, 3, 256),
+    (1280, 20, 16, 2, 640), (1279, 20, 16, 3, 448)])
+def test_no_second_round(room, B, M, splits, keys):
+    """8 heads of 128: parts that all have keys are no more than a round of workgroups; where a launch merges them no parts are."""
+    assert ops.ext().decode_attn_plan(room, B, 8, M, 128, room, True)[:2] == (splits, keys)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,T,L", [(5, 4, 1024), (7, 4, 640), (8, 3, 384), (13, 4, 768), (20, 1, 512), (10, 3, 1280)])
+def test_attention_in_one_round(B, T, L):
+    g = torch.Generator(device="cuda").manual_seed(L + B)
+    q, k, v = (torch.randn(s, generator=g, device="cuda").bfloat16() for s in ((B, T, 32, 128), (B, 8, L, 128), (B, 8, L, 128)))
+    lengths = [max(n, T) for n in (L, 1, 255, 257, L - 1, L // 2, 129, 321, 0)]
+    lengths = [min(lengths[i % len(lengths)], L) for i in range(B)]
+    for b, n in enumerate(lengths):   # keys past the end are never read
+        k[b, :, n:] = float("nan")
+        v[b, :, n:] = float("nan")
+    tickets = torch.zeros(B * 8, dtype=torch.int32, device="cuda")
+    out = ops.decode_attention(q, k, v, torch.tensor(lengths, dtype=torch.int32, device="cuda"), tickets=tickets).double().cpu()
+    ref, size = (_reference(q, k, x, lengths, range(B)) for x in (v, v.abs()))
+    # half an ulp of bf16 (8 significant bits) of the result and of each probability: 2^-8 of |result| and of the sum of p |v|; fp32 sums
+    assert ((out - ref).abs() <= 2.0 ** -8 * (ref.abs() + size) + 2.0 ** -16 * size).all() and not tickets.any()
