@@ -78,7 +78,7 @@ void wgrad_gemm_plan(int, int, int, int, int*);
 int decode_attn_oproj_launch(const void*, const int64_t*, const void*, const void*, const int64_t*, const int*, const int*,
                              const void*, int64_t, int, float*, float*, float*, float*, float*, int, int, int, int, int, int, float, hipStream_t);
 int grouped_rowgemm_launch(int, const void*, const void*, void*, const int*, int, int, int, int, hipStream_t, float*, int*);
-int64_t grouped_rowgemm_workspace(int, int*);
+int64_t grouped_rowgemm_workspace(int, int, int, int, int*);
 int wgrad_gemm_grouped_launch(const void*, int64_t, const void*, int64_t, float*, int64_t, int64_t, const int*, int, int,
                               int, int, hipStream_t);
 int dense_gemm_launch(int, int, const void*, int64_t, const void*, int64_t, void*, int64_t, int, int, int, int, hipStream_t);
@@ -921,7 +921,7 @@ void grouped_gemm(int64_t mode, at::Tensor a, at::Tensor b, at::Tensor offs, at:
   if ((mode == 0 || mode == 1) && row_kernel) {
     // 256 x 256 tiles (csrc/grouped_rowgemm.hip); -1 = shape it does not take (reduction % 32)
     int tickets = 0;
-    const int64_t floats = M > 0 ? nxd::grouped_rowgemm_workspace((int)(mode == 0 ? K : N), &tickets) : 0;
+    const int64_t floats = nxd::grouped_rowgemm_workspace((int)(mode == 0 ? K : N), (int)(mode == 0 ? N : K), (int)M, (int)E, &tickets);
     at::Tensor ws, counters;
     if (floats) {
       ws = at::empty({floats}, a.options().dtype(at::kFloat));
@@ -1256,6 +1256,13 @@ PYBIND11_MODULE(_C, m) {
     nxd::wgrad_gemm_plan((int)T, (int)M, (int)N, (int)splits, out);
     return std::make_pair(out[0], (bool)out[1]);
   }, py::arg("T"), py::arg("M"), py::arg("N"), py::arg("splits") = 0);
+  // {bytes, counters} with which grouped_gemm splits reductions of `red` (modes 0 and 1)
+  m.def("grouped_gemm_workspace", [](int64_t red, int64_t ncols, int64_t rows, int64_t E) {
+    TORCH_CHECK(red >= 0 && ncols >= 0 && rows >= 0 && E >= 0 && std::max({red, ncols, rows}) <= INT32_MAX && E < 65536, "grouped_gemm_workspace: sizes");
+    int tickets = 0;
+    const int64_t floats = nxd::grouped_rowgemm_workspace((int)red, (int)ncols, (int)rows, (int)E, &tickets);
+    return std::make_pair(4 * floats, tickets);
+  });
   m.def("wgrad_gemm_splits", [](int64_t T, int64_t M, int64_t N) { return nxd::wgrad_gemm_choose_splits((int)T, (int)M, (int)N); });
   m.def("moe_combine_fwd", &moe_combine_fwd);
   m.def("moe_combine_bwd", &moe_combine_bwd);

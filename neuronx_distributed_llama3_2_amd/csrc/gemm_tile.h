@@ -58,6 +58,7 @@ struct Loop {
   uint32_t off[16];        // of this lane's pieces of A (0 .. 7) and B from a step's base
   const char *pa, *pb;     // the bases of the next step to load
   int64_t da, db;          // ... and from one step to the next
+  int pieces;              // (ROW images) pieces of A with rows that there are
   uint32_t back;           // (reductions that end with half a step) pieces of the last step whose second half is past the end, a bit each
 
   // A: rows 0 .. rows - 1 from `a` on (ROW: a row is lda elements; TR: a reduction row), clamped to the last; B likewise
@@ -66,7 +67,7 @@ struct Loop {
     lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
     pa = uniform(reinterpret_cast<const char*>(a)), pb = uniform(reinterpret_cast<const char*>(b));
     da = AT ? (int64_t)BK * lda * 2 : BK * 2, db = BT ? (int64_t)BK * ldb * 2 : BK * 2;
-    back = 0;
+    back = 0, pieces = min(max((rows + 7) / 8 - 8 * wid, 0), 8);
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const bool tr = i < 8 ? AT : BT;
@@ -125,8 +126,9 @@ struct Loop {
     else return read_row(rb[h ^ (j & 1)] + buf + (j & 1) * 512 + (j >> 1) * 4096);
   }
 
-  template <bool HALF>
+  template <bool HALF, bool FEW>
   __device__ __forceinline__ void load(int i, int buf, bool last) {   // piece i of the next step; HALF, last: its second half is past the end
+    if (FEW && i < 8 && i >= pieces) return;
     const uint32_t to = lds + buf + (i < 8 ? 0 : IMG_BYTES) + (8 * wid + (i & 7)) * 1024;
     uint32_t from = off[i];
     if constexpr (HALF) {   // (the first half again: not used)
@@ -142,6 +144,7 @@ struct Loop {
   __device__ __forceinline__ void run(f32x4_t (&acc)[8][8], int steps, bool end = false, int rows = BK) {
     static_assert(!FIRST || AT && BT && !HALF, "images of whole reduction rows");
     static_assert(IM == 8 || IM == 4, "rows");
+    constexpr bool FEW = IM == 4 && !AT;   // only rows that there are (what the LDS holds in the others' place counts for no result)
     bf16x8_t a0[IM], b0[8], a1[IM], b1[8];
     auto advance = [&](int s) {   // towards step s
       if (s < steps) pa += da, pb += db;
@@ -157,16 +160,17 @@ struct Loop {
       if (steps > 1) pa += da / BK * rows, pb += db / BK * rows;
     } else {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) load<HALF>(i, 0, end && steps == 1);
+      for (int i = 0; i < 16; ++i) load<HALF, FEW>(i, 0, end && steps == 1);
       advance(1);
     }
     if (!FIRST || steps > 1) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) load<HALF>(i, STEP_BYTES, end && steps <= 2);   // (past the end: the last step again, not used)
+      for (int i = 0; i < 16; ++i) load<HALF, FEW>(i, STEP_BYTES, end && steps <= 2);   // (past the end: the last step again, not used)
     }
     advance(2);
     addresses();
     if (FIRST && steps == 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    else if (FEW) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");   // (B's pieces of the second step are 8 in every wave)
     else asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -209,7 +213,7 @@ struct Loop {
       for (int u = 0; u < 16; ++u) {
         if (u < 8) b0[u] = frag_b(u, 0, next);
         else if (u - 8 < IM) a0[u - 8] = frag_a(u - 8, 0, next);
-        load<HALF>(u, buf, end && t + 3 >= steps);
+        load<HALF, FEW>(u, buf, end && t + 3 >= steps);
         mfmas(u, a1, b1);
       }
       buf = next;

@@ -14,6 +14,10 @@
 // the tiles are numbered in an L2 band raster over (row tile, column tile).
 // 8,192 rows of 8 experts, 4096 -> 28672 and 14336 -> 4096, us: FWD 2,170 -> 1,934 and 1,049 -> 943, DGRAD 2,263 -> 1,770 and
 // 1,057 -> 832 (two ping-pong groups of 4 waves, grid of the worst case's tiles).
+// Few rows (bound by the weights' bytes): a tile of at most 128 rows loads and leaves in memory only the rows that there are.  16 rows of 8
+// experts, FWD / DGRAD us, two groups of 4 waves -> here, and with all rows loaded and left: 4096 -> 28672 414 / 422 -> 414 / 387, 444 / 420; 14336 -> 4096
+// 311 / 307 -> 214 / 217, 245 / 245; 4096 -> 1024 93 / 91 -> 55 / 52, 76 / 72.  What is not split waits for each step's loads, one step ahead: 16
+// experts, 6144 -> 2688, 140 / 152 -> 142 / 162.
 #include "gemm_tile.h"
 
 #include <cstdlib>
@@ -39,17 +43,27 @@ struct Params {
   int rt, nt;           // worst-case row tiles, column tiles
   int band;
   // Sums of the tiles left over from whole rounds of an XCD's CUs, their reductions in parts (nullable: never), and zeroed counters
-  // (left zeroed); sizes: grouped_rowgemm_workspace
+  // (left zeroed): so many places an XCD, of so many fragments of 32 rows (room_for)
   float* ws;
   int* tickets;
+  int slots, frags;
 };
 
 constexpr int XCDS = 8, XCD_CUS = 32;
 // Parts of a tile at most; reduction steps of a part at least: writing a part's sums and reading them all back takes 25-40 us, 32
 // steps take 55
 constexpr int MAX_PARTS = 8, MIN_STEPS = 32;
-constexpr int TILE_FLOATS = BM * BN;
+constexpr int FRAG_FLOATS = 32 * BN;   // 32 rows of a tile
 
+// Room for what may be split, by what is known of the rows: an expert's tile has no more rows than there are, and of the places one XCD's
+// tiles need all (32 CUs) or, where there are few tiles, their parts.  8 experts, reduction 4096, columns 256 / 1,024 / 28,672: 16 rows 0.5, 2.1,
+// 8.4 MB, 256 rows 8.4, 21, 67 MB (for a whole tile a CU always 67).
+static void room_for(int red, int ncols, int rows, int E, int* slots, int* frags) {
+  const int most = ceil_div(red, BK) / MIN_STEPS, parts = most < MAX_PARTS ? most : MAX_PARTS;
+  const int64_t tiles = (int64_t)ceil_div(ncols, BN) * (rows / BM + (E < rows ? E : rows)), places = ceil_div64(tiles, XCDS) * parts;
+  *slots = parts < 2 || rows <= 0 ? 0 : (int)(places < XCD_CUS ? places : XCD_CUS);
+  *frags = rows > BM / 2 ? BM / 32 : ceil_div(rows, 32);
+}
 
 // HALF: the reduction ends with half a step
 template <int MODE, bool HALF>
@@ -65,7 +79,7 @@ __global__ void __launch_bounds__(NT, 1) rowgemm_kernel(Params p) {
   const int whole = share / XCD_CUS * XCD_CUS, tail = share - whole;
   const int steps = (p.red + BK - 1) / BK;
   int parts = 1, part = 0, id = base + idx;
-  if (p.ws && tail > 0) parts = max(1, min(min(XCD_CUS / tail, MAX_PARTS), steps / MIN_STEPS));
+  if (p.ws && tail > 0) parts = max(1, min(min(p.slots / tail, MAX_PARTS), steps / MIN_STEPS));
   if (idx >= whole) {
     const int j = idx - whole;
     if (j >= tail * parts) return;
@@ -121,13 +135,26 @@ __global__ void __launch_bounds__(NT, 1) rowgemm_kernel(Params p) {
 
   // ---- parts of a tile: sums to memory; the last part to come adds them up, in their order
   if (parts > 1) {
-    const int slot = xcd * XCD_CUS + idx - whole - part;   // of the tile's first part
-    float* sums = p.ws + (int64_t)slot * TILE_FLOATS;
-    auto at = [&](int s, int i, int j) { return reinterpret_cast<f32x4_t*>(sums + (int64_t)s * TILE_FLOATS) + ((wid * 8 + i) * 8 + j) * 64 + lane; };
+    const int slot = xcd * p.slots + idx - whole - part;   // of the tile's first part
+    const int64_t place = (int64_t)p.frags * FRAG_FLOATS;
+    float* sums = p.ws + slot * place;
+    const bool most = r1 - r0 > BM / 2;
+    const int have = most ? 8 : (r1 - r0 + 31) / 32;       // fragments with rows, or all
+    // (each wave's sums lie together: a fragment's of all waves beside each other, 1,024 rows of 4 experts, 8192 -> 256, 99 -> 111 us)
+    auto at = [&](int s, int i, int j) { return reinterpret_cast<f32x4_t*>(sums + s * place) + ((wid * p.frags + i) * 8 + j) * 64 + lane; };
+    if (most) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+      for (int i = 0; i < 8; ++i)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) *at(part, i, j) = acc[i][j];
+        for (int j = 0; j < 8; ++j) *at(part, i, j) = acc[i][j];
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (i < have) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) *at(part, i, j) = acc[i][j];
+        }
+    }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
     __syncthreads();
     int* last = reinterpret_cast<int*>(smem);
@@ -138,14 +165,26 @@ __global__ void __launch_bounds__(NT, 1) rowgemm_kernel(Params p) {
     __syncthreads();
     if (!*last) return;
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    for (int s = 0; s < parts; ++s) {
+    if (most) {
+      for (int s = 0; s < parts; ++s) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
+        for (int i = 0; i < 8; ++i)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const f32x4_t v = *at(s, i, j);
-          acc[i][j] = s == 0 ? v : acc[i][j] + v;
-        }
+          for (int j = 0; j < 8; ++j) {
+            const f32x4_t v = *at(s, i, j);
+            acc[i][j] = s == 0 ? v : acc[i][j] + v;
+          }
+      }
+    } else {
+      for (int s = 0; s < parts; ++s) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)   // (fragments without rows: any sums)
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            const f32x4_t v = *at(s, min(i, have - 1), j);
+            acc[i][j] = s == 0 ? v : acc[i][j] + v;
+          }
+      }
     }
   }
 
@@ -184,18 +223,20 @@ static int band_rows() {
 
 }  // namespace grg
 
-// Floats of ws and the number of tickets for a reduction of `red` (0: its tiles are never split)
-int64_t grouped_rowgemm_workspace(int red, int* tickets) {
-  const bool pays = red / grg::BK >= 2 * grg::MIN_STEPS;
-  *tickets = pays ? grg::XCDS * grg::XCD_CUS : 0;
-  return (int64_t)*tickets * grg::TILE_FLOATS;
+// Floats of ws and the number of tickets for a product of `rows` rows of E experts, a reduction of `red` and `ncols` columns (0: its tiles are
+// never split)
+int64_t grouped_rowgemm_workspace(int red, int ncols, int rows, int E, int* tickets) {
+  int slots, frags;
+  grg::room_for(red, ncols, rows, E, &slots, &frags);
+  *tickets = grg::XCDS * slots;
+  return (int64_t)*tickets * frags * grg::FRAG_FLOATS;
 }
 
 // mode 0 FWD:   a = x [rows, K],  W [E, K, N], c = y  [rows, N]
 // mode 1 DGRAD: a = dy [rows, N], W [E, K, N], c = dx [rows, K]
 // Requires the reduction length % 32 == 0 and K, N % 8 == 0 (checked; returns -1 otherwise, the
 // caller then takes the 128-tile kernel).  Rows past offs[E] are not written.
-// ws, tickets: of grouped_rowgemm_workspace()'s sizes (tickets zeroed), or null.
+// ws, tickets: of grouped_rowgemm_workspace()'s sizes (tickets zeroed), or null: unsplit.
 int grouped_rowgemm_launch(int mode, const void* a, const void* w, void* c, const int* offs, int E, int rows, int K,
                            int N, hipStream_t stream, float* ws, int* tickets) {
   if (E <= 0 || K <= 0 || N <= 0 || rows < 0 || K % 8 || N % 8) return -1;
@@ -220,7 +261,8 @@ int grouped_rowgemm_launch(int mode, const void* a, const void* w, void* c, cons
   p.rt = ceil_div(rows, grg::BM) + E;
   p.nt = ceil_div(p.ncols, grg::BN);
   p.band = grg::band_rows();
-  p.ws = tickets ? ws : nullptr;
+  grg::room_for(p.red, p.ncols, rows, E, &p.slots, &p.frags);
+  p.ws = tickets && p.slots ? ws : nullptr;
   p.tickets = tickets;
   const int64_t nwg = (ceil_div64((int64_t)p.rt * p.nt, grg::XCDS) + (p.ws ? grg::XCD_CUS : 0)) * grg::XCDS;
   if (nwg > INT32_MAX) return -2;

@@ -22,7 +22,7 @@ int linear_few_launch(const LinearFewParams&, hipStream_t);
 int expert_rows_launch(bool, const ExpertRowsParams&, hipStream_t);
 int grouped_gemm_launch(int, const void*, const void*, void*, const int*, int, int, int, int, int, hipStream_t);
 int grouped_rowgemm_launch(int, const void*, const void*, void*, const int*, int, int, int, int, hipStream_t, float*, int*);
-int64_t grouped_rowgemm_workspace(int, int*);
+int64_t grouped_rowgemm_workspace(int, int, int, int, int*);
 }  // namespace nxd
 
 namespace {
@@ -242,7 +242,7 @@ void grouped_linear(Tensor x, Tensor w, Tensor offs, Tensor y) {
   check_align(w, "w");
   check_align(y, "y");
   int tickets = 0;
-  const int64_t floats = nxd::grouped_rowgemm_workspace((int)K, &tickets);
+  const int64_t floats = nxd::grouped_rowgemm_workspace((int)K, (int)N, (int)P, (int)E, &tickets);
   Tensor ws, counters;
   if (floats) {
     ws = at::empty({floats}, x.options().dtype(at::kFloat));
