@@ -497,6 +497,14 @@ PYBIND11_MODULE(_hybrid, m) {
         py::arg("softcap"), py::arg("window"), py::arg("lam"), py::arg("out_scale"), py::arg("out_eps"), py::arg("pos"),
         py::arg("lens"), py::arg("slots"), py::arg("kc"), py::arg("vc"), py::arg("y"), py::arg("from_buf"), py::arg("fused") = true);
   m.def("attn_decode", &attn_decode);
+  // (on the matrix instructions, query heads of a workgroup, workgroups that share their keys, 64-key tiles of each) for at most `seen` visible keys
+  m.def("attn_decode_plan", [](int64_t B, std::vector<int64_t> sizes, int64_t seen, bool f32) {
+    TORCH_CHECK(sizes.size() == 5 && sizes[1] >= 1 && sizes[0] % sizes[1] == 0 && B >= 1 && seen >= 1, "attn_decode_plan: B, (H, G, maps, D, V), keys");
+    nxd::WindowAttnParams p{};
+    p.B = (int)B, p.H = (int)sizes[0], p.G = (int)sizes[1], p.maps = (int)sizes[2], p.D = (int)sizes[3], p.V = (int)sizes[4];
+    nxd::attn_decode_plan(p, seen, f32);
+    return std::make_tuple(p.mfma, p.share, p.splits, p.tiles);
+  });
   m.def("pooled_prep", &pooled_prep);
   m.def("pooled_attn", &pooled_attn);
   m.def("pooled_decode", &pooled_decode);

@@ -10,6 +10,9 @@
 // that has a new key which ends a block writes the block's means (no query sees them before a later step).
 #include "window_attn.h"
 
+#include <algorithm>
+#include <cmath>
+
 namespace nxd {
 namespace hybrid {
 
@@ -875,18 +878,31 @@ static int run_decode(const WindowAttnParams& p, hipStream_t s) {
 // most `seen` visible keys
 void attn_decode_plan(WindowAttnParams& p, int64_t seen, bool f32) {
   const int rep = p.H / p.G;
-  // (few heads of few keys of one map have nothing to share: 1 sequence of 320 keys, 16 heads of 128 8.4 us by the kernel above, 8.7 here)
-  const bool brief = p.maps == 1 && (int64_t)p.B * p.G < 16 && seen <= 512;
-  p.mfma = !f32 && p.pool == 0 && (p.D == 64 || p.D == 128) && (p.V == 64 || p.V == 128) && rep * p.maps <= 16 && !brief;
+  const int64_t pairs = (int64_t)p.B * p.G;
+  // (few heads of few keys of one map have nothing to share: 1 sequence of 320 keys, 16 heads of 128 8.4 us by the kernel above, 8.7 here; 16
+  // sequences of 300 keys, 16 heads of a pair 11.5 / 12.2)
+  const bool brief = p.maps == 1 && pairs < (rep > 8 ? 17 : 16) && seen <= 512;
+  // Many heads of a key / value head are prepared and merged by four waves one after another, which the kernel above shares out over workgroups
+  // where there are few (sequence, key / value head) pairs with few keys: it stays up to pairs^1.5 keys = 25 maps heads^2.5.  us above / here, pairs
+  // x keys: 16 heads of 64 a pair 1 x 1,024 10.1 / 13.8, 8 x 1,024 12.7 / 14.1, 2 x 4,096 17.5 / 18.5, 1 x 16,384 26.7 / 29.4; 16 x 640 15.2 / 13.2, 4 x
+  // 4,096 19.4 / 18.8, 2 x 16,384 33.2 / 29.8; of 128 4 x 1,024 12.8 / 15.5, 12 x 1,024 18.0 / 15.9; 12 heads 2 x 1,024 10.3 / 12.1, 8 x 1,024 12.7 / 12.0; 8 heads
+  // 1 x 1,024 9.5 / 10.2, 2 x 2,048 14.3 / 13.7; 8 heads of two maps 4 x 300 10.8 / 12.9, 4 x 1,024 13.7 / 15.0, 8 x 640 14.7 / 14.1, 16 x 300 14.2 / 13.1; four
+  // heads never.
+  const bool serial = rep > 4 && pairs * sqrt((double)pairs) * seen <= 25. * p.maps * rep * rep * sqrt((double)rep);
+  p.mfma = !f32 && p.pool == 0 && (p.D == 64 || p.D == 128) && (p.V == 64 || p.V == 128) && rep * p.maps <= 16 && !brief && !serial;
   if (p.mfma) {
     // One workgroup a CU, as long as each of its waves has a chunk of 32 keys.  us by the kernel above -> here (256 workgroups / 512 / 1,024),
     // 16 heads of 64 + 128 with two maps and 4 key / value heads: 1 sequence of 1,024 visible keys 13.1 -> 11.2 (in twice as many parts 12.8),
     // 8 17.7 -> 13.5, 16 24.1 -> 16.1 / 17.4 / 17.3 (33 MB), 32 33.2 -> 20.7 / 21.3 / 30.4; 16 of 4,096 52 -> 31 / 32 / 40, of 300 20.6 -> 13.9; one map of
     // 128 16 of 1,024 19.2 -> 14.4 / 15.1 / 14.9.  A key / value head a head: two maps of 64 + 64, 16 of 1,024 29.2 -> 21.5; one of 64,
     // 32 of 300 13.3 -> 13.3.
+    // No more parts than their merge pays for: eight of them, of four heads, are a trip to memory of 1.2 us, a tile of 64 keys takes 0.8-1.0.  1
+    // sequence, parts by this / one a CU: 4 heads of 128 4,096 keys 13.0 / 13.2, 16,384 18 / 28.3; 8 of 64 4,096 14.2 / 16.9, 16,384 22.1 / 45.3.
     p.share = rep;
-    const int64_t tiles = (seen + 63) / 64, groups = (int64_t)p.B * p.G, most = (tiles + 1) / 2;
-    int64_t splits = 256 / groups;
+    const int64_t tiles = (seen + 63) / 64, most = (tiles + 1) / 2;
+    int64_t pays = 8;
+    while (pays < most && (2 * pays + 8) * (2 * pays + 8) * ((rep + 3) / 4) < 23 * tiles) pays += 8;   // (nearest to the square root of 5.7 tiles a trip)
+    int64_t splits = std::min(256 / pairs, pays);
     splits = splits < 1 ? 1 : (splits > most ? most : splits);
     p.tiles = (int)((tiles + splits - 1) / splits);
     p.splits = (int)((tiles + p.tiles - 1) / p.tiles);
