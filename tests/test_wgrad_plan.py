@@ -31,3 +31,21 @@ def test_at_the_lines(T, M, N, splits):
     before = mg.clone()
     ext().wgrad_gemm(mg, dy, x, splits, True)
     _check(mg, before, dy, x)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes", [[9000, 1000, 0, 6000], [2100] * 4, [12000, 1, 63, 4032]])
+def test_split_groups(sizes):
+    """Groups of more tokens than one loop takes, in splits by the longest that is likely; empty ones and ones shorter than the splits."""
+    g = torch.Generator(device="cuda").manual_seed(sum(sizes))
+    x, dy = (torch.randn(sum(sizes), n, generator=g, device="cuda").bfloat16() for n in (264, 520))
+    offs = torch.tensor([0] + sizes, device="cuda").cumsum(0).to(torch.int32)
+    mg = torch.randn(len(sizes), 264, 520, generator=g, device="cuda")
+    before = mg.clone()
+    ext().grouped_gemm(2, x, dy, offs, mg, True)
+    for e in range(len(sizes)):
+        a, b = int(offs[e]), int(offs[e + 1])
+        if b > a:
+            _check(mg[e], before[e], x[a:b], dy[a:b])
+        else:
+            assert torch.equal(mg[e], before[e])
