@@ -1278,6 +1278,7 @@ PYBIND11_MODULE(_C, m) {
     nxd::few_rows_workspace(M, N, K, &need);
     return need;
   });
+  m.def("few_rows_halved", &nxd::few_rows_halved);
   m.def("decode_set_knob", [](int which, int value) {
     if (which == 2) nxd::decode_attn_set_v2(value);
     else if (which == 3) nxd::dgemv_set_knob(2, value);

@@ -44,6 +44,9 @@ struct FewRowsParams {
 // Floats of FewRowsParams::ws and the number of its tickets for a product that is better split (0: it is not)
 int64_t few_rows_workspace(int M, int N, int K, int* tickets);
 
+// Whether a product of M rows with a norm, of N weight rows, takes half of the rows a workgroup
+bool few_rows_halved(int M, int N, int K);
+
 // 0: launched; < 0: not a call this kernel takes; 1: launch error
 int few_rows_launch(int epi, const FewRowsParams& p, hipStream_t stream);
 

@@ -633,6 +633,9 @@ static int parts(int M, int N, int K) {   // of the reduction; 0: not split
   return n > 32 || ceil_div(tiles, 256 / n) > 64 ? 0 : n;   // (a lane for every tile's ticket)
 }
 
+// Of 17 to 32 rows with a norm: whether a workgroup takes half of them
+static bool halved(int nck, int64_t tiles) { return nck <= 16 ? tiles <= 512 : tiles <= 2048; }
+
 template <int EPI, bool NORM, bool XI, int MT, bool I8>
 static int pick(const FewRowsParams& p, hipStream_t s) {
   constexpr int DA = I8 ? (MT == 1 ? 6 : 4) : MT == 1 ? 4 : 3;   // (int8 stages have half the bytes)
@@ -641,8 +644,10 @@ static int pick(const FewRowsParams& p, hipStream_t s) {
   if constexpr (NORM) {
     if (nck > 33) return -1;
     if (MT == 1 && tiles <= 256 && nck <= 16) return launch<EPI, true, XI, 16, 1, I8, 8, 0, 2>(p, s);
-    if (MT == 2 && nck <= 16 && tiles <= 512) return launch<EPI, true, XI, 16, 1, I8, 8, 2, 2, false, true>(p, s);
-    if (MT == 2 && nck > 16 && tiles <= 2048) return launch<EPI, true, XI, 16, 1, I8, 11, 3, 3, false, true>(p, s);
+    if (MT == 2 && halved(nck, tiles)) {
+      if (nck <= 16) return launch<EPI, true, XI, 16, 1, I8, 8, 2, 2, false, true>(p, s);
+      return launch<EPI, true, XI, 16, 1, I8, 11, 3, 3, false, true>(p, s);
+    }
     if (nck <= 16) return launch<EPI, true, XI, 16, MT, I8, 8, 2, DA>(p, s);
     return launch<EPI, true, XI, 16, MT, I8, 11, 3, 3>(p, s);
   } else {
@@ -684,6 +689,8 @@ int64_t few_rows_workspace(int M, int N, int K, int* tickets) {
   *tickets = n ? ceil_div(N, 16) * (M <= 16 ? 1 : 2) : 0;
   return (int64_t)*tickets * n * 256;
 }
+
+bool few_rows_halved(int M, int N, int K) { return M > 16 && M <= FEW_MAX_ROWS && ceil_div(K, few::KC) <= 33 && few::halved(ceil_div(K, few::KC), ceil_div64(N, 16)); }
 
 int few_rows_launch(int epi, const FewRowsParams& p, hipStream_t s) {
   const int unit = p.wscale ? 16 : 8;   // elements of 16 bytes of weights

@@ -10,6 +10,7 @@ void register_gemm(pybind11::module& m);      // ../gemm.cpp
 void register_parallel(pybind11::module& m);  // bindings_parallel.cpp
 
 namespace nxd {
+int hyper_step_threads(int64_t, int, int64_t, int64_t);
 int hyper_step_launch(bool, float*, const void*, const int64_t*, int64_t, const void*, int64_t, const float*, const float*,
                       const float*, const float*, const float*, float, void*, int64_t, const int64_t*, bool, int64_t, int,
                       int, hipStream_t);
@@ -481,6 +482,7 @@ PYBIND11_MODULE(_hybrid, m) {
   register_gemm(m);
   register_parallel(m);
   namespace py = pybind11;
+  m.def("hyper_step_threads", &nxd::hyper_step_threads);   // of the one-pass kernel for R rows of W columns, strides ldy and ldh; 0: the loop
   m.def("hyper_step", &hyper_step, py::arg("x"), py::arg("embed") = py::none(), py::arg("ids") = py::none(),
         py::arg("y") = py::none(), py::arg("bias") = py::none(), py::arg("mix") = py::none(), py::arg("write") = py::none(),
         py::arg("read") = py::none(), py::arg("norm_w") = py::none(), py::arg("eps") = 0.0, py::arg("h") = py::none(),

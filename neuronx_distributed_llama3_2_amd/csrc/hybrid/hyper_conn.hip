@@ -234,14 +234,20 @@ __global__ void __launch_bounds__(256) softcap_kernel(float* x, int64_t n, float
     x[i] = cap * tanhf(x[i] / cap);
 }
 
+// Threads of the one-pass kernel for so many rows of W columns, 0: the loop
+static int row_threads(int64_t R, int W, int64_t ldy, int64_t ldh) {
+  if (W % 4 || ldy % 4 || ldh % 4 || R > FEW_ROWS || W > 4096) return 0;
+  return W <= 1024 ? 256 : W <= 2048 ? 512 : 1024;
+}
+
 template <typename T, int S>
 static int launch_hyper(const HyperParams& p, int64_t R, hipStream_t s) {
   const size_t lds = p.read ? (size_t)p.W * 4 : 0;
-  const bool fours = p.W % 4 == 0 && p.ldy % 4 == 0 && p.ldh % 4 == 0;
-  if (fours && R <= FEW_ROWS && p.W <= 4096) {
-    auto* f = p.W <= 1024 ? &hyper_row_kernel<T, S, 256> : p.W <= 2048 ? &hyper_row_kernel<T, S, 512> : &hyper_row_kernel<T, S, 1024>;
-    hipLaunchKernelGGL(f, dim3((unsigned)R), dim3(p.W <= 1024 ? 256 : p.W <= 2048 ? 512 : 1024), 0, s, p);
-  } else if (fours)
+  const int nt = row_threads(R, p.W, p.ldy, p.ldh);
+  if (nt) {
+    auto* f = nt == 256 ? &hyper_row_kernel<T, S, 256> : nt == 512 ? &hyper_row_kernel<T, S, 512> : &hyper_row_kernel<T, S, 1024>;
+    hipLaunchKernelGGL(f, dim3((unsigned)R), dim3(nt), 0, s, p);
+  } else if (p.W % 4 == 0 && p.ldy % 4 == 0 && p.ldh % 4 == 0)
     hipLaunchKernelGGL((hyper_step_kernel<T, S, 4>), dim3((unsigned)R), dim3(256), lds, s, p);
   else
     hipLaunchKernelGGL((hyper_step_kernel<T, S, 1>), dim3((unsigned)R), dim3(256), lds, s, p);
@@ -273,6 +279,8 @@ int hyper_step_launch(bool f32, float* x, const void* embed, const int64_t* ids,
   hybrid::HyperParams p{x, embed, ids, vocab, y, ldy, bias, mix, write, read, norm_w, eps, h, ldh, rows, store ? 1 : 0, W};
   return f32 ? hybrid::dispatch_hyper<float>(p, S, R, s) : hybrid::dispatch_hyper<uint16_t>(p, S, R, s);
 }
+
+int hyper_step_threads(int64_t R, int W, int64_t ldy, int64_t ldh) { return hybrid::row_threads(R, W, ldy, ldh); }
 
 int relu_squared_launch(bool f32, const void* x, void* y, int64_t n, hipStream_t s) {
   if (n == 0) return 0;
