@@ -623,6 +623,7 @@ static int most_splits(const Splits& sp) { return ceil_div(sp.room, std::min(sp.
 // Whether the last split merges: its trips to memory (8 splits at a time) come one after another, 0.7-1.2 us each, and a launch of
 // its own takes about 4 us.  In the launch / apart, us: 2 trips 8.5 / 10.0, 3 trips 7.8 / 9.0, 4 trips 9.9 / 11.4 and 12.2 / 13.3, 6 trips
 // 12.2 / 11.5, 8 trips 13.0 / 12.6 and 16.8 / 14.3, 12 trips 14.9 / 13.8, 64 trips (four tokens, 128 wide, 64 splits) 68 / 31.
+// The trips counted are those of 4 waves, which these were; workgroups of 8 waves make half as many (few splits: 1-2 of them).
 static bool merge_in_launch(int MD, const Splits& sp) { return ceil_div(MD, 64 * WAVES) * ceil_div(ceil_div(sp.room, sp.full), 8) <= 4; }
 
 // Split attention's partials -> merged attention row block (bf16-rounded, as the merge kernel's

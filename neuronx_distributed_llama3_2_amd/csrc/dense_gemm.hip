@@ -1,10 +1,10 @@
-// Dense bf16 GEMMs of the training hot path on gfx950 MFMA: one main loop, two operand layouts,
-// three epilogues.
+// Dense bf16 GEMMs on gfx950 MFMA: one main loop, two operand layouts, three epilogues.  Called by its name
+// (ext().dense_gemm) only: training's products go to the library, its weight gradients to the library or wgrad_gemm.hip.
 //
 //   NT  C[m, n] = sum_k A[m, k] B[n, k]    A [M][K], B [N][K]  (contraction contiguous in both):
-//       the forward y = x W^T and the input gradient dx = dy W (W's K-major copy);
+//       the shapes of the forward y = x W^T and the input gradient dx = dy W (W's K-major copy);
 //   TN  C[m, n] = sum_k A[k, m] B[k, n]    A [K][M], B [K][N]  (contraction along the ROWS), BF16 only: the
-//       weight gradient dW += dy^T x goes to wgrad_gemm.hip (8,192 tokens, 4096 x 4096: 240 us here, 211 there).
+//       weight gradient dW += dy^T x is handed on to wgrad_gemm.hip (8,192 tokens, 4096 x 4096: 240 us here, 211 there).
 //   Epilogues: BF16 store, F32_ACC (C fp32 += acc, one read-modify-write per element: exact and
 //   deterministic), F32_ATOMIC (split-K partial sums into C fp32 by no-return float atomics).
 //
@@ -12,7 +12,7 @@
 // backward matmuls (src/neuronx_distributed/parallel_layers/layers.py:322,348,391-409), which the
 // Neuron compiler lowers for its own matrix engine; here they are hand-scheduled for CDNA4.
 //
-// Structure (cdna_hip_programming.md §5, "The 256^2 8-phase template" and "Pipelining across barriers"):
+// Structure:
 //   * 256 x 256 output tile, 8 waves (512 threads), one workgroup per CU, reduction step BK = 64;
 //     wave (wr, wc) = (wid >> 2, wid & 3) owns rows {wr*64 + [0,64)} and {128 + wr*64 + [0,64)}
 //     and columns {wc*32 + [0,32)} and {128 + wc*32 + [0,32)}: four 64 x 32 quadrants, each
@@ -419,7 +419,7 @@ __global__ void __launch_bounds__(NT, 1) gemm_kernel(Params p) {
 // so a tile's DMA has four k-steps (~2,000 cycles) to land.  (The 16x16x32 form of this structure
 // made hipcc shuttle the 64 four-register accumulators between AGPRs and VGPRs every iteration.)
 // LDS images as above except the TN swizzle: 256-B rows with chunk c of row t at
-// c ^ (((t & 3) << 2) | ((t >> 2) & 3)) (cdna_hip_programming.md T10 (b)), under which the 32-lane
+// c ^ (((t & 3) << 2) | ((t >> 2) & 3)), under which the 32-lane
 // halves of the 32x32x16 transposed operand reads are conflict-free.
 constexpr int NT4 = 256;
 

@@ -1,6 +1,7 @@
 // The main loop of the 256 x 256-tile products (grouped_rowgemm.hip, wgrad_gemm.hip): C = A B over a reduction in steps of 64, bf16 operands, fp32 sums.
 //
-// What bounds it is power (2.1 GHz and less under matrix cores that are half busy) and what feeds them: LDS reads, and loads of a CU.
+// What bounds it is the clock that the numbers allow (8192 x 8192 x 8192: 1.99 GHz with random ones, 2.40 with zeros, counted as
+// GRBM_GUI_ACTIVE over the kernel's time) and what feeds the matrix cores: LDS reads, and loads of a CU.
 //   * 4 waves, one a SIMD, of 128 x 128 results each: 64 v_mfma_f32_16x16x32_bf16 for 16 fragments read from LDS, two thirds of what
 //     8 waves of 128 x 64 read -- those read 192 KB a step where LDS gives 128 bytes a clock, as long as the MFMAs take.  The
 //     256 sums of a lane are in AGPRs; the MFMAs are written in asm, because hipcc moves such sums between registers
@@ -9,8 +10,8 @@
 //     with the reads of the next half, four to a read; after the first half a barrier says that the step has been read and the
 //     next one is there, and the loads of the step after that go out between the MFMAs of the second half.
 //   * Loads go straight to LDS, 128 bytes of a row and more: whole lines (with 64 bytes of a row a CU gets 50 GB/s, with 128 it gets 90).
-//   8192 x 8192 x 8192 of random numbers 1.24 PFLOP/s, 8192 x 4096 x 28672 1.38 (of zeros 1.60, 1.53); the ping-pong of two wave groups
-//   that was here before 0.9.
+//   8192 x 8192 x 8192 of random numbers 1.35 PFLOP/s, 8192 x 28672 x 4096 1.40, 8192 x 4096 x 28672 1.41 (of zeros 1.64, 1.54, 1.52);
+//   the ping-pong of two wave groups that was here before 0.9.
 //
 // Images of a step in LDS, 16-byte chunks XORed so that 16 lanes of a read cover all banks once:
 //   ROW  the reduction is contiguous: [256 rows][64], 128-byte rows

@@ -32,7 +32,8 @@ def select_bucket(length: int, buckets: Sequence[int]) -> int:
 
 # Tokens of a padded batch from which on a length halfway between two buckets pays: below, the weights' bytes bound the prefill and a
 # quarter fewer tokens take little off (Llama-3.2-1B, 1 x 512 -> 1 x 384 tokens 2.22 -> 2.10 ms; 1 x 1,024 -> 768 3.12 -> 2.65, 3 x 1,024 -> 768
-# 6.31 -> 5.34, 1 x 2,048 -> 1,536 4.98 -> 4.09), while each length costs its graph's capture once (0.2 s).
+# 6.31 -> 5.34, 1 x 2,048 -> 1,536 4.98 -> 4.09), while each length costs its graph's capture once
+# (0.2 s, in the first request that needs it: no length is captured ahead).
 HALFWAY_TOKENS = 1024
 
 

@@ -1,6 +1,7 @@
-"""Hand-written dense GEMM (csrc/dense_gemm.hip) against fp32 torch: NT (forward / input gradient on
-the K-major weight copy) and TN (token-major weight gradient), bf16 / fp32-accumulate / split-K
-atomic epilogues, full and ragged tiles."""
+"""Hand-written dense GEMM (csrc/dense_gemm.hip) against fp32 torch: NT (the shapes of forward and input
+gradient on the K-major weight copy) with bf16 / fp32-accumulate epilogues, TN with bf16 output, full and
+ragged tiles; TN into fp32 (token-major weight gradient) is handed on to csrc/wgrad_gemm.hip, which these
+cases then run by dense_gemm's name and with its checks."""
 import pytest
 import torch
 
@@ -71,8 +72,8 @@ def test_dense_gemm_rejects_bad_shapes():
 
 def test_framework_wgrad_routes_skinny_shards_to_dense_tn():
     """ops.gemm.wgrad_accumulate_ sends the tensor-parallel shards and the TP=1 o_proj (no producer copy,
-    M N / (M + N) < 2200) to the hand-written TN kernel -- RMW epilogue when one K split fills the chip,
-    split-K atomics otherwise -- and keeps hipBLASLt for the wide TP=1 shapes; all accumulate like fp64."""
+    M N / (M + N) < 2200) to csrc/wgrad_gemm.hip -- one read-modify-write per element with one split of the
+    tokens, atomics otherwise -- and keeps hipBLASLt for the wide TP=1 shapes; all accumulate like fp64."""
     from neuronx_distributed_llama3_2_amd.ops import gemm as G
 
     torch.manual_seed(3)

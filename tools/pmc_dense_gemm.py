@@ -1,5 +1,5 @@
-"""PMC workload: the hand-written dense GEMM (csrc/dense_gemm.hip) and hipBLASLt on one shape, a few
-launches each (rocprofv3 --pmc passes aggregate per kernel name).
+"""PMC workload: the hand-written dense GEMM (csrc/dense_gemm.hip; --tn: the weight gradient, csrc/wgrad_gemm.hip)
+and hipBLASLt on one shape, a few launches each (rocprofv3 --pmc passes aggregate per kernel name).
 Usage: python tools/pmc_dense_gemm.py [T N K] [--tn]"""
 import os
 import sys
@@ -19,7 +19,7 @@ if "--tn" in sys.argv:
     dy = torch.randn(T, N, device="cuda").to(torch.bfloat16)
     mg = torch.zeros(N, K, device="cuda")
     for _ in range(5):
-        ext().dense_gemm(1, 1, dy, x, mg)
+        ext().wgrad_gemm(mg, dy, x, 0, True)
         G.ext().gemm(G.transpose(dy), G.transpose(x).t(), mg, None, 1.0, 1.0)
 else:
     for _ in range(5):
