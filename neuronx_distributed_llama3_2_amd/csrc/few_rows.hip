@@ -2,7 +2,7 @@
 // step, each one launch with the element-wise work around it (RMSNorm of the input, residual add, SwiGLU, rotary
 // positions and cache write, squared ReLU, capped fp32 logits).
 //
-// What bounds it is reading the weights once.  So weights go from memory straight to LDS (global_load_lds: no registers
+// What bounds it is reading the weights once.  So weights go from memory straight to LDS (no registers
 // held while they are on the way), 256 contiguous bytes (int8: 128) of a row at a time -- whole lines --, with several
 // stages of every wave under way; the row pieces are stored rotated (XOR of the piece's number with the row's), so that
 // the MFMA operands (16 rows x 16 bytes) are read back without bank conflicts.  A workgroup has tiles of R weight rows;
@@ -21,13 +21,29 @@ namespace few {
 
 constexpr int KC = 128;   // reduction elements of a stage
 
-__device__ __forceinline__ void dma16(const void* base, uint32_t at, uint32_t lds) {   // 64 lanes x 16 B: base + at -> LDS lds + 16 lane
-  uint32_t keep;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt\n\ts_mov_b32 m0, %0"
-               : "=&s"(keep)
-               : "v"(at), "s"(base), "s"(lds)
+// What a wave waits for.  Loads end in their order, so a wave that waits for its activations (in registers: the compiler places the wait) also waits for
+// every load before them, and for as many after them as the compiler does not know of or, across a branch, is not sure of.  So weights are loaded by a
+// builtin (as asm they were not counted: a streaming wave waited for all its stages whenever it came round to the first, 4096 x 4096 at 5 rows
+// 8.7 -> 7.8 us, 2048 x 8192 at 4 rows 8.8 -> 8.1), a buffer load (global_load_lds counts as an access to both memories, after which the compiler
+// waits for everything), in straight lines of whole rounds; and since the compiler lets an access to LDS that it sees wait for all such
+// loads, the accesses of waves that stream weights are asm.
+__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t base, uint32_t at, uint32_t lds) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(base, (__attribute__((address_space(3))) void*)(uintptr_t)lds, 16, (int)at, 0, 0, 2 /* nt */);
+}
+__device__ __forceinline__ void lds_read(u32x4_t (&v)[4], const uint32_t (&at)[4]) {
+  asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\tds_read_b128 %2, %6\n\tds_read_b128 %3, %7\n\ts_waitcnt lgkmcnt(0)"
+               : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3])
+               : "v"(at[0]), "v"(at[1]), "v"(at[2]), "v"(at[3])
                : "memory");
 }
+__device__ __forceinline__ void lds_read(u32x4_t (&v)[2], const uint32_t (&at)[2]) {
+  asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %3\n\ts_waitcnt lgkmcnt(0)" : "=&v"(v[0]), "=&v"(v[1]) : "v"(at[0]), "v"(at[1]) : "memory");
+}
+__device__ __forceinline__ void lds_write(uint32_t at, const f32x4_t& v) { asm volatile("ds_write_b128 %0, %1" ::"v"(at), "v"(v) : "memory"); }
+// (the result of a matrix product: asm has to wait for it by itself, 11 cycles for 8 passes)
+__device__ __forceinline__ void lds_write_sum(uint32_t at, const f32x4_t& v) { asm volatile("s_nop 15\n\tds_write_b128 %0, %1" ::"v"(at), "v"(v) : "memory"); }
+__device__ __forceinline__ void lds_write(uint32_t at, float v) { asm volatile("ds_write_b32 %0, %1" ::"v"(at), "v"(v) : "memory"); }
+__device__ __forceinline__ uint32_t lds_at(const void* p) { return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)p; }
 
 // int8 x 8 -> bf16 x 8 (exact)
 __device__ __forceinline__ u32x4_t widen8(uint32_t lo, uint32_t hi) {
@@ -58,12 +74,14 @@ __device__ __forceinline__ int row_of(const FewRowsParams& p, int tile, int r) {
 // all tiles (0: any number, activations streamed beside the weights)
 template <int R, int MT, bool I8, int NW, int CW, int D>
 struct Shape {
+  static constexpr int GC = CW > 0 ? CW : 2;             // chunks of a wave with a norm
   static constexpr int ROWB = I8 ? KC : 2 * KC;          // bytes of a row in a stage
   static constexpr int STAGE = R * ROWB;                 // bytes of a stage of a wave
   static constexpr int DMAS = STAGE / 1024;              // loads of a stage
   static constexpr int RING = NW * D * STAGE;
   static constexpr int PART = NW * MT * 64 * 16;         // the waves' sums of a tile
   static constexpr int SQ = NW * MT * 16 * 4;            // the waves' sums of squares
+  static constexpr int G = CW > 0 ? 0 : NW * GC * 256;   // the waves' parts of the norm's weight (CW > 0: in their parts of PART, where they wait for no more than one tile)
   static constexpr int FW = NW + MT > 12 ? 1 : MT;       // waves that finish tiles (12 waves leave each 168 registers)
 };
 
@@ -254,7 +272,7 @@ struct Finish {
 };
 
 template <int EPI, bool NORM, bool XI, int R, int MT, bool I8, int NW, int CW, int D, bool SPLIT, bool HALF>
-__global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) kernel(FewRowsParams p, int tiles) {
+__global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) kernel(FewRowsParams p, int tiles, int per) {
   using S = Shape<R, MT, I8, NW, CW, D>;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   f32x4_t* part = reinterpret_cast<f32x4_t*>(smem + S::RING);       // [NW][MT][64]
@@ -263,12 +281,10 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
   const int c = lane & 15, q = lane >> 4, m0 = SPLIT ? 0 : blockIdx.y * (HALF ? p.half : 16 * MT);   // its first row
   if constexpr (HALF) p.M = min(p.M, m0 + p.half);
   static_assert(!SPLIT || (CW > 0 && !NORM), "split reductions hold their activations and need no norm");
-  const int step = SPLIT ? gridDim.x / p.splits : gridDim.x, tile0 = SPLIT ? blockIdx.x / p.splits : blockIdx.x;
-
-  // NORM: the weight of the norm waits in `part` for the activations to come
-  uint16_t* gs = reinterpret_cast<uint16_t*>(part);
-  constexpr bool GS = NORM && CW > 0;
-  static_assert(!GS || NW * CW * KC * 2 <= S::PART, "the norm's weight in LDS");
+  // its tiles: per of them next to each other, or (1) one of each round
+  const int group = SPLIT ? blockIdx.x / p.splits : blockIdx.x, tile0 = group * per;
+  const int step = per > 1 ? 1 : SPLIT ? gridDim.x / p.splits : gridDim.x;
+  if (per > 1) tiles = min(tiles, tile0 + per);
 
   // SPLIT: all waves of a workgroup share the tiles of which its part was the last to come
   auto finish_last = [&]() {
@@ -291,11 +307,6 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
 
   // Twice a tile all waves meet: when `part` is free, and when it is full
   if (w >= NW) {
-    if (GS) {
-      for (int k = (tid - NW * 64) * 8; k < p.K; k += S::FW * 512)
-        *reinterpret_cast<u32x4_t*>(gs + k) = *reinterpret_cast<const u32x4_t*>(p.norm_w + k);
-      meet();
-    }
     constexpr int T = MT / S::FW;
     Finish<EPI, NORM, R, I8> f0(p, lane, m0 + 16 * (w - NW) * T);
     Finish<EPI, NORM, R, I8> f1(p, lane, m0 + 16 * ((w - NW) * T + T - 1));
@@ -354,7 +365,7 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
   }
   const int wc = c0 + w, cw = (c1 - wc + NW - 1) / NW;   // of this wave: wc, wc + NW, ...
   char* ring = smem + w * D * S::STAGE;
-  const uint32_t ring_at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)ring;
+  const uint32_t ring_at = lds_at(ring);
 
   // ---- this lane's input rows (rows past M repeat the last one: their sums are not stored)
   uint32_t xrow[MT];   // (element offsets: the rows lie within 4 GB)
@@ -368,10 +379,6 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
     for (int t = 0; t < MT; ++t)   // (both halves of a line one after the other)
 #pragma unroll
       for (int f = 0; f < 4; ++f) xv[t][f] = *reinterpret_cast<const u32x4_t*>(p.x + (xrow[t] + (uint32_t)min(chunk * KC + kof(f), p.K - 8)));
-  };
-  auto load_g = [&](u32x4_t (&g)[4], int chunk) {
-#pragma unroll
-    for (int f = 0; f < 4; ++f) g[f] = *reinterpret_cast<const u32x4_t*>(p.norm_w + min(chunk * KC + kof(f), p.K - 8));
   };
   float ss[MT];
 #pragma unroll
@@ -404,6 +411,7 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
   };
 
   // ---- weights: the next stage to issue
+  const __amdgpu_buffer_rsrc_t wbase = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.w), 0, -1, 0x00020000);   // (4 GB)
   uint32_t wrow[S::DMAS];   // (byte offsets: the weights take less than 4 GB)
   int it = tile0, ic = 0, is = 0, ahead = 0;   // its tile, chunk and place in the ring; stages under way
   // Every workgroup begins elsewhere in the reduction: rows lie a power of two apart, and the same piece of all of
@@ -414,13 +422,13 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
     const int j = i + rot;
     return j < cw ? j : j - cw;
   };
-  auto issue = [&]() {
-    if (it >= tiles || cw <= 0) return;
+  auto start = [&]() {
+    asm volatile("" ::: "memory");   // (in this order: waits count what came later)
     if (ic == 0) {
 #pragma unroll
       for (int j = 0; j < S::DMAS; ++j) {
         const int r = I8 ? 8 * j + (lane >> 3) : 4 * j + (lane >> 4);
-        wrow[j] = (uint32_t)row_of<EPI, R>(p, it, r) * (uint32_t)p.ldw * (I8 ? 1 : 2);
+        wrow[j] = (uint32_t)row_of<EPI, R>(p, min(it, tiles - 1), r) * (uint32_t)p.ldw * (I8 ? 1 : 2);
       }
     }
     const int chunk = wc + order(ic) * NW;
@@ -435,22 +443,30 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
         seg = (lane & 15) ^ (r & 15);
       }
       const uint32_t at = min(chunk * S::ROWB + 16 * seg, p.K * (I8 ? 1 : 2) - 16);
-      dma16(p.w, wrow[j] + at, __builtin_amdgcn_readfirstlane(ring_at + is * S::STAGE + j * 1024));
+      dma16(wbase, wrow[j] + at, __builtin_amdgcn_readfirstlane(ring_at + is * S::STAGE + j * 1024));
     }
+    asm volatile("" ::: "memory");
     ++ahead;
     if (++ic == cw) ic = 0, it += step;
     if (++is == D) is = 0;
   };
+  auto issue = [&]() {
+    if (it < tiles && cw > 0) start();
+  };
 
   f32x4_t acc[MT];
   int cs = 0;   // place in the ring of the stage to use
-  auto take = [&](u32x4_t (&wf)[I8 ? 2 : 4]) {   // its pieces, as this lane's operands
-    const char* st = ring + cs * S::STAGE;
-    const int r = c & (R - 1);
+  uint32_t wat[I8 ? 2 : 4];   // its pieces, as this lane's operands, in the first place
 #pragma unroll
-    for (int s = 0; s < (I8 ? 2 : 4); ++s)
-      wf[s] = *reinterpret_cast<const u32x4_t*>(st + r * S::ROWB + (((4 * s + q) ^ (I8 ? (r >> 1) & 7 : r & 15)) << 4));
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (the place may be filled again)
+  for (int i = 0; i < (I8 ? 2 : 4); ++i) {
+    const int r = c & (R - 1);
+    wat[i] = ring_at + r * S::ROWB + (((4 * i + q) ^ (I8 ? (r >> 1) & 7 : r & 15)) << 4);
+  }
+  auto take = [&](u32x4_t (&wf)[I8 ? 2 : 4]) {   // (the place may be filled again)
+    uint32_t at[I8 ? 2 : 4];
+#pragma unroll
+    for (int i = 0; i < (I8 ? 2 : 4); ++i) at[i] = wat[i] + cs * S::STAGE;
+    lds_read(wf, at);
     --ahead;
     if (++cs == D) cs = 0;
   };
@@ -469,6 +485,25 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
 #pragma unroll
     for (int t = 0; t < MT; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   };
+  // NORM: the weight of this wave's chunks, 16 lanes a chunk, turned into operands through LDS of its own
+  const uint32_t gs = CW > 0 ? lds_at(part + w * MT * 64) : lds_at(smem + S::RING + S::PART + S::SQ) + w * S::GC * 256;
+  auto load_g = [&]() {
+    u32x4_t v = {0u, 0u, 0u, 0u};
+    if constexpr (NORM) v = *reinterpret_cast<const u32x4_t*>(p.norm_w + min((wc + min(q, S::GC - 1) * NW) * KC + 8 * c, p.K - 8));
+    return v;
+  };
+  auto keep_g = [&](const u32x4_t& v) {
+    static_assert(S::GC <= 4 && (CW == 0 || CW * 256 <= MT * 1024), "16 lanes a chunk");
+    if (NORM && q < S::GC) lds_write(gs + 16 * lane, __builtin_bit_cast(f32x4_t, v));
+  };
+  auto read_g = [&](u32x4_t (&g)[4], int i) {   // of the wave's i-th chunk
+    if constexpr (NORM) {
+      uint32_t at[4];
+#pragma unroll
+      for (int f = 0; f < 4; ++f) at[f] = gs + i * 256 + 2 * kof(f);
+      lds_read(g, at);
+    }
+  };
   auto squares = [&]() {
     if (!NORM) return;
 #pragma unroll
@@ -476,30 +511,30 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
       float v = ss[t];
       v += __shfl_xor(v, 16, 64);
       v += __shfl_xor(v, 32, 64);
-      if (q == 0) sq[w * 16 * MT + 16 * t + c] = v;
+      if (q == 0) lds_write(lds_at(sq + w * 16 * MT + 16 * t + c), v);
     }
   };
   auto publish = [&]() {
     meet();
 #pragma unroll
-    for (int t = 0; t < MT; ++t) part[(w * MT + t) * 64 + lane] = acc[t];
+    for (int t = 0; t < MT; ++t) lds_write_sum(lds_at(part + (w * MT + t) * 64 + lane), acc[t]);
     meet();
   };
 
   if constexpr (CW > 0) {
     u32x4_t x[CW][MT][4];
+    const u32x4_t gl = load_g();
 #pragma unroll
     for (int i = 0; i < CW; ++i) load_x(x[i], min(wc + i * NW, nck - 1));   // (chunks past the last one are not used)
+    // the first D stages, without a branch (past the last one: a piece that is there, not used), or the compiler would wait for them with
+    // the activations
 #pragma unroll
-    for (int i = 0; i < D; ++i) issue();
-    if (GS) meet();
+    for (int i = 0; i < D; ++i) start();
+    keep_g(gl);
 #pragma unroll
     for (int i = 0; i < CW; ++i) {
       u32x4_t g[4];
-      if (GS) {
-#pragma unroll
-        for (int f = 0; f < 4; ++f) g[f] = *reinterpret_cast<const u32x4_t*>(gs + min((wc + i * NW) * KC + kof(f), p.K - 8));
-      }
+      read_g(g, i);
       ready_x(x[i], g, wc + i * NW, i < cw);
     }
     squares();
@@ -516,19 +551,50 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
       }
       publish();
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (pieces that are not used)
     if constexpr (SPLIT) finish_last();
   } else {
-    constexpr int XL = 4 * MT + (NORM ? 4 : 0);   // loads of a stage beside the weights'
-    u32x4_t x[D][MT][4], g[NORM ? D : 1][4];
-    auto fetch = [&](u32x4_t (&xv)[MT][4], u32x4_t (&gv)[4]) {
-      if (it < tiles && cw > 0) {
-        load_x(xv, wc + order(ic) * NW);
-        if (NORM) load_g(gv, wc + order(ic) * NW);
-      }
+    constexpr int XL = 4 * MT;   // loads of a stage beside the weights'
+    u32x4_t x[D][MT][4], g[4];
+    const u32x4_t gl = load_g();
+    auto fetch = [&](u32x4_t (&xv)[MT][4]) {
+      if (it < tiles && cw > 0) load_x(xv, wc + order(ic) * NW);
       issue();
     };
+    if (tile0 + step >= tiles && cw > 0 && cw % D == 0) {   // one tile: no branch between the loads, so that the compiler knows what is under way
+      clear();
+      auto get = [&](int u) {
+        load_x(x[u], wc + order(ic) * NW);
+        start();
+      };
+      auto use = [&](int u, int i, int later) {   // the stage of chunk i, `later` ones are under way
+        u32x4_t wf[I8 ? 2 : 4];
+        wait_stages<XL + S::DMAS, D>(later);
+        take(wf);
+        read_g(g, order(i));
+        ready_x(x[u], g, wc + order(i) * NW, true);
+        multiply(wf, x[u]);
+      };
 #pragma unroll
-    for (int i = 0; i < D; ++i) fetch(x[i], g[NORM ? i : 0]);
+      for (int u = 0; u < D; ++u) get(u);
+      keep_g(gl);
+      int i = 0;
+      for (; i + D < cw; i += D) {
+#pragma unroll
+        for (int u = 0; u < D; ++u) {
+          use(u, i + u, D - 1);
+          get(u);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < D; ++u) use(u, i + u, D - 1 - u);
+      squares();
+      publish();
+      return;
+    }
+#pragma unroll
+    for (int i = 0; i < D; ++i) fetch(x[i]);
+    keep_g(gl);
     int tile = tile0, i = 0;
     bool first = true;
     clear();
@@ -541,9 +607,10 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
         u32x4_t wf[I8 ? 2 : 4];
         wait_stages<XL, D>(ahead - 1);   // (of XL + DMAS loads a stage: the stage has come, and the next one's x nearly)
         take(wf);
-        ready_x(x[u], g[NORM ? u : 0], wc + order(i) * NW, first);
+        read_g(g, order(i));
+        ready_x(x[u], g, wc + order(i) * NW, first);
         multiply(wf, x[u]);
-        fetch(x[u], g[NORM ? u : 0]);
+        fetch(x[u]);
         if (++i == cw) {
           if (first) squares();
           first = false;
@@ -569,8 +636,8 @@ template <int EPI, bool NORM, bool XI, int R, int MT, bool I8, int NW, int CW, i
 static int launch(FewRowsParams p, hipStream_t s, int splits = 1) {
   using S = Shape<R, MT, I8, NW, CW, D>;
   const int nck = ceil_div(p.K, KC);
-  if (CW > 0 && ceil_div(nck, splits) > NW * CW) return -2;
-  constexpr size_t lds = S::RING + S::PART + S::SQ;
+  if ((CW > 0 || NORM) && ceil_div(nck, splits) > NW * S::GC) return -2;
+  constexpr size_t lds = S::RING + S::PART + S::SQ + (NORM ? S::G : 0);
   static_assert(lds <= 160 * 1024, "LDS of a workgroup");
   const int64_t tiles = tiles_of<EPI, R>(p);
   auto* f = &kernel<EPI, NORM, XI, R, MT, I8, NW, CW, D, SPLIT, HALF>;
@@ -592,11 +659,19 @@ static int launch(FewRowsParams p, hipStream_t s, int splits = 1) {
   if (SPLIT && rounds > 64) return -2;   // (a lane for every tile's ticket)
   p.splits = splits;
   if (HALF) p.half = (p.M + 1) / 2;
-  hipLaunchKernelGGL(f, dim3((unsigned)(groups * splits), (unsigned)(SPLIT ? 1 : HALF ? 2 : ceil_div(p.M, 16 * MT))), dim3((NW + S::FW) * 64), lds, s, p, (int)tiles);
+  // Tiles next to each other (a workgroup reads one stretch of the weights, and a line of the output is written on one XCD), but not where the rows
+  // of a tile lie in two or three places, unless there are many tiles, nor parts of rows.  One of each round / next to each other, us: 16 rows,
+  // 16384 x 2048 13.6 / 12.3, 32000 x 2048 23.5 / 22.1, 128256 x 2048 88.9 / 85.9, 128256 x 4096 167 / 159 (28 rows 26.3 / 23.3 for 32000 x 2048); SwiGLU 8192 x 2048
+  // 13.3 / 13.5, 8192 x 4096 25.1 / 26.2, 14336 x 4096 40.4 / 39.3, 28 rows 29.1 / 27.0 and 47.7 / 45.9; rotary 6144 x 4096 13.3 / 13.9; in parts
+  // 8192 x 8192 29.6 / 33.3, 4096 x 14336 24.3 / 25.3
+  const int next = SPLIT || EPI == FEW_ROPE_KV || (EPI == FEW_GLU && rounds < 7) ? 1 : (int)rounds;
+  hipLaunchKernelGGL(f, dim3((unsigned)(groups * splits), (unsigned)(SPLIT ? 1 : HALF ? 2 : ceil_div(p.M, 16 * MT))), dim3((NW + S::FW) * 64), lds, s, p, (int)tiles, next);
   return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
-// Which geometry (times in us at 4 / 16 / 32 rows, bf16, weights from memory):
+// Which geometry (times in us at 4 / 16 / 32 rows, bf16, weights from memory; the choices were measured before the waits at the top of this file, what they
+// take now: 16384 x 2048 with norm and SwiGLU 12.7 / 13.3 / 15.3, 128256 x 2048 79.5 / 85.9 / 91.7, 3072 x 2048 rotary 6.0 / 6.7 / 7.7, 28672 x 4096 at 5 /
+// 13 / 28 rows 37.5 / 38.4 / 43.3, 2048 x 8192 8.1 / 10.8 / 12.2, 4096 x 4096 at 5 / 13 / 28 7.8 / 8.5 / 11.4):
 //   K <= 2048: activations stay in 8 waves' registers and a workgroup goes over the tiles of 16 rows: 16384 x 2048 with
 //     norm and SwiGLU 14.1 / 15.0 / 16.9 (activations streamed 15.8 / 19.0 / 71; int8 11.6 / 12.4 / 14.8),
 //     128256 x 2048 86 / 92 / 98 (int8 46 / 50 / 54).
@@ -663,6 +738,7 @@ static int pick(const FewRowsParams& p, hipStream_t s) {
       if (n) return launch<EPI, false, false, 16, MT, I8, 8, 1, 2 * X, true>(p, s, n);
     }
     if (tiles > 128) return launch<EPI, false, false, 16, MT, I8, 8, 0, D>(p, s);
+    if (nck <= 16) return MT == 2 ? launch<EPI, false, false, 16, 1, I8, 8, 0, 2>(p, s) : launch<EPI, false, false, 8, 1, I8, 8, 0, 2>(p, s);
     if (MT == 2) return launch<EPI, false, false, 16, 1, I8, 8, 0, 4>(p, s);
     return launch<EPI, false, false, 8, 1, I8, 8, 0, 4>(p, s);
   }
