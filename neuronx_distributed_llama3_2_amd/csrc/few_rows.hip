@@ -15,6 +15,7 @@
 #include "few_rows.h"
 
 #include <atomic>
+#include <type_traits>
 
 namespace nxd {
 namespace few {
@@ -29,6 +30,13 @@ constexpr int KC = 128;   // reduction elements of a stage
 // loads, the accesses of waves that stream weights are asm.
 __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t base, uint32_t at, uint32_t lds) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(base, (__attribute__((address_space(3))) void*)(uintptr_t)lds, 16, (int)at, 0, 0, 2 /* nt */);
+}
+__device__ __forceinline__ void dma16_uncounted(const void* base, uint32_t at, uint32_t lds) {
+  uint32_t keep;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep)
+               : "v"(at), "s"(base), "s"(lds)
+               : "memory");
 }
 __device__ __forceinline__ void lds_read(u32x4_t (&v)[4], const uint32_t (&at)[4]) {
   asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\tds_read_b128 %2, %6\n\tds_read_b128 %3, %7\n\ts_waitcnt lgkmcnt(0)"
@@ -411,7 +419,6 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
   };
 
   // ---- weights: the next stage to issue
-  const __amdgpu_buffer_rsrc_t wbase = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.w), 0, -1, 0x00020000);   // (4 GB)
   uint32_t wrow[S::DMAS];   // (byte offsets: the weights take less than 4 GB)
   int it = tile0, ic = 0, is = 0, ahead = 0;   // its tile, chunk and place in the ring; stages under way
   // Every workgroup begins elsewhere in the reduction: rows lie a power of two apart, and the same piece of all of
@@ -422,7 +429,7 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
     const int j = i + rot;
     return j < cw ? j : j - cw;
   };
-  auto start = [&]() {
+  auto start = [&](auto counted) {
     asm volatile("" ::: "memory");   // (in this order: waits count what came later)
     if (ic == 0) {
 #pragma unroll
@@ -432,6 +439,8 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
       }
     }
     const int chunk = wc + order(ic) * NW;
+    // (past the last stage; a part may have one only, and a range of nothing is not read: 1024 x 8192 at 16 rows 9.3 -> 8.9 us)
+    const __amdgpu_buffer_rsrc_t wbase = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.w), 0, SPLIT && it >= tiles ? 0 : -1, 0x00020000);
 #pragma unroll
     for (int j = 0; j < S::DMAS; ++j) {
       int seg;   // the piece of the row that goes to this lane's place
@@ -443,15 +452,17 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
         seg = (lane & 15) ^ (r & 15);
       }
       const uint32_t at = min(chunk * S::ROWB + 16 * seg, p.K * (I8 ? 1 : 2) - 16);
-      dma16(wbase, wrow[j] + at, __builtin_amdgcn_readfirstlane(ring_at + is * S::STAGE + j * 1024));
+      const uint32_t to = __builtin_amdgcn_readfirstlane(ring_at + is * S::STAGE + j * 1024);
+      if constexpr (counted.value) dma16(wbase, wrow[j] + at, to);
+      else dma16_uncounted(p.w, wrow[j] + at, to);
     }
     asm volatile("" ::: "memory");
     ++ahead;
     if (++ic == cw) ic = 0, it += step;
     if (++is == D) is = 0;
   };
-  auto issue = [&]() {
-    if (it < tiles && cw > 0) start();
+  auto issue = [&](auto counted) {
+    if (it < tiles && cw > 0) start(counted);
   };
 
   f32x4_t acc[MT];
@@ -467,6 +478,13 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
 #pragma unroll
     for (int i = 0; i < (I8 ? 2 : 4); ++i) at[i] = wat[i] + cs * S::STAGE;
     lds_read(wf, at);
+    --ahead;
+    if (++cs == D) cs = 0;
+  };
+  auto look = [&](u32x4_t (&wf)[I8 ? 2 : 4]) {   // the same, of loads that are not counted
+#pragma unroll
+    for (int i = 0; i < (I8 ? 2 : 4); ++i) wf[i] = *reinterpret_cast<const u32x4_t*>(ring + (wat[i] - ring_at) + cs * S::STAGE);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     --ahead;
     if (++cs == D) cs = 0;
   };
@@ -529,7 +547,7 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
     // the first D stages, without a branch (past the last one: a piece that is there, not used), or the compiler would wait for them with
     // the activations
 #pragma unroll
-    for (int i = 0; i < D; ++i) start();
+    for (int i = 0; i < D; ++i) start(std::true_type{});
     keep_g(gl);
 #pragma unroll
     for (int i = 0; i < CW; ++i) {
@@ -546,7 +564,7 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
         u32x4_t wf[I8 ? 2 : 4];
         wait_stages<S::DMAS, D>(ahead - 1);
         take(wf);
-        issue();
+        issue(std::true_type{});
         multiply(wf, x[i]);
       }
       publish();
@@ -559,13 +577,13 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
     const u32x4_t gl = load_g();
     auto fetch = [&](u32x4_t (&xv)[MT][4]) {
       if (it < tiles && cw > 0) load_x(xv, wc + order(ic) * NW);
-      issue();
+      issue(std::false_type{});
     };
     if (tile0 + step >= tiles && cw > 0 && cw % D == 0) {   // one tile: no branch between the loads, so that the compiler knows what is under way
       clear();
       auto get = [&](int u) {
         load_x(x[u], wc + order(ic) * NW);
-        start();
+        start(std::true_type{});
       };
       auto use = [&](int u, int i, int later) {   // the stage of chunk i, `later` ones are under way
         u32x4_t wf[I8 ? 2 : 4];
@@ -606,7 +624,7 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
         if (tile >= tiles) break;
         u32x4_t wf[I8 ? 2 : 4];
         wait_stages<XL, D>(ahead - 1);   // (of XL + DMAS loads a stage: the stage has come, and the next one's x nearly)
-        take(wf);
+        look(wf);
         read_g(g, order(i));
         ready_x(x[u], g, wc + order(i) * NW, first);
         multiply(wf, x[u]);
@@ -662,9 +680,9 @@ static int launch(FewRowsParams p, hipStream_t s, int splits = 1) {
   // Tiles next to each other (a workgroup reads one stretch of the weights, and a line of the output is written on one XCD), but not where the rows
   // of a tile lie in two or three places, unless there are many tiles, nor parts of rows.  One of each round / next to each other, us: 16 rows,
   // 16384 x 2048 13.6 / 12.3, 32000 x 2048 23.5 / 22.1, 128256 x 2048 88.9 / 85.9, 128256 x 4096 167 / 159 (28 rows 26.3 / 23.3 for 32000 x 2048); SwiGLU 8192 x 2048
-  // 13.3 / 13.5, 8192 x 4096 25.1 / 26.2, 14336 x 4096 40.4 / 39.3, 28 rows 29.1 / 27.0 and 47.7 / 45.9; rotary 6144 x 4096 13.3 / 13.9; in parts
-  // 8192 x 8192 29.6 / 33.3, 4096 x 14336 24.3 / 25.3
-  const int next = SPLIT || EPI == FEW_ROPE_KV || (EPI == FEW_GLU && rounds < 7) ? 1 : (int)rounds;
+  // 13.3 / 13.5, 8192 x 4096 25.1 / 26.2, 14336 x 4096 40.4 / 39.3, 28 rows 29.1 / 27.0 and 47.7 / 45.9; rotary 6144 x 4096 13.3 / 13.9; streamed 8192 x 8192
+  // 26.7 / 30.5; in parts 8192 x 8192 29.6 / 33.3, 4096 x 14336 24.3 / 25.3, but 2048 x 12288 (long parts, four rounds) 14.1 / 13.8, 28 rows 15.7 / 15.1
+  const int next = (SPLIT && (CW < 2 || rounds > 4)) || CW == 0 || EPI == FEW_ROPE_KV || (EPI == FEW_GLU && rounds < 7) ? 1 : (int)rounds;
   hipLaunchKernelGGL(f, dim3((unsigned)(groups * splits), (unsigned)(SPLIT ? 1 : HALF ? 2 : ceil_div(p.M, 16 * MT))), dim3((NW + S::FW) * 64), lds, s, p, (int)tiles, next);
   return hipGetLastError() == hipSuccess ? 0 : 1;
 }
@@ -698,12 +716,16 @@ static int launch(FewRowsParams p, hipStream_t s, int splits = 1) {
 //     2048 at 17 / 32 rows 5.8 / 7.1 -> 5.9 / 6.1 (int8 6.9 -> 5.3 at 32); with more tiles two would share a CU and its loads
 //     (4096 x 4096 at 32 13.2 -> 18.7).
 //     The parts' sums meet in memory; the last to come adds them up, its waves sharing its tiles (by one wave: 2.5 us more).
+//     Streamed loads are waited for best where a wave has whole rounds of stages: two stages where it has two chunks (2048 x 2048 at 4 rows 4.3 ->
+//     4.2 us, int8 4.25 -> 4.0), 7 or 11 waves where 8 leave a rest (4096 x 14336 at 4 / 9 rows 22.6 / 23.5 -> 21.4 / 22.3, 2048 x 5632 7.0 / 7.8 -> 6.6 /
+//     7.5; 9 waves for 5120 x 13824 no better).  So fewer rows than before are worth splitting for: unsplit / in parts 2048 x 8192 at 14 / 16
+//     rows 10.5 / 11.1 and 11.1 / 11.0, 2048 x 5632 at 12 / 16 8.0 / 9.7 and 8.9 / 10.0, 1024 x 8192 at 11 / 12 9.2 and 9.4 / 8.7.
 constexpr int kLongPart = 72;   // chunks of the reduction from which parts are long
 
 static int parts(int M, int N, int K) {   // of the reduction; 0: not split
   const int nck = ceil_div(K, KC), tiles = ceil_div(N, 16), per = nck > kLongPart ? 14 : 8;
   if (nck <= 33 || M > FEW_MAX_ROWS) return 0;
-  if (tiles <= 128 ? M < (nck > kLongPart ? 9 : 12) : M <= 16 && (M < 12 || nck <= 96)) return 0;
+  if (tiles <= 128 ? M < (nck > kLongPart ? 9 : tiles <= 64 || nck > 64 ? 12 : nck <= 44 ? 17 : 15) : M <= 16 && (M < 12 || nck <= 96)) return 0;
   const int n = ceil_div(nck, per);
   return n > 32 || ceil_div(tiles, 256 / n) > 64 ? 0 : n;   // (a lane for every tile's ticket)
 }
@@ -737,8 +759,13 @@ static int pick(const FewRowsParams& p, hipStream_t s) {
       if (n && nck > kLongPart) return launch<EPI, false, false, 16, MT, I8, 7, 2, 4 * X, true>(p, s, n);
       if (n) return launch<EPI, false, false, 16, MT, I8, 8, 1, 2 * X, true>(p, s, n);
     }
+    // (as many waves as give each whole rounds of stages)
+    if (MT == 1 && nck > 33 && nck % 32) {
+      if (nck % 28 == 0) return tiles > 128 ? launch<EPI, false, false, 16, 1, I8, 7, 0, 4>(p, s) : launch<EPI, false, false, 8, 1, I8, 7, 0, 4>(p, s);
+      if (nck % 44 == 0) return tiles > 128 ? launch<EPI, false, false, 16, 1, I8, 11, 0, 3>(p, s) : launch<EPI, false, false, 8, 1, I8, 11, 0, 4>(p, s);
+    }
     if (tiles > 128) return launch<EPI, false, false, 16, MT, I8, 8, 0, D>(p, s);
-    if (nck <= 16) return MT == 2 ? launch<EPI, false, false, 16, 1, I8, 8, 0, 2>(p, s) : launch<EPI, false, false, 8, 1, I8, 8, 0, 2>(p, s);
+    if (nck > 8 && nck <= 16) return MT == 2 ? launch<EPI, false, false, 16, 1, I8, 8, 0, 2>(p, s) : launch<EPI, false, false, 8, 1, I8, 8, 0, 2>(p, s);
     if (MT == 2) return launch<EPI, false, false, 16, 1, I8, 8, 0, 4>(p, s);
     return launch<EPI, false, false, 8, 1, I8, 8, 0, 4>(p, s);
   }

@@ -51,10 +51,10 @@ def test_rounds_of_tiles(M, N, K, int8):
     _run(M, N, K, 0, True, int8)
 
 
-# one tile a workgroup, activations streamed: chunks a wave 1, 2, both, 3 and 4, 4, 5, 8, 8 and 9
+# one tile a workgroup, activations streamed: chunks a wave 1, 2, both, 3 and 4, 4, 5, 8, 8 and 9; 44 and 56 chunks: 11 and 7 waves
 @pytest.mark.parametrize("int8", [False, True])
-@pytest.mark.parametrize("K", [1024, 2048, 1664, 3200, 4096, 5120, 8192, 8448])
-@pytest.mark.parametrize("M,N", [(3, 2048), (8, 40), (4, 4096), (20, 1000), (18, 3072)])
+@pytest.mark.parametrize("K", [1024, 2048, 1664, 3200, 4096, 5120, 8192, 8448, 5632, 7168])
+@pytest.mark.parametrize("M,N", [(3, 2048), (8, 40), (4, 4096), (20, 1000), (18, 3072), (5, 8192)])
 def test_single_tiles(M, N, K, int8):
     _run(M, N, K, 0, False, int8)
     if K <= 2048:
