@@ -6,12 +6,15 @@
 //     8 waves of 128 x 64 read -- those read 192 KB a step where LDS gives 128 bytes a clock, as long as the MFMAs take.  The
 //     256 sums of a lane are in AGPRs; the MFMAs are written in asm, because hipcc moves such sums between registers
 //     (216 moves and 124 waits a step of 128 MFMAs: 0.22 PFLOP/s).
-//   * A step's operands are 64 KB of LDS, two steps are there.  The MFMAs of one half of a step (32 of the reduction) are interleaved
-//     with the reads of the next half, four to a read; after the first half a barrier says that the step has been read and the
-//     next one is there, and the loads of the step after that go out between the MFMAs of the second half.
+//   * A step's operands are 64 KB of LDS.  Three steps of A are there and two of B (160 KB): the MFMAs of one half of a step (32 of the reduction) are
+//     interleaved with the reads of the next half, four to a read; in the first half the loads of A go out, two steps ahead; after it a barrier
+//     says that the step has been read and the next one is there, and B's loads go out with the first MFMAs of the second half.  (With two of
+//     both, the loads of A and B spread over the second half had to be there half a step after the last of them: without any loads the loop took 22 to 28 % less time.)
 //   * Loads go straight to LDS, 128 bytes of a row and more: whole lines (with 64 bytes of a row a CU gets 50 GB/s, with 128 it gets 90).
-//   8192 x 8192 x 8192 of random numbers 1.35 PFLOP/s, 8192 x 28672 x 4096 1.40, 8192 x 4096 x 28672 1.41 (of zeros 1.64, 1.54, 1.52);
-//   the ping-pong of two wave groups that was here before 0.9.
+//   * Weight gradients, whose images can be cut in halves of whole lines, have a ring of half steps instead (LoopTR).
+//   us, two steps of both -> now: 8 experts, 8,192 rows uneven, 4096 -> 28672 1,711 / 2,064 (input gradient) -> 1,681 / 1,846, 14336 -> 4096 1,015 / 836 -> 929 /
+//   821; 8192 x 8192 x 8192 of random numbers 809 / 756 -> 779 / 756, of zeros 697 / 663 -> 617 / 595: with random numbers it is the clock that bounds it.  256 rows of 8
+//   experts 421 / 390 -> 401 / 371.
 //
 // Images of a step in LDS, 16-byte chunks XORed so that 16 lanes of a read cover all banks once:
 //   ROW  the reduction is contiguous: [256 rows][64], 128-byte rows
@@ -23,7 +26,7 @@ namespace nxd {
 namespace tile {
 
 constexpr int BM = 256, BN = 256, BK = 64, THREADS = 256;
-constexpr int IMG_BYTES = 256 * BK * 2, STEP_BYTES = 2 * IMG_BYTES, LDS_BYTES = 2 * STEP_BYTES;
+constexpr int IMG_BYTES = 256 * BK * 2, B_BASE = 3 * IMG_BYTES, LDS_BYTES = 5 * IMG_BYTES;   // images: three of A, two of B
 
 typedef __attribute__((address_space(3))) short4_t lds_short4_t;
 
@@ -51,7 +54,7 @@ __device__ __forceinline__ int col(int wn, int j, int lane) {
   return 128 * wn + (BT ? 16 * j + 4 * g : 32 * (j >> 1) + 8 * g + 4 * (j & 1));
 }
 
-template <bool AT, bool BT>
+template <bool BT>
 struct Loop {
   char* smem;
   int lane, wid, wm, wn;
@@ -67,11 +70,11 @@ struct Loop {
     lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wid >> 1, wn = wid & 1;
     lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
     pa = uniform(reinterpret_cast<const char*>(a)), pb = uniform(reinterpret_cast<const char*>(b));
-    da = AT ? (int64_t)BK * lda * 2 : BK * 2, db = BT ? (int64_t)BK * ldb * 2 : BK * 2;
+    da = BK * 2, db = BT ? (int64_t)BK * ldb * 2 : BK * 2;
     back = 0, pieces = min(max((rows + 7) / 8 - 8 * wid, 0), 8);
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      const bool tr = i < 8 ? AT : BT;
+      const bool tr = i >= 8 && BT;
       const int piece = 8 * wid + (i & 7), n = i < 8 ? rows : cols;
       const int64_t ld = i < 8 ? lda : ldb;
       if (tr) {
@@ -87,23 +90,18 @@ struct Loop {
   }
 
   // the half step's fragment addresses (of the first buffer): ROW: [chunk bit 2], TR: [fragment]
-  int ra[AT ? 8 : 2], rb[BT ? 8 : 2];
+  int ra[2], rb[BT ? 8 : 2];
   __device__ __forceinline__ void addresses() {
     const int r = lane & 15, g = lane >> 4;
-    if constexpr (AT) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) ra[i] = tr_at(32 * i + 16 * wm);
-    } else {
-      const int row = 16 * wm + r;
-      ra[0] = row * 128 + 16 * (g ^ row_swz(row));
-      ra[1] = ra[0] ^ 64;
-    }
+    const int row = 16 * wm + r;
+    ra[0] = row * 128 + 16 * (g ^ row_swz(row));
+    ra[1] = ra[0] ^ 64;
     if constexpr (BT) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) rb[j] = IMG_BYTES + tr_at(128 * wn + 16 * j);
+      for (int j = 0; j < 8; ++j) rb[j] = B_BASE + tr_at(128 * wn + 16 * j);
     } else {
       const int c = 128 * wn + 8 * (r >> 2) + (r & 3);
-      rb[0] = IMG_BYTES + c * 128 + 16 * (g ^ row_swz(c));
+      rb[0] = B_BASE + c * 128 + 16 * (g ^ row_swz(c));
       rb[1] = rb[0] ^ 64;
     }
   }
@@ -119,8 +117,7 @@ struct Loop {
   }
   __device__ __forceinline__ bf16x8_t read_row(int at) const { return __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(smem + at)); }
   __device__ __forceinline__ bf16x8_t frag_a(int i, int h, int buf) const {
-    if constexpr (AT) return read_tr(ra[i] + buf + h * (IMG_BYTES / 2));
-    else return read_row(ra[h] + buf + i * 4096);
+    return read_row(ra[h] + buf + i * 4096);
   }
   __device__ __forceinline__ bf16x8_t frag_b(int j, int h, int buf) const {
     if constexpr (BT) return read_tr(rb[j] + buf + h * (IMG_BYTES / 2));
@@ -128,62 +125,47 @@ struct Loop {
   }
 
   template <bool HALF, bool FEW>
-  __device__ __forceinline__ void load(int i, int buf, bool last) {   // piece i of the next step; HALF, last: its second half is past the end
+  __device__ __forceinline__ void load(int i, int img, bool last) {   // piece i (A: 0 .. 7) of the next step; HALF, last: its second half is past the end
     if (FEW && i < 8 && i >= pieces) return;
-    const uint32_t to = lds + buf + (i < 8 ? 0 : IMG_BYTES) + (8 * wid + (i & 7)) * 1024;
+    const uint32_t to = lds + (i < 8 ? 0 : B_BASE) + img + (8 * wid + (i & 7)) * 1024;
     uint32_t from = off[i];
     if constexpr (HALF) {   // (the first half again: not used)
-      const bool tr = i < 8 ? AT : BT;
+      const bool tr = i >= 8 && BT;
       if (last) from -= (back >> i & 1) * (tr ? (uint32_t)((i < 8 ? da : db) / 2) : 64u);
     }
     load_lds(from, i < 8 ? pa : pb, to);
   }
+  template <bool FEW>
+  __device__ __forceinline__ void wait_a() const {   // all loads but A's of the newest step have come
+    if (!FEW || pieces == 8) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+    else if (pieces >= 4) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+    else if (pieces >= 2) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
 
   // acc += the products of so many steps.  IM: row fragments that have rows.  HALF, end: the last step has half the reduction.
-  // FIRST (TR images): the first step has `rows` of the reduction only (1 .. 64); nothing past them is read.
-  template <int IM, bool HALF, bool FIRST = false>
-  __device__ __forceinline__ void run(f32x4_t (&acc)[8][8], int steps, bool end = false, int rows = BK) {
-    static_assert(!FIRST || AT && BT && !HALF, "images of whole reduction rows");
-    static_assert(IM == 8 || IM == 4, "rows");
-    constexpr bool FEW = IM == 4 && !AT;   // only rows that there are (what the LDS holds in the others' place counts for no result)
+  template <int IM, bool HALF>
+  __device__ __forceinline__ void run(f32x4_t (&acc)[8][8], int steps, bool end) {
+    static_assert(IM == 8 || IM == 4 || IM == 2, "rows");
+    constexpr bool FEW = IM < 8;   // only rows that there are (what the LDS holds in the others' place counts for no result)
     bf16x8_t a0[IM], b0[8], a1[IM], b1[8];
-    auto advance = [&](int s) {   // towards step s
-      if (s < steps) pa += da, pb += db;
+    auto advance_a = [&](int s) {   // towards step s
+      if (s < steps) pa += da;
     };
-    if constexpr (FIRST) {
+    auto advance_b = [&](int s) {
+      if (s < steps) pb += db;
+    };
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {   // (rows past the last: that one again)
-        const int past = max(0, 2 * (8 * wid + (i & 7)) + (lane >> 5) - (rows - 1));
-        const uint32_t from = off[i] - past * (uint32_t)((i < 8 ? da : db) / BK);
-        load_lds(from, i < 8 ? pa : pb, lds + (i < 8 ? 0 : IMG_BYTES) + (8 * wid + (i & 7)) * 1024);
-        if (steps == 1) off[i] = from;   // (for the loads that nothing reads)
-      }
-      if (steps > 1) pa += da / BK * rows, pb += db / BK * rows;
-    } else {
+    for (int i = 0; i < 16; ++i) load<HALF, FEW>(i, 0, end && steps == 1);
+    advance_a(1), advance_b(1);
 #pragma unroll
-      for (int i = 0; i < 16; ++i) load<HALF, FEW>(i, 0, end && steps == 1);
-      advance(1);
-    }
-    if (!FIRST || steps > 1) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) load<HALF, FEW>(i, STEP_BYTES, end && steps <= 2);   // (past the end: the last step again, not used)
-    }
-    advance(2);
+    for (int i = 0; i < 16; ++i) load<HALF, FEW>(i, IMG_BYTES, end && steps <= 2);   // (past the end: the last step again, not used)
+    advance_a(2), advance_b(2);
     addresses();
-    if (FIRST && steps == 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    else if (FEW) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");   // (B's pieces of the second step are 8 in every wave)
+    if (FEW) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");   // (B's pieces of the second step are 8 in every wave)
     else asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    if constexpr (FIRST) {   // what was loaded twice counts nothing
-      for (int i = threadIdx.x; i < 2 * (BK - rows) * 32; i += THREADS) {
-        const int t = rows + (i >> 6);
-        *reinterpret_cast<u32x4_t*>(smem + (i >> 5 & 1) * IMG_BYTES + t * 512 + (i & 31) * 16) = u32x4_t{0u, 0u, 0u, 0u};
-      }
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      __builtin_amdgcn_s_barrier();
-      asm volatile("" ::: "memory");
-    }
 #pragma unroll
     for (int j = 0; j < 8; ++j) b0[j] = frag_b(j, 0, 0);
 #pragma unroll
@@ -197,34 +179,173 @@ struct Loop {
       }
       __builtin_amdgcn_sched_barrier(0);
     };
-    int buf = 0;
+    int a_now = 0, a_next = IMG_BYTES, a_free = 2 * IMG_BYTES, b_now = 0;
 #pragma unroll 1
     for (int t = 0, whole = steps - (HALF && end); t < whole; ++t) {
 #pragma unroll
       for (int u = 0; u < 16; ++u) {
-        if (u < 8) b1[u] = frag_b(u, 1, buf);
-        else if (u - 8 < IM) a1[u - 8] = frag_a(u - 8, 1, buf);
+        if (u < 8) b1[u] = frag_b(u, 1, b_now);
+        else if (u - 8 < IM) a1[u - 8] = frag_a(u - 8, 1, a_now);
+        if (u & 1) load<HALF, FEW>(u >> 1, a_free, end && t + 3 >= steps);
         mfmas(u, a0, b0);
       }
-      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      advance_a(t + 3);
+      wait_a<FEW>();
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __builtin_amdgcn_s_barrier();
       __builtin_amdgcn_sched_barrier(0);
-      const int next = buf ^ STEP_BYTES;
 #pragma unroll
       for (int u = 0; u < 16; ++u) {
-        if (u < 8) b0[u] = frag_b(u, 0, next);
-        else if (u - 8 < IM) a0[u - 8] = frag_a(u - 8, 0, next);
-        load<HALF, FEW>(u, buf, end && t + 3 >= steps);
+        if (u < 8) b0[u] = frag_b(u, 0, b_now ^ IMG_BYTES);
+        else if (u - 8 < IM) a0[u - 8] = frag_a(u - 8, 0, a_next);
+        if (u < 8) load<HALF, FEW>(8 + u, b_now, end && t + 3 >= steps);
         mfmas(u, a1, b1);
       }
-      buf = next;
-      advance(t + 3);
+      advance_b(t + 3);
+      b_now ^= IMG_BYTES;
+      const int freed = a_now;
+      a_now = a_next, a_next = a_free, a_free = freed;
     }
     if (HALF && end) {
 #pragma unroll
       for (int u = 0; u < 16; ++u) mfmas(u, a0, b0);
     }
     asm volatile("s_waitcnt vmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");   // (loads that nothing reads; the last sums)
+  }
+};
+
+// Both operands' rows / columns contiguous (weight gradients): half steps of 32 of the reduction, 32 KB each, four of them there.  While the products of
+// half step q run, the fragments of q + 1 are read, and q + 4 is loaded into the place of q, read during q - 1: a step to a step and a half for a
+// load's way, where whole steps left half a step to one.  8 experts 4096 x 28672 over 12,288 rows 3,484 -> 3,397 us, 14336 x 4096 over 16,384
+// 2,159 -> 2,069; one gradient of 8,192 or 3,000 tokens the same within 1 % (its reads and writes, and the clock).  Five half steps: 1 % less for
+// 128256 x 2048, 2 % more for 1,344 to 4,096 tokens.
+struct LoopTR {
+  static constexpr int HK = BK / 2, HALF_BYTES = HK * 256 * 2, PLACE_BYTES = 2 * HALF_BYTES, PLACES = 4;
+  static_assert(PLACES * PLACE_BYTES <= LDS_BYTES, "LDS");
+  char* smem;
+  int lane, wid, wm, wn;
+  uint32_t lds;
+  uint32_t off[8];   // of this lane's pieces of A (0 .. 3) and B from a half step's base
+  const char *pa, *pb;
+  int64_t da, db;    // bytes of 32 reduction rows
+
+  __device__ __forceinline__ LoopTR(char* smem_, const uint16_t* a, int64_t lda, int rows, const uint16_t* b, int64_t ldb, int cols) : smem(smem_) {
+    lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wid >> 1, wn = wid & 1;
+    lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+    pa = uniform(reinterpret_cast<const char*>(a)), pb = uniform(reinterpret_cast<const char*>(b));
+    da = (int64_t)HK * lda * 2, db = (int64_t)HK * ldb * 2;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int t = 2 * (4 * wid + (i & 3)) + (lane >> 5), c = (lane & 31) ^ tr_swz(t);
+      off[i] = (uint32_t)(t * (i < 4 ? lda : ldb) + min(8 * c, (i < 4 ? rows : cols) - 8)) * 2;
+    }
+  }
+  __device__ __forceinline__ int tr_at(int c0) const {   // lane 16 g + 4 q + p: 4 columns from c0 + 4 p on, of reduction rows 8 g + q (and + 4)
+    const int t = 8 * (lane >> 4) + (lane >> 2 & 3), c = c0 + 4 * (lane & 3);
+    return t * 512 + 16 * (c >> 3 ^ tr_swz(t)) + 8 * (c >> 2 & 1);
+  }
+  __device__ __forceinline__ bf16x8_t read(int at) const {
+    const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(smem + at));
+    const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(smem + at + 4 * 512));
+    const short __attribute__((ext_vector_type(8))) v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    return __builtin_bit_cast(bf16x8_t, v);
+  }
+  __device__ __forceinline__ void load(int i, int place) const {
+    load_lds(off[i], i < 4 ? pa : pb, lds + place + (i < 4 ? 0 : HALF_BYTES) + (4 * wid + (i & 3)) * 1024);
+  }
+
+  // acc += the products of so many steps (of two halves).  FIRST: the first step has `rows` of the reduction only (1 .. 64); nothing past them is read.
+  template <bool FIRST>
+  __device__ __forceinline__ void run(f32x4_t (&acc)[8][8], int steps, int rows = BK) {
+    const int n = 2 * steps;
+    if constexpr (FIRST) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {   // (rows past the last: that one again)
+        const int have = max(min(rows - h * HK, HK), 1);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const int past = max(0, 2 * (4 * wid + (i & 3)) + (lane >> 5) - (have - 1));
+          const uint32_t from = off[i] - past * (uint32_t)((i < 4 ? da : db) / HK);
+          load_lds(from, i < 4 ? pa : pb, lds + h * PLACE_BYTES + (i < 4 ? 0 : HALF_BYTES) + (4 * wid + (i & 3)) * 1024);
+          if (h == 1 && steps == 1) off[i] = from;   // (for the loads that nothing reads)
+        }
+        if (h == 0 ? rows > HK : steps > 1) {
+          const int by = h == 0 ? HK : rows > HK ? rows - HK : rows;
+          pa += da / HK * by, pb += db / HK * by;
+        }
+      }
+    }
+    auto advance = [&](int q) {   // towards half step q
+      if (q < n) pa += da, pb += db;
+    };
+#pragma unroll
+    for (int q = FIRST ? 2 : 0; q < PLACES; ++q) {   // (past the end: the last one again, not used)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) load(i, q * PLACE_BYTES);
+      advance(q + 1);
+    }
+    int ra[8], rb[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ra[i] = tr_at(32 * i + 16 * wm), rb[i] = HALF_BYTES + tr_at(128 * wn + 16 * i);
+    auto there = [&]() {   // all loads but those of the three newest half steps have come, and all waves have read so far
+      asm volatile("s_waitcnt vmcnt(16) lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    there();
+    if constexpr (FIRST) {   // what was loaded twice counts nothing
+      for (int i = threadIdx.x; i < 2 * (BK - rows) * 32; i += THREADS) {
+        const int t = rows + (i >> 6);
+        *reinterpret_cast<u32x4_t*>(smem + (t >> 5) * PLACE_BYTES + (i >> 5 & 1) * HALF_BYTES + (t & 31) * 512 + (i & 31) * 16) = u32x4_t{0u, 0u, 0u, 0u};
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    }
+    bf16x8_t a0[8], b0[8], a1[8], b1[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) b0[j] = read(rb[j]);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) a0[i] = read(ra[i]);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();   // (half step 0 has been read)
+    __builtin_amdgcn_sched_barrier(0);
+    int now = 0;   // place of half step q
+    auto mfmas = [&](int u, const bf16x8_t (&a)[8], const bf16x8_t (&b)[8]) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int m = 4 * u + v;
+        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[m >> 3][m & 7]) : "v"(b[m & 7]), "v"(a[m >> 3]));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto after = [](int place) { return place == (PLACES - 1) * PLACE_BYTES ? 0 : place + PLACE_BYTES; };
+#pragma unroll 1
+    for (int q = 0; q < n; q += 2) {
+      int next = after(now);
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        if (u < 8) b1[u] = read(rb[u] + next);
+        else a1[u - 8] = read(ra[u - 8] + next);
+        if (u & 1) load(u >> 1, now);
+        mfmas(u, a0, b0);
+      }
+      advance(q + PLACES + 1);
+      there();
+      now = next, next = after(now);
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        if (u < 8) b0[u] = read(rb[u] + next);
+        else a0[u - 8] = read(ra[u - 8] + next);
+        if (u & 1) load(u >> 1, now);
+        mfmas(u, a1, b1);
+      }
+      advance(q + PLACES + 2);
+      there();
+      now = next;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (loads that nothing reads)
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");   // (the last sums)
   }
 };
 

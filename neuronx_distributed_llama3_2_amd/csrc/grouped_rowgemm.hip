@@ -13,7 +13,7 @@
 // reduction (ROW images), FWD's B along the columns (TR).  Each workgroup finds its (expert, row tile) by a scan of the offsets;
 // the tiles are numbered in an L2 band raster over (row tile, column tile).
 // 8,192 rows of 8 experts, 4096 -> 28672 and 14336 -> 4096, us: FWD 2,170 -> 1,934 and 1,049 -> 943, DGRAD 2,263 -> 1,770 and
-// 1,057 -> 832 (two ping-pong groups of 4 waves, grid of the worst case's tiles).
+// 1,057 -> 832 (two ping-pong groups of 4 waves, grid of the worst case's tiles; the loop's ring since: gemm_tile.h).
 // Few rows (bound by the weights' bytes): a tile of at most 128 rows loads and leaves in memory only the rows that there are.  16 rows of 8
 // experts, FWD / DGRAD us, two groups of 4 waves -> here, and with all rows loaded and left: 4096 -> 28672 414 / 422 -> 414 / 387, 444 / 420; 14336 -> 4096
 // 311 / 307 -> 214 / 217, 245 / 245; 4096 -> 1024 93 / 91 -> 55 / 52, 76 / 72.  What is not split waits for each step's loads, one step ahead: 16
@@ -117,7 +117,7 @@ __global__ void __launch_bounds__(NT, 1) rowgemm_kernel(Params p) {
   const int per = (steps + parts - 1) / parts, first = min(part * per, steps), nk = min(per, steps - first);
   e = __builtin_amdgcn_readfirstlane(e), r0 = __builtin_amdgcn_readfirstlane(r0), r1 = __builtin_amdgcn_readfirstlane(r1);
   const uint16_t* bw = p.b + (int64_t)e * p.b_es;
-  tile::Loop<false, MODE == FWD> loop(smem, p.a + (int64_t)r0 * p.lda + first * BK, p.lda, r1 - r0,
+  tile::Loop<MODE == FWD> loop(smem, p.a + (int64_t)r0 * p.lda + first * BK, p.lda, r1 - r0,
                                       MODE == FWD ? bw + (int64_t)first * BK * p.ldb + n0 : bw + (int64_t)n0 * p.ldb + first * BK, p.ldb,
                                       min(BN, p.ncols - n0));
   f32x4_t acc[8][8];
@@ -125,11 +125,13 @@ __global__ void __launch_bounds__(NT, 1) rowgemm_kernel(Params p) {
   for (int i = 0; i < 8; ++i)
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  // (an expert's last tile: with at most half the rows half the work)
+  // (an expert's last tile: with at most half the rows half the work, with a quarter a quarter: 8 experts of about 1,024 rows each, of which half have a
+  // few rows more, 4096 -> 28672 1,744 -> 1,681 us)
   const bool end = HALF && part == parts - 1;
   if (nk > 0) {
     if (r1 - r0 > BM / 2) loop.template run<8, HALF>(acc, nk, end);
-    else loop.template run<4, HALF>(acc, nk, end);
+    else if (r1 - r0 > BM / 4) loop.template run<4, HALF>(acc, nk, end);
+    else loop.template run<2, HALF>(acc, nk, end);
   }
   const int lane = loop.lane, wid = loop.wid, wm = loop.wm, wn = loop.wn;
 

@@ -87,7 +87,7 @@ __global__ void __launch_bounds__(NT, 1) wgrad_kernel(Params p) {
     t_end = min(p.T, t_begin + p.t_per_split);
   }
   t_begin = __builtin_amdgcn_readfirstlane(t_begin), t_end = __builtin_amdgcn_readfirstlane(t_end);
-  tile::Loop<true, true> loop(smem, p.dy + (int64_t)t_begin * p.ld_dy + m0, p.ld_dy, min(BM, p.M - m0),
+  tile::LoopTR loop(smem, p.dy + (int64_t)t_begin * p.ld_dy + m0, p.ld_dy, min(BM, p.M - m0),
                               p.x + (int64_t)t_begin * p.ld_x + n0, p.ld_x, min(BN, p.N - n0));
   f32x4_t acc[8][8];
 #pragma unroll
@@ -95,7 +95,7 @@ __global__ void __launch_bounds__(NT, 1) wgrad_kernel(Params p) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   const int tokens = t_end - t_begin;
-  loop.template run<8, false, TAIL>(acc, ceil_div(tokens, BK), false, (tokens - 1) % BK + 1);
+  loop.template run<TAIL>(acc, ceil_div(tokens, BK), (tokens - 1) % BK + 1);
   const int lane = loop.lane, wid = loop.wid, wm = loop.wm, wn = loop.wn;
 
   // 8 rounds of a wave's 16 rows x 128 columns through a padded LDS slab of its own
