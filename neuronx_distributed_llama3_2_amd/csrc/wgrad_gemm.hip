@@ -16,11 +16,12 @@
 //
 // Structure: the loop of gemm_tile.h (4 waves of 128 x 128 results, one workgroup per CU), both operands' images with contiguous
 // features, read with the hardware's transposing read; a token count that is no multiple of 64 makes the first step a partial one.
-//   * With one token split per tile the workgroup alone adds to its tile: it loads, adds and stores straight from the registers, 64
-//     contiguous bytes of 16 rows each, the line's other half right after, the loads of 6 of 8 rounds on their way together.  Through LDS, 512
-//     bytes of a row each, 1,000 tokens 128256 x 2048 took 900 us instead of 777, 3,000 1,623 instead of 1,532, 8 experts' 4096 x 28672 over 16,384
-//     4,693 instead of 4,385.  With S splits the adds are S atomics in any order, through LDS so that they cover 256 contiguous bytes, issued
-//     without return and left in flight when the workgroup exits.
+//   * With one token split per tile the workgroup alone adds to its tile: it loads, adds and stores straight from the registers, the loads of 6 of 8
+//     rounds on their way together.  Lanes exchange halves of their fragments so that 8 of them have a line; whole lines can be read and written past the
+//     caches, which then keep the operands (64 bytes of 16 rows a time, through the caches: 3,000 tokens 128256 x 2048 1,561 us, now 1,518, 16384 x 2048 201 / 193; 1,344
+//     3072 x 4096 55 / 50; 8,192 12288 x 4096 674 / 640; 8 experts' 14336 x 4096 over 16,384 2,177 / 1,991; half lines past the caches are read
+//     twice, 4 to 8 % more).  Through LDS, 512 bytes of a row each, 2 to 16 % more.  With S splits the adds are S atomics in any order, through LDS so
+//     that they cover 256 contiguous bytes, issued without return and left in flight when the workgroup exits.
 //   * Against 8 waves of 128 x 64 in ping-pong: 1,000 tokens 4096 x 4096 54 -> 48 us, 16384 x 2048 97 -> 86; 3,000 128256 x 2048 1,708 -> 1,526; 8,192
 //     6144 x 4096 406 -> 372; 8 experts' 14336 x 4096 over 32,768 3,903 -> 3,561.
 //   * grouped (MoE expert weight gradients, dW[e] += x_e^T dy_e over expert-sorted rows): the grid covers (split, expert, tile); each
@@ -102,29 +103,43 @@ __global__ void __launch_bounds__(NT, 1) wgrad_kernel(Params p) {
   constexpr int LD = 132;
   float* slab = reinterpret_cast<float*>(smem) + wid * (2 * 16 * LD);
   if (p.own) {
-    const int row = m0 + 16 * wm + (lane & 15), col = n0 + tile::col<true>(wn, 0, lane);
+    // lanes r and r + 8 exchange halves of a pair of fragments: 128 contiguous bytes of 8 rows
+    const bool up = lane & 8;
+    const int row = m0 + 16 * wm + (lane & 7), col = n0 + tile::col<true>(wn, 0, lane) + (up ? 16 : 0);
     float* cp = cbase + (int64_t)row * p.ldc + col;
     constexpr int AHEAD = 6;
     f32x4_t cur[AHEAD][8];
     const bool whole = m0 + BM <= p.M && n0 + BN <= p.N;
     auto all = [&](auto ok) {
+      auto at = [&](int i, int j) { return reinterpret_cast<f32x4_t*>(cp + (int64_t)(32 * i + 8 * (j & 1)) * p.ldc + 32 * (j >> 1)); };
       auto load = [&](int i) {   // 16 rows
 #pragma unroll
         for (int j = 0; j < 8; ++j)
-          if (ok(i, j)) cur[i % AHEAD][j] = *reinterpret_cast<const f32x4_t*>(cp + (int64_t)(32 * i) * p.ldc + 16 * j);
+          if (ok(i, j)) cur[i % AHEAD][j] = __builtin_nontemporal_load(at(i, j));
       };
 #pragma unroll
       for (int i = 0; i < AHEAD; ++i) load(i);
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-          if (ok(i, j)) *reinterpret_cast<f32x4_t*>(cp + (int64_t)(32 * i) * p.ldc + 16 * j) = cur[i % AHEAD][j] + acc[i][j];
+        for (int j = 0; j < 8; j += 2) {
+          f32x4_t lo, hi;
+          asm volatile("" : "+a"(acc[i][j]), "+a"(acc[i][j + 1]));   // (or all exchanges are made before both branches: 256 spills)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float u = acc[i][j][e], v = acc[i][j + 1][e];
+            const float o = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(up ? u : v), 0x128 /* row_ror:8 */, 0xf, 0xf, false));
+            lo[e] = up ? o : u, hi[e] = up ? v : o;
+          }
+          if (ok(i, j)) __builtin_nontemporal_store(cur[i % AHEAD][j] + lo, at(i, j));
+          if (ok(i, j + 1)) __builtin_nontemporal_store(cur[i % AHEAD][j + 1] + hi, at(i, j + 1));
+        }
         if (i + AHEAD < 8) load(i + AHEAD);
+        __builtin_amdgcn_sched_barrier(0);
       }
     };
     if (whole) all([](int, int) { return true; });
-    else all([&](int i, int j) { return row + 32 * i < p.M && col + 16 * j < p.N; });
+    else all([&](int i, int j) { return row + 32 * i + 8 * (j & 1) < p.M && col + 32 * (j >> 1) < p.N; });
     return;
   }
   __syncthreads();   // every wave is done with the ring
@@ -146,11 +161,13 @@ __global__ void __launch_bounds__(NT, 1) wgrad_kernel(Params p) {
 // Few tokens, where most of the time goes into the gradient's reads and writes and into starting and ending a workgroup: 8 waves of
 // 128 x 64 results with a load, an add and a store of 32 rows at a time, steps of 32 tokens in a ring of four, half the registers to fill and
 // to empty.  us here / by the loop above:
-//   * 8 experts' 4096 x 28672 and 14336 x 4096 gradients: 256 tokens each 1,762, 821 / 1,909, 947; 1,024 2,756, 1,372 / 2,867, 1,483;
-//     1,536 3,639, 1,824 / 3,545, 1,803; 4,096 7,857, 3,903 / 7,070, 3,561;
+//   * 8 experts' 4096 x 28672 and 14336 x 4096 gradients: 256 tokens each 1,505, 697 / 1,588, 807; 768 2,237, 1,056 / 2,300, 1,084; 1,024 2,644,
+//     1,278 / 2,627, 1,308; 1,280 3,107, 1,507 / 3,032, 1,479; 1,536 3,505, 1,715 / 3,382, 1,646 (the gradient past the caches in both; through them, 256
+//     tokens 1,686, 821, 512 1,942, 1,024 2,749, 1,353);
 //   * one gradient, whole steps of 32 tokens: 512 x 512 512 tokens 20 / 27, 1,024 32 / 37, 2,048 53 / 56, 3,072 75.3 / 74.9; 2048 x 2048 23 / 30, 34 /
 //     39, 56 / 58, 78 / 78; 3072 x 4096 1,056 46.3 / 48.9, 2,048 68 / 69; 4096 x 4096 512 39 / 42, 1,056 54 / 56, 1,536 69 / 67; 16384 x 2048 1,024
 //     102 / 109, 2,080 155 / 157, 3,072 205 / 199;
+//     (these two lines were measured with the gradient through the caches; past them both take 3 to 10 % less)
 //   * a partial last step (the loop's is its first): 4096 x 4096, 500 tokens 40 / 36, 700 45 / 40; 768 x 4096 or 128256 x 2048, 500 24, 560 / 28,
 //     608, 700 29, 659 / 32, 668, 1,000 38, 794 / 38, 788.
 //
@@ -164,7 +181,7 @@ __global__ void __launch_bounds__(NT, 1) wgrad_kernel(Params p) {
 //   * pieces issued after stage S's last: S+1 (4) and S+2's first half (2) -> vmcnt(6), less at the tail.
 namespace few {
 
-constexpr int FEW = 1400;   // tokens of a group
+constexpr int FEW = 1150;   // tokens of a group
 constexpr int BK = 32, STAGES = 4, NT = 512;
 inline bool dense(int T, int tiles) {   // (one gradient, unsplit)
   if (T % BK) return T <= 450 || (T <= 700 && (tiles < 192 || tiles > 1024));
@@ -329,7 +346,7 @@ __global__ void __launch_bounds__(NT, 1) kernel(Params p) {
   auto load = [&](int rnd) {
 #pragma unroll
     for (int k = 0; k < 8; ++k)
-      if (32 * rnd + 4 * k < left) cur[k] = *reinterpret_cast<const f32x4_t*>(cp + (int64_t)(32 * rnd + 4 * k) * p.ldc);
+      if (32 * rnd + 4 * k < left) cur[k] = __builtin_nontemporal_load(reinterpret_cast<const f32x4_t*>(cp + (int64_t)(32 * rnd + 4 * k) * p.ldc));
   };
   load(0);
   __syncthreads();   // every wave is done with the ring
@@ -348,7 +365,7 @@ __global__ void __launch_bounds__(NT, 1) kernel(Params p) {
     if (rnd < 3) load(rnd + 1);
 #pragma unroll
     for (int k = 0; k < 8; ++k)
-      if (32 * rnd + 4 * k < left) *reinterpret_cast<f32x4_t*>(cp + (int64_t)(32 * rnd + 4 * k) * p.ldc) = sum[k];
+      if (32 * rnd + 4 * k < left) __builtin_nontemporal_store(sum[k], reinterpret_cast<f32x4_t*>(cp + (int64_t)(32 * rnd + 4 * k) * p.ldc));
     __builtin_amdgcn_wave_barrier();
   }
 }
