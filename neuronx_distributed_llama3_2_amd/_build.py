@@ -90,8 +90,8 @@ def _sources(target: str):
     """(kernel TUs, host TUs that include the torch headers) of one extension module."""
     if target == "_C":
         return sorted(CSRC.glob("*.hip")), sorted(CSRC.glob("*.cpp"))
-    # the experts' matrix products, and projections of a few rows
-    shared = [CSRC / n for n in ("grouped_gemm.hip", "grouped_rowgemm.hip", "few_rows.hip")]
+    # the experts' matrix products, products with an activation, and projections of a few rows
+    shared = [CSRC / n for n in ("grouped_gemm.hip", "grouped_rowgemm.hip", "act_gemm.hip", "few_rows.hip")]
     return [*sorted((CSRC / "hybrid").glob("*.hip")), *shared], [*sorted((CSRC / "hybrid").glob("*.cpp")), CSRC / "gemm.cpp"]
 
 

@@ -35,6 +35,10 @@
 #include <unordered_set>
 #include <vector>
 
+namespace nxd {
+int act_gemm_launch(int, const void*, const void*, void*, int64_t, int64_t, int64_t, hipStream_t);
+}
+
 namespace nxd_gemm {
 
 #define LT_CHECK(x)                                                                          \
@@ -592,12 +596,26 @@ std::vector<std::pair<std::string, float>> gemm_tuned_entries() { return Tuner::
 void gemm_set_no_streamk(int v) { g_no_streamk = v < 0 ? -1 : (v > 0 ? 1 : 0); }
 bool gemm_no_streamk() { return no_streamk(); }
 
+// y = act(x w^T) by the kernel of act_gemm.hip
+void act_gemm(int64_t act, at::Tensor x, at::Tensor w, at::Tensor y) {
+  for (const auto& t : {x, w, y})
+    TORCH_CHECK(t.is_cuda() && t.get_device() == x.get_device() && t.scalar_type() == at::kBFloat16 && t.dim() == 2 && t.is_contiguous() &&
+                    reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0,
+                "act_gemm: contiguous 2-D bf16 on one GPU, 16-byte aligned");
+  const int64_t N = y.size(1);
+  TORCH_CHECK(w.size(1) == x.size(1) && y.size(0) == x.size(0) && w.size(0) == (act ? N : 2 * N), "act_gemm: sizes");
+  const int rc = nxd::act_gemm_launch((int)act, x.data_ptr(), w.data_ptr(), y.data_ptr(), x.size(0), N, x.size(1),
+                                      at::hip::getCurrentHIPStream().stream());
+  TORCH_CHECK(rc == 0, "act_gemm: failed or not such sizes, ", rc);
+}
+
 }  // namespace nxd_gemm
 
 void register_gemm(pybind11::module& m) {
   m.def("gemm", &nxd_gemm::gemm, "d = alpha * a @ b + beta * c (autotuned hipBLASLt)", pybind11::arg("a"),
         pybind11::arg("b"), pybind11::arg("d"), pybind11::arg("c") = pybind11::none(), pybind11::arg("alpha") = 1.0,
         pybind11::arg("beta") = 0.0);
+  m.def("act_gemm", &nxd_gemm::act_gemm);
   m.def("gemm_tuned_entries", &nxd_gemm::gemm_tuned_entries);
   m.def("gemm_set_no_streamk", &nxd_gemm::gemm_set_no_streamk, "1: skip stream-K solutions, 0: allow, -1: env");
   m.def("gemm_no_streamk", &nxd_gemm::gemm_no_streamk);

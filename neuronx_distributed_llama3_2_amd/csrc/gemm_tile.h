@@ -54,6 +54,15 @@ __device__ __forceinline__ int col(int wn, int j, int lane) {
   return 128 * wn + (BT ? 16 * j + 4 * g : 32 * (j >> 1) + 8 * g + 4 * (j & 1));
 }
 
+// After the wait for the last sums: without this the compiler, which doesn't know what the asm of the MFMAs takes, may read them before the wait
+template <int IM>
+__device__ __forceinline__ void settled(f32x4_t (&acc)[8][8]) {
+#pragma unroll
+  for (int i = 0; i < IM; ++i)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) asm volatile("" : "+a"(acc[i][j]));
+}
+
 template <bool BT>
 struct Loop {
   char* smem;
@@ -211,6 +220,7 @@ struct Loop {
       for (int u = 0; u < 16; ++u) mfmas(u, a0, b0);
     }
     asm volatile("s_waitcnt vmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");   // (loads that nothing reads; the last sums)
+    settled<IM>(acc);
   }
 };
 
@@ -346,6 +356,7 @@ struct LoopTR {
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (loads that nothing reads)
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");   // (the last sums)
+    settled<8>(acc);
   }
 };
 

@@ -502,10 +502,10 @@ class DecoderInferenceMixin:
         if w.dtype == torch.int8 or (x.is_cuda and (M <= 8 or M <= _FEW_ROWS and x.dtype == w.dtype == torch.bfloat16
                                                        and b is None and few_rows_pay(M, *w.shape, glu))):
             return skinny_linear(x, w, scale, b, glu=glu)
-        from ..trace.weight_layout import packed_linear
+        from ..trace.weight_layout import packed_linear, packed_linear_act
 
-        y = packed_linear(mod, x, w, b)   # pre-packed K-major copy when the layout pass chose it
-        return ops.swiglu(y) if glu else y
+        # (the pre-packed K-major copy when the layout pass chose it)
+        return packed_linear_act(mod, x, w, b, "swiglu") if glu else packed_linear(mod, x, w, b)
 
     def _ffn(self, layer, h: torch.Tensor) -> torch.Tensor:
         raise NotImplementedError

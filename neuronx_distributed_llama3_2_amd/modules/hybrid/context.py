@@ -57,14 +57,13 @@ def linear(x: torch.Tensor, mod: torch.nn.Module, fused: bool = False, epilogue:
     """x [M, K] @ mod.weight^T: through the module's packed copy when the layout pass chose it; fused: a few
     rows by the kernels that stream the weights.  epilogue "relu2": its squared ReLU."""
     from ... import ops
-    from ...trace.weight_layout import packed_linear
+    from ...trace.weight_layout import packed_linear, packed_linear_act
 
     if fused and few_rows(x, mod.weight, SOME_ROWS) and streams(x.shape[0], *mod.weight.shape, epilogue != "store"):
         if x.shape[0] <= FEW_ROWS:
             return ops.decode_linear(mod.weight, x, epilogue=epilogue)
         return ops.linear_few(x, mod.weight, epilogue, tickets=tickets)
-    y = packed_linear(mod, x, mod.weight)
-    return ops.relu_squared(y) if epilogue == "relu2" else y
+    return packed_linear_act(mod, x, mod.weight, None, "relu2") if epilogue == "relu2" else packed_linear(mod, x, mod.weight)
 
 
 def step_tickets(rows: int, device) -> Optional[torch.Tensor]:

@@ -8,6 +8,7 @@ beta = 1, no bf16 temporary).  On CPU, or with NXD_TUNED_GEMM=0, they fall back 
 from __future__ import annotations
 
 import os
+from typing import Optional
 
 import torch
 
@@ -44,6 +45,30 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias=None, out: torch.Tensor = None
     if out is not None:
         out.copy_(y)
         return out
+    return y
+
+
+_ACTS = {"swiglu": 0, "relu2": 1}
+
+
+def act_pays(rows: int, weight_rows: int, K: int) -> bool:
+    """Whether csrc/act_gemm.hip is faster than a library product and the activation's own pass: work for three quarters of the CUs (256 x 256
+    results each) and a reduction that the pass is not small beside.  us, two launches / one, weights from memory: SwiGLU of 8,192
+    columns, reduction 2,048: 512 rows 41 / 45, 768 56 / 57, 1,024 73 / 62, 2,304 150 / 147, 4,096 245 / 231; of 14,336, 4,096: 256 rows 80 / 85,
+    512 122 / 108, 1,792 385 / 350, 4,096 706 / 708; of 28,672, 8,192: 2,304 rows 1,555 / 1,599; squared ReLU of 12,288, 2,048: 768 rows 46 /
+    51, 1,024 62 / 55, 4,096 189 / 172."""
+    return K % 32 == 0 and K <= 4096 and rows * weight_rows >= 192 * 256 * 256
+
+
+def linear_act(x: torch.Tensor, w: torch.Tensor, act: str) -> Optional[torch.Tensor]:
+    """act(x [..., K] @ w^T) in one launch, or None where that is not done or not faster.  "swiglu": w [2 N, K] = [gate; up]; "relu2": w [N, K]."""
+    K, N = w.shape[1], w.shape[0] // 2 if act == "swiglu" else w.shape[0]
+    if not (_native(x, w) and x.dtype == w.dtype == torch.bfloat16 and act_pays(x.numel() // max(K, 1), w.shape[0], K)
+            and N % (128 if act == "swiglu" else 8) == 0 and (N + 256) * K < 2 ** 31
+            and x.shape[-1] == K and x.is_contiguous() and w.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
+        return None
+    y = torch.empty(x.shape[:-1] + (N,), dtype=x.dtype, device=x.device)
+    gemm_ext().act_gemm(_ACTS[act], x.view(-1, K), w, y.view(-1, N))
     return y
 
 

@@ -9,7 +9,7 @@ from typing import Optional
 import torch
 
 from ._ext import ext, use_native
-from .gemm import linear as _linear
+from .gemm import linear as _linear, linear_act
 
 
 def dequantize_weight(w: torch.Tensor, scale: Optional[torch.Tensor], dtype=torch.bfloat16) -> torch.Tensor:
@@ -77,6 +77,10 @@ def skinny_linear(x: torch.Tensor, w: torch.Tensor, scale: Optional[torch.Tensor
             ext().gemv(x2, w, s, 1.0, bias, y, glu)
             return y.view(lead + (N,))
     wd = dequantize_weight(w, scale, x.dtype) if w.dtype == torch.int8 else w
+    if glu and bias is None:
+        y = linear_act(x, wd, "swiglu")
+        if y is not None:
+            return y
     y = _linear(x, wd, bias)
     if glu:
         from .activations import swiglu

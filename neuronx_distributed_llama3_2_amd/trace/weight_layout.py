@@ -137,6 +137,18 @@ def packed_linear(mod, x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Te
     return _gemm.linear(x, w, bias)
 
 
+def packed_linear_act(mod, x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], act: str) -> torch.Tensor:
+    """act(packed_linear(...)), act "swiglu" or "relu2": in one launch where that is faster."""
+    if bias is None and getattr(mod, "_nxd_packed_kn", None) is None:
+        y = _gemm.linear_act(x, w, act)
+        if y is not None:
+            return y
+    from .. import ops
+
+    y = packed_linear(mod, x, w, bias)
+    return ops.swiglu(y) if act == "swiglu" else ops.relu_squared(y)
+
+
 def save_layouts(path: str, layouts: Dict[str, str]) -> None:
     with open(os.path.join(path, LAYOUT_FILE), "w") as f:
         json.dump(layouts, f, indent=1, sort_keys=True)
