@@ -191,6 +191,7 @@ struct Loop {
     int a_now = 0, a_next = IMG_BYTES, a_free = 2 * IMG_BYTES, b_now = 0;
 #pragma unroll 1
     for (int t = 0, whole = steps - (HALF && end); t < whole; ++t) {
+      asm volatile("s_nop 3");   // (after moves of the sums ahead of the loop)
 #pragma unroll
       for (int u = 0; u < 16; ++u) {
         if (u < 8) b1[u] = frag_b(u, 1, b_now);
@@ -214,10 +215,13 @@ struct Loop {
       b_now ^= IMG_BYTES;
       const int freed = a_now;
       a_now = a_next, a_next = a_free, a_free = freed;
+      if (HALF) asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");   // (the sums may move after the loop)
     }
-    if (HALF && end) {
+    if (HALF && end) {   // (s_nop: the sums may have moved to other registers just before)
 #pragma unroll
-      for (int u = 0; u < 16; ++u) mfmas(u, a0, b0);
+      for (int i = 0; i < IM; ++i)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) asm volatile("s_nop 3\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(b0[j]), "v"(a0[i]));
     }
     asm volatile("s_waitcnt vmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");   // (loads that nothing reads; the last sums)
     settled<IM>(acc);

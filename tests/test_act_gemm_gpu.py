@@ -30,6 +30,7 @@ def _want(act, x, w):
     ("swiglu", 1300, 2048, 192), ("relu2", 1300, 4096, 96),    # 96 tiles, in 2 pieces
     ("swiglu", 2100, 2048, 64), ("relu2", 2200, 4104, 224),    # more, whole
     ("swiglu", 4200, 2048, 256), ("relu2", 4361, 4096, 32),    # a whole round and some more
+    ("swiglu", 700, 256, 416), ("relu2", 200, 512, 2080),      # half steps after longer reductions
 ])
 def test_act_gemm(act, R, N, K):
     from neuronx_distributed_llama3_2_amd.ops._ext import gemm_ext
