@@ -630,8 +630,11 @@ static bool merge_in_launch(int MD, const Splits& sp) { return ceil_div(MD, 64 *
 // output the o_proj GEMV would read) -> this workgroup's o_proj partial, fp32 atomics into oacc: the
 // long-context form of FUSE (one launch instead of the merge + o_proj pair).  Grid (batch, kv head,
 // R row chunks), the split weights of each query row in LDS.
-template <int D, int NWV>
+// NP: passes over the workgroup's rows (p.NP; 0: read there).  Known, the loads of Wo behind the partials' are counted, and what comes first waits for the
+// partials alone: the compiler's wait for an unknown number of loads was for all of them.
+template <int D, int NWV, int NP>
 __global__ void __launch_bounds__(64 * NWV) merge_oproj_kernel(Params p) {
+  if (NP) p.NP = NP;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   float* of = reinterpret_cast<float*>(smem);   // [M][D] merged attention output
   float* wts = of + 16 * D;                     // [nsplit][16] normalised split weights
@@ -652,10 +655,13 @@ __global__ void __launch_bounds__(64 * NWV) merge_oproj_kernel(Params p) {
   const int e0 = tid % elems, h0 = tid / elems;
   const float* src0 = p.po + (pb + e0 / D) * D + e0 % D;
   float pv[PMAX];
-  if (regs && tid < elems * H) {
+  if (regs) {   // (past the last: the last again, not used)
 #pragma unroll
-    for (int i = 0; i < PMAX; ++i)
-      if (h0 + i * H < ns) pv[i] = src0[(h0 + i * H) * st];
+    for (int c = 0; c < PMAX; c += 4)
+      if (c * H < ns) {
+#pragma unroll
+        for (int i = c; i < c + 4; ++i) pv[i] = src0[(uint32_t)min(h0 + i * H, ns - 1) * (uint32_t)st];
+      }
   }
   // split weights of query row m: one wave per row, one split per lane (all loads in parallel: a
   // serial walk over the splits was a chain of dependent L2 round trips, 7.8 us per launch).  The
@@ -925,13 +931,12 @@ int decode_attn_oproj_launch(const void* q, const int64_t* qs, const void* kc, c
     if (rc != 0) return rc;
     if (ns2 != ns) return 3;   // the attention launch split differently: never write the output through null
     p.nsplit = ns; p.po = po; p.pm = pm; p.pl = pl;
-    if (D == 64) {
-      (void)hipFuncSetAttribute((const void*)dattn::merge_oproj_kernel<64, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)mlds);
-      hipLaunchKernelGGL((dattn::merge_oproj_kernel<64, 8>), grid, block, mlds, stream, p);
-    } else {
-      (void)hipFuncSetAttribute((const void*)dattn::merge_oproj_kernel<128, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)mlds);
-      hipLaunchKernelGGL((dattn::merge_oproj_kernel<128, 4>), grid, block, mlds, stream, p);
-    }
+    auto* f = D == 64 ? (p.NP == 1 ? &dattn::merge_oproj_kernel<64, 8, 1> : p.NP == 2 ? &dattn::merge_oproj_kernel<64, 8, 2>
+                                     : p.NP == 4 ? &dattn::merge_oproj_kernel<64, 8, 4> : &dattn::merge_oproj_kernel<64, 8, 0>)
+                      : (p.NP == 1 ? &dattn::merge_oproj_kernel<128, 4, 1> : p.NP == 2 ? &dattn::merge_oproj_kernel<128, 4, 2>
+                                     : p.NP == 4 ? &dattn::merge_oproj_kernel<128, 4, 4> : &dattn::merge_oproj_kernel<128, 4, 0>);
+    (void)hipFuncSetAttribute((const void*)f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)mlds);
+    hipLaunchKernelGGL(f, grid, block, mlds, stream, p);
     return (int)hipGetLastError();
   }
   const size_t lds = (size_t)nwv * dattn::KB * D * 2 + (size_t)nwv * 16 * D * 4 + (size_t)2 * nwv * 16 * 4;
