@@ -66,15 +66,39 @@ __device__ __forceinline__ float dot8_bf16(const u32x4_t& a, const u32x4_t& b, f
   return acc;
 }
 
+// op(v, v of lane ^ O), by the lanes' own data paths: a step of a wave's sum is one or two VALU instructions (__shfl_xor goes through LDS, about 60 cycles a step
+// in a chain of six).  Same order of sums, so the same bits; a lane that is off counts as zero, as there.
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+template <int O, typename F>
+__device__ __forceinline__ float lanes_xor(float v, F op) {
+  static_assert(O == 1 || O == 2 || O == 4 || O == 8 || O == 16 || O == 32, "lanes");
+  const uint32_t u = __builtin_bit_cast(uint32_t, v);
+  if constexpr (O == 32 || O == 16) {   // both operands' halves (rows of 16) swapped: the pair, in all lanes
+    const auto r = [&] {
+      if constexpr (O == 32) return __builtin_amdgcn_permlane32_swap(u, u, false, false);
+      else return __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    }();
+    return op(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1]));
+  } else if constexpr (O == 8) {
+    return op(v, dpp<0x128>(v));              // row_ror:8
+  } else if constexpr (O == 4) {
+    return op(v, dpp<0x1B>(dpp<0x141>(v)));   // 7 - lane of 8, then 3 - lane of 4
+  } else {
+    return op(v, dpp<O == 2 ? 0x4E : 0xB1>(v));
+  }
+}
+template <int O>
+__device__ __forceinline__ float lanes_add(float v) { return lanes_xor<O>(v, [](float a, float b) { return a + b; }); }
+template <int O>
+__device__ __forceinline__ float lanes_max(float v) { return lanes_xor<O>(v, [](float a, float b) { return fmaxf(a, b); }); }
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  return lanes_add<1>(lanes_add<2>(lanes_add<4>(lanes_add<8>(lanes_add<16>(lanes_add<32>(v))))));
 }
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
+  return lanes_max<1>(lanes_max<2>(lanes_max<4>(lanes_max<8>(lanes_max<16>(lanes_max<32>(v))))));
 }
 
 // Block-wide sum for blockDim.x a multiple of 64 (<= 1024); `red` must hold 16 floats.

@@ -157,7 +157,12 @@ __device__ __forceinline__ void oproj_tail(const Params& p, const float* of, con
         const f32x4_t o4 = *reinterpret_cast<const f32x4_t*>(orow + j);
         dot += w[j] * o4[0] + w[j + 1] * o4[1] + w[j + 2] * o4[2] + w[j + 3] * o4[3];
       }
-      for (int off = tpr / 2; off > 0; off >>= 1) dot += __shfl_xor(dot, off, 64);
+      if (tpr > 32) dot = lanes_add<32>(dot);
+      if (tpr > 16) dot = lanes_add<16>(dot);
+      if (tpr > 8) dot = lanes_add<8>(dot);
+      if (tpr > 4) dot = lanes_add<4>(dot);
+      if (tpr > 2) dot = lanes_add<2>(dot);
+      if (tpr > 1) dot = lanes_add<1>(dot);
       if (seg == 0) unsafeAtomicAdd(p.oacc + (int64_t)(b * p.T + tt) * p.Hout + row, dot);
     }
   }
@@ -312,8 +317,7 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(Params p) {
         sc[kt][v] = sv;
         cm = fmaxf(cm, sv);
       }
-    cm = fmaxf(cm, __shfl_xor(cm, 16, 64));
-    cm = fmaxf(cm, __shfl_xor(cm, 32, 64));
+    cm = lanes_max<32>(lanes_max<16>(cm));
     const float nm = fmaxf(run_m, cm);
     const float mu = nm == -INFINITY ? 0.f : nm;
     const float alpha = run_m == -INFINITY ? 0.f : exp2f(run_m - mu);
@@ -330,8 +334,7 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(Params p) {
       p2[kt][0] = pack2bf(e[0], e[1]);
       p2[kt][1] = pack2bf(e[2], e[3]);
     }
-    ls += __shfl_xor(ls, 16, 64);
-    ls += __shfl_xor(ls, 32, 64);
+    ls = lanes_add<32>(lanes_add<16>(ls));
     run_l = run_l * alpha + ls;
     run_m = nm;
     // rescale O rows 4 g + v by their row's alpha (held by lane 4 g + v)
@@ -498,8 +501,7 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(Params p) {
         float gm = -INFINITY;
         for (int sp = lane; sp < ns; sp += 64)
           gm = fmaxf(gm, __hip_atomic_load(p.pm + pb + (int64_t)sp * M + m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) gm = fmaxf(gm, __shfl_xor(gm, off, 64));
+        gm = wave_max(gm);
         float L = 0.f;
         for (int sp = lane; sp < ns; sp += 64) {
           const float ms = __hip_atomic_load(p.pm + pb + (int64_t)sp * M + m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -507,8 +509,7 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(Params p) {
           wts[sp * 16 + m] = w;
           L += w * __hip_atomic_load(p.pl + pb + (int64_t)sp * M + m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) L += __shfl_xor(L, off, 64);
+        L = wave_sum(L);
         const float inv = L > 0.f ? 1.f / L : 0.f;
         for (int sp = lane; sp < ns; sp += 64) wts[sp * 16 + m] *= inv;
       }
@@ -687,19 +688,16 @@ __global__ void __launch_bounds__(64 * NWV) merge_oproj_kernel(Params p) {
       const int m = wid + k * NWV;
       if (m >= M) break;   // wave-uniform
       float gm = pmv[k];
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) gm = fmaxf(gm, __shfl_xor(gm, off, 64));
+      gm = wave_max(gm);
       const float w = pmv[k] == -INFINITY ? 0.f : __expf(pmv[k] - gm);
       float L = w * plv[k];
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) L += __shfl_xor(L, off, 64);
+      L = wave_sum(L);
       if (lane < ns) wts[lane * 16 + m] = L > 0.f ? w / L : 0.f;
     }
   } else for (int m = wid; m < M; m += NWV) {
     float gm = -INFINITY;
     for (int s = lane; s < ns; s += 64) gm = fmaxf(gm, p.pm[pb + (int64_t)s * M + m]);
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) gm = fmaxf(gm, __shfl_xor(gm, off, 64));
+    gm = wave_max(gm);
     float L = 0.f;
     for (int s = lane; s < ns; s += 64) {
       const float ms = p.pm[pb + (int64_t)s * M + m];
@@ -707,8 +705,7 @@ __global__ void __launch_bounds__(64 * NWV) merge_oproj_kernel(Params p) {
       wts[s * 16 + m] = w;
       L += w * p.pl[pb + (int64_t)s * M + m];
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) L += __shfl_xor(L, off, 64);
+    L = wave_sum(L);
     const float inv = L > 0.f ? 1.f / L : 0.f;
     for (int s = lane; s < ns; s += 64) wts[s * 16 + m] *= inv;
   }

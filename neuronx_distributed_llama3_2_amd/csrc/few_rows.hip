@@ -527,8 +527,7 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
       float v = ss[t];
-      v += __shfl_xor(v, 16, 64);
-      v += __shfl_xor(v, 32, 64);
+      v = lanes_add<32>(lanes_add<16>(v));
       if (q == 0) lds_write(lds_at(sq + w * 16 * MT + 16 * t + c), v);
     }
   };

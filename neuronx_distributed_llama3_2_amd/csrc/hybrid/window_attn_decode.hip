@@ -761,8 +761,7 @@ __global__ void __launch_bounds__(256, 2) attn_decode_mfma_kernel(WindowAttnPara
       x[j] = k0 + 16 * (j >> 2) + 4 * g4 + (j & 3) < end ? sv : -INFINITY;
       cm = fmaxf(cm, x[j]);
     }
-    cm = fmaxf(cm, __shfl_xor(cm, 16, 64));
-    cm = fmaxf(cm, __shfl_xor(cm, 32, 64));
+    cm = lanes_max<32>(lanes_max<16>(cm));
     const float nm = fmaxf(run_m, cm), mu = nm == -INFINITY ? 0.f : nm, alpha = run_m == -INFINITY ? 0.f : expf(run_m - mu);
     float sum = 0.f;
 #pragma unroll
@@ -770,8 +769,7 @@ __global__ void __launch_bounds__(256, 2) attn_decode_mfma_kernel(WindowAttnPara
       x[j] = expf(x[j] - mu);
       sum += x[j];
     }
-    sum += __shfl_xor(sum, 16, 64);
-    sum += __shfl_xor(sum, 32, 64);
+    sum = lanes_add<32>(lanes_add<16>(sum));
     run_l = run_l * alpha + sum;
     run_m = nm;
     bf16x8_t pf[3];   // the largest bf16 number below the weight, the largest one below what is left, and the rest
