@@ -19,6 +19,7 @@ int softcap_launch(float*, int64_t, float, hipStream_t);
 int delta_prep_launch(bool, const DeltaParams&, hipStream_t);
 int delta_scan_launch(bool, const DeltaParams&, hipStream_t);
 int delta_chunk_launch(bool, const DeltaParams&, hipStream_t);
+int64_t delta_chunk_split_floats(const DeltaParams&);
 int delta_out_launch(bool, const DeltaParams&, hipStream_t);
 int delta_decode_launch(bool, const DeltaParams&, hipStream_t);
 int attn_prep_launch(bool, const WindowAttnParams&, hipStream_t);
@@ -169,11 +170,16 @@ void delta_rule(Tensor proj, int64_t B, int64_t T, std::vector<int64_t> sizes, T
   Tensor cells;   // (outlives the launches below)
   if (p.nch > 0) {
     const int64_t n = B * p.nch * p.H;
-    cells = at::empty({n * 64 * (p.DP + (p.V + 15) / 16 * 16 + 64 + 2)}, opt);
+    const int64_t one = n * 64 * (p.DP + (p.V + 15) / 16 * 16 + 64 + 2), split = nxd::delta_chunk_split_floats(p);
+    cells = at::empty({one + split}, opt);
     p.cw = cells.data_ptr<float>();
     p.cp = p.cw + n * 64 * p.DP;
     p.ceg = p.cp + n * 64 * 64;
     p.cy = p.ceg + n * 64 * 2;
+    if (split) {
+      p.cs = cells.data_ptr<float>() + one;
+      p.cu = p.cs + n * ((p.V + 15) / 16) * 16 * p.DP;
+    }
     check_rc(nxd::delta_chunk_launch(f32, p, cur_stream()), "delta_chunk");
   } else {
     check_rc(nxd::delta_scan_launch(f32, p, cur_stream()), "delta_scan");

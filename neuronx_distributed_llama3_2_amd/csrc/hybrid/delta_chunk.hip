@@ -10,6 +10,8 @@
 //                         queries, the four 16 x 16 diagonal blocks of I + A inverted by substitution,
 //                         the rest by block substitution with the right-hand sides in registers;
 //   delta_chunk_scan    : the chunks of one head one after another for 16 columns of the state.
+//   delta_chunk_state, delta_chunk_out : the same in two launches, the chain of the states and then all outputs, where few columns leave CUs
+//                         idle or the keys are long (delta_chunk_split_floats).
 //
 // Everything is fp32 (v_mfma_f32_16x16x4_f32); the sums of log decays are formed in fp64, because the
 // differences of large sums are what is exponentiated.
@@ -20,6 +22,9 @@
 // elements of row l % 16.  Everything the scan reads is stored block by block in the order of its lanes
 // (1 KiB a block, element ((l / 16) 16 + l % 16) 4 + i): a block is one contiguous load.
 #include "delta_rule.h"
+
+#include <algorithm>
+#include <type_traits>
 
 namespace nxd {
 namespace hybrid {
@@ -292,6 +297,202 @@ __global__ void __launch_bounds__(512, 2) delta_chunk_scan_kernel(DeltaParams p)
   if (v0 == 0 && h == 0) ring_write<T>(p, b, slot, p0, len, tid, 512);
 }
 
+// The scan in two launches, for few columns in all: what a chunk's columns need of the chunk before is the state alone, so the chain has U and the state
+// only, and the outputs follow for all chunks side by side.  The sums are those of the kernel above, in its order.
+//
+// The chain.  Waves 0-3 compute U of 16 tokens each, all eight the state's blocks; the other four have nothing in a wave's way meanwhile.  Leaves the state each
+// chunk starts from and U.
+template <typename T, int NB>
+__global__ void __launch_bounds__(512, 2) delta_chunk_state_kernel(DeltaParams p) {
+  constexpr int DP = NB * 16, TPW = (NB + 7) / 8;
+  __shared__ __attribute__((aligned(16))) f32x4_t ss[NB][64], ud[4][64];
+  const int tid = threadIdx.x, lane = tid & 63, w8 = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lq = lane >> 4;
+  const int w = w8 & 3;
+  const int bh = blockIdx.x % (p.B * p.H), ct = blockIdx.x / (p.B * p.H), v0 = ct * 16;   // a head's columns on one XCD
+  const int b = bh / p.H, h = bh % p.H, H = p.H, G = p.G, V = p.V, g = h / (H / G), nv = (V + 15) / 16;
+  const int len = p.lens ? min(p.lens[b], p.T) : p.T;
+  if (len <= 0) return;
+  const int slot = slot_of(p.slots, b, p.nslots);
+  const int64_t p0 = pos_of(p.pos, p.pos_stride, b);
+  const int v = v0 + lr;
+  const bool vok = v < V;
+  float* state = p.state + (((int64_t)slot * H + h) * V + min(v, V - 1)) * DP;
+  f32x4_t S[TPW];
+#pragma unroll
+  for (int i = 0; i < TPW; ++i) {
+    const int rt = w8 + 8 * i;
+    S[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    if (rt < NB) {
+      if (p0 > 0) S[i] = ld4(state + rt * 16 + 4 * lq);
+      ss[rt][lane] = S[i];
+    }
+  }
+  const int nch = (len + CH - 1) / CH;
+  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+  // the next chunk's operands to load, and where the present one's state and U go
+  const int64_t cell = (int64_t)b * p.nch * H + h, qkcell = (int64_t)b * p.nch * G + g;
+  const float* pw = p.cw + cell * CH * DP + w * (NB * 256);
+  const float* py = p.cy + (cell * nv + ct) * 1024 + w * 256;
+  const float *pe = p.ceg + cell * (2 * CH), *pc = pe;
+  const float* pk = p.kn + qkcell * CH * DP;
+  float* pu = p.cu + (cell * nv + ct) * 1024 + w * 256;
+  float* ps = p.cs + (cell * nv + ct) * (NB * 256) + w8 * 256;
+  const int64_t sw = (int64_t)H * CH * DP, sy = (int64_t)H * nv * 1024, sk = (int64_t)G * CH * DP, st = (int64_t)H * nv * (NB * 256);
+  const auto loop = [&](auto uwave) __attribute__((always_inline)) {
+    constexpr bool U = decltype(uwave)::value;
+    // one chunk's operands: the own rows of W, of Y and of e^(G_C - G), K^T for the own state blocks and e^(G_C)
+    struct Ops {
+      f32x4_t rowf[U ? NB : 1], kf[TPW][4], y, eg;
+      float ec;
+    };
+    Ops set[2];
+    // Of the chunk's own set, W goes out for the next chunk but one as soon as it has been used; of the other set, K^T for the next one: neither stands
+    // between the last product of a chunk and its barrier.  (Past the last chunk the last one is read again: the number of loads in flight stays known.)
+    auto fetch_w = [&](Ops& o, int c) __attribute__((always_inline)) {
+      if (U) {
+#pragma unroll
+        for (int kb = 0; kb < NB; ++kb) o.rowf[U ? kb : 0] = ld4(pw + kb * 256 + lane * 4);
+        o.y = ld4(py + lane * 4);
+        o.eg = ld4(pe + CH + 16 * w + 4 * lq);
+        if (c + 1 < nch) pw += sw, py += sy, pe += H * (2 * CH);
+      }
+    };
+    auto fetch_k = [&](Ops& o, int c) __attribute__((always_inline)) {
+#pragma unroll
+      for (int j = 0; j < TPW; ++j)
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) o.kf[j][kb] = ld4(pk + ((8 * j + 8 <= NB ? w8 + 8 * j : min(w8 + 8 * j, NB - 1)) * 4 + kb) * 256 + lane * 4);
+      o.ec = pc[CH - 1];
+      if (c + 1 < nch) pk += sk, pc += H * (2 * CH);
+    };
+    fetch_w(set[0], 0);
+    fetch_k(set[0], 0);
+    asm volatile("" ::: "memory");   // (not interleaved: the loop's waits count on the order)
+    fetch_w(set[1], 1);
+    lds_barrier();
+    auto chunk = [&](int c, Ops& o, Ops& other) __attribute__((always_inline)) {
+      f32x4_t sb[U ? NB : 1];
+      if (U) {
+#pragma unroll
+        for (int kb = 0; kb < NB; ++kb) sb[U ? kb : 0] = ss[kb][lane];
+      }
+      __builtin_amdgcn_sched_barrier(0);   // all reads in flight before the first product
+      fetch_k(other, c + 1);
+      if (U) {
+        f32x4_t a0 = zero, a1 = zero;
+#pragma unroll
+        for (int kb = 0; kb < NB; kb += 2) {   // NB is even
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            a0 = __builtin_amdgcn_mfma_f32_16x16x4f32(o.rowf[U ? kb : 0][i], sb[U ? kb : 0][i], a0, 0, 0, 0);
+            a1 = __builtin_amdgcn_mfma_f32_16x16x4f32(o.rowf[U ? kb + 1 : 0][i], sb[U ? kb + 1 : 0][i], a1, 0, 0, 0);
+          }
+        }
+        f32x4_t r = a0 + a1;   // W S
+        r = o.y - r;
+        ud[w][lane] = r * o.eg;
+        st4(pu + lane * 4, r);
+      }
+#pragma unroll
+      for (int j = 0; j < TPW; ++j)
+        if (8 * j + 8 <= NB || w8 + 8 * j < NB) st4(ps + 8 * j * 256 + lane * 4, S[j]);
+      pu += sy, ps += st;
+      lds_barrier();
+      f32x4_t ub[4];
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb) ub[kb] = ud[kb][lane];
+      __builtin_amdgcn_sched_barrier(0);
+      fetch_w(o, c + 2);
+#pragma unroll
+      for (int j = 0; j < TPW; ++j) {
+        if (8 * j + 8 <= NB || w8 + 8 * j < NB) {
+          f32x4_t x = S[j] * o.ec, y = zero;
+#pragma unroll
+          for (int kb = 0; kb < 4; kb += 2) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              x = __builtin_amdgcn_mfma_f32_16x16x4f32(o.kf[j][kb][i], ub[kb][i], x, 0, 0, 0);
+              y = __builtin_amdgcn_mfma_f32_16x16x4f32(o.kf[j][kb + 1][i], ub[kb + 1][i], y, 0, 0, 0);
+            }
+          }
+          S[j] = x + y;
+          ss[w8 + 8 * j][lane] = S[j];
+        }
+      }
+      lds_barrier();
+    };
+    int c = 0;
+    for (; c + 1 < nch; c += 2) {
+      chunk(c, set[0], set[1]);
+      chunk(c + 1, set[1], set[0]);
+    }
+    if (c < nch) chunk(c, set[0], set[1]);
+  };
+  if (w8 < 4) loop(std::true_type{});
+  else loop(std::false_type{});
+  if (vok) {
+#pragma unroll
+    for (int i = 0; i < TPW; ++i)
+      if (w8 + 8 * i < NB) st4(state + (w8 + 8 * i) * 16 + 4 * lq, S[i]);
+  }
+  if (v0 == 0 && h == 0) ring_write<T>(p, b, slot, p0, len, tid, 512);
+}
+
+// The outputs of a chunk and head, a wave 16 tokens: its rows of Q and of P stay in registers for `per` blocks of 16 columns.
+template <int NB>
+__global__ void __launch_bounds__(256, NB <= 8 ? 4 : 2) delta_chunk_out_kernel(DeltaParams p, int per) {
+  constexpr int DP = NB * 16;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lr = lane & 15, lq = lane >> 4;
+  const int nv = (p.V + 15) / 16, groups = (nv + per - 1) / per;
+  const int h = blockIdx.x / groups, ct0 = blockIdx.x % groups * per, c = blockIdx.y, b = blockIdx.z, H = p.H, G = p.G, V = p.V, g = h / (H / G);
+  const int len = p.lens ? min(p.lens[b], p.T) : p.T;
+  if (c * CH + 16 * w >= len) return;
+  const int64_t cell = ((int64_t)b * p.nch + c) * H + h, qkcell = (((int64_t)b * p.nch + c) * G + g) * CH * DP;
+  f32x4_t q[NB], pf[4];
+#pragma unroll
+  for (int kb = 0; kb < NB; ++kb) q[kb] = ld4(p.qn + qkcell + w * (NB * 256) + lane * 4 + kb * 256);
+#pragma unroll
+  for (int kb = 0; kb < 4; ++kb) pf[kb] = ld4(p.cp + cell * (CH * CH) + w * 1024 + lane * 4 + min(kb, w) * 256);   // (up to the diagonal)
+  const f32x4_t eg = ld4(p.ceg + cell * (2 * CH) + 16 * w + 4 * lq);
+  // (each register is loaded for the next block of columns as soon as it has been used)
+  const float *ps = p.cs + (cell * nv + ct0) * (NB * 256) + lane * 4, *pu = p.cu + (cell * nv + ct0) * 1024 + lane * 4;
+  f32x4_t s[NB], u[4];
+#pragma unroll
+  for (int kb = 0; kb < NB; ++kb) s[kb] = ld4(ps + kb * 256);
+#pragma unroll
+  for (int kb = 0; kb < 4; ++kb) u[kb] = ld4(pu + min(kb, w) * 256);
+  const int end = min(ct0 + per, nv);
+#pragma unroll 1
+  for (int ct = ct0; ct < end; ++ct) {
+    if (ct + 1 < end) ps += NB * 256, pu += 1024;
+    f32x4_t a0 = {0.f, 0.f, 0.f, 0.f}, a1 = a0;
+#pragma unroll
+    for (int kb = 0; kb < NB; kb += 2) {   // NB is even
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        a0 = __builtin_amdgcn_mfma_f32_16x16x4f32(q[kb][i], s[kb][i], a0, 0, 0, 0);
+        a1 = __builtin_amdgcn_mfma_f32_16x16x4f32(q[kb + 1][i], s[kb + 1][i], a1, 0, 0, 0);
+      }
+      s[kb] = ld4(ps + kb * 256);
+      s[kb + 1] = ld4(ps + (kb + 1) * 256);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    f32x4_t r = a0 + a1;   // Q S
+    r *= eg;
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) {
+      if (kb <= w) r = mma4(pf[kb], u[kb], r);
+      u[kb] = ld4(pu + min(kb, w) * 256);
+    }
+    const int v = ct * 16 + lr;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int t = c * CH + 16 * w + 4 * lq + i;
+      if (v < V && t < len) p.o[(((int64_t)b * p.T + t) * H + h) * V + v] = r[i];
+    }
+  }
+}
+
 template <int NB, int NW>
 static int run_prepare(const DeltaParams& p, hipStream_t s) {
   const size_t lds = (size_t)CH * (NB * 16 + 4 + CH + 4) * 4;
@@ -307,6 +508,13 @@ static int run_chunk(const DeltaParams& p, hipStream_t s) {
   const int rc = run_prepare<NB, NB <= 8 ? 16 : 8>(p, s);   // (16 waves have 128 registers each)
   if (rc) return rc;
   const int64_t grid = (int64_t)ceil_div(p.V, 16) * p.B * p.H;
+  if (p.cs) {
+    hipLaunchKernelGGL((delta_chunk_state_kernel<T, NB>), dim3((unsigned)grid), dim3(512), 0, s, p);
+    // all columns of a chunk and head in one workgroup if there are enough of these
+    const int nv = ceil_div(p.V, 16), per = ceil_div(nv, (int)std::min<int64_t>(ceil_div64(1024, (int64_t)p.B * p.H * p.nch), nv));
+    hipLaunchKernelGGL((delta_chunk_out_kernel<NB>), dim3((unsigned)(p.H * ceil_div(nv, per)), (unsigned)p.nch, (unsigned)p.B), dim3(256), 0, s, p, per);
+    return hipGetLastError() == hipSuccess ? 0 : 1;
+  }
   hipLaunchKernelGGL((delta_chunk_scan_kernel<T, NB>), dim3((unsigned)grid), dim3(512), 0, s, p);
   return hipGetLastError() == hipSuccess ? 0 : 1;
 }
@@ -327,6 +535,18 @@ static int dispatch_chunk(const DeltaParams& p, hipStream_t s) {
 }
 
 }  // namespace hybrid
+
+// Floats for the scan in two launches, 0: in one.  The chain's part of a chunk takes 1.7 us instead of 3 (16 heads of 128 x 128, 64 chunks: 193 us -> 107
+// and 43 for the outputs), the second launch and its 8 to 14 us of start are lost in longer runs, and with more columns than half of the CUs the
+// one launch fills the chip as well.  The whole operation, us, one launch / two: 16 heads of 128 x 128 (128 blocks of columns), 512 tokens 75 / 78,
+// 768 89 / 85, 1,024 104 / 99, 4,096 317 / 287; 8 of 64 x 64 (32 blocks) 256 tokens 35 / 34, 4,096 156 / 110; 4 of 128 x 128 256 tokens 44 / 43, 4,096 209 /
+// 145; 32 of 96 x 128 (256 blocks) 1,024 tokens 118 / 118, 4,096 392 / 406.  With keys of more than 128 the one launch has not the registers: 16 of 256 x 128, 128
+// tokens 96 / 80, 4,096 903 / 544, two sequences of up to 2,000 542 / 356.  Not past 1 GiB.
+int64_t delta_chunk_split_floats(const DeltaParams& p) {
+  const int64_t nv = ceil_div(p.V, 16), blocks = nv * p.B * p.H, floats = blocks * p.nch * 16 * (64 + p.DP);
+  const bool pays = p.DP > 128 ? blocks <= 256 && p.nch >= 2 : blocks <= 128 && p.nch >= (blocks <= 64 ? 4 : 12);
+  return pays && floats <= (int64_t{1} << 28) ? floats : 0;
+}
 
 int delta_chunk_launch(bool f32, const DeltaParams& p, hipStream_t s) {
   return f32 ? hybrid::dispatch_chunk<float>(p, s) : hybrid::dispatch_chunk<uint16_t>(p, s);

@@ -30,6 +30,7 @@ struct DeltaParams {
   int nch;                   // chunks per sequence (0: token by token)
   float *cw, *cy, *cp;       // W [cells, 64 DP], Y [cells, 64 V rounded up to 16], P [cells, 64 64]
   float* ceg;                // [cells, 2, 64] e^G, e^(G_C - G)
+  float *cs, *cu;            // (nullable: the scan in one launch) states [cells, 16-column blocks, 16 DP], U [cells, blocks, 16 64]
   void* y;                   // [B T, ldy] mixer output before its projection (activation type)
   int64_t ldy;
 };

@@ -1,0 +1,44 @@
+"""The chunked delta rule's scan in two launches (few blocks of columns) gives the bits of the one launch that a larger batch takes, and the oracle's
+numbers: ragged lengths, head sizes that fill no block, a state that goes on, keys of more than 128."""
+import pytest
+import torch
+
+from test_golitar_mechanisms import delta_case, delta_oracle, rel_err, run_delta
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("H,G,D,V,T", [(3, 3, 16, 24, 300), (16, 8, 128, 128, 769), (2, 1, 70, 33, 1000), (9, 9, 144, 16, 130), (4, 2, 256, 40, 250)])
+def test_two_launches(H, G, D, V, T):
+    from neuronx_distributed_llama3_2_amd import ops
+
+    where, taps = ("cuda", torch.float32, 5e-5), 4
+    n = -(-257 // (H * -(-V // 16))) + 1          # sequences of the batch that takes one launch
+    lens = [T, T - 67] + [1] * (n - 2)
+    case = delta_case(where, n, T, H, G, D, V, taps)
+    sz, proj, proj_o = case[:3]
+
+    def run(rows, pos0, state, ring):
+        t = torch.tensor
+        B = len(rows)
+        print(H, G, D, V, T, B, flush=True)
+        return ops.delta_rule(proj[rows].reshape(B * T, -1).contiguous(), B, T, sz, *(v.cuda() for v in case[3:]), 1e-5,
+                              t([pos0] * B, device="cuda"), t([lens[r] for r in rows], dtype=torch.int32, device="cuda"), None, state, ring).view(B, T, H, V)
+
+    def fresh(B):
+        g = torch.Generator().manual_seed(5)
+        return (torch.randn((1, H, V, sz.padded_dim), generator=g).expand(B, -1, -1, -1).contiguous().cuda(),
+                torch.zeros((B, taps, sz.channels), device="cuda"))
+
+    for pos0 in (0, 64):                           # a prompt, and one that goes on from a state
+        s_all, r_all = fresh(n)
+        y_all = run(list(range(n)), pos0, s_all, r_all)
+        for r in (0, 1):
+            s, ring = fresh(1)
+            y = run([r], pos0, s, ring)
+            assert torch.equal(y[0, :lens[r]], y_all[r, :lens[r]]) and torch.equal(s[0], s_all[r]) and torch.equal(ring[0], r_all[r])
+    state = torch.zeros((n, H, V, sz.padded_dim), device="cuda")
+    ring = torch.zeros((n, taps, sz.channels), device="cuda")
+    s, rg = state[:1].clone(), ring[:1].clone()
+    got = run([1], 0, s, rg)
+    assert rel_err(got[0, :lens[1]].reshape(lens[1], -1), delta_oracle(sz, proj_o[1, :lens[1]], *case[3:], 1e-5)) < where[2]
