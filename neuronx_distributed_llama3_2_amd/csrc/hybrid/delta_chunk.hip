@@ -93,18 +93,18 @@ __global__ void __launch_bounds__(64 * NW) delta_chunk_prepare_kernel(DeltaParam
       if (isq) a = ld4(p.qn + qkcell + ((bi * NB + kb) * 64 + lane) * 4);
       else a = ld4(kt + t * KS + 16 * kb + 4 * lq);
       const f32x4_t bb = ld4(kt + (16 * bj + lr) * KS + 16 * kb + 4 * lq);
-      if (kb & 1) acc2 = mma4(a, bb, acc2);
-      else acc = mma4(a, bb, acc);
+      if (kb & 1) acc2 = mma4(bb, a, acc2);   // (transposed: a lane has four columns of row lr, as both are stored)
+      else acc = mma4(bb, a, acc);
     }
     acc += acc2;
+    const int row = 16 * bi + lr, col = 16 * bj + 4 * lq;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int row = 16 * bi + 4 * lq + i, col = 16 * bj + lr;
-      const bool in = isq ? col <= row : col < row;
-      const float v = in ? acc[i] * expf((float)(gd[row] - gd[col])) : 0.f;
-      if (isq) P[((bi * 4 + bj) * 64 + (lr / 4) * 16 + 4 * lq + i) * 4 + (lr & 3)] = v;
-      else am[row * AS + col] = v * beta[row];
+      const bool in = isq ? col + i <= row : col + i < row;
+      acc[i] = in ? acc[i] * expf((float)(gd[row] - gd[col + i])) : 0.f;
+      if (!isq) acc[i] *= beta[row];
     }
+    st4(isq ? P + ((bi * 4 + bj) * 64 + lane) * 4 : am + row * AS + col, acc);
   }
   __syncthreads();
 
