@@ -20,6 +20,7 @@ int delta_prep_launch(bool, const DeltaParams&, hipStream_t);
 int delta_scan_launch(bool, const DeltaParams&, hipStream_t);
 int delta_chunk_launch(bool, const DeltaParams&, hipStream_t);
 int64_t delta_chunk_split_floats(const DeltaParams&);
+bool delta_chunk_norm(const DeltaParams&);
 int delta_out_launch(bool, const DeltaParams&, hipStream_t);
 int delta_decode_launch(bool, const DeltaParams&, hipStream_t);
 int attn_prep_launch(bool, const WindowAttnParams&, hipStream_t);
@@ -184,7 +185,7 @@ void delta_rule(Tensor proj, int64_t B, int64_t T, std::vector<int64_t> sizes, T
   } else {
     check_rc(nxd::delta_scan_launch(f32, p, cur_stream()), "delta_scan");
   }
-  check_rc(nxd::delta_out_launch(f32, p, cur_stream()), "delta_out");
+  if (!nxd::delta_chunk_norm(p)) check_rc(nxd::delta_out_launch(f32, p, cur_stream()), "delta_out");
 }
 
 // sizes (H, G, maps, D, V)

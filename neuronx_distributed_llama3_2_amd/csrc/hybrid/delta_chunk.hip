@@ -27,6 +27,7 @@
 #include <type_traits>
 
 namespace nxd {
+bool delta_chunk_norm(const DeltaParams& p);
 namespace hybrid {
 
 constexpr int CH = 64;   // tokens of a chunk
@@ -439,14 +440,27 @@ __global__ void __launch_bounds__(512, 2) delta_chunk_state_kernel(DeltaParams p
 }
 
 // The outputs of a chunk and head, a wave 16 tokens: its rows of Q and of P stay in registers for `per` blocks of 16 columns.
-template <int NB>
+// NORM (65 to 128 columns, all of them in the workgroup): the wave's outputs go through LDS of its own to the order of delta_out4_kernel's lanes and take the
+// gated norm there, the same sums in the same order: no fp32 outputs in memory, no launch after this one.
+template <typename T, int NB, bool NORM>
 __global__ void __launch_bounds__(256, NB <= 8 ? 4 : 2) delta_chunk_out_kernel(DeltaParams p, int per) {
-  constexpr int DP = NB * 16;
+  constexpr int DP = NB * 16, RS = 128 + 4;
+  __shared__ __attribute__((aligned(16))) float rows[NORM ? 4 : 1][NORM ? 16 * RS : 4];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lr = lane & 15, lq = lane >> 4;
   const int nv = (p.V + 15) / 16, groups = (nv + per - 1) / per;
   const int h = blockIdx.x / groups, ct0 = blockIdx.x % groups * per, c = blockIdx.y, b = blockIdx.z, H = p.H, G = p.G, V = p.V, g = h / (H / G);
   const int len = p.lens ? min(p.lens[b], p.T) : p.T;
-  if (c * CH + 16 * w >= len) return;
+  const int64_t m0 = (int64_t)b * p.T + c * CH + 16 * w;   // the wave's first row
+  const int nrow = p.T - c * CH - 16 * w, live = len - c * CH - 16 * w;
+  const int col = 4 * (lane & 31);
+  T* y = static_cast<T*>(p.y) + m0 * p.ldy + h * V + col;
+  if (live <= 0) {
+    if (NORM && col < V)   // padding: a defined value for the projection
+#pragma unroll
+      for (int i = 0; i < 16; i += 2)
+        if (i + (lane >> 5) < nrow) st4(y + (i + (lane >> 5)) * p.ldy, f32x4_t{0.f, 0.f, 0.f, 0.f});
+    return;
+  }
   const int64_t cell = ((int64_t)b * p.nch + c) * H + h, qkcell = (((int64_t)b * p.nch + c) * G + g) * CH * DP;
   f32x4_t q[NB], pf[4];
 #pragma unroll
@@ -487,8 +501,28 @@ __global__ void __launch_bounds__(256, NB <= 8 ? 4 : 2) delta_chunk_out_kernel(D
     const int v = ct * 16 + lr;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int t = c * CH + 16 * w + 4 * lq + i;
-      if (v < V && t < len) p.o[(((int64_t)b * p.T + t) * H + h) * V + v] = r[i];
+      if (NORM) rows[NORM ? w : 0][(4 * lq + i) * RS + v] = r[i];
+      else if (v < V && 4 * lq + i < live) p.o[((m0 + 4 * lq + i) * H + h) * V + v] = r[i];
+    }
+  }
+  if (NORM) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (the wave's own)
+    const T* gate = static_cast<const T*>(p.proj) + m0 * p.ldp + p.C + h * V + col;
+    const f32x4_t zero = {0.f, 0.f, 0.f, 0.f}, nw = col < V ? ld4(p.norm_w + col) : zero;
+    f32x4_t g[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int i = 2 * k + (lane >> 5);
+      g[k] = zero;
+      if (col < V && i < live) g[k] = ld4(gate + i * p.ldp);
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int i = 2 * k + (lane >> 5);
+      f32x4_t x = ld4(&rows[NORM ? w : 0][NORM ? i * RS + col : 0]);
+      if (!(col < V && i < live)) x = zero;
+      x = gated_norm4<32>(x, g[k], nw, V, p.eps);
+      if (col < V && i < nrow) st4(y + i * p.ldy, x);
     }
   }
 }
@@ -511,8 +545,14 @@ static int run_chunk(const DeltaParams& p, hipStream_t s) {
   if (p.cs) {
     hipLaunchKernelGGL((delta_chunk_state_kernel<T, NB>), dim3((unsigned)grid), dim3(512), 0, s, p);
     // all columns of a chunk and head in one workgroup if there are enough of these
-    const int nv = ceil_div(p.V, 16), per = ceil_div(nv, (int)std::min<int64_t>(ceil_div64(1024, (int64_t)p.B * p.H * p.nch), nv));
-    hipLaunchKernelGGL((delta_chunk_out_kernel<NB>), dim3((unsigned)(p.H * ceil_div(nv, per)), (unsigned)p.nch, (unsigned)p.B), dim3(256), 0, s, p, per);
+    const int nv = ceil_div(p.V, 16);
+    if constexpr (NB <= 8)
+      if (delta_chunk_norm(p)) {
+        hipLaunchKernelGGL((delta_chunk_out_kernel<T, NB, true>), dim3((unsigned)p.H, (unsigned)p.nch, (unsigned)p.B), dim3(256), 0, s, p, nv);
+        return hipGetLastError() == hipSuccess ? 0 : 1;
+      }
+    const int per = ceil_div(nv, (int)std::min<int64_t>(ceil_div64(1024, (int64_t)p.B * p.H * p.nch), nv));
+    hipLaunchKernelGGL((delta_chunk_out_kernel<float, NB, false>), dim3((unsigned)(p.H * ceil_div(nv, per)), (unsigned)p.nch, (unsigned)p.B), dim3(256), 0, s, p, per);
     return hipGetLastError() == hipSuccess ? 0 : 1;
   }
   hipLaunchKernelGGL((delta_chunk_scan_kernel<T, NB>), dim3((unsigned)grid), dim3(512), 0, s, p);
@@ -539,13 +579,21 @@ static int dispatch_chunk(const DeltaParams& p, hipStream_t s) {
 // Floats for the scan in two launches, 0: in one.  The chain's part of a chunk takes 1.7 us instead of 3 (16 heads of 128 x 128, 64 chunks: 193 us -> 107
 // and 43 for the outputs), the second launch and its 8 to 14 us of start are lost in longer runs, and with more columns than half of the CUs the
 // one launch fills the chip as well.  The whole operation, us, one launch / two: 16 heads of 128 x 128 (128 blocks of columns), 512 tokens 75 / 78,
-// 768 89 / 85, 1,024 104 / 99, 4,096 317 / 287; 8 of 64 x 64 (32 blocks) 256 tokens 35 / 34, 4,096 156 / 110; 4 of 128 x 128 256 tokens 44 / 43, 4,096 209 /
-// 145; 32 of 96 x 128 (256 blocks) 1,024 tokens 118 / 118, 4,096 392 / 406.  With keys of more than 128 the one launch has not the registers: 16 of 256 x 128, 128
+// 768 89 / 85, 1,024 104 / 94, 4,096 317 / 274; 8 of 64 x 64 (32 blocks) 256 tokens 35 / 34, 4,096 156 / 110; 4 of 128 x 128 256 tokens 44 / 43, 4,096 209 /
+// 141; 32 of 96 x 128 (256 blocks) 1,024 tokens 118 / 118, 4,096 392 / 406.  With keys of more than 128 the one launch has not the registers: 16 of 256 x 128, 128
 // tokens 96 / 80, 4,096 903 / 544, two sequences of up to 2,000 542 / 356.  Not past 1 GiB.
 int64_t delta_chunk_split_floats(const DeltaParams& p) {
   const int64_t nv = ceil_div(p.V, 16), blocks = nv * p.B * p.H, floats = blocks * p.nch * 16 * (64 + p.DP);
   const bool pays = p.DP > 128 ? blocks <= 256 && p.nch >= 2 : blocks <= 128 && p.nch >= (blocks <= 64 ? 4 : 12);
   return pays && floats <= (int64_t{1} << 28) ? floats : 0;
+}
+
+// Whether the launch of the outputs also norms them: the sizes that delta_out_launch gives 32 lanes a row, and workgroups for half of the CUs when each has all
+// columns.  The outputs' fp32 writes and reads are what it saves.  The whole operation, us, with the norm's own launch / without: 16 heads of 128 x 128, 1,024 tokens 98.2 /
+// 94.1, 2,048 150.9 / 145.5, 4,096 286 / 274, 8,192 605 / 575; 8 of 64 x 128 1,024 (128 workgroups) 60.8 / 60.5, 8,192 234 / 220; 4 of 128 x 72 2,048 (128) 90.3 / 90.3; 2 of 128 x
+// 128 4,096 (128) 136.3 / 133.5; 16 of 64 x 100 800 66.9 / 64.3.
+bool delta_chunk_norm(const DeltaParams& p) {
+  return p.cs && p.DP <= 128 && p.V > 64 && p.V <= 128 && !(p.V % 4 || p.C % 4 || p.ldp % 4 || p.ldy % 4) && (int64_t)p.B * p.H * p.nch >= 128;
 }
 
 int delta_chunk_launch(bool f32, const DeltaParams& p, hipStream_t s) {

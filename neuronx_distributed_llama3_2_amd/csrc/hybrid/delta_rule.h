@@ -48,5 +48,15 @@ __device__ __forceinline__ void ring_write(const DeltaParams& p, int b, int slot
   }
 }
 
+// the gated norm of four columns of a head's row, L lanes a row: y = x / rms(x) w silu(g)
+template <int L>
+__device__ __forceinline__ f32x4_t gated_norm4(f32x4_t x, f32x4_t g, f32x4_t w, int V, float eps) {
+  const float ss = sum_lanes<L>(x[0] * x[0] + x[1] * x[1] + x[2] * x[2] + x[3] * x[3]);
+  const float r = 1.f / sqrtf(ss / (float)V + eps);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) x[j] *= r * w[j] * siluf_(g[j]);
+  return x;
+}
+
 }  // namespace hybrid
 }  // namespace nxd

@@ -14,7 +14,7 @@
 //   delta_prep   : convolution, silu, unit norms, gates of all tokens of a step
 //   delta_scan   : the recurrence, token by token, from the cached state (8 lanes a state column)
 //                  (long runs of tokens: 64 at a time, delta_chunk.hip)
-//   delta_out    : the gated head norm
+//   delta_out    : the gated head norm (of long runs in few sequences: by delta_chunk.hip, with the outputs)
 //   delta_decode : all of it for one new token per sequence, one workgroup per (sequence, head)
 #include "hybrid.h"
 #include "delta_rule.h"
@@ -342,12 +342,8 @@ __global__ void __launch_bounds__(256) delta_out4_kernel(DeltaParams p) {
     g = ld4(static_cast<const T*>(p.proj) + m * p.ldp + p.C + h * V + v);
     w = ld4(p.norm_w + v);
   }
-  const float ss = sum_lanes<L>(x[0] * x[0] + x[1] * x[1] + x[2] * x[2] + x[3] * x[3]);
-  if (!in) return;
-  const float r = 1.f / sqrtf(ss / (float)V + p.eps);
-#pragma unroll
-  for (int j = 0; j < 4; ++j) x[j] *= r * w[j] * siluf_(g[j]);   // padding: zeros
-  st4(static_cast<T*>(p.y) + m * p.ldy + h * V + v, x);
+  x = gated_norm4<L>(x, g, w, V, p.eps);   // padding: zeros
+  if (in) st4(static_cast<T*>(p.y) + m * p.ldy + h * V + v, x);
 }
 
 // ---- one new token per sequence: a workgroup of NTH threads per (head, sequence)

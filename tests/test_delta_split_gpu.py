@@ -1,5 +1,6 @@
 """The chunked delta rule's scan in two launches (few blocks of columns) gives the bits of the one launch that a larger batch takes, and the oracle's
-numbers: ragged lengths, head sizes that fill no block, a state that goes on, keys of more than 128."""
+numbers: ragged lengths, head sizes that fill no block, a state that goes on, keys of more than 128,
+outputs normed where they are formed."""
 import pytest
 import torch
 
@@ -8,7 +9,8 @@ from test_golitar_mechanisms import delta_case, delta_oracle, rel_err, run_delta
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("H,G,D,V,T", [(3, 3, 16, 24, 300), (16, 8, 128, 128, 769), (2, 1, 70, 33, 1000), (9, 9, 144, 16, 130), (4, 2, 256, 40, 250)])
+@pytest.mark.parametrize("H,G,D,V,T", [(3, 3, 16, 24, 300), (16, 8, 128, 128, 769), (2, 1, 70, 33, 1000), (9, 9, 144, 16, 130), (4, 2, 256, 40, 250),
+                                       (16, 8, 32, 68, 2100), (16, 16, 128, 128, 2049)])   # (16 heads: the outputs' launch norms them)
 def test_two_launches(H, G, D, V, T):
     from neuronx_distributed_llama3_2_amd import ops
 
@@ -36,6 +38,7 @@ def test_two_launches(H, G, D, V, T):
         for r in (0, 1):
             s, ring = fresh(1)
             y = run([r], pos0, s, ring)
+            assert not y[0, lens[r]:].any() and not y_all[r, lens[r]:].any()
             assert torch.equal(y[0, :lens[r]], y_all[r, :lens[r]]) and torch.equal(s[0], s_all[r]) and torch.equal(ring[0], r_all[r])
     state = torch.zeros((n, H, V, sz.padded_dim), device="cuda")
     ring = torch.zeros((n, taps, sz.channels), device="cuda")
