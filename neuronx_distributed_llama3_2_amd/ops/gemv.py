@@ -38,15 +38,21 @@ def few_rows_pay(rows: int, weight_rows: int, K: int, fused: bool = False) -> bo
     an element-wise epilogue (SwiGLU, squared ReLU), which the library follows with a launch.
 
     Up to 8 rows always (the library's time is that of 16).  Up to K = 4,224 the kernel keeps the activations in registers:
-    9 to 16 rows take 0.42-1.01 of the library's time over 256 to 128,256 weight rows; 17 to 32 rows 0.43-1.04 up to K = 2,048,
-    beyond it 0.69-1.01 up to 4,096 weight rows and 24 rows (1.09 at 32) and 0.79-1.01 from 16,384 weight rows on, but 1.01-1.13
-    between (4,096 x 6,144 at 32: 16.9 us, library 15.6).  Longer reductions read them once per workgroup: 8,192 x
-    10,240 at 9 / 16 / 32 rows 33.9 / 40.1 / 56.4 us, library 34.8 / 35.6 / 37.4."""
+    9 to 16 rows take 0.42-1.01 of the library's time over 256 to 128,256 weight rows; 17 to 32 rows 0.43-1.04 up to K = 2,048.
+    Beyond it (K 2,304 to 4,096): up to 3,072 weight rows 0.39-0.95 at 17 to 32 rows (2,048 x 4,096 at 32 8.4 us, library 12-18);
+    4,096 0.54-0.94 up to 20 rows and 0.58-1.03 at 24, at 25 to 32 0.60-0.82 up to K = 3,072 and 0.98-1.09 at 4,096; from 12,288 on 0.74-0.98 up to
+    24 rows (0.83-1.02 at more from K = 3,072 on, 12,288 x 4,096 at 32 22.5 us, library 25.7; 0.92-1.12 at K = 2,304); between, 0.91-1.16
+    and mostly above 1 (at K = 2,304 0.52-1.30).  Longer reductions read them once per workgroup: 8,192 x 10,240 at 9 / 16 / 32 rows 33.9 /
+    40.1 / 56.4 us, library 34.8 / 35.6 / 37.4."""
     if rows <= 8:
         return True
     if K > 4224:
         return False
-    return rows <= 16 or K <= 2048 or fused or weight_rows >= 16384 or weight_rows <= 4096 and rows <= 24
+    if rows <= 16 or K <= 2048 or fused or weight_rows >= 16384:
+        return True
+    if weight_rows >= 12288:
+        return rows <= 24 or K >= 3072
+    return weight_rows <= (4096 if rows <= 24 or K <= 3072 else 3072)
 
 
 def skinny_linear(x: torch.Tensor, w: torch.Tensor, scale: Optional[torch.Tensor] = None,

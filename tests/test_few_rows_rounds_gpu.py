@@ -65,3 +65,16 @@ def test_single_tiles(M, N, K, int8):
 @pytest.mark.parametrize("M,N,K", [(4, 6 * 2048, 256), (16, 6 * 2048 + 8, 512), (13, 7 * 2048, 384), (30, 7 * 1024 + 24, 2176), (30, 6 * 1024, 2176)])
 def test_swiglu_rounds(M, N, K):
     _run(M, N, K, 2, True, False)
+
+
+# 25 to 32 rows of reductions past 2,048 (few and many weight rows) go to this kernel, between them to the library: in the op, either side of each line
+@pytest.mark.parametrize("M,N,K,few", [(25, 8, 2056, True), (32, 3072, 4224, True), (32, 3073, 3080, False), (32, 4096, 3072, True), (25, 4097, 3072, False),
+                                       (24, 12288, 2056, True), (25, 12288, 3064, False), (32, 12288, 3072, True), (17, 12287, 4096, False), (32, 3072, 4232, False)])
+def test_long_reductions_by_rows_of_weights(M, N, K, few):
+    from neuronx_distributed_llama3_2_amd.ops.gemv import few_rows_pay, skinny_linear
+
+    assert few_rows_pay(M, N, K) is few
+    gen = torch.Generator(device="cuda").manual_seed(M + 3 * N + 5 * K)
+    w, x = (torch.randn(N, K, generator=gen, device="cuda") * 0.02).bfloat16(), torch.randn(M, K, generator=gen, device="cuda").bfloat16()
+    z = x.double() @ w.double().t()
+    assert float((skinny_linear(x, w).double() - z).norm() / z.norm()) < TOL
