@@ -56,7 +56,8 @@ def act_pays(rows: int, weight_rows: int, K: int) -> bool:
     results each) and a reduction that the pass is not small beside.  us, two launches / one, weights from memory: SwiGLU of 8,192
     columns, reduction 2,048: 512 rows 41 / 45, 768 56 / 57, 1,024 73 / 62, 2,304 150 / 147, 4,096 245 / 231; of 14,336, 4,096: 256 rows 80 / 85,
     512 122 / 108, 1,792 385 / 350, 4,096 706 / 708; of 28,672, 8,192: 2,304 rows 1,555 / 1,599; squared ReLU of 12,288, 2,048: 768 rows 46 /
-    51, 1,024 62 / 55, 4,096 189 / 172."""
+    51, 1,024 62 / 55, 4,096 189 / 172.  Long prompts stay with the one launch: SwiGLU of 8,192, 2,048 at 8,192 / 16,384 rows 448 / 435, 894 / 882; 14,336, 4,096 at 8,192
+    / 12,288 / 16,384 1,360 / 1,354, 2,013 / 2,054, 2,714 / 2,700; 11,008, 4,096 at 4,096 / 16,384 672 / 550, 2,208 / 2,088; squared ReLU of 12,288, 2,048 at 16,384 693 / 632."""
     return K % 32 == 0 and K <= 4096 and rows * weight_rows >= 192 * 256 * 256
 
 
