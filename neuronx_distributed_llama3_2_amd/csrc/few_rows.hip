@@ -280,9 +280,12 @@ struct Finish {
 };
 
 template <int EPI, bool NORM, bool XI, int R, int MT, bool I8, int NW, int CW, int D, bool SPLIT, bool HALF>
-__global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) kernel(FewRowsParams p, int tiles, int per) {
+__global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) kernel(FewRowsParams p, int tiles, int per, int step) {
   using S = Shape<R, MT, I8, NW, CW, D>;
   extern __shared__ __attribute__((aligned(16))) char smem[];
+  // (what the first loads need, asked for at once: asked for where it is used, it came in two or three trips one after the other: 1024 x 4096 at 4 rows 4.3
+  // -> 4.2 us, 8192 x 4096 14.4 -> 14.0)
+  asm volatile("" ::"s"(p.x), "s"(p.w), "s"(p.ldx), "s"(p.ldw), "s"(p.M), "s"(p.N), "s"(p.K), "s"(tiles), "s"(per), "s"(step));
   f32x4_t* part = reinterpret_cast<f32x4_t*>(smem + S::RING);       // [NW][MT][64]
   float* sq = reinterpret_cast<float*>(smem + S::RING + S::PART);   // [NW][16 MT]
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -291,8 +294,7 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
   static_assert(!SPLIT || (CW > 0 && !NORM), "split reductions hold their activations and need no norm");
   // its tiles: per of them next to each other, or (1) one of each round
   const int group = SPLIT ? blockIdx.x / p.splits : blockIdx.x, tile0 = group * per;
-  const int step = per > 1 ? 1 : SPLIT ? gridDim.x / p.splits : gridDim.x;
-  if (per > 1) tiles = min(tiles, tile0 + per);
+  tiles = min(tiles, per > 1 ? tile0 + per : tiles);
 
   // SPLIT: all waves of a workgroup share the tiles of which its part was the last to come
   auto finish_last = [&]() {
@@ -682,7 +684,7 @@ static int launch(FewRowsParams p, hipStream_t s, int splits = 1) {
   // 13.3 / 13.5, 8192 x 4096 25.1 / 26.2, 14336 x 4096 40.4 / 39.3, 28 rows 29.1 / 27.0 and 47.7 / 45.9; rotary 6144 x 4096 13.3 / 13.9; streamed 8192 x 8192
   // 26.7 / 30.5; in parts 8192 x 8192 29.6 / 33.3, 4096 x 14336 24.3 / 25.3, but 2048 x 12288 (long parts, four rounds) 14.1 / 13.8, 28 rows 15.7 / 15.1
   const int next = (SPLIT && (CW < 2 || rounds > 4)) || CW == 0 || EPI == FEW_ROPE_KV || (EPI == FEW_GLU && rounds < 7) ? 1 : (int)rounds;
-  hipLaunchKernelGGL(f, dim3((unsigned)(groups * splits), (unsigned)(SPLIT ? 1 : HALF ? 2 : ceil_div(p.M, 16 * MT))), dim3((NW + S::FW) * 64), lds, s, p, (int)tiles, next);
+  hipLaunchKernelGGL(f, dim3((unsigned)(groups * splits), (unsigned)(SPLIT ? 1 : HALF ? 2 : ceil_div(p.M, 16 * MT))), dim3((NW + S::FW) * 64), lds, s, p, (int)tiles, next, next > 1 ? 1 : (int)groups);
   return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
