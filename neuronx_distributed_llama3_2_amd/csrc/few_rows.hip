@@ -279,7 +279,11 @@ struct Finish {
   }
 };
 
-template <int EPI, bool NORM, bool XI, int R, int MT, bool I8, int NW, int CW, int D, bool SPLIT, bool HALF>
+// FULL: all that is loaded ahead is used: with CW > 0 a wave has D stages or more, with CW = 0 a workgroup has one tile and every wave whole rounds of D
+// stages.  Then loads need no branch and are counted (above); else loads under a branch, which are not, are faster than some that nothing uses.  us, all
+// counted and both ways in one kernel / apart: 32000 x 512 at 8 rows 9.6 / 9.0, 8192 x 512 at 16 5.6 / 4.9, 1024 x 1536 at 8 3.8 / 3.7, int8 8192 x
+// 3072 at 6 11.2 / 9.7, with a norm 3072 x 1024 at 8 4.6 / 4.3
+template <int EPI, bool NORM, bool XI, int R, int MT, bool I8, int NW, int CW, int D, bool SPLIT, bool HALF, bool FULL>
 __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) kernel(FewRowsParams p, int tiles, int per, int step) {
   using S = Shape<R, MT, I8, NW, CW, D>;
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -441,8 +445,8 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
       }
     }
     const int chunk = wc + order(ic) * NW;
-    // (past the last stage; a part may have one only, and a range of nothing is not read: 1024 x 8192 at 16 rows 9.3 -> 8.9 us)
-    const __amdgpu_buffer_rsrc_t wbase = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.w), 0, SPLIT && it >= tiles ? 0 : -1, 0x00020000);
+    // (past the last stage, of a last workgroup or part: a range of nothing is not read)
+    const __amdgpu_buffer_rsrc_t wbase = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.w), 0, CW > 0 && (it >= tiles || cw <= 0) ? 0 : -1, 0x00020000);
 #pragma unroll
     for (int j = 0; j < S::DMAS; ++j) {
       int seg;   // the piece of the row that goes to this lane's place
@@ -530,13 +534,18 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
     for (int t = 0; t < MT; ++t) {
       float v = ss[t];
       v = lanes_add<32>(lanes_add<16>(v));
-      if (q == 0) lds_write(lds_at(sq + w * 16 * MT + 16 * t + c), v);
+      if (q != 0) continue;
+      if constexpr (FULL) lds_write(lds_at(sq + w * 16 * MT + 16 * t + c), v);
+      else sq[w * 16 * MT + 16 * t + c] = v;
     }
   };
   auto publish = [&]() {
     meet();
 #pragma unroll
-    for (int t = 0; t < MT; ++t) lds_write_sum(lds_at(part + (w * MT + t) * 64 + lane), acc[t]);
+    for (int t = 0; t < MT; ++t) {
+      if constexpr (FULL) lds_write_sum(lds_at(part + (w * MT + t) * 64 + lane), acc[t]);
+      else part[(w * MT + t) * 64 + lane] = acc[t];
+    }
     meet();
   };
 
@@ -545,10 +554,13 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
     const u32x4_t gl = load_g();
 #pragma unroll
     for (int i = 0; i < CW; ++i) load_x(x[i], min(wc + i * NW, nck - 1));   // (chunks past the last one are not used)
-    // the first D stages, without a branch (past the last one: a piece that is there, not used), or the compiler would wait for them with
-    // the activations
+    // FULL: the first D stages, without a branch, or the compiler would wait for them with the activations
+    constexpr std::bool_constant<FULL> counted;
 #pragma unroll
-    for (int i = 0; i < D; ++i) start(std::true_type{});
+    for (int i = 0; i < D; ++i) {
+      if constexpr (FULL) start(counted);
+      else issue(counted);
+    }
     keep_g(gl);
 #pragma unroll
     for (int i = 0; i < CW; ++i) {
@@ -564,8 +576,9 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
         if (i >= cw) break;
         u32x4_t wf[I8 ? 2 : 4];
         wait_stages<S::DMAS, D>(ahead - 1);
-        take(wf);
-        issue(std::true_type{});
+        if constexpr (FULL) take(wf);
+        else look(wf);
+        issue(counted);
         multiply(wf, x[i]);
       }
       publish();
@@ -573,14 +586,11 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (pieces that are not used)
     if constexpr (SPLIT) finish_last();
   } else {
-    constexpr int XL = 4 * MT;   // loads of a stage beside the weights'
-    u32x4_t x[D][MT][4], g[4];
-    const u32x4_t gl = load_g();
-    auto fetch = [&](u32x4_t (&xv)[MT][4]) {
-      if (it < tiles && cw > 0) load_x(xv, wc + order(ic) * NW);
-      issue(std::false_type{});
-    };
-    if (tile0 + step >= tiles && cw > 0 && cw % D == 0) {   // one tile: no branch between the loads, so that the compiler knows what is under way
+    constexpr int XL = 4 * MT + (NORM && !FULL ? 4 : 0);   // loads of a stage beside the weights'
+    u32x4_t x[D][MT][4];
+    if constexpr (FULL) {   // no branch between the loads, so that the compiler knows what is under way
+      const u32x4_t gl = load_g();
+      u32x4_t g[4];
       clear();
       auto get = [&](int u) {
         load_x(x[u], wc + order(ic) * NW);
@@ -609,33 +619,41 @@ __global__ void __launch_bounds__((NW + Shape<R, MT, I8, NW, CW, D>::FW) * 64) k
       for (int u = 0; u < D; ++u) use(u, i + u, D - 1 - u);
       squares();
       publish();
-      return;
-    }
+    } else {
+      u32x4_t g[NORM ? D : 1][4];
+      auto fetch = [&](u32x4_t (&xv)[MT][4], u32x4_t (&gv)[4]) {
+        if (it < tiles && cw > 0) {
+          const int chunk = wc + order(ic) * NW;
+          load_x(xv, chunk);
 #pragma unroll
-    for (int i = 0; i < D; ++i) fetch(x[i]);
-    keep_g(gl);
-    int tile = tile0, i = 0;
-    bool first = true;
-    clear();
-    if (cw <= 0) squares();
-    for (; cw <= 0 && tile < tiles; tile += step) publish();
-    while (tile < tiles) {
+          for (int f = 0; NORM && f < 4; ++f) gv[f] = *reinterpret_cast<const u32x4_t*>(p.norm_w + min(chunk * KC + kof(f), p.K - 8));
+        }
+        issue(std::false_type{});
+      };
 #pragma unroll
-      for (int u = 0; u < D; ++u) {
-        if (tile >= tiles) break;
-        u32x4_t wf[I8 ? 2 : 4];
-        wait_stages<XL, D>(ahead - 1);   // (of XL + DMAS loads a stage: the stage has come, and the next one's x nearly)
-        look(wf);
-        read_g(g, order(i));
-        ready_x(x[u], g, wc + order(i) * NW, first);
-        multiply(wf, x[u]);
-        fetch(x[u]);
-        if (++i == cw) {
-          if (first) squares();
-          first = false;
-          publish();
-          clear();
-          i = 0, tile += step;
+      for (int i = 0; i < D; ++i) fetch(x[i], g[NORM ? i : 0]);
+      int tile = tile0, i = 0;
+      bool first = true;
+      clear();
+      if (cw <= 0) squares();
+      for (; cw <= 0 && tile < tiles; tile += step) publish();
+      while (tile < tiles) {
+#pragma unroll
+        for (int u = 0; u < D; ++u) {
+          if (tile >= tiles) break;
+          u32x4_t wf[I8 ? 2 : 4];
+          wait_stages<XL, D>(ahead - 1);   // (of XL + DMAS loads a stage: the stage has come, and the next one's x nearly)
+          look(wf);
+          ready_x(x[u], g[NORM ? u : 0], wc + order(i) * NW, first);
+          multiply(wf, x[u]);
+          fetch(x[u], g[NORM ? u : 0]);
+          if (++i == cw) {
+            if (first) squares();
+            first = false;
+            publish();
+            clear();
+            i = 0, tile += step;
+          }
         }
       }
     }
@@ -651,7 +669,7 @@ static int64_t tiles_of(const FewRowsParams& p) {
 
 
 // HALF: two workgroups for the halves of the activation rows, one a CU
-template <int EPI, bool NORM, bool XI, int R, int MT, bool I8, int NW, int CW, int D, bool SPLIT = false, bool HALF = false>
+template <int EPI, bool NORM, bool XI, int R, int MT, bool I8, int NW, int CW, int D, bool SPLIT = false, bool HALF = false, bool FULL = false>
 static int launch(FewRowsParams p, hipStream_t s, int splits = 1) {
   using S = Shape<R, MT, I8, NW, CW, D>;
   const int nck = ceil_div(p.K, KC);
@@ -659,7 +677,7 @@ static int launch(FewRowsParams p, hipStream_t s, int splits = 1) {
   constexpr size_t lds = S::RING + S::PART + S::SQ + (NORM ? S::G : 0);
   static_assert(lds <= 160 * 1024, "LDS of a workgroup");
   const int64_t tiles = tiles_of<EPI, R>(p);
-  auto* f = &kernel<EPI, NORM, XI, R, MT, I8, NW, CW, D, SPLIT, HALF>;
+  auto* f = &kernel<EPI, NORM, XI, R, MT, I8, NW, CW, D, SPLIT, HALF, FULL>;
   // workgroups of a CU; the limit on LDS and what follows from it are set once on each device
   static std::atomic<int> known[16];
   int dev = 0, per = 0;
@@ -671,7 +689,10 @@ static int launch(FewRowsParams p, hipStream_t s, int splits = 1) {
     if (dev < 16) known[dev].store(per, std::memory_order_relaxed);
   }
   const int64_t room = (HALF ? 128 : 256 * (int64_t)per) / splits;   // workgroups side by side along the rows
-  const int64_t rounds = ceil_div64(tiles, room < 1 ? 1 : room);
+  const int64_t rounds = FULL && CW == 0 ? 1 : ceil_div64(tiles, room < 1 ? 1 : room);
+  if constexpr (!FULL)
+    if (CW > 0 ? ceil_div(nck, splits) / NW * rounds >= D : rounds == 1 && nck % (NW * D) == 0)
+      return launch<EPI, NORM, XI, R, MT, I8, NW, CW, D, SPLIT, HALF, true>(p, s, splits);
   int64_t groups = ceil_div64(tiles, rounds);
   // the two that read the same weights on one XCD (11008 x 4096 with SwiGLU, 17 rows, 126 groups 57.6 us, 128 35.2)
   if (HALF) groups = (groups + 7) / 8 * 8;
@@ -689,8 +710,8 @@ static int launch(FewRowsParams p, hipStream_t s, int splits = 1) {
 }
 
 // Which geometry (times in us at 4 / 16 / 32 rows, bf16, weights from memory; the choices were measured before the waits at the top of this file, what they
-// take now: 16384 x 2048 with norm and SwiGLU 12.7 / 13.3 / 15.3, 128256 x 2048 79.5 / 85.9 / 91.7, 3072 x 2048 rotary 6.0 / 6.7 / 7.7, 28672 x 4096 at 5 /
-// 13 / 28 rows 37.5 / 38.4 / 43.3, 2048 x 8192 8.1 / 10.8 / 12.2, 4096 x 4096 at 5 / 13 / 28 7.8 / 8.5 / 11.4):
+// take now: 16384 x 2048 with norm and SwiGLU 12.8 / 13.2 / 15.0, 128256 x 2048 79.7 / 82.0 / 86.6, 3072 x 2048 rotary 5.8 / 6.2 / 7.9, 28672 x 4096 36.7 / - /
+// 44.1, 2048 x 8192 9.0 / 10.4 / 11.9, 4096 x 4096 at 4 / 13 rows 8.3 / 9.1):
 //   K <= 2048: activations stay in 8 waves' registers and a workgroup goes over the tiles of 16 rows: 16384 x 2048 with
 //     norm and SwiGLU 14.1 / 15.0 / 16.9 (activations streamed 15.8 / 19.0 / 71; int8 11.6 / 12.4 / 14.8),
 //     128256 x 2048 86 / 92 / 98 (int8 46 / 50 / 54).

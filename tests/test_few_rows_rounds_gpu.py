@@ -78,3 +78,24 @@ def test_long_reductions_by_rows_of_weights(M, N, K, few):
     w, x = (torch.randn(N, K, generator=gen, device="cuda") * 0.02).bfloat16(), torch.randn(M, K, generator=gen, device="cuda").bfloat16()
     z = x.double() @ w.double().t()
     assert float((skinny_linear(x, w).double() - z).norm() / z.norm()) < TOL
+
+
+# reductions in parts: a wave with as many stages as are loaded ahead and with fewer, a last part with fewer chunks, parts without a chunk for every wave
+@pytest.mark.parametrize("int8", [False, True])
+@pytest.mark.parametrize("M,N,K", [(13, 1024, 8192), (13, 2048, 8192), (16, 40, 4352), (15, 2048, 5632), (32, 1000, 11008), (9, 3072, 14336)])
+def test_parts(M, N, K, int8):
+    gen = torch.Generator(device="cuda").manual_seed(M + 3 * N + 5 * K)
+    if int8:
+        w = torch.randint(-128, 128, (N, K), generator=gen, device="cuda", dtype=torch.int8)
+        s = torch.rand(N, generator=gen, device="cuda") * 3e-4 + 1e-5
+        exact = w.double() * s.double()[:, None]
+    else:
+        w, s = (torch.randn(N, K, generator=gen, device="cuda") * 0.02).bfloat16(), None
+        exact = w.double()
+    x, y0 = (torch.randn(M, n, generator=gen, device="cuda").bfloat16() for n in (K, N))
+    z = y0.double() + x.double() @ exact.t()
+    tickets = torch.zeros(1024, dtype=torch.int32, device="cuda")
+    for _ in range(3):
+        y = y0.clone()
+        ops.ext().dgemv(1, x, None, 0.0, w, y, 0, 0, 0, None, None, None, 1, None, None, None, wscale=s, tickets=tickets)
+        assert float((y.double() - z).norm() / z.norm()) < TOL and not tickets.any()
