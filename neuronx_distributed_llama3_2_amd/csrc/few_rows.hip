@@ -699,12 +699,16 @@ static int launch(FewRowsParams p, hipStream_t s, int splits = 1) {
   if (SPLIT && rounds > 64) return -2;   // (a lane for every tile's ticket)
   p.splits = splits;
   if (HALF) p.half = (p.M + 1) / 2;
-  // Tiles next to each other (a workgroup reads one stretch of the weights, and a line of the output is written on one XCD), but not where the rows
-  // of a tile lie in two or three places, unless there are many tiles, nor parts of rows.  One of each round / next to each other, us: 16 rows,
-  // 16384 x 2048 13.6 / 12.3, 32000 x 2048 23.5 / 22.1, 128256 x 2048 88.9 / 85.9, 128256 x 4096 167 / 159 (28 rows 26.3 / 23.3 for 32000 x 2048); SwiGLU 8192 x 2048
-  // 13.3 / 13.5, 8192 x 4096 25.1 / 26.2, 14336 x 4096 40.4 / 39.3, 28 rows 29.1 / 27.0 and 47.7 / 45.9; rotary 6144 x 4096 13.3 / 13.9; streamed 8192 x 8192
-  // 26.7 / 30.5; in parts 8192 x 8192 29.6 / 33.3, 4096 x 14336 24.3 / 25.3, but 2048 x 12288 (long parts, four rounds) 14.1 / 13.8, 28 rows 15.7 / 15.1
-  const int next = (SPLIT && (CW < 2 || rounds > 4)) || CW == 0 || EPI == FEW_ROPE_KV || (EPI == FEW_GLU && rounds < 7) ? 1 : (int)rounds;
+  // Tiles next to each other (a workgroup reads one stretch of the weights, and a line of the output is written on one XCD) where rows lie a power of
+  // two apart, but not where the rows of a tile lie in two or three places, unless there are many tiles, nor parts of rows.  One of each round / next to
+  // each other, us: 16 rows, 16384 x 2048 13.6 / 12.3, 32000 x 2048 23.5 / 22.1, 128256 x 2048 88.9 / 85.9, 128256 x 4096 167 / 159 (28 rows 26.3 / 23.3 for
+  // 32000 x 2048); SwiGLU 8192 x 2048 13.3 / 13.5, 11008 x 2048 16.2 / 16.7, 8192 x 4096 25.1 / 26.2, 10240 x 4096 28.1 / 27.1, 14336 x 4096 40.4 / 39.3, 28 rows
+  // 29.1 / 27.0 and 47.7 / 45.9; rotary 6144 x 4096 13.3 / 13.9; streamed 8192 x 8192 26.7 / 30.5; in parts 8192 x 8192 29.6 / 33.3, 4096 x 14336 24.3 / 25.3, but
+  // 2048 x 12288 (long parts, four rounds) 14.1 / 13.8, 28 rows 15.7 / 15.1; rows no power of two apart, up to 16 rows 16384 x 3072 18.1 / 18.5, 32000 x 3072 31.8 / 32.5,
+  // 32000 x 1536 17.5 / 17.8; few rounds of bf16 tiles of 11 waves 8192 x 4096 13.3 / 14.1, 16384 x 4096 23.0 / 23.5 (int8 at 32 rows 20.8 / 19.3)
+  const bool pow2 = (p.ldw & (p.ldw - 1)) == 0;
+  const int next = (SPLIT && (CW < 2 || rounds > 4)) || CW == 0 || EPI == FEW_ROPE_KV || (EPI == FEW_GLU && rounds < 7) ||
+                   (!SPLIT && (!pow2 || (EPI != FEW_GLU && !I8 && CW > 2 && rounds <= 4))) ? 1 : (int)rounds;
   hipLaunchKernelGGL(f, dim3((unsigned)(groups * splits), (unsigned)(SPLIT ? 1 : HALF ? 2 : ceil_div(p.M, 16 * MT))), dim3((NW + S::FW) * 64), lds, s, p, (int)tiles, next, next > 1 ? 1 : (int)groups);
   return hipGetLastError() == hipSuccess ? 0 : 1;
 }
