@@ -785,10 +785,11 @@ static int pick(const FewRowsParams& p, hipStream_t s) {
       if (n && nck > kLongPart) return launch<EPI, false, false, 16, MT, I8, 7, 2, 4 * X, true>(p, s, n);
       if (n) return launch<EPI, false, false, 16, MT, I8, 8, 1, 2 * X, true>(p, s, n);
     }
-    // (as many waves as give each whole rounds of stages)
+    // (as many waves as give each whole rounds of stages, for one tile a workgroup; bf16 of 8192 x 7168 at 4 rows with 8 waves 20.9 us, with 7 21.6, int8 of 8192 x
+    // 5632 at 8 rows 14.0, with 11 14.9, but 8192 x 14336 at 4 rows 38.6 and 37.3)
     if (MT == 1 && nck > 33 && nck % 32) {
-      if (nck % 28 == 0) return tiles > 128 ? launch<EPI, false, false, 16, 1, I8, 7, 0, 4>(p, s) : launch<EPI, false, false, 8, 1, I8, 7, 0, 4>(p, s);
-      if (nck % 44 == 0) return tiles > 128 ? launch<EPI, false, false, 16, 1, I8, 11, 0, 3>(p, s) : launch<EPI, false, false, 8, 1, I8, 11, 0, 4>(p, s);
+      if (nck % 28 == 0 && (tiles <= (I8 ? 512 : 256) || nck > kLongPart)) return tiles > 128 ? launch<EPI, false, false, 16, 1, I8, 7, 0, 4>(p, s) : launch<EPI, false, false, 8, 1, I8, 7, 0, 4>(p, s);
+      if (nck % 44 == 0 && tiles <= 256) return tiles > 128 ? launch<EPI, false, false, 16, 1, I8, 11, 0, 3>(p, s) : launch<EPI, false, false, 8, 1, I8, 11, 0, 4>(p, s);
     }
     if (tiles > 128) return launch<EPI, false, false, 16, MT, I8, 8, 0, D>(p, s);
     if (nck > 8 && nck <= 16) return MT == 2 ? launch<EPI, false, false, 16, 1, I8, 8, 0, 2>(p, s) : launch<EPI, false, false, 8, 1, I8, 8, 0, 2>(p, s);
