@@ -17,11 +17,10 @@
 // Structure: the loop of gemm_tile.h (4 waves of 128 x 128 results, one workgroup per CU), both operands' images with contiguous
 // features, read with the hardware's transposing read; a token count that is no multiple of 64 makes the first step a partial one.
 //   * With one token split per tile the workgroup alone adds to its tile: it loads, adds and stores straight from the registers, the loads of 6 of 8
-//     rounds on their way together.  Lanes exchange halves of their fragments so that 8 of them have a line; whole lines can be read and written past the
-//     caches, which then keep the operands (64 bytes of 16 rows a time, through the caches: 3,000 tokens 128256 x 2048 1,561 us, now 1,518, 16384 x 2048 201 / 193; 1,344
-//     3072 x 4096 55 / 50; 8,192 12288 x 4096 674 / 640; 8 experts' 14336 x 4096 over 16,384 2,177 / 1,991; half lines past the caches are read
-//     twice, 4 to 8 % more).  Through LDS, 512 bytes of a row each, 2 to 16 % more.  With S splits the adds are S atomics in any order, through LDS so
-//     that they cover 256 contiguous bytes, issued without return and left in flight when the workgroup exits.
+//     rounds on their way together.  Lanes exchange halves of their fragments so that 8 of them have a line, as lines can be read and written past the caches
+//     only whole (half lines come twice, 4 to 8 % more): which gradients are, past_caches() says.  Through LDS, 512 bytes of a row each, 2 to 16 % more.  With S
+//     splits the adds are S atomics in any order, through LDS so that they cover 256 contiguous bytes, issued without return and left in flight when the
+//     workgroup exits.
 //   * Against 8 waves of 128 x 64 in ping-pong: 1,000 tokens 4096 x 4096 54 -> 48 us, 16384 x 2048 97 -> 86; 3,000 128256 x 2048 1,708 -> 1,526; 8,192
 //     6144 x 4096 406 -> 372; 8 experts' 14336 x 4096 over 32,768 3,903 -> 3,561.
 //   * grouped (MoE expert weight gradients, dW[e] += x_e^T dy_e over expert-sorted rows): the grid covers (split, expert, tile); each
@@ -56,8 +55,20 @@ struct Params {
   int64_t c_es;
 };
 
-// TAIL: a split may have a partial step (the first one)
-template <bool GROUPED, bool TAIL>
+template <bool PAST>
+__device__ __forceinline__ f32x4_t grad_load(const float* at) {
+  const f32x4_t* v = reinterpret_cast<const f32x4_t*>(at);
+  if constexpr (PAST) return __builtin_nontemporal_load(v);
+  else return *v;
+}
+template <bool PAST>
+__device__ __forceinline__ void grad_store(const f32x4_t& v, float* at) {
+  if constexpr (PAST) __builtin_nontemporal_store(v, reinterpret_cast<f32x4_t*>(at));
+  else *reinterpret_cast<f32x4_t*>(at) = v;
+}
+
+// TAIL: a split may have a partial step (the first one); PAST: the gradient past the caches
+template <bool GROUPED, bool TAIL, bool PAST>
 __global__ void __launch_bounds__(NT, 1) wgrad_kernel(Params p) {
   __shared__ __attribute__((aligned(16))) char smem[tile::LDS_BYTES];
   const int tiles = p.mt * p.nt;
@@ -111,11 +122,11 @@ __global__ void __launch_bounds__(NT, 1) wgrad_kernel(Params p) {
     f32x4_t cur[AHEAD][8];
     const bool whole = m0 + BM <= p.M && n0 + BN <= p.N;
     auto all = [&](auto ok) {
-      auto at = [&](int i, int j) { return reinterpret_cast<f32x4_t*>(cp + (int64_t)(32 * i + 8 * (j & 1)) * p.ldc + 32 * (j >> 1)); };
+      auto at = [&](int i, int j) { return cp + (int64_t)(32 * i + 8 * (j & 1)) * p.ldc + 32 * (j >> 1); };
       auto load = [&](int i) {   // 16 rows
 #pragma unroll
         for (int j = 0; j < 8; ++j)
-          if (ok(i, j)) cur[i % AHEAD][j] = __builtin_nontemporal_load(at(i, j));
+          if (ok(i, j)) cur[i % AHEAD][j] = grad_load<PAST>(at(i, j));
       };
 #pragma unroll
       for (int i = 0; i < AHEAD; ++i) load(i);
@@ -131,8 +142,8 @@ __global__ void __launch_bounds__(NT, 1) wgrad_kernel(Params p) {
             const float o = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(up ? u : v), 0x128 /* row_ror:8 */, 0xf, 0xf, false));
             lo[e] = up ? o : u, hi[e] = up ? v : o;
           }
-          if (ok(i, j)) __builtin_nontemporal_store(cur[i % AHEAD][j] + lo, at(i, j));
-          if (ok(i, j + 1)) __builtin_nontemporal_store(cur[i % AHEAD][j + 1] + hi, at(i, j + 1));
+          if (ok(i, j)) grad_store<PAST>(cur[i % AHEAD][j] + lo, at(i, j));
+          if (ok(i, j + 1)) grad_store<PAST>(cur[i % AHEAD][j + 1] + hi, at(i, j + 1));
         }
         if (i + AHEAD < 8) load(i + AHEAD);
         __builtin_amdgcn_sched_barrier(0);
@@ -162,12 +173,11 @@ __global__ void __launch_bounds__(NT, 1) wgrad_kernel(Params p) {
 // 128 x 64 results with a load, an add and a store of 32 rows at a time, steps of 32 tokens in a ring of four, half the registers to fill and
 // to empty.  us here / by the loop above:
 //   * 8 experts' 4096 x 28672 and 14336 x 4096 gradients: 256 tokens each 1,505, 697 / 1,588, 807; 768 2,237, 1,056 / 2,300, 1,084; 1,024 2,644,
-//     1,278 / 2,627, 1,308; 1,280 3,107, 1,507 / 3,032, 1,479; 1,536 3,505, 1,715 / 3,382, 1,646 (the gradient past the caches in both; through them, 256
-//     tokens 1,686, 821, 512 1,942, 1,024 2,749, 1,353);
+//     1,278 / 2,627, 1,308; 1,280 3,107, 1,507 / 3,032, 1,479; 1,536 3,505, 1,715 / 3,382, 1,646 (the gradient past the caches in both);
 //   * one gradient, whole steps of 32 tokens: 512 x 512 512 tokens 20 / 27, 1,024 32 / 37, 2,048 53 / 56, 3,072 75.3 / 74.9; 2048 x 2048 23 / 30, 34 /
 //     39, 56 / 58, 78 / 78; 3072 x 4096 1,056 46.3 / 48.9, 2,048 68 / 69; 4096 x 4096 512 39 / 42, 1,056 54 / 56, 1,536 69 / 67; 16384 x 2048 1,024
 //     102 / 109, 2,080 155 / 157, 3,072 205 / 199;
-//     (these two lines were measured with the gradient through the caches; past them both take 3 to 10 % less)
+//     (through the caches)
 //   * a partial last step (the loop's is its first): 4096 x 4096, 500 tokens 40 / 36, 700 45 / 40; 768 x 4096 or 128256 x 2048, 500 24, 560 / 28,
 //     608, 700 29, 659 / 32, 668, 1,000 38, 794 / 38, 788.
 //
@@ -181,7 +191,7 @@ __global__ void __launch_bounds__(NT, 1) wgrad_kernel(Params p) {
 //   * pieces issued after stage S's last: S+1 (4) and S+2's first half (2) -> vmcnt(6), less at the tail.
 namespace few {
 
-constexpr int FEW = 1150;   // tokens of a group
+inline int most(bool past) { return past ? 1150 : 1400; }   // tokens of a group
 constexpr int BK = 32, STAGES = 4, NT = 512;
 inline bool dense(int T, int tiles) {   // (one gradient, unsplit)
   if (T % BK) return T <= 450 || (T <= 700 && (tiles < 192 || tiles > 1024));
@@ -225,7 +235,7 @@ __device__ __forceinline__ bf16x8_t frag(const char* img, int c0) {
 
 // TAIL: the last step may be a partial one (always with GROUPED).  The look at it costs every load a comparison and a selection:
 // without them 1024 x 1024 over 512 tokens 22.9 -> 21.2 us, 800 30.0 -> 27.3, 16384 x 2048 over 800 97 -> 93.
-template <bool GROUPED, bool TAIL>
+template <bool GROUPED, bool TAIL, bool PAST>
 __global__ void __launch_bounds__(NT, 1) kernel(Params p) {
   __shared__ __attribute__((aligned(16))) char smem[LDS_BYTES];
   const int tiles = p.mt * p.nt;
@@ -346,7 +356,7 @@ __global__ void __launch_bounds__(NT, 1) kernel(Params p) {
   auto load = [&](int rnd) {
 #pragma unroll
     for (int k = 0; k < 8; ++k)
-      if (32 * rnd + 4 * k < left) cur[k] = __builtin_nontemporal_load(reinterpret_cast<const f32x4_t*>(cp + (int64_t)(32 * rnd + 4 * k) * p.ldc));
+      if (32 * rnd + 4 * k < left) cur[k] = grad_load<PAST>(cp + (int64_t)(32 * rnd + 4 * k) * p.ldc);
   };
   load(0);
   __syncthreads();   // every wave is done with the ring
@@ -365,7 +375,7 @@ __global__ void __launch_bounds__(NT, 1) kernel(Params p) {
     if (rnd < 3) load(rnd + 1);
 #pragma unroll
     for (int k = 0; k < 8; ++k)
-      if (32 * rnd + 4 * k < left) __builtin_nontemporal_store(sum[k], reinterpret_cast<f32x4_t*>(cp + (int64_t)(32 * rnd + 4 * k) * p.ldc));
+      if (32 * rnd + 4 * k < left) grad_store<PAST>(sum[k], cp + (int64_t)(32 * rnd + 4 * k) * p.ldc);
     __builtin_amdgcn_wave_barrier();
   }
 }
@@ -382,9 +392,23 @@ static int band_rows() {
 }
 
 template <bool G, bool TAIL>
-void launch(const Params& p, int64_t nwg, hipStream_t stream) {
-  hipLaunchKernelGGL((wgrad_kernel<G, TAIL>), dim3((unsigned)nwg), dim3(NT), 0, stream, p);
+void launch(const Params& p, int64_t nwg, bool past, hipStream_t stream) {
+  hipLaunchKernelGGL((past ? &wgrad_kernel<G, TAIL, true> : &wgrad_kernel<G, TAIL, false>), dim3((unsigned)nwg), dim3(NT), 0, stream, p);
 }
+template <bool G, bool TAIL>
+void launch_few(const Params& p, int64_t nwg, bool past, hipStream_t stream) {
+  hipLaunchKernelGGL((past ? &few::kernel<G, TAIL, true> : &few::kernel<G, TAIL, false>), dim3((unsigned)nwg), dim3(few::NT), 0, stream, p);
+}
+
+// Whether a gradient of so many bytes is read and written past the caches, which then keep the operands.  Not one that may lie in the memory-side cache (256
+// MB) when it is added to: gradients of up to 48 MB belong to models whose gradients may all lie there.  us, through the caches / past them:
+//   * three gradients in turn: 3072 x 2048 (24 MB), 256 tokens 20.2 / 23.9, 1,024 36 / 41; 4096 x 4096 (64 MB) 31 / 35, 51 / 55; 12288 x 4096 (192 MB) 101 / 94, 150 /
+//     145; 128256 x 2048, 1,000 tokens 754 / 722; 8 experts' 768 x 1024 1,024 rows 18.5 / 24.4, 14336 x 4096 775 / 682, 4096 x 28672 1,650 / 1,521, 8,192 rows
+//     3,209 / 3,110;
+//   * in a training step, where they come from memory: 4096 x 4096, 256 tokens 36 / 34, 500 45 / 42, 1,000 58 / 55, 2,048 84 / 80, 8,192 239 / 240; 12288 x 4096 1,000 162 / 162; 16384 x
+//     2048 3,000 201 / 201; 32000 x 4096 1,000 415 / 393; 128256 x 2048 3,000 1,605 / 1,581; 8 experts' 4096 x 28672 and 14336 x 4096, 2,048 rows 1,664 / 1,543 and
+//     806 / 735, 4,096 rows 1,990 / 1,900 and 960 / 934, 8,192 rows 2,835 / 2,800 and 1,380 / 1,363.
+bool past_caches(int64_t bytes) { return bytes >= (int64_t)48 << 20; }
 
 }  // namespace wg
 
@@ -442,12 +466,14 @@ int wgrad_gemm_launch(const void* dy, int64_t ld_dy, const void* x, int64_t ld_x
   p.band = wg::band_rows();
   const int64_t nwg = (int64_t)p.mt * p.nt * p.splits;
   if (nwg > INT32_MAX) return -2;
-  if (p.own && wg::few::dense(T, p.mt * p.nt))
-    hipLaunchKernelGGL((T % wg::few::BK ? &wg::few::kernel<false, true> : &wg::few::kernel<false, false>), dim3((unsigned)nwg), dim3(wg::few::NT), 0, stream, p);
-  else if (T % wg::BK)
-    wg::launch<false, true>(p, nwg, stream);
+  const bool past = wg::past_caches((int64_t)M * N * 4);
+  if (p.own && wg::few::dense(T, p.mt * p.nt)) {
+    if (T % wg::few::BK) wg::launch_few<false, true>(p, nwg, past, stream);
+    else wg::launch_few<false, false>(p, nwg, past, stream);
+  } else if (T % wg::BK)
+    wg::launch<false, true>(p, nwg, past, stream);
   else
-    wg::launch<false, false>(p, nwg, stream);
+    wg::launch<false, false>(p, nwg, past, stream);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
@@ -478,11 +504,9 @@ int wgrad_gemm_grouped_launch(const void* dy, int64_t ld_dy, const void* x, int6
   p.band = wg::band_rows();
   const int64_t nwg = (int64_t)p.mt * p.nt * E * p.splits;
   if (nwg > INT32_MAX) return -2;
-  if (p.own && rows / E <= wg::few::FEW) {
-    hipLaunchKernelGGL((wg::few::kernel<true, true>), dim3((unsigned)nwg), dim3(wg::few::NT), 0, stream, p);
-    return hipGetLastError() == hipSuccess ? 0 : -3;
-  }
-  wg::launch<true, true>(p, nwg, stream);
+  const bool past = wg::past_caches((int64_t)E * M * N * 4);
+  if (p.own && rows / E <= wg::few::most(past)) wg::launch_few<true, true>(p, nwg, past, stream);
+  else wg::launch<true, true>(p, nwg, past, stream);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 

@@ -79,3 +79,32 @@ def test_route_of_ragged_token_counts(T, M, N, own):
         assert G._wgrad_kernel_splits(mg, dy, x) == (1 if -(-M // 256) * -(-N // 256) >= 128 else 0)
     G.wgrad_accumulate_(mg, dy, x)
     _check(mg, before, dy, x)
+
+
+@pytest.mark.parametrize("M,N", [(3064, 4104), (3072, 4104)])   # 48 MB: through the caches below, past them from there on
+@pytest.mark.parametrize("T", [96, 100, 1000, 2112])            # both kernels, whole and partial steps
+def test_through_and_past_the_caches(M, N, T):
+    g = torch.Generator(device="cuda").manual_seed(T + M)
+    dy, x = (torch.randn(T, n, generator=g, device="cuda").bfloat16() for n in (M, N))
+    whole = torch.randn(M, N + 4, generator=g, device="cuda")
+    before = whole.clone()
+    print(T, M, N, flush=True)
+    ext().wgrad_gemm(whole[:, :N], dy, x, 1, True)
+    _check(whole[:, :N], before[:, :N], dy, x)
+    assert torch.equal(whole[:, N:], before[:, N:])
+
+
+@pytest.mark.parametrize("sizes", [[0, 100, 1300], [700, 1, 4000]])   # a mean below and above the line of each
+@pytest.mark.parametrize("K,N", [(2056, 2040), (2056, 2048)])         # 48 MB
+def test_groups_through_and_past_the_caches(sizes, K, N):
+    g = torch.Generator(device="cuda").manual_seed(sum(sizes))
+    x, dy = (torch.randn(sum(sizes), n, generator=g, device="cuda").bfloat16() for n in (K, N))
+    offs = torch.tensor([0] + sizes, device="cuda").cumsum(0).to(torch.int32)
+    mg = torch.randn(len(sizes), K, N, generator=g, device="cuda")
+    before = mg.clone()
+    print(sizes, K, N, flush=True)
+    ext().grouped_gemm(2, x, dy, offs, mg, True)
+    for e in range(len(sizes)):
+        a, b = int(offs[e]), int(offs[e + 1])
+        _check(mg[e], before[e], x[a:b], dy[a:b]) if b > a else None
+        assert b > a or torch.equal(mg[e], before[e])
