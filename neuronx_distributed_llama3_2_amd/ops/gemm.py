@@ -51,20 +51,31 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias=None, out: torch.Tensor = None
 _ACTS = {"swiglu": 0, "relu2": 1}
 
 
-def act_pays(rows: int, weight_rows: int, K: int) -> bool:
+def act_pays(rows: int, weight_rows: int, K: int, glu: bool = False) -> bool:
     """Whether csrc/act_gemm.hip is faster than a library product and the activation's own pass: work for three quarters of the CUs (256 x 256
-    results each) and a reduction that the pass is not small beside.  us, two launches / one, weights from memory: SwiGLU of 8,192
-    columns, reduction 2,048: 512 rows 41 / 45, 768 56 / 57, 1,024 73 / 62, 2,304 150 / 147, 4,096 245 / 231; of 14,336, 4,096: 256 rows 80 / 85,
-    512 122 / 108, 1,792 385 / 350, 4,096 706 / 708; of 28,672, 8,192: 2,304 rows 1,555 / 1,599; squared ReLU of 12,288, 2,048: 768 rows 46 /
-    51, 1,024 62 / 55, 4,096 189 / 172.  Long prompts stay with the one launch: SwiGLU of 8,192, 2,048 at 8,192 / 16,384 rows 448 / 435, 894 / 882; 14,336, 4,096 at 8,192
-    / 12,288 / 16,384 1,360 / 1,354, 2,013 / 2,054, 2,714 / 2,700; 11,008, 4,096 at 4,096 / 16,384 672 / 550, 2,208 / 2,088; squared ReLU of 12,288, 2,048 at 16,384 693 / 632."""
-    return K % 32 == 0 and K <= 4096 and rows * weight_rows >= 192 * 256 * 256
+    results each), a reduction that the pass is not small beside, and rounds of the CUs that are filled to three quarters: what is left after whole rounds
+    takes a whole one too, or, cut into 2 or 4 pieces, about two thirds of one (half of one if the pieces leave half of the CUs to themselves); up to a reduction of 1,024 the
+    pass is so large a part that this does not matter (SwiGLU of 8,192 at 1,280 rows 58 / 55).  us, two launches / one,
+    weights from memory: SwiGLU of 8,192 columns, reduction 2,048: 768 rows 54 / 57, 1,024 68 / 62, 2,304 150 / 152, 4,096 232 / 231; of 14,336, 4,096: 512 rows
+    111 / 109, 1,792 381 / 347, 5,120 1,001 / 912; of 11,008, 4,096: 4,096 694 / 579; of 28,672, 8,192: 2,304 rows 1,555 / 1,599; squared ReLU of 12,288, 2,048: 768 rows 46 /
+    51, 1,024 60 / 60, 4,096 182 / 170.  Rounds that are not filled (two launches): SwiGLU of 14,336, 4,096 at 640 rows 146 / 165, 24,576 at 640 240 / 265, 8,192 at 1,280 92 /
+    97, 11,008 at 896 161 / 170, squared ReLU of 16,384, 4,096 at 1,280 161 / 173.  The library does best where its tiles fill whole rounds too, and a long reduction hides SwiGLU's
+    pass: of 14,336, 4,096 at 4,096 / 12,288 rows 706 / 714, 2,100 / 2,150, of 24,576 at 3,072 / 10,240 926 / 944, 3,046 / 3,138 (two launches from four rounds on); of 8,192,
+    3,072 at 4,096 / 16,384 330 / 324, 1,254 / 1,251, squared ReLU of 16,384, 4,096 at 16,384 1,632 / 1,603."""
+    if K % 32 or K > 4096 or rows * weight_rows < 192 * 256 * 256:
+        return False
+    if K <= 1024:
+        return True
+    tiles = -(-rows // 256) * -(-weight_rows // 256)
+    whole, tail = divmod(-(-tiles // 8), 32)   # of an XCD's CUs
+    time = whole + (0 if tail == 0 else 0.45 if tail <= 4 else 0.67 if tail <= 16 else 1)
+    return rows * weight_rows >= 0.75 * time * 256 ** 3 and not (glu and K > 3072 and tail == 0 and whole >= 4)
 
 
 def linear_act(x: torch.Tensor, w: torch.Tensor, act: str) -> Optional[torch.Tensor]:
     """act(x [..., K] @ w^T) in one launch, or None where that is not done or not faster.  "swiglu": w [2 N, K] = [gate; up]; "relu2": w [N, K]."""
     K, N = w.shape[1], w.shape[0] // 2 if act == "swiglu" else w.shape[0]
-    if not (_native(x, w) and x.dtype == w.dtype == torch.bfloat16 and act_pays(x.numel() // max(K, 1), w.shape[0], K)
+    if not (_native(x, w) and x.dtype == w.dtype == torch.bfloat16 and act_pays(x.numel() // max(K, 1), w.shape[0], K, act == "swiglu")
             and N % (128 if act == "swiglu" else 8) == 0 and (N + 256) * K < 2 ** 31
             and x.shape[-1] == K and x.is_contiguous() and w.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
         return None

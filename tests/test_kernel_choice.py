@@ -17,3 +17,15 @@ def test_hyper_step(R, W, threads):
 def test_few_rows(N, K, halved):
     f = ops.ext().few_rows_halved
     assert f(17, N, K) == f(32, N, K) == halved and not f(16, N, K) and not f(33, N, K)
+
+
+# the line of three quarters of the CUs; rounds that are not filled; whole rounds of long reductions
+@pytest.mark.parametrize("rows,weight_rows,K,glu,pays", [
+    (768, 16384, 2048, True, True), (767, 16384, 2048, True, False), (4096, 16384, 4128, True, False), (4096, 16384, 2040, True, False),
+    (1280, 16384, 2048, True, False), (1400, 16384, 2048, True, True), (1280, 16384, 2048, False, False), (1280, 16384, 1024, True, True), (640, 28672, 4096, True, False), (896, 22016, 4096, True, False),
+    (896, 28672, 4096, True, True), (1536, 12288, 2048, False, True), (2304, 16384, 2048, True, True),
+    (4096, 28672, 4096, True, False), (4096, 28672, 4096, False, True), (4096, 28672, 3072, True, True), (1024, 16384, 4096, True, True), (5120, 28672, 4096, True, True)])
+def test_products_with_an_activation(rows, weight_rows, K, glu, pays):
+    from neuronx_distributed_llama3_2_amd.ops import gemm
+
+    assert gemm.act_pays(rows, weight_rows, K, glu) is pays
