@@ -64,4 +64,21 @@ def test_rule(act, N, K):
         two = ops.swiglu(z) if act == "swiglu" else ops.relu_squared(z)
         got = packed_linear_act(torch.nn.Module(), x, w, None, act)
         assert (got.float() - two.float()).norm() <= 2 ** -7 * two.float().norm()
-        assert gemm.linear_act(x[:, 1:], w[:, 1:], act) is None      # not contiguous
+
+
+@pytest.mark.parametrize("act", ["swiglu", "relu2"])
+def test_operands_of_other_layouts(act):
+    """Rows further apart than they are long, and contiguous operands that begin 8 bytes past a multiple of 16: two launches, either operand alone."""
+    from neuronx_distributed_llama3_2_amd.ops import gemm
+
+    R, rows, K = 1024, 16384, 2048
+    gen = torch.Generator(device="cuda").manual_seed(1)
+
+    def operands(n):
+        flat = torch.randn(n * (K + 32), device="cuda", generator=gen).bfloat16()
+        return flat[: n * K].view(n, K), flat.view(n, K + 32)[:, :K], flat[4: 4 + n * K].view(n, K)
+
+    (x, *others), (w, *weights) = operands(R), operands(rows)
+    assert gemm.linear_act(x, w, act) is not None
+    for a, b in [(o, w) for o in others] + [(x, o) for o in weights]:
+        assert gemm.linear_act(a, b, act) is None
