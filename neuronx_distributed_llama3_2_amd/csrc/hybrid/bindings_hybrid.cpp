@@ -171,8 +171,15 @@ void delta_rule(Tensor proj, int64_t B, int64_t T, std::vector<int64_t> sizes, T
   Tensor cells;   // (outlives the launches below)
   if (p.nch > 0) {
     const int64_t n = B * p.nch * p.H;
-    const int64_t one = n * 64 * (p.DP + (p.V + 15) / 16 * 16 + 64 + 2), split = nxd::delta_chunk_split_floats(p);
-    cells = at::empty({one + split}, opt);
+    const int64_t one = n * 64 * (p.DP + (p.V + 15) / 16 * 16 + 64 + 2);
+    int64_t split = nxd::delta_chunk_split_floats(p);
+    try {
+      cells = at::empty({one + split}, opt);
+    } catch (const c10::OutOfMemoryError&) {   // (in one launch, then: it needs less)
+      if (split == 0) throw;
+      split = 0;
+      cells = at::empty({one}, opt);
+    }
     p.cw = cells.data_ptr<float>();
     p.cp = p.cw + n * 64 * p.DP;
     p.ceg = p.cp + n * 64 * 64;

@@ -581,7 +581,8 @@ static int dispatch_chunk(const DeltaParams& p, hipStream_t s) {
 // one launch fills the chip as well.  The whole operation, us, one launch / two: 16 heads of 128 x 128 (128 blocks of columns), 512 tokens 75 / 78,
 // 768 89 / 85, 1,024 104 / 94, 4,096 317 / 274; 8 of 64 x 64 (32 blocks) 256 tokens 35 / 34, 4,096 156 / 110; 4 of 128 x 128 256 tokens 44 / 43, 4,096 209 /
 // 141; 32 of 96 x 128 (256 blocks) 1,024 tokens 118 / 118, 4,096 392 / 406.  With keys of more than 128 the one launch has not the registers: 16 of 256 x 128, 128
-// tokens 96 / 80, 4,096 903 / 544, two sequences of up to 2,000 542 / 356.  Not past 1 GiB.
+// tokens 96 / 80, 4,096 903 / 544, two sequences of up to 2,000 542 / 356.  The states and U are 100 MB for 4,096 tokens of 16 heads of 128 x 128 beside 84 MB of the chunks' operands; not past
+// 1 GiB, and the caller takes the one launch where there is no room for them.
 int64_t delta_chunk_split_floats(const DeltaParams& p) {
   const int64_t nv = ceil_div(p.V, 16), blocks = nv * p.B * p.H, floats = blocks * p.nch * 16 * (64 + p.DP);
   const bool pays = p.DP > 128 ? blocks <= 256 && p.nch >= 2 : blocks <= 128 && p.nch >= (blocks <= 64 ? 4 : 12);

@@ -45,3 +45,36 @@ def test_two_launches(H, G, D, V, T):
     s, rg = state[:1].clone(), ring[:1].clone()
     got = run([1], 0, s, rg)
     assert rel_err(got[0, :lens[1]].reshape(lens[1], -1), delta_oracle(sz, proj_o[1, :lens[1]], *case[3:], 1e-5)) < where[2]
+
+
+def test_without_room_for_the_states():
+    """Room for the one launch's operands and not for the states beside them: the same bits, and the scratch is given back."""
+    from neuronx_distributed_llama3_2_amd import ops
+
+    H, D, V, T, taps = 16, 128, 128, 8192, 4                     # operands of the chunks 169 MB, states and U 201 MB
+    case = delta_case(("cuda", torch.bfloat16, 0), 1, T, H, H, D, V, taps)
+    sz, proj = case[0], case[1][0].contiguous()
+    rest = [v.cuda() for v in case[3:]]
+
+    def run():
+        state = torch.zeros((1, H, V, sz.padded_dim), device="cuda")
+        ring = torch.zeros((1, taps, sz.channels), dtype=torch.bfloat16, device="cuda")
+        y = ops.delta_rule(proj, 1, T, sz, *rest, 1e-5, torch.zeros(1, dtype=torch.long, device="cuda"), None, None, state, ring)
+        return y.cpu(), state.cpu(), ring.cpu()
+
+    want = run()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    # what the call has beside them: q, k of all heads, v and o, gates in fp32, y, and blocks of 2 MB or 20 MB that the allocator rounds to
+    need = 4 * (4 * T * H * D + 2 * T * H) + 2 * T * H * V + 4 * 2 ** 20 * 16
+    operands = T // 64 * H * 64 * (D + V + 64 + 2) * 4
+    room = torch.cuda.memory_reserved() + need + operands + 64 * 2 ** 20
+    torch.cuda.set_per_process_memory_fraction(room / torch.cuda.get_device_properties(0).total_memory)
+    try:
+        before = torch.cuda.memory_stats()["num_ooms"]
+        got = run()
+        assert torch.cuda.memory_stats()["num_ooms"] > before    # (there was no room)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
