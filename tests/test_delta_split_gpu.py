@@ -1,6 +1,6 @@
 """The chunked delta rule's scan in two launches (few blocks of columns) gives the bits of the one launch that a larger batch takes, and the oracle's
 numbers: ragged lengths, head sizes that fill no block, a state that goes on, keys of more than 128,
-outputs normed where they are formed."""
+outputs normed where they are formed, in both activation types."""
 import pytest
 import torch
 
@@ -9,12 +9,13 @@ from test_golitar_mechanisms import delta_case, delta_oracle, rel_err, run_delta
 pytestmark = pytest.mark.gpu
 
 
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 5e-5), (torch.bfloat16, 2e-2)], ids=["f32", "bf16"])   # (as in test_golitar_mechanisms)
 @pytest.mark.parametrize("H,G,D,V,T", [(3, 3, 16, 24, 300), (16, 8, 128, 128, 769), (2, 1, 70, 33, 1000), (9, 9, 144, 16, 130), (4, 2, 256, 40, 250),
                                        (16, 8, 32, 68, 2100), (16, 16, 128, 128, 2049)])   # (16 heads: the outputs' launch norms them)
-def test_two_launches(H, G, D, V, T):
+def test_two_launches(H, G, D, V, T, dtype, tol):
     from neuronx_distributed_llama3_2_amd import ops
 
-    where, taps = ("cuda", torch.float32, 5e-5), 4
+    where, taps = ("cuda", dtype, tol), 4
     n = -(-257 // (H * -(-V // 16))) + 1          # sequences of the batch that takes one launch
     lens = [T, T - 67] + [1] * (n - 2)
     case = delta_case(where, n, T, H, G, D, V, taps)
@@ -23,14 +24,14 @@ def test_two_launches(H, G, D, V, T):
     def run(rows, pos0, state, ring):
         t = torch.tensor
         B = len(rows)
-        print(H, G, D, V, T, B, flush=True)
+        print(H, G, D, V, T, B, dtype, flush=True)
         return ops.delta_rule(proj[rows].reshape(B * T, -1).contiguous(), B, T, sz, *(v.cuda() for v in case[3:]), 1e-5,
                               t([pos0] * B, device="cuda"), t([lens[r] for r in rows], dtype=torch.int32, device="cuda"), None, state, ring).view(B, T, H, V)
 
     def fresh(B):
         g = torch.Generator().manual_seed(5)
         return (torch.randn((1, H, V, sz.padded_dim), generator=g).expand(B, -1, -1, -1).contiguous().cuda(),
-                torch.zeros((B, taps, sz.channels), device="cuda"))
+                torch.zeros((B, taps, sz.channels), dtype=dtype, device="cuda"))
 
     for pos0 in (0, 64):                           # a prompt, and one that goes on from a state
         s_all, r_all = fresh(n)
@@ -40,11 +41,11 @@ def test_two_launches(H, G, D, V, T):
             y = run([r], pos0, s, ring)
             assert not y[0, lens[r]:].any() and not y_all[r, lens[r]:].any()
             assert torch.equal(y[0, :lens[r]], y_all[r, :lens[r]]) and torch.equal(s[0], s_all[r]) and torch.equal(ring[0], r_all[r])
-    state = torch.zeros((n, H, V, sz.padded_dim), device="cuda")
-    ring = torch.zeros((n, taps, sz.channels), device="cuda")
-    s, rg = state[:1].clone(), ring[:1].clone()
-    got = run([1], 0, s, rg)
-    assert rel_err(got[0, :lens[1]].reshape(lens[1], -1), delta_oracle(sz, proj_o[1, :lens[1]], *case[3:], 1e-5)) < where[2]
+    for pos0 in (0, 64):                           # (at 64 with a state, and no inputs before it)
+        st, ring = fresh(1)
+        before = st[0, :, :, :D].transpose(1, 2).double().cpu() if pos0 else None
+        got = run([1], pos0, st, ring)
+        assert rel_err(got[0, :lens[1]].reshape(lens[1], -1), delta_oracle(sz, proj_o[1, :lens[1]], *case[3:], 1e-5, before)) < tol
 
 
 def test_without_room_for_the_states():

@@ -82,8 +82,8 @@ def delta_case(where, B, T, H, G, D, V, taps, seed=0, strong=False):
     return sz, proj, proj_o, conv, a_log, dt, norm
 
 
-def delta_oracle(sz, proj, conv, a_log, dt, norm, eps):
-    """proj [T, columns] of one sequence -> [T, H V]."""
+def delta_oracle(sz, proj, conv, a_log, dt, norm, eps, state=None):
+    """proj [T, columns] of one sequence -> [T, H V], from state [H, D, V] on (none: zeros)."""
     H, G, D, V, C = sz.heads, sz.kv_heads, sz.dim, sz.vdim, sz.channels
     T = proj.shape[0]
     x = O.silu(O.causal_conv(proj[:, :C], conv.double().t()))
@@ -93,7 +93,7 @@ def delta_oracle(sz, proj, conv, a_log, dt, norm, eps):
     gates = proj[:, C + H * V:]
     beta = torch.sigmoid(gates[:, :H])
     decay = torch.exp(-torch.exp(a_log.double()) * O.softplus(gates[:, H:2 * H] + dt.double()))
-    o, _ = O.delta_scan(q, k, x[:, 2 * G * D:C].reshape(T, H, V), decay, beta)
+    o, _ = O.delta_scan(q, k, x[:, 2 * G * D:C].reshape(T, H, V), decay, beta, state)
     o = O.rms_normalise(o, eps) * norm.double() * O.silu(proj[:, C:C + H * V]).view(T, H, V)
     return o.reshape(T, H * V)
 
