@@ -496,6 +496,11 @@ PYBIND11_MODULE(_hybrid, m) {
   register_gemm(m);
   register_parallel(m);
   namespace py = pybind11;
+  m.def("delta_split_floats", [](int B, int T, int H, int D, int V) {   // what a prompt's scan in two launches takes, 0: one launch
+    nxd::DeltaParams p{};
+    p.B = B, p.H = H, p.V = V, p.DP = (D + 31) / 32 * 32, p.nch = (T + 63) / 64;
+    return nxd::delta_chunk_split_floats(p);
+  });
   m.def("hyper_step_threads", &nxd::hyper_step_threads);   // of the one-pass kernel for R rows of W columns, strides ldy and ldh; 0: the loop
   m.def("hyper_step", &hyper_step, py::arg("x"), py::arg("embed") = py::none(), py::arg("ids") = py::none(),
         py::arg("y") = py::none(), py::arg("bias") = py::none(), py::arg("mix") = py::none(), py::arg("write") = py::none(),

@@ -580,12 +580,13 @@ static int dispatch_chunk(const DeltaParams& p, hipStream_t s) {
 // and 43 for the outputs), the second launch and its 8 to 14 us of start are lost in longer runs, and with more columns than half of the CUs the
 // one launch fills the chip as well.  The whole operation, us, one launch / two: 16 heads of 128 x 128 (128 blocks of columns), 512 tokens 75 / 78,
 // 768 89 / 85, 1,024 104 / 94, 4,096 317 / 274; 8 of 64 x 64 (32 blocks) 256 tokens 35 / 34, 4,096 156 / 110; 4 of 128 x 128 256 tokens 44 / 43, 4,096 209 /
-// 141; 32 of 96 x 128 (256 blocks) 1,024 tokens 118 / 118, 4,096 392 / 406.  With keys of more than 128 the one launch has not the registers: 16 of 256 x 128, 128
+// 141, 4 x 128 x 72 in two sequences (40 blocks) 256 tokens 44 / 43, but with 64 blocks 4 to 10 chunks are no gain: 4 of 128 x 128 in two sequences 384 tokens 51 / 55, 16 of
+// 96 x 64 512 tokens 54 / 57, 8 of 64 x 128 640 tokens 51 / 53, 896 62 / 60; 32 of 96 x 128 (256 blocks) 1,024 tokens 118 / 118, 4,096 392 / 406.  With keys of more than 128 the one launch has not the registers: 16 of 256 x 128, 128
 // tokens 96 / 80, 4,096 903 / 544, two sequences of up to 2,000 542 / 356.  The states and U are 100 MB for 4,096 tokens of 16 heads of 128 x 128 beside 84 MB of the chunks' operands; not past
 // 1 GiB, and the caller takes the one launch where there is no room for them.
 int64_t delta_chunk_split_floats(const DeltaParams& p) {
   const int64_t nv = ceil_div(p.V, 16), blocks = nv * p.B * p.H, floats = blocks * p.nch * 16 * (64 + p.DP);
-  const bool pays = p.DP > 128 ? blocks <= 256 && p.nch >= 2 : blocks <= 128 && p.nch >= (blocks <= 64 ? 4 : 12);
+  const bool pays = p.DP > 128 ? blocks <= 256 && p.nch >= 2 : blocks <= 128 && p.nch >= (blocks <= 40 ? 4 : 12);
   return pays && floats <= (int64_t{1} << 28) ? floats : 0;
 }
 

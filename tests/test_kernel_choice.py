@@ -29,3 +29,11 @@ def test_products_with_an_activation(rows, weight_rows, K, glu, pays):
     from neuronx_distributed_llama3_2_amd.ops import gemm
 
     assert gemm.act_pays(rows, weight_rows, K, glu) is pays
+
+
+# blocks of 16 columns and chunks of 64 tokens: few blocks from 4 chunks on, up to 128 from 12, long keys from 2 up to 256; a gigabyte
+@pytest.mark.parametrize("B,T,H,D,V,split", [(1, 193, 5, 128, 128, True), (1, 192, 5, 128, 128, False), (1, 704, 41, 64, 16, False), (1, 705, 41, 64, 16, True),
+                                             (2, 512, 4, 128, 128, False), (1, 705, 16, 128, 128, True), (1, 4096, 129, 64, 16, False), (1, 65, 16, 256, 256, True),
+                                             (1, 64, 16, 256, 256, False), (2, 4096, 9, 256, 256, False), (1, 1 << 16, 8, 128, 128, True), (1, 1 << 16, 16, 128, 128, False)])
+def test_delta_rule_in_two_launches(B, T, H, D, V, split):
+    assert (ops.hybrid_ext().delta_split_floats(B, T, H, D, V) > 0) is split
