@@ -67,7 +67,8 @@ __device__ __forceinline__ float dot8_bf16(const u32x4_t& a, const u32x4_t& b, f
 }
 
 // op(v, v of lane ^ O), by the lanes' own data paths: a step of a wave's sum is one or two VALU instructions (__shfl_xor goes through LDS, about 60 cycles a step
-// in a chain of six).  Same order of sums, so the same bits; a lane that is off counts as zero, as there.
+// in a chain of six).  Same order of sums, so the same bits.  All lanes whose values meet have to be active: a lane that is off counts as zero in the steps of 1 to 8
+// and leaves the reader's own value, counted twice, in those of 16 and 32.
 template <int CTRL>
 __device__ __forceinline__ float dpp(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
