@@ -1,4 +1,4 @@
-// The main loop of the 256 x 256-tile products (grouped_rowgemm.hip, wgrad_gemm.hip): C = A B over a reduction in steps of 64, bf16 operands, fp32 sums.
+// The main loop of the 256 x 256-tile products (grouped_rowgemm.hip, wgrad_gemm.hip, act_gemm.hip): C = A B over a reduction in steps of 64, bf16 operands, fp32 sums.
 //
 // What bounds it is the clock that the numbers allow (8192 x 8192 x 8192: 1.99 GHz with random ones, 2.40 with zeros, counted as
 // GRBM_GUI_ACTIVE over the kernel's time) and what feeds the matrix cores: LDS reads, and loads of a CU.
@@ -234,12 +234,12 @@ struct Loop {
 // 2,159 -> 2,069; one gradient of 8,192 or 3,000 tokens the same within 1 % (its reads and writes, and the clock).  Five half steps: 1 % less for
 // 128256 x 2048, 2 % more for 1,344 to 4,096 tokens.
 struct LoopTR {
-  static constexpr int HK = BK / 2, HALF_BYTES = HK * 256 * 2, PLACE_BYTES = 2 * HALF_BYTES, PLACES = 4;
+  static constexpr int HK = BK / 2, HALF_BYTES = HK * 256 * 2, PLACE_BYTES = 2 * HALF_BYTES, PLACES = 4, LOADS = 8;   // loads: of a wave, for a half step
   static_assert(PLACES * PLACE_BYTES <= LDS_BYTES, "LDS");
   char* smem;
   int lane, wid, wm, wn;
   uint32_t lds;
-  uint32_t off[8];   // of this lane's pieces of A (0 .. 3) and B from a half step's base
+  uint32_t off[LOADS];   // of this lane's pieces of A (0 .. 3) and B from a half step's base
   const char *pa, *pb;
   int64_t da, db;    // bytes of 32 reduction rows
 
@@ -249,7 +249,7 @@ struct LoopTR {
     pa = uniform(reinterpret_cast<const char*>(a)), pb = uniform(reinterpret_cast<const char*>(b));
     da = (int64_t)HK * lda * 2, db = (int64_t)HK * ldb * 2;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < LOADS; ++i) {
       const int t = 2 * (4 * wid + (i & 3)) + (lane >> 5), c = (lane & 31) ^ tr_swz(t);
       off[i] = (uint32_t)(t * (i < 4 ? lda : ldb) + min(8 * c, (i < 4 ? rows : cols) - 8)) * 2;
     }
@@ -277,7 +277,7 @@ struct LoopTR {
       for (int h = 0; h < 2; ++h) {   // (rows past the last: that one again)
         const int have = max(min(rows - h * HK, HK), 1);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
+        for (int i = 0; i < LOADS; ++i) {
           const int past = max(0, 2 * (4 * wid + (i & 3)) + (lane >> 5) - (have - 1));
           const uint32_t from = off[i] - past * (uint32_t)((i < 4 ? da : db) / HK);
           load_lds(from, i < 4 ? pa : pb, lds + h * PLACE_BYTES + (i < 4 ? 0 : HALF_BYTES) + (4 * wid + (i & 3)) * 1024);
@@ -295,14 +295,14 @@ struct LoopTR {
 #pragma unroll
     for (int q = FIRST ? 2 : 0; q < PLACES; ++q) {   // (past the end: the last one again, not used)
 #pragma unroll
-      for (int i = 0; i < 8; ++i) load(i, q * PLACE_BYTES);
+      for (int i = 0; i < LOADS; ++i) load(i, q * PLACE_BYTES);
       advance(q + 1);
     }
     int ra[8], rb[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) ra[i] = tr_at(32 * i + 16 * wm), rb[i] = HALF_BYTES + tr_at(128 * wn + 16 * i);
-    auto there = [&]() {   // all loads but those of the three newest half steps have come, and all waves have read so far
-      asm volatile("s_waitcnt vmcnt(16) lgkmcnt(0)" ::: "memory");
+    auto there = [&]() {   // all loads but those of the two newest half steps have come, and all waves have read so far
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(2 * LOADS) : "memory");
       __builtin_amdgcn_s_barrier();
       __builtin_amdgcn_sched_barrier(0);
     };
