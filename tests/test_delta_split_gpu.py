@@ -69,9 +69,17 @@ def test_without_room_for_the_states():
     # what the call has beside them: q, k of all heads, v and o, gates in fp32, y, and blocks of 2 MB or 20 MB that the allocator rounds to
     need = 4 * (4 * T * H * D + 2 * T * H) + 2 * T * H * V + 4 * 2 ** 20 * 16
     operands = T // 64 * H * 64 * (D + V + 64 + 2) * 4
-    room = torch.cuda.memory_reserved() + need + operands + 64 * 2 ** 20
-    torch.cuda.set_per_process_memory_fraction(room / torch.cuda.get_device_properties(0).total_memory)
+    reserved, total = torch.cuda.memory_reserved(), torch.cuda.get_device_properties(0).total_memory
+    held = []
     try:
+        torch.cuda.set_per_process_memory_fraction(reserved / total)
+        for size in (2 ** e for e in range(30, 20, -1)):         # (room that others have left within their blocks)
+            try:
+                while True:
+                    held.append(torch.empty(size, dtype=torch.uint8, device="cuda"))
+            except torch.cuda.OutOfMemoryError:
+                pass
+        torch.cuda.set_per_process_memory_fraction((reserved + need + operands + 64 * 2 ** 20) / total)
         before = torch.cuda.memory_stats()["num_ooms"]
         got = run()
         assert torch.cuda.memory_stats()["num_ooms"] > before    # (there was no room)
