@@ -400,15 +400,19 @@ void launch_few(const Params& p, int64_t nwg, bool past, hipStream_t stream) {
   hipLaunchKernelGGL((past ? &few::kernel<G, TAIL, true> : &few::kernel<G, TAIL, false>), dim3((unsigned)nwg), dim3(few::NT), 0, stream, p);
 }
 
-// Whether a gradient of so many bytes is read and written past the caches, which then keep the operands.  Not one that may lie in the memory-side cache (256
-// MB) when it is added to: gradients of up to 48 MB belong to models whose gradients may all lie there.  us, through the caches / past them:
-//   * three gradients in turn: 3072 x 2048 (24 MB), 256 tokens 20.2 / 23.9, 1,024 36 / 41; 4096 x 4096 (64 MB) 31 / 35, 51 / 55; 12288 x 4096 (192 MB) 101 / 94, 150 /
-//     145; 128256 x 2048, 1,000 tokens 754 / 722; 8 experts' 768 x 1024 1,024 rows 18.5 / 24.4, 14336 x 4096 775 / 682, 4096 x 28672 1,650 / 1,521, 8,192 rows
-//     3,209 / 3,110;
-//   * in a training step, where they come from memory: 4096 x 4096, 256 tokens 36 / 34, 500 45 / 42, 1,000 58 / 55, 2,048 84 / 80, 8,192 239 / 240; 12288 x 4096 1,000 162 / 162; 16384 x
-//     2048 3,000 201 / 201; 32000 x 4096 1,000 415 / 393; 128256 x 2048 3,000 1,605 / 1,581; 8 experts' 4096 x 28672 and 14336 x 4096, 2,048 rows 1,664 / 1,543 and
-//     806 / 735, 4,096 rows 1,990 / 1,900 and 960 / 934, 8,192 rows 2,835 / 2,800 and 1,380 / 1,363.
-bool past_caches(int64_t bytes) { return bytes >= (int64_t)48 << 20; }
+// Whether a gradient of so many bytes is read and written past the caches, which then keep the operands.  What a gradient costs depends on where it lies when it is
+// added to, and in a training step it comes from memory once all gradients together are more than the memory-side cache (256 MB, 64 M parameters).  us, through the caches /
+// past them:
+//   * in a training step: 2048 x 2048 (16 MB), 256 tokens 21.4 / 21.5, 512 26.9 / 27.1, 960 36.8 / 36.8; 3072 x 2048 (24 MB) 23.9 / 22.8, 30.1 / 28.8, 40.2 /
+//     38.7; 4096 x 4096, 256 tokens 36 / 34, 500 45 / 42, 1,000 58 / 55, 2,048 84 / 80, 8,192 239 / 240; 12288 x 4096 1,000 162 / 162; 16384 x 2048 3,000
+//     201 / 201; 32000 x 4096 1,000 415 / 393; 128256 x 2048 3,000 1,605 / 1,581; 8 experts' 4096 x 28672 and 14336 x 4096, 2,048 rows 1,664 / 1,543 and
+//     806 / 735, 4,096 rows 1,990 / 1,900 and 960 / 934, 8,192 rows 2,835 / 2,800 and 1,380 / 1,363;
+//   * 3 GB of gradients in turn: 3840 x 2048 448 tokens 30.1 / 27.6, 15872 x 768 1,920 66.0 / 61.2; 8 experts' 768 x 1024 (24 MB) 9,216 rows 60.4 / 55.3, 12,000 64.4 /
+//     62.5, 768 x 1408 9,216 62.0 / 60.0, 12,000 70.4 / 67.5;
+//   * three gradients in turn, as where all of a small model's lie in that cache (given up for the steps above from 20 MB on): 3072 x 2048, 256 tokens 20.2 / 23.9, 1,024
+//     36 / 41; 4096 x 4096 31 / 35, 51 / 55; 8 experts' 768 x 1024 1,024 rows 18.5 / 24.4; but 12288 x 4096 (192 MB) 101 / 94, 150 / 145, 8 experts' 14336 x 4096 775 /
+//     682, 4096 x 28672 1,650 / 1,521, 8,192 rows 3,209 / 3,110.
+bool past_caches(int64_t bytes) { return bytes >= (int64_t)20 << 20; }
 
 }  // namespace wg
 
