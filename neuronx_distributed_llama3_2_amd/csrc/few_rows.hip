@@ -48,7 +48,7 @@ __device__ __forceinline__ void lds_read(u32x4_t (&v)[2], const uint32_t (&at)[2
   asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %3\n\ts_waitcnt lgkmcnt(0)" : "=&v"(v[0]), "=&v"(v[1]) : "v"(at[0]), "v"(at[1]) : "memory");
 }
 __device__ __forceinline__ void lds_write(uint32_t at, const f32x4_t& v) { asm volatile("ds_write_b128 %0, %1" ::"v"(at), "v"(v) : "memory"); }
-// (the result of a matrix product: asm has to wait for it by itself, 11 cycles for 8 passes)
+// (the result of a matrix product: asm has to wait for it by itself, 8 wait states after 4 passes; these are 16)
 __device__ __forceinline__ void lds_write_sum(uint32_t at, const f32x4_t& v) { asm volatile("s_nop 15\n\tds_write_b128 %0, %1" ::"v"(at), "v"(v) : "memory"); }
 __device__ __forceinline__ void lds_write(uint32_t at, float v) { asm volatile("ds_write_b32 %0, %1" ::"v"(at), "v"(v) : "memory"); }
 __device__ __forceinline__ uint32_t lds_at(const void* p) { return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)p; }
