@@ -229,10 +229,14 @@ struct Loop {
 };
 
 // Both operands' rows / columns contiguous (weight gradients): half steps of 32 of the reduction, 32 KB each, four of them there.  While the products of
-// half step q run, the fragments of q + 1 are read, and q + 4 is loaded into the place of q, read during q - 1: a step to a step and a half for a
-// load's way, where whole steps left half a step to one.  8 experts 4096 x 28672 over 12,288 rows 3,484 -> 3,397 us, 14336 x 4096 over 16,384
+// half step q run, the fragments of q + 1 are read, and q + 4 is loaded into the place of q, read during q - 1: a step to a step and a quarter
+// for a load's way, where whole steps left half a step to one.  8 experts 4096 x 28672 over 12,288 rows 3,484 -> 3,397 us, 14336 x 4096 over 16,384
 // 2,159 -> 2,069; one gradient of 8,192 or 3,000 tokens the same within 1 % (its reads and writes, and the clock).  Five half steps: 1 % less for
 // 128256 x 2048, 2 % more for 1,344 to 4,096 tokens.
+// The reads come in the first half of a half step and the loads in the second: the barrier waits for the reads, and spread over all of it, with the loads between them, the
+// last ones were still on their way there (few tiles in splits took 2 to 4 % more than with whole steps: us, whole steps / half steps, spread / now: 2304 x 1280 over 4,224
+// tokens 57.4 / 58.9 / 57.5, 3072 x 2048 4,608 86.8 / 88.8 / 86.5, 1280 x 512 4,800 30.9 / 32.0 / 31.3, unsplit 4864 x 1792 2,560 73.2 / 73.0 / 70.3; 8 experts' 4096 x
+// 2048 over 12,552 rows 315 / 280 / 272).
 struct LoopTR {
   static constexpr int HK = BK / 2, HALF_BYTES = HK * 256 * 2, PLACE_BYTES = 2 * HALF_BYTES, PLACES = 4, LOADS = 8;   // loads: of a wave, for a half step
   static_assert(PLACES * PLACE_BYTES <= LDS_BYTES, "LDS");
@@ -339,9 +343,8 @@ struct LoopTR {
       int next = after(now);
 #pragma unroll
       for (int u = 0; u < 16; ++u) {
-        if (u < 8) b1[u] = read(rb[u] + next);
-        else a1[u - 8] = read(ra[u - 8] + next);
-        if (u & 1) load(u >> 1, now);
+        if (u < 8) b1[u] = read(rb[u] + next), a1[u] = read(ra[u] + next);
+        else load(u - 8, now);
         mfmas(u, a0, b0);
       }
       advance(q + PLACES + 1);
@@ -349,9 +352,8 @@ struct LoopTR {
       now = next, next = after(now);
 #pragma unroll
       for (int u = 0; u < 16; ++u) {
-        if (u < 8) b0[u] = read(rb[u] + next);
-        else a0[u - 8] = read(ra[u - 8] + next);
-        if (u & 1) load(u >> 1, now);
+        if (u < 8) b0[u] = read(rb[u] + next), a0[u] = read(ra[u] + next);
+        else load(u - 8, now);
         mfmas(u, a1, b1);
       }
       advance(q + PLACES + 2);
