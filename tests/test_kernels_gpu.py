@@ -285,6 +285,8 @@ def test_swiglu_forward_token_major_copy_feeds_down_wgrad(monkeypatch):
     from neuronx_distributed_llama3_2_amd.parallel_layers import layers
 
     monkeypatch.setattr(gemm, "_WGRAD_T", "2")
+    for switch in ("_DENSE_WG", "_WG_KERNEL"):   # (they'd take the product without a copy, and add in another order than the library may)
+        monkeypatch.setattr(gemm, switch, "0")
     C = _ext.ext()
     gu0 = torch.randn(2, 192, 2 * 448, device=DEV, dtype=torch.bfloat16)
     h_ref = torch.empty(2, 192, 448, device=DEV, dtype=torch.bfloat16)
