@@ -1,6 +1,6 @@
 // The main loop of the 256 x 256-tile products (grouped_rowgemm.hip, wgrad_gemm.hip, act_gemm.hip): C = A B over a reduction in steps of 64, bf16 operands, fp32 sums.
 //
-// What bounds it is the clock that the numbers allow (8192 x 8192 x 8192: 1.99 GHz with random ones, 2.40 with zeros, counted as
+// What bounds it is the clock that the numbers allow (8192 x 8192 x 8192: 1.75 GHz with random ones, 2.36 with zeros, counted as
 // GRBM_GUI_ACTIVE over the kernel's time) and what feeds the matrix cores: LDS reads, and loads of a CU.
 //   * 4 waves, one a SIMD, of 128 x 128 results each: 64 v_mfma_f32_16x16x32_bf16 for 16 fragments read from LDS, two thirds of what
 //     8 waves of 128 x 64 read -- those read 192 KB a step where LDS gives 128 bytes a clock, as long as the MFMAs take.  The
