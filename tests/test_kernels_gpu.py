@@ -253,6 +253,8 @@ def test_swiglu_transposed_grad_reaches_gate_up_wgrad(monkeypatch):
     from neuronx_distributed_llama3_2_amd.parallel_layers import layers
 
     monkeypatch.setattr(gemm, "_WGRAD_T", "2")   # TN layout at this small size too
+    for switch in ("_DENSE_WG", "_WG_KERNEL"):   # (they'd take the product without a copy, and add in another order than the library may)
+        monkeypatch.setattr(gemm, switch, "0")
     seen = []
     orig = gemm.wgrad_accumulate_
 
