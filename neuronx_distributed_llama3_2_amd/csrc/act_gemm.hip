@@ -6,8 +6,8 @@
 //
 // The tiles are dealt to the XCDs in equal runs of an L2 band raster.  What is left of a run after whole rounds of its 32 CUs would keep a few CUs for
 // a whole tile's time, so these tiles are cut into 2 or 4 pieces of 128 or 64 rows when all CUs can have one.
-// Against a library product and the activation's own launch, us, weights from memory: SwiGLU of 8,192 columns, reduction 2,048: 1,024 rows 73 -> 62, 2,304 150 ->
-// 147, 4,096 245 -> 231; squared ReLU of 12,288, 2,048: 1,024 rows 62 -> 55, 2,048 115 -> 99, 4,096 189 -> 172 (1.20 PFLOP/s, the product alone at 1.4 in the library).
+// Against a library product and the activation's own launch, us, weights from memory: SwiGLU of 8,192 columns, reduction 2,048: 1,024 rows 68 -> 62, 2,304 150 ->
+// 152 (147 on another card), 4,096 232 -> 231; squared ReLU of 12,288, 2,048: 1,024 rows 60 -> 60, 4,096 182 -> 170 (1.2 PFLOP/s, the product alone at 1.4 in the library).
 // The products are the library's to the bit there (its unsplit kernels sum in the same order).  Fewer rows: the library, with smaller tiles.
 #include "gemm_tile.h"
 
