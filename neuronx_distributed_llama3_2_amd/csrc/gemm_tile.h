@@ -1,26 +1,33 @@
 // The main loop of the 256 x 256-tile products (grouped_rowgemm.hip, wgrad_gemm.hip, act_gemm.hip): C = A B over a reduction in steps of 64, bf16 operands, fp32 sums.
 //
-// What bounds it is the clock that the numbers allow (8192 x 8192 x 8192: 1.75 GHz with random ones, 2.36 with zeros, counted as
-// GRBM_GUI_ACTIVE over the kernel's time) and what feeds the matrix cores: LDS reads, and loads of a CU.
+// What bounds it is the clock that the numbers allow (8192 x 8192 x 8192 with random ones 1.75 to 1.9 GHz, with zeros 2.36, counted as
+// GRBM_GUI_ACTIVE over the kernel's time) and what stands between the MFMAs.
 //   * 4 waves, one a SIMD, of 128 x 128 results each: 64 v_mfma_f32_16x16x32_bf16 for 16 fragments read from LDS, two thirds of what
 //     8 waves of 128 x 64 read -- those read 192 KB a step where LDS gives 128 bytes a clock, as long as the MFMAs take.  The
 //     256 sums of a lane are in AGPRs; the MFMAs are written in asm, because hipcc moves such sums between registers
 //     (216 moves and 124 waits a step of 128 MFMAs: 0.22 PFLOP/s).
-//   * A step's operands are 64 KB of LDS.  Three steps of A are there and two of B (160 KB): the MFMAs of one half of a step (32 of the reduction) are
-//     interleaved with the reads of the next half, four to a read; in the first half the loads of A go out, two steps ahead; after it a barrier
-//     says that the step has been read and the next one is there, and B's loads go out with the first MFMAs of the second half.  (With two of
-//     both, the loads of A and B spread over the second half had to be there half a step after the last of them: without any loads the loop took 22 to 28 % less time.)
+//   * A wave is alone on its SIMD, so the matrix cores wait for whatever it does beyond the 12 cycles that a MFMA leaves free: between two MFMAs
+//     there is at most a read, an address or a load.  Above all no read stands behind the instruction that makes its address (5 cycles a
+//     read): addresses move on by themselves once a step, between MFMAs that nothing else needs.  The word that says where a load goes in LDS (m0)
+//     and the load have a MFMA between them.  Cycles a step of 2,048 for the MFMAs alone, A B^T / A B / A^T B: reads, addresses and loads four MFMAs apart 2,562 / 2,685 /
+//     2,744, now 2,213 / 2,233 / 2,195 (without loads and the barrier 2,085 / 2,120 / 2,024).
+//   * A step's operands are 64 KB of LDS.  Three steps of A are there and two of B (160 KB): during the MFMAs of one half of a step (32 of the reduction) the
+//     next half is read; in the first half the loads of A go out, two steps ahead; after it a barrier
+//     says that the step has been read and the next one is there, and B's loads go out with the first MFMAs of the second half.
 //   * Loads go straight to LDS, 128 bytes of a row and more: whole lines (with 64 bytes of a row a CU gets 50 GB/s, with 128 it gets 90).
 //   * Weight gradients, whose images can be cut in halves of whole lines, have a ring of half steps instead (LoopTR).
-//   us, two steps of both -> now: 8 experts, 8,192 rows uneven, 4096 -> 28672 1,711 / 2,064 (input gradient) -> 1,681 / 1,846, 14336 -> 4096 1,015 / 836 -> 929 /
-//   821; 8192 x 8192 x 8192 of random numbers 809 / 756 -> 779 / 756, of zeros 697 / 663 -> 617 / 595: with random numbers it is the clock that bounds it.  256 rows of 8
-//   experts 421 / 390 -> 401 / 371.
+//   us, four MFMAs apart -> now, one card in turn: 8 experts, 8,192 rows uneven, 4096 -> 28672 1,638 / 1,817 (input gradient) -> 1,504 / 1,664; 8192 x 8192 x 8192 of
+//   random numbers A B^T 745 -> 690, A B 756 -> 693, A^T B 835 -> 742 (a warmer card 776 -> 711, 787 -> 722, 874 -> 792: with random numbers what is saved in cycles
+//   is partly given back in clock); SwiGLU of 8,192 columns, 2,048, 2,304 rows 134 -> 128.
 //
 // Images of a step in LDS, 16-byte chunks XORed so that 16 lanes of a read cover all banks once:
 //   ROW  the reduction is contiguous: [256 rows][64], 128-byte rows
 //   TR   the rows / columns are contiguous: [64][256], 512-byte rows, read with ds_read_b64_tr_b16
 #pragma once
 #include "common.h"
+
+#include <type_traits>
+#include <utility>
 
 namespace nxd {
 namespace tile {
@@ -63,6 +70,32 @@ __device__ __forceinline__ void settled(f32x4_t (&acc)[8][8]) {
     for (int j = 0; j < 8; ++j) asm volatile("" : "+a"(acc[i][j]));
 }
 
+template <int... I, typename F>
+__device__ __forceinline__ void each(std::integer_sequence<int, I...>, F&& f) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void each(F&& f) {   // f(0), .. f(N - 1), each number a constant
+  each(std::make_integer_sequence<int, N>{}, f);
+}
+
+// One product, and one with a load (64 lanes x 16 B: base + at -> LDS lds + MORE + 16 lane): it stands between m0 and the load that reads it.
+__device__ __forceinline__ void mfma(f32x4_t& c, const bf16x8_t& b, const bf16x8_t& a) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(b), "v"(a));
+}
+template <int MORE>
+__device__ __forceinline__ void mfma_load(f32x4_t& c, const bf16x8_t& b, const bf16x8_t& a, uint32_t at, const char* base, uint32_t lds) {
+  asm volatile("s_add_u32 m0, %5, %6\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0\n\tglobal_load_lds_dwordx4 %3, %4"
+               : "+a"(c)
+               : "v"(b), "v"(a), "v"(at), "s"(base), "s"(lds), "n"(MORE)
+               : "memory", "m0", "scc");
+}
+// An address for reads to come, made where nothing waits for it
+__device__ __forceinline__ void move_to(int& at, int base, int by) { asm volatile("v_add_u32 %0, %1, %2" : "=v"(at) : "s"(by), "v"(base)); }
+__device__ __forceinline__ void move_by(int& at, int by) { asm volatile("v_add_u32 %0, %1, %0" : "+v"(at) : "s"(by)); }
+__device__ __forceinline__ void fixed() { __builtin_amdgcn_sched_barrier(0); }   // what stands before stays before
+__device__ __forceinline__ void reads_done() { __builtin_amdgcn_s_waitcnt(0xC07F); }   // (lgkmcnt(0); the compiler knows of it)
+
 template <bool BT>
 struct Loop {
   char* smem;
@@ -98,20 +131,22 @@ struct Loop {
     }
   }
 
-  // the half step's fragment addresses (of the first buffer): ROW: [chunk bit 2], TR: [fragment]
-  int ra[2], rb[BT ? 8 : 2];
+  // fragment addresses: of A's first image by half, of A's images that are read now and of B's (ROW: [chunk bit 2], TR: [fragment])
+  static constexpr int NB = BT ? 8 : 2;
+  int base_a[2], ra[2], rb[NB];
   __device__ __forceinline__ void addresses() {
     const int r = lane & 15, g = lane >> 4;
     const int row = 16 * wm + r;
-    ra[0] = row * 128 + 16 * (g ^ row_swz(row));
-    ra[1] = ra[0] ^ 64;
+    base_a[0] = row * 128 + 16 * (g ^ row_swz(row));
+    base_a[1] = base_a[0] ^ 64;
+    ra[0] = base_a[0], ra[1] = base_a[1];
     if constexpr (BT) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) rb[j] = B_BASE + tr_at(128 * wn + 16 * j);
     } else {
       const int c = 128 * wn + 8 * (r >> 2) + (r & 3);
       rb[0] = B_BASE + c * 128 + 16 * (g ^ row_swz(c));
-      rb[1] = rb[0] ^ 64;
+      rb[1] = rb[0] ^ 64;   // (B_BASE is a multiple of 128)
     }
   }
   __device__ __forceinline__ int tr_at(int c0) const {   // lane 16 g + 4 q + p: 4 columns from c0 + 4 p on, of reduction rows 8 g + q (and + 4)
@@ -125,24 +160,25 @@ struct Loop {
     return __builtin_bit_cast(bf16x8_t, v);
   }
   __device__ __forceinline__ bf16x8_t read_row(int at) const { return __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(smem + at)); }
-  __device__ __forceinline__ bf16x8_t frag_a(int i, int h, int buf) const {
-    return read_row(ra[h] + buf + i * 4096);
-  }
-  __device__ __forceinline__ bf16x8_t frag_b(int j, int h, int buf) const {
-    if constexpr (BT) return read_tr(rb[j] + buf + h * (IMG_BYTES / 2));
-    else return read_row(rb[h ^ (j & 1)] + buf + (j & 1) * 512 + (j >> 1) * 4096);
+  __device__ __forceinline__ bf16x8_t frag_a(int i, int h) const { return read_row(ra[h] + i * 4096); }
+  __device__ __forceinline__ bf16x8_t frag_b(int j, int h) const {
+    if constexpr (BT) return read_tr(rb[j] + h * (IMG_BYTES / 2));
+    else return read_row(rb[h ^ (j & 1)] + (j & 1) * 512 + (j >> 1) * 4096);
   }
 
-  template <bool HALF, bool FEW>
-  __device__ __forceinline__ void load(int i, int img, bool last) {   // piece i (A: 0 .. 7) of the next step; HALF, last: its second half is past the end
-    if (FEW && i < 8 && i >= pieces) return;
-    const uint32_t to = lds + (i < 8 ? 0 : B_BASE) + img + (8 * wid + (i & 7)) * 1024;
-    uint32_t from = off[i];
+  template <bool HALF>
+  __device__ __forceinline__ uint32_t from(int i, bool last) const {   // piece i (A: 0 .. 7) of the next step; HALF, last: its second half is past the end
+    uint32_t at = off[i];
     if constexpr (HALF) {   // (the first half again: not used)
       const bool tr = i >= 8 && BT;
-      if (last) from -= (back >> i & 1) * (tr ? (uint32_t)((i < 8 ? da : db) / 2) : 64u);
+      if (last) at -= (back >> i & 1) * (tr ? (uint32_t)((i < 8 ? da : db) / 2) : 64u);
     }
-    load_lds(from, i < 8 ? pa : pb, to);
+    return at;
+  }
+  template <bool HALF, bool FEW>
+  __device__ __forceinline__ void load(int i, int img, bool last) const {
+    if (FEW && i < 8 && i >= pieces) return;
+    load_lds(from<HALF>(i, last), i < 8 ? pa : pb, lds + (i < 8 ? 0 : B_BASE) + img + (8 * wid + (i & 7)) * 1024);
   }
   template <bool FEW>
   __device__ __forceinline__ void wait_a() const {   // all loads but A's of the newest step have come
@@ -176,42 +212,63 @@ struct Loop {
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 #pragma unroll
-    for (int j = 0; j < 8; ++j) b0[j] = frag_b(j, 0, 0);
+    for (int j = 0; j < 8; ++j) b0[j] = frag_b(j, 0), fixed();   // (in this order: the loop's waits count what came later)
 #pragma unroll
-    for (int i = 0; i < IM; ++i) a0[i] = frag_a(i, 0, 0);
-    // chunk u of a half: a read of the next half's, a load, IM / 2 MFMAs
-    auto mfmas = [&](int u, const bf16x8_t (&a)[IM], const bf16x8_t (&b)[8]) {
-#pragma unroll
-      for (int v = 0; v < IM / 2; ++v) {
-        const int m = u * (IM / 2) + v, i = m >> 3, j = m & 7;
-        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(b[j]), "v"(a[i]));
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    };
+    for (int i = 0; i < IM; ++i) a0[i] = frag_a(i, 0), fixed();
+    // A half step: its products, and between two of them at most a read of the next half's fragments (k: B's, then A's), an address or a load.  A
+    // wave is alone on its SIMD: what stands between two products beyond the 12 cycles that the first leaves free, or waits for what stands just
+    // before it, the matrix cores wait for.
+    constexpr int M = 8 * IM, READS = 8 + IM;
+    constexpr int RD = IM == 2 ? 1 : 2, LD = IM == 2 ? 2 : 4;   // products from one read, or load, to the next
+    // from there on the addresses of B move, their reads of a first half all out (or, with 8 in the 16 products of IM == 2, those of rb[k] from FREE + k on)
+    constexpr int FREE = IM == 2 && BT ? 8 : RD * READS, SP = (M - FREE) / NB;
     int a_now = 0, a_next = IMG_BYTES, a_free = 2 * IMG_BYTES, b_now = 0;
+    const uint32_t mine = lds + wid * 8192;
 #pragma unroll 1
     for (int t = 0, whole = steps - (HALF && end); t < whole; ++t) {
       asm volatile("s_nop 3");   // (after moves of the sums ahead of the loop)
-#pragma unroll
-      for (int u = 0; u < 16; ++u) {
-        if (u < 8) b1[u] = frag_b(u, 1, b_now);
-        else if (u - 8 < IM) a1[u - 8] = frag_a(u - 8, 1, a_now);
-        if (u & 1) load<HALF, FEW>(u >> 1, a_free, end && t + 3 >= steps);
-        mfmas(u, a0, b0);
-      }
-      advance_a(t + 3);
+      const bool last = end && t + 3 >= steps;
+      const uint32_t to_a = mine + a_free, to_b = mine + b_now;
+      const int b_by = b_now ? -IMG_BYTES : IMG_BYTES;
+      each<M>([&](auto mc) __attribute__((always_inline)) {
+        constexpr int m = mc, k = m / RD, l = m / LD;
+        f32x4_t& c = acc[m >> 3][m & 7];
+        if constexpr (m % RD == RD - 1 && k < READS) {   // (one of B's and one of A's in turn)
+          if constexpr (k < 2 * IM && k % 2 == 1) a1[k >> 1] = frag_a(k >> 1, 1);
+          else b1[k < 2 * IM ? k >> 1 : k - IM] = frag_b(k < 2 * IM ? k >> 1 : k - IM, 1);
+          fixed();
+        }
+        if constexpr (m >= FREE && (m - FREE) % SP == 0) move_by(rb[(m - FREE) / SP], b_by), fixed();
+        if constexpr (m == M - 1) move_to(ra[0], base_a[0], a_next), fixed();
+        if constexpr (!FEW && m == 36) advance_a(t + 3), fixed();
+        if constexpr (!FEW && m % LD == LD / 2 && l < 8) {
+          mfma_load<l * 1024>(c, b0[m & 7], a0[m >> 3], from<HALF>(l, last), pa, to_a);
+        } else {
+          if constexpr (m % LD == LD / 2 && l < 8) load<HALF, FEW>(l, a_free, last);
+          mfma(c, b0[m & 7], a0[m >> 3]);
+        }
+        fixed();
+      });
+      if (FEW) advance_a(t + 3);
+      reads_done();
       wait_a<FEW>();
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __builtin_amdgcn_s_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int u = 0; u < 16; ++u) {
-        if (u < 8) b0[u] = frag_b(u, 0, b_now ^ IMG_BYTES);
-        else if (u - 8 < IM) a0[u - 8] = frag_a(u - 8, 0, a_next);
-        if (u < 8) load<HALF, FEW>(8 + u, b_now, end && t + 3 >= steps);
-        mfmas(u, a1, b1);
-      }
-      advance_b(t + 3);
+      fixed();
+      each<M>([&](auto mc) __attribute__((always_inline)) {
+        constexpr int m = mc, RD2 = IM == 8 ? 4 : RD, k = m / RD2, l = m / LD;
+        f32x4_t& c = acc[m >> 3][m & 7];
+        if constexpr (m % RD2 == RD2 / 2 && k < READS) {
+          if constexpr (k < 8) b0[k] = frag_b(k, 0);
+          else a0[k - 8] = frag_a(k - 8, 0);
+          fixed();
+        }
+        if constexpr (m == 0) move_to(ra[1], base_a[1], a_next), fixed();
+        if constexpr (!FEW && m == 36) advance_b(t + 3), fixed();
+        if constexpr (m % LD == LD - 1 && l < 8) mfma_load<B_BASE + l * 1024>(c, b1[m & 7], a1[m >> 3], from<HALF>(8 + l, last), pb, to_b);
+        else mfma(c, b1[m & 7], a1[m >> 3]);
+        fixed();
+      });
+      if (FEW) advance_b(t + 3);
       b_now ^= IMG_BYTES;
       const int freed = a_now;
       a_now = a_next, a_next = a_free, a_free = freed;
@@ -262,11 +319,12 @@ struct LoopTR {
     const int t = 8 * (lane >> 4) + (lane >> 2 & 3), c = c0 + 4 * (lane & 3);
     return t * 512 + 16 * (c >> 3 ^ tr_swz(t)) + 8 * (c >> 2 & 1);
   }
-  __device__ __forceinline__ bf16x8_t read(int at) const {
-    const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(smem + at));
-    const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(smem + at + 4 * 512));
+  __device__ __forceinline__ static bf16x8_t joined(const short4_t& lo, const short4_t& hi) {
     const short __attribute__((ext_vector_type(8))) v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     return __builtin_bit_cast(bf16x8_t, v);
+  }
+  __device__ __forceinline__ bf16x8_t read(int at) const {
+    return joined(__builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(smem + at)), __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(smem + at + 4 * 512)));
   }
   __device__ __forceinline__ void load(int i, int place) const {
     load_lds(off[i], i < 4 ? pa : pb, lds + place + (i < 4 ? 0 : HALF_BYTES) + (4 * wid + (i & 3)) * 1024);
@@ -306,7 +364,8 @@ struct LoopTR {
 #pragma unroll
     for (int i = 0; i < 8; ++i) ra[i] = tr_at(32 * i + 16 * wm), rb[i] = HALF_BYTES + tr_at(128 * wn + 16 * i);
     auto there = [&]() {   // all loads but those of the two newest half steps have come, and all waves have read so far
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(2 * LOADS) : "memory");
+      reads_done();
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * LOADS) : "memory");
       __builtin_amdgcn_s_barrier();
       __builtin_amdgcn_sched_barrier(0);
     };
@@ -328,37 +387,39 @@ struct LoopTR {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();   // (half step 0 has been read)
     __builtin_amdgcn_sched_barrier(0);
-    int now = 0;   // place of half step q
-    auto mfmas = [&](int u, const bf16x8_t (&a)[8], const bf16x8_t (&b)[8]) {
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int m = 4 * u + v;
-        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[m >> 3][m & 7]) : "v"(b[m & 7]), "v"(a[m >> 3]));
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    };
+    for (int i = 0; i < 8; ++i) ra[i] += PLACE_BYTES, rb[i] += PLACE_BYTES;
+    int now = 0;   // place of half step q
     auto after = [](int place) { return place == (PLACES - 1) * PLACE_BYTES ? 0 : place + PLACE_BYTES; };
+    // a half step in `now`: its products, first with the reads of the next one's fragments between them, then with the loads and the addresses of the one after
+    auto half = [&](const bf16x8_t (&a)[8], const bf16x8_t (&b)[8], bf16x8_t (&na)[8], bf16x8_t (&nb)[8]) {
+      const int next = after(now), by = after(next) - next;
+      const uint32_t to = lds + now + wid * 4096;
+      short4_t part[2];
+      each<64>([&](auto mc) __attribute__((always_inline)) {
+        constexpr int m = mc, u = m >> 2, k = (m - 32) >> 1, l = (m - 32) >> 2;
+        f32x4_t& c = acc[m >> 3][m & 7];
+        if constexpr (m < 32) {
+          part[m & 1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(smem + (m & 2 ? ra[u] : rb[u]) + (m & 1) * 4 * 512));
+          if constexpr (m & 1) (m & 2 ? na : nb)[u] = joined(part[0], part[1]);
+          fixed();
+        } else if constexpr (m & 1) {
+          move_by(k < 8 ? rb[k & 7] : ra[k & 7], by), fixed();
+        }
+        if constexpr (m >= 32 && m % 4 == 2) mfma_load<(l < 4 ? 0 : HALF_BYTES) + (l & 3) * 1024>(c, b[m & 7], a[m >> 3], off[l], l < 4 ? pa : pb, to);
+        else mfma(c, b[m & 7], a[m >> 3]);
+        fixed();
+      });
+      now = next;
+    };
 #pragma unroll 1
     for (int q = 0; q < n; q += 2) {
-      int next = after(now);
-#pragma unroll
-      for (int u = 0; u < 16; ++u) {
-        if (u < 8) b1[u] = read(rb[u] + next), a1[u] = read(ra[u] + next);
-        else load(u - 8, now);
-        mfmas(u, a0, b0);
-      }
+      half(a0, b0, a1, b1);
       advance(q + PLACES + 1);
       there();
-      now = next, next = after(now);
-#pragma unroll
-      for (int u = 0; u < 16; ++u) {
-        if (u < 8) b0[u] = read(rb[u] + next), a0[u] = read(ra[u] + next);
-        else load(u - 8, now);
-        mfmas(u, a1, b1);
-      }
+      half(a1, b1, a0, b0);
       advance(q + PLACES + 2);
       there();
-      now = next;
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (loads that nothing reads)
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");   // (the last sums)
