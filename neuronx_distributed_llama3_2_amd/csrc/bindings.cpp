@@ -17,7 +17,7 @@
 namespace nxd {
 int flash_attn_fwd_launch(const void*, const void*, const void*, void*, float*, const int64_t*, const int64_t*,
                           const int64_t*, const int64_t*, int, int, int, int, int, int, float, int, int,
-                          const DropoutArgs&, hipStream_t);
+                          const DropoutArgs&, hipStream_t, const int* cu = nullptr, int rows = 0);
 int64_t flash_attn_bwd_workspace(int, int, int, int, int, int, int, int);
 void flash_attn_bwd_set_knob(int, int);
 int transpose_bf16_launch(const void*, void*, int64_t, int64_t, int64_t, int64_t, hipStream_t);
@@ -54,6 +54,7 @@ int decode_attn_launch(const void*, const int64_t*, const void*, const void*, co
 void decode_attn_plan(int, int, int, int, int, int, bool, int*);
 int kv_cache_write_launch(const void*, const void*, const int64_t*, void*, void*, const int64_t*, const int*, const int*,
                           int, int, int, int, int, hipStream_t);
+int pack_prompts_launch(const int64_t*, int64_t, const int64_t*, const int*, int, int, int, int64_t*, int64_t*, int*, int*, int*, hipStream_t);
 int argmax_launch(const void*, int, int64_t, int, int, int64_t*, hipStream_t);
 int greedy_advance_launch(const void*, int, int64_t, int, int, unsigned long long*, int64_t*, int64_t, int, int64_t*, int64_t*,
                           int64_t*, int*, hipStream_t);
@@ -154,6 +155,42 @@ void flash_attn_fwd(at::Tensor q, at::Tensor k, at::Tensor v, at::Tensor o, at::
                                       vs, os, B, Sq, Sk, Hq, Hkv, D, (float)scale, causal ? 1 : 0, (int)causal_offset,
                                       dropout_args(dropout_p, seed, head_offset), cur_stream()),
            "flash_attn_fwd");
+}
+
+// Causal attention of sequences packed one after the other: q, k, v, o [R, heads, D], sequence b at rows cu[b] .. cu[b + 1], at most `most` of them
+void flash_attn_packed(at::Tensor q, at::Tensor k, at::Tensor v, at::Tensor o, at::Tensor cu, int64_t most, double scale) {
+  int64_t qs[3], ks[3], vs[3], os[3];
+  auto rows = [](const at::Tensor& t, const char* name, int64_t* st) {
+    TORCH_CHECK(t.dim() == 3, name, ": [rows, heads, D]");
+    bshd_strides(t.unsqueeze(0), name, st);
+  };
+  rows(q, "q", qs), rows(k, "k", ks), rows(v, "v", vs), rows(o, "o", os);
+  const int64_t R = q.size(0), Hq = q.size(1), D = q.size(2), Hkv = k.size(1);
+  TORCH_CHECK(k.sizes() == v.sizes() && k.size(0) == R && k.size(2) == D && o.sizes() == q.sizes(), "flash_attn_packed: shapes");
+  TORCH_CHECK(D == 64 || D == 128, "head_dim must be 64 or 128");
+  TORCH_CHECK(Hkv > 0 && Hq % Hkv == 0, "num q heads must be a multiple of num kv heads");
+  TORCH_CHECK(cu.is_cuda() && cu.scalar_type() == at::kInt && cu.is_contiguous() && cu.dim() == 1 && cu.numel() >= 2, "cu: int32 [B + 1]");
+  TORCH_CHECK(most > 0 && most <= R && R < INT32_MAX, "flash_attn_packed: lengths");
+  check_rc(nxd::flash_attn_fwd_launch(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), nullptr, qs, ks, vs, os, (int)cu.numel() - 1, (int)most,
+                                      (int)most, (int)Hq, (int)Hkv, (int)D, (float)scale, 1, 0, dropout_args(0.0, 0, 0), cur_stream(), cu.data_ptr<int>(), (int)R),
+           "flash_attn_packed");
+}
+
+void pack_prompts(at::Tensor ids, at::Tensor lens, at::Tensor slots, at::Tensor out_ids, at::Tensor pos, at::Tensor pos0, at::Tensor row_slot,
+                  at::Tensor cu) {
+  TORCH_CHECK(ids.is_cuda() && ids.scalar_type() == at::kLong && ids.dim() == 2 && ids.stride(1) == 1 && ids.size(1) < INT32_MAX, "pack_prompts: int64 ids [B, T]");
+  const int64_t B = ids.size(0), R = out_ids.numel();
+  for (const auto& t : {lens, out_ids, pos})
+    TORCH_CHECK(t.is_cuda() && t.scalar_type() == at::kLong && t.is_contiguous(), "pack_prompts: int64 lengths, ids and positions");
+  for (const auto& t : {slots, pos0, row_slot, cu})
+    TORCH_CHECK(t.is_cuda() && t.scalar_type() == at::kInt && t.is_contiguous(), "pack_prompts: int32 slots, places and starts");
+  TORCH_CHECK(lens.numel() == B && slots.numel() == B && cu.numel() == B + 1 && pos.numel() == R && pos0.numel() == R && row_slot.numel() == R && R > 0 &&
+                  B > 0 && R < INT32_MAX - 256,
+              "pack_prompts: sizes");
+  check_rc(nxd::pack_prompts_launch(ids.data_ptr<int64_t>(), ids.stride(0), lens.data_ptr<int64_t>(), slots.data_ptr<int>(), (int)B, (int)ids.size(1),
+                                    (int)R, out_ids.data_ptr<int64_t>(), pos.data_ptr<int64_t>(), pos0.data_ptr<int>(), row_slot.data_ptr<int>(),
+                                    cu.data_ptr<int>(), cur_stream()),
+           "pack_prompts");
 }
 
 void flash_attn_bwd(at::Tensor q, at::Tensor k, at::Tensor v, at::Tensor o, at::Tensor dout, at::Tensor lse,
@@ -1288,6 +1325,8 @@ PYBIND11_MODULE(_C, m) {
   m.def("flash_attn_fwd", &flash_attn_fwd, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("o"), py::arg("lse"),
         py::arg("scale"), py::arg("causal"), py::arg("causal_offset"), py::arg("dropout_p") = 0.0, py::arg("seed") = 0,
         py::arg("head_offset") = 0);
+  m.def("flash_attn_packed", &flash_attn_packed);
+  m.def("pack_prompts", &pack_prompts);
   m.def("flash_attn_bwd", &flash_attn_bwd, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("o"), py::arg("dout"),
         py::arg("lse"), py::arg("dq"), py::arg("dk"), py::arg("dv"), py::arg("scale"), py::arg("causal"),
         py::arg("causal_offset"), py::arg("dropout_p") = 0.0, py::arg("seed") = 0, py::arg("head_offset") = 0);

@@ -47,6 +47,8 @@ struct FwdParams {
   int causal;
   int causal_offset;  // query i attends keys <= i + causal_offset (Sk - Sq for bottom-right alignment)
   DropoutArgs drop;   // DROP variants only
+  const int* cu;      // PACKED: [B + 1], sequence b has rows cu[b] .. cu[b + 1] of the `rows` of q, k, v and o (Sq, Sk: the most of a sequence)
+  int rows;
 };
 
 // 16-byte chunk swizzle of a [rows][D] bf16 LDS image (D/8 chunks per row).
@@ -102,7 +104,9 @@ __device__ __forceinline__ float xor32(float x, bool is_max) {
 // DROP: dropout on the probabilities (reference NKI flash_fwd dropout_p / seed): the row sum l and
 // the LSE use the undropped P, the P.V operand is P * keep / (1 - p); the lane's query row hash is
 // computed once, each score costs one more hash.
-template <int D, int W, bool DROP>
+// PACKED: sequences of different lengths one after the other, without padding (a batch of prompts); workgroups past the end of their sequence leave.  What a
+// batch gains is its products: Llama-3.2-1B, 3 prompts of 350 to 700 tokens, 2,304 rows with padding (to 768) and 1,664 without, 5,337 -> 4,237 us.
+template <int D, int W, bool DROP, bool PACKED = false>
 __global__ void __launch_bounds__(W * 64, 8 / W) fwd_kernel(FwdParams p) {
   constexpr int kWaves = W;
   constexpr int kBlockM = W * 32;                 // q rows per workgroup
@@ -128,12 +132,20 @@ __global__ void __launch_bounds__(W * 64, 8 / W) fwd_kernel(FwdParams p) {
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int r = lane & 31, hh = lane >> 5;
   const int qb0 = mblk * kBlockM;
+  int64_t at_b = b;   // the sequence's place: times the strides of a batch, or (PACKED) of a row
+  if constexpr (PACKED) {
+    const int first = min(max(p.cu[b], 0), p.rows);
+    at_b = first;
+    p.Sq = p.Sk = min(p.Sq, min(p.cu[b + 1], p.rows) - first);
+    p.q_sb = p.q_ss, p.k_sb = p.k_ss, p.v_sb = p.v_ss, p.o_sb = p.o_ss;
+    if (qb0 >= p.Sq) return;
+  }
   const int q0 = qb0 + w * 32;  // this wave's first row
   const int my_q = q0 + r;
 
-  const uint16_t* qbase = p.q + (int64_t)b * p.q_sb + (int64_t)hq * p.q_sh;
-  const uint16_t* kbase = p.k + (int64_t)b * p.k_sb + (int64_t)hkv * p.k_sh;
-  const uint16_t* vbase = p.v + (int64_t)b * p.v_sb + (int64_t)hkv * p.v_sh;
+  const uint16_t* qbase = p.q + at_b * p.q_sb + (int64_t)hq * p.q_sh;
+  const uint16_t* kbase = p.k + at_b * p.k_sb + (int64_t)hkv * p.k_sh;
+  const uint16_t* vbase = p.v + at_b * p.v_sb + (int64_t)hkv * p.v_sh;
 
   // ---- Q fragments (B operand of S^T = K Q^T): lane (r, hh) holds Q[q0+r][16s + 8hh .. +7]
   bf16x8_t qf[KS];
@@ -353,7 +365,7 @@ __global__ void __launch_bounds__(W * 64, 8 / W) fwd_kernel(FwdParams p) {
   // ---- epilogue: O[q][d] = acc / l ; lse
   if (my_q < p.Sq) {
     const float inv = l_i > 0.f ? 1.f / l_i : 0.f;
-    uint16_t* orow = p.o + (int64_t)b * p.o_sb + (int64_t)my_q * p.o_ss + (int64_t)hq * p.o_sh;
+    uint16_t* orow = p.o + at_b * p.o_sb + (int64_t)my_q * p.o_ss + (int64_t)hq * p.o_sh;
 #pragma unroll
     for (int db = 0; db < NDB; ++db) {
 #pragma unroll
@@ -377,7 +389,7 @@ __global__ void __launch_bounds__(W * 64, 8 / W) fwd_kernel(FwdParams p) {
 int flash_attn_fwd_launch(const void* q, const void* k, const void* v, void* o, float* lse,
                           const int64_t* qs, const int64_t* ks, const int64_t* vs, const int64_t* os,
                           int B, int Sq, int Sk, int Hq, int Hkv, int D, float softmax_scale,
-                          int causal, int causal_offset, const DropoutArgs& drop, hipStream_t stream) {
+                          int causal, int causal_offset, const DropoutArgs& drop, hipStream_t stream, const int* cu, int rows) {
   using namespace fa;
   FwdParams p{};
   p.q = (const uint16_t*)q;
@@ -394,6 +406,8 @@ int flash_attn_fwd_launch(const void* q, const void* k, const void* v, void* o, 
   p.causal = causal;
   p.causal_offset = causal_offset;
   p.drop = drop;
+  p.cu = cu;
+  p.rows = rows;
   if (Hkv <= 0 || Hq % Hkv != 0) return -1;
   if (D != 128 && D != 64) return -2;
   // 8-wave workgroups (256 query rows: half the K/V tile traffic and barriers per row) while the
@@ -402,12 +416,21 @@ int flash_attn_fwd_launch(const void* q, const void* k, const void* v, void* o, 
   // 574-587 / 406-417 TF/s before the XCD map, 955-966 TF/s with it; the non-pipelined body, per-
   // cluster s_setprio, a 3-stage LDS ring and 128-key tiles measured neutral or slower (removed).
   const bool w8 = ((Sq + 255) / 256) * B * Hq >= 512;
-  const int rows = w8 ? 256 : 128;
-  const int grid = ((Sq + rows - 1) / rows) * B * Hq;
+  const int block = w8 ? 256 : 128;
+  const int grid = ((Sq + block - 1) / block) * B * Hq;
   if (grid == 0) return 0;
   const size_t lds = 2 * 2 * kBlockN * D * 2;
 #define NXD_FA_LAUNCH(DD, WW, DR) hipLaunchKernelGGL((fwd_kernel<DD, WW, DR>), dim3(grid), dim3(WW * 64), lds, stream, p)
-  if (drop.enabled()) {
+  if (cu) {
+    if (drop.enabled() || lse) return -3;
+    if (D == 128) {
+      if (w8) hipLaunchKernelGGL((fwd_kernel<128, 8, false, true>), dim3(grid), dim3(512), lds, stream, p);
+      else hipLaunchKernelGGL((fwd_kernel<128, 4, false, true>), dim3(grid), dim3(256), lds, stream, p);
+    } else {
+      if (w8) hipLaunchKernelGGL((fwd_kernel<64, 8, false, true>), dim3(grid), dim3(512), lds, stream, p);
+      else hipLaunchKernelGGL((fwd_kernel<64, 4, false, true>), dim3(grid), dim3(256), lds, stream, p);
+    }
+  } else if (drop.enabled()) {
     if (D == 128) {
       if (w8) NXD_FA_LAUNCH(128, 8, true); else NXD_FA_LAUNCH(128, 4, true);
     } else {

@@ -518,6 +518,30 @@ __global__ void __launch_bounds__(1024) topk_sample_kernel(const T* __restrict__
   }
 }
 
+// Prompts of a batch without their padding, one after the other: row r is token r - start of its sequence; rows past the last token have the
+// id 0, a position the tables have and no place in the cache (pos0 -1).  cu [B + 1]: where the sequences start.
+__global__ void __launch_bounds__(256) pack_prompts_kernel(const int64_t* __restrict__ ids, int64_t ld, const int64_t* __restrict__ lens,
+                                                          const int* __restrict__ slots, int B, int T, int R, int64_t* __restrict__ out_ids,
+                                                          int64_t* __restrict__ pos, int* __restrict__ pos0, int* __restrict__ row_slot,
+                                                          int* __restrict__ cu) {
+  const int r = blockIdx.x * 256 + threadIdx.x;
+  const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+  int start = 0, mine = -1, at = 0;
+  for (int b = 0; b < B; ++b) {
+    const int64_t len = lens[b];
+    const int n = min(len < 0 ? 0 : len > T ? T : (int)len, R - start);
+    if (r >= start && r < start + n) mine = b, at = r - start;
+    if (first) cu[b] = start;
+    start += n;
+  }
+  if (first) cu[B] = start;
+  if (r >= R) return;
+  out_ids[r] = mine >= 0 ? ids[(int64_t)mine * ld + at] : 0;
+  pos[r] = at;
+  pos0[r] = mine >= 0 ? at : -1;
+  row_slot[r] = mine >= 0 ? slots[mine] : 0;
+}
+
 }  // namespace dec
 
 int decode_attn2_launch(const void*, const int64_t*, const void*, const void*, const int64_t*, const int*, const int*,
@@ -586,6 +610,14 @@ int decode_attn_launch(const void* q, const int64_t* qs, const void* kc, const v
       hipLaunchKernelGGL(merge_kernel<128>, dim3(B * Hkv), dim3(256), mlds, stream, p, (uint16_t*)out, os[0], os[1], os[2]);
     }
   }
+  return (int)hipGetLastError();
+}
+
+int pack_prompts_launch(const int64_t* ids, int64_t ld, const int64_t* lens, const int* slots, int B, int T, int R, int64_t* out_ids, int64_t* pos,
+                        int* pos0, int* row_slot, int* cu, hipStream_t stream) {
+  if (B <= 0 || R <= 0) return -1;
+  hipLaunchKernelGGL(dec::pack_prompts_kernel, dim3((unsigned)((R + 255) / 256)), dim3(256), 0, stream, ids, ld, lens, slots, B, T, R, out_ids, pos, pos0,
+                     row_slot, cu);
   return (int)hipGetLastError();
 }
 

@@ -37,15 +37,33 @@ def select_bucket(length: int, buckets: Sequence[int]) -> int:
 HALFWAY_TOKENS = 1024
 
 
+def generated(config) -> bool:
+    """Whether the configuration's buckets are the generated ones."""
+    top = getattr(config, "max_context_length", 0)
+    return bool(getattr(config, "buckets_generated", False) and top and list(config.buckets) == generate_buckets(min(128, top), top))
+
+
 def prefill_lengths(config, batch: int, halfway: bool = True) -> List[int]:
     """Lengths that prompts of a batch are padded to: the configuration's buckets and its maximum length, and where the buckets are
     the generated ones (a caller's own list stands as it is) and `halfway` lengths may be used 1.5 times every bucket whose next one
     holds HALFWAY_TOKENS in the batch."""
     lengths = list(config.buckets)
-    top = getattr(config, "max_context_length", 0)
-    if halfway and getattr(config, "buckets_generated", False) and top and lengths == generate_buckets(min(128, top), top):
+    if halfway and generated(config):
         lengths += [lo * 3 // 2 for lo, hi in zip(lengths, lengths[1:]) if lo >= 128 and batch * hi >= HALFWAY_TOKENS and lo * 3 // 2 < hi]
     return lengths + [config.max_length]
+
+
+def packed_rows(total: int) -> int:
+    """Rows that `total` tokens of a batch are given where they lie one after the other: multiples of an eighth of the power of two below, of
+    128 at least.  Each is a graph of its own, so there are at most eight for twice the tokens."""
+    step = max(128, (1 << (total - 1).bit_length()) // 16)
+    return -(-total // step) * step
+
+
+def packing_pays(rows: int, batch: int, length: int) -> bool:
+    """Whether prompts are encoded without their padding, in so many rows instead of `batch` times `length`: an eighth fewer, which is more than reading the
+    lengths on the host costs (50 us of 3 to 10 ms)."""
+    return batch * length >= HALFWAY_TOKENS and 8 * rows <= 7 * batch * length
 
 
 def pad_to_bucket(input_ids: torch.Tensor, attention_mask: torch.Tensor, buckets: Sequence[int], pad_token: int):

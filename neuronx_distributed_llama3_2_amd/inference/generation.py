@@ -26,7 +26,7 @@ from ..parallel_layers import parallel_state as ps
 from ..parallel_layers.sharding import shard_state_dict
 from ..utils.logger import get_logger
 from ..utils.sampling import Sampler
-from .bucketing import pad_to_bucket, prefill_lengths
+from .bucketing import HALFWAY_TOKENS, generated, packed_rows, packing_pays, pad_to_bucket, prefill_lengths
 from .config import InferenceConfig
 from .graphs import DecodeGraph, DecodeState, decode_step
 from .modeling_llama import LlamaInferenceModel
@@ -80,6 +80,9 @@ class PrefillGraph:
         self.seq_ids = torch.arange(B, dtype=torch.int32, device=device)
         self.last = torch.full((B,), Tb - 1, dtype=torch.long, device=device)
         self.positions = torch.arange(Tb, device=device).unsqueeze(0).expand(B, Tb).contiguous()
+        self._capture(device, pool)
+
+    def _capture(self, device, pool):
         # warm-up on a side stream (GEMM autotuning, workspace allocation) before capture; it
         # writes KV-cache rows that the real prefill overwrites
         s = torch.cuda.Stream(device)
@@ -101,6 +104,21 @@ class PrefillGraph:
         self.last.copy_(last_index)
         self.graph.replay()
         return self.out
+
+
+class PackedPrefillGraph(PrefillGraph):
+    """The same without the prompts' padding: their tokens one after the other in `rows` rows, packed inside the graph from the padded
+    ids and the lengths."""
+
+    def __init__(self, model, B: int, Tb: int, rows: int, device, pool=None):
+        self.model, self.rows = model, rows
+        self.ids = torch.zeros((B, Tb), dtype=torch.long, device=device)
+        self.seq_ids = torch.arange(B, dtype=torch.int32, device=device)
+        self.last = torch.full((B,), -1, dtype=torch.long, device=device)   # (nothing is written to the cache before the first run)
+        self._capture(device, pool)
+
+    def _fwd(self):
+        return self.model.forward_packed(self.ids, self.last + 1, self.seq_ids, self.rows)
 
 
 class _SubModel:
@@ -325,6 +343,7 @@ class LlamaForCausalLMInference:
         dev = self.device
         input_ids = input_ids.to(dev)
         B, T = input_ids.shape
+        given = attention_mask
         if attention_mask is None:
             attention_mask = torch.ones_like(input_ids)
         attention_mask = attention_mask.to(dev)
@@ -339,7 +358,7 @@ class LlamaForCausalLMInference:
             logits = self.model.forward_tokens(ids, positions, seq_ids, prefill=True, lengths=lengths,
                                                logit_rows=want[:, 0] * Tb + want[:, 1])
         elif self._prefill_graphs_on():
-            logits = self._prefill_graph(B, Tb).run(ids, seq_ids, lengths - 1)
+            logits = self._prefill_graph(B, Tb, self._packed_rows(B, T, Tb, given)).run(ids, seq_ids, lengths - 1)
         else:
             positions = torch.arange(Tb, device=dev).unsqueeze(0).expand(B, Tb)
             logits = self.model.forward_tokens(ids, positions, seq_ids, last_index=lengths - 1, prefill=True)
@@ -373,14 +392,35 @@ class LlamaForCausalLMInference:
     def _prefill_graphs_on(self) -> bool:
         return getattr(self.config, "prefill_graphs", True) and self._graphs_allowed()
 
-    def _prefill_graph(self, B: int, Tb: int) -> "PrefillGraph":
+    def _packed_rows(self, B: int, T: int, Tb: int, mask: Optional[torch.Tensor]) -> int:
+        """Rows in which a batch of prompts is encoded without its padding; 0: as it is, padded.  Waits for the lengths where they are not known
+        and can matter."""
+        if not (self._halfway_lengths and generated(self.config) and self.model.packed_prefill_ok()) or B * Tb < HALFWAY_TOKENS:
+            return 0
+        if mask is None:
+            total = B * T
+        elif B == 1 and not packing_pays(packed_rows(T), 1, Tb) or mask.is_cuda and torch.cuda.is_current_stream_capturing():
+            return 0
+        else:
+            n = mask.sum(1).tolist()
+            if min(n) < 1 or max(n) > T:   # (no prompt, or no mask)
+                return 0
+            total = int(sum(n))
+        rows = packed_rows(total)
+        return rows if packing_pays(rows, B, Tb) else 0
+
+    def _prefill_graph(self, B: int, Tb: int, rows: int = 0) -> "PrefillGraph":
         """One captured context-encoding forward per (batch, bucket) -- the reference compiles one
         NEFF per bucket (trace/model_builder.py:380-451, SPMDBucketModel trace/spmd.py:32-61); here a
         hipGraph per bucket removes the per-kernel launch cost of prefill."""
-        key = (B, Tb)
+        key = (B, Tb, rows) if rows else (B, Tb)
         g = self._prefill_cache.get(key)
         if g is None:
-            g = self._prefill_cache[key] = PrefillGraph(self.model, B, Tb, self.device, self._prefill_pool)
+            if rows:
+                g = PackedPrefillGraph(self.model, B, Tb, rows, self.device, self._prefill_pool)
+            else:
+                g = PrefillGraph(self.model, B, Tb, self.device, self._prefill_pool)
+            self._prefill_cache[key] = g
             self._prefill_pool = g.pool
         return g
 

@@ -158,6 +158,42 @@ class DecoderInferenceMixin:
         logits = self._gather_vocab(self._proj(self.lm_head, h))
         return (logits, h) if return_hidden else logits
 
+    def packed_prefill_ok(self) -> bool:
+        """Whether forward_packed is for this model: a dense decoder whose tokens meet in its causal attention alone, on one GPU."""
+        cls, base = type(self), DecoderInferenceMixin
+        return (self.tp == 1 and cls.forward_tokens is base.forward_tokens and cls._qkv_hook is base._qkv_hook and cls._norm is base._norm
+                and self.head_dim in (64, 128) and self.model.embed_tokens.weight.dtype == torch.bfloat16
+                and all(self._fused_ffn_weights(layer) is not None for layer in self.model.layers))
+
+    @torch.no_grad()
+    def forward_packed(self, input_ids: torch.Tensor, lengths: torch.Tensor, slots: torch.Tensor, rows: int) -> torch.Tensor:
+        """Logits [B, V] of the last token of each prompt input_ids[b, :lengths[b]] (their sum is at most `rows`), whose keys and values go to
+        the cache rows slots[b]: forward_tokens(prefill=True) over the tokens that there are, one after the other.  int64
+        lengths, int32 slots; a length of 0 leaves the cache alone and gives logits of no token."""
+        C, dev = ops.ext(), input_ids.device
+        B, T = input_ids.shape
+        nq, nkv, D = self.nq, self.nkv, self.head_dim
+        ids, pos = (torch.empty(rows, dtype=torch.int64, device=dev) for _ in range(2))
+        place, slot = (torch.empty(rows, dtype=torch.int32, device=dev) for _ in range(2))
+        cu = torch.empty(B + 1, dtype=torch.int32, device=dev)
+        C.pack_prompts(input_ids, lengths, slots, ids, pos, place, slot, cu)
+        cos_t, sin_t = self.model.rope_cache.tables(dev)
+        x = ops.vocab_parallel_embedding(ids.view(1, rows), self.model.embed_tokens.weight, self.model.embed_tokens.start_index)
+        residual = None
+        for i, layer in enumerate(self.model.layers):
+            attn = layer.self_attn
+            h, residual = self._norm(x, layer.input_layernorm.weight, residual)
+            qkv = self._proj(attn.qkv_proj, h)
+            ops.rope_kv_write_(qkv.view(rows, 1, -1), nq, nkv, cos_t, sin_t, pos, self.kv_cache[i, 0], self.kv_cache[i, 1], place, slot)
+            heads = qkv.view(rows, nq + 2 * nkv, D)
+            o = ops.flash_attn_packed(heads[:, :nq], heads[:, nq:nq + nkv], heads[:, nq + nkv:], cu, min(T, rows))
+            x = self._row(attn.o_proj, o.view(1, rows, nq * D))
+            h, residual = self._norm(x, layer.post_attention_layernorm.weight, residual)
+            x = self._ffn(layer, h)
+        last = cu[1:].long() - 1
+        h, _ = self._norm(x[0, last], self.model.norm.weight, residual[0, last])
+        return self._proj(self.lm_head, h)
+
     def _forward_in_steps(self, input_ids, positions, seq_ids, last_index, return_hidden, lengths, logit_rows, step):
         """forward_tokens over the cache, `step` new tokens at a time."""
         B, T = input_ids.shape

@@ -13,7 +13,7 @@ from .experts import (RouterRule, Routing, clamped_glu, expert_linear_rows, expe
 from .group_norm import residual_norms  # noqa: F401
 from .grouped_gemm import (grouped_linear, grouped_linear_reference, moe_dispatch, moe_permutation,  # noqa: F401
                            moe_unpermute_combine)
-from .flash_attn import attention_reference, flash_attn_func, flash_attn_fwd_lse, rope_attention  # noqa: F401
+from .flash_attn import attention_reference, flash_attn_func, flash_attn_fwd_lse, flash_attn_packed, rope_attention  # noqa: F401
 from .hyper import decode_linear, decode_linear_into_streams, hyper_step, relu_squared, softcap_  # noqa: F401
 from .norm import rms_norm, rms_norm_reference  # noqa: F401
 from .optim import (adamw_flat_, clip_coefficient, flat_absmax, flat_sumsq, scale_flat_, sr_seed_for_step,  # noqa: F401

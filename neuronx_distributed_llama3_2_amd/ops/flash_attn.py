@@ -116,6 +116,21 @@ def flash_attn_fwd_lse(q, k, v, causal=True, softmax_scale=None, causal_offset=N
     return o, lse
 
 
+def flash_attn_packed(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu: torch.Tensor, most: int,
+                      softmax_scale: Optional[float] = None) -> torch.Tensor:
+    """Causal attention of sequences packed one after the other, forward only: q [R, Hq, D], k, v [R, Hkv, D], sequence b at rows
+    cu[b] .. cu[b + 1] (int32 [B + 1] on the device), at most `most` of them.  Rows of no sequence are left as they come."""
+    scale = softmax_scale if softmax_scale is not None else 1.0 / math.sqrt(q.shape[-1])
+    o = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+    if use_native(q, k, v):
+        ext().flash_attn_packed(q, k, v, o, cu, int(most), float(scale))
+        return o
+    for a, b in zip(cu.tolist(), cu[1:].tolist()):
+        if b > a:
+            o[a:b] = attention_reference(q[None, a:b], k[None, a:b], v[None, a:b], True, scale, 0)[0][0].to(o.dtype)
+    return o
+
+
 # --------------------------------------------------------------------------------------------
 # fused RoPE + attention core over a [S, B, (Hq + 2Hkv) * D] QKV projection output
 # --------------------------------------------------------------------------------------------
