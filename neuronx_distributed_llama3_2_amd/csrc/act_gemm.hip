@@ -4,10 +4,16 @@
 // leave them, take the activation on their way out.  The loop is that of gemm_tile.h (4 waves, 256 x 256 tile, one workgroup a CU, clock- and
 // feed-bound); reductions are not split, so the sums are in the order of the reduction.
 //
-// The tiles are dealt to the XCDs in equal runs of an L2 band raster.  What is left of a run after whole rounds of its 32 CUs would keep a few CUs for
+// The tiles are dealt to the XCDs in equal runs of an L2 band raster, in rounds of its 32 CUs.  What is left of a run after whole rounds would keep a few CUs for
 // a whole tile's time, so these tiles are cut into 2 or 4 pieces of 128 or 64 rows when all CUs can have one.
-// Against a library product and the activation's own launch, us, weights from memory: SwiGLU of 8,192 columns, reduction 2,048: 1,024 rows 68 -> 62, 2,304 150 ->
-// 152 (147 on another card), 4,096 232 -> 231; squared ReLU of 12,288, 2,048: 1,024 rows 60 -> 60, 4,096 182 -> 170 (1.2 PFLOP/s, the product alone at 1.4 in the library).
+// A workgroup has up to four tiles of rounds one after the other.  The ring of steps goes on from one to the next: during the last two steps of a tile the next one's
+// first two are loaded, and its first sums need no registers cleared, so that a round costs no launch of workgroups, no first trip to memory and no wait for its stores, which
+// are left in flight.  Results go out of the
+// registers, 64 contiguous bytes of 16 rows a store; SwiGLU's gates and the columns they go with are in one wave for that.  (No more than four, so that CUs that
+// something else holds keep no more than that waiting.)
+// One tile a workgroup, results through LDS / now, us, one card in turn: SwiGLU of 8,192 columns, reduction 2,048: 2,304 rows 133 / 123; squared ReLU of 12,288, 2,048, 4,096 rows
+// 154 / 143; rounds of 256 tiles of 512 20.4 / 16.9 each, of 2,048 51 / 47.5.
+// Against a library product and the activation's own launch: act_pays in ops/gemm.py.
 // The products are the library's to the bit there (its unsplit kernels sum in the same order).  Fewer rows: the library, with smaller tiles.
 #include "gemm_tile.h"
 
@@ -28,79 +34,127 @@ struct Params {
 };
 
 constexpr int XCDS = 8, XCD_CUS = 32, BAND = 8;   // row tiles of a band
+constexpr int RUN = 4;                            // tiles of a workgroup at most
 
-// of so many tiles of an XCD: those of whole rounds, and the pieces of each one left
-__host__ __device__ inline int whole_of(int share) { return share / XCD_CUS * XCD_CUS; }
-__host__ __device__ inline int pieces_of(int tail) { return 4 * tail <= XCD_CUS ? 4 : 2 * tail <= XCD_CUS ? 2 : 1; }
+// An XCD's share of so many tiles, in rounds of its CUs: what is left after whole rounds is cut into 2 or 4 pieces of a tile when all CUs can have
+// one (`cut` tiles), else it is a round too
+struct Share {
+  int tiles, rounds, cut, pieces;
+  __host__ __device__ explicit Share(int tiles_) : tiles(tiles_) {
+    const int tail = tiles % XCD_CUS;
+    pieces = 4 * tail <= XCD_CUS ? 4 : 2 * tail <= XCD_CUS ? 2 : 1;
+    cut = pieces > 1 ? tail : 0;
+    rounds = (tiles - cut + XCD_CUS - 1) / XCD_CUS;
+  }
+  __host__ __device__ int runs(bool pipe) const { return pipe ? (rounds + RUN - 1) / RUN : rounds; }
+  __host__ __device__ int workgroups(bool pipe) const { return runs(pipe) * XCD_CUS + cut * pieces; }
+};
 
-template <int ACT, bool HALF>
+// PIPE (whole steps, two or more): a workgroup has up to RUN tiles, of rounds one after the other, and loads the next one's first steps during the last ones of a
+// tile: its results go out of the registers while those are on their way.
+template <int ACT, bool HALF, bool PIPE>
 __global__ void __launch_bounds__(tile::THREADS, 1) kernel(Params p) {
   __shared__ __attribute__((aligned(16))) char smem[tile::LDS_BYTES];
   constexpr int COLS = ACT == SWIGLU ? BN / 2 : BN;   // results of a row
   const int total = p.rt * p.ct, xcd = blockIdx.x % XCDS, idx = blockIdx.x / XCDS;
-  const int share = total / XCDS + (xcd < total % XCDS), base = xcd * (total / XCDS) + min(xcd, total % XCDS);
-  const int whole = whole_of(share), tail = share - whole;
-  int pieces = 1, piece = 0, id = base + idx;
-  if (idx >= whole) {
-    pieces = pieces_of(tail);
-    const int j = idx - whole;
-    if (j >= tail * pieces) return;
-    piece = j % pieces;
-    id = base + whole + j / pieces;
+  const int base = xcd * (total / XCDS) + min(xcd, total % XCDS);
+  const Share share(total / XCDS + (xcd < total % XCDS));
+  const int run = idx / XCD_CUS, runs = share.runs(PIPE);
+  int items, first, pieces = 1, piece = 0;   // tiles of this workgroup, the XCD_CUS-th one after the other
+  if (run < runs) {
+    first = run * (PIPE ? RUN : 1) * XCD_CUS + idx % XCD_CUS;
+    items = min(PIPE ? RUN : 1, (share.tiles - share.cut - first + XCD_CUS - 1) / XCD_CUS);
+  } else {
+    const int j = idx - runs * XCD_CUS;
+    pieces = share.pieces, piece = j % pieces, first = share.tiles - share.cut + j / pieces;
+    items = first < share.tiles ? 1 : 0;
   }
-  const int band = id / (BAND * p.ct), rem = id - band * BAND * p.ct, h = min(BAND, p.rt - band * BAND);
-  const int rows = BM / pieces, r0 = (band * BAND + rem % h) * BM + piece * rows, n0 = rem / h * COLS;
-  const int r1 = min(p.R, r0 + rows);
+  if (items <= 0) return;
+  int r0, r1, n0;
+  auto place = [&](int k) __attribute__((always_inline)) {   // of the workgroup's k-th tile
+    const int id = base + first + k * XCD_CUS, band = id / (BAND * p.ct), rem = id - band * BAND * p.ct, h = min(BAND, p.rt - band * BAND);
+    const int rows = BM / pieces;
+    r0 = __builtin_amdgcn_readfirstlane((band * BAND + rem % h) * BM + piece * rows), n0 = __builtin_amdgcn_readfirstlane(rem / h * COLS);
+    r1 = min(p.R, r0 + rows);
+  };
+  place(0);
   if (r0 >= r1) return;   // (a piece past the last row)
-  tile::Loop<false> loop(smem, p.x + (int64_t)r0 * p.K, p.K, r1 - r0, p.w + (int64_t)n0 * p.K, p.K, ACT == SWIGLU ? BN : min(BN, p.N - n0));
-  if (ACT == SWIGLU && loop.wid >= 2) {   // rows 128 .. of the weights' tile: the other half's (of whole tiles: N % 128 == 0)
+  const auto x = [&](int row) { return p.x + (int64_t)row * p.K; };
+  const auto w = [&](int row) { return p.w + (int64_t)row * p.K; };
+  const auto cols = [&](int col) { return ACT == SWIGLU ? BN : min(BN, p.N - col); };
+  tile::Loop<false> loop(smem, x(r0), p.K, r1 - r0, w(n0), p.K, cols(n0));
+  const int lane = loop.lane, wid = loop.wid, wm = loop.wm, wn = loop.wn;
+  // SwiGLU: a wave's 128 columns are 64 gates and the 64 others that they are multiplied with (of whole tiles: N % 128 == 0), 64 rows of the image each
+  auto pairs = [&]() __attribute__((always_inline)) {
+    if (ACT == SWIGLU) {
+      const uint32_t by = (uint32_t)((wid & 1) * p.N + 64 * (wid >> 1) - 64 * wid) * (uint32_t)p.K * 2;
 #pragma unroll
-    for (int i = 8; i < 16; ++i) loop.off[i] += (uint32_t)(p.N - BN / 2) * (uint32_t)p.K * 2;
-  }
+      for (int i = 8; i < 16; ++i) loop.off[i] += by;
+    }
+  };
+  pairs();
   f32x4_t acc[8][8];
+  // a tile's results, rounded as the product leaves them, with the activation: 8 columns of a row a lane, 64 contiguous bytes of 16 rows a store
+  auto out = [&](auto ok) __attribute__((always_inline)) {
+    const int c0 = n0 + (ACT == SWIGLU ? 64 : 128) * wn + 8 * (lane >> 4);
+    uint16_t* y = p.y + (int64_t)(r0 + 16 * wm + (lane & 15)) * p.N + c0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+#pragma unroll
+      for (int j = 0; j < (ACT == SWIGLU ? 4 : 8); j += 2) {
+        auto rounded = [&](int jj, float (&v)[8]) __attribute__((always_inline)) {
+          unpack8(u32x4_t{pack2bf(acc[i][jj][0], acc[i][jj][1]), pack2bf(acc[i][jj][2], acc[i][jj][3]), pack2bf(acc[i][jj + 1][0], acc[i][jj + 1][1]),
+                          pack2bf(acc[i][jj + 1][2], acc[i][jj + 1][3])}, v);
+        };
+        float v[8];
+        rounded(j, v);
+        if (ACT == SWIGLU) {
+          float u[8];
+          rounded(j + 4, u);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] = v[e] * (1.f / (1.f + __expf(-v[e]))) * u[e];
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] = v[e] > 0.f ? v[e] * v[e] : 0.f;
+        }
+        if (ok(r0 + 32 * i + 16 * wm + (lane & 15), c0 + 16 * j)) *reinterpret_cast<u32x4_t*>(y + (int64_t)32 * i * p.N + 16 * j) = pack8(v);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  const int steps = (p.K + BK - 1) / BK;
+  if (PIPE && pieces == 1) {
+    tile::Loop<false>::Frags<8> frags;
+    loop.template begin<8, false>(frags, steps, false);
+    int stores = 0;
+#pragma unroll 1
+    for (int k = 0; k < items; ++k) {
+      const int R0 = r0, R1 = r1, N0 = n0;
+      const bool another = k + 1 < items;
+      if (another) place(k + 1);
+      const int nr0 = r0, nr1 = r1, nn0 = n0;
+      loop.run_tile(acc, frags, steps, stores, another, [&]() __attribute__((always_inline)) {
+        loop.set(x(nr0), p.K, nr1 - nr0, w(nn0), p.K, cols(nn0));
+        pairs();
+      });
+      r0 = R0, r1 = R1, n0 = N0;
+      const bool whole = r1 - r0 == BM && n0 + COLS <= p.N;
+      if (whole) out([](int, int) { return true; });
+      else out([&](int row, int col) { return row < r1 && col < p.N; });
+      stores = !whole ? 0 : ACT == SWIGLU ? 16 : 32;
+      r0 = nr0, r1 = nr1, n0 = nn0;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (loads that nothing reads)
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < 8; ++i)
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  const int steps = (p.K + BK - 1) / BK;
-  if (r1 - r0 > BM / 2) loop.template run<8, HALF>(acc, steps, HALF);
+  if (!PIPE && r1 - r0 > BM / 2) loop.template run<8, HALF>(acc, steps, HALF);
   else if (r1 - r0 > BM / 4) loop.template run<4, HALF>(acc, steps, HALF);
   else loop.template run<2, HALF>(acc, steps, HALF);
-  const int lane = loop.lane, wid = loop.wid, wm = loop.wm, wn = loop.wn;
-
-  // ---- results through LDS, a wave's 128 x 128 in 32 KB of its own (16-byte chunks XORed with the row)
-  __syncthreads();
-  char* own = smem + wid * (tile::LDS_BYTES / 4);
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-#pragma unroll
-    for (int j = 0; j < 8; j += 2) {
-      const int r = 16 * i + (lane & 15), c = tile::col<false>(0, j, lane);
-      *reinterpret_cast<u32x4_t*>(own + r * 256 + 16 * ((c >> 3) ^ (r & 15))) =
-          u32x4_t{pack2bf(acc[i][j][0], acc[i][j][1]), pack2bf(acc[i][j][2], acc[i][j][3]),
-                  pack2bf(acc[i][j + 1][0], acc[i][j + 1][1]), pack2bf(acc[i][j + 1][2], acc[i][j + 1][3])};
-    }
-  if (ACT == SWIGLU) __syncthreads();   // a wave takes half the rows of its gates and of its neighbour's columns (or the other way round)
-  else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  const char* gate = ACT == SWIGLU ? smem + (wid & ~1) * (tile::LDS_BYTES / 4) : own;
-  const int c0 = (ACT == SWIGLU ? 0 : 128 * wn) + 8 * (lane & 15);
-#pragma unroll 4
-  for (int k = 0; k < (ACT == SWIGLU ? 16 : 32); ++k) {
-    const int r = 4 * (ACT == SWIGLU ? 16 * wn + k : k) + (lane >> 4), row = r0 + 32 * (r >> 4) + 16 * wm + (r & 15);
-    const char* at = gate + r * 256 + 16 * ((lane & 15) ^ (r & 15));
-    float v[8];
-    unpack8(*reinterpret_cast<const u32x4_t*>(at), v);
-    if (ACT == SWIGLU) {
-      float u[8];
-      unpack8(*reinterpret_cast<const u32x4_t*>(at + tile::LDS_BYTES / 4), u);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = v[e] * (1.f / (1.f + __expf(-v[e]))) * u[e];
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = v[e] > 0.f ? v[e] * v[e] : 0.f;
-    }
-    if (row < r1 && n0 + c0 < p.N) *reinterpret_cast<u32x4_t*>(p.y + (int64_t)row * p.N + n0 + c0) = pack8(v);
-  }
+  out([&](int row, int col) { return row < r1 && col < p.N; });
 }
 
 }  // namespace act
@@ -116,14 +170,14 @@ int act_gemm_launch(int act, const void* x, const void* w, void* y, int64_t R, i
                 (int)ceil_div64(R, tile::BM), (int)ceil_div64(N, act ? tile::BN : tile::BN / 2)};
   const int64_t total = (int64_t)p.rt * p.ct;
   if (total > INT32_MAX / 64) return -1;
+  const bool half = K % tile::BK != 0, pipe = !half && K >= 2 * tile::BK;
   int most = 0;
-  for (int share : {(int)(total / act::XCDS), (int)ceil_div64(total, act::XCDS)}) {
-    const int whole = act::whole_of(share), tail = share - whole, n = whole + tail * act::pieces_of(tail);
+  for (int64_t tiles : {total / act::XCDS, ceil_div64(total, act::XCDS)}) {
+    const int n = act::Share((int)tiles).workgroups(pipe);
     most = n > most ? n : most;
   }
-  const bool half = K % tile::BK != 0;
-  auto* f = act ? (half ? &act::kernel<act::RELU2, true> : &act::kernel<act::RELU2, false>)
-                : (half ? &act::kernel<act::SWIGLU, true> : &act::kernel<act::SWIGLU, false>);
+  auto* f = act ? (half ? &act::kernel<act::RELU2, true, false> : pipe ? &act::kernel<act::RELU2, false, true> : &act::kernel<act::RELU2, false, false>)
+                : (half ? &act::kernel<act::SWIGLU, true, false> : pipe ? &act::kernel<act::SWIGLU, false, true> : &act::kernel<act::SWIGLU, false, false>);
   hipLaunchKernelGGL(f, dim3((unsigned)most * act::XCDS), dim3(tile::THREADS), 0, stream, p);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }

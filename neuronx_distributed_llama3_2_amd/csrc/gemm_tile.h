@@ -80,15 +80,24 @@ __device__ __forceinline__ void each(F&& f) {   // f(0), .. f(N - 1), each numbe
 }
 
 // One product, and one with a load (64 lanes x 16 B: base + at -> LDS lds + MORE + 16 lane): it stands between m0 and the load that reads it.
+// ZERO: the first product of a sum, whatever the registers hold.
+template <bool ZERO = false>
 __device__ __forceinline__ void mfma(f32x4_t& c, const bf16x8_t& b, const bf16x8_t& a) {
-  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(b), "v"(a));
+  if constexpr (ZERO) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(c) : "v"(b), "v"(a));
+  else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(b), "v"(a));
 }
-template <int MORE>
+template <int MORE, bool ZERO = false>
 __device__ __forceinline__ void mfma_load(f32x4_t& c, const bf16x8_t& b, const bf16x8_t& a, uint32_t at, const char* base, uint32_t lds) {
-  asm volatile("s_add_u32 m0, %5, %6\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0\n\tglobal_load_lds_dwordx4 %3, %4"
-               : "+a"(c)
-               : "v"(b), "v"(a), "v"(at), "s"(base), "s"(lds), "n"(MORE)
-               : "memory", "m0", "scc");
+  if constexpr (ZERO)
+    asm volatile("s_add_u32 m0, %5, %6\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, 0\n\tglobal_load_lds_dwordx4 %3, %4"
+                 : "=&a"(c)
+                 : "v"(b), "v"(a), "v"(at), "s"(base), "s"(lds), "n"(MORE)
+                 : "memory", "m0", "scc");
+  else
+    asm volatile("s_add_u32 m0, %5, %6\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0\n\tglobal_load_lds_dwordx4 %3, %4"
+                 : "+a"(c)
+                 : "v"(b), "v"(a), "v"(at), "s"(base), "s"(lds), "n"(MORE)
+                 : "memory", "m0", "scc");
 }
 // An address for reads to come, made where nothing waits for it
 __device__ __forceinline__ void move_to(int& at, int base, int by) { asm volatile("v_add_u32 %0, %1, %2" : "=v"(at) : "s"(by), "v"(base)); }
@@ -111,21 +120,26 @@ struct Loop {
   __device__ __forceinline__ Loop(char* smem_, const uint16_t* a, int64_t lda, int rows, const uint16_t* b, int64_t ldb, int cols) : smem(smem_) {
     lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wid >> 1, wn = wid & 1;
     lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+    set(a, lda, rows, b, ldb, cols);
+  }
+  __device__ __forceinline__ void set(const uint16_t* a, int64_t lda, int rows, const uint16_t* b, int64_t ldb, int cols) {   // the tile that is loaded from now on
     pa = uniform(reinterpret_cast<const char*>(a)), pb = uniform(reinterpret_cast<const char*>(b));
     da = BK * 2, db = BT ? (int64_t)BK * ldb * 2 : BK * 2;
     back = 0, pieces = min(max((rows + 7) / 8 - 8 * wid, 0), 8);
+    int lane = this->lane;
+    asm volatile("" : "+v"(lane));   // (made anew for each tile: kept, what does not change takes the registers of a loop around this one)
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const bool tr = i >= 8 && BT;
       const int piece = 8 * wid + (i & 7), n = i < 8 ? rows : cols;
-      const int64_t ld = i < 8 ? lda : ldb;
+      const uint32_t ld = (uint32_t)(i < 8 ? lda : ldb);   // (offsets have 32 bits)
       if (tr) {
         const int t = 2 * piece + (lane >> 5), c = (lane & 31) ^ tr_swz(t);
-        off[i] = (uint32_t)(t * ld + min(8 * c, n - 8)) * 2;
+        off[i] = ((uint32_t)t * ld + (uint32_t)min(8 * c, n - 8)) * 2;
         if (t >= BK / 2) back |= 1u << i;
       } else {
         const int row = 8 * piece + (lane >> 3), c = (lane & 7) ^ row_swz(row);
-        off[i] = (uint32_t)(min(row, n - 1) * ld + 8 * c) * 2;
+        off[i] = ((uint32_t)min(row, n - 1) * ld + (uint32_t)(8 * c)) * 2;
         if (c >= 4) back |= 1u << i;
       }
     }
@@ -188,100 +202,139 @@ struct Loop {
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
 
-  // acc += the products of so many steps.  IM: row fragments that have rows.  HALF, end: the last step has half the reduction.
-  template <int IM, bool HALF>
-  __device__ __forceinline__ void run(f32x4_t (&acc)[8][8], int steps, bool end) {
-    static_assert(IM == 8 || IM == 4 || IM == 2, "rows");
-    constexpr bool FEW = IM < 8;   // only rows that there are (what the LDS holds in the others' place counts for no result)
+  // Fragments of the two halves of a step, and where its images lie: A's go round three places, B's take turns
+  template <int IM>
+  struct Frags {
     bf16x8_t a0[IM], b0[8], a1[IM], b1[8];
-    auto advance_a = [&](int s) {   // towards step s
-      if (s < steps) pa += da;
-    };
-    auto advance_b = [&](int s) {
-      if (s < steps) pb += db;
-    };
+    int a_now = 0, a_next = IMG_BYTES, a_free = 2 * IMG_BYTES, b_now = 0;
+  };
+  __device__ __forceinline__ void advance_a(bool there) {   // towards the next step, if there is one
+    if (there) pa += da;
+  }
+  __device__ __forceinline__ void advance_b(bool there) {
+    if (there) pb += db;
+  }
+  // The loads of the first two of so many steps, and the first half's fragments
+  template <int IM, bool HALF>
+  __device__ __forceinline__ void begin(Frags<IM>& f, int steps, bool end) {
+    constexpr bool FEW = IM < 8;
 #pragma unroll
     for (int i = 0; i < 16; ++i) load<HALF, FEW>(i, 0, end && steps == 1);
-    advance_a(1), advance_b(1);
+    advance_a(1 < steps), advance_b(1 < steps);
 #pragma unroll
     for (int i = 0; i < 16; ++i) load<HALF, FEW>(i, IMG_BYTES, end && steps <= 2);   // (past the end: the last step again, not used)
-    advance_a(2), advance_b(2);
+    advance_a(2 < steps), advance_b(2 < steps);
     addresses();
     if (FEW) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");   // (B's pieces of the second step are 8 in every wave)
     else asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 #pragma unroll
-    for (int j = 0; j < 8; ++j) b0[j] = frag_b(j, 0), fixed();   // (in this order: the loop's waits count what came later)
+    for (int j = 0; j < 8; ++j) f.b0[j] = frag_b(j, 0), fixed();   // (in this order: the loop's waits count what came later)
 #pragma unroll
-    for (int i = 0; i < IM; ++i) a0[i] = frag_a(i, 0), fixed();
-    // A half step: its products, and between two of them at most a read of the next half's fragments (k: B's, then A's), an address or a load.  A
-    // wave is alone on its SIMD: what stands between two products beyond the 12 cycles that the first leaves free, or waits for what stands just
-    // before it, the matrix cores wait for.
+    for (int i = 0; i < IM; ++i) f.a0[i] = frag_a(i, 0), fixed();
+  }
+  // One step: two halves, each its products, and between two of them at most a read of the next half's fragments (k: B's, then A's), an address or a load.  A
+  // wave is alone on its SIMD: what stands between two products beyond the 12 cycles that the first leaves free, or waits for what stands just
+  // before it, the matrix cores wait for.  ZERO: the first of its sums; last: what is loaded is the last step, of half the reduction; more: there is a step
+  // after the one that is loaded; wait(): its turn's loads have come.
+  template <int IM, bool HALF, bool ZERO, typename WAIT>
+  __device__ __forceinline__ void step(f32x4_t (&acc)[8][8], Frags<IM>& f, bool last, bool more, WAIT&& wait) {
+    constexpr bool FEW = IM < 8;   // only rows that there are (what the LDS holds in the others' place counts for no result)
     constexpr int M = 8 * IM, READS = 8 + IM;
     constexpr int RD = IM == 2 ? 1 : 2, LD = IM == 2 ? 2 : 4;   // products from one read, or load, to the next
     // from there on the addresses of B move, their reads of a first half all out (or, with 8 in the 16 products of IM == 2, those of rb[k] from FREE + k on)
     constexpr int FREE = IM == 2 && BT ? 8 : RD * READS, SP = (M - FREE) / NB;
-    int a_now = 0, a_next = IMG_BYTES, a_free = 2 * IMG_BYTES, b_now = 0;
-    const uint32_t mine = lds + wid * 8192;
+    const uint32_t mine = lds + wid * 8192, to_a = mine + f.a_free, to_b = mine + f.b_now;
+    const int b_by = f.b_now ? -IMG_BYTES : IMG_BYTES;
+    each<M>([&](auto mc) __attribute__((always_inline)) {
+      constexpr int m = mc, k = m / RD, l = m / LD;
+      f32x4_t& c = acc[m >> 3][m & 7];
+      if constexpr (m % RD == RD - 1 && k < READS) {   // (one of B's and one of A's in turn)
+        if constexpr (k < 2 * IM && k % 2 == 1) f.a1[k >> 1] = frag_a(k >> 1, 1);
+        else f.b1[k < 2 * IM ? k >> 1 : k - IM] = frag_b(k < 2 * IM ? k >> 1 : k - IM, 1);
+        fixed();
+      }
+      if constexpr (m >= FREE && (m - FREE) % SP == 0) move_by(rb[(m - FREE) / SP], b_by), fixed();
+      if constexpr (m == M - 1) move_to(ra[0], base_a[0], f.a_next), fixed();
+      if constexpr (!FEW && m == 36) advance_a(more), fixed();
+      if constexpr (!FEW && m % LD == LD / 2 && l < 8) {
+        mfma_load<l * 1024, ZERO>(c, f.b0[m & 7], f.a0[m >> 3], from<HALF>(l, last), pa, to_a);
+      } else {
+        if constexpr (m % LD == LD / 2 && l < 8) load<HALF, FEW>(l, f.a_free, last);
+        mfma<ZERO>(c, f.b0[m & 7], f.a0[m >> 3]);
+      }
+      fixed();
+    });
+    if (FEW) advance_a(more);
+    reads_done();
+    wait();
+    __builtin_amdgcn_s_barrier();
+    fixed();
+    each<M>([&](auto mc) __attribute__((always_inline)) {
+      constexpr int m = mc, RD2 = IM == 8 ? 4 : RD, k = m / RD2, l = m / LD;
+      f32x4_t& c = acc[m >> 3][m & 7];
+      if constexpr (m % RD2 == RD2 / 2 && k < READS) {
+        if constexpr (k < 8) f.b0[k] = frag_b(k, 0);
+        else f.a0[k - 8] = frag_a(k - 8, 0);
+        fixed();
+      }
+      if constexpr (m == 0) move_to(ra[1], base_a[1], f.a_next), fixed();
+      if constexpr (!FEW && m == 36) advance_b(more), fixed();
+      if constexpr (m % LD == LD - 1 && l < 8) mfma_load<B_BASE + l * 1024>(c, f.b1[m & 7], f.a1[m >> 3], from<HALF>(8 + l, last), pb, to_b);
+      else mfma(c, f.b1[m & 7], f.a1[m >> 3]);
+      fixed();
+    });
+    if (FEW) advance_b(more);
+    f.b_now ^= IMG_BYTES;
+    const int freed = f.a_now;
+    f.a_now = f.a_next, f.a_next = f.a_free, f.a_free = freed;
+  }
+
+  // acc += the products of so many steps.  IM: row fragments that have rows.  HALF, end: the last step has half the reduction.
+  template <int IM, bool HALF>
+  __device__ __forceinline__ void run(f32x4_t (&acc)[8][8], int steps, bool end) {
+    static_assert(IM == 8 || IM == 4 || IM == 2, "rows");
+    Frags<IM> f;
+    begin<IM, HALF>(f, steps, end);
 #pragma unroll 1
     for (int t = 0, whole = steps - (HALF && end); t < whole; ++t) {
       asm volatile("s_nop 3");   // (after moves of the sums ahead of the loop)
-      const bool last = end && t + 3 >= steps;
-      const uint32_t to_a = mine + a_free, to_b = mine + b_now;
-      const int b_by = b_now ? -IMG_BYTES : IMG_BYTES;
-      each<M>([&](auto mc) __attribute__((always_inline)) {
-        constexpr int m = mc, k = m / RD, l = m / LD;
-        f32x4_t& c = acc[m >> 3][m & 7];
-        if constexpr (m % RD == RD - 1 && k < READS) {   // (one of B's and one of A's in turn)
-          if constexpr (k < 2 * IM && k % 2 == 1) a1[k >> 1] = frag_a(k >> 1, 1);
-          else b1[k < 2 * IM ? k >> 1 : k - IM] = frag_b(k < 2 * IM ? k >> 1 : k - IM, 1);
-          fixed();
-        }
-        if constexpr (m >= FREE && (m - FREE) % SP == 0) move_by(rb[(m - FREE) / SP], b_by), fixed();
-        if constexpr (m == M - 1) move_to(ra[0], base_a[0], a_next), fixed();
-        if constexpr (!FEW && m == 36) advance_a(t + 3), fixed();
-        if constexpr (!FEW && m % LD == LD / 2 && l < 8) {
-          mfma_load<l * 1024>(c, b0[m & 7], a0[m >> 3], from<HALF>(l, last), pa, to_a);
-        } else {
-          if constexpr (m % LD == LD / 2 && l < 8) load<HALF, FEW>(l, a_free, last);
-          mfma(c, b0[m & 7], a0[m >> 3]);
-        }
-        fixed();
-      });
-      if (FEW) advance_a(t + 3);
-      reads_done();
-      wait_a<FEW>();
-      __builtin_amdgcn_s_barrier();
-      fixed();
-      each<M>([&](auto mc) __attribute__((always_inline)) {
-        constexpr int m = mc, RD2 = IM == 8 ? 4 : RD, k = m / RD2, l = m / LD;
-        f32x4_t& c = acc[m >> 3][m & 7];
-        if constexpr (m % RD2 == RD2 / 2 && k < READS) {
-          if constexpr (k < 8) b0[k] = frag_b(k, 0);
-          else a0[k - 8] = frag_a(k - 8, 0);
-          fixed();
-        }
-        if constexpr (m == 0) move_to(ra[1], base_a[1], a_next), fixed();
-        if constexpr (!FEW && m == 36) advance_b(t + 3), fixed();
-        if constexpr (m % LD == LD - 1 && l < 8) mfma_load<B_BASE + l * 1024>(c, b1[m & 7], a1[m >> 3], from<HALF>(8 + l, last), pb, to_b);
-        else mfma(c, b1[m & 7], a1[m >> 3]);
-        fixed();
-      });
-      if (FEW) advance_b(t + 3);
-      b_now ^= IMG_BYTES;
-      const int freed = a_now;
-      a_now = a_next, a_next = a_free, a_free = freed;
+      step<IM, HALF, false>(acc, f, end && t + 3 >= steps, t + 3 < steps, [&]() { wait_a<(IM < 8)>(); });
       if (HALF) asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");   // (the sums may move after the loop)
     }
     if (HALF && end) {   // (s_nop: the sums may have moved to other registers just before)
 #pragma unroll
       for (int i = 0; i < IM; ++i)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) asm volatile("s_nop 3\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(b0[j]), "v"(a0[i]));
+        for (int j = 0; j < 8; ++j) asm volatile("s_nop 3\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(f.b0[j]), "v"(f.a0[i]));
     }
     asm volatile("s_waitcnt vmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");   // (loads that nothing reads; the last sums)
     settled<IM>(acc);
+  }
+
+  // acc = the products of one of several tiles, of so many whole steps each (2 or more), after begin() for the first one.  next(), if there is another one: the
+  // loads go over to it, two steps before the end, so that it begins without a wait.  stores: vector stores since the last tile, where all of them were made,
+  // else 0: the first step's loads came before them and are waited for alone.
+  template <typename NEXT>
+  __device__ __forceinline__ void run_tile(f32x4_t (&acc)[8][8], Frags<8>& f, int steps, int stores, bool another, NEXT&& next) {
+    const auto rest = [&](int t, int end) __attribute__((always_inline)) {   // towards step t + 3, or the next tile's t + 3 - steps
+#pragma unroll 1
+      for (; t < end; ++t)
+        step<8, false, false>(acc, f, false, t + 3 < steps || (another && t + 3 > steps && t + 3 < 2 * steps), [&]() { asm volatile("s_waitcnt vmcnt(8)" ::: "memory"); });
+    };
+    const int turn = steps - 2;
+    if (turn == 0 && another) next();
+    step<8, false, true>(acc, f, false, 3 < steps || (another && steps == 2), [&]() {
+      if (stores == 32) asm volatile("s_waitcnt vmcnt(40)" ::: "memory");
+      else if (stores == 16) asm volatile("s_waitcnt vmcnt(24)" ::: "memory");
+      else asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+    });
+    rest(1, turn);
+    if (turn > 0 && another) next();
+    rest(max(1, turn), steps);
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+    settled<8>(acc);
   }
 };
 

@@ -55,13 +55,13 @@ def act_pays(rows: int, weight_rows: int, K: int, glu: bool = False) -> bool:
     """Whether csrc/act_gemm.hip is faster than a library product and the activation's own pass: work for three quarters of the CUs (256 x 256
     results each), a reduction that the pass is not small beside, and rounds of the CUs that are filled to three quarters: what is left after whole rounds
     takes a whole one too, or, cut into 2 or 4 pieces, about two thirds of one (half of one if the pieces leave half of the CUs to themselves); up to a reduction of 1,024 the
-    pass is so large a part that this does not matter (SwiGLU of 8,192 at 1,280 rows 58 / 55).  us, two launches / one,
-    weights from memory: SwiGLU of 8,192 columns, reduction 2,048: 768 rows 54 / 57, 1,024 68 / 62, 2,304 150 / 152, 4,096 232 / 231; of 14,336, 4,096: 512 rows
-    111 / 109, 1,792 381 / 347, 5,120 1,001 / 912; of 11,008, 4,096: 4,096 694 / 579; of 28,672, 8,192: 2,304 rows 1,555 / 1,599; squared ReLU of 12,288, 2,048: 768 rows 46 /
-    51, 1,024 60 / 60, 4,096 182 / 170.  Rounds that are not filled (two launches): SwiGLU of 14,336, 4,096 at 640 rows 146 / 165, 24,576 at 640 240 / 265, 8,192 at 1,280 92 /
-    97, 11,008 at 896 161 / 170, squared ReLU of 16,384, 4,096 at 1,280 161 / 173.  The library does best where its tiles fill whole rounds too, and a long reduction hides SwiGLU's
-    pass: of 14,336, 4,096 at 4,096 / 12,288 rows 706 / 714, 2,100 / 2,150, of 24,576 at 3,072 / 10,240 926 / 944, 3,046 / 3,138 (two launches from four rounds on); of 8,192,
-    3,072 at 4,096 / 16,384 330 / 324, 1,254 / 1,251, squared ReLU of 16,384, 4,096 at 16,384 1,632 / 1,603."""
+    pass is so large a part that this does not matter (SwiGLU of 4,096 at 2,304 rows 53 / 43).  us, two launches / one,
+    weights from memory: SwiGLU of 8,192 columns, reduction 2,048: 768 rows 52 / 47, 1,024 64 / 53, 1,664 110 / 94, 2,304 144 / 132, 4,096 226 / 197; of 14,336, 4,096: 512 rows
+    108 / 94, 1,792 367 / 305, 5,120 977 / 799; of 11,008, 4,096: 4,096 681 / 507; squared ReLU of 12,288, 2,048: 640 rows 42 /
+    42, 1,024 55 / 44, 4,096 178 / 145.  Rounds that are not filled (two launches): SwiGLU of 14,336, 4,096 at 384 rows 92 / 96, 640 146 / 157, 1,152 239 / 240, 8,192 at 1,152 85 /
+    86, 3,072 at 1,280 121 / 126, 11,008 at 896 155 / 156, squared ReLU of 16,384, 4,096 at 1,280 150 / 156 (a part of a round below three quarters of it would pay in some places: 11,008 at
+    512 rows 93 / 82, squared ReLU of 12,288 at 896 50 / 44).  The library does best where its tiles fill whole rounds too, and a long reduction hides SwiGLU's
+    pass: there two launches stay, although they are the slower ones since a workgroup has several tiles: of 14,336, 4,096 at 4,096 / 12,288 rows 685 / 618, 2,047 / 1,886."""
     if K % 32 or K > 4096 or rows * weight_rows < 192 * 256 * 256:
         return False
     if K <= 1024:
