@@ -125,7 +125,7 @@ __global__ void __launch_bounds__(tile::THREADS, 1) kernel(Params p) {
   const int steps = (p.K + BK - 1) / BK;
   if (PIPE && pieces == 1) {
     tile::Loop<false>::Frags<8> frags;
-    loop.template begin<8, false>(frags, steps, false);
+    loop.template begin<false>(frags, steps, false);
     int stores = 0;
 #pragma unroll 1
     for (int k = 0; k < items; ++k) {

@@ -113,7 +113,8 @@ struct Loop {
   uint32_t off[16];        // of this lane's pieces of A (0 .. 7) and B from a step's base
   const char *pa, *pb;     // the bases of the next step to load
   int64_t da, db;          // ... and from one step to the next
-  int pieces;              // (ROW images) pieces of A with rows that there are
+  uint32_t ld_a;           // for run_few: A's row, and how many there are
+  int rows_a;
   uint32_t back;           // (reductions that end with half a step) pieces of the last step whose second half is past the end, a bit each
 
   // A: rows 0 .. rows - 1 from `a` on (ROW: a row is lda elements; TR: a reduction row), clamped to the last; B likewise
@@ -125,7 +126,7 @@ struct Loop {
   __device__ __forceinline__ void set(const uint16_t* a, int64_t lda, int rows, const uint16_t* b, int64_t ldb, int cols) {   // the tile that is loaded from now on
     pa = uniform(reinterpret_cast<const char*>(a)), pb = uniform(reinterpret_cast<const char*>(b));
     da = BK * 2, db = BT ? (int64_t)BK * ldb * 2 : BK * 2;
-    back = 0, pieces = min(max((rows + 7) / 8 - 8 * wid, 0), 8);
+    back = 0, ld_a = (uint32_t)lda, rows_a = rows;
     int lane = this->lane;
     asm volatile("" : "+v"(lane));   // (made anew for each tile: kept, what does not change takes the registers of a loop around this one)
 #pragma unroll
@@ -148,7 +149,7 @@ struct Loop {
   // fragment addresses: of A's first image by half, of A's images that are read now and of B's (ROW: [chunk bit 2], TR: [fragment])
   static constexpr int NB = BT ? 8 : 2;
   int base_a[2], ra[2], rb[NB];
-  __device__ __forceinline__ void addresses() {
+  __device__ __forceinline__ void addresses(int b_base) {
     const int r = lane & 15, g = lane >> 4;
     const int row = 16 * wm + r;
     base_a[0] = row * 128 + 16 * (g ^ row_swz(row));
@@ -156,11 +157,11 @@ struct Loop {
     ra[0] = base_a[0], ra[1] = base_a[1];
     if constexpr (BT) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) rb[j] = B_BASE + tr_at(128 * wn + 16 * j);
+      for (int j = 0; j < 8; ++j) rb[j] = b_base + tr_at(128 * wn + 16 * j);
     } else {
       const int c = 128 * wn + 8 * (r >> 2) + (r & 3);
-      rb[0] = B_BASE + c * 128 + 16 * (g ^ row_swz(c));
-      rb[1] = rb[0] ^ 64;   // (B_BASE is a multiple of 128)
+      rb[0] = b_base + c * 128 + 16 * (g ^ row_swz(c));
+      rb[1] = rb[0] ^ 64;   // (b_base is a multiple of 128)
     }
   }
   __device__ __forceinline__ int tr_at(int c0) const {   // lane 16 g + 4 q + p: 4 columns from c0 + 4 p on, of reduction rows 8 g + q (and + 4)
@@ -189,17 +190,9 @@ struct Loop {
     }
     return at;
   }
-  template <bool HALF, bool FEW>
+  template <bool HALF>
   __device__ __forceinline__ void load(int i, int img, bool last) const {
-    if (FEW && i < 8 && i >= pieces) return;
     load_lds(from<HALF>(i, last), i < 8 ? pa : pb, lds + (i < 8 ? 0 : B_BASE) + img + (8 * wid + (i & 7)) * 1024);
-  }
-  template <bool FEW>
-  __device__ __forceinline__ void wait_a() const {   // all loads but A's of the newest step have come
-    if (!FEW || pieces == 8) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-    else if (pieces >= 4) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-    else if (pieces >= 2) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
 
   // Fragments of the two halves of a step, and where its images lie: A's go round three places, B's take turns
@@ -215,94 +208,188 @@ struct Loop {
     if (there) pb += db;
   }
   // The loads of the first two of so many steps, and the first half's fragments
-  template <int IM, bool HALF>
-  __device__ __forceinline__ void begin(Frags<IM>& f, int steps, bool end) {
-    constexpr bool FEW = IM < 8;
+  template <bool HALF>
+  __device__ __forceinline__ void begin(Frags<8>& f, int steps, bool end) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) load<HALF, FEW>(i, 0, end && steps == 1);
+    for (int i = 0; i < 16; ++i) load<HALF>(i, 0, end && steps == 1);
     advance_a(1 < steps), advance_b(1 < steps);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) load<HALF, FEW>(i, IMG_BYTES, end && steps <= 2);   // (past the end: the last step again, not used)
+    for (int i = 0; i < 16; ++i) load<HALF>(i, IMG_BYTES, end && steps <= 2);   // (past the end: the last step again, not used)
     advance_a(2 < steps), advance_b(2 < steps);
-    addresses();
-    if (FEW) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");   // (B's pieces of the second step are 8 in every wave)
-    else asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+    addresses(B_BASE);
+    asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 #pragma unroll
     for (int j = 0; j < 8; ++j) f.b0[j] = frag_b(j, 0), fixed();   // (in this order: the loop's waits count what came later)
 #pragma unroll
-    for (int i = 0; i < IM; ++i) f.a0[i] = frag_a(i, 0), fixed();
+    for (int i = 0; i < 8; ++i) f.a0[i] = frag_a(i, 0), fixed();
   }
   // One step: two halves, each its products, and between two of them at most a read of the next half's fragments (k: B's, then A's), an address or a load.  A
   // wave is alone on its SIMD: what stands between two products beyond the 12 cycles that the first leaves free, or waits for what stands just
   // before it, the matrix cores wait for.  ZERO: the first of its sums; last: what is loaded is the last step, of half the reduction; more: there is a step
   // after the one that is loaded; wait(): its turn's loads have come.
-  template <int IM, bool HALF, bool ZERO, typename WAIT>
-  __device__ __forceinline__ void step(f32x4_t (&acc)[8][8], Frags<IM>& f, bool last, bool more, WAIT&& wait) {
-    constexpr bool FEW = IM < 8;   // only rows that there are (what the LDS holds in the others' place counts for no result)
-    constexpr int M = 8 * IM, READS = 8 + IM;
-    constexpr int RD = IM == 2 ? 1 : 2, LD = IM == 2 ? 2 : 4;   // products from one read, or load, to the next
-    // from there on the addresses of B move, their reads of a first half all out (or, with 8 in the 16 products of IM == 2, those of rb[k] from FREE + k on)
-    constexpr int FREE = IM == 2 && BT ? 8 : RD * READS, SP = (M - FREE) / NB;
+  template <bool HALF, bool ZERO, typename WAIT>
+  __device__ __forceinline__ void step(f32x4_t (&acc)[8][8], Frags<8>& f, bool last, bool more, WAIT&& wait) {
+    constexpr int M = 64, READS = 16, RD = 2, RD2 = 4, LD = 4;   // products; from one read (of the second half: RD2), or load, to the next
+    constexpr int FREE = RD * READS, SP = (M - FREE) / NB;       // from there on the addresses of B move, their reads of a first half all out
     const uint32_t mine = lds + wid * 8192, to_a = mine + f.a_free, to_b = mine + f.b_now;
     const int b_by = f.b_now ? -IMG_BYTES : IMG_BYTES;
     each<M>([&](auto mc) __attribute__((always_inline)) {
       constexpr int m = mc, k = m / RD, l = m / LD;
       f32x4_t& c = acc[m >> 3][m & 7];
       if constexpr (m % RD == RD - 1 && k < READS) {   // (one of B's and one of A's in turn)
-        if constexpr (k < 2 * IM && k % 2 == 1) f.a1[k >> 1] = frag_a(k >> 1, 1);
-        else f.b1[k < 2 * IM ? k >> 1 : k - IM] = frag_b(k < 2 * IM ? k >> 1 : k - IM, 1);
+        if constexpr (k % 2 == 1) f.a1[k >> 1] = frag_a(k >> 1, 1);
+        else f.b1[k >> 1] = frag_b(k >> 1, 1);
         fixed();
       }
       if constexpr (m >= FREE && (m - FREE) % SP == 0) move_by(rb[(m - FREE) / SP], b_by), fixed();
       if constexpr (m == M - 1) move_to(ra[0], base_a[0], f.a_next), fixed();
-      if constexpr (!FEW && m == 36) advance_a(more), fixed();
-      if constexpr (!FEW && m % LD == LD / 2 && l < 8) {
-        mfma_load<l * 1024, ZERO>(c, f.b0[m & 7], f.a0[m >> 3], from<HALF>(l, last), pa, to_a);
-      } else {
-        if constexpr (m % LD == LD / 2 && l < 8) load<HALF, FEW>(l, f.a_free, last);
-        mfma<ZERO>(c, f.b0[m & 7], f.a0[m >> 3]);
-      }
+      if constexpr (m == 36) advance_a(more), fixed();
+      if constexpr (m % LD == LD / 2 && l < 8) mfma_load<l * 1024, ZERO>(c, f.b0[m & 7], f.a0[m >> 3], from<HALF>(l, last), pa, to_a);
+      else mfma<ZERO>(c, f.b0[m & 7], f.a0[m >> 3]);
       fixed();
     });
-    if (FEW) advance_a(more);
     reads_done();
     wait();
     __builtin_amdgcn_s_barrier();
     fixed();
     each<M>([&](auto mc) __attribute__((always_inline)) {
-      constexpr int m = mc, RD2 = IM == 8 ? 4 : RD, k = m / RD2, l = m / LD;
+      constexpr int m = mc, k = m / RD2, l = m / LD;
       f32x4_t& c = acc[m >> 3][m & 7];
-      if constexpr (m % RD2 == RD2 / 2 && k < READS) {
+      if constexpr (m % RD2 == RD2 / 2) {
         if constexpr (k < 8) f.b0[k] = frag_b(k, 0);
         else f.a0[k - 8] = frag_a(k - 8, 0);
         fixed();
       }
       if constexpr (m == 0) move_to(ra[1], base_a[1], f.a_next), fixed();
-      if constexpr (!FEW && m == 36) advance_b(more), fixed();
+      if constexpr (m == 36) advance_b(more), fixed();
       if constexpr (m % LD == LD - 1 && l < 8) mfma_load<B_BASE + l * 1024>(c, f.b1[m & 7], f.a1[m >> 3], from<HALF>(8 + l, last), pb, to_b);
       else mfma(c, f.b1[m & 7], f.a1[m >> 3]);
       fixed();
     });
-    if (FEW) advance_b(more);
     f.b_now ^= IMG_BYTES;
     const int freed = f.a_now;
     f.a_now = f.a_next, f.a_next = f.a_free, f.a_free = freed;
   }
 
-  // acc += the products of so many steps.  IM: row fragments that have rows.  HALF, end: the last step has half the reduction.
+  // Tiles of at most 32 IM rows: a step's products take a fourth of the time of a step's of 256 rows, or half, and its operands are 40 or 48 KB.  Four or three steps of both
+  // operands are there, so that loads have two steps and more for their way; with the places above, B's had half a step, and a step took as long as a load.  What
+  // bounds it now is the weights' bytes (from memory 5.2 TB/s, 16 rows of 8 experts).  us, before / now: 16 rows of each of 8 experts 4096 -> 28672 389 / 363, input gradient 369 / 360,
+  // 100 rows 430 / 409 and 401 / 391; SwiGLU of 8,192 columns, reduction 2,048, 64 or 100 rows 25.3 / 21.3.
+  // beside: other tiles with the same B run at the same time, and it is better to stay with them, so that the L2 has what it reads, than to run ahead: up to 64 rows wait for all loads of a
+  // step (8,192 rows of 8 experts, about 1,024 each, 4096 -> 28672 1,526 before, 1,531 ahead, 1,523 beside; input gradient 1,526 / 1,544 / 1,512; 65 to 128 rows take as long as
+  // the others if they wait so: input gradient 1,573 before, 1,660 with all of them, 1,530 with up to 64).
+  template <int IM>
+  struct Few {
+    static constexpr int PLACES = IM == 2 ? 4 : 3, A_BYTES = IM * 4096, PLACE = A_BYTES + IMG_BYTES, LOADS = 8 + IM;
+    static_assert(PLACES * PLACE <= LDS_BYTES, "LDS");
+  };
+  template <int IM>
+  __device__ __forceinline__ void wait_few(int pieces, bool beside) const {   // all loads but those of the PLACES - 2 newest steps have come
+    constexpr int S = Few<IM>::PLACES - 2;
+    if (IM == 2 && beside) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    else
+    each<IM + 1>([&](auto n) __attribute__((always_inline)) {
+      if (pieces == n) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(S * (8 + n)) : "memory");
+    });
+  }
   template <int IM, bool HALF>
-  __device__ __forceinline__ void run(f32x4_t (&acc)[8][8], int steps, bool end) {
-    static_assert(IM == 8 || IM == 4 || IM == 2, "rows");
+  __device__ __forceinline__ void load_few(int i, int pieces, uint32_t place, bool last) const {   // (A: 0 .. IM - 1)
+    if (i < IM && i >= pieces) return;
+    if (i < IM) load_lds(from<HALF>(i, last), pa, place + (wid + 4 * i) * 1024);
+    else load_lds(from<HALF>(8 + i - IM, last), pb, place + Few<IM>::A_BYTES + (8 * wid + i - IM) * 1024);
+  }
+  template <int IM, bool HALF>
+  __device__ __forceinline__ void run_few(f32x4_t (&acc)[8][8], int steps, bool end, bool beside) {
+    using F = Few<IM>;
+    constexpr int M = 8 * IM, RD = IM == 2 ? 1 : 2;   // products; from one read to the next
+    // of A, those with rows that there are; every fourth is this wave's
+    const int pieces = min(((rows_a + 7) / 8 - wid + 3) / 4, IM);
+    back &= ~((1u << IM) - 1);
+#pragma unroll
+    for (int i = 0; i < IM; ++i) {
+      const int row = 8 * (wid + 4 * i) + (lane >> 3), c = (lane & 7) ^ row_swz(row);
+      off[i] = ((uint32_t)min(row, rows_a - 1) * ld_a + (uint32_t)(8 * c)) * 2;
+      if (c >= 4) back |= 1u << i;
+    }
+#pragma unroll
+    for (int s = 0; s < F::PLACES - 1; ++s) {   // (past the end: the last step again, not used)
+#pragma unroll
+      for (int i = 0; i < F::LOADS; ++i) load_few<IM, HALF>(i, pieces, lds + s * F::PLACE, end && s + 1 >= steps);
+      advance_a(s + 1 < steps), advance_b(s + 1 < steps);
+    }
+    addresses(F::A_BYTES);
     Frags<IM> f;
-    begin<IM, HALF>(f, steps, end);
+    wait_few<IM>(pieces, false);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int j = 0; j < 8; ++j) f.b0[j] = frag_b(j, 0), fixed();   // (in this order: the loop's waits count what came later)
+#pragma unroll
+    for (int i = 0; i < IM; ++i) f.a0[i] = frag_a(i, 0), fixed();
+    int now = 0, free = (F::PLACES - 1) * F::PLACE;   // places of this step and of the one that is loaded
 #pragma unroll 1
     for (int t = 0, whole = steps - (HALF && end); t < whole; ++t) {
+      const int next = now == (F::PLACES - 1) * F::PLACE ? 0 : now + F::PLACE;
+      const bool last = end && t + F::PLACES >= steps;
       asm volatile("s_nop 3");   // (after moves of the sums ahead of the loop)
-      step<IM, HALF, false>(acc, f, end && t + 3 >= steps, t + 3 < steps, [&]() { wait_a<(IM < 8)>(); });
-      if (HALF) asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");   // (the sums may move after the loop)
+      each<M>([&](auto mc) __attribute__((always_inline)) {
+        constexpr int m = mc, k = m / RD, l = IM == 2 ? m - (M - F::LOADS) : m % 2 == 0 ? m / 2 - (M / 2 - F::LOADS) : -1;
+        if constexpr (m % RD == RD - 1 && k < 8 + IM) {   // (one of B's and one of A's in turn)
+          if constexpr (k < 2 * IM && k % 2 == 1) f.a1[k >> 1] = frag_a(k >> 1, 1);
+          else f.b1[k < 2 * IM ? k >> 1 : k - IM] = frag_b(k < 2 * IM ? k >> 1 : k - IM, 1);
+          fixed();
+        }
+        if constexpr (l >= 0) load_few<IM, HALF>(l, pieces, lds + free, last), fixed();
+        mfma(acc[m >> 3][m & 7], f.b0[m & 7], f.a0[m >> 3]);
+        fixed();
+      });
+      advance_a(t + F::PLACES < steps), advance_b(t + F::PLACES < steps);
+#pragma unroll
+      for (int j = 0; j < NB; ++j) move_by(rb[j], next - now);
+      move_to(ra[0], base_a[0], next);
+      reads_done();
+      wait_few<IM>(pieces, beside);
+      __builtin_amdgcn_s_barrier();
+      fixed();
+      each<M>([&](auto mc) __attribute__((always_inline)) {
+        constexpr int m = mc, k = m / RD;
+        if constexpr (m % RD == RD / 2 && k < 8 + IM) {
+          if constexpr (k < 8) f.b0[k] = frag_b(k, 0);
+          else f.a0[k - 8] = frag_a(k - 8, 0);
+          fixed();
+        }
+        mfma(acc[m >> 3][m & 7], f.b1[m & 7], f.a1[m >> 3]);
+        fixed();
+      });
+      move_to(ra[1], base_a[1], next);
+      free = now, now = next;
+      asm volatile("s_nop 7" ::: "memory");   // (the sums may move after the loop)
     }
+    last_half<IM, HALF>(acc, f, end);
+  }
+
+  // acc += the products of so many steps.  IM: row fragments that have rows.  HALF, end: the last step has half the reduction.
+  template <int IM, bool HALF>
+  __device__ __forceinline__ void run(f32x4_t (&acc)[8][8], int steps, bool end, bool beside = false) {
+    static_assert(IM == 8 || IM == 4 || IM == 2, "rows");
+    if constexpr (IM < 8) {
+      run_few<IM, HALF>(acc, steps, end, beside);
+    } else {
+      Frags<8> f;
+      begin<HALF>(f, steps, end);
+#pragma unroll 1
+      for (int t = 0, whole = steps - (HALF && end); t < whole; ++t) {
+        asm volatile("s_nop 3");   // (after moves of the sums ahead of the loop)
+        step<HALF, false>(acc, f, end && t + 3 >= steps, t + 3 < steps, [&]() { asm volatile("s_waitcnt vmcnt(8)" ::: "memory"); });   // (all but A's of the newest step)
+        if (HALF) asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");   // (the sums may move after the loop)
+      }
+      last_half<8, HALF>(acc, f, end);
+    }
+  }
+  template <int IM, bool HALF>
+  __device__ __forceinline__ void last_half(f32x4_t (&acc)[8][8], Frags<IM>& f, bool end) {   // after the whole steps
     if (HALF && end) {   // (s_nop: the sums may have moved to other registers just before)
 #pragma unroll
       for (int i = 0; i < IM; ++i)
@@ -321,11 +408,11 @@ struct Loop {
     const auto rest = [&](int t, int end) __attribute__((always_inline)) {   // towards step t + 3, or the next tile's t + 3 - steps
 #pragma unroll 1
       for (; t < end; ++t)
-        step<8, false, false>(acc, f, false, t + 3 < steps || (another && t + 3 > steps && t + 3 < 2 * steps), [&]() { asm volatile("s_waitcnt vmcnt(8)" ::: "memory"); });
+        step<false, false>(acc, f, false, t + 3 < steps || (another && t + 3 > steps && t + 3 < 2 * steps), [&]() { asm volatile("s_waitcnt vmcnt(8)" ::: "memory"); });
     };
     const int turn = steps - 2;
     if (turn == 0 && another) next();
-    step<8, false, true>(acc, f, false, 3 < steps || (another && steps == 2), [&]() {
+    step<false, true>(acc, f, false, 3 < steps || (another && steps == 2), [&]() {
       if (stores == 32) asm volatile("s_waitcnt vmcnt(40)" ::: "memory");
       else if (stores == 16) asm volatile("s_waitcnt vmcnt(24)" ::: "memory");
       else asm volatile("s_waitcnt vmcnt(8)" ::: "memory");

@@ -127,11 +127,11 @@ __global__ void __launch_bounds__(NT, 1) rowgemm_kernel(Params p) {
     for (int j = 0; j < 8; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   // (an expert's last tile: with at most half the rows half the work, with a quarter a quarter: 8 experts of about 1,024 rows each, of which half have a
   // few rows more, 4096 -> 28672 1,744 -> 1,681 us)
-  const bool end = HALF && part == parts - 1;
+  const bool end = HALF && part == parts - 1, beside = r0 > p.offs[e];   // (beside: run_few)
   if (nk > 0) {
     if (r1 - r0 > BM / 2) loop.template run<8, HALF>(acc, nk, end);
-    else if (r1 - r0 > BM / 4) loop.template run<4, HALF>(acc, nk, end);
-    else loop.template run<2, HALF>(acc, nk, end);
+    else if (r1 - r0 > BM / 4) loop.template run<4, HALF>(acc, nk, end, beside);
+    else loop.template run<2, HALF>(acc, nk, end, beside);
   }
   const int lane = loop.lane, wid = loop.wid, wm = loop.wm, wn = loop.wn;
 
