@@ -50,8 +50,8 @@ struct Params {
 };
 
 constexpr int XCDS = 8, XCD_CUS = 32;
-// Parts of a tile at most; reduction steps of a part at least: writing a part's sums and reading them all back takes 25-40 us, 32
-// steps take 55
+// Parts of a tile at most; reduction steps of a part at least: writing a part's sums and reading them all back takes 10-20 us (25-40 with a fence that
+// wrote back the L2), 32 steps take 35-55
 constexpr int MAX_PARTS = 8, MIN_STEPS = 32;
 constexpr int FRAG_FLOATS = 32 * BN;   // 32 rows of a tile
 
@@ -135,7 +135,9 @@ __global__ void __launch_bounds__(NT, 1) rowgemm_kernel(Params p) {
   }
   const int lane = loop.lane, wid = loop.wid, wm = loop.wm, wn = loop.wn;
 
-  // ---- parts of a tile: sums to memory; the last part to come adds them up, in their order
+  // ---- parts of a tile: sums to memory; the last part to come adds them up, in their order.  They are stored past the L2 (write-through) and waited for: a release
+  // fence ahead of the ticket writes back all of an XCD's L2 for each part.  us, with the fence / now: 16 rows of each of 8 experts 4096 -> 28672 350 / 318, input gradient
+  // 383 / 350, 100 rows 390 / 357 and 411 / 375; 8,192 rows 14336 -> 4096 791 / 766, 28672 -> 4096 (input gradient) 1,504 / 1,486.
   if (parts > 1) {
     const int slot = xcd * p.slots + idx - whole - part;   // of the tile's first part
     const int64_t place = (int64_t)p.frags * FRAG_FLOATS;
@@ -143,21 +145,32 @@ __global__ void __launch_bounds__(NT, 1) rowgemm_kernel(Params p) {
     const bool most = r1 - r0 > BM / 2;
     const int have = most ? 8 : (r1 - r0 + 31) / 32;       // fragments with rows, or all
     // (each wave's sums lie together: a fragment's of all waves beside each other, 1,024 rows of 4 experts, 8192 -> 256, 99 -> 111 us)
-    auto at = [&](int s, int i, int j) { return reinterpret_cast<f32x4_t*>(sums + s * place) + ((wid * p.frags + i) * 8 + j) * 64 + lane; };
+    auto at = [&](int s, int i, int j) { return reinterpret_cast<uint64_t*>(sums + s * place) + ((wid * p.frags + i) * 8 + j) * 128 + lane; };
+    auto leave = [&](int i, int j) __attribute__((always_inline)) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const f32x2_t two = {acc[i][j][2 * h], acc[i][j][2 * h + 1]};
+        __hip_atomic_store(at(part, i, j) + 64 * h, __builtin_bit_cast(uint64_t, two), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    };
+    auto left = [&](int s, int i, int j) __attribute__((always_inline)) {
+      const f32x2_t lo = __builtin_bit_cast(f32x2_t, at(s, i, j)[0]), hi = __builtin_bit_cast(f32x2_t, at(s, i, j)[64]);
+      return f32x4_t{lo[0], lo[1], hi[0], hi[1]};
+    };
     if (most) {
 #pragma unroll
       for (int i = 0; i < 8; ++i)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) *at(part, i, j) = acc[i][j];
+        for (int j = 0; j < 8; ++j) leave(i, j);
     } else {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         if (i < have) {
 #pragma unroll
-          for (int j = 0; j < 8; ++j) *at(part, i, j) = acc[i][j];
+          for (int j = 0; j < 8; ++j) leave(i, j);
         }
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (each wave's own, and the barrier: all of them are there before the ticket)
     __syncthreads();
     int* last = reinterpret_cast<int*>(smem);
     if (threadIdx.x == 0) {
@@ -173,7 +186,7 @@ __global__ void __launch_bounds__(NT, 1) rowgemm_kernel(Params p) {
         for (int i = 0; i < 8; ++i)
 #pragma unroll
           for (int j = 0; j < 8; ++j) {
-            const f32x4_t v = *at(s, i, j);
+            const f32x4_t v = left(s, i, j);
             acc[i][j] = s == 0 ? v : acc[i][j] + v;
           }
       }
@@ -183,7 +196,7 @@ __global__ void __launch_bounds__(NT, 1) rowgemm_kernel(Params p) {
         for (int i = 0; i < 4; ++i)   // (fragments without rows: any sums)
 #pragma unroll
           for (int j = 0; j < 8; ++j) {
-            const f32x4_t v = *at(s, min(i, have - 1), j);
+            const f32x4_t v = left(s, min(i, have - 1), j);
             acc[i][j] = s == 0 ? v : acc[i][j] + v;
           }
       }
