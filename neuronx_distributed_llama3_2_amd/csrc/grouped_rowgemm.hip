@@ -50,8 +50,8 @@ struct Params {
 };
 
 constexpr int XCDS = 8, XCD_CUS = 32;
-// Parts of a tile at most; reduction steps of a part at least: writing a part's sums and reading them all back takes 10-20 us (25-40 with a fence that
-// wrote back the L2), 32 steps take 35-55
+// Parts of a tile at most; reduction steps of a part at least: writing a part's sums and reading them all back takes 15-30 us, 32
+// steps take 35-55
 constexpr int MAX_PARTS = 8, MIN_STEPS = 32;
 constexpr int FRAG_FLOATS = 32 * BN;   // 32 rows of a tile
 
@@ -135,6 +135,19 @@ __global__ void __launch_bounds__(NT, 1) rowgemm_kernel(Params p) {
   }
   const int lane = loop.lane, wid = loop.wid, wm = loop.wm, wn = loop.wn;
 
+  // ---- results through LDS, a wave's 128 x 128 in 32 KB of its own (16-byte chunks XORed with the row): 256 contiguous bytes of a row
+  // a store
+  char* own = smem + wid * (tile::LDS_BYTES / 4);
+  auto put = [&](int i, const f32x4_t (&sums)[8]) __attribute__((always_inline)) {   // of row fragment i
+#pragma unroll
+    for (int j = 0; j < 8; j += MODE == FWD ? 1 : 2) {
+      const int r = 16 * i + (lane & 15), c = tile::col<MODE == FWD>(0, j, lane);
+      const u32x2_t lo = {pack2bf(sums[j][0], sums[j][1]), pack2bf(sums[j][2], sums[j][3])};
+      char* to = own + r * 256 + 16 * ((c >> 3) ^ (r & 15));
+      if (MODE == FWD) *reinterpret_cast<u32x2_t*>(to + 2 * (c & 7)) = lo;
+      else *reinterpret_cast<u32x4_t*>(to) = u32x4_t{lo[0], lo[1], pack2bf(sums[j + 1][0], sums[j + 1][1]), pack2bf(sums[j + 1][2], sums[j + 1][3])};
+    }
+  };
   // ---- parts of a tile: sums to memory; the last part to come adds them up, in their order.  They are stored past the L2 (write-through) and waited for: a release
   // fence ahead of the ticket writes back all of an XCD's L2 for each part.  us, with the fence / now: 16 rows of each of 8 experts 4096 -> 28672 350 / 318, input gradient
   // 383 / 350, 100 rows 390 / 357 and 411 / 375; 8,192 rows 14336 -> 4096 791 / 766, 28672 -> 4096 (input gradient) 1,504 / 1,486.
@@ -142,34 +155,20 @@ __global__ void __launch_bounds__(NT, 1) rowgemm_kernel(Params p) {
     const int slot = xcd * p.slots + idx - whole - part;   // of the tile's first part
     const int64_t place = (int64_t)p.frags * FRAG_FLOATS;
     float* sums = p.ws + slot * place;
-    const bool most = r1 - r0 > BM / 2;
-    const int have = most ? 8 : (r1 - r0 + 31) / 32;       // fragments with rows, or all
+    const int have = r1 - r0 > BM / 2 ? 8 : (r1 - r0 + 31) / 32;       // fragments with rows, or all
     // (each wave's sums lie together: a fragment's of all waves beside each other, 1,024 rows of 4 experts, 8192 -> 256, 99 -> 111 us)
     auto at = [&](int s, int i, int j) { return reinterpret_cast<uint64_t*>(sums + s * place) + ((wid * p.frags + i) * 8 + j) * 128 + lane; };
-    auto leave = [&](int i, int j) __attribute__((always_inline)) {
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const f32x2_t two = {acc[i][j][2 * h], acc[i][j][2 * h + 1]};
-        __hip_atomic_store(at(part, i, j) + 64 * h, __builtin_bit_cast(uint64_t, two), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int i = 0; i < 8; ++i)
+      if (i < have) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const f32x2_t two = {acc[i][j][2 * h], acc[i][j][2 * h + 1]};
+            __hip_atomic_store(at(part, i, j) + 64 * h, __builtin_bit_cast(uint64_t, two), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          }
       }
-    };
-    auto left = [&](int s, int i, int j) __attribute__((always_inline)) {
-      const f32x2_t lo = __builtin_bit_cast(f32x2_t, at(s, i, j)[0]), hi = __builtin_bit_cast(f32x2_t, at(s, i, j)[64]);
-      return f32x4_t{lo[0], lo[1], hi[0], hi[1]};
-    };
-    if (most) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) leave(i, j);
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (i < have) {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) leave(i, j);
-        }
-    }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (each wave's own, and the barrier: all of them are there before the ticket)
     __syncthreads();
     int* last = reinterpret_cast<int*>(smem);
@@ -180,43 +179,48 @@ __global__ void __launch_bounds__(NT, 1) rowgemm_kernel(Params p) {
     __syncthreads();
     if (!*last) return;
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    if (most) {
-      for (int s = 0; s < parts; ++s) {
+    __syncthreads();   // (*last has been read by all)
+    // Row fragment by row fragment, straight to the results, and four loads of a fragment (8 KB of a wave's) on their way at any time, over to the next one: with all
+    // fragments of a part and then the next part, a part of 256 KB took 14 us.  Reduction x columns, us, so / now: 8,192 uneven rows of 8 experts 14336 x 4096 773 / 755, 28672 x
+    // 4096 (input gradient) 1,499 / 1,478; one expert, 4,096 rows 12288 x 2048 171 / 162, 1,000 rows 16384 x 2048 (8 parts) 174 / 92, 512 rows 8192 x 2048 92 / 60.
+    // P: parts, or more (the last one again, not used).
+    auto add_up = [&](auto np) __attribute__((always_inline)) {
+      constexpr int P = np, RING = 4, STEPS = P > RING ? P : RING;
+      f32x4_t v[RING][8], row[8];
+      auto fetch = [&](int u, int s, int i) __attribute__((always_inline)) {
+        const uint64_t* from = at(min(s, parts - 1), min(i, have - 1), 0);
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
+        for (int j = 0; j < 8; ++j) {
+          const f32x2_t lo = __builtin_bit_cast(f32x2_t, from[128 * j]), hi = __builtin_bit_cast(f32x2_t, from[128 * j + 64]);
+          v[u][j] = f32x4_t{lo[0], lo[1], hi[0], hi[1]};
+        }
+      };
+#pragma unroll
+      for (int u = 0; u < RING; ++u) fetch(u, u % P, u / P);
+#pragma unroll 1
+      for (int i = 0; i < have; i += STEPS / P) {
+#pragma unroll
+        for (int u = 0; u < STEPS; ++u) {
+          const bool there = u % P < parts;
 #pragma unroll
           for (int j = 0; j < 8; ++j) {
-            const f32x4_t v = left(s, i, j);
-            acc[i][j] = s == 0 ? v : acc[i][j] + v;
+            const f32x4_t sum = row[j] + v[u % RING][j];
+            row[j] = u % P == 0 ? v[u % RING][j] : there ? sum : row[j];
           }
+          fetch(u % RING, (u + RING) % P, i + (u + RING) / P);
+          if (u % P == P - 1) put(i + u / P, row);
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
-    } else {
-      for (int s = 0; s < parts; ++s) {
+    };
+    if (parts == 2) add_up(std::integral_constant<int, 2>{});
+    else if (parts <= 4) add_up(std::integral_constant<int, 4>{});
+    else add_up(std::integral_constant<int, 8>{});
+  } else {
+    __syncthreads();
 #pragma unroll
-        for (int i = 0; i < 4; ++i)   // (fragments without rows: any sums)
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            const f32x4_t v = left(s, min(i, have - 1), j);
-            acc[i][j] = s == 0 ? v : acc[i][j] + v;
-          }
-      }
-    }
+    for (int i = 0; i < 8; ++i) put(i, acc[i]);
   }
-
-  // ---- results through LDS, a wave's 128 x 128 in 32 KB of its own (16-byte chunks XORed with the row): 256 contiguous bytes of a row
-  // a store
-  __syncthreads();
-  char* own = smem + wid * (tile::LDS_BYTES / 4);
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-#pragma unroll
-    for (int j = 0; j < 8; j += MODE == FWD ? 1 : 2) {
-      const int r = 16 * i + (lane & 15), c = tile::col<MODE == FWD>(0, j, lane);
-      const u32x2_t lo = {pack2bf(acc[i][j][0], acc[i][j][1]), pack2bf(acc[i][j][2], acc[i][j][3])};
-      char* to = own + r * 256 + 16 * ((c >> 3) ^ (r & 15));
-      if (MODE == FWD) *reinterpret_cast<u32x2_t*>(to + 2 * (c & 7)) = lo;
-      else *reinterpret_cast<u32x4_t*>(to) = u32x4_t{lo[0], lo[1], pack2bf(acc[i][j + 1][0], acc[i][j + 1][1]), pack2bf(acc[i][j + 1][2], acc[i][j + 1][3])};
-    }
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   const int c0 = 128 * wn + 8 * (lane & 15);
 #pragma unroll
