@@ -75,9 +75,9 @@ class LlamaMLP(nn.Module):
     def forward(self, x):
         gu = self.gate_up_proj(x)
         if self.selective_checkpoint and self.training:
-            h = checkpoint(ops.swiglu, gu, True, use_reentrant=False)
+            h = checkpoint(ops.swiglu, gu, True, x.shape[-1], use_reentrant=False)
         else:
-            h = ops.swiglu(gu, token_major=True)   # token-major copies feed the TN weight gradients
+            h = ops.swiglu(gu, token_major=True, width=x.shape[-1])   # token-major copies feed the TN weight gradients
         return self.down_proj(h)
 
 
@@ -194,9 +194,9 @@ class LlamaDecoderLayer(nn.Module):
         gu = mlp.gate_up_proj(normed)
         yield
         if mlp.selective_checkpoint and self.training:
-            h = checkpoint(ops.swiglu, gu, True, use_reentrant=False)
+            h = checkpoint(ops.swiglu, gu, True, normed.shape[-1], use_reentrant=False)
         else:
-            h = ops.swiglu(gu, token_major=True)
+            h = ops.swiglu(gu, token_major=True, width=normed.shape[-1])
         out = mlp.down_proj(h)
         yield
         return out, residual

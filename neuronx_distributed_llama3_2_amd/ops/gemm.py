@@ -159,12 +159,6 @@ _WG_KERNEL = os.environ.get("NXD_WGRAD_KERNEL", "auto")
 _WG_SKINNY = 1100.0
 _WG_WIDE = 16000
 _WG_RAGGED = 4000.0
-# Larger products without a producer's copy, where the last round of 256 tiles is at least seven eighths full: time of the library with
-# its two transposes = 1, 12,288 x 4,096 0.92-0.94, 22,016 x 4,096 0.89-0.93, 4,096 x 14,336 0.93-0.99, 8,192 x 8,192 0.94-1.01 from 4,096 to
-# 32,768 tokens (2,048 tokens 0.88-1.03; 6,144 x 4,096, one and a half rounds, 1.02-1.03 up to 8,192).
-_WG_FULL_TOKENS = 4096
-
-
 def _ragged_tokens(tiles: int, odd: bool) -> int:
     """Token counts (no multiple of 64) up to which a product of so many tiles goes to the wgrad kernel."""
     full = tiles / (256 * -(-tiles // 256))
@@ -186,8 +180,6 @@ def _wgrad_kernel_splits(mg: torch.Tensor, go2: torch.Tensor, x2: torch.Tensor, 
     if T % 32 == 0 and (_WG_KERNEL == "1" or M * N / (M + N) < _WG_SKINNY or (not has_copy and max(M, N) >= _WG_WIDE)):
         return 0
     tiles = -(-M // 256) * -(-N // 256)
-    if T % 32 == 0 and T >= _WG_FULL_TOKENS and not has_copy and 8 * tiles >= 7 * 256 * -(-tiles // 256):
-        return 0
     if T % 64 and not has_copy and M * N / (M + N) < _WG_RAGGED and T <= _ragged_tokens(tiles, T % 8 != 0):
         return 1 if tiles >= 128 else 0
     return None
@@ -221,6 +213,35 @@ def _use_dense_wgrad(mg: torch.Tensor, go2: torch.Tensor, x2, has_copy: bool) ->
     return _DENSE_WG == "1" or (not has_copy and M * N / (M + N) < _DENSE_WG_SKINNY)
 
 
+# Products of whole rounds of 256 tiles, or nearly: the wgrad kernel ahead of all the rules above and below, a producer's copy or not.  Its time over that of the
+# library with its transposes (main loop with one read, address or load between two MFMAs, gradients from memory): counts that are no multiple of 64, 2,998 to
+# 20,001 tokens: 256 tiles 0.72-0.81, 352 (two rounds, 0.69 full) 0.88-0.94, 384 0.87-0.94, 640 0.73-0.82, 768 0.71-0.80, 1,376 0.70-0.80, 2,000 0.74, 4,008 0.75; 1,000 to 1,501 of
+# them: 352 0.83, 384 0.80-0.92, 640 0.80, 1,024 0.82, 4,096 0.69; 200: 4,096 0.75.  Whole steps of 64, 3,072 tokens: 384 0.95, 640 0.85, 688 0.85, 768 0.87, 896 0.92; 4,096 and
+# 8,192: 352 0.93, 384 0.91-0.95, 400 0.86-0.89, 768 0.82-0.86, 1,376 0.76-0.78, 2,000 0.87.  Not: 512 to 2,048 tokens in whole steps (0.92-1.11), rounds that are less full (320 tiles
+# 0.95-1.04 from 4,096 tokens on), one round below seven eighths.
+_WG_WHOLE_TOKENS = 3072
+
+
+def wgrad_in_rounds(T: int, M: int, N: int) -> bool:
+    """Whether the weight gradient [M, N] of T tokens goes to the wgrad kernel because it fills its rounds of tiles: it reads both operands as they are, so
+    nobody needs to write transposed copies for it."""
+    tiles = -(-M // 256) * -(-N // 256)
+    rounds = -(-tiles // 256)
+    if _WG_KERNEL == "0" or M % 8 or N % 8 or (T % 64 == 0 and T < _WG_WHOLE_TOKENS):
+        return False
+    return 8 * tiles >= 7 * 256 if rounds == 1 else 3 * tiles >= 2 * 256 * rounds
+
+
+def _use_wgrad_in_rounds(mg: torch.Tensor, go2: torch.Tensor, x2) -> bool:
+    if x2 is None or not _native(go2, x2) or go2.dtype != torch.bfloat16 or x2.dtype != torch.bfloat16 or mg.dtype != torch.float32:
+        return False
+    if go2.stride(1) != 1 or x2.stride(1) != 1 or mg.stride(1) != 1 or go2.stride(0) % 8 or x2.stride(0) % 8 or mg.stride(0) % 4:
+        return False
+    if go2.data_ptr() % 16 or x2.data_ptr() % 16 or mg.data_ptr() % 16:
+        return False
+    return wgrad_in_rounds(go2.shape[0], go2.shape[1], x2.shape[1])
+
+
 def _wgrad_scratch(n: int, dtype, device, tag: str = "") -> torch.Tensor:
     # one buffer per stream: the two halves of parallel_layers/stream_split.py transpose concurrently
     sid = torch.cuda.current_stream(device).stream_id if torch.device(device).type == "cuda" else 0
@@ -246,7 +267,7 @@ def wgrad_accumulate_(mg: torch.Tensor, go2: torch.Tensor, x2, go_t: torch.Tenso
     if go2.shape[0] == 0:
         return
     has_copy = go_t is not None or x_t is not None
-    if _use_dense_wgrad(mg, go2, x2, has_copy):
+    if _use_wgrad_in_rounds(mg, go2, x2) or _use_dense_wgrad(mg, go2, x2, has_copy):
         ext().wgrad_gemm(mg, go2, x2, 0, True)
         return
     splits = _wgrad_kernel_splits(mg, go2, x2, has_copy)

@@ -1,0 +1,60 @@
+"""Weight gradients that fill their rounds of 256 tiles go to csrc/wgrad_gemm.hip, whatever the tokens, and nobody writes transposed copies for them.  The lines
+were measured (ops/gemm.py); the gradients are compared with float64."""
+import pytest
+import torch
+
+from test_wgrad_tiles_gpu import _check
+
+from neuronx_distributed_llama3_2_amd import ops
+from neuronx_distributed_llama3_2_amd.ops import gemm
+
+
+@pytest.mark.parametrize("T,M,N,own", [
+    (3072, 4096, 4096, True), (3008, 4096, 4096, False), (3009, 4096, 4096, True), (1, 4096, 4096, True), (2048, 16384, 16384, False),   # tokens
+    (3072, 4096, 3584, True), (3072, 4096, 3328, False), (3072, 4096, 5504, True), (3072, 4096, 5376, False), (3001, 4096, 5376, False),     # fill: 224, 208, 352, 336 tiles
+    (3072, 8192, 5376, True), (3072, 8192, 5120 + 256 * 3 + 8, True), (3001, 4096, 4092, False), (3001, 4100, 4096, False),
+])
+def test_rule(T, M, N, own):
+    assert gemm.wgrad_in_rounds(T, M, N) == (own and gemm._WG_KERNEL != "0")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,M,N", [(3072, 4096, 3592), (3009, 3592, 4096), (1, 4096, 4096), (72, 5640, 4096), (4100, 4096, 4096), (3079, 5632, 4096)])
+@pytest.mark.parametrize("copy", [False, True])
+def test_gradient(T, M, N, copy):
+    g = torch.Generator(device="cuda").manual_seed(T + M)
+    dy, x = (torch.randn(T, n, generator=g, device="cuda").bfloat16() for n in (M, N))
+    mg = torch.randn(M, N, generator=g, device="cuda")
+    before = mg.clone()
+    assert gemm._use_wgrad_in_rounds(mg, dy, x) == gemm.wgrad_in_rounds(T, M, N)
+    gemm.wgrad_accumulate_(mg, dy, x, go_t=dy.t().contiguous() if copy else None)
+    _check(mg, before, dy, x)
+
+
+@pytest.mark.gpu
+def test_operands_that_the_kernel_does_not_take():
+    g = torch.Generator(device="cuda").manual_seed(1)
+    dy, x = (torch.randn(100, 4104, generator=g, device="cuda").bfloat16() for _ in range(2))
+    mg = torch.zeros(4096, 4096, device="cuda")
+    assert gemm._use_wgrad_in_rounds(mg, dy[:, :4096], x[:, 8:]) == (gemm._WG_KERNEL != "0")
+    for a, b in ((dy[:, 4:4100], x[:, 8:]), (dy[:, 8:], x[:, 4:4100]), (dy[:, :4096], x[:, 8:].half()), (dy[:, :4096], None)):
+        assert not gemm._use_wgrad_in_rounds(mg, a, b)
+    assert not gemm._use_wgrad_in_rounds(mg.bfloat16(), dy[:, :4096], x[:, 8:])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,width,copies", [(3072, 4096, False), (3008, 4096, True), (3072, None, True)])
+def test_swiglu_writes_copies_for_the_library_only(rows, width, copies):
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    gu = torch.randn(rows, 8192, generator=g, device="cuda").bfloat16()
+    dh = torch.randn(rows, 4096, generator=g, device="cuda").bfloat16()
+    seen, out = [], []
+    for token_major in (True, False):
+        leaf = gu.clone().requires_grad_()
+        leaf.register_hook(lambda d: seen.append(hasattr(d, "_nxd_t")))
+        h = ops.swiglu(leaf, token_major=token_major, width=width)
+        assert hasattr(h, "_nxd_t") == (copies and token_major)
+        h.backward(dh)
+        out.append((h.detach(), leaf.grad))
+    assert seen == [copies, False]
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
