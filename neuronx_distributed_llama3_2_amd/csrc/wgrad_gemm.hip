@@ -173,7 +173,9 @@ __global__ void __launch_bounds__(NT, 1) wgrad_kernel(Params p) {
 // 128 x 64 results with a load, an add and a store of 32 rows at a time, steps of 32 tokens in a ring of four, half the registers to fill and
 // to empty.  us here / by the loop above:
 //   * 8 experts' 4096 x 28672 and 14336 x 4096 gradients: 256 tokens each 1,505, 697 / 1,588, 807; 768 2,237, 1,056 / 2,300, 1,084; 1,024 2,644,
-//     1,278 / 2,627, 1,308; 1,280 3,107, 1,507 / 3,032, 1,479; 1,536 3,505, 1,715 / 3,382, 1,646 (the gradient past the caches in both);
+//     1,278 / 2,627, 1,308; 1,280 3,107, 1,507 / 3,032, 1,479; 1,536 3,505, 1,715 / 3,382, 1,646 (the gradient past the caches in both).  With one read,
+//     address or load between two MFMAs of the loop above: 768 2,610, 1,265 / 2,623, 1,281; 1,024 2,845, 1,374 / 2,777, 1,366; 1,280 14336 x 4096 1,750 / 1,664; 2048 x 2816 768 147 /
+//     146, 1,024 162 / 152; 128 experts' 2048 x 1536 1,024 1,130 / 1,092 (but 64 experts' 2048 x 1408 553 / 560): the line for groups is at 900;
 //   * one gradient, whole steps of 32 tokens: 512 x 512 512 tokens 20 / 27, 1,024 32 / 37, 2,048 53 / 56, 3,072 75.3 / 74.9; 2048 x 2048 23 / 30, 34 /
 //     39, 56 / 58, 78 / 78; 3072 x 4096 1,056 46.3 / 48.9, 2,048 68 / 69; 4096 x 4096 512 39 / 42, 1,056 54 / 56, 1,536 69 / 67; 16384 x 2048 1,024
 //     102 / 109, 2,080 155 / 157, 3,072 205 / 199;
@@ -191,7 +193,7 @@ __global__ void __launch_bounds__(NT, 1) wgrad_kernel(Params p) {
 //   * pieces issued after stage S's last: S+1 (4) and S+2's first half (2) -> vmcnt(6), less at the tail.
 namespace few {
 
-inline int most(bool past) { return past ? 1150 : 1400; }   // tokens of a group
+inline int most(bool past) { return past ? 900 : 1400; }   // tokens of a group
 constexpr int BK = 32, STAGES = 4, NT = 512;
 inline bool dense(int T, int tiles) {   // (one gradient, unsplit)
   if (T % BK) return T <= 450 || (T <= 700 && (tiles < 192 || tiles > 1024));
