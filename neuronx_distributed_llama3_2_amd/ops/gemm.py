@@ -155,6 +155,7 @@ def _use_wgrad_t(go2: torch.Tensor, x2: torch.Tensor = None, K: int = None) -> b
 # to 1,000 (0.75-0.92; at 1,500 0.89-1.07), and from 7/8 at any even count (0.73-0.97 from 224 to 1,576 tiles up to 16,392
 # tokens).  Less full: 128 tiles 1.13 over 1,000, 1.70 over 8,200; 280 tiles 1.22 over 3,000; 96 tiles 1.08 over 500.  Odd
 # counts take no transposes: 0.83-0.95 at 1,001, 0.91-0.98 at 3,071, slower from 4,001 on.  M N / (M + N) measured up to 3,737.
+# (All of that with the main loop as it was; what fills its rounds comes here no more: wgrad_in_rounds.)
 _WG_KERNEL = os.environ.get("NXD_WGRAD_KERNEL", "auto")
 _WG_SKINNY = 1100.0
 _WG_WIDE = 16000
