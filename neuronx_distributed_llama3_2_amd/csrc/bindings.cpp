@@ -73,7 +73,7 @@ int dgemv_launch(int, const void*, int64_t, const void*, float, const void*, int
                  int, int, const float*, const float*, const int64_t*, int, void*, void*, int64_t, int64_t, int64_t,
                  const int*, int, int, const float*, float*, hipStream_t, const int64_t*, int64_t, void*, float*);
 int grouped_gemm_launch(int, const void*, const void*, void*, const int*, int, int, int, int, int, hipStream_t);
-int wgrad_gemm_launch(const void*, int64_t, const void*, int64_t, float*, int64_t, int, int, int, int, bool, hipStream_t);
+int wgrad_gemm_launch(const void*, int64_t, const void*, int64_t, float*, int64_t, int, int, int, int, hipStream_t);
 int wgrad_gemm_choose_splits(int, int, int);
 void wgrad_gemm_plan(int, int, int, int, int*);
 int decode_attn_oproj_launch(const void*, const int64_t*, const void*, const void*, const int64_t*, const int*, const int*,
@@ -845,8 +845,7 @@ void dequant_int8(at::Tensor w, c10::optional<at::Tensor> scale, double tscale, 
 
 // main_grad [M, N] fp32 += dy [T, M]^T x [T, N] (csrc/wgrad_gemm.hip): token-major bf16 operands with
 // unit inner strides, row strides multiples of 8 elements, T % 32 == 0 unless tail; splits <= 0 -> auto.
-// zero: mg is zeros (and need not be read)
-void wgrad_gemm(at::Tensor mg, at::Tensor dy, at::Tensor x, int64_t splits, bool tail, bool zero) {
+void wgrad_gemm(at::Tensor mg, at::Tensor dy, at::Tensor x, int64_t splits, bool tail) {
   check_bf16(dy, "dy");
   check_bf16(x, "x");
   check_cuda(mg, "main_grad");
@@ -861,7 +860,7 @@ void wgrad_gemm(at::Tensor mg, at::Tensor dy, at::Tensor x, int64_t splits, bool
   check_aligned16(dy, "dy");
   check_aligned16(x, "x");
   check_rc(nxd::wgrad_gemm_launch(dy.data_ptr(), dy.stride(0), x.data_ptr(), x.stride(0), mg.data_ptr<float>(),
-                                  mg.stride(0), (int)T, (int)M, (int)N, (int)splits, zero, cur_stream()),
+                                  mg.stride(0), (int)T, (int)M, (int)N, (int)splits, cur_stream()),
            "wgrad_gemm");
 }
 
@@ -903,8 +902,8 @@ void dense_gemm(int64_t layout, int64_t epi, at::Tensor a, at::Tensor b, at::Ten
 // MoE grouped GEMMs over expert-sorted rows (csrc/grouped_gemm.hip); offs int32 [E + 1] on device.
 //   mode 0: a = x [M, K], b = W [E, K, N], c = y [M, N] bf16
 //   mode 1: a = dy [M, N], b = W [E, K, N], c = dx [M, K] bf16
-//   mode 2: a = x [M, K], b = dy [M, N], c = dW [E, K, N] fp32 (accumulate: +=; zero: they are zeros and need not be read)
-void grouped_gemm(int64_t mode, at::Tensor a, at::Tensor b, at::Tensor offs, at::Tensor c, bool accumulate, bool zero) {
+//   mode 2: a = x [M, K], b = dy [M, N], c = dW [E, K, N] fp32 (accumulate: +=)
+void grouped_gemm(int64_t mode, at::Tensor a, at::Tensor b, at::Tensor offs, at::Tensor c, bool accumulate) {
   check_bf16(a, "a");
   check_bf16(b, "b");
   check_cuda(c, "c");
@@ -948,7 +947,7 @@ void grouped_gemm(int64_t mode, at::Tensor a, at::Tensor b, at::Tensor offs, at:
     if (!accumulate) c.zero_();
     if (M == 0) return;
     check_rc(nxd::wgrad_gemm_grouped_launch(a.data_ptr(), K, b.data_ptr(), N, c.data_ptr<float>(), N, K * N,
-                                            offs.data_ptr<int32_t>(), (int)E, (int)M, (int)K, (int)N, zero || !accumulate, cur_stream()),
+                                            offs.data_ptr<int32_t>(), (int)E, (int)M, (int)K, (int)N, !accumulate, cur_stream()),
              "grouped_gemm wgrad");
     return;
   }
@@ -1250,10 +1249,8 @@ PYBIND11_MODULE(_C, m) {
   m.def("gemv", &gemv);
   m.def("dequant_int8", &dequant_int8);
   m.def("expert_gemv", &expert_gemv);
-  m.def("grouped_gemm", &grouped_gemm, py::arg("mode"), py::arg("a"), py::arg("b"), py::arg("offs"), py::arg("c"), py::arg("accumulate"),
-        py::arg("zero") = false);
-  m.def("wgrad_gemm", &wgrad_gemm, py::arg("main_grad"), py::arg("dy"), py::arg("x"), py::arg("splits"), py::arg("tail") = false,
-        py::arg("zero") = false);
+  m.def("grouped_gemm", &grouped_gemm);
+  m.def("wgrad_gemm", &wgrad_gemm, py::arg("main_grad"), py::arg("dy"), py::arg("x"), py::arg("splits"), py::arg("tail") = false);
   m.def("dense_gemm", &dense_gemm, py::arg("layout"), py::arg("epi"), py::arg("a"), py::arg("b"), py::arg("c"),
         py::arg("splits") = 0);
   m.def("dense_gemm_set_pipe", [](int64_t v) { nxd::dense_gemm_set_pipe((int)v); });

@@ -633,7 +633,7 @@ int dense_gemm_choose_splits(int M, int N, int K) {
 }
 
 int wgrad_gemm_launch(const void* dy, int64_t ld_dy, const void* x, int64_t ld_x, float* c, int64_t ldc, int T, int M, int N, int splits,
-                      bool zero, hipStream_t stream);   // wgrad_gemm.hip
+                      hipStream_t stream);   // wgrad_gemm.hip
 
 // layout 0 NT: a [M][K] (lda), b [N][K] (ldb); layout 1 TN: a [K][M], b [K][N].
 // epi 0: c bf16 [M][N] = acc; 1: c fp32 += acc (splits forced to 1); 2: c fp32 += acc by atomics,
@@ -645,7 +645,7 @@ int dense_gemm_launch(int layout, int epi, const void* a, int64_t lda, const voi
   if (layout == dg::LTN && M % 8) return -1;
   if (epi == dg::BF16 && ldc % 8) return -1;
   if (layout == dg::LTN && epi != dg::BF16)   // weight gradients have a kernel of their own
-    return wgrad_gemm_launch(a, lda, b, ldb, static_cast<float*>(c), ldc, K, M, N, epi == dg::F32_ACC ? 1 : splits, false, stream);
+    return wgrad_gemm_launch(a, lda, b, ldb, static_cast<float*>(c), ldc, K, M, N, epi == dg::F32_ACC ? 1 : splits, stream);
   dg::Params p{};
   p.a = static_cast<const uint16_t*>(a);
   p.b = static_cast<const uint16_t*>(b);

@@ -67,8 +67,7 @@ __device__ __forceinline__ void grad_store(const f32x4_t& v, float* at) {
   else *reinterpret_cast<f32x4_t*>(at) = v;
 }
 
-// TAIL: a split may have a partial step (the first one); PAST: the gradient past the caches; ZERO: it is zeros and is not read (one split; it costs a third of a
-// short reduction's time: 8 experts' 4096 x 28672 and 14336 x 4096 over 1,024 uneven rows each, a layer forward and backward 10,381 -> 9,805)
+// TAIL: a split may have a partial step (the first one); PAST: the gradient past the caches; ZERO: the call itself has just cleared it, and it is not read (one split)
 template <bool GROUPED, bool TAIL, bool PAST, bool ZERO>
 __global__ void __launch_bounds__(NT, 1) wgrad_kernel(Params p) {
   __shared__ __attribute__((aligned(16))) char smem[tile::LDS_BYTES];
@@ -394,17 +393,13 @@ static int band_rows() {
   return b;
 }
 
-template <bool G, bool TAIL>
-void launch(const Params& p, int64_t nwg, bool past, bool zero, hipStream_t stream) {
-  auto* f = zero && p.own ? (past ? &wgrad_kernel<G, TAIL, true, true> : &wgrad_kernel<G, TAIL, false, true>)
-                          : (past ? &wgrad_kernel<G, TAIL, true, false> : &wgrad_kernel<G, TAIL, false, false>);
-  hipLaunchKernelGGL(f, dim3((unsigned)nwg), dim3(NT), 0, stream, p);
+template <bool G, bool TAIL, bool ZERO = false>
+void launch(const Params& p, int64_t nwg, bool past, hipStream_t stream) {
+  hipLaunchKernelGGL((past ? &wgrad_kernel<G, TAIL, true, ZERO> : &wgrad_kernel<G, TAIL, false, ZERO>), dim3((unsigned)nwg), dim3(NT), 0, stream, p);
 }
-template <bool G, bool TAIL>
-void launch_few(const Params& p, int64_t nwg, bool past, bool zero, hipStream_t stream) {
-  auto* f = zero ? (past ? &few::kernel<G, TAIL, true, true> : &few::kernel<G, TAIL, false, true>)
-                 : (past ? &few::kernel<G, TAIL, true, false> : &few::kernel<G, TAIL, false, false>);
-  hipLaunchKernelGGL(f, dim3((unsigned)nwg), dim3(few::NT), 0, stream, p);
+template <bool G, bool TAIL, bool ZERO = false>
+void launch_few(const Params& p, int64_t nwg, bool past, hipStream_t stream) {
+  hipLaunchKernelGGL((past ? &few::kernel<G, TAIL, true, ZERO> : &few::kernel<G, TAIL, false, ZERO>), dim3((unsigned)nwg), dim3(few::NT), 0, stream, p);
 }
 
 // Whether a gradient of so many bytes is read and written past the caches, which then keep the operands.  What a gradient costs depends on where it lies when it is
@@ -457,7 +452,7 @@ void wgrad_gemm_plan(int T, int M, int N, int splits, int* out) {
 
 // c [M, N] fp32 += dy[T, M]^T x[T, N]; M % 8 == 0, N % 8 == 0, 16-B aligned rows.
 int wgrad_gemm_launch(const void* dy, int64_t ld_dy, const void* x, int64_t ld_x, float* c, int64_t ldc, int T, int M,
-                      int N, int splits, bool zero, hipStream_t stream) {
+                      int N, int splits, hipStream_t stream) {
   if (T <= 0 || M <= 0 || N <= 0) return 0;
   if (M % 8 || N % 8 || ld_dy % 8 || ld_x % 8) return -1;
   wg::Params p{};
@@ -479,17 +474,16 @@ int wgrad_gemm_launch(const void* dy, int64_t ld_dy, const void* x, int64_t ld_x
   if (nwg > INT32_MAX) return -2;
   const bool past = wg::past_caches((int64_t)M * N * 4);
   if (p.own && wg::few::dense(T, p.mt * p.nt)) {
-    if (T % wg::few::BK) wg::launch_few<false, true>(p, nwg, past, zero, stream);
-    else wg::launch_few<false, false>(p, nwg, past, zero, stream);
+    if (T % wg::few::BK) wg::launch_few<false, true>(p, nwg, past, stream);
+    else wg::launch_few<false, false>(p, nwg, past, stream);
   } else if (T % wg::BK)
-    wg::launch<false, true>(p, nwg, past, zero, stream);
+    wg::launch<false, true>(p, nwg, past, stream);
   else
-    wg::launch<false, false>(p, nwg, past, zero, stream);
+    wg::launch<false, false>(p, nwg, past, stream);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
-// zero: c is zeros.
-// Grouped: c[e] [M, N] fp32 += dy[g0:g1]^T x[g0:g1] for every expert e, rows g0 = offs[e],
+// Grouped (zero: the caller has just cleared c, in this stream): c[e] [M, N] fp32 += dy[g0:g1]^T x[g0:g1] for every expert e, rows g0 = offs[e],
 // g1 = offs[e+1] read on the device; splits per group chosen for the mean group size rows / E.
 // M % 8 == 0, N % 8 == 0.
 int wgrad_gemm_grouped_launch(const void* dy, int64_t ld_dy, const void* x, int64_t ld_x, float* c, int64_t ldc,
@@ -517,8 +511,13 @@ int wgrad_gemm_grouped_launch(const void* dy, int64_t ld_dy, const void* x, int6
   const int64_t nwg = (int64_t)p.mt * p.nt * E * p.splits;
   if (nwg > INT32_MAX) return -2;
   const bool past = wg::past_caches((int64_t)E * M * N * 4);
-  if (p.own && rows / E <= wg::few::most(past)) wg::launch_few<true, true>(p, nwg, past, zero, stream);
-  else wg::launch<true, true>(p, nwg, past, zero, stream);
+  if (p.own && rows / E <= wg::few::most(past)) {
+    if (zero) wg::launch_few<true, true, true>(p, nwg, past, stream);
+    else wg::launch_few<true, true>(p, nwg, past, stream);
+  } else if (p.own && zero)
+    wg::launch<true, true, true>(p, nwg, past, stream);
+  else
+    wg::launch<true, true>(p, nwg, past, stream);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 

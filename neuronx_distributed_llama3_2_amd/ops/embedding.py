@@ -11,7 +11,6 @@ import torch
 import torch.nn.functional as F
 
 from ._ext import ext, use_native
-from .gemm import take_zero
 
 
 class EmbeddingFunc(torch.autograd.Function):
@@ -35,7 +34,6 @@ class EmbeddingFunc(torch.autograd.Function):
             from ..parallel_layers import stream_split
 
             stream_split.accumulate_begin(w)
-            take_zero(mg)
         ext().embedding_bwd(idc, dout.contiguous(), dw.view(w.shape), int(ctx.vocab_start))
         if mg is not None:
             stream_split.accumulate_end(w)

@@ -253,26 +253,6 @@ def _wgrad_scratch(n: int, dtype, device, tag: str = "") -> torch.Tensor:
     return t[:n]
 
 
-# A gradient that was just cleared need not be read by the product that is first added to it, which a short reduction spends a third of its time on.  The
-# mark is the version that clearing left the gradient at: whatever torch writes since, to it or to its flat buffer, makes it void; what writes without a
-# version (the kernels here that add to gradients, collectives) takes it, so that it is used once.  A product recorded into a graph reads what is there at every replay,
-# and a replay takes no mark: a gradient that a graph adds to is never marked again.
-def mark_zero(grads) -> None:
-    """The gradients have just been filled with zeros."""
-    recording = any(g.is_cuda for g in grads) and torch.cuda.is_current_stream_capturing()
-    for g in grads:
-        g._nxd_zero = None if recording or g.is_inference() or getattr(g, "_nxd_recorded", False) else g._version
-
-
-def take_zero(g: torch.Tensor) -> bool:
-    """Whether g still holds the zeros that mark_zero() was told of; whoever asks writes it."""
-    version = getattr(g, "_nxd_zero", None)
-    if g.is_cuda and torch.cuda.is_current_stream_capturing():
-        g._nxd_recorded, version = True, None
-    g._nxd_zero = None
-    return version is not None and version == g._version
-
-
 def wgrad_accumulate_(mg: torch.Tensor, go2: torch.Tensor, x2, go_t: torch.Tensor = None,
                       x_t: torch.Tensor = None) -> None:
     """mg [N, K] (fp32) += go2[T, N]^T @ x2[T, K].
@@ -288,13 +268,12 @@ def wgrad_accumulate_(mg: torch.Tensor, go2: torch.Tensor, x2, go_t: torch.Tenso
     if go2.shape[0] == 0:
         return
     has_copy = go_t is not None or x_t is not None
-    zero = take_zero(mg)
     if _use_wgrad_in_rounds(mg, go2, x2) or _use_dense_wgrad(mg, go2, x2, has_copy):
-        ext().wgrad_gemm(mg, go2, x2, 0, True, zero)
+        ext().wgrad_gemm(mg, go2, x2, 0, True)
         return
     splits = _wgrad_kernel_splits(mg, go2, x2, has_copy)
     if splits is not None:
-        ext().wgrad_gemm(mg, go2, x2, splits, True, zero)
+        ext().wgrad_gemm(mg, go2, x2, splits, True)
         return
     if x_t is not None and not (x_t.dim() == 2 and x_t.is_contiguous() and x_t.shape[1] == go2.shape[0]):
         x_t = None

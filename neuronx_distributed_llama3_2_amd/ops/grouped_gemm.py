@@ -18,7 +18,6 @@ from typing import List, Optional, Tuple
 import torch
 
 from ._ext import ext, use_native
-from .gemm import take_zero
 
 # "grouped" (default): the device-side grouped kernel, no host sync (hipGraph-capturable).
 # "loop": one hipBLASLt GEMM per expert (torch.matmul: its first heuristic -- the group sizes change
@@ -127,11 +126,11 @@ class GroupedLinearFunc(torch.autograd.Function):
             else:
                 ext().grouped_gemm(1, dy, w, offs, dx, False)
 
-        def wgrad(g, accumulate, zero=False):
+        def wgrad(g, accumulate):
             if bounds is not None:
                 _loop_wgrad(x, dy, bounds, g, accumulate)
             else:
-                ext().grouped_gemm(2, x, dy, offs, g, accumulate, zero)
+                ext().grouped_gemm(2, x, dy, offs, g, accumulate)
 
         dw = None
         if ctx.needs_input_grad[1]:
@@ -140,7 +139,7 @@ class GroupedLinearFunc(torch.autograd.Function):
                 from ..parallel_layers import stream_split
 
                 stream_split.accumulate_begin(w)   # (a load and a store of main_grad, as in the dense layers)
-                wgrad(mg, True, take_zero(mg))
+                wgrad(mg, True)
                 stream_split.accumulate_end(w)
                 cb = getattr(w, "_nxd_grad_ready", None)
                 if cb is not None:

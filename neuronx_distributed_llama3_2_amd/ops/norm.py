@@ -15,7 +15,6 @@ from typing import Optional, Tuple
 import torch
 
 from ._ext import ext, use_native
-from .gemm import take_zero
 
 
 def rms_norm_reference(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
@@ -75,7 +74,6 @@ class RMSNormFunc(torch.autograd.Function):
             from ..parallel_layers import stream_split   # (lazy: parallel_layers imports ops)
 
             stream_split.accumulate_begin(w)
-            take_zero(mg)
         ext().rmsnorm_bwd(dy, h, w, rstd, dres, dx, dw.view(-1), accumulate)
         if accumulate:
             stream_split.accumulate_end(w)

@@ -177,11 +177,7 @@ class FlatBuffer:
 
     def finish_grad_sync(self, average: bool = True) -> None:
         """Launch any bucket not yet launched, wait for all, average over DP."""
-        from ..ops.gemm import take_zero
-
         self.sync_enabled = False
-        for p in self.params:   # (collectives write them)
-            take_zero(p.main_grad)
         if self.dp == 1:
             if average and self.avg_world > 1:
                 self.grad_data.div_(self.avg_world)
@@ -234,10 +230,7 @@ class FlatBuffer:
         comm.assert_no_pending_collectives("gather_params")
 
     def zero_grad(self) -> None:
-        from ..ops.gemm import mark_zero
-
         self.grad_data.zero_()
-        mark_zero([p.main_grad for p in self.params])
 
     def set_sync(self, enabled: bool) -> None:
         self.sync_enabled = enabled

@@ -564,8 +564,6 @@ class NxDPPModel(nn.Module):
     def _reduce_shared_grads(self):
         if not self.shared_weights or self.pp_size == 1 or self._shared_groups is None:
             return
-        from ..ops.gemm import take_zero
-
         for grp, pg, ranks in self._shared_groups:
             if pg is None or dist.get_rank() not in ranks:
                 continue
@@ -575,7 +573,6 @@ class NxDPPModel(nn.Module):
                     g = getattr(p, "main_grad", None)
                     g = p.grad if g is None else g
                     if g is not None:
-                        take_zero(g)   # (other stages' sums come into it)
                         dist.all_reduce(g, group=pg)
                     break
 
