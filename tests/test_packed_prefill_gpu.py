@@ -86,3 +86,29 @@ def test_application_packs_what_pays():
     packed(torch.randint(1, 4096, (3, 450), device="cuda"), (torch.arange(450)[None] < torch.tensor([[450], [100], [90]])).long().cuda(),
            seq_ids=torch.tensor([2, 0, 3], dtype=torch.int32, device="cuda"))
     assert (3, 512, 640) in packed._prefill_cache and torch.equal(before, packed.model.kv_cache[:, :, 1])
+
+
+def test_runs_before_and_after_the_capture():
+    """The first runs of a key are launched one by one, the later ones replay its graph: the same kernels on the same rows, for ids and slots of any type and stride."""
+    from neuronx_distributed_llama3_2_amd.inference import InferenceConfig, LlamaForCausalLMInference
+    from neuronx_distributed_llama3_2_amd.inference.generation import PackedPrefill
+    from neuronx_distributed_llama3_2_amd.models.llama.modeling_llama import llama_config
+
+    cfg = llama_config("tiny", num_hidden_layers=2, hidden_size=512, intermediate_size=1024, num_attention_heads=8, num_key_value_heads=2, vocab_size=4096,
+                       max_position_embeddings=2048)
+    app = LlamaForCausalLMInference(cfg, InferenceConfig(batch_size=4, seq_len=1024, max_context_length=1024, enable_bucketing=True))
+    lens = torch.tensor([384, 70, 300])
+    mask = (torch.arange(384)[None] < lens[:, None]).long().cuda()
+    slots = torch.tensor([[2, 9], [0, 9], [3, 9]], device="cuda")[:, 0]
+    seen = None
+    for n in range(PackedPrefill.EAGER_RUNS + 3):
+        app.model.kv_cache.zero_()
+        ids = torch.randint(1, 4096, (384, 3), device="cuda", generator=torch.Generator(device="cuda").manual_seed(1), dtype=torch.int32).t()
+        logits = app(ids, mask, seq_ids=slots)
+        g = app._prefill_cache[(3, 384, 768)]
+        assert (g.graph is not None) == (n >= PackedPrefill.EAGER_RUNS)
+        got = (logits.clone(), app.model.kv_cache.clone())
+        seen = got if seen is None else seen
+        for a, b in zip(got, seen):
+            assert float((a.float() - b.float()).norm()) <= 0.01 * float(b.float().norm())
+        assert not app.model.kv_cache[:, :, 1].any() and not app.model.kv_cache[:, :, 2, :, 384:].any()

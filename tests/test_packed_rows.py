@@ -10,7 +10,7 @@ def test_rows():
     for n in range(1, 20000):
         r = packed_rows(n)
         assert n <= r < n + max(128, n / 8) and r % 128 == 0
-    for lo in (1024, 2048, 8192):   # at most eight graphs for twice the tokens
+    for lo in (1024, 2048, 8192):   # eight row counts for twice the tokens
         assert len({packed_rows(n) for n in range(lo + 1, 2 * lo + 1)}) == 8
     assert not packing_pays(128, 1, 512) and packing_pays(2016, 3, 768) and not packing_pays(2017, 3, 768) and packing_pays(128, 2, 512)
 
@@ -28,3 +28,66 @@ def test_packed_attention_reference():
     for a, b in ((0, 2), (2, 8)):
         want = ops.flash_attn_fwd_lse(q[None, a:b], k[None, a:b], v[None, a:b])[0][0]
         assert torch.allclose(o[a:b], want, atol=1e-6)
+
+
+class _Model:
+    def __init__(self):
+        self.rows = []
+
+    def forward_packed(self, ids, lengths, slots, rows):
+        assert ids.dtype == lengths.dtype == torch.int64 and slots.dtype == torch.int32
+        self.rows.append(rows)
+        return lengths.float()
+
+
+def _app(monkeypatch):
+    """An application's prefill cache alone; captures are counted."""
+    from neuronx_distributed_llama3_2_amd.inference import generation
+
+    captured = []
+
+    def capture(self, device, pool):
+        captured.append((*self.shape, self.rows))
+        self.graph = type("Graph", (), {"replay": lambda g: None})()
+        self.out = self._fwd()
+
+    monkeypatch.setattr(generation.PackedPrefill, "_capture", capture)
+    monkeypatch.setattr(torch.cuda, "graph_pool_handle", lambda: (0, 1))
+    waits = []
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda device=None: waits.append(device))
+    app = object.__new__(generation.LlamaForCausalLMInference)
+    app.model, app.device, app._prefill_cache, app._prefill_pool = _Model(), torch.device("cpu"), {}, None
+    return app, captured, waits
+
+
+def _ask(app, B, Tb, rows):
+    ids = torch.ones(B, Tb, dtype=torch.int32)
+    return app._prefill_graph(B, Tb, rows).run(ids, torch.arange(B), torch.full((B,), 4))
+
+
+def test_a_key_is_captured_when_it_has_come_often(monkeypatch):
+    app, captured, _ = _app(monkeypatch)
+    for n in range(1, 12):
+        assert _ask(app, 3, 768, 1664).tolist() == ([5, 5, 5] if n <= 8 else [0, 0, 0])   # (the stand-in's graph is that of no tokens)
+        _ask(app, 3, 768, 1536 - 128 * (n % 4))   # (four others, three times at most)
+        assert captured == ([] if n <= 8 else [(3, 768, 1664)])
+
+
+def test_keys_are_bounded_and_the_oldest_one_goes(monkeypatch):
+    from neuronx_distributed_llama3_2_amd.inference.bucketing import PACKED_KEYS
+
+    app, captured, waits = _app(monkeypatch)
+    app._prefill_cache[(1, 128)] = "padded"
+    for _ in range(9):
+        _ask(app, 9, 1024, 1024)
+    assert captured == [(9, 1024, 1024)]
+    for i in range(PACKED_KEYS - 1):
+        _ask(app, 9, 1024, 2048 + 128 * i)
+    _ask(app, 9, 1024, 1024)
+    _ask(app, 9, 1024, 128)   # (one too many: 2,048 rows were asked for first)
+    assert len(app._prefill_cache) == PACKED_KEYS + 1 and (9, 1024, 2048) not in app._prefill_cache and (9, 1024, 1024) in app._prefill_cache
+    assert not waits
+    for i in range(PACKED_KEYS):
+        _ask(app, 9, 2048, 2048 + 128 * i)
+    assert len(app._prefill_cache) == PACKED_KEYS + 1 and (9, 1024, 1024) not in app._prefill_cache
+    assert len(waits) == 1 and app._prefill_cache[(1, 128)] == "padded"   # (a graph that may run is waited for)
