@@ -95,13 +95,14 @@ __global__ void __launch_bounds__(tile::THREADS, 1) kernel(Params p) {
   pairs();
   f32x4_t acc[8][8];
   // a tile's results, rounded as the product leaves them, with the activation: 8 columns of a row a lane, 64 contiguous bytes of 16 rows a store
+  constexpr int FRAG_STORES = ACT == SWIGLU ? 2 : 4, STORES = 8 * FRAG_STORES;   // of a row fragment, of a tile
   auto out = [&](auto ok) __attribute__((always_inline)) {
     const int c0 = n0 + (ACT == SWIGLU ? 64 : 128) * wn + 8 * (lane >> 4);
     uint16_t* y = p.y + (int64_t)(r0 + 16 * wm + (lane & 15)) * p.N + c0;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
 #pragma unroll
-      for (int j = 0; j < (ACT == SWIGLU ? 4 : 8); j += 2) {
+      for (int j = 0; j < 2 * FRAG_STORES; j += 2) {
         auto rounded = [&](int jj, float (&v)[8]) __attribute__((always_inline)) {
           unpack8(u32x4_t{pack2bf(acc[i][jj][0], acc[i][jj][1]), pack2bf(acc[i][jj][2], acc[i][jj][3]), pack2bf(acc[i][jj + 1][0], acc[i][jj + 1][1]),
                           pack2bf(acc[i][jj + 1][2], acc[i][jj + 1][3])}, v);
@@ -126,14 +127,14 @@ __global__ void __launch_bounds__(tile::THREADS, 1) kernel(Params p) {
   if (PIPE && pieces == 1) {
     tile::Loop<false>::Frags<8> frags;
     loop.template begin<false>(frags, steps, false);
-    int stores = 0;
+    bool stored = false;
 #pragma unroll 1
     for (int k = 0; k < items; ++k) {
       const int R0 = r0, R1 = r1, N0 = n0;
       const bool another = k + 1 < items;
       if (another) place(k + 1);
       const int nr0 = r0, nr1 = r1, nn0 = n0;
-      loop.run_tile(acc, frags, steps, stores, another, [&]() __attribute__((always_inline)) {
+      loop.template run_tile<STORES>(acc, frags, steps, stored, another, [&]() __attribute__((always_inline)) {
         loop.set(x(nr0), p.K, nr1 - nr0, w(nn0), p.K, cols(nn0));
         pairs();
       });
@@ -141,7 +142,7 @@ __global__ void __launch_bounds__(tile::THREADS, 1) kernel(Params p) {
       const bool whole = r1 - r0 == BM && n0 + COLS <= p.N;
       if (whole) out([](int, int) { return true; });
       else out([&](int row, int col) { return row < r1 && col < p.N; });
-      stores = !whole ? 0 : ACT == SWIGLU ? 16 : 32;
+      stored = whole;
       r0 = nr0, r1 = nr1, n0 = nn0;
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (loads that nothing reads)

@@ -401,10 +401,11 @@ struct Loop {
   }
 
   // acc = the products of one of several tiles, of so many whole steps each (2 or more), after begin() for the first one.  next(), if there is another one: the
-  // loads go over to it, two steps before the end, so that it begins without a wait.  stores: vector stores since the last tile, where all of them were made,
-  // else 0: the first step's loads came before them and are waited for alone.
-  template <typename NEXT>
-  __device__ __forceinline__ void run_tile(f32x4_t (&acc)[8][8], Frags<8>& f, int steps, int stores, bool another, NEXT&& next) {
+  // loads go over to it, two steps before the end, so that it begins without a wait.  stored: every wave has made STORES vector stores since the last tile, no
+  // fewer: the first step's loads came before them and are waited for alone (more stores, or other vector memory operations, would only be waited for too).
+  template <int STORES, typename NEXT>
+  __device__ __forceinline__ void run_tile(f32x4_t (&acc)[8][8], Frags<8>& f, int steps, bool stored, bool another, NEXT&& next) {
+    static_assert(8 + STORES < 64, "vmcnt");
     const auto rest = [&](int t, int end) __attribute__((always_inline)) {   // towards step t + 3, or the next tile's t + 3 - steps
 #pragma unroll 1
       for (; t < end; ++t)
@@ -413,8 +414,7 @@ struct Loop {
     const int turn = steps - 2;
     if (turn == 0 && another) next();
     step<false, true>(acc, f, false, 3 < steps || (another && steps == 2), [&]() {
-      if (stores == 32) asm volatile("s_waitcnt vmcnt(40)" ::: "memory");
-      else if (stores == 16) asm volatile("s_waitcnt vmcnt(24)" ::: "memory");
+      if (stored) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 + STORES) : "memory");
       else asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
     });
     rest(1, turn);

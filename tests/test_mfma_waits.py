@@ -89,6 +89,25 @@ def test_products_have_their_waits(name, tmp_path):
         assert not _close(code, labels)[:5], f
 
 
+def test_stores_between_tiles_are_as_many_as_the_wait_says(tmp_path):
+    """A tile's stores are in flight while the next tile's first step waits for the loads ahead of them by their count: vmcnt(8 + stores), in products whose workgroups
+    have several tiles.  Fewer stores in its path would let it go on too early; registers in scratch memory would make that path another one."""
+    asm = _assembly("act_gemm", tmp_path)
+    assert set(re.findall(r"; ScratchSize: (\d+)", asm)) == {"0"}
+    seen = {}
+    for f, (code, labels) in _functions(asm).items():
+        counts = {int(n) for op, args in code if op == "s_waitcnt" for n in re.findall(r"vmcnt\((\d+)\)", args)}
+        several = counts & {8 + 16, 8 + 32}
+        if several and any(op.startswith("v_mfma") for op, _ in code):
+            edges = sorted({0, len(code), *labels.values(), *(i + 1 for i, (op, _) in enumerate(code) if op.startswith(("s_branch", "s_cbranch")))})
+            # the path without checks: a straight line with more than one store
+            lines = [[op for op, _ in code[a:b] if op.startswith(("global_", "flat_", "buffer_", "scratch_"))] for a, b in zip(edges, edges[1:])]
+            seen[f] = (max(several), [ops for ops in lines if sum(op.startswith("global_store") for op in ops) > 1])
+    assert len(seen) == 2
+    for f, (wait, paths) in seen.items():
+        assert [set(p) for p in paths] == [{"global_store_dwordx4"}] and len(paths[0]) == wait - 8, f
+
+
 def test_what_is_too_near_is_found():
     near = "k:\n\tv_mfma_f32_16x16x32_bf16 a[0:3], v[0:3], v[4:7], a[0:3]\n\ts_nop {}\n\tv_accvgpr_read_b32 v9, a2\n"
     assert not _close(*_functions(near.format(7))["k"]) and _close(*_functions(near.format(6))["k"])
