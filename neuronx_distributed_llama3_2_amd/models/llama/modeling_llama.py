@@ -30,6 +30,7 @@ from torch.utils.checkpoint import checkpoint
 
 from ... import ops
 from ...modules.qkv_linear import GQAQKVColumnParallelLinear
+from ...ops.gemm import kernel_gradients
 from ...parallel_layers.layer_norm import RMSNorm
 from ...parallel_layers.layers import ColumnParallelLinear, ParallelEmbedding, RowParallelLinear
 from ...parallel_layers.loss_functions import parallel_cross_entropy
@@ -72,13 +73,15 @@ class LlamaMLP(nn.Module):
                                            dtype=dtype, device=device)
         self.selective_checkpoint = getattr(config, "selective_checkpoint_enabled", False)
 
-    def forward(self, x):
-        gu = self.gate_up_proj(x)
+    def act(self, gu, width):
+        """SwiGLU of gate_up's output; width: gate_up's input's and down's output's."""
+        width = width if kernel_gradients(self.gate_up_proj, self.down_proj) else None
         if self.selective_checkpoint and self.training:
-            h = checkpoint(ops.swiglu, gu, True, x.shape[-1], use_reentrant=False)
-        else:
-            h = ops.swiglu(gu, token_major=True, width=x.shape[-1])   # token-major copies feed the TN weight gradients
-        return self.down_proj(h)
+            return checkpoint(ops.swiglu, gu, True, width, use_reentrant=False)
+        return ops.swiglu(gu, token_major=True, width=width)   # token-major copies feed the TN weight gradients
+
+    def forward(self, x):
+        return self.down_proj(self.act(self.gate_up_proj(x), x.shape[-1]))
 
 
 class LlamaAttention(nn.Module):
@@ -193,11 +196,7 @@ class LlamaDecoderLayer(nn.Module):
         mlp = self.mlp
         gu = mlp.gate_up_proj(normed)
         yield
-        if mlp.selective_checkpoint and self.training:
-            h = checkpoint(ops.swiglu, gu, True, normed.shape[-1], use_reentrant=False)
-        else:
-            h = ops.swiglu(gu, token_major=True, width=normed.shape[-1])
-        out = mlp.down_proj(h)
+        out = mlp.down_proj(mlp.act(gu, normed.shape[-1]))
         yield
         return out, residual
 

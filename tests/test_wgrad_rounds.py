@@ -58,3 +58,52 @@ def test_swiglu_writes_copies_for_the_library_only(rows, width, copies):
         out.append((h.detach(), leaf.grad))
     assert seen == [copies, False]
     assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+
+
+def _mlp(width, inter, device, grad_dtype):
+    """A Llama MLP and what its SwiGLU was told of the width; grad_dtype: of its gradient buffer, None: it has none."""
+    from neuronx_distributed_llama3_2_amd.models.llama.modeling_llama import LlamaMLP, llama_config
+    from neuronx_distributed_llama3_2_amd.parallel.grad_buffer import FlatBuffer
+    from neuronx_distributed_llama3_2_amd.parallel_layers import parallel_state as ps
+    import torch.distributed as dist
+
+    if not dist.is_initialized():
+        dist.init_process_group("gloo", store=dist.HashStore(), rank=0, world_size=1)
+    if not ps.model_parallel_is_initialized():
+        ps.initialize_model_parallel(1)
+    mlp = LlamaMLP(llama_config("tiny", hidden_size=width, intermediate_size=inter), torch.bfloat16, torch.device(device))
+    buf = FlatBuffer(list(mlp.parameters()), grad_dtype=grad_dtype) if grad_dtype is not None else None
+    return mlp, buf
+
+
+@pytest.mark.parametrize("grad_dtype,width", [(torch.float32, 64), (torch.bfloat16, None), (None, None)])
+def test_swiglu_is_told_the_width_where_the_kernel_can_add_to_the_gradients(grad_dtype, width, monkeypatch):
+    from neuronx_distributed_llama3_2_amd.models.llama import modeling_llama
+
+    mlp, _ = _mlp(64, 128, "cpu", grad_dtype)
+    told = []
+    monkeypatch.setattr(modeling_llama.ops, "swiglu", lambda gu, token_major=False, width=None: told.append(width) or ops.swiglu_reference(gu))
+    for selective in (False, True):
+        mlp.selective_checkpoint = selective
+        mlp(torch.randn(5, 1, 64).bfloat16().requires_grad_())
+    assert told == [width, width]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("grad_dtype", [torch.float32, torch.bfloat16, None])
+def test_an_mlp_whose_gradients_go_to_the_library_has_its_copies(grad_dtype):
+    """3,072 tokens, 4096 wide, 3840: both gradients fill their rounds of tiles.  Against float64; a 16-bit gradient is rounded once more (2^-9)."""
+    mlp, buf = _mlp(4096, 3840, "cuda", grad_dtype)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn(3072, 1, 4096, generator=g, device="cuda").bfloat16().requires_grad_()
+    gu = mlp.gate_up_proj(x)
+    h = mlp.act(gu, 4096)
+    assert hasattr(h, "_nxd_t") == (grad_dtype is not torch.float32)
+    dy = torch.randn(3072, 1, 4096, generator=g, device="cuda").bfloat16()
+    if buf is not None:
+        buf.zero_grad()
+    mlp.down_proj(h).backward(dy)
+    w = mlp.down_proj.weight
+    got = w.main_grad if buf is not None else w.grad
+    want = dy[:, 0].double().t() @ h[:, 0].double()
+    assert float((got.double() - want).norm()) < (1e-5 if grad_dtype is torch.float32 else 3 * 2 ** -9) * float(want.norm())
