@@ -228,7 +228,9 @@ def wgrad_in_rounds(T: int, M: int, N: int) -> bool:
     nobody needs to write transposed copies for it."""
     tiles = -(-M // 256) * -(-N // 256)
     rounds = -(-tiles // 256)
-    if _WG_KERNEL == "0" or M % 8 or N % 8 or (T % 64 == 0 and T < _WG_WHOLE_TOKENS):
+    if _WG_KERNEL == "0" or _WGRAD_BF16 or _WGRAD_T == "2":   # (NXD_WGRAD_BF16=1, NXD_WGRAD_T=2: the library's products are asked for)
+        return False
+    if M % 8 or N % 8 or (T % 64 == 0 and T < _WG_WHOLE_TOKENS):
         return False
     return 8 * tiles >= 7 * 256 if rounds == 1 else 3 * tiles >= 2 * 256 * rounds
 

@@ -60,6 +60,25 @@ def test_swiglu_writes_copies_for_the_library_only(rows, width, copies):
     assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
 
 
+@pytest.mark.parametrize("name,value", [("_WGRAD_BF16", True), ("_WGRAD_T", "2"), ("_WG_KERNEL", "0")])
+def test_switches_that_ask_for_the_library(name, value, monkeypatch):
+    monkeypatch.setattr(gemm, name, value)
+    assert not gemm.wgrad_in_rounds(8192, 4096, 4096)
+
+
+@pytest.mark.gpu
+def test_a_gradient_that_is_asked_for_in_16_bits(monkeypatch):
+    """NXD_WGRAD_BF16=1: what a producer's copies come with is rounded to bf16 before it is added to the fp32 gradient."""
+    monkeypatch.setattr(gemm, "_WGRAD_BF16", True)
+    g = torch.Generator(device="cuda").manual_seed(2)
+    dy, x = torch.randn(4096, 8192, generator=g, device="cuda").bfloat16(), torch.randn(4096, 8192, generator=g, device="cuda").bfloat16()
+    mg = torch.zeros(8192, 8192, device="cuda")
+    gemm.wgrad_accumulate_(mg, dy, x, go_t=dy.t().contiguous())
+    assert torch.equal(mg, mg.bfloat16().float())
+    want = dy.double().t() @ x.double()
+    assert float((mg.double() - want).norm()) < 2 ** -8 * float(want.norm())
+
+
 def _mlp(width, inter, device, grad_dtype):
     """A Llama MLP and what its SwiGLU was told of the width; grad_dtype: of its gradient buffer, None: it has none."""
     from neuronx_distributed_llama3_2_amd.models.llama.modeling_llama import LlamaMLP, llama_config
