@@ -16,8 +16,8 @@
 // 1,057 -> 832 (two ping-pong groups of 4 waves, grid of the worst case's tiles; the loop's ring since: gemm_tile.h).
 // Few rows (bound by the weights' bytes): a tile of at most 128 rows loads and leaves in memory only the rows that there are.  16 rows of 8
 // experts, FWD / DGRAD us, two groups of 4 waves -> here, and with all rows loaded and left: 4096 -> 28672 414 / 422 -> 414 / 387, 444 / 420; 14336 -> 4096
-// 311 / 307 -> 214 / 217, 245 / 245; 4096 -> 1024 93 / 91 -> 55 / 52, 76 / 72.  What is not split waits for each step's loads, the weights one
-// step ahead and the rows two: 16 experts, 6144 -> 2688, 140 / 152 -> 142 / 162 (rows one step ahead too).
+// 311 / 307 -> 214 / 217, 245 / 245; 4096 -> 1024 93 / 91 -> 55 / 52, 76 / 72.  Such tiles have a ring of three or four steps of both operands
+// (run_few in gemm_tile.h), and split ones leave their sums past the L2: 4096 -> 28672 389 / 369 -> 318 / 350.
 #include "gemm_tile.h"
 
 #include <cstdlib>

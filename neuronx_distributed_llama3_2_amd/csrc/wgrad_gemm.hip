@@ -421,10 +421,10 @@ bool past_caches(int64_t bytes) { return bytes >= (int64_t)20 << 20; }
 // Token splits per output tile.  Cost model in token steps (1.2 us) of one workgroup, times 256: grid waves of 256 workgroups x the steps
 // per split, and the epilogues: 8 steps without a split; with splits 10 for one of them, and the atomics' rate bounds all workgroups together, 40
 // steps for 256 tiles.  The smallest split count of minimal cost, of 4 steps at least, from 1,024 tokens on (below, unsplit products of few tiles take
-// no longer than the shortest split ones and add in one order).  Unsplit / in the given splits, us: 1,000 tokens 6144 x 4096 83 / 2: 199,
-// 2048 x 2048 40 / 2: 40; 1,024 tokens 512 x 512 32 / 2: 25.7 / 4: 21.0, 1024 x 1024 32 / 2: 26.3 / 4: 22.0 / 8: 32, 768 x 4096 34 / 2: 34 / 3: 40;
-// 3,000 tokens 3072 x 2048 76 / 2: 73 / 3: 109, 2048 x 2048 76 / 2: 59 / 4: 71; 4,096 tokens 512 x 512 94 / 8: 26 / 16: 22; 8,192 tokens 6144 x 4096
-// 372 / 2: 411, 512 x 4096 168 / 4: 67 / 8: 76; 32,768 tokens 6144 x 4096 1,485 / 2: 1,305, 768 x 4096 670 / 5: 195 / 6: 288.
+// no longer than the shortest split ones and add in one order).  (A step takes 1.0 us since the loop has one read, address or load between two MFMAs; the choices are within 3 % of
+// the best all the same.)  Unsplit / in the given splits, us, gradients from memory: 1,000 tokens 6144 x 4096 90 / 2: 196, 2048 x 2048 39 / 2: 41; 1,024 tokens 512 x 512 34 /
+// 2: 27 / 4: 22, 1024 x 1024 35 / 2: 27 / 4: 24 / 8: 35, 768 x 4096 37 / 2: 35 / 3: 42; 3,000 tokens 3072 x 2048 74 / 2: 74 / 3: 106, 2048 x 2048 71 / 2: 58 / 4: 71; 4,096 tokens 512 x
+// 512 84 / 8: 27 / 16: 24; 8,192 tokens 6144 x 4096 346 / 2: 409, 512 x 4096 157 / 4: 72 / 8: 80; 32,768 tokens 6144 x 4096 1,323 / 2: 1,163, 768 x 4096 579 / 5: 188 / 6: 270.
 int wgrad_gemm_choose_splits(int T, int M, int N) {
   const int64_t tiles = (int64_t)ceil_div(M, wg::BM) * ceil_div(N, wg::BN);
   const int steps = ceil_div(T, wg::BK);

@@ -52,16 +52,17 @@ _ACTS = {"swiglu": 0, "relu2": 1}
 
 
 def act_pays(rows: int, weight_rows: int, K: int, glu: bool = False) -> bool:
-    """Whether csrc/act_gemm.hip is faster than a library product and the activation's own pass: work for three quarters of the CUs (256 x 256
+    """Whether csrc/act_gemm.hip takes a product and its activation, instead of a library product and the activation's own pass, which it was measured to be faster than: work for three quarters of the CUs (256 x 256
     results each), a reduction that the pass is not small beside, and rounds of the CUs that are filled to three quarters: what is left after whole rounds
     takes a whole one too, or, cut into 2 or 4 pieces, about two thirds of one (half of one if the pieces leave half of the CUs to themselves); up to a reduction of 1,024 the
     pass is so large a part that this does not matter (SwiGLU of 4,096 at 2,304 rows 53 / 43).  us, two launches / one,
     weights from memory: SwiGLU of 8,192 columns, reduction 2,048: 768 rows 52 / 47, 1,024 64 / 53, 1,664 110 / 94, 2,304 144 / 132, 4,096 226 / 197; of 14,336, 4,096: 512 rows
     108 / 94, 1,792 367 / 305, 5,120 977 / 799; of 11,008, 4,096: 4,096 681 / 507; squared ReLU of 12,288, 2,048: 640 rows 42 /
     42, 1,024 55 / 44, 4,096 178 / 145.  Rounds that are not filled (two launches): SwiGLU of 14,336, 4,096 at 384 rows 92 / 96, 640 146 / 157, 1,152 239 / 240, 8,192 at 1,152 85 /
-    86, 3,072 at 1,280 121 / 126, 11,008 at 896 155 / 156, squared ReLU of 16,384, 4,096 at 1,280 150 / 156 (a part of a round below three quarters of it would pay in some places: 11,008 at
-    512 rows 93 / 82, squared ReLU of 12,288 at 896 50 / 44).  The library does best where its tiles fill whole rounds too, and a long reduction hides SwiGLU's
-    pass: there two launches stay, although they are the slower ones since a workgroup has several tiles: of 14,336, 4,096 at 4,096 / 12,288 rows 685 / 618, 2,047 / 1,886."""
+    86, 3,072 at 1,280 121 / 126, 11,008 at 896 155 / 156, squared ReLU of 16,384, 4,096 at 1,280 150 / 156 (a part of a round below three quarters of it would pay in some places, which the rule
+    leaves to two launches: 11,008 at 512 rows 93 / 82, squared ReLU of 12,288 at 896 50 / 44).  One line is older than the kernel is now: SwiGLU's reductions above 3,072 in four
+    whole rounds and more went to two launches when a workgroup had one tile (706 / 714), and still do, though one would be the faster since it has up to four: of 14,336, 4,096 at
+    4,096 / 12,288 rows 685 / 618, 2,047 / 1,886."""
     if K % 32 or K > 4096 or rows * weight_rows < 192 * 256 * 256:
         return False
     if K <= 1024:
@@ -155,7 +156,11 @@ def _use_wgrad_t(go2: torch.Tensor, x2: torch.Tensor = None, K: int = None) -> b
 # to 1,000 (0.75-0.92; at 1,500 0.89-1.07), and from 7/8 at any even count (0.73-0.97 from 224 to 1,576 tiles up to 16,392
 # tokens).  Less full: 128 tiles 1.13 over 1,000, 1.70 over 8,200; 280 tiles 1.22 over 3,000; 96 tiles 1.08 over 500.  Odd
 # counts take no transposes: 0.83-0.95 at 1,001, 0.91-0.98 at 3,071, slower from 4,001 on.  M N / (M + N) measured up to 3,737.
-# (All of that with the main loop as it was; what fills its rounds comes here no more: wgrad_in_rounds.)
+# All of that with the main loop as it was; what fills its rounds comes here no more (wgrad_in_rounds).  With the loop as it is, time over the library's: ragged counts of 192 and
+# 208 tiles 0.69-0.81 from 72 to 1,000 tokens, 128 tiles 0.81 up to 200 and 1.05 at 500, 264 and 280 tiles 0.86-0.94 up to 200 and 0.97 at 500, 96 tiles 0.87-0.93 up to 320, but 64
+# tiles 1.3-1.6 there; vocabulary-sized ones in whole steps (16,032 to 128,256, 256 to 2,944 tokens) 0.79-0.95; M N / (M + N) < 1,100: 0.72-0.89 from 16,384 tokens on, 0.8-1.0
+# at 8,192, and slower for fewer tokens (1.1-1.3 at 4,096, 1.4-1.7 at 512 to 2,048, 512 x 512 1.7-2.4): the line was drawn at 16,384 tokens of tensor-parallel
+# shards, and has not been moved.  Nor have single rounds below seven eighths past 1,000 tokens (208 tiles, 3,001 tokens: 0.75).
 _WG_KERNEL = os.environ.get("NXD_WGRAD_KERNEL", "auto")
 _WG_SKINNY = 1100.0
 _WG_WIDE = 16000
@@ -191,10 +196,10 @@ def _use_wgrad_kernel(mg: torch.Tensor, go2: torch.Tensor, x2: torch.Tensor, has
 
 
 # Whole steps of 64 tokens and no producer copy, M N / (M + N) < 2200: the wgrad kernel as well, with its own choice of splits.
-# Its time over the library's (with two transposes from M N / (M + N) = 1,200 on), 64 to 32,768 tokens: 4,096 x 4,096 0.74-0.88,
-# 2,048 x 8,192 0.77-0.85, 16,384 x 2,048 0.82-0.95, 3,584 x 4,096 0.81-0.95, 3,072 x 4,096 0.81-1.0; from 16,384 tokens on also smaller
-# ones (2,048 x 2,048 0.8, 512 x 4,096 0.7-0.8).  The library is faster for few tiles over few tokens: 2,048 x 2,048 1.4-1.6 over 64 to 4,096
-# tokens, 768 x 4,096 1.3-1.9, 512 x 512 1.2-2.5.  Time over that of the TN form of csrc/dense_gemm.hip, which was here before: 0.67-1.01.
+# Its time over the library's (with two transposes from M N / (M + N) = 1,200 on), 64 to 16,384 tokens: 4,096 x 4,096 0.74-0.86,
+# 2,048 x 8,192 0.69-0.85, 16,384 x 2,048 0.70-0.93, 3,584 x 4,096 0.77-0.90, 3,072 x 4,096 0.77-0.92; from 16,384 tokens on also smaller
+# ones (2,048 x 2,048 0.76, 768 x 4,096 0.83).  The library is faster for few tiles over few tokens: 2,048 x 2,048 1.2-1.65 over 64 to 4,096
+# tokens, 768 x 4,096 1.1-1.7, 512 x 512 1.1-2.4.  Time over that of the TN form of csrc/dense_gemm.hip, which was here before: 0.67-1.01.
 # NXD_DENSE_WGRAD = auto | 1 (whenever the shapes allow) | 0.
 _DENSE_WG = os.environ.get("NXD_DENSE_WGRAD", "auto")
 _DENSE_WG_SKINNY = 2200.0
