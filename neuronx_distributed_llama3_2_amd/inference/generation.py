@@ -414,9 +414,11 @@ class LlamaForCausalLMInference:
         and can matter."""
         if not (self._halfway_lengths and generated(self.config) and self.model.packed_prefill_ok()) or B * Tb < HALFWAY_TOKENS:
             return 0
+        if torch.cuda.is_current_stream_capturing():   # (a call inside a caller's capture is no key's first run: it is what it is with padding)
+            return 0
         if mask is None:
             total = B * T
-        elif B == 1 and not packing_pays(packed_rows(T), 1, Tb) or mask.is_cuda and torch.cuda.is_current_stream_capturing():
+        elif B == 1 and not packing_pays(packed_rows(T), 1, Tb):
             return 0
         else:
             n = mask.sum(1).tolist()

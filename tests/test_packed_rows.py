@@ -1,4 +1,5 @@
 """How many rows prompts without their padding are given, and when that is done; attention over packed sequences on the CPU."""
+import pytest
 import torch
 
 from neuronx_distributed_llama3_2_amd import ops
@@ -91,3 +92,13 @@ def test_keys_are_bounded_and_the_oldest_one_goes(monkeypatch):
         _ask(app, 9, 2048, 2048 + 128 * i)
     assert len(app._prefill_cache) == PACKED_KEYS + 1 and (9, 1024, 1024) not in app._prefill_cache
     assert len(waits) == 1 and app._prefill_cache[(1, 128)] == "padded"   # (a graph that may run is waited for)
+
+
+@pytest.mark.parametrize("capturing,mask,rows", [(False, None, 1664), (True, None, 0), (False, "cpu", 1152), (True, "cpu", 0)])
+def test_a_call_inside_a_callers_capture_is_not_packed(monkeypatch, capturing, mask, rows):
+    app, _, _ = _app(monkeypatch)
+    app.config = InferenceConfig(enable_bucketing=True, batch_size=3, seq_len=2048, max_context_length=2048)
+    app.model.packed_prefill_ok = lambda: True
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
+    mask = mask and (torch.arange(540)[None] < torch.tensor([[540], [400], [200]])).long()
+    assert app._packed_rows(3, 540, 768, mask) == rows
