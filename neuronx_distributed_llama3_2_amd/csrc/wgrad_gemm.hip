@@ -67,7 +67,8 @@ __device__ __forceinline__ void grad_store(const f32x4_t& v, float* at) {
   else *reinterpret_cast<f32x4_t*>(at) = v;
 }
 
-// TAIL: a split may have a partial step (the first one); PAST: the gradient past the caches; ZERO: the call itself has just cleared it, and it is not read (one split)
+// TAIL: a split may have a partial step (the first one); PAST: the gradient past the caches; ZERO: the call itself has just cleared it, and it is not read (one split): 8 experts 4096 x 28672,
+// with the clearing, 8,192 rows 3,167 -> 2,665 us, 1,024 2,011 -> 1,295; 14336 x 4096 8,192 rows 1,569 -> 1,283
 template <bool GROUPED, bool TAIL, bool PAST, bool ZERO>
 __global__ void __launch_bounds__(NT, 1) wgrad_kernel(Params p) {
   __shared__ __attribute__((aligned(16))) char smem[tile::LDS_BYTES];
